@@ -211,8 +211,9 @@ class Buffer:
           handle   (src_info [E_l, N] int32, layout_range [E_l, R] int64 = (begin << 32) | count,
                    num_max_dispatch_tokens_per_rank, hidden, num_experts);
           the returned tensors are reused by the next call with the same shape.
-        async_finish is accepted and an event is returned either way, as in the reference
-        (deep_ep/buffer.py:2449 returns EventOverlap(EventHandle()) whatever the flag says).
+        An event is returned either way, as in the reference (deep_ep/buffer.py:2449 returns
+        EventOverlap(EventHandle()) whatever the flag says); without async_finish it is recorded when another
+        stream waits on it, since the call's own stream is in order already.
         """
         prof = None
         if _PROFILE_ENABLED:
@@ -222,13 +223,13 @@ class Buffer:
             prof.mark("start")
         recv_x, recv_scales, recv_count, src_info, layout_range, event, hook = self.runtime.low_latency_dispatch(
             x, topk_idx, cumulative_local_expert_recv_stats, dispatch_wait_recv_cost_stats,
-            num_max_dispatch_tokens_per_rank, num_experts, use_fp8, round_scale, use_ue8m0, True, return_recv_hook)
+            num_max_dispatch_tokens_per_rank, num_experts, use_fp8, round_scale, use_ue8m0, async_finish, return_recv_hook)
         handle = (src_info, layout_range, num_max_dispatch_tokens_per_rank, x.size(1), num_experts)
         if prof:
             prof.mark("end")
             prof.finish_iter()
         out = (recv_x, recv_scales) if use_fp8 else recv_x
-        return out, recv_count, handle, EventOverlap(event), hook
+        return out, recv_count, handle, EventOverlap(event or EventHandle.deferred()), hook
 
     def low_latency_combine(self, x: torch.Tensor, topk_idx: torch.Tensor, topk_weights: torch.Tensor, handle: tuple,
                             use_logfmt: bool = False, zero_copy: bool = False, async_finish: bool = False,
@@ -242,8 +243,9 @@ class Buffer:
         accumulate (needs `out`): the sum starts from float32(out[t]) instead of zero — the flag the
         reference's reduce takes (csrc/kernels/coop_combine_recv.cuh:174-179) and its Python fixes to False
         (deep_ep/buffer.py:2541).
-        async_finish is accepted and an event is returned either way, as in the reference
-        (deep_ep/buffer.py:2801-2803 returns EventOverlap(EventHandle()) whatever the flag says).
+        An event is returned either way, as in the reference (deep_ep/buffer.py:2801-2803 returns
+        EventOverlap(EventHandle()) whatever the flag says); without async_finish it is recorded when another
+        stream waits on it, since the call's own stream is in order already.
         """
         assert not accumulate or out is not None, "accumulate adds to `out`"
         src_info, layout_range, num_max_dispatch_tokens_per_rank, hidden, num_experts = handle
@@ -255,12 +257,12 @@ class Buffer:
             prof.mark("start")
         combined_x, event, hook = self.runtime.low_latency_combine(
             x, topk_idx, topk_weights, src_info, layout_range, combine_wait_recv_cost_stats,
-            num_max_dispatch_tokens_per_rank, num_experts, use_logfmt, zero_copy, True, return_recv_hook, out,
+            num_max_dispatch_tokens_per_rank, num_experts, use_logfmt, zero_copy, async_finish, return_recv_hook, out,
             accumulate)
         if prof:
             prof.mark("end")
             prof.finish_iter()
-        return combined_x, EventOverlap(event), hook
+        return combined_x, EventOverlap(event or EventHandle.deferred()), hook
 
     def low_latency_update_mask_buffer(self, rank_to_mask: int, mask: bool = False) -> None:
         self.runtime.low_latency_update_mask_buffer(rank_to_mask, mask)

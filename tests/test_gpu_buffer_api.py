@@ -220,6 +220,40 @@ def test_dispatch_matches_oracle_through_the_api(deep_ep):
     buffer.destroy()
 
 
+@pytest.mark.parametrize("async_finish", (False, True))
+@pytest.mark.parametrize("caller", ("pool", "default"))
+def test_another_stream_waits_on_the_returned_events(deep_ep, caller, async_finish):
+    """The event of a call covers its work for a stream that did not make the call, however late it is asked."""
+    num_ranks, rank, t, h, k, e = 8, 2, 32, 1024, 4, 64
+    buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=num_ranks,
+                            sim_rank=rank, sim_seed=13)
+    x, topk_idx = buffer.loopback_synthesise(t, h, k, e)
+    w = torch.rand((t, k), generator=torch.Generator().manual_seed(4)).cuda()
+    recv_x, count, handle, _, _ = buffer.low_latency_dispatch(x, topk_idx, t, e, use_fp8=False)
+    y = recv_x.clone()
+    combined, _, _ = buffer.low_latency_combine(y, topk_idx, w, handle)
+    want_count, want_combined = count.clone(), combined.clone()
+    count.zero_(), combined.zero_()
+    torch.cuda.synchronize()
+    mine = torch.cuda.Stream() if caller == "pool" else torch.cuda.default_stream()
+    other = torch.cuda.Stream()
+    with torch.cuda.stream(mine):
+        torch.cuda._sleep(4_000_000)
+        _, count, handle, dispatched, _ = buffer.low_latency_dispatch(x, topk_idx, t, e, use_fp8=False,
+                                                                      async_finish=async_finish)
+        combined, reduced, _ = buffer.low_latency_combine(y, topk_idx, w, handle, async_finish=async_finish)
+        dispatched.current_stream_wait()  # its own stream: in order already
+    with torch.cuda.stream(other):
+        dispatched.current_stream_wait()
+        got_count = count.clone()
+        with reduced:
+            pass
+        got_combined = combined.clone()
+    torch.cuda.synchronize()
+    assert torch.equal(got_count, want_count) and torch.equal(got_combined, want_combined)
+    buffer.destroy()
+
+
 def test_combine_accumulates_into_out_through_the_api(deep_ep):
     """accumulate=True starts the float32 sum from what `out` holds (csrc/kernels/coop_combine_recv.cuh:174-179):
     checked bit for bit against the float32 FMA chain started from the previous contents."""
