@@ -7,6 +7,7 @@
 // There is no device code in this file and no CPU fallback: a missing or
 // failing HIP library is an exception.
 #include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPFunctions.h>
@@ -60,6 +61,29 @@ template <typename T>
 static T align_up(T a, T b) {
     return (a + b - 1) / b * b;
 }
+
+// Several results of one call in one allocation.  A torch::empty costs the host 1.2 us and a tensor over a piece
+// of storage that exists 0.1 us, so a call with many small results asks the allocator once.
+struct ResultBlock {
+    int64_t bytes = 0;
+    torch::Tensor block;
+
+    int64_t reserve(int64_t size) {  // a byte offset, on a line of its own
+        const int64_t at = bytes;
+        bytes += align_up<int64_t>(size, 256);
+        return at;
+    }
+    void allocate(const torch::Device& device) {
+        block = torch::Tensor(at::detail::empty_cuda({std::max<int64_t>(bytes, 256)}, torch::kUInt8, device, std::nullopt));
+    }
+    torch::Tensor take(int64_t at, at::IntArrayRef sizes, torch::ScalarType type) const {
+        auto t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(block.storage()), block.key_set(),
+                                                          c10::scalarTypeToTypeMeta(type));
+        t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+        t.unsafeGetTensorImpl()->set_storage_offset(at / int64_t(c10::elementSize(type)));
+        return t;
+    }
+};
 
 // ---------------------------------------------------------------------------
 // Config (reference: csrc/config.hpp:23-105) — arithmetic only.
@@ -835,6 +859,213 @@ ll_exchange_metadata(const torch::Tensor& all_num_routed, int rank, int num_max_
     return {send_counts, recv_counts, totals, remote, records, num_recv_tokens, tokens_per_expert};
 }
 
+// ---------------------------------------------------------------------------
+// The calls of ll_runtime.AllToAllState.  A call is given the state's attribute dictionary and takes the tensors
+// out of it by interned name, so whatever the attributes hold at that moment is what the kernels get; through
+// ctypes the argument lists cost the host 5 us a call on top of the launch, and the ten results of the metadata
+// call 14 us more.
+// ---------------------------------------------------------------------------
+struct Attributes {
+    PyObject* dict;
+
+    explicit Attributes(const pybind11::dict& d) : dict(d.ptr()) {}
+    PyObject* get(PyObject* key) const {
+        PyObject* v = PyDict_GetItemWithError(dict, key);  // borrowed
+        if (v == nullptr) {
+            if (!PyErr_Occurred()) PyErr_SetObject(PyExc_AttributeError, key);
+            throw pybind11::error_already_set();
+        }
+        return v;
+    }
+    const torch::Tensor* tensor(PyObject* key) const {
+        PyObject* v = get(key);
+        if (v == Py_None) return nullptr;
+        if (!THPVariable_Check(v)) throw pybind11::type_error("a tensor or None was expected");
+        return &THPVariable_Unpack(v);
+    }
+    template <typename T = void>
+    T* ptr(PyObject* key) const {
+        const torch::Tensor* t = tensor(key);
+        return t != nullptr ? static_cast<T*>(t->data_ptr()) : nullptr;
+    }
+    int64_t size_bytes(PyObject* key) const {
+        const torch::Tensor* t = tensor(key);
+        return t != nullptr ? int64_t(t->nbytes()) : 0;
+    }
+    int64_t integer(PyObject* key) const {
+        const int64_t v = PyLong_AsLongLong(get(key));
+        if (v == -1 and PyErr_Occurred()) throw pybind11::error_already_set();
+        return v;
+    }
+};
+
+// An attribute name as the interned string Python's own lookups use; made once, when the module is loaded.
+#define DEEPEP_NAME(x) static PyObject* const x = PyUnicode_InternFromString(#x)
+
+template <typename T = void>
+static T* optional_ptr(const std::optional<torch::Tensor>& t) {
+    return t.has_value() ? static_cast<T*>(t->data_ptr()) : nullptr;
+}
+
+// A failed call raises what the ctypes view of the library raises.
+static void capi_check(int rc) {
+    if (rc == 0) return;
+    const pybind11::object kind = pybind11::module_::import("deepep_efa_amd._capi").attr("DeepEPError");
+    PyErr_SetString(kind.ptr(), deepep_last_error());
+    throw pybind11::error_already_set();
+}
+
+struct ExchangeMetadata {
+    torch::Tensor send_counts, recv_counts, totals, combine_remote_recv_offset, source_rank, source_offset,
+        padded_index, combine_send_offset, num_recv_tokens, tokens_per_expert;
+};
+
+static ExchangeMetadata exchange_metadata_of(const torch::Tensor& all_num_routed, int rank, int max_tokens,
+                                             int64_t row_capacity) {
+    const int num_ranks = static_cast<int>(all_num_routed.size(0)), num_experts = static_cast<int>(all_num_routed.size(1));
+    const int64_t r = num_ranks, cap = std::max<int64_t>(row_capacity, 0), el = num_experts / std::max(num_ranks, 1);
+    ResultBlock b;
+    const int64_t send_at = b.reserve(4 * r), recv_at = b.reserve(4 * r), totals_at = b.reserve(12);
+    const int64_t remote_at = b.reserve(8 * r), num_at = b.reserve(8), per_expert_at = b.reserve(4 * el);
+    int64_t record_at[4];
+    for (auto& at : record_at) at = b.reserve(4 * cap);
+    b.allocate(all_num_routed.device());
+    const auto i32 = torch::kInt32;
+    ExchangeMetadata m{b.take(send_at, {r}, i32),          b.take(recv_at, {r}, i32),
+                       b.take(totals_at, {3}, i32),        b.take(remote_at, {r}, torch::kInt64),
+                       b.take(record_at[0], {cap}, i32),   b.take(record_at[1], {cap}, i32),
+                       b.take(record_at[2], {cap}, i32),   b.take(record_at[3], {cap}, i32),
+                       b.take(num_at, {2}, i32),           b.take(per_expert_at, {el}, i32)};
+    auto u32 = [](const torch::Tensor& t) { return static_cast<uint32_t*>(t.data_ptr()); };
+    capi_check(deepep_ll_exchange_metadata(
+        static_cast<const int32_t*>(all_num_routed.data_ptr()), num_experts, num_ranks, rank, max_tokens, row_capacity,
+        static_cast<int32_t*>(m.send_counts.data_ptr()), static_cast<int32_t*>(m.recv_counts.data_ptr()),
+        static_cast<int32_t*>(m.totals.data_ptr()), static_cast<int64_t*>(m.combine_remote_recv_offset.data_ptr()),
+        u32(m.source_rank), u32(m.source_offset), u32(m.padded_index), u32(m.combine_send_offset),
+        u32(m.num_recv_tokens), u32(m.tokens_per_expert), current_stream()));
+    return m;
+}
+
+namespace name {
+DEEPEP_NAME(send_counts);
+DEEPEP_NAME(recv_counts);
+DEEPEP_NAME(totals);
+DEEPEP_NAME(combine_remote_recv_offset);
+DEEPEP_NAME(source_rank);
+DEEPEP_NAME(source_offset);
+DEEPEP_NAME(padded_index);
+DEEPEP_NAME(combine_send_offset);
+DEEPEP_NAME(num_recv_tokens);
+DEEPEP_NAME(tokens_per_expert);
+DEEPEP_NAME(send_rows);
+DEEPEP_NAME(send_capacity);
+DEEPEP_NAME(send_count);
+DEEPEP_NAME(send_expert_prefix);
+DEEPEP_NAME(send_cumsum);
+DEEPEP_NAME(pair_slot);
+DEEPEP_NAME(workspace);
+DEEPEP_NAME(slot_rows);
+DEEPEP_NAME(row_capacity);
+DEEPEP_NAME(recv_by_source);
+DEEPEP_NAME(by_source_workspace);
+DEEPEP_NAME(record_packed_row);
+DEEPEP_NAME(packed_recv_x);
+DEEPEP_NAME(packed_recv_scales);
+DEEPEP_NAME(packed_recv_count);
+DEEPEP_NAME(packed_recv_src_info);
+DEEPEP_NAME(packed_recv_layout_range);
+DEEPEP_NAME(send_flat);
+DEEPEP_NAME(recv_flat);
+DEEPEP_NAME(expected_rows);
+}  // namespace name
+
+static pybind11::dict exchange_metadata_dict(const torch::Tensor& all_num_routed, int rank, int max_tokens,
+                                             int64_t capacity) {
+    using namespace name;
+    const ExchangeMetadata m = exchange_metadata_of(all_num_routed, rank, max_tokens, capacity);
+    pybind11::dict out;
+    auto put = [&](PyObject* key, const torch::Tensor& t) {
+        PyObject* v = THPVariable_Wrap(t);
+        const bool ok = v != nullptr and PyDict_SetItem(out.ptr(), key, v) == 0;
+        Py_XDECREF(v);
+        if (!ok) throw pybind11::error_already_set();
+    };
+    put(send_counts, m.send_counts), put(recv_counts, m.recv_counts), put(totals, m.totals);
+    put(combine_remote_recv_offset, m.combine_remote_recv_offset);
+    put(source_rank, m.source_rank), put(source_offset, m.source_offset), put(padded_index, m.padded_index);
+    put(combine_send_offset, m.combine_send_offset), put(num_recv_tokens, m.num_recv_tokens);
+    put(tokens_per_expert, m.tokens_per_expert);
+    return out;
+}
+
+struct AllToAllCalls {
+    int num_ranks, rank, num_experts, max_tokens, hidden, num_topk, fmt;
+
+    void dispatch_send(const pybind11::dict& state, const torch::Tensor& x, const torch::Tensor& topk_idx) const {
+        using namespace name;
+        const Attributes s(state);
+        capi_check(deepep_ll_dispatch_send_by_dest(
+            x.data_ptr(), static_cast<const int64_t*>(topk_idx.data_ptr()), static_cast<int>(x.size(0)), hidden,
+            num_topk, num_experts, num_ranks, rank, max_tokens, fmt, s.ptr(send_rows), s.integer(send_capacity),
+            s.ptr<int32_t>(send_count), s.ptr<int32_t>(send_expert_prefix), s.ptr<int32_t>(send_counts),
+            s.ptr<int64_t>(send_cumsum), s.ptr<int32_t>(pair_slot), s.ptr(workspace), size_t(s.size_bytes(workspace)),
+            current_stream()));
+    }
+
+    void dispatch_recv_ordered(const pybind11::dict& state, const torch::Tensor& all_num_routed,
+                               const std::optional<torch::Tensor>& stats) const {
+        using namespace name;
+        const Attributes s(state);
+        capi_check(deepep_ll_dispatch_recv_by_source_ordered(
+            s.ptr(recv_by_source), s.integer(slot_rows), static_cast<const int32_t*>(all_num_routed.data_ptr()), hidden,
+            num_experts, num_ranks, rank, max_tokens, fmt, s.ptr(packed_recv_x), s.ptr(packed_recv_scales),
+            s.ptr<int32_t>(packed_recv_src_info), s.ptr<int64_t>(packed_recv_layout_range),
+            s.ptr<int32_t>(packed_recv_count), optional_ptr<int32_t>(stats), s.ptr<uint32_t>(tokens_per_expert),
+            s.ptr<int32_t>(record_packed_row), s.integer(row_capacity), s.integer(expected_rows),
+            s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream()));
+    }
+
+    void dispatch_recv(const pybind11::dict& state, const pybind11::dict& meta,
+                       const std::optional<torch::Tensor>& stats) const {
+        using namespace name;
+        const Attributes s(state), m(meta);
+        capi_check(deepep_ll_dispatch_recv_by_source(
+            s.ptr(recv_by_source), s.integer(slot_rows), m.ptr<int32_t>(recv_counts), m.ptr<uint32_t>(source_offset),
+            m.ptr<uint32_t>(num_recv_tokens), s.integer(row_capacity), hidden, num_experts, num_ranks, max_tokens, fmt,
+            s.ptr(packed_recv_x), s.ptr(packed_recv_scales), s.ptr<int32_t>(packed_recv_src_info),
+            s.ptr<int64_t>(packed_recv_layout_range), s.ptr<int32_t>(packed_recv_count), optional_ptr<int32_t>(stats),
+            s.ptr<uint32_t>(tokens_per_expert), s.ptr<int32_t>(record_packed_row), s.integer(expected_rows),
+            s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream()));
+    }
+
+    void combine_send(const pybind11::dict& state, const pybind11::dict& meta, const torch::Tensor& y,
+                      const std::optional<torch::Tensor>& peer_recv_flat,
+                      const std::optional<torch::Tensor>& peer_recv_rows) const {
+        using namespace name;
+        const Attributes s(state), m(meta);
+        capi_check(deepep_ll_combine_send_by_dest(
+            y.data_ptr(), s.ptr<int32_t>(record_packed_row), m.ptr<uint32_t>(source_rank),
+            m.ptr<uint32_t>(padded_index), m.ptr<uint32_t>(combine_send_offset), m.ptr<uint32_t>(num_recv_tokens),
+            s.integer(row_capacity), hidden, num_experts, num_ranks, max_tokens, s.ptr(send_flat),
+            m.ptr<int32_t>(recv_counts), m.ptr<int64_t>(combine_remote_recv_offset),
+            optional_ptr<void*>(peer_recv_flat), optional_ptr<int64_t>(peer_recv_rows), s.integer(expected_rows),
+            current_stream()));
+    }
+
+    void combine_recv(const pybind11::dict& state, const torch::Tensor& topk_idx, const torch::Tensor& topk_weights,
+                      const torch::Tensor& out, const std::optional<torch::Tensor>& recv, int64_t recv_slot_rows,
+                      bool accumulate) const {
+        using namespace name;
+        const Attributes s(state);
+        const torch::Tensor* buf = recv.has_value() ? &recv.value() : s.tensor(recv_flat);
+        capi_check(deepep_ll_combine_recv_flat(
+            buf->data_ptr(), buf->size(0), recv_slot_rows, s.ptr<int32_t>(send_expert_prefix),
+            static_cast<const int64_t*>(topk_idx.data_ptr()), static_cast<const float*>(topk_weights.data_ptr()),
+            s.ptr<int32_t>(pair_slot), static_cast<int>(topk_idx.size(0)), hidden, num_topk, num_experts, num_ranks,
+            max_tokens, accumulate ? 1 : 0, out.data_ptr(), current_stream()));
+    }
+};
+
 // reference: deep_ep/buffer.py:1542-1557 — zero_() + index_add_ over the returned rows, then the biases
 static std::tuple<torch::Tensor, std::optional<torch::Tensor>> combine_reduce(
     const torch::Tensor& recv_x, const std::optional<torch::Tensor>& recv_topk_weights,
@@ -970,6 +1201,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("loopback_own_inputs", &deep_ep::Buffer::loopback_own_inputs)
         .def("loopback_world", &deep_ep::Buffer::loopback_world)
         .def("loopback_set_combine_mode", &deep_ep::Buffer::loopback_set_combine_mode);
+
+    pybind11::class_<deep_ep::AllToAllCalls>(m, "AllToAllCalls")
+        .def(pybind11::init([](int num_ranks, int rank, int num_experts, int max_tokens, int hidden, int num_topk,
+                               int fmt) {
+            return deep_ep::AllToAllCalls{num_ranks, rank, num_experts, max_tokens, hidden, num_topk, fmt};
+        }))
+        .def("dispatch_send", &deep_ep::AllToAllCalls::dispatch_send)
+        .def("dispatch_recv_ordered", &deep_ep::AllToAllCalls::dispatch_recv_ordered)
+        .def("dispatch_recv", &deep_ep::AllToAllCalls::dispatch_recv)
+        .def("combine_send", &deep_ep::AllToAllCalls::combine_send)
+        .def("combine_recv", &deep_ep::AllToAllCalls::combine_recv);
+    m.def("exchange_metadata_dict", &deep_ep::exchange_metadata_dict,
+          "Send/receive counts, combine offsets and per-row records by name");
 
     m.def("is_sm90_compiled", deep_ep::is_sm90_compiled);
     m.attr("topk_idx_t") = py::reinterpret_borrow<py::object>(

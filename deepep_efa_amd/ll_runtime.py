@@ -11,7 +11,7 @@ from dataclasses import dataclass
 
 import torch
 
-from . import _capi
+from . import _capi, deep_ep_cpp
 
 ROW_BF16, ROW_FP8, ROW_FP8_POW2, ROW_FP8_UE8M0 = 0, 1, 2, 3
 
@@ -166,22 +166,7 @@ class LowLatencyState:
 def exchange_metadata(all_num_routed: torch.Tensor, rank: int, max_tokens: int, row_capacity: int) -> dict:
     """Send / receive counts, combine offsets and one record per expected row from the gathered
     per-expert route counts [R, E] int32 (csrc/transport/ll_pipeline.cpp:1204-1361), on the current stream."""
-    lib = _capi.load()
-    r, e = all_num_routed.shape
-    dev = all_num_routed.device
-    i32 = dict(dtype=torch.int32, device=dev)
-    out = dict(send_counts=torch.empty(r, **i32), recv_counts=torch.empty(r, **i32), totals=torch.empty(3, **i32),
-               combine_remote_recv_offset=torch.empty(r, dtype=torch.int64, device=dev),
-               source_rank=torch.empty(row_capacity, **i32), source_offset=torch.empty(row_capacity, **i32),
-               padded_index=torch.empty(row_capacity, **i32), combine_send_offset=torch.empty(row_capacity, **i32),
-               num_recv_tokens=torch.empty(2, **i32), tokens_per_expert=torch.empty(e // r, **i32))
-    _capi.check(lib.deepep_ll_exchange_metadata(
-        _capi.ptr(all_num_routed), e, r, rank, max_tokens, row_capacity, _capi.ptr(out["send_counts"]),
-        _capi.ptr(out["recv_counts"]), _capi.ptr(out["totals"]), _capi.ptr(out["combine_remote_recv_offset"]),
-        _capi.ptr(out["source_rank"]), _capi.ptr(out["source_offset"]), _capi.ptr(out["padded_index"]),
-        _capi.ptr(out["combine_send_offset"]), _capi.ptr(out["num_recv_tokens"]), _capi.ptr(out["tokens_per_expert"]),
-        current_stream_ptr()))
-    return out
+    return deep_ep_cpp.exchange_metadata_dict(all_num_routed, rank, max_tokens, row_capacity)
 
 
 class AllToAllState:
@@ -198,6 +183,7 @@ class AllToAllState:
         self.lib = lib
         self.shape = s = shape
         el, r, m, e, h, k = s.num_local_experts, s.num_ranks, s.max_tokens, s.num_experts, s.hidden, s.num_topk
+        self.calls = deep_ep_cpp.AllToAllCalls(r, s.rank, e, m, h, k, s.fmt)
         self.stride = lib.deepep_ll_row_stride(h, s.fmt)
         u8 = dict(dtype=torch.uint8, device=device)
         i32 = dict(dtype=torch.int32, device=device)
@@ -236,12 +222,7 @@ class AllToAllState:
         self.expected_rows = m * k  # what a balanced world delivers; sizes grids, never the result
 
     def dispatch_send(self, x: torch.Tensor, topk_idx: torch.Tensor) -> None:
-        s = self.shape
-        _capi.check(self.lib.deepep_ll_dispatch_send_by_dest(
-            _capi.ptr(x), _capi.ptr(topk_idx), x.shape[0], s.hidden, s.num_topk, s.num_experts, s.num_ranks, s.rank,
-            s.max_tokens, s.fmt, _capi.ptr(self.send_rows), self.send_capacity, _capi.ptr(self.send_count),
-            _capi.ptr(self.send_expert_prefix), _capi.ptr(self.send_counts), _capi.ptr(self.send_cumsum),
-            _capi.ptr(self.pair_slot), _capi.ptr(self.workspace), self.workspace.numel(), current_stream_ptr()))
+        self.calls.dispatch_send(self.__dict__, x, topk_idx)
 
     def exchange_metadata(self, all_num_routed: torch.Tensor) -> dict:
         """all_num_routed [R, E] int32: the ranks' send_count, as an all-gather leaves them everywhere."""
@@ -251,44 +232,17 @@ class AllToAllState:
     def dispatch_recv_ordered(self, all_num_routed: torch.Tensor, stats: torch.Tensor = None) -> None:
         """The receive for messages in this build's own order (what dispatch_send emits): places every row by
         arithmetic on the gathered counts, without the record list and without reading the rows' tails."""
-        s = self.shape
-        _capi.check(self.lib.deepep_ll_dispatch_recv_by_source_ordered(
-            _capi.ptr(self.recv_by_source), self.slot_rows, _capi.ptr(all_num_routed), s.hidden, s.num_experts,
-            s.num_ranks, s.rank, s.max_tokens, s.fmt, _capi.ptr(self.packed_recv_x),
-            _capi.ptr(self.packed_recv_scales), _capi.ptr(self.packed_recv_src_info),
-            _capi.ptr(self.packed_recv_layout_range), _capi.ptr(self.packed_recv_count), _capi.ptr(stats),
-            _capi.ptr(self.tokens_per_expert), _capi.ptr(self.record_packed_row), self.row_capacity,
-            self.expected_rows, _capi.ptr(self.by_source_workspace), self.by_source_workspace.numel(),
-            current_stream_ptr()))
+        self.calls.dispatch_recv_ordered(self.__dict__, all_num_routed, stats)
 
     def dispatch_recv(self, stats: torch.Tensor = None) -> None:
-        s, m = self.shape, self.meta
-        _capi.check(self.lib.deepep_ll_dispatch_recv_by_source(
-            _capi.ptr(self.recv_by_source), self.slot_rows, _capi.ptr(m["recv_counts"]), _capi.ptr(m["source_offset"]),
-            _capi.ptr(m["num_recv_tokens"]), self.row_capacity, s.hidden, s.num_experts, s.num_ranks, s.max_tokens,
-            s.fmt, _capi.ptr(self.packed_recv_x), _capi.ptr(self.packed_recv_scales),
-            _capi.ptr(self.packed_recv_src_info), _capi.ptr(self.packed_recv_layout_range),
-            _capi.ptr(self.packed_recv_count), _capi.ptr(stats), _capi.ptr(self.tokens_per_expert),
-            _capi.ptr(self.record_packed_row), self.expected_rows, _capi.ptr(self.by_source_workspace),
-            self.by_source_workspace.numel(), current_stream_ptr()))
+        self.calls.dispatch_recv(self.__dict__, self.meta, stats)
 
     def combine_send(self, y: torch.Tensor, peer_recv_flat: torch.Tensor = None,
                      peer_recv_rows: torch.Tensor = None) -> None:
         """Rows owed to the other ranks into send_flat, or, with a table of the ranks' recv_flat addresses
         (int64 [R]) and their row counts, straight to their place in those buffers."""
-        s, m = self.shape, self.meta
-        _capi.check(self.lib.deepep_ll_combine_send_by_dest(
-            _capi.ptr(y), _capi.ptr(self.record_packed_row), _capi.ptr(m["source_rank"]), _capi.ptr(m["padded_index"]),
-            _capi.ptr(m["combine_send_offset"]), _capi.ptr(m["num_recv_tokens"]), self.row_capacity, s.hidden,
-            s.num_experts, s.num_ranks, s.max_tokens, _capi.ptr(self.send_flat), _capi.ptr(m["recv_counts"]),
-            _capi.ptr(m["combine_remote_recv_offset"]), _capi.ptr(peer_recv_flat), _capi.ptr(peer_recv_rows),
-            self.expected_rows, current_stream_ptr()))
+        self.calls.combine_send(self.__dict__, self.meta, y, peer_recv_flat, peer_recv_rows)
 
     def combine_recv(self, topk_idx: torch.Tensor, topk_weights: torch.Tensor, out: torch.Tensor,
                      recv: torch.Tensor = None, slot_rows: int = 0, accumulate: bool = False) -> None:
-        s = self.shape
-        buf = self.recv_flat if recv is None else recv
-        _capi.check(self.lib.deepep_ll_combine_recv_flat(
-            _capi.ptr(buf), buf.shape[0], slot_rows, _capi.ptr(self.send_expert_prefix), _capi.ptr(topk_idx),
-            _capi.ptr(topk_weights), _capi.ptr(self.pair_slot), topk_idx.shape[0], s.hidden, s.num_topk,
-            s.num_experts, s.num_ranks, s.max_tokens, int(accumulate), _capi.ptr(out), current_stream_ptr()))
+        self.calls.combine_recv(self.__dict__, topk_idx, topk_weights, out, recv, slot_rows, accumulate)
