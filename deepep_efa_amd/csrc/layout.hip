@@ -9,6 +9,9 @@ namespace deepep {
 
 constexpr int kLayoutThreads = 256;
 constexpr int kMaxRankWords = 4;  // membership bitmask: up to 256 ranks
+// Up to here one workgroup of 1024 threads counts everything and no second launch adds up partial rows.
+constexpr int kLayoutOneBlockTokens = 2048;
+constexpr int kLayoutOneBlockThreads = 1024;
 
 // Spreads the 8 bits of b into 8 bytes (byte i = bit i, value 0 or 1).
 __device__ __forceinline__ uint64_t bits_to_bool_bytes(uint32_t b) {
@@ -26,58 +29,79 @@ __device__ __forceinline__ uint64_t bits_to_bool_bytes(uint32_t b) {
 //   * is_token_in_rank: the bitmask expanded to bool bytes, 8 per store.
 // Each workgroup writes a partial row [E | R | R/8]; with one workgroup the
 // partial row is the result, otherwise a second small kernel adds the rows.
+// What bounds it is latency and launches, not the few hundred KB it reads: hence
+// one workgroup while its two tokens a thread cost less than the second launch,
+// and a bitmask of as many words as there are ranks for (an index into a longer
+// one that the compiler cannot resolve goes through selects).
 // Reference: csrc/kernels/layout.cu:9-121 (which re-reads topk_idx once per
 // 4 experts / 8 ranks).
 // ---------------------------------------------------------------------
-__global__ __launch_bounds__(kLayoutThreads) void layout_count_kernel(
+template <int kRankWords>
+__global__ __launch_bounds__(kLayoutOneBlockThreads) void layout_count_kernel(
     const int64_t* __restrict__ topk_idx, int num_tokens, int num_topk, int num_ranks, int num_experts,
     uint32_t rank_magic, int num_nodes, uint8_t* __restrict__ is_token_in_rank, int32_t* __restrict__ partial,
     int32_t* __restrict__ per_rank, int32_t* __restrict__ per_node, int32_t* __restrict__ per_expert) {
     extern __shared__ int32_t hist[];  // [E + R + nodes]
-    const int tid = threadIdx.x, lane = lane_id();
+    const int tid = threadIdx.x, lane = lane_id(), threads = blockDim.x;
     const int width = num_experts + num_ranks + num_nodes;
-    for (int j = tid; j < width; j += kLayoutThreads) hist[j] = 0;
-    __syncthreads();
+    for (int j = tid; j < width; j += threads) hist[j] = 0;
+    lds_barrier();
 
-    const int t = blockIdx.x * kLayoutThreads + tid;
-    uint64_t member[kMaxRankWords] = {0, 0, 0, 0};
-    if (t < num_tokens) {
-        const int64_t* row = topk_idx + int64_t(t) * num_topk;
-        for (int k0 = 0; k0 < num_topk; k0 += 8) {
-            int64_t e[8];  // the eight loads of a round in flight before the first is used
+    // whole waves go round together: the ballots below want every lane
+    for (int t0 = blockIdx.x * threads; t0 < num_tokens; t0 += int(gridDim.x) * threads) {
+        const int t = t0 + tid;
+        uint64_t member[kRankWords];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) e[u] = k0 + u < num_topk ? row[k0 + u] : -1;
+        for (int q = 0; q < kRankWords; ++q) member[q] = 0;
+        if (t < num_tokens) {
+            const int64_t* row = topk_idx + int64_t(t) * num_topk;
+            for (int k0 = 0; k0 < num_topk; k0 += 8) {
+                int64_t e[8];  // the eight loads of a round in flight before the first is used
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (e[u] < 0 || e[u] >= num_experts) continue;
-                atomicAdd(&hist[int(e[u])], 1);
-                // e / E_l by multiply-high (exact below 2^16 experts); magic 0 stands for E_l == 1
-                const int r = rank_magic != 0 ? int(__umulhi(uint32_t(e[u]), rank_magic)) : int(e[u]);
+                for (int u = 0; u < 8; ++u) e[u] = k0 + u < num_topk ? row[k0 + u] : -1;
 #pragma unroll
-                for (int q = 0; q < kMaxRankWords; ++q)
-                    if ((r >> 6) == q) member[q] |= uint64_t(1) << (r & 63);
+                for (int u = 0; u < 8; ++u) {
+                    if (e[u] < 0 || e[u] >= num_experts) continue;
+                    atomicAdd(&hist[int(e[u])], 1);
+                    // e / E_l by multiply-high (exact below 2^16 experts); magic 0 stands for E_l == 1
+                    const int r = rank_magic != 0 ? int(__umulhi(uint32_t(e[u]), rank_magic)) : int(e[u]);
+#pragma unroll
+                    for (int q = 0; q < kRankWords; ++q)
+                        if (kRankWords == 1 || (r >> 6) == q) member[q] |= uint64_t(1) << (r & 63);
+                }
+            }
+            uint8_t* out = is_token_in_rank + int64_t(t) * num_ranks;
+#pragma unroll
+            for (int q = 0; q < kRankWords; ++q) {
+                const int begin = q * kWave, end = num_ranks < begin + kWave ? num_ranks : begin + kWave;
+                if ((num_ranks & 7) == 0) {
+                    for (int r8 = begin; r8 < end; r8 += 8)
+                        *reinterpret_cast<uint64_t*>(out + r8) = bits_to_bool_bytes(uint32_t(member[q] >> (r8 - begin)));
+                } else {
+                    for (int r = begin; r < end; ++r) out[r] = uint8_t((member[q] >> (r - begin)) & 1);
+                }
             }
         }
-        uint8_t* out = is_token_in_rank + int64_t(t) * num_ranks;
-        if ((num_ranks & 7) == 0) {
-            for (int r8 = 0; r8 < num_ranks; r8 += 8)
-                *reinterpret_cast<uint64_t*>(out + r8) = bits_to_bool_bytes(uint32_t(member[r8 >> 6] >> (r8 & 63)));
-        } else {
-            for (int r = 0; r < num_ranks; ++r) out[r] = uint8_t((member[r >> 6] >> (r & 63)) & 1);
+        // lane r keeps rank (q * 64 + r)'s count of the wave, so that one atomic per lane adds them all
+#pragma unroll
+        for (int q = 0; q < kRankWords; ++q) {
+            const int begin = q * kWave, n = num_ranks - begin < kWave ? num_ranks - begin : kWave;
+            int count = 0;
+            for (int r = 0; r < n; ++r) {
+                const int votes = __popcll(__ballot((member[q] >> r) & 1));
+                if (lane == r) count = votes;
+            }
+            if (count != 0) atomicAdd(&hist[num_experts + begin + lane], count);
+            // 8 ranks per node (reference: NUM_MAX_NVL_PEERS, csrc/kernels/configs.cuh:3)
+            for (int nd = 0; nd < 8 && q * 8 + nd < num_nodes; ++nd) {
+                const int votes = __popcll(__ballot((member[q] >> (nd * 8)) & 0xffull));
+                if (lane == 0 && votes != 0) atomicAdd(&hist[num_experts + num_ranks + q * 8 + nd], votes);
+            }
         }
     }
-    for (int r = 0; r < num_ranks; ++r) {
-        const uint64_t votes = __ballot((member[r >> 6] >> (r & 63)) & 1);
-        if (lane == 0 && votes != 0) atomicAdd(&hist[num_experts + r], __popcll(votes));
-    }
-    for (int nd = 0; nd < num_nodes; ++nd) {
-        const int r0 = nd * 8;  // 8 ranks per node (reference: NUM_MAX_NVL_PEERS, csrc/kernels/configs.cuh:3)
-        const uint64_t votes = __ballot((member[r0 >> 6] >> (r0 & 63)) & 0xffull);
-        if (lane == 0 && votes != 0) atomicAdd(&hist[num_experts + num_ranks + nd], __popcll(votes));
-    }
-    __syncthreads();
+    lds_barrier();
     if (gridDim.x == 1) {  // the partial row is the result
-        for (int j = tid; j < width; j += kLayoutThreads) {
+        for (int j = tid; j < width; j += threads) {
             if (j < num_experts)
                 per_expert[j] = hist[j];
             else if (j < num_experts + num_ranks)
@@ -88,7 +112,7 @@ __global__ __launch_bounds__(kLayoutThreads) void layout_count_kernel(
         return;
     }
     int32_t* dst = partial + int64_t(blockIdx.x) * width;
-    for (int j = tid; j < width; j += kLayoutThreads) dst[j] = hist[j];
+    for (int j = tid; j < width; j += threads) dst[j] = hist[j];
 }
 
 __global__ __launch_bounds__(kLayoutThreads) void layout_reduce_kernel(const int32_t* __restrict__ partial,
@@ -114,6 +138,13 @@ __global__ __launch_bounds__(kLayoutThreads) void layout_reduce_kernel(const int
         per_rank[j - num_experts] = sum;
     else
         per_node[j - num_experts - num_ranks] = sum;
+}
+
+// The total of a routing sort into memory the host reads while the stream runs on (null: nobody asked).  One
+// 8-byte store at system scope: a host that polls it sees the whole value or the old one.
+__device__ __forceinline__ void tell_host_total(int64_t* total_host, int64_t total) {
+    if (total_host != nullptr)
+        __hip_atomic_store(total_host, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------------
@@ -174,7 +205,8 @@ __global__ __launch_bounds__(kSortChunk) void routing_sort_pass_kernel(
 
 __global__ __launch_bounds__(256) void routing_sort_scan_kernel(int32_t* __restrict__ chunk_table, int num_chunks,
                                                                 int num_ranks, int32_t* __restrict__ send_counts,
-                                                                int64_t* __restrict__ send_cumsum) {
+                                                                int64_t* __restrict__ send_cumsum,
+                                                                int64_t* __restrict__ total_host) {
     extern __shared__ int64_t rank_base[];  // [R + 1]
     const int tid = threadIdx.x;
     for (int r = tid; r < num_ranks; r += 256) {
@@ -187,6 +219,7 @@ __global__ __launch_bounds__(256) void routing_sort_scan_kernel(int32_t* __restr
     if (tid == 0) {
         rank_base[0] = 0;
         for (int r = 0; r < num_ranks; ++r) rank_base[r + 1] += rank_base[r];
+        tell_host_total(total_host, rank_base[num_ranks]);
     }
     __syncthreads();
     for (int r = tid; r <= num_ranks; r += 256) send_cumsum[r] = rank_base[r];
@@ -228,7 +261,7 @@ __device__ __forceinline__ uint64_t membership_mask(const uint8_t* row, int num_
 __global__ __launch_bounds__(kSortChunk) void routing_sort_single_kernel(
     const uint8_t* __restrict__ is_token_in_rank, int num_tokens, int num_ranks, int tokens_per_thread,
     int32_t* __restrict__ send_counts, int64_t* __restrict__ send_cumsum, int64_t* __restrict__ sorted_token_ids,
-    int32_t* __restrict__ row_of_pair) {
+    int32_t* __restrict__ row_of_pair, int64_t* __restrict__ total_host) {
     constexpr int kWaves = kSortChunk / kWave;
     __shared__ int32_t wave_own[kWaves];    // tokens of this rank in each wave
     __shared__ int32_t wave_lower[kWaves];  // memberships of lower ranks in each wave
@@ -272,7 +305,135 @@ __global__ __launch_bounds__(kSortChunk) void routing_sort_single_kernel(
     if (tid == 0) {
         send_counts[r] = total;
         send_cumsum[r] = base;
-        if (r == num_ranks - 1) send_cumsum[num_ranks] = int64_t(base) + total;
+        if (r == num_ranks - 1) {
+            send_cumsum[num_ranks] = int64_t(base) + total;
+            tell_host_total(total_host, int64_t(base) + total);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------
+// The same sort in one launch for 8, 16, 32 or 64 ranks and a matrix of up to 512 KB.  One workgroup per 256
+// tokens; each reads the whole matrix (from L2), 8 ranks of a token per 8-byte word, adding the bool bytes of a
+// word up eight at a time, once over all tokens and once over those before its own: the first gives where every
+// rank's ids begin, the second where its own tokens' ids do.  Against one workgroup per rank, a token's row of
+// row_of_pair is written in one piece, and the loads are independent of one another; against three launches
+// (count, scan, scatter) it is one.  The total goes to the host before any id is written.  What bounds it is
+// latency: about three memory round trips.
+// ---------------------------------------------------------------------
+constexpr int kWideSortTokens = 256;    // tokens per workgroup
+constexpr int kWideSortThreads = 1024;  // a byte counter of a thread takes at most 255 tokens: 255 * 1024 in all
+constexpr int64_t kWideSortMaxBytes = 512 * 1024;
+
+// 1 in every byte of v that is not zero.
+__device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {
+    v |= v >> 4, v |= v >> 2, v |= v >> 1;
+    return v & 0x0101010101010101ull;
+}
+
+template <int kWords>  // 8-byte words of a token's row: ranks / 8
+__global__ __launch_bounds__(kWideSortThreads) void routing_sort_wide_kernel(
+    const uint64_t* __restrict__ is_token_in_rank, int num_tokens, int32_t* __restrict__ send_counts,
+    int64_t* __restrict__ send_cumsum, int64_t* __restrict__ sorted_token_ids, int32_t* __restrict__ row_of_pair,
+    int64_t* __restrict__ total_host) {
+    constexpr int kRanks = kWords * 8, kWaves = kWideSortThreads / kWave, kAhead = kWords <= 2 ? 4 : 2;
+    constexpr int kTokenWaves = kWideSortTokens / kWave, kRankShares = kWaves / kTokenWaves;
+    __shared__ int32_t wave_all[kWaves][kRanks], wave_before[kWaves][kRanks];
+    __shared__ int32_t start[kRanks];                // where the ids of this workgroup's tokens begin, per rank
+    __shared__ int32_t chunk_cnt[kTokenWaves][kRanks];
+    const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block();
+    const int begin = blockIdx.x * kWideSortTokens;
+    // this thread's own token, loaded with the rest: wave w has tokens (w % 4) * 64 + lane
+    const int tw = w & (kTokenWaves - 1), share = w / kTokenWaves;
+    const int own = begin + tw * kWave + lane;
+    uint64_t own_row[kWords];
+#pragma unroll
+    for (int q = 0; q < kWords; ++q) {
+        own_row[q] = num_tokens > 0 ? is_token_in_rank[int64_t(own < num_tokens ? own : num_tokens - 1) * kWords + q] : 0;
+        if (own >= num_tokens) own_row[q] = 0;
+    }
+    uint64_t all[kWords], before[kWords];
+#pragma unroll
+    for (int q = 0; q < kWords; ++q) all[q] = before[q] = 0;
+    for (int t0 = tid; t0 < num_tokens; t0 += kAhead * kWideSortThreads) {
+        uint64_t v[kAhead][kWords];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {  // unconditional loads, all in flight together
+            const int t = t0 + u * kWideSortThreads;
+#pragma unroll
+            for (int q = 0; q < kWords; ++q)
+                v[u][q] = is_token_in_rank[int64_t(t < num_tokens ? t : num_tokens - 1) * kWords + q];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int t = t0 + u * kWideSortThreads;
+#pragma unroll
+            for (int q = 0; q < kWords; ++q) {
+                const uint64_t one = t < num_tokens ? nonzero_bytes(v[u][q]) : 0;
+                all[q] += one;
+                before[q] += t < begin ? one : 0;
+            }
+        }
+    }
+    // the wave's sums: bytes widened to 16 bits (64 lanes of at most 255 fit), four ranks in two words
+#pragma unroll
+    for (int q = 0; q < kWords; ++q)
+#pragma unroll
+        for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd) {
+                const int a = int((uint32_t(all[q] >> (32 * half)) >> (8 * odd)) & 0x00ff00ffu);
+                const int b = int((uint32_t(before[q] >> (32 * half)) >> (8 * odd)) & 0x00ff00ffu);
+                const uint32_t sa = uint32_t(wave_inclusive_sum(a)), sb = uint32_t(wave_inclusive_sum(b));
+                if (lane == kWave - 1) {
+                    const int r = q * 8 + half * 4 + odd;
+                    wave_all[w][r] = int(sa & 0xffffu), wave_all[w][r + 2] = int(sa >> 16);
+                    wave_before[w][r] = int(sb & 0xffffu), wave_before[w][r + 2] = int(sb >> 16);
+                }
+            }
+    // this workgroup's own tokens per rank and wave
+    int mine = 0;
+#pragma unroll
+    for (int q = 0; q < kWords; ++q)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int votes = __popcll(__ballot(((own_row[q] >> (8 * i)) & 0xff) != 0));
+            if (lane == q * 8 + i) mine = votes;
+        }
+    if (share == 0 && lane < kRanks) chunk_cnt[tw][lane] = mine;
+    lds_barrier();
+    if (w == 0) {
+        int total = 0, ahead = 0;
+        if (lane < kRanks)
+#pragma unroll
+            for (int w2 = 0; w2 < kWaves; ++w2) total += wave_all[w2][lane], ahead += wave_before[w2][lane];
+        const int incl = wave_inclusive_sum(total);
+        if (lane < kRanks) start[lane] = incl - total + ahead;
+        if (blockIdx.x == 0) {
+            if (lane == kRanks - 1) {
+                tell_host_total(total_host, incl);
+                send_cumsum[kRanks] = incl;
+            }
+            if (lane < kRanks) send_counts[lane] = total, send_cumsum[lane] = incl - total;
+        }
+    }
+    lds_barrier();
+    // wave (share, tw) writes its 64 tokens' places in its share of the ranks
+    constexpr int kPerShare = kRanks / kRankShares;
+#pragma unroll
+    for (int i = 0; i < kPerShare; ++i) {
+        const int r = share * kPerShare + i;
+        uint64_t word = 0;  // own_row[r / 8] with an index the compiler can resolve
+#pragma unroll
+        for (int q = 0; q < kWords; ++q)
+            if (q == (r >> 3)) word = own_row[q];
+        const bool in = ((word >> (8 * (r & 7))) & 0xff) != 0;
+        const uint64_t votes = __ballot(in);
+        int pos = start[r] + __popcll(votes & lanes_below(lane));
+#pragma unroll
+        for (int t2 = 0; t2 < kTokenWaves - 1; ++t2) pos += t2 < tw ? chunk_cnt[t2][r] : 0;
+        if (in) sorted_token_ids[pos] = own;
+        if (row_of_pair != nullptr && own < num_tokens) row_of_pair[int64_t(own) * kRanks + r] = in ? pos : -1;
     }
 }
 
@@ -310,6 +471,57 @@ __global__ __launch_bounds__(1024) void channel_prefix_kernel(const uint8_t* __r
         for (int ch = 0; ch < num_channels; ++ch) {
             run += per_channel[ch];
             cpm[int64_t(dst) * num_channels + ch] = run;
+        }
+    }
+}
+
+// The same for a multiple of 8 ranks: one workgroup per 8 of them, so a wave reads the membership of eight ranks
+// with one 8-byte load per token, sixteen of them in flight, and adds the bool bytes up eight at a time.  The
+// bytes of a row that eight workgroups used to fetch for themselves are fetched once (12289 tokens, 8 ranks,
+// 10 channels: 8.7 us, two thirds of it waiting for loads).
+constexpr int kChannelAhead = 16;
+
+__global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64_t* __restrict__ is_token_in_rank,
+                                                                    int num_tokens, int num_words, int num_channels,
+                                                                    int32_t* __restrict__ cpm) {
+    extern __shared__ int32_t per_channel[];  // [C][8]
+    const int q = blockIdx.x, lane = lane_id(), w = wave_in_block();
+    const int waves = int(blockDim.x) >> 6;
+    const int per = (num_tokens + num_channels - 1) / num_channels;
+    for (int ch = w; ch < num_channels; ch += waves) {
+        const int begin = min(per * ch, num_tokens), end = min(begin + per, num_tokens);
+        int count[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) count[i] = 0;
+        for (int t0 = begin + lane; t0 - lane < end; t0 += kWave * kChannelAhead) {
+            uint64_t v[kChannelAhead], sum = 0;
+#pragma unroll
+            for (int u = 0; u < kChannelAhead; ++u) {
+                const int t = t0 + u * kWave;
+                v[u] = is_token_in_rank[int64_t(t < end ? t : end - 1) * num_words + q];
+            }
+#pragma unroll
+            for (int u = 0; u < kChannelAhead; ++u) sum += t0 + u * kWave < end ? nonzero_bytes(v[u]) : 0;
+#pragma unroll
+            for (int half = 0; half < 2; ++half)  // bytes widened to 16 bits: 64 lanes of at most 16 fit
+#pragma unroll
+                for (int odd = 0; odd < 2; ++odd) {
+                    const int part = int((uint32_t(sum >> (32 * half)) >> (8 * odd)) & 0x00ff00ffu);
+                    const uint32_t all = uint32_t(__builtin_amdgcn_readlane(wave_inclusive_sum(part), kWave - 1));
+                    count[half * 4 + odd] += int(all & 0xffffu);
+                    count[half * 4 + odd + 2] += int(all >> 16);
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (lane == i) per_channel[ch * 8 + i] = count[i];
+    }
+    lds_barrier();
+    if (threadIdx.x < 8) {
+        int run = 0;
+        for (int ch = 0; ch < num_channels; ++ch) {
+            run += per_channel[ch * 8 + threadIdx.x];
+            cpm[int64_t(q * 8 + threadIdx.x) * num_channels + ch] = run;
         }
     }
 }
@@ -378,17 +590,23 @@ int deepep_get_dispatch_layout(const int64_t* topk_idx, int num_tokens, int num_
     const int num_nodes = num_tokens_per_rdma_rank != nullptr ? num_ranks / 8 : 0;
     const int width = num_experts + num_ranks + num_nodes;
     EP_HOST_ASSERT(size_t(width) * 4 <= 64 * 1024);
-    const int blocks = num_tokens == 0 ? 1 : (num_tokens + kLayoutThreads - 1) / kLayoutThreads;
-    EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(blocks) * width * 4);
+    const int partials = num_tokens == 0 ? 1 : (num_tokens + kLayoutThreads - 1) / kLayoutThreads;
+    EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(partials) * width * 4);
+    const int blocks = num_tokens <= kLayoutOneBlockTokens ? 1 : partials;
+    const int threads = blocks == 1 && num_tokens > kLayoutThreads ? kLayoutOneBlockThreads : kLayoutThreads;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     int32_t* partial = reinterpret_cast<int32_t*>(workspace);
     const uint32_t experts_per_rank = uint32_t(num_experts / num_ranks);
     EP_HOST_ASSERT(num_experts < 65536);
     const uint32_t rank_magic =
         experts_per_rank == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + experts_per_rank - 1) / experts_per_rank);
-    layout_count_kernel<<<blocks, kLayoutThreads, size_t(width) * 4, s>>>(
-        topk_idx, num_tokens, num_topk, num_ranks, num_experts, rank_magic, num_nodes, is_token_in_rank, partial,
-        num_tokens_per_rank, num_tokens_per_rdma_rank, num_tokens_per_expert);
+#define DEEPEP_LAUNCH_LAYOUT(WORDS)                                                                              \
+    layout_count_kernel<WORDS><<<blocks, threads, size_t(width) * 4, s>>>(                                        \
+        topk_idx, num_tokens, num_topk, num_ranks, num_experts, rank_magic, num_nodes, is_token_in_rank, partial, \
+        num_tokens_per_rank, num_tokens_per_rdma_rank, num_tokens_per_expert)
+    if (num_ranks <= kWave) DEEPEP_LAUNCH_LAYOUT(1);
+    else DEEPEP_LAUNCH_LAYOUT(kMaxRankWords);
+#undef DEEPEP_LAUNCH_LAYOUT
     EP_LAUNCH_CHECK();
     if (blocks == 1) return 0;
     layout_reduce_kernel<<<(width + kLayoutThreads - 1) / kLayoutThreads, kLayoutThreads, 0, s>>>(
@@ -403,21 +621,44 @@ size_t deepep_routing_sort_workspace_bytes(int num_tokens, int num_ranks) {
     return size_t((chunks < 1 ? 1 : chunks) * num_ranks * 4);
 }
 
-int deepep_moe_routing_sort(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
-                            int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
-                            int32_t* row_of_pair, void* workspace, size_t workspace_bytes, void* stream) {
+int deepep_moe_routing_sort_total(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
+                                  int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
+                                  int32_t* row_of_pair, int64_t* total_host, void* workspace, size_t workspace_bytes,
+                                  void* stream) {
     clear_error();
     EP_HOST_ASSERT(num_tokens >= 0 && num_ranks > 0 && num_ranks <= 1024);
     EP_HOST_ASSERT(send_counts != nullptr && send_cumsum != nullptr);
     EP_HOST_ASSERT(num_tokens == 0 || (is_token_in_rank != nullptr && sorted_token_ids != nullptr));
+    EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(total_host) & 7) == 0);
     const int chunks = num_tokens == 0 ? 1 : (num_tokens + kSortChunk - 1) / kSortChunk;
     EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(chunks) * num_ranks * 4);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    // Every workgroup of the wide form reads the whole matrix: 512 KB take one of them about 5 us, less than
+    // the two further launches of the chunked form; past that its work grows with the square of the batch.
+    const bool wide = (num_ranks == 8 || num_ranks == 16 || num_ranks == 32 || num_ranks == 64) &&
+                      (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 &&
+                      int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
+    if (wide) {
+        const int blocks = num_tokens == 0 ? 1 : (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
+        const uint64_t* rows = reinterpret_cast<const uint64_t*>(is_token_in_rank);
+#define DEEPEP_LAUNCH_SORT(WORDS)                                                                             \
+    routing_sort_wide_kernel<WORDS><<<blocks, kWideSortThreads, 0, s>>>(rows, num_tokens, send_counts, send_cumsum, \
+                                                                        sorted_token_ids, row_of_pair, total_host)
+        switch (num_ranks) {
+            case 8: DEEPEP_LAUNCH_SORT(1); break;
+            case 16: DEEPEP_LAUNCH_SORT(2); break;
+            case 32: DEEPEP_LAUNCH_SORT(4); break;
+            default: DEEPEP_LAUNCH_SORT(8); break;
+        }
+#undef DEEPEP_LAUNCH_SORT
+        EP_LAUNCH_CHECK();
+        return 0;
+    }
     if (num_tokens <= kSortChunk * kSingleSortTokensPerThread && num_ranks <= 64) {
         const int per_thread = num_tokens == 0 ? 1 : (num_tokens + kSortChunk - 1) / kSortChunk;
         routing_sort_single_kernel<<<num_ranks, kSortChunk, 0, s>>>(is_token_in_rank, num_tokens, num_ranks, per_thread,
                                                                    send_counts, send_cumsum, sorted_token_ids,
-                                                                   row_of_pair);
+                                                                   row_of_pair, total_host);
         EP_LAUNCH_CHECK();
         return 0;
     }
@@ -427,7 +668,7 @@ int deepep_moe_routing_sort(const uint8_t* is_token_in_rank, int num_tokens, int
                                                                     sorted_token_ids, nullptr);
     EP_LAUNCH_CHECK();
     routing_sort_scan_kernel<<<1, 256, size_t(num_ranks + 1) * 8, s>>>(table, chunks, num_ranks, send_counts,
-                                                                       send_cumsum);
+                                                                       send_cumsum, total_host);
     EP_LAUNCH_CHECK();
     if (num_tokens > 0) {
         routing_sort_pass_kernel<true><<<chunks, kSortChunk, lds, s>>>(is_token_in_rank, num_tokens, num_ranks,
@@ -435,6 +676,13 @@ int deepep_moe_routing_sort(const uint8_t* is_token_in_rank, int num_tokens, int
         EP_LAUNCH_CHECK();
     }
     return 0;
+}
+
+int deepep_moe_routing_sort(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
+                            int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
+                            int32_t* row_of_pair, void* workspace, size_t workspace_bytes, void* stream) {
+    return deepep_moe_routing_sort_total(is_token_in_rank, num_tokens, num_ranks, sorted_token_ids, send_counts,
+                                         send_cumsum, row_of_pair, nullptr, workspace, workspace_bytes, stream);
 }
 
 int deepep_channel_prefix_matrix(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks, int num_channels,
@@ -445,6 +693,14 @@ int deepep_channel_prefix_matrix(const uint8_t* is_token_in_rank, int num_tokens
     EP_HOST_ASSERT(num_tokens == 0 || is_token_in_rank != nullptr);
     // one wave per channel, up to sixteen at a time
     const int threads = num_channels >= 16 ? 1024 : ((num_channels + 3) / 4) * 256;
+    if ((num_ranks & 7) == 0 && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 && num_channels <= 1024) {
+        channel_prefix_words_kernel<<<num_ranks / 8, threads, size_t(num_channels) * 32,
+                                      reinterpret_cast<hipStream_t>(stream)>>>(
+            reinterpret_cast<const uint64_t*>(is_token_in_rank), num_tokens, num_ranks / 8, num_channels,
+            channel_prefix_matrix);
+        EP_LAUNCH_CHECK();
+        return 0;
+    }
     channel_prefix_kernel<<<num_ranks, threads, size_t(num_channels) * 4, reinterpret_cast<hipStream_t>(stream)>>>(
         is_token_in_rank, num_tokens, num_ranks, num_channels, channel_prefix_matrix);
     EP_LAUNCH_CHECK();

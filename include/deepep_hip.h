@@ -116,6 +116,14 @@ int deepep_moe_routing_sort(const uint8_t* is_token_in_rank, int num_tokens, int
                             int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
                             int32_t* row_of_pair, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same, with the total also stored to `total_host` (8 bytes the device can write and the host read, pinned
+ * memory; NULL: not wanted) as soon as the counts are known, ahead of the ids: a host that needs the total to
+ * size what comes next polls it instead of copying send_cumsum[R] back behind the whole sort. */
+int deepep_moe_routing_sort_total(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
+                                  int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
+                                  int32_t* row_of_pair, int64_t* total_host,
+                                  void* workspace, size_t workspace_bytes, void* stream);
+
 /* channel_prefix_matrix[d, c] = number of tokens bound for rank d in
  * channels 0..c, channel c owning tokens [min(c*ceil(T/C),T), min(+ceil(T/C),T)).
  *   is_token_in_rank       [T, R] bool bytes
