@@ -7,6 +7,7 @@
 // There is no device code in this file and no CPU fallback: a missing or
 // failing HIP library is an exception.
 #include <torch/extension.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -15,6 +16,8 @@
 #include <pybind11/functional.h>
 
 #include <algorithm>
+#include <chrono>
+#include <atomic>
 #include <functional>
 #include <memory>
 #include <optional>
@@ -62,6 +65,11 @@ static T align_up(T a, T b) {
     return (a + b - 1) / b * b;
 }
 
+// torch::empty without the dispatcher in front of the caching allocator, which is most of its 1.2 us.
+static torch::Tensor empty_on(const torch::Device& device, at::IntArrayRef sizes, torch::ScalarType type) {
+    return torch::Tensor(at::detail::empty_cuda(sizes, type, device, std::nullopt));
+}
+
 // Several results of one call in one allocation.  A torch::empty costs the host 1.2 us and a tensor over a piece
 // of storage that exists 0.1 us, so a call with many small results asks the allocator once.
 struct ResultBlock {
@@ -74,7 +82,7 @@ struct ResultBlock {
         return at;
     }
     void allocate(const torch::Device& device) {
-        block = torch::Tensor(at::detail::empty_cuda({std::max<int64_t>(bytes, 256)}, torch::kUInt8, device, std::nullopt));
+        block = empty_on(device, {std::max<int64_t>(bytes, 256)}, torch::kUInt8);
     }
     torch::Tensor take(int64_t at, at::IntArrayRef sizes, torch::ScalarType type) const {
         auto t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(block.storage()), block.key_set(),
@@ -355,12 +363,15 @@ struct Buffer {
             stream_wait(comm_stream, compute_stream);
 
         const int num_tokens = static_cast<int>(topk_idx.size(0)), num_topk = static_cast<int>(topk_idx.size(1));
-        auto i32 = torch::dtype(torch::kInt32).device(torch::kCUDA);
-        auto num_tokens_per_rank = torch::empty({num_ranks}, i32);
+        ResultBlock b;
+        const int64_t rank_at = b.reserve(4 * num_ranks), rdma_at = b.reserve(4 * num_rdma_ranks);
+        const int64_t expert_at = b.reserve(4 * num_experts), member_at = b.reserve(int64_t(num_tokens) * num_ranks);
+        b.allocate(torch::kCUDA);
+        auto num_tokens_per_rank = b.take(rank_at, {num_ranks}, torch::kInt32);
         auto num_tokens_per_rdma_rank = std::optional<torch::Tensor>();
-        auto num_tokens_per_expert = torch::empty({num_experts}, i32);
-        auto is_token_in_rank = torch::empty({num_tokens, num_ranks}, torch::dtype(torch::kBool).device(torch::kCUDA));
-        if (is_internode_available()) num_tokens_per_rdma_rank = torch::empty({num_rdma_ranks}, i32);
+        auto num_tokens_per_expert = b.take(expert_at, {num_experts}, torch::kInt32);
+        auto is_token_in_rank = b.take(member_at, {num_tokens, num_ranks}, torch::kBool);
+        if (is_internode_available()) num_tokens_per_rdma_rank = b.take(rdma_at, {num_rdma_ranks}, torch::kInt32);
 
         const int64_t ws_bytes =
             std::max<int64_t>(256, int64_t(deepep_layout_workspace_bytes(num_tokens, num_ranks, num_experts)));
@@ -732,42 +743,82 @@ static std::tuple<torch::Tensor, torch::Tensor> per_token_cast_to_fp8(const torc
     EP_HOST_ASSERT(n % 128 == 0);
     EP_HOST_ASSERT(not use_ue8m0 or round_scale);
     const int g = n / 128;
-    auto x_fp8 = torch::empty({m, n}, torch::dtype(torch::kFloat8_e4m3fn).device(x.device()));
+    auto x_fp8 = empty_on(x.device(), {m, n}, torch::kFloat8_e4m3fn);
     torch::Tensor scales;
     if (use_ue8m0) {
         EP_HOST_ASSERT(g % 4 == 0);
-        scales = torch::empty({m, g / 4}, torch::dtype(torch::kInt32).device(x.device()));
+        scales = empty_on(x.device(), {m, g / 4}, torch::kInt32);
     } else {
-        scales = torch::empty({m, g}, torch::dtype(torch::kFloat32).device(x.device()));
+        scales = empty_on(x.device(), {m, g}, torch::kFloat32);
     }
     abi_check(deepep_per_token_cast_to_fp8(x.data_ptr(), m, n, row_format_of(true, round_scale, use_ue8m0),
                                            x_fp8.data_ptr(), scales.data_ptr(), current_stream()));
     return {x_fp8, scales};
 }
 
-// reference: csrc/kernels/efa_kernels.cu:1591-1651 (the .item() host sync is the reference's)
+// A word of pinned memory that a kernel stores a result to and the host polls.  Reading the same 8 bytes back
+// with a copy and a synchronisation takes 16 us of an idle stream (the copy is a kernel of its own, and the wait
+// ends when the whole stream is done); the poll ends 5.5 us after the launch, while the kernel may still run.
+class HostWord {
+    at::DataPtr memory;
+    std::atomic<int64_t>* word;
+    static constexpr int64_t kUnset = INT64_MIN;
+
+public:
+    HostWord() : memory(at::getHostAllocator(at::kCUDA)->allocate(sizeof(int64_t))) {
+        static_assert(sizeof(std::atomic<int64_t>) == sizeof(int64_t));
+        word = new (memory.get()) std::atomic<int64_t>(kUnset);
+    }
+    int64_t* device_pointer() const { return reinterpret_cast<int64_t*>(word); }
+    // Waits for the value; `stream` is the one whose kernel stores it.  A stream that is busy for long is waited
+    // for in the ordinary way, which also reports what went wrong on it.
+    int64_t wait(hipStream_t stream) const {
+        pybind11::gil_scoped_release release;
+        const auto began = std::chrono::steady_clock::now();
+        for (int spins = 0; word->load(std::memory_order_acquire) == kUnset;) {
+            __builtin_ia32_pause();
+            if (++spins % 1024 == 0 and std::chrono::steady_clock::now() - began > std::chrono::milliseconds(1)) {
+                const hipError_t e = hipStreamSynchronize(stream);
+                if (e != hipSuccess) throw EPException("HIP", "deep_ep_cpp.cpp", __LINE__, hipGetErrorString(e));
+                break;
+            }
+        }
+        const int64_t value = word->load(std::memory_order_acquire);
+        if (value == kUnset) throw EPException("HIP", "deep_ep_cpp.cpp", __LINE__, "the kernel did not report its total");
+        return value;
+    }
+};
+
+// reference: csrc/kernels/efa_kernels.cu:1591-1651 (the host wait for the total is the reference's .item())
 static std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, int64_t, torch::Tensor> routing_sort_impl(
     const torch::Tensor& is_token_in_rank, bool with_positions) {
     EP_HOST_ASSERT(is_token_in_rank.dim() == 2);
     EP_HOST_ASSERT(is_token_in_rank.scalar_type() == torch::kBool);
     EP_HOST_ASSERT(is_token_in_rank.is_contiguous());
     EP_HOST_ASSERT(is_token_in_rank.is_cuda());
+    // the total is waited for, which a stream that is being captured cannot give
+    EP_HOST_ASSERT(c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None);
     const int num_tokens = static_cast<int>(is_token_in_rank.size(0)), num_ranks = static_cast<int>(is_token_in_rank.size(1));
-    auto dev = is_token_in_rank.device();
-    auto send_counts = torch::empty({num_ranks}, torch::dtype(torch::kInt32).device(dev));
-    auto send_cumsum = torch::empty({num_ranks + 1}, torch::dtype(torch::kInt64).device(dev));
-    auto ids = torch::empty({std::max<int64_t>(1, int64_t(num_tokens) * num_ranks)}, torch::dtype(torch::kInt64).device(dev));
-    auto ws = torch::empty({std::max<int64_t>(256, int64_t(deepep_routing_sort_workspace_bytes(num_tokens, num_ranks)))},
-                           torch::dtype(torch::kUInt8).device(dev));
+    const int64_t pairs = int64_t(num_tokens) * num_ranks;
+    const int64_t ws_bytes = std::max<int64_t>(256, int64_t(deepep_routing_sort_workspace_bytes(num_tokens, num_ranks)));
+    ResultBlock b;
+    const int64_t counts_at = b.reserve(4 * num_ranks), cumsum_at = b.reserve(8 * (num_ranks + 1)), ws_at = b.reserve(ws_bytes);
+    const int64_t ids_at = b.reserve(8 * std::max<int64_t>(1, pairs)), positions_at = b.reserve(with_positions ? 4 * pairs : 0);
+    b.allocate(is_token_in_rank.device());
+    auto send_counts = b.take(counts_at, {num_ranks}, torch::kInt32);
+    auto send_cumsum = b.take(cumsum_at, {num_ranks + 1}, torch::kInt64);
     torch::Tensor row_of_pair;
-    if (with_positions) row_of_pair = torch::empty({num_tokens, num_ranks}, torch::dtype(torch::kInt32).device(dev));
-    abi_check(deepep_moe_routing_sort(reinterpret_cast<const uint8_t*>(is_token_in_rank.data_ptr<bool>()), num_tokens,
-                                      num_ranks, ids.data_ptr<int64_t>(), send_counts.data_ptr<int>(),
-                                      send_cumsum.data_ptr<int64_t>(),
-                                      with_positions and num_tokens > 0 ? row_of_pair.data_ptr<int>() : nullptr,
-                                      ws.data_ptr(), size_t(ws.numel()), current_stream()));
-    const int64_t total = send_cumsum.select(0, num_ranks).item<int64_t>();
-    return {ids.slice(0, 0, total), send_counts, send_cumsum, total, row_of_pair};
+    if (with_positions) row_of_pair = b.take(positions_at, {num_tokens, num_ranks}, torch::kInt32);
+    uint8_t* base = b.block.data_ptr<uint8_t>();
+    const HostWord total_word;
+    const hipStream_t stream = current_stream();
+    abi_check(deepep_moe_routing_sort_total(
+        reinterpret_cast<const uint8_t*>(is_token_in_rank.data_ptr<bool>()), num_tokens, num_ranks,
+        reinterpret_cast<int64_t*>(base + ids_at), send_counts.data_ptr<int>(), send_cumsum.data_ptr<int64_t>(),
+        with_positions and num_tokens > 0 ? row_of_pair.data_ptr<int>() : nullptr, total_word.device_pointer(),
+        base + ws_at, size_t(ws_bytes), stream));
+    const int64_t total = total_word.wait(stream);
+    return {b.take(ids_at, {total}, torch::kInt64), send_counts, send_cumsum, total, row_of_pair};
 }
 
 static std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, int64_t> moe_routing_sort(const torch::Tensor& is_token_in_rank) {
@@ -788,7 +839,7 @@ static torch::Tensor channel_prefix_matrix(const torch::Tensor& is_token_in_rank
     EP_HOST_ASSERT(is_token_in_rank.scalar_type() == torch::kBool);
     EP_HOST_ASSERT(num_channels > 0);
     const int num_tokens = static_cast<int>(is_token_in_rank.size(0)), num_ranks = static_cast<int>(is_token_in_rank.size(1));
-    auto cpm = torch::empty({num_ranks, num_channels}, torch::dtype(torch::kInt32).device(is_token_in_rank.device()));
+    auto cpm = empty_on(is_token_in_rank.device(), {num_ranks, num_channels}, torch::kInt32);
     abi_check(deepep_channel_prefix_matrix(reinterpret_cast<const uint8_t*>(is_token_in_rank.data_ptr<bool>()),
                                            num_tokens, num_ranks, num_channels, cpm.data_ptr<int>(), current_stream()));
     return cpm;
@@ -810,8 +861,8 @@ static std::tuple<torch::Tensor, torch::Tensor> topk_remap(const torch::Tensor& 
     EP_HOST_ASSERT(send_cumsum.numel() == num_ranks + 1);
     EP_HOST_ASSERT(total_send >= 0 and total_send <= sorted_token_ids.numel());
     const int num_topk = static_cast<int>(topk_idx.size(1));
-    auto remapped_topk = torch::empty({total_send, num_topk}, topk_idx.options());
-    auto remapped_weights = torch::empty({total_send, num_topk}, topk_weights.options());
+    auto remapped_topk = empty_on(topk_idx.device(), {total_send, num_topk}, torch::kInt64);
+    auto remapped_weights = empty_on(topk_weights.device(), {total_send, num_topk}, torch::kFloat32);
     abi_check(deepep_topk_remap(topk_idx.data_ptr<int64_t>(), topk_weights.data_ptr<float>(),
                                 sorted_token_ids.data_ptr<int64_t>(), send_cumsum.data_ptr<int64_t>(),
                                 static_cast<int>(topk_idx.size(0)), num_topk, num_ranks, num_local_experts, total_send,
@@ -825,7 +876,7 @@ static torch::Tensor build_recv_src_meta(const torch::Tensor& recv_counts, const
     EP_HOST_ASSERT(recv_counts.is_cuda() and recv_cumsum.is_cuda());
     EP_HOST_ASSERT(recv_cumsum.scalar_type() == torch::kInt64 and recv_cumsum.is_contiguous());
     EP_HOST_ASSERT(recv_cumsum.numel() == num_ranks + 1 and num_recv_tokens >= 0);
-    auto meta = torch::empty({num_recv_tokens, 8}, torch::dtype(torch::kUInt8).device(recv_cumsum.device()));
+    auto meta = empty_on(recv_cumsum.device(), {num_recv_tokens, 8}, torch::kUInt8);
     abi_check(deepep_build_recv_src_meta(recv_cumsum.data_ptr<int64_t>(), num_ranks, num_local_ranks, num_recv_tokens,
                                          meta.data_ptr<uint8_t>(), current_stream()));
     return meta;
@@ -1097,11 +1148,15 @@ static std::tuple<torch::Tensor, std::optional<torch::Tensor>> combine_reduce(
         EP_HOST_ASSERT(row_of_pair->scalar_type() == torch::kInt32 and row_of_pair->is_contiguous() and row_of_pair->is_cuda());
         EP_HOST_ASSERT(row_of_pair->dim() == 2 and row_of_pair->size(0) == num_tokens and row_of_pair->size(1) == num_ranks);
     }
-    auto combined_x = torch::empty({num_tokens, hidden}, recv_x.options());
+    auto combined_x = empty_on(recv_x.device(), {num_tokens, hidden}, torch::kBFloat16);
     std::optional<torch::Tensor> combined_w;
-    if (recv_topk_weights.has_value()) combined_w = torch::empty({num_tokens, num_topk}, recv_topk_weights->options());
-    auto ws = torch::empty({std::max<int64_t>(256, int64_t(deepep_combine_reduce_workspace_bytes(num_tokens, num_ranks)))},
-                           torch::dtype(torch::kUInt8).device(recv_x.device()));
+    if (recv_topk_weights.has_value())
+        combined_w = empty_on(recv_topk_weights->device(), {num_tokens, num_topk}, torch::kFloat32);
+    torch::Tensor ws;  // where the pairs' rows are looked up, unless the sort's table is given
+    if (!row_of_pair.has_value())
+        ws = empty_on(recv_x.device(),
+                      {std::max<int64_t>(256, int64_t(deepep_combine_reduce_workspace_bytes(num_tokens, num_ranks)))},
+                      torch::kUInt8);
     abi_check(deepep_combine_reduce(
         recv_x.data_ptr(), recv_topk_weights.has_value() ? recv_topk_weights->data_ptr<float>() : nullptr,
         sorted_token_ids.data_ptr<int64_t>(), send_cumsum.data_ptr<int64_t>(),
@@ -1109,7 +1164,8 @@ static std::tuple<torch::Tensor, std::optional<torch::Tensor>> combine_reduce(
         bias_0.has_value() ? bias_0->data_ptr() : nullptr, bias_1.has_value() ? bias_1->data_ptr() : nullptr, num_tokens,
         hidden, num_topk, num_ranks, max_rows, row_of_pair.has_value() ? row_of_pair->data_ptr<int>() : nullptr,
         combined_x.data_ptr(),
-        combined_w.has_value() ? combined_w->data_ptr<float>() : nullptr, ws.data_ptr(), size_t(ws.numel()),
+        combined_w.has_value() ? combined_w->data_ptr<float>() : nullptr,
+        ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? size_t(ws.numel()) : 0,
         current_stream()));
     return {combined_x, combined_w};
 }
@@ -1126,14 +1182,14 @@ static std::tuple<torch::Tensor, std::optional<torch::Tensor>> pack_rows(const t
     const int64_t rows = sorted_token_ids.numel();
     const int64_t row_bytes = x.size(1) * x.element_size();
     EP_HOST_ASSERT(row_bytes % 16 == 0);
-    auto out = torch::empty({rows, x.size(1)}, x.options());
+    auto out = empty_on(x.device(), {rows, x.size(1)}, x.scalar_type());
     std::optional<torch::Tensor> out_scales;
     int64_t scale_row_bytes = 0;
     if (x_scales.has_value()) {
         EP_HOST_ASSERT(x_scales->dim() == 2 and x_scales->is_contiguous() and x_scales->size(0) == x.size(0));
         scale_row_bytes = x_scales->size(1) * x_scales->element_size();
         EP_HOST_ASSERT(scale_row_bytes % 4 == 0);
-        out_scales = torch::empty({rows, x_scales->size(1)}, x_scales->options());
+        out_scales = empty_on(x_scales->device(), {rows, x_scales->size(1)}, x_scales->scalar_type());
     }
     abi_check(deepep_pack_rows(x.data_ptr(), x_scales.has_value() ? x_scales->data_ptr() : nullptr,
                                sorted_token_ids.data_ptr<int64_t>(),

@@ -141,6 +141,30 @@ def test_routing_sort_channel_prefix(capi, t, r, p):
         assert torch.equal(cpm.cpu(), O.channel_prefix_matrix(is_in, c))
 
 
+@pytest.mark.parametrize("t,r", [(1, 8), (64, 16), (255, 32), (256, 64), (257, 8), (1025, 16), (2048, 64), (2049, 72),
+                                 (8192, 64), (8193, 64), (16384, 32), (16385, 32), (65536, 8), (65537, 8)])
+def test_layout_sort_and_prefix_where_their_launch_forms_meet(t, r):
+    """Sizes either side of the one-workgroup layout and the one-launch sort, through the host module, which also
+    waits for the sort's total."""
+    from deepep_efa_amd import deep_ep_cpp, normal
+    topk = _topk(t, min(6, 2 * r), 2 * r, seed=t + r, drop=3)
+    buffer = deep_ep_cpp.Buffer(r - 1, r, 0, 0, r > 8 and r % 8 != 0, False, False, False)
+    buffer.sync([0], [None], None)
+    per_rank, _, per_expert, is_in, _ = buffer.get_dispatch_layout(topk.cuda(), 2 * r, None, False, False)
+    want = O.get_dispatch_layout(topk, 2 * r, r)
+    assert torch.equal(per_rank.cpu(), want[0]) and torch.equal(per_expert.cpu(), want[2])
+    assert torch.equal(is_in.cpu(), want[3])
+    w_ids, w_counts, w_cumsum, w_total = O.moe_routing_sort(want[3])
+    torch.cuda._sleep(1_000_000 if t == 257 else 8_000_000 if t == 1025 else 1)  # a short and a long wait
+    ids, counts, cumsum, total, inverse = normal.moe_routing_sort_with_positions(is_in)
+    assert total == int(w_total)
+    assert torch.equal(ids.cpu(), w_ids) and torch.equal(counts.cpu(), w_counts)
+    assert torch.equal(cumsum.cpu(), w_cumsum)
+    assert torch.equal(inverse.cpu(), _want_row_of_pair(want[3], w_ids, w_cumsum))
+    for c in (1, 10, 33):
+        assert torch.equal(normal.channel_prefix_matrix(is_in, c).cpu(), O.channel_prefix_matrix(want[3], c))
+
+
 @pytest.mark.parametrize("seed", range(int(os.environ.get("DEEPEP_TEST_RANDOM_SHAPES", "16"))))
 def test_layout_sort_prefix_seeded_random_shapes(capi, seed):
     """Layout, routing sort and channel prefix on shapes nobody picked by hand (both sort paths)."""
