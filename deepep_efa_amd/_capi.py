@@ -28,6 +28,7 @@ PROTOTYPES = {
     "deepep_moe_routing_sort_total": (_I, [_VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),
     "deepep_channel_prefix_matrix": (_I, [_VP, _I, _I, _I, _VP, _VP]),
     "deepep_pack_rows": (_I, [_VP, _VP, _VP, _VP, _I64, _I, _I, _I, _VP, _VP, _VP]),
+    "deepep_pack_rows_by_rank": (_I, [_VP, _VP, _VP, _VP, _VP, _I, _I64, _I, _I, _I, _VP, _VP, _VP]),
     "deepep_per_token_cast_to_fp8": (_I, [_VP, _I, _I, _I, _VP, _VP, _VP]),
     "deepep_ll_dispatch_workspace_bytes": (_SZ, [_I, _I, _I]),
     "deepep_ll_dispatch_send": (_I, [_VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),

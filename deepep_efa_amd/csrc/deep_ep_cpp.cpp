@@ -1191,12 +1191,13 @@ static std::tuple<torch::Tensor, std::optional<torch::Tensor>> pack_rows(const t
         EP_HOST_ASSERT(scale_row_bytes % 4 == 0);
         out_scales = empty_on(x_scales->device(), {rows, x_scales->size(1)}, x_scales->scalar_type());
     }
-    abi_check(deepep_pack_rows(x.data_ptr(), x_scales.has_value() ? x_scales->data_ptr() : nullptr,
-                               sorted_token_ids.data_ptr<int64_t>(),
-                               send_cumsum.data_ptr<int64_t>() + (send_cumsum.numel() - 1), rows,
-                               static_cast<int>(x.size(0)), static_cast<int>(row_bytes), static_cast<int>(scale_row_bytes),
-                               out.data_ptr(), out_scales.has_value() ? out_scales->data_ptr() : nullptr,
-                               current_stream()));
+    const int num_ranks = static_cast<int>(send_cumsum.numel() - 1);
+    const int64_t* cumsum = send_cumsum.data_ptr<int64_t>();
+    abi_check(deepep_pack_rows_by_rank(
+        x.data_ptr(), x_scales.has_value() ? x_scales->data_ptr() : nullptr, sorted_token_ids.data_ptr<int64_t>(),
+        cumsum + num_ranks, num_ranks > 0 ? cumsum : nullptr, num_ranks, rows, static_cast<int>(x.size(0)),
+        static_cast<int>(row_bytes), static_cast<int>(scale_row_bytes), out.data_ptr(),
+        out_scales.has_value() ? out_scales->data_ptr() : nullptr, current_stream()));
     return {out, out_scales};
 }
 

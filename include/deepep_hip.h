@@ -144,6 +144,14 @@ int deepep_pack_rows(const void* src, const void* scale_src, const int64_t* sort
                      int row_bytes, int scale_row_bytes,
                      void* dst, void* scale_dst, void* stream);
 
+/* The same for a list that is known to be `num_ranks` ascending lists one after another, list r being rows
+ * [send_cumsum[r], send_cumsum[r + 1]) (what deepep_moe_routing_sort writes): large packs then take the copies of
+ * a token together, so that its row is read from HBM once.  num_rows_dev as above (send_cumsum + num_ranks). */
+int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64_t* sorted_token_ids,
+                             const int64_t* num_rows_dev, const int64_t* send_cumsum, int num_ranks,
+                             int64_t max_rows, int num_src_rows, int row_bytes, int scale_row_bytes,
+                             void* dst, void* scale_dst, void* stream);
+
 /* Top-k of the rows being sent, in the destination rank's expert numbering:
  * for send row i (destination rank d, send_cumsum[d] <= i < send_cumsum[d+1])
  * and selection k, (e - d*E_l, w) if the token's expert e is one of rank d's,

@@ -226,6 +226,40 @@ def test_pack_rows(capi, rows, row_bytes, scale_bytes):
         assert torch.equal(dsc[:total].cpu(), sc[ids]) and (dsc[total:] == 0xEE).all()
 
 
+@pytest.mark.parametrize("rows,row_bytes,scale_bytes,r,odds,keep", [
+    (2500, 1040, 8, 8, 0.66, 1.0),     # just past one group's worth: 8 groups, rows that are no multiple of a line
+    (1500, 1024, 0, 8, 0.66, 1.0),     # just below: list order
+    (3000, 2048, 16, 64, 0.1, 1.0),    # a rank per lane
+    (3000, 2048, 0, 72, 0.1, 1.0),     # more ranks than lanes: list order
+    (900, 16384 + 16, 4, 16, 0.9, 1.0),   # a row wider than one round of 512 threads
+    (6000, 2048, 0, 8, (1.0, 0.0, 0.02, 1.0, 0.5, 0.0, 0.9, 0.001), 1.0),  # lists of very different lengths
+    (4000, 2048, 0, 8, 0.66, 0.6),     # a list cut off before its end
+    (4000, 2048, 0, 8, 0.66, 1.5),     # room for more rows than there are
+])
+def test_pack_rows_by_rank(capi, rows, row_bytes, scale_bytes, r, odds, keep):
+    lib = capi.load()
+    g = torch.Generator().manual_seed(rows + r)
+    src = torch.randint(0, 256, (rows, row_bytes), dtype=torch.uint8, generator=g)
+    sc = torch.randint(0, 256, (rows, scale_bytes), dtype=torch.uint8, generator=g) if scale_bytes else None
+    is_in = torch.rand((rows, r), generator=g) < torch.tensor(odds)
+    ids, _, cumsum, total = O.moe_routing_sort(is_in)
+    cap = int(total * keep)
+    ids_full = torch.full((max(cap, total),), -1, dtype=torch.int64)
+    ids_full[:total] = ids
+    d_src, d_ids, d_cumsum = src.cuda(), ids_full[:cap].cuda(), cumsum.cuda()
+    d_sc = sc.cuda() if sc is not None else None
+    dst = torch.full((cap, row_bytes), 0xEE, dtype=torch.uint8, device="cuda")
+    dsc = torch.full((cap, scale_bytes), 0xEE, dtype=torch.uint8, device="cuda") if scale_bytes else None
+    capi.check(lib.deepep_pack_rows_by_rank(
+        capi.ptr(d_src), capi.ptr(d_sc), capi.ptr(d_ids), d_cumsum.data_ptr() + 8 * r, capi.ptr(d_cumsum), r, cap, rows,
+        row_bytes, scale_bytes, capi.ptr(dst), capi.ptr(dsc), stream()))
+    torch.cuda.synchronize()
+    n = min(cap, total)
+    assert torch.equal(dst[:n].cpu(), src[ids[:n]]) and (dst[n:] == 0xEE).all()
+    if scale_bytes:
+        assert torch.equal(dsc[:n].cpu(), sc[ids[:n]]) and (dsc[n:] == 0xEE).all()
+
+
 def run_cast(capi, x, fmt):
     lib = capi.load()
     m, n = x.shape
