@@ -247,12 +247,11 @@ struct Buffer {
     LowLatencyCache ll;
     std::vector<torch::Tensor> combine_input_buffers;
     int combine_buffer_idx = 0;
-    // Rows the last large dispatch received, read back without blocking: the next large call is sized by it.
-    // (Under skewed routing a rank can receive many times num_tokens * num_topk rows; the row-copy kernels
-    // take their grid from the rows expected, and one sized for a balanced world walks such a batch in a slow loop.)
-    torch::Tensor observed_count_host;
-    std::optional<torch::Event> observed_ready;
-    int64_t observed_rows = 0;
+    // What the last dispatch that has run received, stored there by its kernel as (tokens << 32) | rows: the next
+    // call is sized by it.  Under skewed routing a rank can receive many times num_tokens * num_topk rows, and
+    // kernels sized for a balanced world walk such a batch in a slow loop.
+    at::DataPtr observed_memory;
+    std::atomic<uint64_t>* observed = nullptr;
     // loopback world
     std::optional<torch::Tensor> world_x, world_topk_idx;
     torch::Tensor ranks_below, ranks_above, peer_workspace;
@@ -315,8 +314,8 @@ struct Buffer {
         rdma_buffer = torch::Tensor();
         layout_workspaces.clear();
         ll = LowLatencyCache();
-        observed_ready.reset();
-        observed_count_host = torch::Tensor();
+        observed = nullptr;
+        observed_memory.clear();
         combine_input_buffers.clear();
         world_x.reset();
         world_topk_idx.reset();
@@ -484,9 +483,8 @@ struct Buffer {
         ll.pair_slot = torch::full({m, num_topk}, -1, i32);
         ll.workspace = torch::empty(
             {std::max<int64_t>(256, int64_t(deepep_ll_dispatch_workspace_bytes(max_tokens, num_topk, num_experts)))}, u8);
-        if (int64_t(m) * num_topk > 8192)  // index + flat-copy scratch, only used by large batches
-            ll.segment_workspace =
-                torch::empty({int64_t(deepep_ll_segment_workspace_bytes(num_experts, max_tokens))}, u8);
+        // index + flat-copy scratch, used where more than 8192 rows are expected
+        ll.segment_workspace = torch::empty({int64_t(deepep_ll_segment_workspace_bytes(num_experts, max_tokens))}, u8);
         if (fmt == DEEPEP_ROW_BF16) {
             ll.packed_recv_x = torch::empty({el, r * m, h}, bf16);
         } else {
@@ -503,6 +501,18 @@ struct Buffer {
         ll.combine_send_slots = torch::empty({el, r, m, h}, bf16);
         ll.combined_x = torch::empty({m, h}, bf16);
         return ll;
+    }
+
+    // Rows a batch of num_tokens probably receives: what a balanced world sends or, if more, what the last batch
+    // received, in proportion (a batch of less than a quarter of the tokens says too little).  A hint: kernels
+    // and grids are chosen by it, never results.
+    int64_t rows_expected(int num_tokens, int num_topk, int num_experts, int max_tokens) const {
+        const int64_t balanced = std::max<int64_t>(num_tokens, 1) * num_topk;
+        if (observed == nullptr) return balanced;
+        const uint64_t last = observed->load(std::memory_order_relaxed);
+        const int64_t tokens = int64_t(last >> 32), rows = int64_t(last & 0xffffffffu);
+        if (tokens == 0 or tokens * 4 < num_tokens) return balanced;
+        return std::max(balanced, std::min(rows * num_tokens / tokens, int64_t(num_experts) * max_tokens));
     }
 
     void stage_peer_rows(LowLatencyCache& c) {
@@ -563,20 +573,14 @@ struct Buffer {
         auto stream = current_stream();
 
         stage_peer_rows(c);  // what the exchange would have delivered
-        // Large batches: the hint is what the dispatch before this one received, if that has arrived on the host
-        const bool large = int64_t(num_tokens) * num_topk > 8192;
-        int64_t expected_rows = std::max<int64_t>(num_tokens, 1) * num_topk;
-        const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
-        if (large) {
-            // (an event may not be queried while a stream is being captured: a captured call keeps the last hint)
-            if (not capturing and observed_ready.has_value() and observed_ready->query()) {
-                observed_rows = observed_count_host.sum().item<int64_t>();
-                observed_ready.reset();
-            }
-            expected_rows = std::max(expected_rows, observed_rows);
+        if (observed == nullptr) {
+            observed_memory = at::getHostAllocator(at::kCUDA)->allocate(sizeof(uint64_t));
+            observed = new (observed_memory.get()) std::atomic<uint64_t>(0);
         }
+        // a captured call takes the hint but does not report: its replays may outlive the buffer
+        const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
         // send and receive phase in one call (one kernel launch for decode-sized batches)
-        abi_check(deepep_ll_dispatch(
+        abi_check(deepep_ll_dispatch_observed(
             x.data_ptr(), topk_idx.data_ptr<int64_t>(), num_tokens, hidden, num_topk, num_experts, num_ranks, rank,
             num_max_dispatch_tokens_per_rank, fmt, c.recv_staging.data_ptr(), c.recv_count.data_ptr<int>(),
             c.send_slots.data_ptr(), c.send_count.data_ptr<int>(), c.pair_slot.data_ptr<int>(),
@@ -584,19 +588,10 @@ struct Buffer {
             c.packed_recv_src_info.data_ptr<int>(), c.packed_recv_layout_range.data_ptr<int64_t>(),
             c.packed_recv_count.data_ptr<int>(),
             cumulative_local_expert_recv_stats.has_value() ? cumulative_local_expert_recv_stats->data_ptr<int>() : nullptr,
-            expected_rows, c.workspace.data_ptr(),
-            size_t(c.workspace.numel()), c.segment_workspace.defined() ? c.segment_workspace.data_ptr() : nullptr,
-            c.segment_workspace.defined() ? size_t(c.segment_workspace.numel()) : 0, stream));
+            rows_expected(num_tokens, num_topk, num_experts, num_max_dispatch_tokens_per_rank), c.workspace.data_ptr(),
+            size_t(c.workspace.numel()), c.segment_workspace.data_ptr(), size_t(c.segment_workspace.numel()),
+            capturing ? nullptr : reinterpret_cast<uint64_t*>(observed), stream));
         c.dispatched = true;
-        if (large and not capturing and not observed_ready.has_value()) {
-            if (!observed_count_host.defined() or observed_count_host.numel() != c.packed_recv_count.numel())
-                observed_count_host = torch::empty({c.packed_recv_count.numel()},
-                                                   torch::dtype(torch::kInt32).pinned_memory(true));
-            observed_count_host.copy_(c.packed_recv_count, /*non_blocking=*/true);
-            observed_ready = torch::Event(torch::kCUDA);
-            observed_ready->record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA());
-        }
-
         std::optional<EventHandle> event;
         if (async) event = EventHandle();
         std::optional<std::function<void()>> hook;
@@ -678,10 +673,9 @@ struct Buffer {
                                     accumulate ? 1 : 0, c.combine_staging.data_ptr(),
                                     zero_copy ? nullptr : c.combine_send_slots.data_ptr(),
                                     combined_x.data_ptr(),
-                                    /*expected_rows=*/std::max<int64_t>(std::max<int64_t>(num_combined_tokens, 1) * num_topk,
-                                                                         int64_t(num_combined_tokens) * num_topk > 8192 ? observed_rows : 0),
-                                    c.segment_workspace.defined() ? c.segment_workspace.data_ptr() : nullptr,
-                                    c.segment_workspace.defined() ? size_t(c.segment_workspace.numel()) : 0, stream));
+                                    rows_expected(num_combined_tokens, num_topk, num_experts,
+                                                  num_max_dispatch_tokens_per_rank),
+                                    c.segment_workspace.data_ptr(), size_t(c.segment_workspace.numel()), stream));
 
         std::optional<EventHandle> event;
         if (async) event = EventHandle();

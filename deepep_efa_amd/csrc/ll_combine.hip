@@ -452,7 +452,7 @@ static int launch_combine_send(const void* x, const int64_t* layout_range, int h
         ll_segment_index_kernel<<<num_experts, kIndexThreads, 0, hs>>>(
             skip_own ? 2 : 1, nullptr, layout_range, num_local_experts, num_ranks, rank,
             num_max_dispatch_tokens_per_rank, nullptr,
-            nullptr, nullptr, flat, desc);
+            nullptr, nullptr, flat, desc, ObservedRows{nullptr, 0});
         EP_LAUNCH_CHECK();
         const int num_vec = hidden * 2 / 16;
         int threads = ((num_vec + 63) / 64) * 64;

@@ -545,6 +545,7 @@ struct RecvArgs {
     int64_t* layout_range;
     int32_t* packed_count;
     int32_t* stats;
+    ObservedRows observed;
 };
 
 __device__ __forceinline__ int clamp_count(int c, int max_tokens) {
@@ -640,6 +641,7 @@ __device__ __forceinline__ void recv_rows_impl(const RecvArgs& a, int block, int
         }
         lds_barrier();
         block_exclusive_scan(lds, num_segments, wave_totals);
+        if (tid == 0) report_observed(a.observed, lds[num_segments]);
         for (int s = tid; s < num_segments; s += threads) {
             const int le = s / num_ranks;
             const int64_t cnt = lds[s + 1] - lds[s];
@@ -1192,7 +1194,7 @@ static RecvArgs make_recv_args(const void* recv_staging, const int32_t* recv_cou
                                int num_ranks, int max_tokens, int row_format, void* packed_recv_x,
                                void* packed_recv_scales, int32_t* packed_recv_src_info,
                                int64_t* packed_recv_layout_range, int32_t* packed_recv_count, int32_t* stats,
-                               int64_t expected_rows) {
+                               int64_t expected_rows, const ObservedRows& observed) {
     RecvArgs ra;
     ra.recv_staging = reinterpret_cast<const uint8_t*>(recv_staging);
     ra.recv_count = recv_count;
@@ -1204,6 +1206,7 @@ static RecvArgs make_recv_args(const void* recv_staging, const int32_t* recv_cou
     ra.packed_scales = reinterpret_cast<uint8_t*>(packed_recv_scales);
     ra.src_info = packed_recv_src_info, ra.layout_range = packed_recv_layout_range;
     ra.packed_count = packed_recv_count, ra.stats = stats;
+    ra.observed = observed;
     return ra;
 }
 
@@ -1214,7 +1217,8 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
                             void* packed_recv_x, void* packed_recv_scales, int32_t* packed_recv_src_info,
                             int64_t* packed_recv_layout_range, int32_t* packed_recv_count,
                             int32_t* cumulative_local_expert_recv_stats, int64_t expected_rows, void* workspace,
-                            size_t workspace_bytes, int own_rank, void* stream, bool index_done = false) {
+                            size_t workspace_bytes, int own_rank, void* stream, bool index_done = false,
+                            const ObservedRows& observed = ObservedRows{nullptr, 0}) {
     if (int rc = check_recv_args(recv_staging, recv_count, hidden, num_experts, num_ranks,
                                  num_max_dispatch_tokens_per_rank, row_format, packed_recv_x, packed_recv_scales,
                                  packed_recv_src_info, packed_recv_layout_range, packed_recv_count))
@@ -1232,7 +1236,7 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
         if (!index_done) {  // (a large one-call dispatch builds the index inside its send launch)
             ll_segment_index_kernel<<<num_experts, kIndexThreads, 0, hs>>>(
                 0, recv_count, nullptr, num_local_experts, num_ranks, own_rank, num_max_dispatch_tokens_per_rank,
-                packed_recv_layout_range, packed_recv_count, cumulative_local_expert_recv_stats, flat, desc);
+                packed_recv_layout_range, packed_recv_count, cumulative_local_expert_recv_stats, flat, desc, observed);
             EP_LAUNCH_CHECK();
         }
         const int64_t data_bytes = row_data_bytes(hidden, row_format);
@@ -1255,7 +1259,7 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
     const RecvArgs ra = make_recv_args(recv_staging, recv_count, hidden, num_experts, num_ranks,
                                        num_max_dispatch_tokens_per_rank, row_format, packed_recv_x, packed_recv_scales,
                                        packed_recv_src_info, packed_recv_layout_range, packed_recv_count,
-                                       cumulative_local_expert_recv_stats, expected_rows);
+                                       cumulative_local_expert_recv_stats, expected_rows, observed);
     int64_t blocks = ((max_rows << ra.parts_log2) + 3) / 4;
     const int64_t cap = large ? 4096 : 1024;
     if (blocks > cap) blocks = cap;
@@ -1286,15 +1290,17 @@ int deepep_ll_dispatch_is_single_launch(int num_tokens, int num_topk, int num_ex
                : 0;
 }
 
-int deepep_ll_dispatch(const void* x, const int64_t* topk_idx, int num_tokens, int hidden, int num_topk,
-                       int num_experts, int num_ranks, int rank, int num_max_dispatch_tokens_per_rank, int row_format,
-                       void* recv_staging, int32_t* recv_count, void* send_slots, int32_t* send_count,
-                       int32_t* pair_slot, void* packed_recv_x, void* packed_recv_scales,
-                       int32_t* packed_recv_src_info, int64_t* packed_recv_layout_range, int32_t* packed_recv_count,
-                       int32_t* cumulative_local_expert_recv_stats, int64_t expected_rows, void* workspace,
-                       size_t workspace_bytes, void* segment_workspace, size_t segment_workspace_bytes,
-                       void* stream) {
+int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx, int num_tokens, int hidden, int num_topk,
+                                int num_experts, int num_ranks, int rank, int num_max_dispatch_tokens_per_rank, int row_format,
+                                void* recv_staging, int32_t* recv_count, void* send_slots, int32_t* send_count,
+                                int32_t* pair_slot, void* packed_recv_x, void* packed_recv_scales,
+                                int32_t* packed_recv_src_info, int64_t* packed_recv_layout_range, int32_t* packed_recv_count,
+                                int32_t* cumulative_local_expert_recv_stats, int64_t expected_rows, void* workspace,
+                                size_t workspace_bytes, void* segment_workspace, size_t segment_workspace_bytes,
+                                uint64_t* observed_host, void* stream) {
     clear_error();
+    EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(observed_host) & 7) == 0);
+    const ObservedRows observed = {observed_host, uint32_t(num_tokens < 0 ? 0 : num_tokens)};
     const int64_t max_rows = int64_t(num_experts) * num_max_dispatch_tokens_per_rank;
     const bool fused = deepep_ll_dispatch_is_single_launch(num_tokens, num_topk, num_experts,
                                                            num_max_dispatch_tokens_per_rank, expected_rows) != 0;
@@ -1331,6 +1337,7 @@ int deepep_ll_dispatch(const void* x, const int64_t* topk_idx, int num_tokens, i
             index.num_ranks = num_ranks, index.rank = rank, index.max_tokens = num_max_dispatch_tokens_per_rank;
             index.layout_out = packed_recv_layout_range, index.packed_count = packed_recv_count;
             index.stats = cumulative_local_expert_recv_stats;
+            index.observed = observed;
             index.flat_out = reinterpret_cast<int32_t*>(segment_workspace);
             index.desc = reinterpret_cast<RowDesc*>(reinterpret_cast<uint8_t*>(segment_workspace) +
                                                     (((int64_t(num_experts) + 1) * 4 + 255) & ~int64_t(255)));
@@ -1346,7 +1353,7 @@ int deepep_ll_dispatch(const void* x, const int64_t* topk_idx, int num_tokens, i
                                 num_max_dispatch_tokens_per_rank, row_format, packed_recv_x, packed_recv_scales,
                                 packed_recv_src_info, packed_recv_layout_range, packed_recv_count,
                                 cumulative_local_expert_recv_stats, expected_rows, segment_workspace,
-                                segment_workspace_bytes, rank, stream, index_done);
+                                segment_workspace_bytes, rank, stream, index_done, observed);
     }
     EP_HOST_ASSERT(num_tokens == 0 || (x != nullptr && topk_idx != nullptr));
     EP_HOST_ASSERT(send_count != nullptr && pair_slot != nullptr);
@@ -1359,7 +1366,7 @@ int deepep_ll_dispatch(const void* x, const int64_t* topk_idx, int num_tokens, i
     const RecvArgs ra = make_recv_args(recv_staging, recv_count, hidden, num_experts, num_ranks,
                                        num_max_dispatch_tokens_per_rank, row_format, packed_recv_x, packed_recv_scales,
                                        packed_recv_src_info, packed_recv_layout_range, packed_recv_count,
-                                       cumulative_local_expert_recv_stats, expected_rows);
+                                       cumulative_local_expert_recv_stats, expected_rows, observed);
     int64_t rows = expected_rows > 0 ? expected_rows : int64_t(num_max_dispatch_tokens_per_rank) * num_topk;
     rows += rows / 8 + 16;
     if (rows > max_rows) rows = max_rows;
@@ -1367,6 +1374,21 @@ int deepep_ll_dispatch(const void* x, const int64_t* topk_idx, int num_tokens, i
                             num_max_dispatch_tokens_per_rank, row_format, recv_staging, recv_count, send_slots,
                             send_count, pair_slot, workspace, workspace_bytes,
                             reinterpret_cast<hipStream_t>(stream), &ra, rows << ra.parts_log2);
+}
+
+int deepep_ll_dispatch(const void* x, const int64_t* topk_idx, int num_tokens, int hidden, int num_topk,
+                       int num_experts, int num_ranks, int rank, int num_max_dispatch_tokens_per_rank, int row_format,
+                       void* recv_staging, int32_t* recv_count, void* send_slots, int32_t* send_count,
+                       int32_t* pair_slot, void* packed_recv_x, void* packed_recv_scales,
+                       int32_t* packed_recv_src_info, int64_t* packed_recv_layout_range, int32_t* packed_recv_count,
+                       int32_t* cumulative_local_expert_recv_stats, int64_t expected_rows, void* workspace,
+                       size_t workspace_bytes, void* segment_workspace, size_t segment_workspace_bytes,
+                       void* stream) {
+    return deepep_ll_dispatch_observed(
+        x, topk_idx, num_tokens, hidden, num_topk, num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank,
+        row_format, recv_staging, recv_count, send_slots, send_count, pair_slot, packed_recv_x, packed_recv_scales,
+        packed_recv_src_info, packed_recv_layout_range, packed_recv_count, cumulative_local_expert_recv_stats,
+        expected_rows, workspace, workspace_bytes, segment_workspace, segment_workspace_bytes, nullptr, stream);
 }
 
 }  // extern "C"

@@ -185,6 +185,18 @@ struct RowDesc {
     int32_t dst_row;  // >= 0: row index in the primary destination; < 0: -(1 + row) in the secondary one
 };
 
+// Where a dispatch reports the rows it received to a host that sizes the next one by it: (tokens sent << 32) | rows,
+// one 8-byte store into pinned memory that the host reads whenever it likes.  A null word reports nothing.
+struct ObservedRows {
+    uint64_t* host;
+    uint32_t tokens;
+};
+__device__ __forceinline__ void report_observed(const ObservedRows& o, int rows) {
+    if (o.host != nullptr)
+        __hip_atomic_store(o.host, (uint64_t(o.tokens) << 32) | uint32_t(rows), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 constexpr int kIndexThreads = 1024;
 
 // Exclusive prefix over one value per thread of a 1024-thread workgroup; returns the prefix, sets total.
@@ -213,7 +225,7 @@ __device__ __forceinline__ int block_exclusive_scan_1024(int v, int32_t* wave_to
 static __global__ __launch_bounds__(kIndexThreads) void ll_segment_index_kernel(
     int mode, const int32_t* __restrict__ counts32, const int64_t* __restrict__ layout_in, int num_local_experts,
     int num_ranks, int rank, int max_tokens, int64_t* __restrict__ layout_out, int32_t* __restrict__ packed_count,
-    int32_t* __restrict__ stats, int32_t* __restrict__ flat_out, RowDesc* __restrict__ desc) {
+    int32_t* __restrict__ stats, int32_t* __restrict__ flat_out, RowDesc* __restrict__ desc, ObservedRows observed) {
     __shared__ int32_t flat[kIndexThreads + 1];   // prefix over the rows that get descriptors
     __shared__ int32_t place[kIndexThreads + 1];  // mode 0: prefix over all rows (where a segment lands)
     __shared__ int32_t begin_in[kIndexThreads];
@@ -254,6 +266,7 @@ static __global__ __launch_bounds__(kIndexThreads) void ll_segment_index_kernel(
     if (blockIdx.x == 0) {
         for (int s = tid; s <= num_segments; s += kIndexThreads) flat_out[s] = flat[s];
         if (mode == 0) {
+            if (tid == 0) report_observed(observed, place[num_segments]);
             if (tid < num_segments) {
                 const int le = tid / num_ranks;
                 const int64_t cnt = c_all;
@@ -300,6 +313,7 @@ struct FusedIndexArgs {
     int32_t* stats;
     int32_t* flat_out;
     RowDesc* desc;
+    ObservedRows observed;
 };
 
 __device__ __forceinline__ void recv_index_block(const FusedIndexArgs& a, int seg, int32_t* lds, int32_t* wave_totals) {
@@ -333,6 +347,7 @@ __device__ __forceinline__ void recv_index_block(const FusedIndexArgs& a, int se
     block_exclusive_scan(place, num_segments, wave_totals);
     const int64_t slots_per_expert = int64_t(max_tokens) * num_ranks;
     if (seg == 0) {
+        if (tid == 0) report_observed(a.observed, place[num_segments]);
         for (int s = tid; s <= num_segments; s += threads) a.flat_out[s] = flat[s];
         for (int s = tid; s < num_segments; s += threads) {
             const int le = s / num_ranks;

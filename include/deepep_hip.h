@@ -567,6 +567,21 @@ int deepep_ll_dispatch(const void* x, const int64_t* topk_idx,
                        int64_t expected_rows, void* workspace, size_t workspace_bytes,
                        void* segment_workspace, size_t segment_workspace_bytes, void* stream);
 
+/* The same, reporting what it received: observed_host (8 bytes the device can write and the host read, pinned
+ * memory; NULL: as above) receives (num_tokens << 32) | rows received.  A caller that reads it before its next
+ * call has a hint for expected_rows under skewed routing, without a copy or a wait. */
+int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx,
+                       int num_tokens, int hidden, int num_topk, int num_experts,
+                       int num_ranks, int rank, int num_max_dispatch_tokens_per_rank,
+                       int row_format,
+                       void* recv_staging, int32_t* recv_count,
+                       void* send_slots, int32_t* send_count, int32_t* pair_slot,
+                       void* packed_recv_x, void* packed_recv_scales,
+                       int32_t* packed_recv_src_info, int64_t* packed_recv_layout_range,
+                       int32_t* packed_recv_count, int32_t* cumulative_local_expert_recv_stats,
+                       int64_t expected_rows, void* workspace, size_t workspace_bytes,
+                       void* segment_workspace, size_t segment_workspace_bytes, uint64_t* observed_host, void* stream);
+
 /* deepep_ll_combine_send followed by deepep_ll_combine_recv, for a caller
  * whose remote experts' answers are already in combine_staging when the call
  * is made (the reference: Buffer::low_latency_combine,
