@@ -455,10 +455,8 @@ static int launch_combine_send(const void* x, const int64_t* layout_range, int h
             nullptr, nullptr, flat, desc, ObservedRows{nullptr, 0});
         EP_LAUNCH_CHECK();
         const int num_vec = hidden * 2 / 16;
-        int threads = ((num_vec + 63) / 64) * 64;
-        if (threads > 1024) threads = 1024;
-        ll_rows_flat_kernel<<<flat_grid_blocks(expected_rows, max_rows, num_max_dispatch_tokens_per_rank), threads, 0,
-                              hs>>>(flat, num_experts, desc, reinterpret_cast<const uint8_t*>(x), int64_t(hidden) * 2,
+        ll_rows_flat_kernel<<<flat_grid_blocks(expected_rows, max_rows, num_max_dispatch_tokens_per_rank),
+                              flat_row_threads(num_vec), 0, hs>>>(flat, num_experts, desc, reinterpret_cast<const uint8_t*>(x), int64_t(hidden) * 2,
                                     num_vec, reinterpret_cast<uint8_t*>(combine_send_slots),
                                     reinterpret_cast<uint8_t*>(combine_staging), int64_t(hidden) * 2, 0, 0, nullptr, 0,
                                     nullptr, 0);

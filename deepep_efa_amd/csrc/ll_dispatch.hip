@@ -1242,9 +1242,7 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
         const int64_t data_bytes = row_data_bytes(hidden, row_format);
         const int64_t scale_bytes = row_scale_bytes(hidden, row_format);
         const int num_vec = int(data_bytes / 16);
-        int threads = ((num_vec + 63) / 64) * 64;
-        int extra = 64;  // one more wave for scales + source index
-        if (threads + extra > 1024) threads = 1024, extra = 0;
+        const int threads = flat_row_threads(num_vec), extra = 64;  // one more wave for scales + source index
         ll_rows_flat_kernel<<<flat_grid_blocks(expected_rows, max_rows, num_max_dispatch_tokens_per_rank),
                               threads + extra, 0,
                               hs>>>(flat, num_experts, desc, reinterpret_cast<const uint8_t*>(recv_staging),

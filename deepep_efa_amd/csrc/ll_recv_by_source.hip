@@ -617,9 +617,7 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
     }
     if (row_capacity == 0) return 0;
     const int num_vec = int(data_bytes / 16);
-    int threads = ((num_vec + 63) / 64) * 64;
-    int extra = 64;  // one more wave for scales + source index
-    if (threads + extra > 1024) threads = 1024, extra = 0;
+    const int threads = flat_row_threads(num_vec), extra = 64;  // one more wave for scales + source index
     // the copy's grid follows the rows expected, not the capacity: a workgroup that finds no row still costs
     // a fraction of a nanosecond, and a capacity of R slots is many times what a balanced world fills
     const unsigned blocks = flat_grid_blocks(expected_rows > 0 ? expected_rows : row_capacity, row_capacity,
@@ -701,9 +699,7 @@ int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_
     const int64_t data_bytes = row_data_bytes(hidden, row_format);
     const int64_t scale_bytes = row_scale_bytes(hidden, row_format);
     const int num_vec = int(data_bytes / 16);
-    int threads = ((num_vec + 63) / 64) * 64;
-    int extra = 64;  // one more wave for scales + source index
-    if (threads + extra > 1024) threads = 1024, extra = 0;
+    const int threads = flat_row_threads(num_vec), extra = 64;  // one more wave for scales + source index
     const unsigned blocks = flat_grid_blocks(expected_rows > 0 ? expected_rows : most_rows, most_rows,
                                              num_max_dispatch_tokens_per_rank);
     ll_rows_flat_kernel<<<blocks, threads + extra, 0, hs>>>(
