@@ -221,15 +221,14 @@ class Buffer:
                 self._ll_dispatch_profiler = _LLProfiler("DISPATCH", self.rank)
             prof = self._ll_dispatch_profiler
             prof.mark("start")
-        recv_x, recv_scales, recv_count, src_info, layout_range, event, hook = self.runtime.low_latency_dispatch(
-            x, topk_idx, cumulative_local_expert_recv_stats, dispatch_wait_recv_cost_stats,
-            num_max_dispatch_tokens_per_rank, num_experts, use_fp8, round_scale, use_ue8m0, async_finish, return_recv_hook)
-        handle = (src_info, layout_range, num_max_dispatch_tokens_per_rank, x.size(1), num_experts)
+        recv_x, recv_count, handle, event, hook = deep_ep_cpp.low_latency_dispatch(
+            self.runtime, x, topk_idx, cumulative_local_expert_recv_stats, dispatch_wait_recv_cost_stats,
+            num_max_dispatch_tokens_per_rank, num_experts, use_fp8, round_scale, use_ue8m0, async_finish,
+            return_recv_hook)
         if prof:
             prof.mark("end")
             prof.finish_iter()
-        out = (recv_x, recv_scales) if use_fp8 else recv_x
-        return out, recv_count, handle, EventOverlap(event or EventHandle.deferred()), hook
+        return recv_x, recv_count, handle, EventOverlap(event), hook
 
     def low_latency_combine(self, x: torch.Tensor, topk_idx: torch.Tensor, topk_weights: torch.Tensor, handle: tuple,
                             use_logfmt: bool = False, zero_copy: bool = False, async_finish: bool = False,
@@ -248,21 +247,19 @@ class Buffer:
         stream waits on it, since the call's own stream is in order already.
         """
         assert not accumulate or out is not None, "accumulate adds to `out`"
-        src_info, layout_range, num_max_dispatch_tokens_per_rank, hidden, num_experts = handle
         prof = None
         if _PROFILE_ENABLED:
             if not hasattr(self, "_ll_combine_profiler"):
                 self._ll_combine_profiler = _LLProfiler("COMBINE", self.rank)
             prof = self._ll_combine_profiler
             prof.mark("start")
-        combined_x, event, hook = self.runtime.low_latency_combine(
-            x, topk_idx, topk_weights, src_info, layout_range, combine_wait_recv_cost_stats,
-            num_max_dispatch_tokens_per_rank, num_experts, use_logfmt, zero_copy, async_finish, return_recv_hook, out,
-            accumulate)
+        combined_x, event, hook = deep_ep_cpp.low_latency_combine(
+            self.runtime, x, topk_idx, topk_weights, handle, combine_wait_recv_cost_stats, zero_copy, async_finish,
+            return_recv_hook, out, accumulate)
         if prof:
             prof.mark("end")
             prof.finish_iter()
-        return combined_x, EventOverlap(event or EventHandle.deferred()), hook
+        return combined_x, EventOverlap(event), hook
 
     def low_latency_update_mask_buffer(self, rank_to_mask: int, mask: bool = False) -> None:
         self.runtime.low_latency_update_mask_buffer(rank_to_mask, mask)

@@ -70,6 +70,16 @@ static torch::Tensor empty_on(const torch::Device& device, at::IntArrayRef sizes
     return torch::Tensor(at::detail::empty_cuda(sizes, type, device, std::nullopt));
 }
 
+// The first n rows of a contiguous tensor, made without the dispatcher (narrow() takes 0.8 us).
+static torch::Tensor leading_rows(const torch::Tensor& t, int64_t n) {
+    auto rows = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(t.storage()), t.key_set(), t.dtype());
+    c10::SmallVector<int64_t, 4> sizes(t.sizes().begin(), t.sizes().end());
+    sizes[0] = n;
+    rows.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+    rows.unsafeGetTensorImpl()->set_storage_offset(t.storage_offset());
+    return rows;
+}
+
 // Several results of one call in one allocation.  A torch::empty costs the host 1.2 us and a tensor over a piece
 // of storage that exists 0.1 us, so a call with many small results asks the allocator once.
 struct ResultBlock {
@@ -181,24 +191,24 @@ struct EventHandle {
 
     // The handle of a call that was not asked to be asynchronous.  Its work is ordered on the caller's stream
     // already, so a wait from that stream is no wait; recording a HIP event for it costs the host 5 us a call
-    // (a decode step with two of them: 20 us against 9.7 without), more than the launch.  It is recorded only
-    // when another stream waits, and then covers the call and whatever that stream was given since.
+    // (a decode step with two of them: 20 us against 9.7 without), more than the launch.  It is recorded when
+    // another stream waits, and then covers the call and whatever that stream was given since; nothing is kept,
+    // so one handle stands for every such call on its stream.
     // A stream made outside PyTorch may be gone by then, so there the event is recorded at once.
-    static EventHandle deferred() {
-        auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
-        const bool external = stream.id() != 0 and (stream.id() & 1) == 0;  // c10: pool streams have odd ids
-        return external ? EventHandle(stream) : EventHandle(stream, Deferred{});
+    static bool can_defer(const HostStream& stream) {  // c10: the default stream is 0, pool streams have odd ids
+        return stream.id() == 0 or (stream.id() & 1) != 0;
     }
 
-    void stream_wait_for(const HostStream& waiter) {
-        if (event == nullptr) {
-            if (waiter == origin.value()) return;
-            event = std::make_shared<torch::Event>(torch::kCUDA);
-            event->record(origin.value());
+    void stream_wait_for(const HostStream& waiter) const {
+        if (event != nullptr) {
+            waiter.unwrap().wait(*event);
+        } else if (waiter != origin.value()) {
+            torch::Event now(torch::kCUDA);
+            now.record(origin.value());
+            waiter.unwrap().wait(now);
         }
-        waiter.unwrap().wait(*event);
     }
-    void current_stream_wait() { stream_wait_for(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
+    void current_stream_wait() const { stream_wait_for(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
 };
 
 static void stream_wait(const HostStream& waiter, const HostStream& other) {
@@ -208,7 +218,7 @@ static void stream_wait(const HostStream& waiter, const HostStream& other) {
     waiter.unwrap().wait(ev);
 }
 
-static void stream_wait(const HostStream& waiter, EventHandle& event) { event.stream_wait_for(waiter); }
+static void stream_wait(const HostStream& waiter, const EventHandle& event) { event.stream_wait_for(waiter); }
 
 // ---------------------------------------------------------------------------
 // Low-latency tensors of one shape (reference: the Python-side cache of
@@ -220,6 +230,8 @@ struct LowLatencyCache {
     torch::Tensor packed_recv_x, packed_recv_scales, packed_recv_count, packed_recv_src_info, packed_recv_layout_range;
     torch::Tensor combine_staging, combine_send_slots, combined_x;
     bool dispatched = false;
+    // What Buffer.low_latency_dispatch returns of it, as the Python objects: ((recv_x, scales) or recv_x, the handle)
+    pybind11::object recv_result, handle_result;
 };
 
 static int row_format_of(bool use_fp8, bool round_scale, bool use_ue8m0) {
@@ -252,6 +264,8 @@ struct Buffer {
     // kernels sized for a balanced world walk such a batch in a slow loop.
     at::DataPtr observed_memory;
     std::atomic<uint64_t>* observed = nullptr;
+    std::optional<HostStream> event_stream;  // the stream that event_of_stream stands for
+    pybind11::object event_of_stream;
     // loopback world
     std::optional<torch::Tensor> world_x, world_topk_idx;
     torch::Tensor ranks_below, ranks_above, peer_workspace;
@@ -537,13 +551,11 @@ struct Buffer {
         }
     }
 
-    std::tuple<torch::Tensor, std::optional<torch::Tensor>, torch::Tensor, torch::Tensor, torch::Tensor,
-               std::optional<EventHandle>, std::optional<std::function<void()>>>
-    low_latency_dispatch(const torch::Tensor& x, const torch::Tensor& topk_idx,
-                         const std::optional<torch::Tensor>& cumulative_local_expert_recv_stats,
-                         const std::optional<torch::Tensor>& dispatch_wait_recv_cost_stats,
-                         int num_max_dispatch_tokens_per_rank, int num_experts, bool use_fp8, bool round_scale,
-                         bool use_ue8m0, bool async, bool return_recv_hook) {
+    LowLatencyCache& run_low_latency_dispatch(const torch::Tensor& x, const torch::Tensor& topk_idx,
+                                              const torch::Tensor* cumulative_local_expert_recv_stats,
+                                              const torch::Tensor* dispatch_wait_recv_cost_stats,
+                                              int num_max_dispatch_tokens_per_rank, int num_experts, bool use_fp8,
+                                              bool round_scale, bool use_ue8m0) {
         EP_HOST_ASSERT(low_latency_mode);
         // reference checks: csrc/deep_ep.cpp:1674-1693
         EP_HOST_ASSERT(x.dim() == 2 and x.is_contiguous() and x.scalar_type() == torch::kBFloat16);
@@ -555,13 +567,13 @@ struct Buffer {
         EP_HOST_ASSERT(num_experts % num_ranks == 0);
         EP_HOST_ASSERT(not use_ue8m0 or round_scale);
         EP_HOST_ASSERT(not use_ue8m0 or (x.size(1) / 128) % 4 == 0);
-        if (cumulative_local_expert_recv_stats.has_value()) {
+        if (cumulative_local_expert_recv_stats != nullptr) {
             EP_HOST_ASSERT(cumulative_local_expert_recv_stats->scalar_type() == torch::kInt);
             EP_HOST_ASSERT(cumulative_local_expert_recv_stats->dim() == 1 and
                            cumulative_local_expert_recv_stats->is_contiguous());
             EP_HOST_ASSERT(cumulative_local_expert_recv_stats->size(0) == num_experts / num_ranks);
         }
-        if (dispatch_wait_recv_cost_stats.has_value()) {
+        if (dispatch_wait_recv_cost_stats != nullptr) {
             EP_HOST_ASSERT(dispatch_wait_recv_cost_stats->scalar_type() == torch::kInt64);
             EP_HOST_ASSERT(dispatch_wait_recv_cost_stats->dim() == 1 and dispatch_wait_recv_cost_stats->is_contiguous());
             EP_HOST_ASSERT(dispatch_wait_recv_cost_stats->size(0) == num_ranks);
@@ -587,11 +599,25 @@ struct Buffer {
             c.packed_recv_x.data_ptr(), c.packed_recv_scales.defined() ? c.packed_recv_scales.data_ptr() : nullptr,
             c.packed_recv_src_info.data_ptr<int>(), c.packed_recv_layout_range.data_ptr<int64_t>(),
             c.packed_recv_count.data_ptr<int>(),
-            cumulative_local_expert_recv_stats.has_value() ? cumulative_local_expert_recv_stats->data_ptr<int>() : nullptr,
+            cumulative_local_expert_recv_stats != nullptr ? cumulative_local_expert_recv_stats->data_ptr<int>() : nullptr,
             rows_expected(num_tokens, num_topk, num_experts, num_max_dispatch_tokens_per_rank), c.workspace.data_ptr(),
             size_t(c.workspace.numel()), c.segment_workspace.data_ptr(), size_t(c.segment_workspace.numel()),
             capturing ? nullptr : reinterpret_cast<uint64_t*>(observed), stream));
         c.dispatched = true;
+        return c;
+    }
+
+    std::tuple<torch::Tensor, std::optional<torch::Tensor>, torch::Tensor, torch::Tensor, torch::Tensor,
+               std::optional<EventHandle>, std::optional<std::function<void()>>>
+    low_latency_dispatch(const torch::Tensor& x, const torch::Tensor& topk_idx,
+                         const std::optional<torch::Tensor>& cumulative_local_expert_recv_stats,
+                         const std::optional<torch::Tensor>& dispatch_wait_recv_cost_stats,
+                         int num_max_dispatch_tokens_per_rank, int num_experts, bool use_fp8, bool round_scale,
+                         bool use_ue8m0, bool async, bool return_recv_hook) {
+        auto given = [](const std::optional<torch::Tensor>& t) { return t.has_value() ? &t.value() : nullptr; };
+        auto& c = run_low_latency_dispatch(x, topk_idx, given(cumulative_local_expert_recv_stats),
+                                           given(dispatch_wait_recv_cost_stats), num_max_dispatch_tokens_per_rank,
+                                           num_experts, use_fp8, round_scale, use_ue8m0);
         std::optional<EventHandle> event;
         if (async) event = EventHandle();
         std::optional<std::function<void()>> hook;
@@ -602,16 +628,15 @@ struct Buffer {
                 event, hook};
     }
 
-    std::tuple<torch::Tensor, std::optional<EventHandle>, std::optional<std::function<void()>>> low_latency_combine(
-        const torch::Tensor& x, const torch::Tensor& topk_idx, const torch::Tensor& topk_weights,
-        const torch::Tensor& src_info, const torch::Tensor& layout_range,
-        const std::optional<torch::Tensor>& combine_wait_recv_cost_stats, int num_max_dispatch_tokens_per_rank,
-        int num_experts, bool use_logfmt, bool zero_copy, bool async, bool return_recv_hook,
-        const std::optional<torch::Tensor>& out, bool accumulate) {
-        (void)use_logfmt;
+    torch::Tensor run_low_latency_combine(const torch::Tensor& x, const torch::Tensor& topk_idx,
+                                          const torch::Tensor& topk_weights, const torch::Tensor& src_info,
+                                          const torch::Tensor& layout_range,
+                                          const torch::Tensor* combine_wait_recv_cost_stats,
+                                          int num_max_dispatch_tokens_per_rank, int num_experts, bool zero_copy,
+                                          const torch::Tensor* out, bool accumulate) {
         // accumulate: the sum starts from what `out` holds (the reference has the flag on its reduce binding,
         // csrc/deep_ep.cpp:3850-3857, kernel csrc/kernels/coop_combine_recv.cuh:174-179)
-        EP_HOST_ASSERT(not accumulate or out.has_value());
+        EP_HOST_ASSERT(not accumulate or out != nullptr);
         EP_HOST_ASSERT(low_latency_mode);
         // reference checks: csrc/deep_ep.cpp:1816-1837
         EP_HOST_ASSERT(x.dim() == 3 and x.is_contiguous() and x.scalar_type() == torch::kBFloat16);
@@ -629,7 +654,7 @@ struct Buffer {
         EP_HOST_ASSERT(layout_range.dim() == 2 and layout_range.is_contiguous());
         EP_HOST_ASSERT(layout_range.scalar_type() == torch::kInt64);
         EP_HOST_ASSERT(layout_range.size(0) == num_experts / num_ranks and layout_range.size(1) == num_ranks);
-        if (combine_wait_recv_cost_stats.has_value()) {
+        if (combine_wait_recv_cost_stats != nullptr) {
             EP_HOST_ASSERT(combine_wait_recv_cost_stats->scalar_type() == torch::kInt64);
             EP_HOST_ASSERT(combine_wait_recv_cost_stats->dim() == 1 and combine_wait_recv_cost_stats->is_contiguous());
             EP_HOST_ASSERT(combine_wait_recv_cost_stats->size(0) == num_ranks);
@@ -643,22 +668,22 @@ struct Buffer {
         auto& c = ll;
         auto stream = current_stream();
 
-        torch::Tensor src = x;
+        const torch::Tensor* src = &x;
         // zero_copy: the caller wrote its expert outputs into the buffer handed out earlier, and that buffer is
         // what the transport sends from (the ranges of layout_range are contiguous in it), so the combine skips
         // the row return -- "the next combine kernel can skip the copying", deep_ep/buffer.py:2831-2852
         if (zero_copy) {
             EP_HOST_ASSERT(!combine_input_buffers.empty() and combine_input_buffers[combine_buffer_idx].defined());
-            src = combine_input_buffers[combine_buffer_idx];
-            EP_HOST_ASSERT(src.size(0) == x.size(0) and src.size(1) == x.size(1) and src.size(2) == x.size(2));
+            src = &combine_input_buffers[combine_buffer_idx];
+            EP_HOST_ASSERT(src->size(0) == x.size(0) and src->size(1) == x.size(1) and src->size(2) == x.size(2));
         }
         torch::Tensor combined_x;
-        if (out.has_value()) {
+        if (out != nullptr) {
             EP_HOST_ASSERT(out->dim() == 2 and out->is_contiguous() and out->scalar_type() == torch::kBFloat16);
             EP_HOST_ASSERT(out->size(0) == num_combined_tokens and out->size(1) == hidden);
-            combined_x = out.value();
+            combined_x = *out;
         } else {
-            combined_x = c.combined_x.narrow(0, 0, num_combined_tokens);
+            combined_x = leading_rows(c.combined_x, num_combined_tokens);
         }
 
         if (world_x.has_value())  // what the remote experts would have returned
@@ -667,7 +692,7 @@ struct Buffer {
                                                          c.row_format, combine_peer_mode, combine_peer_seed,
                                                          c.combine_staging.data_ptr(), stream));
         // row return and weighted reduce in one call (one kernel launch for decode-sized batches)
-        abi_check(deepep_ll_combine(src.data_ptr(), layout_range.data_ptr<int64_t>(), topk_idx.data_ptr<int64_t>(),
+        abi_check(deepep_ll_combine(src->data_ptr(), layout_range.data_ptr<int64_t>(), topk_idx.data_ptr<int64_t>(),
                                     topk_weights.data_ptr<float>(), c.pair_slot.data_ptr<int>(), num_combined_tokens,
                                     hidden, num_topk, num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank,
                                     accumulate ? 1 : 0, c.combine_staging.data_ptr(),
@@ -677,6 +702,20 @@ struct Buffer {
                                                   num_max_dispatch_tokens_per_rank),
                                     c.segment_workspace.data_ptr(), size_t(c.segment_workspace.numel()), stream));
 
+        return combined_x;
+    }
+
+    std::tuple<torch::Tensor, std::optional<EventHandle>, std::optional<std::function<void()>>> low_latency_combine(
+        const torch::Tensor& x, const torch::Tensor& topk_idx, const torch::Tensor& topk_weights,
+        const torch::Tensor& src_info, const torch::Tensor& layout_range,
+        const std::optional<torch::Tensor>& combine_wait_recv_cost_stats, int num_max_dispatch_tokens_per_rank,
+        int num_experts, bool use_logfmt, bool zero_copy, bool async, bool return_recv_hook,
+        const std::optional<torch::Tensor>& out, bool accumulate) {
+        (void)use_logfmt;
+        auto given = [](const std::optional<torch::Tensor>& t) { return t.has_value() ? &t.value() : nullptr; };
+        auto combined_x = run_low_latency_combine(x, topk_idx, topk_weights, src_info, layout_range,
+                                                  given(combine_wait_recv_cost_stats), num_max_dispatch_tokens_per_rank,
+                                                  num_experts, zero_copy, given(out), accumulate);
         std::optional<EventHandle> event;
         if (async) event = EventHandle();
         std::optional<std::function<void()>> hook;
@@ -704,6 +743,17 @@ struct Buffer {
             if (b.defined()) b.zero_();
         if (ll.recv_count.defined()) ll.recv_count.zero_();
         ll.dispatched = false;
+    }
+
+    // The event that Buffer's Python methods hand back.
+    pybind11::object returned_event(bool async) {
+        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
+        if (async or not EventHandle::can_defer(stream)) return pybind11::cast(EventHandle(stream));
+        if (!event_stream.has_value() or event_stream.value() != stream) {
+            event_of_stream = pybind11::cast(EventHandle(stream, EventHandle::Deferred{}));
+            event_stream = stream;
+        }
+        return event_of_stream;
     }
 
     void ensure_mask() {
@@ -1195,6 +1245,106 @@ static std::tuple<torch::Tensor, std::optional<torch::Tensor>> pack_rows(const t
     return {out, out_scales};
 }
 
+// ---------------------------------------------------------------------------
+// The two calls of a decode step as plain C functions for Buffer's Python methods: the arguments come in by
+// position and the results are handed over as Python objects that live as long as the tensors behind them.  Through
+// pybind11, with an event object and a view made for every call, the two cost the host 3 us more.
+// ---------------------------------------------------------------------------
+static const torch::Tensor& tensor_argument(PyObject* v) {
+    if (!THPVariable_Check(v)) throw pybind11::type_error("a torch.Tensor was expected");
+    return THPVariable_Unpack(v);
+}
+static const torch::Tensor* optional_tensor_argument(PyObject* v) { return v == Py_None ? nullptr : &tensor_argument(v); }
+static int int_argument(PyObject* v) {
+    const long n = PyLong_AsLong(v);
+    if (n == -1 and PyErr_Occurred()) throw pybind11::error_already_set();
+    if (n != int(n)) throw pybind11::value_error("an argument is out of range");
+    return int(n);
+}
+static bool bool_argument(PyObject* v) {
+    const int b = PyObject_IsTrue(v);
+    if (b < 0) throw pybind11::error_already_set();
+    return b != 0;
+}
+static pybind11::object tensor_object(const torch::Tensor& t) {
+    PyObject* v = THPVariable_Wrap(t);
+    if (v == nullptr) throw pybind11::error_already_set();
+    return pybind11::reinterpret_steal<pybind11::object>(v);
+}
+static pybind11::object hook_object(bool wanted) {
+    if (!wanted) return pybind11::none();
+    return pybind11::cpp_function([] {});
+}
+
+// Runs f and turns what it throws into the Python error that pybind11 would raise.
+template <typename F>
+static PyObject* as_python_call(Py_ssize_t got, Py_ssize_t wanted, F&& f) {
+    static const pybind11::handle ep_exception =
+        pybind11::object(pybind11::module_::import("deepep_efa_amd.deep_ep_cpp").attr("EPException")).release();
+    try {
+        if (got != wanted) throw pybind11::type_error("wrong number of arguments");
+        return f().release().ptr();
+    } catch (pybind11::error_already_set& e) {
+        e.restore();
+    } catch (const pybind11::builtin_exception& e) {
+        e.set_error();
+    } catch (const EPException& e) {
+        PyErr_SetString(ep_exception.ptr(), e.what());
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+
+// (buffer, x, topk_idx, stats, wait stats, max tokens, experts, use_fp8, round_scale, use_ue8m0, async, hook)
+//   -> (recv_x, recv_count, handle, event, hook)
+static PyObject* low_latency_dispatch_call(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return as_python_call(n, 12, [&] {
+        Buffer& buffer = pybind11::handle(a[0]).cast<Buffer&>();
+        const bool use_fp8 = bool_argument(a[7]);
+        LowLatencyCache& c = buffer.run_low_latency_dispatch(
+            tensor_argument(a[1]), tensor_argument(a[2]), optional_tensor_argument(a[3]), optional_tensor_argument(a[4]),
+            int_argument(a[5]), int_argument(a[6]), use_fp8, bool_argument(a[8]), bool_argument(a[9]));
+        if (!c.handle_result) {
+            c.recv_result = tensor_object(c.packed_recv_x);
+            if (use_fp8) c.recv_result = pybind11::make_tuple(c.recv_result, tensor_object(c.packed_recv_scales));
+            c.handle_result = pybind11::make_tuple(tensor_object(c.packed_recv_src_info),
+                                                   tensor_object(c.packed_recv_layout_range), c.max_tokens, c.hidden,
+                                                   c.num_experts);
+        }
+        const pybind11::object count = tensor_object(c.packed_recv_count), event = buffer.returned_event(bool_argument(a[10])),
+                               hook = hook_object(bool_argument(a[11]));
+        return pybind11::reinterpret_steal<pybind11::object>(
+            PyTuple_Pack(5, c.recv_result.ptr(), count.ptr(), c.handle_result.ptr(), event.ptr(), hook.ptr()));
+    });
+}
+
+// (buffer, x, topk_idx, topk_weights, handle, wait stats, zero_copy, async, hook, out, accumulate)
+//   -> (combined_x, event, hook)
+static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return as_python_call(n, 11, [&] {
+        Buffer& buffer = pybind11::handle(a[0]).cast<Buffer&>();
+        const auto h = pybind11::reinterpret_steal<pybind11::object>(
+            PySequence_Fast(a[4], "the handle of a low_latency_dispatch was expected"));
+        if (!h) throw pybind11::error_already_set();
+        if (PySequence_Fast_GET_SIZE(h.ptr()) != 5) throw pybind11::value_error("a handle has five entries");
+        auto of_handle = [&](int i) { return PySequence_Fast_GET_ITEM(h.ptr(), i); };
+        const pybind11::object combined = tensor_object(buffer.run_low_latency_combine(
+            tensor_argument(a[1]), tensor_argument(a[2]), tensor_argument(a[3]), tensor_argument(of_handle(0)),
+            tensor_argument(of_handle(1)), optional_tensor_argument(a[5]), int_argument(of_handle(2)),
+            int_argument(of_handle(4)), bool_argument(a[6]), optional_tensor_argument(a[9]), bool_argument(a[10])));
+        const pybind11::object event = buffer.returned_event(bool_argument(a[7])), hook = hook_object(bool_argument(a[8]));
+        return pybind11::reinterpret_steal<pybind11::object>(PyTuple_Pack(3, combined.ptr(), event.ptr(), hook.ptr()));
+    });
+}
+
+static PyMethodDef step_calls[] = {
+    {"low_latency_dispatch", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(low_latency_dispatch_call)), METH_FASTCALL,
+     "Buffer.low_latency_dispatch without its wrapper"},
+    {"low_latency_combine", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(low_latency_combine_call)), METH_FASTCALL,
+     "Buffer.low_latency_combine without its wrapper"},
+    {nullptr, nullptr, 0, nullptr}};
+
 static bool is_sm90_compiled() { return true; }  // FP8 paths are always built for gfx950
 
 }  // namespace deep_ep
@@ -1219,7 +1369,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
 
     pybind11::class_<deep_ep::EventHandle>(m, "EventHandle")
         .def(pybind11::init<>())
-        .def_static("deferred", &deep_ep::EventHandle::deferred)
         .def("current_stream_wait", &deep_ep::EventHandle::current_stream_wait);
 
     pybind11::class_<deep_ep::Buffer>(m, "Buffer")
@@ -1252,6 +1401,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("loopback_own_inputs", &deep_ep::Buffer::loopback_own_inputs)
         .def("loopback_world", &deep_ep::Buffer::loopback_world)
         .def("loopback_set_combine_mode", &deep_ep::Buffer::loopback_set_combine_mode);
+
+    if (PyModule_AddFunctions(m.ptr(), deep_ep::step_calls) != 0) throw pybind11::error_already_set();
 
     pybind11::class_<deep_ep::AllToAllCalls>(m, "AllToAllCalls")
         .def(pybind11::init([](int num_ranks, int rank, int num_experts, int max_tokens, int hidden, int num_topk,
