@@ -322,7 +322,7 @@ __global__ __launch_bounds__(kSortChunk) void routing_sort_single_kernel(
 // latency: about three memory round trips.
 // ---------------------------------------------------------------------
 constexpr int kWideSortTokens = 256;    // tokens per workgroup
-constexpr int kWideSortThreads = 1024;  // a byte counter of a thread takes at most 255 tokens: 255 * 1024 in all
+constexpr int kWideSortThreads = 1024;  // 256 where one workgroup has all the tokens
 constexpr int64_t kWideSortMaxBytes = 512 * 1024;
 
 // 1 in every byte of v that is not zero.
@@ -331,12 +331,12 @@ __device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {
     return v & 0x0101010101010101ull;
 }
 
-template <int kWords>  // 8-byte words of a token's row: ranks / 8
-__global__ __launch_bounds__(kWideSortThreads) void routing_sort_wide_kernel(
+template <int kWords, int kThreads>  // 8-byte words of a token's row: ranks / 8
+__global__ __launch_bounds__(kThreads) void routing_sort_wide_kernel(
     const uint64_t* __restrict__ is_token_in_rank, int num_tokens, int32_t* __restrict__ send_counts,
     int64_t* __restrict__ send_cumsum, int64_t* __restrict__ sorted_token_ids, int32_t* __restrict__ row_of_pair,
     int64_t* __restrict__ total_host) {
-    constexpr int kRanks = kWords * 8, kWaves = kWideSortThreads / kWave, kAhead = kWords <= 2 ? 4 : 2;
+    constexpr int kRanks = kWords * 8, kWaves = kThreads / kWave, kAhead = kWords <= 2 ? 4 : 2;
     constexpr int kTokenWaves = kWideSortTokens / kWave, kRankShares = kWaves / kTokenWaves;
     __shared__ int32_t wave_all[kWaves][kRanks], wave_before[kWaves][kRanks];
     __shared__ int32_t start[kRanks];                // where the ids of this workgroup's tokens begin, per rank
@@ -355,18 +355,18 @@ __global__ __launch_bounds__(kWideSortThreads) void routing_sort_wide_kernel(
     uint64_t all[kWords], before[kWords];
 #pragma unroll
     for (int q = 0; q < kWords; ++q) all[q] = before[q] = 0;
-    for (int t0 = tid; t0 < num_tokens; t0 += kAhead * kWideSortThreads) {
+    for (int t0 = tid; t0 < num_tokens; t0 += kAhead * kThreads) {
         uint64_t v[kAhead][kWords];
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) {  // unconditional loads, all in flight together
-            const int t = t0 + u * kWideSortThreads;
+            const int t = t0 + u * kThreads;
 #pragma unroll
             for (int q = 0; q < kWords; ++q)
                 v[u][q] = is_token_in_rank[int64_t(t < num_tokens ? t : num_tokens - 1) * kWords + q];
         }
 #pragma unroll
         for (int u = 0; u < kAhead; ++u) {
-            const int t = t0 + u * kWideSortThreads;
+            const int t = t0 + u * kThreads;
 #pragma unroll
             for (int q = 0; q < kWords; ++q) {
                 const uint64_t one = t < num_tokens ? nonzero_bytes(v[u][q]) : 0;
@@ -476,11 +476,10 @@ __global__ __launch_bounds__(1024) void channel_prefix_kernel(const uint8_t* __r
 }
 
 // The same for a multiple of 8 ranks: one workgroup per 8 of them, so a wave reads the membership of eight ranks
-// with one 8-byte load per token, sixteen of them in flight, and adds the bool bytes up eight at a time.  The
+// with one 8-byte load per token, up to sixteen of them in flight, and adds the bool bytes up eight at a time.  The
 // bytes of a row that eight workgroups used to fetch for themselves are fetched once (12289 tokens, 8 ranks,
 // 10 channels: 8.7 us, two thirds of it waiting for loads).
-constexpr int kChannelAhead = 16;
-
+template <int kAhead>  // loads in flight per lane: 4 for channels of up to 256 tokens, else 16
 __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64_t* __restrict__ is_token_in_rank,
                                                                     int num_tokens, int num_words, int num_channels,
                                                                     int32_t* __restrict__ cpm) {
@@ -493,15 +492,15 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
         int count[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i) count[i] = 0;
-        for (int t0 = begin + lane; t0 - lane < end; t0 += kWave * kChannelAhead) {
-            uint64_t v[kChannelAhead], sum = 0;
+        for (int t0 = begin + lane; t0 - lane < end; t0 += kWave * kAhead) {
+            uint64_t v[kAhead], sum = 0;
 #pragma unroll
-            for (int u = 0; u < kChannelAhead; ++u) {
+            for (int u = 0; u < kAhead; ++u) {
                 const int t = t0 + u * kWave;
                 v[u] = is_token_in_rank[int64_t(t < end ? t : end - 1) * num_words + q];
             }
 #pragma unroll
-            for (int u = 0; u < kChannelAhead; ++u) sum += t0 + u * kWave < end ? nonzero_bytes(v[u]) : 0;
+            for (int u = 0; u < kAhead; ++u) sum += t0 + u * kWave < end ? nonzero_bytes(v[u]) : 0;
 #pragma unroll
             for (int half = 0; half < 2; ++half)  // bytes widened to 16 bits: 64 lanes of at most 16 fit
 #pragma unroll
@@ -692,9 +691,15 @@ int deepep_moe_routing_sort_total(const uint8_t* is_token_in_rank, int num_token
     if (wide) {
         const int blocks = num_tokens == 0 ? 1 : (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
         const uint64_t* rows = reinterpret_cast<const uint64_t*>(is_token_in_rank);
-#define DEEPEP_LAUNCH_SORT(WORDS)                                                                             \
-    routing_sort_wide_kernel<WORDS><<<blocks, kWideSortThreads, 0, s>>>(rows, num_tokens, send_counts, send_cumsum, \
-                                                                        sorted_token_ids, row_of_pair, total_host)
+#define DEEPEP_LAUNCH_SORT(WORDS)                                                                                 \
+    do {                                                                                                          \
+        if (blocks == 1)                                                                                          \
+            routing_sort_wide_kernel<WORDS, kWideSortTokens><<<1, kWideSortTokens, 0, s>>>(                       \
+                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, total_host);           \
+        else                                                                                                      \
+            routing_sort_wide_kernel<WORDS, kWideSortThreads><<<blocks, kWideSortThreads, 0, s>>>(                \
+                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, total_host);           \
+    } while (0)
         switch (num_ranks) {
             case 8: DEEPEP_LAUNCH_SORT(1); break;
             case 16: DEEPEP_LAUNCH_SORT(2); break;
@@ -745,10 +750,14 @@ int deepep_channel_prefix_matrix(const uint8_t* is_token_in_rank, int num_tokens
     // one wave per channel, up to sixteen at a time
     const int threads = num_channels >= 16 ? 1024 : ((num_channels + 3) / 4) * 256;
     if ((num_ranks & 7) == 0 && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 && num_channels <= 1024) {
-        channel_prefix_words_kernel<<<num_ranks / 8, threads, size_t(num_channels) * 32,
-                                      reinterpret_cast<hipStream_t>(stream)>>>(
-            reinterpret_cast<const uint64_t*>(is_token_in_rank), num_tokens, num_ranks / 8, num_channels,
-            channel_prefix_matrix);
+#define DEEPEP_LAUNCH_CHANNELS(AHEAD)                                                                              \
+    channel_prefix_words_kernel<AHEAD><<<num_ranks / 8, threads, size_t(num_channels) * 32,                        \
+                                         reinterpret_cast<hipStream_t>(stream)>>>(                                 \
+        reinterpret_cast<const uint64_t*>(is_token_in_rank), num_tokens, num_ranks / 8, num_channels,              \
+        channel_prefix_matrix)
+        if ((int64_t(num_tokens) + num_channels - 1) / num_channels <= 4 * kWave) DEEPEP_LAUNCH_CHANNELS(4);
+        else DEEPEP_LAUNCH_CHANNELS(16);
+#undef DEEPEP_LAUNCH_CHANNELS
         EP_LAUNCH_CHECK();
         return 0;
     }

@@ -22,7 +22,9 @@ __device__ __forceinline__ int rank_of_row(const int64_t* cumsum, int num_ranks,
 // topk_remap: for every row of the per-rank send list, the token's top-k
 // entries in the expert numbering of the destination rank; entries for
 // other ranks' experts become (-1, 0.0).  One thread per (row, k); the
-// R + 1 prefix lives in LDS.
+// R + 1 prefix lives in LDS.  A short list is a chain of memory round trips and
+// nothing else, so the token's number is asked for before the prefix has come
+// and its weight before its expert has.
 // Reference: csrc/kernels/efa_kernels.cu:339-387.
 // ---------------------------------------------------------------------
 __global__ __launch_bounds__(kMetaThreads) void topk_remap_kernel(
@@ -31,29 +33,32 @@ __global__ __launch_bounds__(kMetaThreads) void topk_remap_kernel(
     int num_topk, int num_ranks, int num_local_experts, int64_t max_send, int64_t* __restrict__ remapped_topk,
     float* __restrict__ remapped_weights) {
     extern __shared__ int64_t cumsum[];  // [R + 1]
+    // rows of a step of the grid; all of max_send's rows have a list entry, valid or not
+    const int64_t step = int64_t(gridDim.x) * kMetaThreads;
+    int64_t idx = int64_t(blockIdx.x) * kMetaThreads + threadIdx.x;
+    auto row_of = [&](int64_t i) { return i < (int64_t(1) << 32) ? int64_t(uint32_t(i) / uint32_t(num_topk)) : i / num_topk; };
+    int64_t row = row_of(idx);
+    int64_t token = row < max_send ? sorted_token_ids[row] : -1;
     for (int r = threadIdx.x; r <= num_ranks; r += kMetaThreads) cumsum[r] = send_cumsum[r];
-    __syncthreads();
+    lds_barrier();
     int64_t total = cumsum[num_ranks];
     if (total > max_send) total = max_send;
     const int64_t work = total * num_topk;
-    for (int64_t idx = int64_t(blockIdx.x) * kMetaThreads + threadIdx.x; idx < work;
-         idx += int64_t(gridDim.x) * kMetaThreads) {
-        const int64_t row = idx / num_topk;
-        const int k = int(idx - row * num_topk);
-        const int dst_rank = rank_of_row(cumsum, num_ranks, row);
-        const int64_t token = sorted_token_ids[row];
+    while (idx < work) {
         int64_t out_e = -1;
         float out_w = 0.0f;
         if (token >= 0 && token < num_tokens) {
-            const int64_t e = topk_idx[token * num_topk + k];
-            const int64_t first = int64_t(dst_rank) * num_local_experts;
-            if (e >= first && e < first + num_local_experts) {
-                out_e = e - first;
-                out_w = topk_weights[token * num_topk + k];
-            }
+            const int64_t at = token * num_topk + (idx - row * num_topk);
+            const int64_t e = topk_idx[at];
+            const float w = topk_weights[at];
+            const int64_t first = int64_t(rank_of_row(cumsum, num_ranks, row)) * num_local_experts;
+            if (e >= first && e < first + num_local_experts) out_e = e - first, out_w = w;
         }
         remapped_topk[idx] = out_e;
         remapped_weights[idx] = out_w;
+        idx += step;
+        row = row_of(idx);
+        token = row < max_send ? sorted_token_ids[row] : -1;
     }
 }
 
@@ -68,7 +73,7 @@ __global__ __launch_bounds__(kMetaThreads) void recv_src_meta_kernel(const int64
                                                                      int64_t max_recv, u32x2* __restrict__ meta) {
     extern __shared__ int64_t cumsum[];  // [R + 1]
     for (int r = threadIdx.x; r <= num_ranks; r += kMetaThreads) cumsum[r] = recv_cumsum[r];
-    __syncthreads();
+    lds_barrier();
     int64_t total = cumsum[num_ranks];
     if (total > max_recv) total = max_recv;
     for (int64_t i = int64_t(blockIdx.x) * kMetaThreads + threadIdx.x; i < total;
@@ -107,7 +112,8 @@ __global__ __launch_bounds__(kMetaThreads) void combine_positions_kernel(
 // accumulated in float32 in that fixed order and rounded once; the top-k
 // weights are added the same way.  One wave = one (token, 1 KiB piece):
 // lane r fetches rank r's membership byte and row index (one round of loads
-// for all ranks), the rows are then loaded eight at a time.
+// for all ranks, neither waiting for the other), the rows and their weights are
+// then loaded eight at a time.
 // Reference: the zero_() + index_add_ of deep_ep/buffer.py:1542-1557, which
 // accumulates in bf16 through atomics in arrival order.
 // ---------------------------------------------------------------------
@@ -136,13 +142,15 @@ __global__ __launch_bounds__(kMetaThreads) void combine_reduce_kernel(
     for (int r0 = 0; r0 < num_ranks; r0 += kWave) {
         const int r = r0 + lane;
         int64_t my_row = -1;
-        if (r < num_ranks && is_token_in_rank[int64_t(t) * num_ranks + r] != 0) {
-            my_row = row_of_pair[int64_t(t) * num_ranks + r];
-            if (my_row < 0 || my_row >= max_rows) my_row = -1;
+        if (r < num_ranks) {
+            const uint8_t member = is_token_in_rank[int64_t(t) * num_ranks + r];
+            my_row = row_of_pair[int64_t(t) * num_ranks + r];  // means nothing for a rank the token is not sent to
+            if (member == 0 || my_row < 0 || my_row >= max_rows) my_row = -1;
         }
         uint64_t present = __ballot(my_row >= 0);
         while (present != 0) {
             u32x4 v[8];
+            float wv[8];
             int rows[8];
             int n = 0;
 #pragma unroll
@@ -153,6 +161,7 @@ __global__ __launch_bounds__(kMetaThreads) void combine_reduce_kernel(
                     present &= present - 1;
                     rows[u] = __builtin_amdgcn_readlane(int(my_row), src_lane);
                     if (lane_live) v[u] = load_u32x4<kStream>(recv_x + int64_t(rows[u]) * row_bytes + off);
+                    if (weights_here && lane < num_topk) wv[u] = recv_w[int64_t(rows[u]) * num_topk + lane];
                     n = u + 1;
                 }
             }
@@ -166,7 +175,7 @@ __global__ __launch_bounds__(kMetaThreads) void combine_reduce_kernel(
                         acc[2 * i + 1] += bf16_hi(v[u][i]);
                     }
                 }
-                if (weights_here && lane < num_topk) w_acc += recv_w[int64_t(rows[u]) * num_topk + lane];
+                if (weights_here && lane < num_topk) w_acc += wv[u];
             }
         }
     }
