@@ -166,8 +166,9 @@ class Buffer:
                             allocate_on_comm_stream: bool = False):
         """Returns (num_tokens_per_rank [R] int32, num_tokens_per_rdma_rank [R/8] int32 or None,
         num_tokens_per_expert [E] int32, is_token_in_rank [T, R] bool, EventOverlap)."""
-        per_rank, per_rdma, per_expert, is_in, event = self.runtime.get_dispatch_layout(
-            topk_idx, num_experts, getattr(previous_event, "event", None), async_finish, allocate_on_comm_stream)
+        per_rank, per_rdma, per_expert, is_in, event = deep_ep_cpp.get_dispatch_layout(
+            self.runtime, topk_idx, num_experts, getattr(previous_event, "event", None), async_finish,
+            allocate_on_comm_stream)
         return per_rank, per_rdma, per_expert, is_in, EventOverlap(event)
 
     # -- loopback world -------------------------------------------------------------

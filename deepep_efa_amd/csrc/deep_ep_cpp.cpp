@@ -905,8 +905,11 @@ static std::tuple<torch::Tensor, torch::Tensor> topk_remap(const torch::Tensor& 
     EP_HOST_ASSERT(send_cumsum.numel() == num_ranks + 1);
     EP_HOST_ASSERT(total_send >= 0 and total_send <= sorted_token_ids.numel());
     const int num_topk = static_cast<int>(topk_idx.size(1));
-    auto remapped_topk = empty_on(topk_idx.device(), {total_send, num_topk}, torch::kInt64);
-    auto remapped_weights = empty_on(topk_weights.device(), {total_send, num_topk}, torch::kFloat32);
+    ResultBlock b;
+    const int64_t topk_at = b.reserve(8 * total_send * num_topk), weights_at = b.reserve(4 * total_send * num_topk);
+    b.allocate(topk_idx.device());
+    auto remapped_topk = b.take(topk_at, {total_send, num_topk}, torch::kInt64);
+    auto remapped_weights = b.take(weights_at, {total_send, num_topk}, torch::kFloat32);
     abi_check(deepep_topk_remap(topk_idx.data_ptr<int64_t>(), topk_weights.data_ptr<float>(),
                                 sorted_token_ids.data_ptr<int64_t>(), send_cumsum.data_ptr<int64_t>(),
                                 static_cast<int>(topk_idx.size(0)), num_topk, num_ranks, num_local_experts, total_send,
@@ -1246,18 +1249,24 @@ static std::tuple<torch::Tensor, std::optional<torch::Tensor>> pack_rows(const t
 }
 
 // ---------------------------------------------------------------------------
-// The two calls of a decode step as plain C functions for Buffer's Python methods: the arguments come in by
-// position and the results are handed over as Python objects that live as long as the tensors behind them.  Through
-// pybind11, with an event object and a view made for every call, the two cost the host 3 us more.
+// The calls a step makes as plain C functions (METH_FASTCALL) for the Python methods around them: arguments by
+// position, converted one by one.  pybind11's dispatcher takes 0.3 to 0.5 us of host time a call more, of the 4 to 5
+// that a call with its launch takes, and small steps are bound by that.
 // ---------------------------------------------------------------------------
+static PyObject* ep_exception_type = nullptr;  // set when the module is made
+
 static const torch::Tensor& tensor_argument(PyObject* v) {
     if (!THPVariable_Check(v)) throw pybind11::type_error("a torch.Tensor was expected");
     return THPVariable_Unpack(v);
 }
 static const torch::Tensor* optional_tensor_argument(PyObject* v) { return v == Py_None ? nullptr : &tensor_argument(v); }
-static int int_argument(PyObject* v) {
-    const long n = PyLong_AsLong(v);
+static int64_t int64_argument(PyObject* v) {
+    const int64_t n = PyLong_AsLongLong(v);
     if (n == -1 and PyErr_Occurred()) throw pybind11::error_already_set();
+    return n;
+}
+static int int_argument(PyObject* v) {
+    const int64_t n = int64_argument(v);
     if (n != int(n)) throw pybind11::value_error("an argument is out of range");
     return int(n);
 }
@@ -1266,21 +1275,79 @@ static bool bool_argument(PyObject* v) {
     if (b < 0) throw pybind11::error_already_set();
     return b != 0;
 }
-static pybind11::object tensor_object(const torch::Tensor& t) {
-    PyObject* v = THPVariable_Wrap(t);
+
+template <typename A>
+struct Argument;
+template <>
+struct Argument<const torch::Tensor&> {
+    const torch::Tensor& value;
+    explicit Argument(PyObject* v) : value(tensor_argument(v)) {}
+};
+template <>
+struct Argument<const std::optional<torch::Tensor>&> {
+    std::optional<torch::Tensor> value;
+    explicit Argument(PyObject* v) {
+        if (v != Py_None) value = tensor_argument(v);
+    }
+};
+template <>
+struct Argument<std::optional<EventHandle>&> {
+    std::optional<EventHandle> value;
+    explicit Argument(PyObject* v) {
+        if (v != Py_None) value = pybind11::handle(v).cast<EventHandle>();
+    }
+};
+template <>
+struct Argument<const pybind11::dict&> {
+    pybind11::dict value;
+    explicit Argument(PyObject* v) : value(pybind11::reinterpret_borrow<pybind11::dict>(v)) {
+        if (!PyDict_Check(v)) throw pybind11::type_error("a dict was expected");
+    }
+};
+template <>
+struct Argument<int> {
+    int value;
+    explicit Argument(PyObject* v) : value(int_argument(v)) {}
+};
+template <>
+struct Argument<int64_t> {
+    int64_t value;
+    explicit Argument(PyObject* v) : value(int64_argument(v)) {}
+};
+template <>
+struct Argument<bool> {
+    bool value;
+    explicit Argument(PyObject* v) : value(bool_argument(v)) {}
+};
+
+static pybind11::object result_object(const torch::Tensor& t) {
+    PyObject* v = THPVariable_Wrap(t);  // None for an undefined one
     if (v == nullptr) throw pybind11::error_already_set();
     return pybind11::reinterpret_steal<pybind11::object>(v);
 }
-static pybind11::object hook_object(bool wanted) {
-    if (!wanted) return pybind11::none();
-    return pybind11::cpp_function([] {});
+static pybind11::object result_object(int64_t n) { return pybind11::int_(n); }
+static pybind11::object result_object(const EventHandle& e) { return pybind11::cast(e); }
+static pybind11::object result_object(const pybind11::dict& d) { return d; }
+template <typename T>
+static pybind11::object result_object(const std::optional<T>& v) {
+    if (!v.has_value()) return pybind11::none();
+    return result_object(*v);
+}
+template <typename... T>
+static pybind11::object result_object(const std::tuple<T...>& v) {
+    return std::apply(
+        [](const T&... item) {
+            pybind11::tuple out(sizeof...(T));
+            Py_ssize_t i = 0;
+            (PyTuple_SET_ITEM(out.ptr(), i++, result_object(item).release().ptr()), ...);
+            return pybind11::object(std::move(out));
+        },
+        v);
 }
 
 // Runs f and turns what it throws into the Python error that pybind11 would raise.
 template <typename F>
 static PyObject* as_python_call(Py_ssize_t got, Py_ssize_t wanted, F&& f) {
-    static const pybind11::handle ep_exception =
-        pybind11::object(pybind11::module_::import("deepep_efa_amd.deep_ep_cpp").attr("EPException")).release();
     try {
         if (got != wanted) throw pybind11::type_error("wrong number of arguments");
         return f().release().ptr();
@@ -1289,11 +1356,63 @@ static PyObject* as_python_call(Py_ssize_t got, Py_ssize_t wanted, F&& f) {
     } catch (const pybind11::builtin_exception& e) {
         e.set_error();
     } catch (const EPException& e) {
-        PyErr_SetString(ep_exception.ptr(), e.what());
+        PyErr_SetString(ep_exception_type, e.what());
     } catch (const std::exception& e) {
         PyErr_SetString(PyExc_RuntimeError, e.what());
     }
     return nullptr;
+}
+
+// PlainCall<&f>::call is f as a METH_FASTCALL function; a member function takes its object first.
+template <auto F>
+struct PlainCall;
+
+template <typename R, typename... A, R (*F)(A...)>
+struct PlainCall<F> {
+    template <size_t... I>
+    static pybind11::object with(PyObject* const* a, std::index_sequence<I...>) {
+        std::tuple<Argument<A>...> given{Argument<A>(a[I])...};
+        return result_object(F(std::get<I>(given).value...));
+    }
+    static PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n) {
+        return as_python_call(n, sizeof...(A), [&] { return with(a, std::index_sequence_for<A...>()); });
+    }
+};
+
+template <typename C, typename M, typename R, typename... A>
+struct PlainMemberCall {
+    template <M F, size_t... I>
+    static pybind11::object with(PyObject* const* a, std::index_sequence<I...>) {
+        C& self = pybind11::handle(a[0]).cast<C&>();
+        std::tuple<Argument<A>...> given{Argument<A>(a[1 + I])...};
+        if constexpr (std::is_void_v<R>) {
+            (self.*F)(std::get<I>(given).value...);
+            return pybind11::none();
+        } else {
+            return result_object((self.*F)(std::get<I>(given).value...));
+        }
+    }
+    template <M F>
+    static PyObject* run(PyObject* const* a, Py_ssize_t n) {
+        return as_python_call(n, 1 + sizeof...(A), [&] { return with<F>(a, std::index_sequence_for<A...>()); });
+    }
+};
+template <typename C, typename R, typename... A, R (C::*F)(A...)>
+struct PlainCall<F> {
+    static PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n) {
+        return PlainMemberCall<C, R (C::*)(A...), R, A...>::template run<F>(a, n);
+    }
+};
+template <typename C, typename R, typename... A, R (C::*F)(A...) const>
+struct PlainCall<F> {
+    static PyObject* call(PyObject*, PyObject* const* a, Py_ssize_t n) {
+        return PlainMemberCall<const C, R (C::*)(A...) const, R, A...>::template run<F>(a, n);
+    }
+};
+
+static pybind11::object hook_object(bool wanted) {
+    if (!wanted) return pybind11::none();
+    return pybind11::cpp_function([] {});
 }
 
 // (buffer, x, topk_idx, stats, wait stats, max tokens, experts, use_fp8, round_scale, use_ue8m0, async, hook)
@@ -1306,13 +1425,13 @@ static PyObject* low_latency_dispatch_call(PyObject*, PyObject* const* a, Py_ssi
             tensor_argument(a[1]), tensor_argument(a[2]), optional_tensor_argument(a[3]), optional_tensor_argument(a[4]),
             int_argument(a[5]), int_argument(a[6]), use_fp8, bool_argument(a[8]), bool_argument(a[9]));
         if (!c.handle_result) {
-            c.recv_result = tensor_object(c.packed_recv_x);
-            if (use_fp8) c.recv_result = pybind11::make_tuple(c.recv_result, tensor_object(c.packed_recv_scales));
-            c.handle_result = pybind11::make_tuple(tensor_object(c.packed_recv_src_info),
-                                                   tensor_object(c.packed_recv_layout_range), c.max_tokens, c.hidden,
+            c.recv_result = result_object(c.packed_recv_x);
+            if (use_fp8) c.recv_result = pybind11::make_tuple(c.recv_result, result_object(c.packed_recv_scales));
+            c.handle_result = pybind11::make_tuple(result_object(c.packed_recv_src_info),
+                                                   result_object(c.packed_recv_layout_range), c.max_tokens, c.hidden,
                                                    c.num_experts);
         }
-        const pybind11::object count = tensor_object(c.packed_recv_count), event = buffer.returned_event(bool_argument(a[10])),
+        const pybind11::object count = result_object(c.packed_recv_count), event = buffer.returned_event(bool_argument(a[10])),
                                hook = hook_object(bool_argument(a[11]));
         return pybind11::reinterpret_steal<pybind11::object>(
             PyTuple_Pack(5, c.recv_result.ptr(), count.ptr(), c.handle_result.ptr(), event.ptr(), hook.ptr()));
@@ -1329,7 +1448,7 @@ static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssiz
         if (!h) throw pybind11::error_already_set();
         if (PySequence_Fast_GET_SIZE(h.ptr()) != 5) throw pybind11::value_error("a handle has five entries");
         auto of_handle = [&](int i) { return PySequence_Fast_GET_ITEM(h.ptr(), i); };
-        const pybind11::object combined = tensor_object(buffer.run_low_latency_combine(
+        const pybind11::object combined = result_object(buffer.run_low_latency_combine(
             tensor_argument(a[1]), tensor_argument(a[2]), tensor_argument(a[3]), tensor_argument(of_handle(0)),
             tensor_argument(of_handle(1)), optional_tensor_argument(a[5]), int_argument(of_handle(2)),
             int_argument(of_handle(4)), bool_argument(a[6]), optional_tensor_argument(a[9]), bool_argument(a[10])));
@@ -1338,11 +1457,34 @@ static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssiz
     });
 }
 
-static PyMethodDef step_calls[] = {
-    {"low_latency_dispatch", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(low_latency_dispatch_call)), METH_FASTCALL,
-     "Buffer.low_latency_dispatch without its wrapper"},
-    {"low_latency_combine", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(low_latency_combine_call)), METH_FASTCALL,
-     "Buffer.low_latency_combine without its wrapper"},
+static PyMethodDef plain(const char* name, PyObject* (*f)(PyObject*, PyObject* const*, Py_ssize_t), const char* doc) {
+    return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(f)), METH_FASTCALL, doc};
+}
+static PyMethodDef plain_calls[] = {
+    plain("low_latency_dispatch", low_latency_dispatch_call, "Buffer.low_latency_dispatch without its wrapper"),
+    plain("low_latency_combine", low_latency_combine_call, "Buffer.low_latency_combine without its wrapper"),
+    plain("get_dispatch_layout", PlainCall<&Buffer::get_dispatch_layout>::call, "Buffer.get_dispatch_layout without its wrapper"),
+    plain("per_token_cast_to_fp8", PlainCall<&per_token_cast_to_fp8>::call,
+          "Per-token FP8 e4m3 quantisation with 128-channel groups"),
+    plain("moe_routing_sort", PlainCall<&moe_routing_sort>::call, "Token ids grouped by destination rank"),
+    plain("moe_routing_sort_with_positions", PlainCall<&moe_routing_sort_with_positions>::call,
+          "moe_routing_sort plus row_of_pair [T, R], the inverse of the list"),
+    plain("channel_prefix_matrix", PlainCall<&channel_prefix_matrix>::call,
+          "Per-rank prefix of token counts over channels"),
+    plain("pack_rows", PlainCall<&pack_rows>::call, "Gather rows into per-rank contiguous send buffers"),
+    plain("topk_remap", PlainCall<&topk_remap>::call,
+          "Top-k of the send rows in the destination rank's expert numbering"),
+    plain("build_recv_src_meta", PlainCall<&build_recv_src_meta>::call, "Source-rank metadata of the received rows"),
+    plain("combine_reduce_call", PlainCall<&combine_reduce>::call, "combine_reduce with every argument given"),
+    plain("ll_exchange_metadata", PlainCall<&ll_exchange_metadata>::call,
+          "Send/receive counts, combine offsets and per-row records from the gathered route counts"),
+    plain("exchange_metadata_dict", PlainCall<&exchange_metadata_dict>::call, "The same by name"),
+    plain("a2a_dispatch_send", PlainCall<&AllToAllCalls::dispatch_send>::call, "AllToAllState.dispatch_send"),
+    plain("a2a_dispatch_recv_ordered", PlainCall<&AllToAllCalls::dispatch_recv_ordered>::call,
+          "AllToAllState.dispatch_recv_ordered"),
+    plain("a2a_dispatch_recv", PlainCall<&AllToAllCalls::dispatch_recv>::call, "AllToAllState.dispatch_recv"),
+    plain("a2a_combine_send", PlainCall<&AllToAllCalls::combine_send>::call, "AllToAllState.combine_send"),
+    plain("a2a_combine_recv", PlainCall<&AllToAllCalls::combine_recv>::call, "AllToAllState.combine_recv"),
     {nullptr, nullptr, 0, nullptr}};
 
 static bool is_sm90_compiled() { return true; }  // FP8 paths are always built for gfx950
@@ -1352,7 +1494,8 @@ static bool is_sm90_compiled() { return true; }  // FP8 paths are always built f
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "DeepEP dispatch/combine hot path for MI355X (gfx950): host module over libdeepep_hip.so";
 
-    pybind11::register_exception<deep_ep::EPException>(m, "EPException", PyExc_RuntimeError);
+    deep_ep::ep_exception_type =
+        pybind11::register_exception<deep_ep::EPException>(m, "EPException", PyExc_RuntimeError).ptr();
 
     pybind11::class_<deep_ep::Config>(m, "Config")
         .def(pybind11::init<int, int, int, int, int>(), py::arg("num_sms") = 20,
@@ -1402,36 +1545,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         .def("loopback_world", &deep_ep::Buffer::loopback_world)
         .def("loopback_set_combine_mode", &deep_ep::Buffer::loopback_set_combine_mode);
 
-    if (PyModule_AddFunctions(m.ptr(), deep_ep::step_calls) != 0) throw pybind11::error_already_set();
+    if (PyModule_AddFunctions(m.ptr(), deep_ep::plain_calls) != 0) throw pybind11::error_already_set();
 
     pybind11::class_<deep_ep::AllToAllCalls>(m, "AllToAllCalls")
         .def(pybind11::init([](int num_ranks, int rank, int num_experts, int max_tokens, int hidden, int num_topk,
                                int fmt) {
             return deep_ep::AllToAllCalls{num_ranks, rank, num_experts, max_tokens, hidden, num_topk, fmt};
-        }))
-        .def("dispatch_send", &deep_ep::AllToAllCalls::dispatch_send)
-        .def("dispatch_recv_ordered", &deep_ep::AllToAllCalls::dispatch_recv_ordered)
-        .def("dispatch_recv", &deep_ep::AllToAllCalls::dispatch_recv)
-        .def("combine_send", &deep_ep::AllToAllCalls::combine_send)
-        .def("combine_recv", &deep_ep::AllToAllCalls::combine_recv);
-    m.def("exchange_metadata_dict", &deep_ep::exchange_metadata_dict,
-          "Send/receive counts, combine offsets and per-row records by name");
+        }));
 
     m.def("is_sm90_compiled", deep_ep::is_sm90_compiled);
     m.attr("topk_idx_t") = py::reinterpret_borrow<py::object>(
         (PyObject*)torch::getTHPDtype(c10::CppTypeToScalarType<deep_ep::topk_idx_t>::value));
 
-    m.def("per_token_cast_to_fp8", &deep_ep::per_token_cast_to_fp8,
-          "Per-token FP8 e4m3 quantisation with 128-channel groups");
-    m.def("moe_routing_sort", &deep_ep::moe_routing_sort, "Token ids grouped by destination rank");
-    m.def("moe_routing_sort_with_positions", &deep_ep::moe_routing_sort_with_positions,
-          "moe_routing_sort plus row_of_pair [T, R], the inverse of the list");
-    m.def("channel_prefix_matrix", &deep_ep::channel_prefix_matrix, "Per-rank prefix of token counts over channels");
-    m.def("pack_rows", &deep_ep::pack_rows, "Gather rows into per-rank contiguous send buffers");
-    m.def("topk_remap", &deep_ep::topk_remap, "Top-k of the send rows in the destination rank's expert numbering");
-    m.def("build_recv_src_meta", &deep_ep::build_recv_src_meta, "Source-rank metadata of the received rows");
-    m.def("ll_exchange_metadata", &deep_ep::ll_exchange_metadata,
-          "Send/receive counts, combine offsets and per-row records from the gathered route counts");
     m.def("combine_reduce", &deep_ep::combine_reduce, "Per-token sum of the rows that came back (normal-mode combine)",
           py::arg("recv_x"), py::arg("recv_topk_weights"), py::arg("sorted_token_ids"), py::arg("send_cumsum"),
           py::arg("is_token_in_rank"), py::arg("bias_0") = py::none(), py::arg("bias_1") = py::none(),
