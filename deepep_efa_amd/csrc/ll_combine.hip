@@ -309,7 +309,9 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
 // its place in the destination's receive buffer, behind what that rank sent to the
 // ranks below this one (combine_remote_recv_offset,
 // csrc/transport/ll_pipeline.cpp:1283-1295; the reference's peer stores:
-// coop_combine_send.cuh:205-246).  One workgroup per record, one 16-byte vector per thread.
+// coop_combine_send.cuh:205-246).  One workgroup per record, walked like the rows of ll_rows_flat_kernel: HBM
+// bounds it, and neighbouring records are neighbouring rows on both sides.  Against one vector a thread and
+// neighbouring records on eight XCDs: 16376 rows of 14336 bytes 95 -> 77 us (6.1 TB/s), 1024 rows 10.9 -> 7.9 us.
 // ---------------------------------------------------------------------
 struct CombineByDestArgs {
     const uint8_t* x;
@@ -329,19 +331,23 @@ struct CombineByDestArgs {
 };
 
 template <bool kStream>
-__global__ __launch_bounds__(1024) void ll_combine_send_by_dest_kernel(CombineByDestArgs a) {
-    int64_t records = a.num_recv_tokens[1];
-    if (records > a.row_capacity) records = a.row_capacity;
+__global__ __launch_bounds__(512) void ll_combine_send_by_dest_kernel(CombineByDestArgs a) {
     const int lane = lane_id();
     const int64_t row_bytes = int64_t(a.num_vec) * 16;
-    for (int64_t i = blockIdx.x; i < records; i += gridDim.x) {
-        // padded_index[i] is i whenever the records come from deepep_ll_exchange_metadata, so the packed row
-        // is fetched for that guess together with the record itself, and again only if the guess was wrong:
-        // one round trip in front of the row loads instead of two
-        const uint32_t p = a.padded_index[i];
-        int64_t src_row = a.record_packed_row[i];
-        const int64_t offset = a.combine_send_offset[i];
-        if (int64_t(p) >= a.row_capacity) continue;
+    for (int64_t block = blockIdx.x;; block += gridDim.x) {
+        const int64_t i = flat_row_of_block(block);
+        // The record is fetched together with the number of records (both sides of the bound are memory the
+        // tables have), and padded_index[i] is i whenever the records come from deepep_ll_exchange_metadata, so
+        // the packed row is fetched for that guess as well and again only if the guess was wrong: one round trip
+        // in front of the row loads instead of three.
+        const int64_t at = i < a.row_capacity ? i : a.row_capacity - 1;
+        const uint32_t num_records = a.num_recv_tokens[1];
+        const uint32_t p = a.padded_index[at];
+        int64_t src_row = a.record_packed_row[at];
+        const int64_t offset = a.combine_send_offset[at];
+        const int64_t records = int64_t(num_records) < a.row_capacity ? int64_t(num_records) : a.row_capacity;
+        if (block >= flat_rounds_end(records)) break;
+        if (i >= records || int64_t(p) >= a.row_capacity) continue;
         if (int64_t(p) != i) src_row = a.record_packed_row[p];
         if (src_row < 0 || src_row >= a.x_rows) continue;  // the record has no row
         uint8_t* dst;
@@ -355,13 +361,11 @@ __global__ __launch_bounds__(1024) void ll_combine_send_by_dest_kernel(CombineBy
             int part = 0;
             for (int r = lane; r < int(s); r += kWave) part += a.recv_counts[r] < 0 ? 0 : a.recv_counts[r];
             const int64_t j = offset - __builtin_amdgcn_readlane(wave_inclusive_sum(part), kWave - 1);
-            const int64_t at = a.remote_offset[s] + j;
-            if (j < 0 || j >= a.recv_counts[s] || at < 0 || at >= a.peer_rows[s]) continue;
-            dst = a.peer_recv[s] + at * row_bytes;
+            const int64_t at_peer = a.remote_offset[s] + j;
+            if (j < 0 || j >= a.recv_counts[s] || at_peer < 0 || at_peer >= a.peer_rows[s]) continue;
+            dst = a.peer_recv[s] + at_peer * row_bytes;
         }
-        const uint8_t* src = a.x + src_row * row_bytes;
-        for (int v = threadIdx.x; v < a.num_vec; v += blockDim.x)
-            store_u32x4<kStream>(dst + int64_t(v) * 16, load_u32x4<kStream>(src + int64_t(v) * 16));
+        block_copy_row<kStream>(a.x + src_row * row_bytes, dst, a.num_vec, threadIdx.x, blockDim.x);
     }
 }
 
@@ -553,8 +557,7 @@ int deepep_ll_combine_send_by_dest(const void* x, const int32_t* record_packed_r
     a.send_flat = reinterpret_cast<uint8_t*>(send_flat);
     a.peer_recv = reinterpret_cast<uint8_t* const*>(peer_recv_flat), a.peer_rows = peer_recv_rows;
     a.recv_counts = recv_counts, a.remote_offset = combine_remote_recv_offset;
-    int threads = ((a.num_vec + 63) / 64) * 64;
-    if (threads > 1024) threads = 1024;
+    const int threads = flat_row_threads(a.num_vec);
     // grid from the rows expected, not from the capacity (an idle workgroup is not free)
     const int64_t rows = expected_rows > 0 && expected_rows < row_capacity ? expected_rows : row_capacity;
     const unsigned blocks = flat_grid_blocks(rows, row_capacity, num_max_dispatch_tokens_per_rank);

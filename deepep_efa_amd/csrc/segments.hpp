@@ -381,16 +381,36 @@ __device__ __forceinline__ void recv_index_block(const FusedIndexArgs& a, int se
 constexpr int kFlatWindow = 32;
 constexpr int kFlatRound = 8 * kFlatWindow;
 
+__device__ __forceinline__ int64_t flat_row_of_block(int64_t block) {
+    const int in_round = int(block % kFlatRound);
+    return block - in_round + (in_round & 7) * kFlatWindow + (in_round >> 3);
+}
+__device__ __forceinline__ int64_t flat_rounds_end(int64_t rows) {
+    return (rows + kFlatRound - 1) / kFlatRound * kFlatRound;
+}
+
+// Thread `tid` of `threads` moves its vectors of a row, two in flight.
+template <bool kStream>
+__device__ __forceinline__ void block_copy_row(const uint8_t* src, uint8_t* dst, int num_vec, int tid, int threads) {
+    for (int v = tid; v < num_vec; v += 2 * threads) {
+        const bool second = v + threads < num_vec;
+        const u32x4 r0 = load_u32x4<kStream>(src + int64_t(v) * 16);
+        u32x4 r1 = r0;
+        if (second) r1 = load_u32x4<kStream>(src + int64_t(v + threads) * 16);
+        store_u32x4<kStream>(dst + int64_t(v) * 16, r0);
+        if (second) store_u32x4<kStream>(dst + int64_t(v + threads) * 16, r1);
+    }
+}
+
 static __global__ __launch_bounds__(1024) void ll_rows_flat_kernel(
     const int32_t* __restrict__ flat, int num_segments, const RowDesc* __restrict__ desc,
     const uint8_t* __restrict__ src, int64_t src_stride, int num_vec, uint8_t* __restrict__ dst_primary,
     uint8_t* __restrict__ dst_secondary, int64_t dst_stride, int scale_dwords, int64_t src_scale_off,
     uint8_t* __restrict__ scale_dst, int64_t tail_off, int32_t* __restrict__ src_info, int extra_threads) {
     const int total = flat[num_segments];
-    const int rounds_end = (total + kFlatRound - 1) / kFlatRound * kFlatRound;
-    for (int i = blockIdx.x; i < rounds_end; i += gridDim.x) {
-        const int in_round = i % kFlatRound;
-        const int row = i - in_round + (in_round & 7) * kFlatWindow + (in_round >> 3);
+    const int64_t rounds_end = flat_rounds_end(total);
+    for (int64_t i = blockIdx.x; i < rounds_end; i += gridDim.x) {
+        const int64_t row = flat_row_of_block(i);
         if (row >= total) continue;
         const RowDesc d = desc[row];
         if (d.src_row < 0) continue;  // a record that names no row
@@ -406,15 +426,7 @@ static __global__ __launch_bounds__(1024) void ll_rows_flat_kernel(
         // them, those move scales and the source index in the same pass instead of a second one
         const int data_threads = int(blockDim.x) - extra_threads;
         const int tid = threadIdx.x;
-        if (tid < data_threads)
-            for (int v = tid; v < num_vec; v += 2 * data_threads) {
-                const bool second = v + data_threads < num_vec;
-                const u32x4 r0 = load_u32x4<true>(s + int64_t(v) * 16);
-                u32x4 r1 = r0;
-                if (second) r1 = load_u32x4<true>(s + int64_t(v + data_threads) * 16);
-                store_u32x4<true>(o + int64_t(v) * 16, r0);
-                if (second) store_u32x4<true>(o + int64_t(v + data_threads) * 16, r1);
-            }
+        if (tid < data_threads) block_copy_row<true>(s, o, num_vec, tid, data_threads);
         if (extra_threads == 0 || tid >= data_threads) {
             const int t2 = extra_threads > 0 ? tid - data_threads : tid;
             const int step = extra_threads > 0 ? extra_threads : int(blockDim.x);

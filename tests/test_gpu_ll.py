@@ -1523,3 +1523,30 @@ def test_ordered_receive_with_slots_too_small_and_counts_too_large(rt):
                 n1 = int(kept[le, 1])
                 full0 = int(want["packed_recv_layout_range"][le, 0] & 0xFFFFFFFF)
                 assert torch.equal(px[le, n0:n0 + n1], want["packed_recv_x"][le, full0:full0 + n1])
+
+
+@pytest.mark.parametrize("hidden", [128, 1152, 7168, 16512])
+@pytest.mark.parametrize("records", [0, 1, 33, 255, 257, 700])
+def test_return_by_destination_over_record_counts(rt, records, hidden):
+    """Record counts around the windows the rows are walked in, rows below, at and above two vectors a thread, records
+    in another order than the rows, records without a row, and more records than the grid was sized for."""
+    r, e, m = 4, 8, 128
+    capacity = 512 if records > 512 else max(records, 1)
+    g = torch.Generator().manual_seed(records * 7 + hidden)
+    x = torch.randn((e * m, hidden), generator=g).bfloat16().cuda()
+    packed = torch.randperm(e * m, generator=g)[:capacity].int()
+    packed[::5] = -1
+    padded, offset = (torch.randperm(capacity, generator=g).int() for _ in range(2))
+    out = torch.full((capacity, hidden), 3.0, dtype=torch.bfloat16, device="cuda")
+    num = torch.tensor([records, records], dtype=torch.int32, device="cuda")
+    on_gpu = [v.cuda() for v in (packed, padded, offset)]
+    rt.capi.check(rt.capi.load().deepep_ll_combine_send_by_dest(
+        rt.capi.ptr(x), rt.capi.ptr(on_gpu[0]), None, rt.capi.ptr(on_gpu[1]), rt.capi.ptr(on_gpu[2]), rt.capi.ptr(num), capacity,
+        hidden, e, r, m, rt.capi.ptr(out), None, None, None, None, 64, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    want = torch.full((capacity, hidden), 3.0, dtype=torch.bfloat16)
+    for i in range(min(records, capacity)):
+        row = int(packed[int(padded[i])])
+        if row >= 0:
+            want[int(offset[i])] = x[row].cpu()
+    assert torch.equal(out.cpu(), want)
