@@ -497,14 +497,17 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
         if (lane == 0) a.src_info[out_row] = tail_info;
     }
 
-    // The records' packed rows, a pair per wave (the first E_l * R waves of the grid, after their copies).
+    // The records' packed rows, a pair per wave (the last E_l * R copying waves of the grid, which the slack of
+    // its size mostly leaves without a row of their own: 1024 rows 7.6 -> 6.9 us against the first ones, which
+    // did this after their copies).
     // Record of row j of pair (e, s): the records of the lower sources (their whole messages, kept or
     // not), then the source's rows for the lower experts, then j.
     if (a.record_packed_row == nullptr) return;
-    for (int seg = block * waves + w; seg < num_segments; seg += waves_total) {
+    for (int seg = waves_total - 1 - (block * waves + w); seg < num_segments; seg += waves_total) {
         const int le = seg / num_ranks, src = seg - le * num_ranks;
         int lower = 0;  // rows the lower sources sent, all experts
-        for (int q = lane; q < num_local * src; q += kWave) lower += sent[(q / src) * num_ranks + q % src];
+        for (int r = lane; r < src; r += kWave)
+            for (int e2 = 0; e2 < num_local; ++e2) lower += sent[e2 * num_ranks + r];
         const int64_t record0 = int64_t(wave_sum(lower)) + first[seg];
         const int64_t packed0 = int64_t(le) * slots_per_expert +
                                 (wave_segments_prefix(seg_table, seg) - wave_segments_prefix(seg_table, le * num_ranks));
