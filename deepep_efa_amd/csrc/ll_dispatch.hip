@@ -928,6 +928,11 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     const int max_waves = fused_recv != nullptr ? 8 : kSendMaxWaves;
     int waves = items < max_waves ? items : max_waves;
     const int blocks_per_token = (items + waves - 1) / waves;
+    // Every workgroup of the single launch goes through the batch's entries, the send ones for their slots and the
+    // receive ones for the own counts: from some 1500 entries on the eighth wave that a 7168-wide row has no piece
+    // for is worth its place (256 tokens, top-8 15.9 -> 15.1 us, 1024 tokens 40.9 -> 39.6; 128 tokens 8.0 -> 8.1).
+    // Workgroups of four waves stay: with eight, 509 tokens of hidden 4096 took 19.1 us instead of 17.0.
+    if (fused_recv != nullptr && n > 1536 && waves > 4) waves = 8;
     if (fused_recv != nullptr && waves < 4) waves = 4;  // the receive workgroups want a few waves each
     EP_HOST_ASSERT(num_tokens < 65535 && num_src <= 65535);
     // floor(e / E_l) == umulhi(e, ceil(2^32 / E_l)) for every e below 2^16.
@@ -1200,8 +1205,13 @@ static RecvArgs make_recv_args(const void* recv_staging, const int32_t* recv_cou
     ra.recv_count = recv_count;
     ra.hidden = hidden, ra.num_local_experts = num_experts / num_ranks, ra.num_ranks = num_ranks;
     ra.max_tokens = max_tokens, ra.fmt = row_format;
-    ra.parts_log2 = choose_row_parts_log2(estimated_rows(expected_rows, num_experts, max_tokens),
-                                          row_data_bytes(hidden, row_format));
+    const int64_t rows = estimated_rows(expected_rows, num_experts, max_tokens), row_bytes = row_data_bytes(hidden, row_format);
+    ra.parts_log2 = choose_row_parts_log2(rows, row_bytes);
+    // A row of up to 4 KiB is what a wave loads at once (kRecvDepth): with enough rows to occupy the chip a wave
+    // takes it whole, which halves the lookups and the trips of a wave.  The dispatch alone, halves against whole
+    // rows: 1200 x 4096 bytes 7.4 -> 6.8 us, 2400 x 4096 12.0 -> 10.7, 4072 x 4096 17.0 -> 15.8, 2048 x 2048 8.7 ->
+    // 8.0; 1024 x 4096 6.8 both ways; rows of 7168 bytes lose (40.9 -> 43.2), and so does the combine's row return.
+    if (rows > 1024 && row_bytes <= int64_t(kRecvDepth) * kWave * 16) ra.parts_log2 = 0;
     ra.packed_x = reinterpret_cast<uint8_t*>(packed_recv_x);
     ra.packed_scales = reinterpret_cast<uint8_t*>(packed_recv_scales);
     ra.src_info = packed_recv_src_info, ra.layout_range = packed_recv_layout_range;

@@ -150,6 +150,22 @@ def test_dispatch_small_worlds(rt, fmt, r, rank, t, h, k, e, one_call):
     assert torch.equal(st.pair_slot[:t].cpu(), pair_slot)
 
 
+@pytest.mark.parametrize("rows", [1024, 1025])
+@pytest.mark.parametrize("fmt,h", [(O.ROW_BF16, 2048), (O.ROW_BF16, 2176), (O.ROW_FP8, 4096), (O.ROW_FP8, 4224)])
+@pytest.mark.parametrize("t,k", [(192, 8), (193, 8)])
+def test_single_launch_dispatch_around_its_split_bounds(rt, rows, fmt, h, t, k):
+    """Whole and split rows of 4096 bytes and just past it, expected rows and entries (1536) on both sides."""
+    r, rank, e = 4, 2, 32
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + h, drop=20)
+    shape = rt.ll.LLShape(num_ranks=r, rank=rank, num_experts=e, max_tokens=t, hidden=h, num_topk=k, fmt=fmt)
+    st = rt.ll.LowLatencyState(shape)
+    st.expected_rows = rows
+    world = rt.lb.LoopbackWorld(r, rank, seed=0)
+    world.set_inputs(x_all.cuda(), topk_all.cuda())
+    run_dispatch(st, world, *world.own_inputs(), one_call=True)
+    check_dispatch(st, O.ll_dispatch(list(x_all), list(topk_all), rank, e, t, fmt), fmt)
+
+
 @pytest.mark.parametrize("key,rank", [("rank0_ascending", 0), ("rank1_ascending", 1)])
 @ONE_CALL
 @pytest.mark.parametrize("fmt", [O.ROW_BF16, O.ROW_FP8])
