@@ -248,12 +248,20 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, int
 // kStream: the gathered rows exceed what the caches hold, so they are read (and the result written)
 // with the non-temporal hint.  own_x != null: the answers of this rank's own experts are read from
 // the expert-output tensor directly (layout_range says where each own segment begins).
+// index_blocks > 0: that many workgroups in front of the reduce's build the index of the row return that follows
+// (a launch of its own took 3 to 5 us of a large combine).
 template <bool kStream>
-__global__ __launch_bounds__(1024) void ll_combine_recv_kernel(CombineRecvArgs a, const uint8_t* own_x,
-                                                               const int64_t* layout_range, int rank,
-                                                               int num_local_experts, int num_ranks) {
-    extern __shared__ int32_t own_begin[];  // [E_l], with own_x only
-    const int64_t item = int64_t(blockIdx.x) * (blockDim.x >> 6) + wave_in_block();
+__global__ __launch_bounds__(256) void ll_combine_recv_kernel(CombineRecvArgs a, const uint8_t* own_x,
+                                                              const int64_t* layout_range, int rank,
+                                                              int num_local_experts, int num_ranks,
+                                                              CombineIndexArgs index, int index_blocks) {
+    extern __shared__ int32_t own_begin[];  // [E_l], with own_x only; index workgroups: [segments + 1]
+    __shared__ int32_t index_wave_totals[kMaxBlockWaves];
+    if (int(blockIdx.x) < index_blocks) {
+        combine_index_block(index, blockIdx.x, own_begin, index_wave_totals);
+        return;
+    }
+    const int64_t item = (int64_t(blockIdx.x) - index_blocks) * (blockDim.x >> 6) + wave_in_block();
     const CombineSelection sel = combine_load_selection(a, item);  // in flight while the own ranges are fetched
     if (own_x != nullptr) {
         for (int le = threadIdx.x; le < num_local_experts; le += blockDim.x) {
@@ -264,6 +272,12 @@ __global__ __launch_bounds__(1024) void ll_combine_recv_kernel(CombineRecvArgs a
     }
     combine_recv_piece<kStream>(a, item, sel, own_x, own_x != nullptr ? own_begin : nullptr, rank * num_local_experts,
                                 num_local_experts, int64_t(a.max_tokens) * num_ranks);
+}
+
+__global__ __launch_bounds__(256) void ll_combine_index_kernel(CombineIndexArgs index) {
+    extern __shared__ int32_t flat[];  // [segments + 1]
+    __shared__ int32_t wave_totals[kMaxBlockWaves];
+    combine_index_block(index, blockIdx.x, flat, wave_totals);
 }
 
 // ---------------------------------------------------------------------
@@ -435,6 +449,34 @@ using namespace deepep;
 
 extern "C" {
 
+// The index and the flat copy of a large row return, in `workspace`.
+static int make_combine_index(const int64_t* layout_range, int num_experts, int num_ranks, int rank,
+                              int num_max_dispatch_tokens_per_rank, bool skip_own, void* workspace,
+                              size_t workspace_bytes, CombineIndexArgs& index) {
+    EP_HOST_ASSERT(workspace_bytes >= size_t(segment_workspace_bytes(num_experts, num_max_dispatch_tokens_per_rank)));
+    EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(workspace) & 15) == 0);
+    index.layout_range = layout_range;
+    index.num_local_experts = num_experts / num_ranks, index.num_ranks = num_ranks, index.rank = rank;
+    index.max_tokens = num_max_dispatch_tokens_per_rank, index.skip_own = skip_own;
+    index.flat_out = reinterpret_cast<int32_t*>(workspace);
+    index.desc = reinterpret_cast<RowDesc*>(reinterpret_cast<uint8_t*>(workspace) +
+                                            (((int64_t(num_experts) + 1) * 4 + 255) & ~int64_t(255)));
+    return 0;
+}
+
+static int launch_combine_rows(const CombineIndexArgs& index, const void* x, int hidden, void* combine_staging,
+                               void* combine_send_slots, int64_t expected_rows, hipStream_t hs) {
+    const int num_experts = index.num_local_experts * index.num_ranks, num_vec = hidden * 2 / 16;
+    const int64_t max_rows = int64_t(num_experts) * index.max_tokens;
+    ll_rows_flat_kernel<<<flat_grid_blocks(expected_rows, max_rows, index.max_tokens), flat_row_threads(num_vec), 0,
+                          hs>>>(index.flat_out, num_experts, index.desc, reinterpret_cast<const uint8_t*>(x),
+                                int64_t(hidden) * 2, num_vec, reinterpret_cast<uint8_t*>(combine_send_slots),
+                                reinterpret_cast<uint8_t*>(combine_staging), int64_t(hidden) * 2, 0, 0, nullptr, 0,
+                                nullptr, 0);
+    EP_LAUNCH_CHECK();
+    return 0;
+}
+
 // skip_own: the rows owed to this rank itself are not moved (the reduce will read them from x).
 static int launch_combine_send(const void* x, const int64_t* layout_range, int hidden, int num_experts, int num_ranks,
                                int rank, int num_max_dispatch_tokens_per_rank, void* combine_staging,
@@ -443,29 +485,17 @@ static int launch_combine_send(const void* x, const int64_t* layout_range, int h
     if (int rc = check_combine_send_args(x, layout_range, hidden, num_experts, num_ranks, rank,
                                          num_max_dispatch_tokens_per_rank, combine_staging, combine_send_slots))
         return rc;
-    const int num_local_experts = num_experts / num_ranks;
     const int64_t max_rows = int64_t(num_experts) * num_max_dispatch_tokens_per_rank;
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     const bool large = estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank) > kLargeBatchRows;
     if (large && workspace != nullptr) {
-        EP_HOST_ASSERT(workspace_bytes >= size_t(segment_workspace_bytes(num_experts, num_max_dispatch_tokens_per_rank)));
-        EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(workspace) & 15) == 0);
-        int32_t* flat = reinterpret_cast<int32_t*>(workspace);
-        RowDesc* desc = reinterpret_cast<RowDesc*>(reinterpret_cast<uint8_t*>(workspace) +
-                                                   (((int64_t(num_experts) + 1) * 4 + 255) & ~int64_t(255)));
-        ll_segment_index_kernel<<<num_experts, kIndexThreads, 0, hs>>>(
-            skip_own ? 2 : 1, nullptr, layout_range, num_local_experts, num_ranks, rank,
-            num_max_dispatch_tokens_per_rank, nullptr,
-            nullptr, nullptr, flat, desc, ObservedRows{nullptr, 0});
+        CombineIndexArgs index;
+        if (int rc = make_combine_index(layout_range, num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank,
+                                        skip_own, workspace, workspace_bytes, index))
+            return rc;
+        ll_combine_index_kernel<<<num_experts, 256, size_t(num_experts + 1) * sizeof(int32_t), hs>>>(index);
         EP_LAUNCH_CHECK();
-        const int num_vec = hidden * 2 / 16;
-        ll_rows_flat_kernel<<<flat_grid_blocks(expected_rows, max_rows, num_max_dispatch_tokens_per_rank),
-                              flat_row_threads(num_vec), 0, hs>>>(flat, num_experts, desc, reinterpret_cast<const uint8_t*>(x), int64_t(hidden) * 2,
-                                    num_vec, reinterpret_cast<uint8_t*>(combine_send_slots),
-                                    reinterpret_cast<uint8_t*>(combine_staging), int64_t(hidden) * 2, 0, 0, nullptr, 0,
-                                    nullptr, 0);
-        EP_LAUNCH_CHECK();
-        return 0;
+        return launch_combine_rows(index, x, hidden, combine_staging, combine_send_slots, expected_rows, hs);
     }
     const CombineSendArgs sa = make_combine_send_args(x, layout_range, hidden, num_experts, num_ranks, rank,
                                                       num_max_dispatch_tokens_per_rank, combine_staging,
@@ -488,12 +518,28 @@ int deepep_ll_combine_send(const void* x, const int64_t* layout_range, int hidde
                                workspace, workspace_bytes, false, stream);
 }
 
+static void launch_reduce(const CombineRecvArgs& ra, const uint8_t* own, const int64_t* layout_range, int rank,
+                          int num_local_experts, int num_ranks, const CombineIndexArgs* index, hipStream_t hs) {
+    const int waves = 4;  // block shape makes no measurable difference (1..16 waves: within 5 %)
+    const int index_blocks = index != nullptr ? index->num_local_experts * index->num_ranks : 0;
+    const CombineIndexArgs ia = index != nullptr ? *index : CombineIndexArgs{};
+    const int64_t blocks = index_blocks + (int64_t(ra.num_tokens) * ra.pieces_per_row + waves - 1) / waves;
+    const size_t lds = size_t(index_blocks > 0 ? index_blocks + 1 : num_local_experts) * sizeof(int32_t);
+    if (int64_t(ra.num_tokens) * ra.num_topk * ra.hidden * 2 > stream_bytes())
+        ll_combine_recv_kernel<true><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(
+            ra, own, layout_range, rank, num_local_experts, num_ranks, ia, index_blocks);
+    else
+        ll_combine_recv_kernel<false><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(
+            ra, own, layout_range, rank, num_local_experts, num_ranks, ia, index_blocks);
+}
+
 // own_x != null: the answers of this rank's own experts are read from own_x at the positions
 // layout_range gives, instead of from combine_staging.
 static int launch_combine_recv(const void* combine_staging, const int64_t* topk_idx, const float* topk_weights,
                                const int32_t* pair_slot, int num_tokens, int hidden, int num_topk, int num_experts,
                                int num_max_dispatch_tokens_per_rank, int accumulate, void* out, const void* own_x,
-                               const int64_t* layout_range, int rank, int num_ranks, void* stream) {
+                               const int64_t* layout_range, int rank, int num_ranks, const CombineIndexArgs* index,
+                               void* stream) {
     if (int rc = check_combine_recv_args(combine_staging, topk_idx, topk_weights, pair_slot, num_tokens, hidden,
                                          num_topk, num_experts, num_max_dispatch_tokens_per_rank, out))
         return rc;
@@ -501,18 +547,9 @@ static int launch_combine_recv(const void* combine_staging, const int64_t* topk_
     const CombineRecvArgs ra = make_combine_recv_args(combine_staging, topk_idx, topk_weights, pair_slot, num_tokens,
                                                       hidden, num_topk, num_experts,
                                                       num_max_dispatch_tokens_per_rank, accumulate, out);
-    const int waves = 4;  // block shape makes no measurable difference (1..16 waves: within 5 %)
-    const int64_t blocks = (int64_t(num_tokens) * ra.pieces_per_row + waves - 1) / waves;
-    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
-    const int num_local_experts = own_x != nullptr ? num_experts / num_ranks : 0;
-    const size_t lds = size_t(num_local_experts) * sizeof(int32_t);
-    const uint8_t* own = reinterpret_cast<const uint8_t*>(own_x);
-    if (int64_t(num_tokens) * num_topk * hidden * 2 > stream_bytes())
-        ll_combine_recv_kernel<true><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(ra, own, layout_range, rank,
-                                                                                        num_local_experts, num_ranks);
-    else
-        ll_combine_recv_kernel<false><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(ra, own, layout_range, rank,
-                                                                                         num_local_experts, num_ranks);
+    launch_reduce(ra, reinterpret_cast<const uint8_t*>(own_x), layout_range, rank,
+                  own_x != nullptr ? num_experts / num_ranks : 0, num_ranks, index,
+                  reinterpret_cast<hipStream_t>(stream));
     EP_LAUNCH_CHECK();
     return 0;
 }
@@ -523,7 +560,7 @@ int deepep_ll_combine_recv(const void* combine_staging, const int64_t* topk_idx,
     clear_error();
     return launch_combine_recv(combine_staging, topk_idx, topk_weights, pair_slot, num_tokens, hidden, num_topk,
                                num_experts, num_max_dispatch_tokens_per_rank, accumulate, out, nullptr, nullptr, 0, 1,
-                               stream);
+                               nullptr, stream);
 }
 
 int deepep_ll_combine_send_by_dest(const void* x, const int32_t* record_packed_row, const uint32_t* source_rank,
@@ -589,13 +626,7 @@ int deepep_ll_combine_recv_flat(const void* recv_flat, int64_t recv_flat_rows, i
                                                 out);
     ra.flat_prefix = send_expert_prefix, ra.flat_rows = recv_flat_rows, ra.flat_slot_rows = slot_rows;
     ra.experts_per_rank = num_experts / num_ranks;
-    const int waves = 4;
-    const int64_t blocks = (int64_t(num_tokens) * ra.pieces_per_row + waves - 1) / waves;
-    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
-    if (int64_t(num_tokens) * num_topk * hidden * 2 > stream_bytes())
-        ll_combine_recv_kernel<true><<<dim3(unsigned(blocks)), waves * kWave, 0, hs>>>(ra, nullptr, nullptr, 0, 0, 1);
-    else
-        ll_combine_recv_kernel<false><<<dim3(unsigned(blocks)), waves * kWave, 0, hs>>>(ra, nullptr, nullptr, 0, 0, 1);
+    launch_reduce(ra, nullptr, nullptr, 0, 0, 1, nullptr, reinterpret_cast<hipStream_t>(stream));
     EP_LAUNCH_CHECK();
     return 0;
 }
@@ -613,19 +644,30 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
         // the two phases back to back, with the single launch's shortcut: the rows owed to this rank
         // itself are not moved, the reduce reads them from x.  Without send slots (zero copy: the transport
         // sends layout_range's ranges straight from x) there is nothing to return.
-        if (combine_send_slots == nullptr) {
-            if (int rc = check_combine_send_args(x, layout_range, hidden, num_experts, num_ranks, rank,
-                                                 num_max_dispatch_tokens_per_rank, combine_staging, nullptr))
-                return rc;
-        } else if (int rc = launch_combine_send(x, layout_range, hidden, num_experts, num_ranks, rank,
-                                                num_max_dispatch_tokens_per_rank, combine_staging,
-                                                combine_send_slots, expected_rows, workspace, workspace_bytes, true,
-                                                stream)) {
+        if (int rc = check_combine_send_args(x, layout_range, hidden, num_experts, num_ranks, rank,
+                                             num_max_dispatch_tokens_per_rank, combine_staging, combine_send_slots))
             return rc;
+        // The reduce goes first and builds the row return's index on the way, unless there is nothing to reduce
+        // or no memory for an index.
+        const bool index_in_reduce = combine_send_slots != nullptr && workspace != nullptr && num_tokens > 0;
+        CombineIndexArgs index;
+        if (index_in_reduce) {
+            if (int rc = make_combine_index(layout_range, num_experts, num_ranks, rank,
+                                            num_max_dispatch_tokens_per_rank, true, workspace, workspace_bytes, index))
+                return rc;
+        } else if (combine_send_slots != nullptr) {
+            if (int rc = launch_combine_send(x, layout_range, hidden, num_experts, num_ranks, rank,
+                                             num_max_dispatch_tokens_per_rank, combine_staging, combine_send_slots,
+                                             expected_rows, workspace, workspace_bytes, true, stream))
+                return rc;
         }
-        return launch_combine_recv(combine_staging, topk_idx, topk_weights, pair_slot, num_tokens, hidden, num_topk,
-                                   num_experts, num_max_dispatch_tokens_per_rank, accumulate, out, x, layout_range,
-                                   rank, num_ranks, stream);
+        if (int rc = launch_combine_recv(combine_staging, topk_idx, topk_weights, pair_slot, num_tokens, hidden,
+                                         num_topk, num_experts, num_max_dispatch_tokens_per_rank, accumulate, out, x,
+                                         layout_range, rank, num_ranks, index_in_reduce ? &index : nullptr, stream))
+            return rc;
+        if (!index_in_reduce) return 0;
+        return launch_combine_rows(index, x, hidden, combine_staging, combine_send_slots, expected_rows,
+                                   reinterpret_cast<hipStream_t>(stream));
     }
     if (int rc = check_combine_send_args(x, layout_range, hidden, num_experts, num_ranks, rank,
                                          num_max_dispatch_tokens_per_rank, combine_staging, combine_send_slots))

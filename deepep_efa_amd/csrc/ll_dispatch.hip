@@ -1245,7 +1245,7 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
                                                    (((int64_t(num_experts) + 1) * 4 + 255) & ~int64_t(255)));
         if (!index_done) {  // (a large one-call dispatch builds the index inside its send launch)
             ll_segment_index_kernel<<<num_experts, kIndexThreads, 0, hs>>>(
-                0, recv_count, nullptr, num_local_experts, num_ranks, own_rank, num_max_dispatch_tokens_per_rank,
+                recv_count, num_local_experts, num_ranks, own_rank, num_max_dispatch_tokens_per_rank,
                 packed_recv_layout_range, packed_recv_count, cumulative_local_expert_recv_stats, flat, desc, observed);
             EP_LAUNCH_CHECK();
         }

@@ -215,90 +215,69 @@ __device__ __forceinline__ int block_exclusive_scan_1024(int v, int32_t* wave_to
     return offset;
 }
 
-// mode 0 (dispatch receive): counts = recv_count; writes layout_range / packed_count / stats;
-//        descriptor = {staging row seg*M + j, packed row e_l*N + begin + j}; rank = -1, or the rank
-//        whose own rows the send side has already put at their packed position (they keep their
-//        place in the ranges, in ascending source order, and get no descriptors).
-// mode 1 (combine send; mode 2: the same without this rank's own rows): counts and begins from layout_range;
-//        descriptor = {expert-output row e_l*N + begin + j, seg*M + j for other ranks or
-//        -(1 + (rank*E_l + e_l)*M + j) for this rank's own rows}.
+// Dispatch receive: counts = recv_count; writes layout_range / packed_count / stats;
+// descriptor = {staging row seg*M + j, packed row e_l*N + begin + j}; rank = -1, or the rank
+// whose own rows the send side has already put at their packed position (they keep their
+// place in the ranges, in ascending source order, and get no descriptors).
 static __global__ __launch_bounds__(kIndexThreads) void ll_segment_index_kernel(
-    int mode, const int32_t* __restrict__ counts32, const int64_t* __restrict__ layout_in, int num_local_experts,
-    int num_ranks, int rank, int max_tokens, int64_t* __restrict__ layout_out, int32_t* __restrict__ packed_count,
-    int32_t* __restrict__ stats, int32_t* __restrict__ flat_out, RowDesc* __restrict__ desc, ObservedRows observed) {
+    const int32_t* __restrict__ counts32, int num_local_experts, int num_ranks, int rank, int max_tokens,
+    int64_t* __restrict__ layout_out, int32_t* __restrict__ packed_count, int32_t* __restrict__ stats,
+    int32_t* __restrict__ flat_out, RowDesc* __restrict__ desc, ObservedRows observed) {
     __shared__ int32_t flat[kIndexThreads + 1];   // prefix over the rows that get descriptors
-    __shared__ int32_t place[kIndexThreads + 1];  // mode 0: prefix over all rows (where a segment lands)
-    __shared__ int32_t begin_in[kIndexThreads];
+    __shared__ int32_t place[kIndexThreads + 1];  // prefix over all rows: where a segment lands
     __shared__ int32_t wave_totals[kIndexThreads / kWave];
     __shared__ int32_t wave_totals_place[kIndexThreads / kWave];
     const int tid = threadIdx.x;
     const int num_segments = num_local_experts * num_ranks;
     int c = 0;
     if (tid < num_segments) {
-        if (mode == 0) {
-            c = counts32[tid];
-        } else {
-            const int64_t lr = layout_in[tid];
-            c = int(lr & 0xffffffffll);
-            begin_in[tid] = int(lr >> 32);
-            if (mode == 2 && tid % num_ranks == rank) c = 0;  // own rows stay where they are
-        }
+        c = counts32[tid];
         c = c < 0 ? 0 : (c > max_tokens ? max_tokens : c);
     }
-    // mode 0 with rank >= 0: the rank's own rows are already in place (reference order: a range
+    // rank >= 0: the rank's own rows are already in place (reference order: a range
     // begins where the lower source ranks' rows end, csrc/kernels/efa_kernels.cu:991-1010), so
     // they count towards where the later segments land but take no descriptors
-    const bool own_placed = mode == 0 && rank >= 0;
+    const bool own_placed = rank >= 0;
     const int c_all = c;
     if (own_placed && tid < num_segments && tid % num_ranks == rank) c = 0;
     int total;
     const int prefix = block_exclusive_scan_1024(c, wave_totals, total);
     if (tid < num_segments) flat[tid] = prefix;
     if (tid == 0) flat[num_segments] = total;
-    if (mode == 0) {
-        int total_all = total, prefix_all = prefix;
-        if (own_placed) prefix_all = block_exclusive_scan_1024(c_all, wave_totals_place, total_all);
-        if (tid < num_segments) place[tid] = prefix_all;
-        if (tid == 0) place[num_segments] = total_all;
-    }
+    int total_all = total, prefix_all = prefix;
+    if (own_placed) prefix_all = block_exclusive_scan_1024(c_all, wave_totals_place, total_all);
+    if (tid < num_segments) place[tid] = prefix_all;
+    if (tid == 0) place[num_segments] = total_all;
     __syncthreads();
     const int64_t slots_per_expert = int64_t(max_tokens) * num_ranks;
     if (blockIdx.x == 0) {
         for (int s = tid; s <= num_segments; s += kIndexThreads) flat_out[s] = flat[s];
-        if (mode == 0) {
-            if (tid == 0) report_observed(observed, place[num_segments]);
-            if (tid < num_segments) {
-                const int le = tid / num_ranks;
-                const int64_t cnt = c_all;
-                const int64_t begin = place[tid] - place[le * num_ranks];
-                layout_out[tid] = cnt > 0 ? ((begin << 32) | cnt) : 0;
-            }
-            if (tid < num_local_experts) {
-                const int n = place[(tid + 1) * num_ranks] - place[tid * num_ranks];
-                packed_count[tid] = n;
-                if (stats != nullptr) stats[tid] += n;
-            }
+        if (tid == 0) report_observed(observed, place[num_segments]);
+        if (tid < num_segments) {
+            const int le = tid / num_ranks;
+            const int64_t cnt = c_all;
+            const int64_t begin = place[tid] - place[le * num_ranks];
+            layout_out[tid] = cnt > 0 ? ((begin << 32) | cnt) : 0;
+        }
+        if (tid < num_local_experts) {
+            const int n = place[(tid + 1) * num_ranks] - place[tid * num_ranks];
+            packed_count[tid] = n;
+            if (stats != nullptr) stats[tid] += n;
         }
     }
     const int seg = blockIdx.x;
-    const int le = seg / num_ranks, s = seg - le * num_ranks;
+    const int le = seg / num_ranks;
     const int cnt = flat[seg + 1] - flat[seg];
-    const int64_t begin = mode == 0 ? place[seg] - place[le * num_ranks] : begin_in[seg];
-    if (mode != 0 && (begin < 0 || begin + cnt > slots_per_expert)) return;  // malformed range: emit nothing
+    const int64_t begin = place[seg] - place[le * num_ranks];
     for (int j = tid; j < cnt; j += kIndexThreads) {
         RowDesc d;
-        if (mode == 0) {
-            d.src_row = seg * max_tokens + j;
-            d.dst_row = int32_t(le * slots_per_expert + begin + j);
-        } else {
-            d.src_row = int32_t(le * slots_per_expert + begin + j);
-            d.dst_row = s == rank ? -(1 + (rank * num_local_experts + le) * max_tokens + j) : seg * max_tokens + j;
-        }
+        d.src_row = seg * max_tokens + j;
+        d.dst_row = int32_t(le * slots_per_expert + begin + j);
         desc[flat[seg] + j] = d;
     }
 }
 
-// The dispatch-receive index (mode 0 above with the rank's own rows already placed) as one workgroup's
+// The dispatch-receive index (the kernel above with the rank's own rows already placed) as one workgroup's
 // share inside another launch: the send kernel of a large one-call dispatch carries these workgroups
 // beside its own, so the index costs no launch.  The launch that carries it is still writing the
 // rank's own counts into recv_count, so they are taken from what that launch reads them from: the
@@ -369,6 +348,44 @@ __device__ __forceinline__ void recv_index_block(const FusedIndexArgs& a, int se
         d.src_row = seg * max_tokens + j;
         d.dst_row = int32_t(le * slots_per_expert + begin + j);
         a.desc[flat[seg] + j] = d;
+    }
+}
+
+// The index of the combine's row return: counts and begins from layout_range; descriptor = {expert-output row
+// e_l*N + begin + j, seg*M + j for other ranks or -(1 + (rank*E_l + e_l)*M + j) for this rank's own rows}.  One
+// workgroup's share: of a launch of its own or, in front of the reduce's workgroups, of the reduce's launch.
+// Any workgroup size that is a multiple of 64; lds holds segments + 1 ints, wave_totals 16.
+struct CombineIndexArgs {
+    const int64_t* layout_range;  // [E_l][R]
+    int num_local_experts, num_ranks, rank, max_tokens;
+    bool skip_own;  // own rows stay where they are
+    int32_t* flat_out;
+    RowDesc* desc;
+};
+
+__device__ __forceinline__ void combine_index_block(const CombineIndexArgs& a, int seg, int32_t* flat,
+                                                    int32_t* wave_totals) {
+    const int tid = threadIdx.x, threads = blockDim.x;
+    const int num_ranks = a.num_ranks, max_tokens = a.max_tokens;
+    const int num_segments = a.num_local_experts * num_ranks;
+    const int64_t begin = a.layout_range[seg] >> 32;
+    for (int s = tid; s < num_segments; s += threads) {
+        const int c = int(a.layout_range[s] & 0xffffffffll);
+        flat[s] = c < 0 || (a.skip_own && s % num_ranks == a.rank) ? 0 : (c > max_tokens ? max_tokens : c);
+    }
+    lds_barrier();
+    block_exclusive_scan(flat, num_segments, wave_totals);
+    if (seg == 0)
+        for (int s = tid; s <= num_segments; s += threads) a.flat_out[s] = flat[s];
+    const int le = seg / num_ranks, s = seg - le * num_ranks;
+    const int first = flat[seg], cnt = flat[seg + 1] - first;
+    const int64_t slots_per_expert = int64_t(max_tokens) * num_ranks;
+    const bool sound = begin >= 0 && begin + cnt <= slots_per_expert;  // rows of a malformed range are not moved
+    for (int j = tid; j < cnt; j += threads) {
+        RowDesc d;
+        d.src_row = sound ? int32_t(le * slots_per_expert + begin + j) : -1;
+        d.dst_row = s == a.rank ? -(1 + (a.rank * a.num_local_experts + le) * max_tokens + j) : seg * max_tokens + j;
+        a.desc[first + j] = d;
     }
 }
 

@@ -1566,3 +1566,36 @@ def test_return_by_destination_over_record_counts(rt, records, hidden):
         if row >= 0:
             want[int(offset[i])] = x[row].cpu()
     assert torch.equal(out.cpu(), want)
+
+
+@pytest.mark.parametrize("t,k", [(1025, 8), (1100, 8)])
+def test_large_combine_moves_no_rows_of_a_malformed_range(rt, t, k):
+    """Past 8192 rows the reduce's launch builds the row return's index; a segment whose range leaves its expert gets
+    no rows moved, all others do, and the reduce does not depend on it."""
+    r, rank, h, e = 8, 3, 512, 16
+    x_all, topk_all, w = make_world(r, t, h, k, e, seed=t, drop=30)
+    st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, t, O.ROW_BF16, one_call=True)
+    topk, weights = topk_all[rank].cuda(), w[rank].cuda()
+    y = torch.randn(st.packed_recv_x.shape, generator=torch.Generator().manual_seed(t)).bfloat16().cuda()
+    world.combine_from_peers(st, mode=1, seed=5)
+    got = []
+    sound = st.packed_recv_layout_range
+    bad = sound.clone()
+    le, source = 1, 6
+    bad[le, source] = (int(r * t) << 32) | int(sound[le, source] & 0xffffffff)
+    for lr in (sound, bad):
+        st.combine_send_slots.view(torch.int16).fill_(0x7FC0)
+        out = torch.zeros((t, h), dtype=torch.bfloat16, device="cuda")
+        st.combine(y, topk, weights, out, layout_range=lr)
+        torch.cuda.synchronize()
+        got.append((st.combine_send_slots.view(torch.int16).view(e // r, r, t, h).cpu(), out.cpu()))
+    want = got[0][0].clone()
+    for l2 in range(e // r):  # what a row return moves, worked out from the ranges
+        for s in range(r):
+            n, begin = int(sound[l2, s] & 0xffffffff), int(sound[l2, s] >> 32)
+            rows = y[l2, begin:begin + n].view(torch.int16).cpu()
+            if s != rank:
+                assert torch.equal(want[l2, s, :n], rows)
+    want[le, source] = 0x7FC0
+    assert torch.equal(got[1][0], want)
+    assert torch.equal(got[0][1], got[1][1])
