@@ -297,6 +297,7 @@ struct Buffer {
         if (!explicitly_destroy) {
             destroy();
         } else if (!destroyed) {
+            release_observed();
             printf("WARNING: destroy() was not called before DeepEP buffer destruction, which can leak resources.\n");
             fflush(stdout);
         }
@@ -321,15 +322,24 @@ struct Buffer {
         available = true;
     }
 
+    // The host allocator does not know of the kernels that store to the pinned word: it gets the word back when
+    // none is left in flight, or its next owner would find a row count in it.
+    void release_observed() {
+        if (observed == nullptr) return;
+        const c10::DeviceGuard on_device(torch::Device(torch::kCUDA, static_cast<c10::DeviceIndex>(device_id)));
+        (void)hipDeviceSynchronize();
+        observed = nullptr;
+        observed_memory.clear();
+    }
+
     void destroy() {
         if (destroyed) return;
         if (available) (void)hipDeviceSynchronize();
+        release_observed();
         nvl_buffer = torch::Tensor();
         rdma_buffer = torch::Tensor();
         layout_workspaces.clear();
         ll = LowLatencyCache();
-        observed = nullptr;
-        observed_memory.clear();
         combine_input_buffers.clear();
         world_x.reset();
         world_topk_idx.reset();
@@ -585,12 +595,13 @@ struct Buffer {
         auto stream = current_stream();
 
         stage_peer_rows(c);  // what the exchange would have delivered
-        if (observed == nullptr) {
+        // a captured call takes the hint but does not report: its replays may outlive the buffer, and a capture is
+        // no place to allocate pinned memory
+        const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+        if (observed == nullptr and not capturing) {
             observed_memory = at::getHostAllocator(at::kCUDA)->allocate(sizeof(uint64_t));
             observed = new (observed_memory.get()) std::atomic<uint64_t>(0);
         }
-        // a captured call takes the hint but does not report: its replays may outlive the buffer
-        const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
         // send and receive phase in one call (one kernel launch for decode-sized batches)
         abi_check(deepep_ll_dispatch_observed(
             x.data_ptr(), topk_idx.data_ptr<int64_t>(), num_tokens, hidden, num_topk, num_experts, num_ranks, rank,

@@ -487,3 +487,42 @@ def test_dispatch_and_combine_replay_in_a_hip_graph(deep_ep, num_ranks, rank, t,
         assert torch.equal(got[3][live], want[3][live]), f"replay {replay}: src_info"
         assert torch.equal(got[5].view(torch.int16), want[5].view(torch.int16)), f"replay {replay}: combined"
     buffer.destroy()
+
+
+def _small_dispatch(deep_ep):
+    buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=4, sim_rank=1)
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn((32, 512), generator=g).bfloat16().cuda()
+    topk_idx = torch.topk(torch.rand((32, 16), generator=g), 4, dim=-1)[1].cuda()
+    return buffer, lambda: buffer.low_latency_dispatch(x, topk_idx, 32, 16)
+
+
+def test_the_first_call_of_a_buffer_may_be_captured(deep_ep):
+    buffer, dispatch = _small_dispatch(deep_ep)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        (rows, _), count, _, _, _ = dispatch()
+    for _ in range(3):
+        count.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = count.clone()
+        want = dispatch()[1]
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    buffer.destroy()
+
+
+def test_a_dropped_buffer_leaves_no_store_behind(deep_ep):
+    """Pinned memory handed out after a buffer is gone, without destroy(), is not written by its last dispatch."""
+    buffer, dispatch = _small_dispatch(deep_ep)
+    dispatch()
+    busy = torch.randn((8192, 8192), device="cuda")
+    for _ in range(4):
+        busy = busy @ busy
+        busy /= busy.norm()
+    dispatch()
+    del buffer, dispatch
+    words = [torch.full((1,), 7, dtype=torch.int64, pin_memory=True) for _ in range(64)]
+    torch.cuda.synchronize()
+    assert all(int(w) == 7 for w in words)
