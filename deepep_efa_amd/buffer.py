@@ -212,9 +212,8 @@ class Buffer:
           handle   (src_info [E_l, N] int32, layout_range [E_l, R] int64 = (begin << 32) | count,
                    num_max_dispatch_tokens_per_rank, hidden, num_experts);
           the returned tensors are reused by the next call with the same shape.
-        An event is returned either way, as in the reference (deep_ep/buffer.py:2449 returns
-        EventOverlap(EventHandle()) whatever the flag says); without async_finish it is recorded when another
-        stream waits on it, since the call's own stream is in order already.
+        An event is returned either way, recorded behind the call's work before it returns, as in the reference
+        (deep_ep/buffer.py:2449 returns EventOverlap(EventHandle()) whatever async_finish says).
         """
         prof = None
         if _PROFILE_ENABLED:
@@ -243,9 +242,8 @@ class Buffer:
         accumulate (needs `out`): the sum starts from float32(out[t]) instead of zero — the flag the
         reference's reduce takes (csrc/kernels/coop_combine_recv.cuh:174-179) and its Python fixes to False
         (deep_ep/buffer.py:2541).
-        An event is returned either way, as in the reference (deep_ep/buffer.py:2801-2803 returns
-        EventOverlap(EventHandle()) whatever the flag says); without async_finish it is recorded when another
-        stream waits on it, since the call's own stream is in order already.
+        An event is returned either way, recorded behind the call's work before it returns, as in the reference
+        (deep_ep/buffer.py:2801-2803 returns EventOverlap(EventHandle()) whatever async_finish says).
         """
         assert not accumulate or out is not None, "accumulate adds to `out`"
         prof = None

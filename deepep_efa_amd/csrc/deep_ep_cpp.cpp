@@ -176,38 +176,13 @@ static size_t get_low_latency_rdma_size_hint(int num_max_dispatch_tokens_per_ran
 // ---------------------------------------------------------------------------
 struct EventHandle {
     std::shared_ptr<torch::Event> event;
-    std::optional<HostStream> origin;  // deferred: the stream whose work the handle stands for, not recorded yet
 
-    EventHandle() {
-        event = std::make_shared<torch::Event>(torch::kCUDA);
-        event->record(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA());
-    }
+    EventHandle() : EventHandle(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()) {}
     explicit EventHandle(const HostStream& stream) {
         event = std::make_shared<torch::Event>(torch::kCUDA);
         event->record(stream);
     }
-    struct Deferred {};
-    EventHandle(const HostStream& stream, Deferred) : origin(stream) {}
-
-    // The handle of a call that was not asked to be asynchronous.  Its work is ordered on the caller's stream
-    // already, so a wait from that stream is no wait; recording a HIP event for it costs the host 5 us a call
-    // (a decode step with two of them: 20 us against 9.7 without), more than the launch.  It is recorded when
-    // another stream waits, and then covers the call and whatever that stream was given since; nothing is kept,
-    // so one handle stands for every such call on its stream.
-    // A stream made outside PyTorch may be gone by then, so there the event is recorded at once.
-    static bool can_defer(const HostStream& stream) {  // c10: the default stream is 0, pool streams have odd ids
-        return stream.id() == 0 or (stream.id() & 1) != 0;
-    }
-
-    void stream_wait_for(const HostStream& waiter) const {
-        if (event != nullptr) {
-            waiter.unwrap().wait(*event);
-        } else if (waiter != origin.value()) {
-            torch::Event now(torch::kCUDA);
-            now.record(origin.value());
-            waiter.unwrap().wait(now);
-        }
-    }
+    void stream_wait_for(const HostStream& waiter) const { waiter.unwrap().wait(*event); }
     void current_stream_wait() const { stream_wait_for(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
 };
 
@@ -264,8 +239,6 @@ struct Buffer {
     // kernels sized for a balanced world walk such a batch in a slow loop.
     at::DataPtr observed_memory;
     std::atomic<uint64_t>* observed = nullptr;
-    std::optional<HostStream> event_stream;  // the stream that event_of_stream stands for
-    pybind11::object event_of_stream;
     // loopback world
     std::optional<torch::Tensor> world_x, world_topk_idx;
     torch::Tensor ranks_below, ranks_above, peer_workspace;
@@ -754,17 +727,6 @@ struct Buffer {
             if (b.defined()) b.zero_();
         if (ll.recv_count.defined()) ll.recv_count.zero_();
         ll.dispatched = false;
-    }
-
-    // The event that Buffer's Python methods hand back.
-    pybind11::object returned_event(bool async) {
-        const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
-        if (async or not EventHandle::can_defer(stream)) return pybind11::cast(EventHandle(stream));
-        if (!event_stream.has_value() or event_stream.value() != stream) {
-            event_of_stream = pybind11::cast(EventHandle(stream, EventHandle::Deferred{}));
-            event_stream = stream;
-        }
-        return event_of_stream;
     }
 
     void ensure_mask() {
@@ -1421,6 +1383,12 @@ struct PlainCall<F> {
     }
 };
 
+// The event of a low-latency call, with or without async_finish.  It is recorded before the call returns: recorded
+// when somebody waits, it would also cover what the caller's stream was given in between, which takes away the
+// overlap with it and hangs where that work waits for the waiter.  A record takes the stream 3 us beside kernels of
+// 8 us and the host 2 (two launches and a record each: 24.3 us against 18.6 without); a step records two.
+static pybind11::object recorded_event() { return pybind11::cast(EventHandle()); }
+
 static pybind11::object hook_object(bool wanted) {
     if (!wanted) return pybind11::none();
     return pybind11::cpp_function([] {});
@@ -1442,7 +1410,8 @@ static PyObject* low_latency_dispatch_call(PyObject*, PyObject* const* a, Py_ssi
                                                    result_object(c.packed_recv_layout_range), c.max_tokens, c.hidden,
                                                    c.num_experts);
         }
-        const pybind11::object count = result_object(c.packed_recv_count), event = buffer.returned_event(bool_argument(a[10])),
+        (void)bool_argument(a[10]);
+        const pybind11::object count = result_object(c.packed_recv_count), event = recorded_event(),
                                hook = hook_object(bool_argument(a[11]));
         return pybind11::reinterpret_steal<pybind11::object>(
             PyTuple_Pack(5, c.recv_result.ptr(), count.ptr(), c.handle_result.ptr(), event.ptr(), hook.ptr()));
@@ -1463,7 +1432,8 @@ static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssiz
             tensor_argument(a[1]), tensor_argument(a[2]), tensor_argument(a[3]), tensor_argument(of_handle(0)),
             tensor_argument(of_handle(1)), optional_tensor_argument(a[5]), int_argument(of_handle(2)),
             int_argument(of_handle(4)), bool_argument(a[6]), optional_tensor_argument(a[9]), bool_argument(a[10])));
-        const pybind11::object event = buffer.returned_event(bool_argument(a[7])), hook = hook_object(bool_argument(a[8]));
+        (void)bool_argument(a[7]);
+        const pybind11::object event = recorded_event(), hook = hook_object(bool_argument(a[8]));
         return pybind11::reinterpret_steal<pybind11::object>(PyTuple_Pack(3, combined.ptr(), event.ptr(), hook.ptr()));
     });
 }

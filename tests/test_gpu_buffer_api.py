@@ -254,6 +254,51 @@ def test_another_stream_waits_on_the_returned_events(deep_ep, caller, async_fini
     buffer.destroy()
 
 
+def _step_with_events(deep_ep):
+    """A buffer and a call that runs one small step on the current stream and returns its two events."""
+    num_ranks, rank, t, h, k, e = 8, 2, 32, 1024, 4, 64
+    buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=num_ranks,
+                            sim_rank=rank, sim_seed=13)
+    x, topk_idx = buffer.loopback_synthesise(t, h, k, e)
+    w = torch.rand((t, k), generator=torch.Generator().manual_seed(4)).cuda()
+    y = buffer.low_latency_dispatch(x, topk_idx, t, e, use_fp8=False)[0].clone()
+
+    def step(async_finish):
+        _, _, handle, dispatched, _ = buffer.low_latency_dispatch(x, topk_idx, t, e, use_fp8=False,
+                                                                  async_finish=async_finish)
+        _, reduced, _ = buffer.low_latency_combine(y, topk_idx, w, handle, async_finish=async_finish)
+        return dispatched, reduced
+
+    return buffer, step
+
+
+@pytest.mark.parametrize("async_finish", (False, True))
+@pytest.mark.parametrize("which", (0, 1))
+def test_a_returned_event_covers_nothing_that_came_after_the_call(deep_ep, which, async_finish):
+    """Work given to the caller's stream after the call (expert GEMMs, say) is not waited for.  Streams share the
+    hardware queues, so of several waiting streams one that passes the long kernel is what can be asked for."""
+    buffer, step = _step_with_events(deep_ep)
+    mine, others = torch.cuda.Stream(), [torch.cuda.Stream() for _ in range(8)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(mine):
+        event = step(async_finish)[which]
+        torch.cuda._sleep(200_000_000)
+        later = torch.cuda.Event()
+        later.record()
+    passed = []
+    for s in others:
+        with torch.cuda.stream(s):
+            event.current_stream_wait()
+            passed.append(torch.cuda.Event())
+            passed[-1].record()
+    overlapped = False
+    while not overlapped and not later.query():
+        overlapped = any(p.query() for p in passed) and not later.query()
+    torch.cuda.synchronize()
+    assert overlapped
+    buffer.destroy()
+
+
 def test_combine_accumulates_into_out_through_the_api(deep_ep):
     """accumulate=True starts the float32 sum from what `out` holds (csrc/kernels/coop_combine_recv.cuh:174-179):
     checked bit for bit against the float32 FMA chain started from the previous contents."""
