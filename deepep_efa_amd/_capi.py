@@ -25,7 +25,8 @@ PROTOTYPES = {
     "deepep_get_dispatch_layout": (_I, [_VP, _I, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),
     "deepep_routing_sort_workspace_bytes": (_SZ, [_I, _I]),
     "deepep_moe_routing_sort": (_I, [_VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),
-    "deepep_moe_routing_sort_total": (_I, [_VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),
+    "deepep_moe_routing_sort_reporting": (_I, [_VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _VP]),
+    "deepep_routing_sort_report_words": (_I, [_VP, _I, _I]),
     "deepep_channel_prefix_matrix": (_I, [_VP, _I, _I, _I, _VP, _VP]),
     "deepep_pack_rows": (_I, [_VP, _VP, _VP, _VP, _I64, _I, _I, _I, _VP, _VP, _VP]),
     "deepep_pack_rows_by_rank": (_I, [_VP, _VP, _VP, _VP, _VP, _I, _I64, _I, _I, _I, _VP, _VP, _VP]),

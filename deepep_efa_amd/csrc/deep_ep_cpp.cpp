@@ -773,36 +773,43 @@ static std::tuple<torch::Tensor, torch::Tensor> per_token_cast_to_fp8(const torc
     return {x_fp8, scales};
 }
 
-// A word of pinned memory that a kernel stores a result to and the host polls.  Reading the same 8 bytes back
-// with a copy and a synchronisation takes 16 us of an idle stream (the copy is a kernel of its own, and the wait
-// ends when the whole stream is done); the poll ends 5.5 us after the launch, while the kernel may still run.
-class HostWord {
+// Words of pinned memory that the workgroups of a kernel store to when they are done and the host polls.  Reading 8
+// bytes back with a copy and a synchronisation takes 16 us of an idle stream (the copy is a kernel of its own); a launch
+// and a synchronisation take 11 us, a launch and the poll 6.
+class HostWords {
     at::DataPtr memory;
-    std::atomic<int64_t>* word;
+    std::atomic<int64_t>* words;
+    int count;
     static constexpr int64_t kUnset = INT64_MIN;
 
 public:
-    HostWord() : memory(at::getHostAllocator(at::kCUDA)->allocate(sizeof(int64_t))) {
+    explicit HostWords(int n) : memory(at::getHostAllocator(at::kCUDA)->allocate(sizeof(int64_t) * size_t(n))), count(n) {
         static_assert(sizeof(std::atomic<int64_t>) == sizeof(int64_t));
-        word = new (memory.get()) std::atomic<int64_t>(kUnset);
+        words = static_cast<std::atomic<int64_t>*>(memory.get());
+        for (int i = 0; i < n; ++i) new (words + i) std::atomic<int64_t>(kUnset);
     }
-    int64_t* device_pointer() const { return reinterpret_cast<int64_t*>(word); }
-    // Waits for the value; `stream` is the one whose kernel stores it.  A stream that is busy for long is waited
-    // for in the ordinary way, which also reports what went wrong on it.
+    int64_t* device_pointer() const { return reinterpret_cast<int64_t*>(words); }
+    // Waits for all words and returns the last; `stream` is the one whose kernel stores them.  A stream that is busy
+    // for long is waited for in the ordinary way, which also reports what went wrong on it.
     int64_t wait(hipStream_t stream) const {
         pybind11::gil_scoped_release release;
         const auto began = std::chrono::steady_clock::now();
-        for (int spins = 0; word->load(std::memory_order_acquire) == kUnset;) {
+        int spins = 0;
+        for (int i = 0; i < count;) {
+            if (words[i].load(std::memory_order_acquire) != kUnset) {
+                ++i;
+                continue;
+            }
             __builtin_ia32_pause();
             if (++spins % 1024 == 0 and std::chrono::steady_clock::now() - began > std::chrono::milliseconds(1)) {
                 const hipError_t e = hipStreamSynchronize(stream);
                 if (e != hipSuccess) throw EPException("HIP", "deep_ep_cpp.cpp", __LINE__, hipGetErrorString(e));
-                break;
+                for (; i < count; ++i)
+                    if (words[i].load(std::memory_order_acquire) == kUnset)
+                        throw EPException("HIP", "deep_ep_cpp.cpp", __LINE__, "the kernel did not report its end");
             }
         }
-        const int64_t value = word->load(std::memory_order_acquire);
-        if (value == kUnset) throw EPException("HIP", "deep_ep_cpp.cpp", __LINE__, "the kernel did not report its total");
-        return value;
+        return words[count - 1].load(std::memory_order_acquire);
     }
 };
 
@@ -827,14 +834,15 @@ static std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, int64_t, torch::T
     torch::Tensor row_of_pair;
     if (with_positions) row_of_pair = b.take(positions_at, {num_tokens, num_ranks}, torch::kInt32);
     uint8_t* base = b.block.data_ptr<uint8_t>();
-    const HostWord total_word;
+    const auto* member = reinterpret_cast<const uint8_t*>(is_token_in_rank.data_ptr<bool>());
+    const HostWords report(deepep_routing_sort_report_words(member, num_tokens, num_ranks));
     const hipStream_t stream = current_stream();
-    abi_check(deepep_moe_routing_sort_total(
-        reinterpret_cast<const uint8_t*>(is_token_in_rank.data_ptr<bool>()), num_tokens, num_ranks,
+    abi_check(deepep_moe_routing_sort_reporting(
+        member, num_tokens, num_ranks,
         reinterpret_cast<int64_t*>(base + ids_at), send_counts.data_ptr<int>(), send_cumsum.data_ptr<int64_t>(),
-        with_positions and num_tokens > 0 ? row_of_pair.data_ptr<int>() : nullptr, total_word.device_pointer(),
+        with_positions and num_tokens > 0 ? row_of_pair.data_ptr<int>() : nullptr, report.device_pointer(),
         base + ws_at, size_t(ws_bytes), stream));
-    const int64_t total = total_word.wait(stream);
+    const int64_t total = report.wait(stream);
     return {b.take(ids_at, {total}, torch::kInt64), send_counts, send_cumsum, total, row_of_pair};
 }
 

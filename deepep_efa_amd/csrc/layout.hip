@@ -140,11 +140,18 @@ __global__ __launch_bounds__(kLayoutThreads) void layout_reduce_kernel(const int
         per_node[j - num_experts - num_ranks] = sum;
 }
 
-// The total of a routing sort into memory the host reads while the stream runs on (null: nobody asked).  One
-// 8-byte store at system scope: a host that polls it sees the whole value or the old one.
-__device__ __forceinline__ void tell_host_total(int64_t* total_host, int64_t total) {
-    if (total_host != nullptr)
-        __hip_atomic_store(total_host, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+// Tells a host that polls `report` that this workgroup of a routing sort is done (null: nobody asked): one word a
+// workgroup, stored when everything the workgroup wrote is in memory that every stream, copy engine and the host see.
+// So a host that has seen all words may use the results from another stream too, as after a wait for this one.  (Told
+// the total as soon as it is known, the host is 2 to 3 us further ahead -- 131, 4096 and 12289 tokens through the whole
+// dispatch side 38.5, 130.4, 412.5 us against 40.7, 132.5, 415.5 -- and a reader on another stream gets what the list
+// held before.)  The whole workgroup takes part; `value` is thread 0's.
+__device__ __forceinline__ void report_done(int64_t* report, int64_t value) {
+    if (report == nullptr) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have reached the XCD's L2
+    __syncthreads();
+    if (threadIdx.x == 0)  // the release writes that L2 back
+        __hip_atomic_store(report + blockIdx.x, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------------
@@ -163,7 +170,8 @@ constexpr int kSortChunk = 1024;
 template <bool kScatter>
 __global__ __launch_bounds__(kSortChunk) void routing_sort_pass_kernel(
     const uint8_t* __restrict__ is_token_in_rank, int num_tokens, int num_ranks, int32_t* __restrict__ chunk_table,
-    int64_t* __restrict__ sorted_token_ids, int32_t* __restrict__ row_of_pair) {
+    int64_t* __restrict__ sorted_token_ids, int32_t* __restrict__ row_of_pair, const int64_t* __restrict__ total,
+    int64_t* __restrict__ report) {
     extern __shared__ int32_t wave_cnt[];  // [16][R]
     const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block();
     const int c = blockIdx.x;
@@ -200,13 +208,14 @@ __global__ __launch_bounds__(kSortChunk) void routing_sort_pass_kernel(
             if (in) sorted_token_ids[pos] = t;
             if (row_of_pair != nullptr && t < num_tokens) row_of_pair[int64_t(t) * num_ranks + r] = in ? pos : -1;
         }
+        report_done(report, report != nullptr ? *total : 0);
     }
 }
 
 __global__ __launch_bounds__(256) void routing_sort_scan_kernel(int32_t* __restrict__ chunk_table, int num_chunks,
                                                                 int num_ranks, int32_t* __restrict__ send_counts,
                                                                 int64_t* __restrict__ send_cumsum,
-                                                                int64_t* __restrict__ total_host) {
+                                                                int64_t* __restrict__ report) {
     extern __shared__ int64_t rank_base[];  // [R + 1]
     const int tid = threadIdx.x;
     for (int r = tid; r < num_ranks; r += 256) {
@@ -219,7 +228,6 @@ __global__ __launch_bounds__(256) void routing_sort_scan_kernel(int32_t* __restr
     if (tid == 0) {
         rank_base[0] = 0;
         for (int r = 0; r < num_ranks; ++r) rank_base[r + 1] += rank_base[r];
-        tell_host_total(total_host, rank_base[num_ranks]);
     }
     __syncthreads();
     for (int r = tid; r <= num_ranks; r += 256) send_cumsum[r] = rank_base[r];
@@ -231,6 +239,7 @@ __global__ __launch_bounds__(256) void routing_sort_scan_kernel(int32_t* __restr
             run += cnt;
         }
     }
+    report_done(report, rank_base[num_ranks]);
 }
 
 // ---------------------------------------------------------------------
@@ -261,7 +270,7 @@ __device__ __forceinline__ uint64_t membership_mask(const uint8_t* row, int num_
 __global__ __launch_bounds__(kSortChunk) void routing_sort_single_kernel(
     const uint8_t* __restrict__ is_token_in_rank, int num_tokens, int num_ranks, int tokens_per_thread,
     int32_t* __restrict__ send_counts, int64_t* __restrict__ send_cumsum, int64_t* __restrict__ sorted_token_ids,
-    int32_t* __restrict__ row_of_pair, int64_t* __restrict__ total_host) {
+    int32_t* __restrict__ row_of_pair, int64_t* __restrict__ report) {
     constexpr int kWaves = kSortChunk / kWave;
     __shared__ int32_t wave_own[kWaves];    // tokens of this rank in each wave
     __shared__ int32_t wave_lower[kWaves];  // memberships of lower ranks in each wave
@@ -305,11 +314,9 @@ __global__ __launch_bounds__(kSortChunk) void routing_sort_single_kernel(
     if (tid == 0) {
         send_counts[r] = total;
         send_cumsum[r] = base;
-        if (r == num_ranks - 1) {
-            send_cumsum[num_ranks] = int64_t(base) + total;
-            tell_host_total(total_host, int64_t(base) + total);
-        }
+        if (r == num_ranks - 1) send_cumsum[num_ranks] = int64_t(base) + total;
     }
+    report_done(report, int64_t(base) + total);  // the last rank's end is the total
 }
 
 // ---------------------------------------------------------------------
@@ -318,8 +325,7 @@ __global__ __launch_bounds__(kSortChunk) void routing_sort_single_kernel(
 // word up eight at a time, once over all tokens and once over those before its own: the first gives where every
 // rank's ids begin, the second where its own tokens' ids do.  Against one workgroup per rank, a token's row of
 // row_of_pair is written in one piece, and the loads are independent of one another; against three launches
-// (count, scan, scatter) it is one.  The total goes to the host before any id is written.  What bounds it is
-// latency: about three memory round trips.
+// (count, scan, scatter) it is one.  What bounds it is latency: about three memory round trips.
 // ---------------------------------------------------------------------
 constexpr int kWideSortTokens = 256;    // tokens per workgroup
 constexpr int kWideSortThreads = 1024;  // 256 where one workgroup has all the tokens
@@ -335,12 +341,13 @@ template <int kWords, int kThreads>  // 8-byte words of a token's row: ranks / 8
 __global__ __launch_bounds__(kThreads) void routing_sort_wide_kernel(
     const uint64_t* __restrict__ is_token_in_rank, int num_tokens, int32_t* __restrict__ send_counts,
     int64_t* __restrict__ send_cumsum, int64_t* __restrict__ sorted_token_ids, int32_t* __restrict__ row_of_pair,
-    int64_t* __restrict__ total_host) {
+    int64_t* __restrict__ report) {
     constexpr int kRanks = kWords * 8, kWaves = kThreads / kWave, kAhead = kWords <= 2 ? 4 : 2;
     constexpr int kTokenWaves = kWideSortTokens / kWave, kRankShares = kWaves / kTokenWaves;
     __shared__ int32_t wave_all[kWaves][kRanks], wave_before[kWaves][kRanks];
     __shared__ int32_t start[kRanks];                // where the ids of this workgroup's tokens begin, per rank
     __shared__ int32_t chunk_cnt[kTokenWaves][kRanks];
+    __shared__ int32_t total_of_all;
     const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block();
     const int begin = blockIdx.x * kWideSortTokens;
     // this thread's own token, loaded with the rest: wave w has tokens (w % 4) * 64 + lane
@@ -409,11 +416,9 @@ __global__ __launch_bounds__(kThreads) void routing_sort_wide_kernel(
             for (int w2 = 0; w2 < kWaves; ++w2) total += wave_all[w2][lane], ahead += wave_before[w2][lane];
         const int incl = wave_inclusive_sum(total);
         if (lane < kRanks) start[lane] = incl - total + ahead;
+        if (lane == kRanks - 1) total_of_all = incl;
         if (blockIdx.x == 0) {
-            if (lane == kRanks - 1) {
-                tell_host_total(total_host, incl);
-                send_cumsum[kRanks] = incl;
-            }
+            if (lane == kRanks - 1) send_cumsum[kRanks] = incl;
             if (lane < kRanks) send_counts[lane] = total, send_cumsum[lane] = incl - total;
         }
     }
@@ -435,6 +440,7 @@ __global__ __launch_bounds__(kThreads) void routing_sort_wide_kernel(
         if (in) sorted_token_ids[pos] = own;
         if (row_of_pair != nullptr && own < num_tokens) row_of_pair[int64_t(own) * kRanks + r] = in ? pos : -1;
     }
+    report_done(report, total_of_all);
 }
 
 // ---------------------------------------------------------------------
@@ -671,34 +677,47 @@ size_t deepep_routing_sort_workspace_bytes(int num_tokens, int num_ranks) {
     return size_t((chunks < 1 ? 1 : chunks) * num_ranks * 4);
 }
 
-int deepep_moe_routing_sort_total(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
-                                  int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
-                                  int32_t* row_of_pair, int64_t* total_host, void* workspace, size_t workspace_bytes,
-                                  void* stream) {
+// Every workgroup of the wide form reads the whole matrix: 512 KB take one of them about 5 us, less than
+// the two further launches of the chunked form; past that its work grows with the square of the batch.
+static bool sort_is_wide(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks) {
+    return (num_ranks == 8 || num_ranks == 16 || num_ranks == 32 || num_ranks == 64) &&
+           (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 &&
+           int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
+}
+static bool sort_is_single(int num_tokens, int num_ranks) {
+    return num_tokens <= kSortChunk * kSingleSortTokensPerThread && num_ranks <= 64;
+}
+
+int deepep_routing_sort_report_words(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks) {
+    if (num_tokens <= 0) return sort_is_single(0, num_ranks) && !sort_is_wide(is_token_in_rank, 0, num_ranks) ? num_ranks : 1;
+    if (sort_is_wide(is_token_in_rank, num_tokens, num_ranks)) return (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
+    if (sort_is_single(num_tokens, num_ranks)) return num_ranks;
+    return (num_tokens + kSortChunk - 1) / kSortChunk;
+}
+
+int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
+                                      int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
+                                      int32_t* row_of_pair, int64_t* report_host, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
     clear_error();
     EP_HOST_ASSERT(num_tokens >= 0 && num_ranks > 0 && num_ranks <= 1024);
     EP_HOST_ASSERT(send_counts != nullptr && send_cumsum != nullptr);
     EP_HOST_ASSERT(num_tokens == 0 || (is_token_in_rank != nullptr && sorted_token_ids != nullptr));
-    EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(total_host) & 7) == 0);
+    EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(report_host) & 7) == 0);
     const int chunks = num_tokens == 0 ? 1 : (num_tokens + kSortChunk - 1) / kSortChunk;
     EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(chunks) * num_ranks * 4);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    // Every workgroup of the wide form reads the whole matrix: 512 KB take one of them about 5 us, less than
-    // the two further launches of the chunked form; past that its work grows with the square of the batch.
-    const bool wide = (num_ranks == 8 || num_ranks == 16 || num_ranks == 32 || num_ranks == 64) &&
-                      (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 &&
-                      int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
-    if (wide) {
+    if (sort_is_wide(is_token_in_rank, num_tokens, num_ranks)) {
         const int blocks = num_tokens == 0 ? 1 : (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
         const uint64_t* rows = reinterpret_cast<const uint64_t*>(is_token_in_rank);
 #define DEEPEP_LAUNCH_SORT(WORDS)                                                                                 \
     do {                                                                                                          \
         if (blocks == 1)                                                                                          \
             routing_sort_wide_kernel<WORDS, kWideSortTokens><<<1, kWideSortTokens, 0, s>>>(                       \
-                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, total_host);           \
+                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host);           \
         else                                                                                                      \
             routing_sort_wide_kernel<WORDS, kWideSortThreads><<<blocks, kWideSortThreads, 0, s>>>(                \
-                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, total_host);           \
+                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host);           \
     } while (0)
         switch (num_ranks) {
             case 8: DEEPEP_LAUNCH_SORT(1); break;
@@ -710,25 +729,27 @@ int deepep_moe_routing_sort_total(const uint8_t* is_token_in_rank, int num_token
         EP_LAUNCH_CHECK();
         return 0;
     }
-    if (num_tokens <= kSortChunk * kSingleSortTokensPerThread && num_ranks <= 64) {
+    if (sort_is_single(num_tokens, num_ranks)) {
         const int per_thread = num_tokens == 0 ? 1 : (num_tokens + kSortChunk - 1) / kSortChunk;
         routing_sort_single_kernel<<<num_ranks, kSortChunk, 0, s>>>(is_token_in_rank, num_tokens, num_ranks, per_thread,
                                                                    send_counts, send_cumsum, sorted_token_ids,
-                                                                   row_of_pair, total_host);
+                                                                   row_of_pair, report_host);
         EP_LAUNCH_CHECK();
         return 0;
     }
     int32_t* table = reinterpret_cast<int32_t*>(workspace);
     const size_t lds = size_t(kSortChunk / kWave) * num_ranks * 4;
     routing_sort_pass_kernel<false><<<chunks, kSortChunk, lds, s>>>(is_token_in_rank, num_tokens, num_ranks, table,
-                                                                    sorted_token_ids, nullptr);
+                                                                    sorted_token_ids, nullptr, nullptr, nullptr);
     EP_LAUNCH_CHECK();
     routing_sort_scan_kernel<<<1, 256, size_t(num_ranks + 1) * 8, s>>>(table, chunks, num_ranks, send_counts,
-                                                                       send_cumsum, total_host);
+                                                                       send_cumsum,
+                                                                       num_tokens == 0 ? report_host : nullptr);
     EP_LAUNCH_CHECK();
     if (num_tokens > 0) {
         routing_sort_pass_kernel<true><<<chunks, kSortChunk, lds, s>>>(is_token_in_rank, num_tokens, num_ranks,
-                                                                       table, sorted_token_ids, row_of_pair);
+                                                                       table, sorted_token_ids, row_of_pair,
+                                                                       send_cumsum + num_ranks, report_host);
         EP_LAUNCH_CHECK();
     }
     return 0;
@@ -737,8 +758,8 @@ int deepep_moe_routing_sort_total(const uint8_t* is_token_in_rank, int num_token
 int deepep_moe_routing_sort(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
                             int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
                             int32_t* row_of_pair, void* workspace, size_t workspace_bytes, void* stream) {
-    return deepep_moe_routing_sort_total(is_token_in_rank, num_tokens, num_ranks, sorted_token_ids, send_counts,
-                                         send_cumsum, row_of_pair, nullptr, workspace, workspace_bytes, stream);
+    return deepep_moe_routing_sort_reporting(is_token_in_rank, num_tokens, num_ranks, sorted_token_ids, send_counts,
+                                             send_cumsum, row_of_pair, nullptr, workspace, workspace_bytes, stream);
 }
 
 int deepep_channel_prefix_matrix(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks, int num_channels,

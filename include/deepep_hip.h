@@ -42,7 +42,7 @@ const char* deepep_last_error(void);
 
 /* ABI revision of this header; bumped on any signature change.  deepep_abi_version() returns the
  * revision the library was built from: a binding compares the two before its first call. */
-#define DEEPEP_HIP_ABI_VERSION 10
+#define DEEPEP_HIP_ABI_VERSION 11
 int deepep_abi_version(void);
 
 /* ------------------------------------------------------------------ */
@@ -116,13 +116,19 @@ int deepep_moe_routing_sort(const uint8_t* is_token_in_rank, int num_tokens, int
                             int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
                             int32_t* row_of_pair, void* workspace, size_t workspace_bytes, void* stream);
 
-/* The same, with the total also stored to `total_host` (8 bytes the device can write and the host read, pinned
- * memory; NULL: not wanted) as soon as the counts are known, ahead of the ids: a host that needs the total to
- * size what comes next polls it instead of copying send_cumsum[R] back behind the whole sort. */
-int deepep_moe_routing_sort_total(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
-                                  int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
-                                  int32_t* row_of_pair, int64_t* total_host,
-                                  void* workspace, size_t workspace_bytes, void* stream);
+/* The same, reporting to a host that needs the total to size what comes next, so that it polls instead of copying
+ * send_cumsum[R] back behind the sort.
+ *   report_host  deepep_routing_sort_report_words() words of 8 bytes that the device can write and the host read
+ *                (pinned memory), set to a negative value by the caller; NULL: no report.
+ * Every workgroup stores one word when what it wrote is visible to the whole device and the host: when no word is
+ * negative any more, all outputs may be used from any stream, and the last word is the total. */
+int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
+                                      int64_t* sorted_token_ids, int32_t* send_counts, int64_t* send_cumsum,
+                                      int32_t* row_of_pair, int64_t* report_host,
+                                      void* workspace, size_t workspace_bytes, void* stream);
+
+/* Words that deepep_moe_routing_sort_reporting stores for the same first three arguments (at least 1). */
+int deepep_routing_sort_report_words(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks);
 
 /* channel_prefix_matrix[d, c] = number of tokens bound for rank d in
  * channels 0..c, channel c owning tokens [min(c*ceil(T/C),T), min(+ceil(T/C),T)).

@@ -165,6 +165,55 @@ def test_layout_sort_and_prefix_where_their_launch_forms_meet(t, r):
         assert torch.equal(normal.channel_prefix_matrix(is_in, c).cpu(), O.channel_prefix_matrix(want[3], c))
 
 
+# every form of the sort: one workgroup a rank, one per 256 tokens, count + scan + scatter; no tokens at all
+SORT_FORMS = [(0, 8), (0, 9), (0, 72), (1, 9), (300, 24), (131, 16), (5000, 16), (8192, 64), (40000, 8), (9000, 12),
+              (70000, 8), (3000, 72), (1, 130)]
+
+
+@pytest.mark.parametrize("t,r", SORT_FORMS)
+def test_routing_sort_reports_every_workgroup(capi, t, r):
+    """As many words as promised are set, the last to the total, and none beyond them."""
+    lib = capi.load()
+    is_in = torch.rand((t, r), generator=torch.Generator().manual_seed(t + r)) < 0.3
+    dev = is_in.cuda()
+    words = lib.deepep_routing_sort_report_words(capi.ptr(dev), t, r)
+    report = torch.full((words + 16,), -1, dtype=torch.int64, pin_memory=True)
+    ids = torch.empty(max(1, t * r), dtype=torch.int64, device="cuda")
+    counts = torch.empty(r, dtype=torch.int32, device="cuda")
+    cumsum = torch.empty(r + 1, dtype=torch.int64, device="cuda")
+    ws = torch.empty(max(256, lib.deepep_routing_sort_workspace_bytes(t, r)), dtype=torch.uint8, device="cuda")
+    capi.check(lib.deepep_moe_routing_sort_reporting(
+        capi.ptr(dev), t, r, capi.ptr(ids), capi.ptr(counts), capi.ptr(cumsum), None, capi.ptr(report), capi.ptr(ws),
+        ws.numel(), stream()))
+    torch.cuda.synchronize()
+    assert words >= 1 and (report[:words] >= 0).all() and (report[words:] == -1).all()
+    assert int(report[words - 1]) == int(is_in.sum()) == int(cumsum[r])
+
+
+@pytest.mark.parametrize("t,r", [f for f in SORT_FORMS if f[0] > 0] + [(300000, 8)])
+def test_routing_sort_results_are_there_for_another_stream(t, r):
+    """The sort waits for its total, and a caller may then read what it returned from any stream, without an event."""
+    from deepep_efa_amd import normal
+    is_in = torch.rand((t, r), generator=torch.Generator().manual_seed(t)) < 0.4
+    dev = is_in.cuda()
+    w_ids, w_counts, w_cumsum, w_total = O.moe_routing_sort(is_in)
+    want = (w_ids, w_counts, w_cumsum, _want_row_of_pair(is_in, w_ids, w_cumsum))
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+    copies = [torch.full(v.shape, -7, dtype=v.dtype, device="cuda") for v in want]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        with torch.cuda.stream(mine):
+            ids, counts, cumsum, total, inverse = normal.moe_routing_sort_with_positions(dev)
+        with torch.cuda.stream(other):
+            for copy, v in zip(copies, (ids, counts, cumsum, inverse)):
+                copy.copy_(v)
+        torch.cuda.synchronize()
+        assert total == int(w_total)
+        for copy, v, w in zip(copies, (ids, counts, cumsum, inverse), want):
+            assert torch.equal(copy.cpu(), w)
+            v.fill_(-7)  # what the next round's block holds, unless the sort has written it
+
+
 @pytest.mark.parametrize("seed", range(int(os.environ.get("DEEPEP_TEST_RANDOM_SHAPES", "16"))))
 def test_layout_sort_prefix_seeded_random_shapes(capi, seed):
     """Layout, routing sort and channel prefix on shapes nobody picked by hand (both sort paths)."""
