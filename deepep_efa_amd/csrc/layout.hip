@@ -320,15 +320,16 @@ __global__ __launch_bounds__(kSortChunk) void routing_sort_single_kernel(
 }
 
 // ---------------------------------------------------------------------
-// The same sort in one launch for 8, 16, 32 or 64 ranks and a matrix of up to 512 KB.  One workgroup per 256
+// The same sort in one launch for a multiple of 8 ranks up to 64 and a matrix of up to 512 KB.  One workgroup per 256
 // tokens; each reads the whole matrix (from L2), 8 ranks of a token per 8-byte word, adding the bool bytes of a
 // word up eight at a time, once over all tokens and once over those before its own: the first gives where every
 // rank's ids begin, the second where its own tokens' ids do.  Against one workgroup per rank, a token's row of
 // row_of_pair is written in one piece, and the loads are independent of one another; against three launches
-// (count, scan, scatter) it is one.  What bounds it is latency: about three memory round trips.
+// (count, scan, scatter) it is one.  What bounds it is the sums over a wave, one for every two ranks and pass, which
+// small batches pay for as much as large ones.
 // ---------------------------------------------------------------------
-constexpr int kWideSortTokens = 256;    // tokens per workgroup
-constexpr int kWideSortThreads = 1024;  // 256 where one workgroup has all the tokens
+constexpr int kWideSortTokens = 256;  // tokens per workgroup
+constexpr int kWideSortThreads = 1024;
 constexpr int64_t kWideSortMaxBytes = 512 * 1024;
 
 // 1 in every byte of v that is not zero.
@@ -337,11 +338,12 @@ __device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {
     return v & 0x0101010101010101ull;
 }
 
-template <int kWords, int kThreads>  // 8-byte words of a token's row: ranks / 8
-__global__ __launch_bounds__(kThreads) void routing_sort_wide_kernel(
+template <int kWords>  // 8-byte words of a token's row: ranks / 8
+__global__ __launch_bounds__(kWideSortThreads) void routing_sort_wide_kernel(
     const uint64_t* __restrict__ is_token_in_rank, int num_tokens, int32_t* __restrict__ send_counts,
     int64_t* __restrict__ send_cumsum, int64_t* __restrict__ sorted_token_ids, int32_t* __restrict__ row_of_pair,
     int64_t* __restrict__ report) {
+    constexpr int kThreads = kWideSortThreads;
     constexpr int kRanks = kWords * 8, kWaves = kThreads / kWave, kAhead = kWords <= 2 ? 4 : 2;
     constexpr int kTokenWaves = kWideSortTokens / kWave, kRankShares = kWaves / kTokenWaves;
     __shared__ int32_t wave_all[kWaves][kRanks], wave_before[kWaves][kRanks];
@@ -356,7 +358,7 @@ __global__ __launch_bounds__(kThreads) void routing_sort_wide_kernel(
     uint64_t own_row[kWords];
 #pragma unroll
     for (int q = 0; q < kWords; ++q) {
-        own_row[q] = num_tokens > 0 ? is_token_in_rank[int64_t(own < num_tokens ? own : num_tokens - 1) * kWords + q] : 0;
+        own_row[q] = is_token_in_rank[int64_t(own < num_tokens ? own : num_tokens - 1) * kWords + q];
         if (own >= num_tokens) own_row[q] = 0;
     }
     uint64_t all[kWords], before[kWords];
@@ -677,22 +679,29 @@ size_t deepep_routing_sort_workspace_bytes(int num_tokens, int num_ranks) {
     return size_t((chunks < 1 ? 1 : chunks) * num_ranks * 4);
 }
 
-// Every workgroup of the wide form reads the whole matrix: 512 KB take one of them about 5 us, less than
-// the two further launches of the chunked form; past that its work grows with the square of the batch.
+// Which form sorts.  Microseconds of the wide form against one workgroup per rank, with row_of_pair:
+//   ranks       8            16           32            64
+//   131 tokens  3.4 / 3.1    4.9 / 3.3    8.0 / 3.5     15.0 / 4.1
+//   2048        4.5 / 4.3    6.7 / 4.7    10.9 / 6.0    20.9 / 12.6
+//   2560        4.5 / 4.8    6.7 / 5.6    11.5 / 7.9    22.0 / 14.7
+//   4096        4.5 / 6.0    6.9 / 7.2    12.0 / 12.7   23.2 / 23.3
+//   8192        5.2 / 10.0   8.0 / 15.0   14.3 / 23.2   27.7 / 41.7
+// 24, 40, 48 and 56 ranks meet at 4096 tokens too (9.3 / 9.4 to 20.1 / 20.4), and without row_of_pair nothing moves
+// the line by more than 1 us.  Upwards every workgroup reads the whole matrix: at 512 KB that still beats the three
+// launches (8 ranks, 20000 tokens 7.2 against 16.5; 24 ranks, 12289 12.7 against 34.2; 48 ranks, 9300 21.5 against
+// 76.9), past that its work grows with the square of the batch.
 static bool sort_is_wide(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks) {
-    return (num_ranks == 8 || num_ranks == 16 || num_ranks == 32 || num_ranks == 64) &&
-           (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 &&
-           int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
+    return num_ranks % 8 == 0 && num_ranks <= 64 && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 &&
+           num_tokens >= (num_ranks == 8 ? 2560 : 4096) && int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
 }
 static bool sort_is_single(int num_tokens, int num_ranks) {
     return num_tokens <= kSortChunk * kSingleSortTokensPerThread && num_ranks <= 64;
 }
 
 int deepep_routing_sort_report_words(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks) {
-    if (num_tokens <= 0) return sort_is_single(0, num_ranks) && !sort_is_wide(is_token_in_rank, 0, num_ranks) ? num_ranks : 1;
     if (sort_is_wide(is_token_in_rank, num_tokens, num_ranks)) return (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
     if (sort_is_single(num_tokens, num_ranks)) return num_ranks;
-    return (num_tokens + kSortChunk - 1) / kSortChunk;
+    return num_tokens <= 0 ? 1 : (num_tokens + kSortChunk - 1) / kSortChunk;
 }
 
 int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks,
@@ -708,22 +717,22 @@ int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_t
     EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(chunks) * num_ranks * 4);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (sort_is_wide(is_token_in_rank, num_tokens, num_ranks)) {
-        const int blocks = num_tokens == 0 ? 1 : (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
+        const int blocks = (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
         const uint64_t* rows = reinterpret_cast<const uint64_t*>(is_token_in_rank);
-#define DEEPEP_LAUNCH_SORT(WORDS)                                                                                 \
-    do {                                                                                                          \
-        if (blocks == 1)                                                                                          \
-            routing_sort_wide_kernel<WORDS, kWideSortTokens><<<1, kWideSortTokens, 0, s>>>(                       \
-                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host);           \
-        else                                                                                                      \
-            routing_sort_wide_kernel<WORDS, kWideSortThreads><<<blocks, kWideSortThreads, 0, s>>>(                \
-                rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host);           \
-    } while (0)
-        switch (num_ranks) {
-            case 8: DEEPEP_LAUNCH_SORT(1); break;
-            case 16: DEEPEP_LAUNCH_SORT(2); break;
-            case 32: DEEPEP_LAUNCH_SORT(4); break;
-            default: DEEPEP_LAUNCH_SORT(8); break;
+#define DEEPEP_LAUNCH_SORT(WORDS)                                                                  \
+    case WORDS:                                                                                    \
+        routing_sort_wide_kernel<WORDS><<<blocks, kWideSortThreads, 0, s>>>(                       \
+            rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host); \
+        break
+        switch (num_ranks / 8) {
+            DEEPEP_LAUNCH_SORT(1);
+            DEEPEP_LAUNCH_SORT(2);
+            DEEPEP_LAUNCH_SORT(3);
+            DEEPEP_LAUNCH_SORT(4);
+            DEEPEP_LAUNCH_SORT(5);
+            DEEPEP_LAUNCH_SORT(6);
+            DEEPEP_LAUNCH_SORT(7);
+            DEEPEP_LAUNCH_SORT(8);
         }
 #undef DEEPEP_LAUNCH_SORT
         EP_LAUNCH_CHECK();

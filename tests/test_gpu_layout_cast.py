@@ -168,6 +168,9 @@ def test_layout_sort_and_prefix_where_their_launch_forms_meet(t, r):
 # every form of the sort: one workgroup a rank, one per 256 tokens, count + scan + scatter; no tokens at all
 SORT_FORMS = [(0, 8), (0, 9), (0, 72), (1, 9), (300, 24), (131, 16), (5000, 16), (8192, 64), (40000, 8), (9000, 12),
               (70000, 8), (3000, 72), (1, 130)]
+# either side of the lines between them, and every width of a token's row in words
+SORT_FORMS += [(2559, 8), (2560, 8), (4095, 16), (4096, 16), (4096, 24), (13107, 40), (13108, 40), (10922, 48),
+               (10923, 48), (4097, 56), (16385, 32)]
 
 
 @pytest.mark.parametrize("t,r", SORT_FORMS)
@@ -188,6 +191,26 @@ def test_routing_sort_reports_every_workgroup(capi, t, r):
     torch.cuda.synchronize()
     assert words >= 1 and (report[:words] >= 0).all() and (report[words:] == -1).all()
     assert int(report[words - 1]) == int(is_in.sum()) == int(cumsum[r])
+
+
+@pytest.mark.parametrize("t,r", [(1, 8), (131, 16), (2000, 64), (4096, 48)])
+def test_routing_sort_takes_the_form_measured_fastest(capi, t, r):
+    """One workgroup per rank up to 4095 tokens (2559 at 8 ranks), where the form that adds up eight ranks at a time
+    is up to four times as slow; a matrix whose address does not allow 8-byte loads never takes that form."""
+    lib = capi.load()
+    assert lib.deepep_routing_sort_report_words(None, t, r) == (r if t < 4096 else (t + 255) // 256)
+    assert lib.deepep_routing_sort_report_words(4, t, r) == r
+    is_in = torch.rand((t, r), generator=torch.Generator().manual_seed(t + r)) < 0.3
+    shifted = torch.zeros(t * r + 4, dtype=torch.bool, device="cuda")[4:].view(t, r)
+    shifted.copy_(is_in)
+    ids, counts, cumsum = (torch.empty(n, dtype=d, device="cuda") for n, d in
+                           ((t * r, torch.int64), (r, torch.int32), (r + 1, torch.int64)))
+    ws = torch.empty(max(256, lib.deepep_routing_sort_workspace_bytes(t, r)), dtype=torch.uint8, device="cuda")
+    capi.check(lib.deepep_moe_routing_sort(capi.ptr(shifted), t, r, capi.ptr(ids), capi.ptr(counts), capi.ptr(cumsum),
+                                           None, capi.ptr(ws), ws.numel(), stream()))
+    w_ids, w_counts, w_cumsum, w_total = O.moe_routing_sort(is_in)
+    assert torch.equal(ids[:int(w_total)].cpu(), w_ids)
+    assert torch.equal(counts.cpu(), w_counts) and torch.equal(cumsum.cpu(), w_cumsum)
 
 
 @pytest.mark.parametrize("t,r", [f for f in SORT_FORMS if f[0] > 0] + [(300000, 8)])
