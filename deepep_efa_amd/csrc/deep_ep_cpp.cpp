@@ -500,16 +500,10 @@ struct Buffer {
         return ll;
     }
 
-    // Rows a batch of num_tokens probably receives: what a balanced world sends or, if more, what the last batch
-    // received, in proportion (a batch of less than a quarter of the tokens says too little).  A hint: kernels
-    // and grids are chosen by it, never results.
+    // Rows a batch of num_tokens probably receives, from what the last one did.
     int64_t rows_expected(int num_tokens, int num_topk, int num_experts, int max_tokens) const {
-        const int64_t balanced = std::max<int64_t>(num_tokens, 1) * num_topk;
-        if (observed == nullptr) return balanced;
-        const uint64_t last = observed->load(std::memory_order_relaxed);
-        const int64_t tokens = int64_t(last >> 32), rows = int64_t(last & 0xffffffffu);
-        if (tokens == 0 or tokens * 4 < num_tokens) return balanced;
-        return std::max(balanced, std::min(rows * num_tokens / tokens, int64_t(num_experts) * max_tokens));
+        return deepep_ll_expected_rows(num_tokens, num_topk, num_experts, max_tokens,
+                                       observed != nullptr ? observed->load(std::memory_order_relaxed) : 0);
     }
 
     void stage_peer_rows(LowLatencyCache& c) {

@@ -1384,6 +1384,20 @@ int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx, int num_
                             reinterpret_cast<hipStream_t>(stream), &ra, rows << ra.parts_log2);
 }
 
+// Kernels and grids are chosen by it, never results.  The rows come from the other ranks, so they do not grow with
+// this rank's own tokens: scaled up, 1 token that received 2100 rows made 4 tokens expect 8400 and leave the single
+// launch (a step of 4 tokens 18.8 -> 27.8 us).  They are scaled down, because the ranks leave a prefill together: a
+// decode step of 128 tokens sized by the 32768 rows of one took 35.0 us instead of 18.8.  A hint that is too small
+// costs a looping copy (1000 tokens, 165885 rows: 1550 us sized for 8000, 1199 for what arrives).
+int64_t deepep_ll_expected_rows(int num_tokens, int num_topk, int num_experts, int num_max_dispatch_tokens_per_rank,
+                                uint64_t observed) {
+    const int64_t balanced = std::max<int64_t>(num_tokens, 1) * num_topk;
+    const int64_t tokens = int64_t(observed >> 32), rows = int64_t(observed & 0xffffffffu);
+    if (tokens == 0) return balanced;
+    const int64_t again = num_tokens < tokens ? rows * num_tokens / tokens : rows;
+    return std::max(balanced, std::min(again, int64_t(num_experts) * num_max_dispatch_tokens_per_rank));
+}
+
 int deepep_ll_dispatch(const void* x, const int64_t* topk_idx, int num_tokens, int hidden, int num_topk,
                        int num_experts, int num_ranks, int rank, int num_max_dispatch_tokens_per_rank, int row_format,
                        void* recv_staging, int32_t* recv_count, void* send_slots, int32_t* send_count,

@@ -588,6 +588,11 @@ int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx,
                        int64_t expected_rows, void* workspace, size_t workspace_bytes,
                        void* segment_workspace, size_t segment_workspace_bytes, uint64_t* observed_host, void* stream);
 
+/* expected_rows of a batch of num_tokens, given what deepep_ll_dispatch_observed last stored (0: nothing yet):
+ * num_tokens * num_topk or, if more, the rows of that batch, scaled down for a smaller one. */
+int64_t deepep_ll_expected_rows(int num_tokens, int num_topk, int num_experts, int num_max_dispatch_tokens_per_rank,
+                                uint64_t observed);
+
 /* deepep_ll_combine_send followed by deepep_ll_combine_recv, for a caller
  * whose remote experts' answers are already in combine_staging when the call
  * is made (the reference: Buffer::low_latency_combine,

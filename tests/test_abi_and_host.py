@@ -77,6 +77,27 @@ def test_host_argument_checks_without_a_gpu():
         _capi.check(rc)
 
 
+@pytest.mark.parametrize("tokens,seen_tokens,seen_rows,want", [
+    (128, 0, 0, 1024),          # nothing seen yet: what a balanced world sends
+    (0, 0, 0, 8),
+    (128, 128, 900, 1024),      # less than balanced
+    (128, 128, 5000, 5000),
+    (4, 1, 2100, 2100),         # other ranks' rows do not grow with this rank's tokens
+    (1000, 1, 2100, 8000),
+    (1000, 100, 40000, 40000),
+    (4, 1000, 60000, 240),      # the decode step behind a prefill
+    (0, 1000, 60000, 8),
+    (128, 128, 2 ** 32 - 1, 256 * 128),  # never more than there is room for
+])
+def test_rows_expected_of_a_batch_follow_the_last_one(tokens, seen_tokens, seen_rows, want):
+    from deepep_efa_amd import _capi
+    lib = _capi.load()
+    got = lib.deepep_ll_expected_rows(tokens, 8, 256, 128 if tokens <= 128 else 1024, seen_tokens << 32 | seen_rows)
+    assert got == want
+    if tokens <= 4:  # a decode batch stays in the single launch
+        assert lib.deepep_ll_dispatch_is_single_launch(tokens, 8, 256, 128, got) == 1
+
+
 def test_config_follows_reference_rules():
     import deep_ep
     cfg = deep_ep.Config(20, 6, 256, 6, 250)

@@ -534,6 +534,49 @@ def test_dispatch_and_combine_replay_in_a_hip_graph(deep_ep, num_ranks, rank, t,
     buffer.destroy()
 
 
+def test_batches_that_change_from_call_to_call(deep_ep):
+    """Uneven, skewed and balanced batches in turn through one buffer, each sized by the one before, give what a
+    buffer of their own gives; they take the single launch and the index + copy form in both directions."""
+    num_ranks, rank, m, h, k, e = 16, 0, 640, 512, 8, 64
+
+    def make():
+        return deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=num_ranks,
+                              sim_rank=rank, sim_seed=2)
+
+    def step(buffer, world, x, topk_idx, w):
+        buffer.loopback_set_world(*world)
+        (rows, scales), count, handle, _, _ = buffer.low_latency_dispatch(x, topk_idx, m, e)
+        y = torch.zeros((e // num_ranks, num_ranks * m, h), dtype=torch.bfloat16, device="cuda")
+        for i, n in enumerate(count.tolist()):
+            y[i, :n] = rows[i, :n].bfloat16()
+        combined = buffer.low_latency_combine(y, topk_idx, w, handle)[0]
+        torch.cuda.synchronize()
+        valid = [(rows[i, :n].view(torch.uint8).clone(), scales[i, :n].clone(), handle[0][i, :n].clone())
+                 for i, n in enumerate(count.tolist())]
+        return [count.clone(), handle[1].clone(), combined.clone()] + [v for part in valid for v in part]
+
+    shared, worlds = make(), {}
+    for popularity, tokens in (("zipf", 640), ("uniform", 640), ("zipf", 64)):
+        source = make()
+        source.loopback_synthesise(tokens, h, k, e, popularity, 0, tokens)
+        worlds[popularity, tokens] = tuple(v.clone() for v in source.runtime.loopback_world())
+        source.destroy()
+    received = []
+    for key, own in ((("uniform", 640), 640), (("zipf", 640), 1), (("zipf", 640), 4), (("zipf", 640), 640),
+                     (("uniform", 640), 640), (("zipf", 64), 3), (("zipf", 640), 640), (("zipf", 64), 64)):
+        x_all, topk_all = (v.clone() for v in worlds[key])
+        x, topk_idx = x_all[rank, :own].contiguous(), topk_all[rank, :own].contiguous()
+        w = torch.rand((own, k), generator=torch.Generator().manual_seed(own)).cuda()
+        alone = make()
+        want = step(alone, (x_all, topk_all), x, topk_idx, w)
+        got = step(shared, (x_all, topk_all), x, topk_idx, w)
+        alone.destroy()
+        received.append(int(want[0].sum()))
+        assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want)), (key, own)
+    assert min(received) < 8192 < max(received)
+    shared.destroy()
+
+
 def _small_dispatch(deep_ep):
     buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=4, sim_rank=1)
     g = torch.Generator().manual_seed(3)
