@@ -547,14 +547,20 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // each list ascends, and workgroups 8 apart -- on one XCD, sharing an L2 -- work
 // through one group, so a source row is read once and found in that L2 by the
 // other ranks.  Any routing gives the same result; a skewed one only shares less.
-// The packed rows are stored with the non-temporal hint: otherwise they push the
-// source rows, and whatever the caches hold of others, out again.  Measured
-// (R = 8, 5.3 ranks a token), list order and plain stores with one vector a
-// thread against this: 12289 x 14336 bytes 305 -> 211 us (5.2 TB/s on the bytes
-// that have to move), 4096 x 7168 48.1 -> 27.3 us (6.7), 900 x 7168 10.9 -> 6.7 us.
+// Past 128 MB the packed rows are stored with the non-temporal hint: otherwise they push the source rows, and
+// whatever the caches hold of others, out again.  Below that a transport that reads them next finds them in the
+// memory-side cache (256 MB), which is worth more to the two together than the hint is to the pack.  Microseconds of
+// pack and pack + copy of the packed rows, ordinary stores against the hint (R = 8, four sets of tensors in turn):
+//    19 MB   7.0 / 5.0    13.8 / 15.3     118 MB  35.7 / 21.7   72.4 / 78.0
+//    39 MB  10.0 / 8.9    25.6 / 29.5     129 MB  40.4 / 23.2   83.8 / 85.6
+//    78 MB  24.0 / 15.3   48.8 / 54.2     140 MB  42.0 / 25.3   93.9 / 91.4
+//    97 MB  29.3 / 18.4   59.8 / 65.7     155 MB  48.5 / 27.4  107.2 / 102.5    311 MB  88.7 / 54.6  209 / 197
+// Grouping and hint against list order and ordinary stores: 12289 x 14336 bytes (934 MB) 305 -> 211 us (5.2 TB/s on
+// the bytes that have to move), 4096 x 7168 (155 MB) 48.1 -> 27.3 us (6.7).
 // Half the threads with two vectors each against all with one: 260 -> 211 us.
 // ---------------------------------------------------------------------
 constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of a group: about 2 MB of source rows
+constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
 
 struct PackArgs {
     const uint8_t* src;
@@ -569,6 +575,7 @@ struct PackArgs {
     uint8_t* scale_dst;
 };
 
+template <bool kStream>
 __device__ __forceinline__ void pack_row(const PackArgs& a, int64_t row) {
     const int64_t id = a.ids[row];
     if (id < 0 || id >= a.num_src_rows) return;
@@ -579,8 +586,8 @@ __device__ __forceinline__ void pack_row(const PackArgs& a, int64_t row) {
         const bool second = v + threads < num_vec;
         u32x4 r0 = load_u32x4<false>(s + int64_t(v) * 16), r1 = r0;
         if (second) r1 = load_u32x4<false>(s + int64_t(v + threads) * 16);
-        store_u32x4<true>(d + int64_t(v) * 16, r0);
-        if (second) store_u32x4<true>(d + int64_t(v + threads) * 16, r1);
+        store_u32x4<kStream>(d + int64_t(v) * 16, r0);
+        if (second) store_u32x4<kStream>(d + int64_t(v + threads) * 16, r1);
     }
     if (a.scale_src != nullptr) {
         const uint32_t* ss = reinterpret_cast<const uint32_t*>(a.scale_src + id * a.scale_row_bytes);
@@ -589,12 +596,12 @@ __device__ __forceinline__ void pack_row(const PackArgs& a, int64_t row) {
     }
 }
 
-template <bool kGrouped>
+template <bool kGrouped, bool kStream>
 __global__ __launch_bounds__(512) void pack_rows_kernel(PackArgs a) {
     if constexpr (!kGrouped) {
         int64_t num_rows = *a.num_rows_dev;
         if (num_rows > a.max_rows) num_rows = a.max_rows;
-        for (int64_t i = blockIdx.x; i < num_rows; i += gridDim.x) pack_row(a, i);
+        for (int64_t i = blockIdx.x; i < num_rows; i += gridDim.x) pack_row<kStream>(a, i);
     } else {
         const int lane = lane_id(), xcd = int(blockIdx.x) & 7, i = int(blockIdx.x) >> 3;
         const int g = (i / a.slots) * 8 + xcd;
@@ -615,7 +622,7 @@ __global__ __launch_bounds__(512) void pack_rows_kernel(PackArgs a) {
             const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(begin), r);
             const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(begin >> 32), r);
             const int64_t row = int64_t((uint64_t(hi) << 32) | lo) + slot;
-            if (row >= 0 && row < a.max_rows) pack_row(a, row);
+            if (row >= 0 && row < a.max_rows) pack_row<kStream>(a, row);
         }
     }
 }
@@ -819,6 +826,7 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
     int threads = (row_bytes / 32 + 63) / 64 * 64;  // two vectors a thread
     threads = threads < 64 ? 64 : (threads > 512 ? 512 : threads);
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
+    const bool stream_rows = max_rows * row_bytes > kPackStreamBytes;
     // Below a group's worth of packed rows everything stays in the caches and the grouping's lookup is one more
     // round trip in front of the rows: 6.5 MB 2.9 us against 3.4, 12 MB 3.9 either way, 22 MB 6.7 against 5.0.
     // A wave holds the ranks' parts one a lane, hence the 64.
@@ -828,10 +836,12 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
         const int64_t slots = ((max_rows + (int64_t(1) << a.group_log2) - 1) >> a.group_log2) + num_ranks;
         a.slots = int(slots < (1 << 14) ? slots : (1 << 14));  // the kernel goes round for the rest
         const int64_t blocks = int64_t(a.slots) << a.group_log2;
-        pack_rows_kernel<true><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
+        if (stream_rows) pack_rows_kernel<true, true><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
+        else pack_rows_kernel<true, false><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
     } else {
         const int64_t blocks = max_rows < (int64_t(1) << 22) ? max_rows : int64_t(1) << 22;
-        pack_rows_kernel<false><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
+        if (stream_rows) pack_rows_kernel<false, true><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
+        else pack_rows_kernel<false, false><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
     }
     EP_LAUNCH_CHECK();
     return 0;

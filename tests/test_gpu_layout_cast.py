@@ -307,6 +307,8 @@ def test_pack_rows(capi, rows, row_bytes, scale_bytes):
     (6000, 2048, 0, 8, (1.0, 0.0, 0.02, 1.0, 0.5, 0.0, 0.9, 0.001), 1.0),  # lists of very different lengths
     (4000, 2048, 0, 8, 0.66, 0.6),     # a list cut off before its end
     (4000, 2048, 0, 8, 0.66, 1.5),     # room for more rows than there are
+    (9000, 4096, 4, 8, 0.5, 1.0),      # past 128 MB of packed rows, where they are stored past the caches
+    (5500, 4112, 0, 72, 0.1, 1.0),     # the same in list order
 ])
 def test_pack_rows_by_rank(capi, rows, row_bytes, scale_bytes, r, odds, keep):
     lib = capi.load()
