@@ -1235,21 +1235,22 @@ static const torch::Tensor& tensor_argument(PyObject* v) {
     return THPVariable_Unpack(v);
 }
 static const torch::Tensor* optional_tensor_argument(PyObject* v) { return v == Py_None ? nullptr : &tensor_argument(v); }
-static int64_t int64_argument(PyObject* v) {
-    const int64_t n = PyLong_AsLongLong(v);
-    if (n == -1 and PyErr_Occurred()) throw pybind11::error_already_set();
-    return n;
+// Numbers and truth values by pybind11's own rules, implicit conversions included: what it refuses for a bound
+// function (a float for an int, a str or a list for a bool) is refused here, with the same TypeError.
+template <typename T>
+static T scalar_argument(PyObject* v) {
+    pybind11::detail::make_caster<T> caster;
+    if (!caster.load(v, true)) throw pybind11::type_error("incompatible function arguments");
+    return pybind11::detail::cast_op<T>(caster);
 }
-static int int_argument(PyObject* v) {
-    const int64_t n = int64_argument(v);
-    if (n != int(n)) throw pybind11::value_error("an argument is out of range");
-    return int(n);
+template <typename T>
+static T& object_argument(PyObject* v) {
+    pybind11::detail::make_caster<T> caster;
+    if (!caster.load(v, true) or v == Py_None) throw pybind11::type_error("incompatible function arguments");
+    return pybind11::detail::cast_op<T&>(caster);
 }
-static bool bool_argument(PyObject* v) {
-    const int b = PyObject_IsTrue(v);
-    if (b < 0) throw pybind11::error_already_set();
-    return b != 0;
-}
+static int int_argument(PyObject* v) { return scalar_argument<int>(v); }
+static bool bool_argument(PyObject* v) { return scalar_argument<bool>(v); }
 
 template <typename A>
 struct Argument;
@@ -1269,7 +1270,7 @@ template <>
 struct Argument<std::optional<EventHandle>&> {
     std::optional<EventHandle> value;
     explicit Argument(PyObject* v) {
-        if (v != Py_None) value = pybind11::handle(v).cast<EventHandle>();
+        if (v != Py_None) value = object_argument<EventHandle>(v);
     }
 };
 template <>
@@ -1287,7 +1288,7 @@ struct Argument<int> {
 template <>
 struct Argument<int64_t> {
     int64_t value;
-    explicit Argument(PyObject* v) : value(int64_argument(v)) {}
+    explicit Argument(PyObject* v) : value(scalar_argument<int64_t>(v)) {}
 };
 template <>
 struct Argument<bool> {
@@ -1358,7 +1359,7 @@ template <typename C, typename M, typename R, typename... A>
 struct PlainMemberCall {
     template <M F, size_t... I>
     static pybind11::object with(PyObject* const* a, std::index_sequence<I...>) {
-        C& self = pybind11::handle(a[0]).cast<C&>();
+        C& self = object_argument<std::remove_const_t<C>>(a[0]);
         std::tuple<Argument<A>...> given{Argument<A>(a[1 + I])...};
         if constexpr (std::is_void_v<R>) {
             (self.*F)(std::get<I>(given).value...);
@@ -1400,7 +1401,7 @@ static pybind11::object hook_object(bool wanted) {
 //   -> (recv_x, recv_count, handle, event, hook)
 static PyObject* low_latency_dispatch_call(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return as_python_call(n, 12, [&] {
-        Buffer& buffer = pybind11::handle(a[0]).cast<Buffer&>();
+        Buffer& buffer = object_argument<Buffer>(a[0]);
         const bool use_fp8 = bool_argument(a[7]);
         LowLatencyCache& c = buffer.run_low_latency_dispatch(
             tensor_argument(a[1]), tensor_argument(a[2]), optional_tensor_argument(a[3]), optional_tensor_argument(a[4]),
@@ -1424,7 +1425,7 @@ static PyObject* low_latency_dispatch_call(PyObject*, PyObject* const* a, Py_ssi
 //   -> (combined_x, event, hook)
 static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return as_python_call(n, 11, [&] {
-        Buffer& buffer = pybind11::handle(a[0]).cast<Buffer&>();
+        Buffer& buffer = object_argument<Buffer>(a[0]);
         const auto h = pybind11::reinterpret_steal<pybind11::object>(
             PySequence_Fast(a[4], "the handle of a low_latency_dispatch was expected"));
         if (!h) throw pybind11::error_already_set();

@@ -1,10 +1,13 @@
 """CPU-only checks: the C-ABI library exports what include/deepep_hip.h declares, size
 arithmetic matches the oracle, and the host module's argument checks raise the reference's
 EPException text.  No kernel is launched here."""
+import decimal
 import os
 import re
 
+import numpy as np
 import pytest
+import torch
 
 from oracle import deepep_oracle as O
 
@@ -96,6 +99,38 @@ def test_rows_expected_of_a_batch_follow_the_last_one(tokens, seen_tokens, seen_
     assert got == want
     if tokens <= 4:  # a decode batch stays in the single launch
         assert lib.deepep_ll_dispatch_is_single_launch(tokens, 8, 256, 128, got) == 1
+
+
+@pytest.mark.parametrize("flag,taken", [
+    (True, True), (False, True), (None, True), (1, True), (np.bool_(False), True), (0.0, True),
+    ("False", False), ([], False), ((1,), False), ({}, False)])
+def test_truth_values_are_taken_by_pybind11s_rules(flag, taken):
+    from deepep_efa_amd import deep_ep_cpp
+    x = torch.zeros((1, 128), dtype=torch.bfloat16)  # not on a GPU: what takes the flag refuses the tensor
+    with pytest.raises(RuntimeError if taken else TypeError, match="is_cuda" if taken else "incompatible"):
+        deep_ep_cpp.per_token_cast_to_fp8(x, flag, False)
+
+
+@pytest.mark.parametrize("number,taken", [
+    (3, True), (True, True), (np.int64(3), True), (decimal.Decimal(3), True), (torch.tensor(3), True),
+    (3.0, False), ("3", False), (None, False), (2 ** 31, False), (-2 ** 40, False)])
+def test_numbers_are_taken_by_pybind11s_rules(number, taken):
+    from deepep_efa_amd import deep_ep_cpp
+    member = torch.zeros((1, 8), dtype=torch.bool)
+    with pytest.raises(RuntimeError if taken else TypeError, match="is_cuda" if taken else "incompatible"):
+        deep_ep_cpp.channel_prefix_matrix(member, number)
+
+
+def test_calls_refuse_what_is_not_their_object():
+    from deepep_efa_amd import deep_ep_cpp
+    x, idx = torch.zeros((1, 128), dtype=torch.bfloat16), torch.zeros((1, 2), dtype=torch.int64)
+    for other in (None, 3, deep_ep_cpp.AllToAllCalls(2, 0, 2, 1, 128, 2, 0)):  # what a destroyed Buffer's runtime is
+        with pytest.raises(TypeError, match="incompatible"):
+            deep_ep_cpp.low_latency_dispatch(other, x, idx, None, None, 1, 2, True, False, False, False, False)
+        with pytest.raises(TypeError, match="incompatible"):
+            deep_ep_cpp.get_dispatch_layout(other, idx, 2, None, False, False)
+    with pytest.raises(TypeError, match="incompatible"):
+        deep_ep_cpp.a2a_dispatch_send(None, {}, x, idx)
 
 
 def test_config_follows_reference_rules():
