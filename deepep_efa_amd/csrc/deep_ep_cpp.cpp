@@ -988,6 +988,18 @@ static void capi_check(int rc) {
     throw pybind11::error_already_set();
 }
 
+// f(args...) with the GIL released, as the ctypes view calls the library: a launch that waits for a full queue does
+// not hold up the other Python threads.
+template <typename... P, typename... A>
+static void capi_call(int (*f)(P...), A... args) {
+    int rc;
+    {
+        const pybind11::gil_scoped_release release;
+        rc = f(args...);
+    }
+    capi_check(rc);
+}
+
 struct ExchangeMetadata {
     torch::Tensor send_counts, recv_counts, totals, combine_remote_recv_offset, source_rank, source_offset,
         padded_index, combine_send_offset, num_recv_tokens, tokens_per_expert;
@@ -1010,12 +1022,13 @@ static ExchangeMetadata exchange_metadata_of(const torch::Tensor& all_num_routed
                        b.take(record_at[2], {cap}, i32),   b.take(record_at[3], {cap}, i32),
                        b.take(num_at, {2}, i32),           b.take(per_expert_at, {el}, i32)};
     auto u32 = [](const torch::Tensor& t) { return static_cast<uint32_t*>(t.data_ptr()); };
-    capi_check(deepep_ll_exchange_metadata(
+    capi_call(
+        &deepep_ll_exchange_metadata,
         static_cast<const int32_t*>(all_num_routed.data_ptr()), num_experts, num_ranks, rank, max_tokens, row_capacity,
         static_cast<int32_t*>(m.send_counts.data_ptr()), static_cast<int32_t*>(m.recv_counts.data_ptr()),
         static_cast<int32_t*>(m.totals.data_ptr()), static_cast<int64_t*>(m.combine_remote_recv_offset.data_ptr()),
         u32(m.source_rank), u32(m.source_offset), u32(m.padded_index), u32(m.combine_send_offset),
-        u32(m.num_recv_tokens), u32(m.tokens_per_expert), current_stream()));
+        u32(m.num_recv_tokens), u32(m.tokens_per_expert), current_stream());
     return m;
 }
 
@@ -1077,38 +1090,41 @@ struct AllToAllCalls {
     void dispatch_send(const pybind11::dict& state, const torch::Tensor& x, const torch::Tensor& topk_idx) const {
         using namespace name;
         const Attributes s(state);
-        capi_check(deepep_ll_dispatch_send_by_dest(
+        capi_call(
+            &deepep_ll_dispatch_send_by_dest,
             x.data_ptr(), static_cast<const int64_t*>(topk_idx.data_ptr()), static_cast<int>(x.size(0)), hidden,
             num_topk, num_experts, num_ranks, rank, max_tokens, fmt, s.ptr(send_rows), s.integer(send_capacity),
             s.ptr<int32_t>(send_count), s.ptr<int32_t>(send_expert_prefix), s.ptr<int32_t>(send_counts),
             s.ptr<int64_t>(send_cumsum), s.ptr<int32_t>(pair_slot), s.ptr(workspace), size_t(s.size_bytes(workspace)),
-            current_stream()));
+            current_stream());
     }
 
     void dispatch_recv_ordered(const pybind11::dict& state, const torch::Tensor& all_num_routed,
                                const std::optional<torch::Tensor>& stats) const {
         using namespace name;
         const Attributes s(state);
-        capi_check(deepep_ll_dispatch_recv_by_source_ordered(
+        capi_call(
+            &deepep_ll_dispatch_recv_by_source_ordered,
             s.ptr(recv_by_source), s.integer(slot_rows), static_cast<const int32_t*>(all_num_routed.data_ptr()), hidden,
             num_experts, num_ranks, rank, max_tokens, fmt, s.ptr(packed_recv_x), s.ptr(packed_recv_scales),
             s.ptr<int32_t>(packed_recv_src_info), s.ptr<int64_t>(packed_recv_layout_range),
             s.ptr<int32_t>(packed_recv_count), optional_ptr<int32_t>(stats), s.ptr<uint32_t>(tokens_per_expert),
             s.ptr<int32_t>(record_packed_row), s.integer(row_capacity), s.integer(expected_rows),
-            s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream()));
+            s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream());
     }
 
     void dispatch_recv(const pybind11::dict& state, const pybind11::dict& meta,
                        const std::optional<torch::Tensor>& stats) const {
         using namespace name;
         const Attributes s(state), m(meta);
-        capi_check(deepep_ll_dispatch_recv_by_source(
+        capi_call(
+            &deepep_ll_dispatch_recv_by_source,
             s.ptr(recv_by_source), s.integer(slot_rows), m.ptr<int32_t>(recv_counts), m.ptr<uint32_t>(source_offset),
             m.ptr<uint32_t>(num_recv_tokens), s.integer(row_capacity), hidden, num_experts, num_ranks, max_tokens, fmt,
             s.ptr(packed_recv_x), s.ptr(packed_recv_scales), s.ptr<int32_t>(packed_recv_src_info),
             s.ptr<int64_t>(packed_recv_layout_range), s.ptr<int32_t>(packed_recv_count), optional_ptr<int32_t>(stats),
             s.ptr<uint32_t>(tokens_per_expert), s.ptr<int32_t>(record_packed_row), s.integer(expected_rows),
-            s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream()));
+            s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream());
     }
 
     void combine_send(const pybind11::dict& state, const pybind11::dict& meta, const torch::Tensor& y,
@@ -1116,13 +1132,14 @@ struct AllToAllCalls {
                       const std::optional<torch::Tensor>& peer_recv_rows) const {
         using namespace name;
         const Attributes s(state), m(meta);
-        capi_check(deepep_ll_combine_send_by_dest(
+        capi_call(
+            &deepep_ll_combine_send_by_dest,
             y.data_ptr(), s.ptr<int32_t>(record_packed_row), m.ptr<uint32_t>(source_rank),
             m.ptr<uint32_t>(padded_index), m.ptr<uint32_t>(combine_send_offset), m.ptr<uint32_t>(num_recv_tokens),
             s.integer(row_capacity), hidden, num_experts, num_ranks, max_tokens, s.ptr(send_flat),
             m.ptr<int32_t>(recv_counts), m.ptr<int64_t>(combine_remote_recv_offset),
             optional_ptr<void*>(peer_recv_flat), optional_ptr<int64_t>(peer_recv_rows), s.integer(expected_rows),
-            current_stream()));
+            current_stream());
     }
 
     void combine_recv(const pybind11::dict& state, const torch::Tensor& topk_idx, const torch::Tensor& topk_weights,
@@ -1131,11 +1148,12 @@ struct AllToAllCalls {
         using namespace name;
         const Attributes s(state);
         const torch::Tensor* buf = recv.has_value() ? &recv.value() : s.tensor(recv_flat);
-        capi_check(deepep_ll_combine_recv_flat(
+        capi_call(
+            &deepep_ll_combine_recv_flat,
             buf->data_ptr(), buf->size(0), recv_slot_rows, s.ptr<int32_t>(send_expert_prefix),
             static_cast<const int64_t*>(topk_idx.data_ptr()), static_cast<const float*>(topk_weights.data_ptr()),
             s.ptr<int32_t>(pair_slot), static_cast<int>(topk_idx.size(0)), hidden, num_topk, num_experts, num_ranks,
-            max_tokens, accumulate ? 1 : 0, out.data_ptr(), current_stream()));
+            max_tokens, accumulate ? 1 : 0, out.data_ptr(), current_stream());
     }
 };
 

@@ -1599,3 +1599,41 @@ def test_large_combine_moves_no_rows_of_a_malformed_range(rt, t, k):
     want[le, source] = 0x7FC0
     assert torch.equal(got[1][0], want)
     assert torch.equal(got[0][1], got[1][1])
+
+
+def test_all_to_all_calls_let_other_threads_run(rt):
+    """A launch of the all-to-all surface releases the GIL.  The interpreter is told never to take it away from a
+    running thread, and nothing else in the loop gives it up, so the second thread gets on only through the calls."""
+    import _thread
+    import sys
+    import time
+    r, rank, t, h, k, e = 4, 1, 64, 512, 4, 16
+    a2a = rt.ll.AllToAllState(rt.ll.LLShape(r, rank, e, t, h, k, O.ROW_BF16))
+    world = rt.lb.LoopbackWorld(r, rank, seed=3)
+    world.synthesise(t, h, k, e)
+    x, topk = world.own_inputs()
+    w, out = torch.ones((t, k), device="cuda"), torch.empty((t, h), dtype=torch.bfloat16, device="cuda")
+    routed = torch.zeros((r, e), dtype=torch.int32, device="cuda")
+    calls = [lambda: a2a.dispatch_send(x, topk), lambda: a2a.exchange_metadata(routed),
+             lambda: a2a.dispatch_recv_ordered(routed), lambda: a2a.dispatch_recv(),
+             lambda: a2a.combine_send(a2a.packed_recv_x), lambda: a2a.combine_recv(topk, w, out)]
+    for call in calls:
+        call()
+    torch.cuda.synchronize()
+    interval = sys.getswitchinterval()
+    for i, call in enumerate(calls):
+        ran = []
+        sys.setswitchinterval(1000)
+        try:
+            _thread.start_new_thread(lambda: ran.append(True), ())
+            for _ in range(20000):
+                if ran:
+                    break
+                call()
+            got_on = bool(ran)
+        finally:
+            sys.setswitchinterval(interval)
+        while not ran:
+            time.sleep(0.001)
+        torch.cuda.synchronize()
+        assert got_on, i
