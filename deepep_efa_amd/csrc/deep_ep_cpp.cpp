@@ -20,6 +20,7 @@
 #include <atomic>
 #include <functional>
 #include <memory>
+#include <mutex>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -215,6 +216,35 @@ static int row_format_of(bool use_fp8, bool round_scale, bool use_ue8m0) {
     return round_scale ? DEEPEP_ROW_FP8_POW2 : DEEPEP_ROW_FP8;
 }
 
+// Row-count words (Buffer::observed) of buffers dropped without destroy().  Kernels may still store to them, and the
+// garbage collector may drop a buffer during a capture, where nothing can be waited for: such a word stays what it
+// is and goes to the next buffer of the device, for which a late count is a poor hint and no more.  So there are
+// never more of them than buffers were alive at a time.
+struct RetiredWords {
+    std::mutex mutex;
+    std::vector<std::pair<int, at::DataPtr>> words;
+
+    static RetiredWords& all() {
+        static auto* const the = new RetiredWords;  // never destroyed: the allocator may be gone by then
+        return *the;
+    }
+    static void put(int device, at::DataPtr word) {
+        const std::lock_guard<std::mutex> lock(all().mutex);
+        all().words.emplace_back(device, std::move(word));
+    }
+    static at::DataPtr take(int device) {
+        const std::lock_guard<std::mutex> lock(all().mutex);
+        auto& words = all().words;
+        for (auto it = words.begin(); it != words.end(); ++it) {
+            if (it->first != device) continue;
+            at::DataPtr word = std::move(it->second);
+            words.erase(it);
+            return word;
+        }
+        return {};
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Buffer (reference: csrc/deep_ep.hpp:60-707, csrc/deep_ep.cpp:206-581)
 // One process, one GPU.  `num_ranks`/`rank` describe the expert-parallel world
@@ -270,7 +300,7 @@ struct Buffer {
         if (!explicitly_destroy) {
             destroy();
         } else if (!destroyed) {
-            release_observed();
+            if (observed != nullptr) RetiredWords::put(device_id, std::move(observed_memory));
             printf("WARNING: destroy() was not called before DeepEP buffer destruction, which can leak resources.\n");
             fflush(stdout);
         }
@@ -566,7 +596,8 @@ struct Buffer {
         // no place to allocate pinned memory
         const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
         if (observed == nullptr and not capturing) {
-            observed_memory = at::getHostAllocator(at::kCUDA)->allocate(sizeof(uint64_t));
+            observed_memory = RetiredWords::take(device_id);
+            if (!observed_memory) observed_memory = at::getHostAllocator(at::kCUDA)->allocate(sizeof(uint64_t));
             observed = new (observed_memory.get()) std::atomic<uint64_t>(0);
         }
         // send and receive phase in one call (one kernel launch for decode-sized batches)

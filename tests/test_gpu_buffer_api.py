@@ -614,3 +614,27 @@ def test_a_dropped_buffer_leaves_no_store_behind(deep_ep):
     words = [torch.full((1,), 7, dtype=torch.int64, pin_memory=True) for _ in range(64)]
     torch.cuda.synchronize()
     assert all(int(w) == 7 for w in words)
+
+
+def test_a_buffer_may_be_dropped_during_a_capture(deep_ep):
+    """Without destroy(), as the garbage collector does it: nothing is waited for, and the next buffer works."""
+    buffer, dispatch = _small_dispatch(deep_ep)
+    want = dispatch()[1].clone()
+    v = torch.zeros(64, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        v += 1
+        del buffer, dispatch
+        v += 1
+    for replays in (1, 2, 3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (v == 2 * replays).all()
+    for _ in range(3):  # takes over the word, then with the dropped one's counts replaced by its own
+        buffer, dispatch = _small_dispatch(deep_ep)
+        for _ in range(3):
+            got = dispatch()[1]
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+        del buffer, dispatch
