@@ -935,34 +935,6 @@ static torch::Tensor build_recv_src_meta(const torch::Tensor& recv_counts, const
     return meta;
 }
 
-// reference: csrc/transport/ll_pipeline.cpp:1204-1269,1277-1361 — the bookkeeping between the gather of the
-// route counts and the exchange, on the stream instead of on the host.  Returns (send_counts [R] i32,
-// recv_counts [R] i32, totals [3] i32 = sent / received / corrupt, combine_remote_recv_offset [R] i64,
-// records [4, row_capacity] i32 = source_rank / source_offset / padded_index / combine_send_offset,
-// num_recv_tokens [2] i32, tokens_per_expert [E_l] i32).
-static std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor>
-ll_exchange_metadata(const torch::Tensor& all_num_routed, int rank, int num_max_dispatch_tokens_per_rank,
-                     int64_t row_capacity) {
-    EP_HOST_ASSERT(all_num_routed.dim() == 2 and all_num_routed.is_contiguous() and all_num_routed.is_cuda());
-    EP_HOST_ASSERT(all_num_routed.scalar_type() == torch::kInt32);
-    EP_HOST_ASSERT(row_capacity >= 0);
-    const int num_ranks = static_cast<int>(all_num_routed.size(0)), num_experts = static_cast<int>(all_num_routed.size(1));
-    EP_HOST_ASSERT(num_ranks > 0 and num_experts % num_ranks == 0);
-    const auto i32 = torch::dtype(torch::kInt32).device(all_num_routed.device());
-    auto send_counts = torch::empty({num_ranks}, i32), recv_counts = torch::empty({num_ranks}, i32);
-    auto totals = torch::empty({3}, i32), num_recv_tokens = torch::empty({2}, i32);
-    auto remote = torch::empty({num_ranks}, i32.dtype(torch::kInt64));
-    auto records = torch::empty({4, row_capacity}, i32);
-    auto tokens_per_expert = torch::empty({num_experts / num_ranks}, i32);
-    auto rec = [&](int i) { return reinterpret_cast<uint32_t*>(records.data_ptr<int>()) + int64_t(i) * row_capacity; };
-    abi_check(deepep_ll_exchange_metadata(
-        all_num_routed.data_ptr<int>(), num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank, row_capacity,
-        send_counts.data_ptr<int>(), recv_counts.data_ptr<int>(), totals.data_ptr<int>(), remote.data_ptr<int64_t>(),
-        rec(0), rec(1), rec(2), rec(3), reinterpret_cast<uint32_t*>(num_recv_tokens.data_ptr<int>()),
-        reinterpret_cast<uint32_t*>(tokens_per_expert.data_ptr<int>()), current_stream()));
-    return {send_counts, recv_counts, totals, remote, records, num_recv_tokens, tokens_per_expert};
-}
-
 // ---------------------------------------------------------------------------
 // The calls of ll_runtime.AllToAllState.  A call is given the state's attribute dictionary and takes the tensors
 // out of it by interned name, so whatever the attributes hold at that moment is what the kernels get; through
@@ -1022,45 +994,64 @@ static void capi_check(int rc) {
 // f(args...) with the GIL released, as the ctypes view calls the library: a launch that waits for a full queue does
 // not hold up the other Python threads.
 template <typename... P, typename... A>
+static int without_gil(int (*f)(P...), A... args) {
+    const pybind11::gil_scoped_release release;
+    return f(args...);
+}
+template <typename... P, typename... A>
 static void capi_call(int (*f)(P...), A... args) {
-    int rc;
-    {
-        const pybind11::gil_scoped_release release;
-        rc = f(args...);
-    }
-    capi_check(rc);
+    capi_check(without_gil(f, args...));
 }
 
+// reference: csrc/transport/ll_pipeline.cpp:1204-1269,1277-1361 — the bookkeeping between the gather of the
+// route counts and the exchange, on the stream instead of on the host.
 struct ExchangeMetadata {
-    torch::Tensor send_counts, recv_counts, totals, combine_remote_recv_offset, source_rank, source_offset,
-        padded_index, combine_send_offset, num_recv_tokens, tokens_per_expert;
+    torch::Tensor send_counts, recv_counts, totals, combine_remote_recv_offset, num_recv_tokens, tokens_per_expert;
+    ResultBlock block;
+    int64_t records_at, record_pitch, capacity;  // source_rank / source_offset / padded_index / combine_send_offset
+
+    torch::Tensor record(int i) const { return block.take(records_at + i * record_pitch, {capacity}, torch::kInt32); }
 };
 
-static ExchangeMetadata exchange_metadata_of(const torch::Tensor& all_num_routed, int rank, int max_tokens,
-                                             int64_t row_capacity) {
+// The launch's return code is left to the caller, whose callers know different exceptions for it.
+static int exchange_metadata_of(const torch::Tensor& all_num_routed, int rank, int max_tokens, int64_t row_capacity,
+                                int64_t record_pitch, ExchangeMetadata& m) {
     const int num_ranks = static_cast<int>(all_num_routed.size(0)), num_experts = static_cast<int>(all_num_routed.size(1));
-    const int64_t r = num_ranks, cap = std::max<int64_t>(row_capacity, 0), el = num_experts / std::max(num_ranks, 1);
-    ResultBlock b;
+    const int64_t r = num_ranks, el = num_experts / std::max(num_ranks, 1);
+    m.capacity = std::max<int64_t>(row_capacity, 0), m.record_pitch = record_pitch;
+    ResultBlock& b = m.block;
     const int64_t send_at = b.reserve(4 * r), recv_at = b.reserve(4 * r), totals_at = b.reserve(12);
     const int64_t remote_at = b.reserve(8 * r), num_at = b.reserve(8), per_expert_at = b.reserve(4 * el);
-    int64_t record_at[4];
-    for (auto& at : record_at) at = b.reserve(4 * cap);
+    m.records_at = b.reserve(4 * record_pitch);
     b.allocate(all_num_routed.device());
     const auto i32 = torch::kInt32;
-    ExchangeMetadata m{b.take(send_at, {r}, i32),          b.take(recv_at, {r}, i32),
-                       b.take(totals_at, {3}, i32),        b.take(remote_at, {r}, torch::kInt64),
-                       b.take(record_at[0], {cap}, i32),   b.take(record_at[1], {cap}, i32),
-                       b.take(record_at[2], {cap}, i32),   b.take(record_at[3], {cap}, i32),
-                       b.take(num_at, {2}, i32),           b.take(per_expert_at, {el}, i32)};
-    auto u32 = [](const torch::Tensor& t) { return static_cast<uint32_t*>(t.data_ptr()); };
-    capi_call(
-        &deepep_ll_exchange_metadata,
-        static_cast<const int32_t*>(all_num_routed.data_ptr()), num_experts, num_ranks, rank, max_tokens, row_capacity,
-        static_cast<int32_t*>(m.send_counts.data_ptr()), static_cast<int32_t*>(m.recv_counts.data_ptr()),
-        static_cast<int32_t*>(m.totals.data_ptr()), static_cast<int64_t*>(m.combine_remote_recv_offset.data_ptr()),
-        u32(m.source_rank), u32(m.source_offset), u32(m.padded_index), u32(m.combine_send_offset),
-        u32(m.num_recv_tokens), u32(m.tokens_per_expert), current_stream());
-    return m;
+    m.send_counts = b.take(send_at, {r}, i32), m.recv_counts = b.take(recv_at, {r}, i32);
+    m.totals = b.take(totals_at, {3}, i32), m.combine_remote_recv_offset = b.take(remote_at, {r}, torch::kInt64);
+    m.num_recv_tokens = b.take(num_at, {2}, i32), m.tokens_per_expert = b.take(per_expert_at, {el}, i32);
+    auto at = [&](int64_t offset) { return static_cast<uint8_t*>(b.block.data_ptr()) + offset; };
+    auto record = [&](int i) { return reinterpret_cast<uint32_t*>(at(m.records_at + i * record_pitch)); };
+    return without_gil(&deepep_ll_exchange_metadata, static_cast<const int32_t*>(all_num_routed.data_ptr()), num_experts,
+                       num_ranks, rank, max_tokens, row_capacity, reinterpret_cast<int32_t*>(at(send_at)),
+                       reinterpret_cast<int32_t*>(at(recv_at)), reinterpret_cast<int32_t*>(at(totals_at)),
+                       reinterpret_cast<int64_t*>(at(remote_at)), record(0), record(1), record(2), record(3),
+                       reinterpret_cast<uint32_t*>(at(num_at)), reinterpret_cast<uint32_t*>(at(per_expert_at)),
+                       current_stream());
+}
+
+// Returns (send_counts [R] i32, recv_counts [R] i32, totals [3] i32 = sent / received / corrupt,
+// combine_remote_recv_offset [R] i64, records [4, row_capacity] i32 = source_rank / source_offset / padded_index /
+// combine_send_offset, num_recv_tokens [2] i32, tokens_per_expert [E_l] i32).
+static std::tuple<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor>
+ll_exchange_metadata(const torch::Tensor& all_num_routed, int rank, int num_max_dispatch_tokens_per_rank,
+                     int64_t row_capacity) {
+    EP_HOST_ASSERT(all_num_routed.dim() == 2 and all_num_routed.is_contiguous() and all_num_routed.is_cuda());
+    EP_HOST_ASSERT(all_num_routed.scalar_type() == torch::kInt32);
+    EP_HOST_ASSERT(row_capacity >= 0);
+    EP_HOST_ASSERT(all_num_routed.size(0) > 0 and all_num_routed.size(1) % all_num_routed.size(0) == 0);
+    ExchangeMetadata m;
+    abi_check(exchange_metadata_of(all_num_routed, rank, num_max_dispatch_tokens_per_rank, row_capacity, 4 * row_capacity, m));
+    return {m.send_counts, m.recv_counts, m.totals, m.combine_remote_recv_offset,
+            m.block.take(m.records_at, {4, row_capacity}, torch::kInt32), m.num_recv_tokens, m.tokens_per_expert};
 }
 
 namespace name {
@@ -1096,10 +1087,14 @@ DEEPEP_NAME(recv_flat);
 DEEPEP_NAME(expected_rows);
 }  // namespace name
 
+// The same by name, every record an array of its own.
 static pybind11::dict exchange_metadata_dict(const torch::Tensor& all_num_routed, int rank, int max_tokens,
                                              int64_t capacity) {
     using namespace name;
-    const ExchangeMetadata m = exchange_metadata_of(all_num_routed, rank, max_tokens, capacity);
+    if (all_num_routed.dim() != 2) throw pybind11::value_error("the route counts are [ranks, experts]");
+    ExchangeMetadata m;
+    const int64_t pitch = align_up<int64_t>(4 * std::max<int64_t>(capacity, 0), 256);
+    capi_check(exchange_metadata_of(all_num_routed, rank, max_tokens, capacity, pitch, m));
     pybind11::dict out;
     auto put = [&](PyObject* key, const torch::Tensor& t) {
         PyObject* v = THPVariable_Wrap(t);
@@ -1109,8 +1104,8 @@ static pybind11::dict exchange_metadata_dict(const torch::Tensor& all_num_routed
     };
     put(send_counts, m.send_counts), put(recv_counts, m.recv_counts), put(totals, m.totals);
     put(combine_remote_recv_offset, m.combine_remote_recv_offset);
-    put(source_rank, m.source_rank), put(source_offset, m.source_offset), put(padded_index, m.padded_index);
-    put(combine_send_offset, m.combine_send_offset), put(num_recv_tokens, m.num_recv_tokens);
+    put(source_rank, m.record(0)), put(source_offset, m.record(1)), put(padded_index, m.record(2));
+    put(combine_send_offset, m.record(3)), put(num_recv_tokens, m.num_recv_tokens);
     put(tokens_per_expert, m.tokens_per_expert);
     return out;
 }
@@ -1490,6 +1485,31 @@ static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssiz
     });
 }
 
+// combine_reduce by position or by name; the last three are None unless given.
+static PyObject* combine_reduce_call(PyObject*, PyObject* const* a, Py_ssize_t n, PyObject* names) {
+    static constexpr const char* kNames[] = {"recv_x",           "recv_topk_weights", "sorted_token_ids", "send_cumsum",
+                                             "is_token_in_rank", "bias_0",            "bias_1",           "row_of_pair"};
+    constexpr Py_ssize_t kArguments = 8, kRequired = 5;
+    return as_python_call(std::min(n, kArguments), n, [&] {
+        PyObject* given[kArguments] = {};
+        std::copy(a, a + n, given);
+        for (Py_ssize_t i = 0; names != nullptr and i < PyTuple_GET_SIZE(names); ++i) {
+            PyObject* const name = PyTuple_GET_ITEM(names, i);
+            const auto* at = std::find_if(kNames, kNames + kArguments, [&](const char* s) {
+                return PyUnicode_CompareWithASCIIString(name, s) == 0;
+            });
+            if (at == kNames + kArguments or given[at - kNames] != nullptr)
+                throw pybind11::type_error("an argument is unknown or given twice");
+            given[at - kNames] = a[n + i];
+        }
+        for (Py_ssize_t i = 0; i < kArguments; ++i) {
+            if (given[i] == nullptr and i < kRequired) throw pybind11::type_error("an argument is missing");
+            if (given[i] == nullptr) given[i] = Py_None;
+        }
+        return PlainCall<&combine_reduce>::with(given, std::make_index_sequence<kArguments>());
+    });
+}
+
 static PyMethodDef plain(const char* name, PyObject* (*f)(PyObject*, PyObject* const*, Py_ssize_t), const char* doc) {
     return {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(f)), METH_FASTCALL, doc};
 }
@@ -1508,7 +1528,8 @@ static PyMethodDef plain_calls[] = {
     plain("topk_remap", PlainCall<&topk_remap>::call,
           "Top-k of the send rows in the destination rank's expert numbering"),
     plain("build_recv_src_meta", PlainCall<&build_recv_src_meta>::call, "Source-rank metadata of the received rows"),
-    plain("combine_reduce_call", PlainCall<&combine_reduce>::call, "combine_reduce with every argument given"),
+    {"combine_reduce", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(combine_reduce_call)),
+     METH_FASTCALL | METH_KEYWORDS, "Per-token sum of the rows that came back (normal-mode combine)"},
     plain("ll_exchange_metadata", PlainCall<&ll_exchange_metadata>::call,
           "Send/receive counts, combine offsets and per-row records from the gathered route counts"),
     plain("exchange_metadata_dict", PlainCall<&exchange_metadata_dict>::call, "The same by name"),
@@ -1589,9 +1610,4 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("is_sm90_compiled", deep_ep::is_sm90_compiled);
     m.attr("topk_idx_t") = py::reinterpret_borrow<py::object>(
         (PyObject*)torch::getTHPDtype(c10::CppTypeToScalarType<deep_ep::topk_idx_t>::value));
-
-    m.def("combine_reduce", &deep_ep::combine_reduce, "Per-token sum of the rows that came back (normal-mode combine)",
-          py::arg("recv_x"), py::arg("recv_topk_weights"), py::arg("sorted_token_ids"), py::arg("send_cumsum"),
-          py::arg("is_token_in_rank"), py::arg("bias_0") = py::none(), py::arg("bias_1") = py::none(),
-          py::arg("row_of_pair") = py::none());
 }

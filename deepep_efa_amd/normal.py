@@ -54,5 +54,5 @@ def combine_reduce(recv_x: torch.Tensor, recv_topk_weights: Optional[torch.Tenso
                    bias_1: Optional[torch.Tensor] = None, row_of_pair: Optional[torch.Tensor] = None):
     """combined_x[t] = sum over the ranks holding t of the row that came back (+ biases), float32 accumulate.
     row_of_pair: the table of moe_routing_sort_with_positions (one launch instead of two)."""
-    return deep_ep_cpp.combine_reduce_call(recv_x, recv_topk_weights, sorted_token_ids, send_cumsum, is_token_in_rank,
-                                           bias_0, bias_1, row_of_pair)
+    return deep_ep_cpp.combine_reduce(recv_x, recv_topk_weights, sorted_token_ids, send_cumsum, is_token_in_rank,
+                                      bias_0, bias_1, row_of_pair)

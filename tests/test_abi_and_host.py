@@ -133,6 +133,29 @@ def test_calls_refuse_what_is_not_their_object():
         deep_ep_cpp.a2a_dispatch_send(None, {}, x, idx)
 
 
+def test_combine_reduce_takes_its_arguments_by_position_and_by_name():
+    from deepep_efa_amd import deep_ep_cpp
+    x = torch.zeros((1, 128), dtype=torch.bfloat16)  # refused for not being on a GPU once the arguments are sorted out
+    ids, cumsum, member = torch.zeros(1, dtype=torch.int64), torch.zeros(9, dtype=torch.int64), torch.zeros((1, 8), dtype=torch.bool)
+    by_position = (x, None, ids, cumsum, member)
+    names = ("recv_x", "recv_topk_weights", "sorted_token_ids", "send_cumsum", "is_token_in_rank")
+    for args, kwargs in ((by_position, {}), (by_position, dict(row_of_pair=None)), (by_position + (None,) * 3, {}),
+                         ((), dict(zip(names, by_position))), (by_position[:3], dict(zip(names[3:], by_position[3:])))):
+        with pytest.raises(RuntimeError, match="is_cuda"):
+            deep_ep_cpp.combine_reduce(*args, **kwargs)
+    for args, kwargs in ((by_position[:4], {}), (by_position + (None,) * 4, {}), (by_position, dict(recv_x=x)),
+                         (by_position, dict(bias=None)), (by_position, dict(bias_0=3)), ((3,) + by_position[1:], {})):
+        with pytest.raises(TypeError):
+            deep_ep_cpp.combine_reduce(*args, **kwargs)
+
+
+def test_exchange_metadata_wants_a_matrix():
+    from deepep_efa_amd import ll_runtime
+    for shape in ((8,), (2, 2, 4)):
+        with pytest.raises(ValueError):
+            ll_runtime.exchange_metadata(torch.zeros(shape, dtype=torch.int32), 0, 8, 16)
+
+
 def test_config_follows_reference_rules():
     import deep_ep
     cfg = deep_ep.Config(20, 6, 256, 6, 250)

@@ -534,6 +534,39 @@ def test_dispatch_and_combine_replay_in_a_hip_graph(deep_ep, num_ranks, rank, t,
     buffer.destroy()
 
 
+@pytest.mark.parametrize("use_fp8", (True, False))
+def test_the_bound_methods_give_what_the_wrappers_give(deep_ep, use_fp8):
+    """deep_ep_cpp.Buffer.low_latency_dispatch / low_latency_combine, the reference's own binding surface
+    (csrc/deep_ep.cpp:4440-4476), against the deep_ep.Buffer methods of the same names."""
+    r, rank, t, h, k, e = 8, 3, 48, 1024, 4, 64
+    buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=r, sim_rank=rank, sim_seed=9)
+    x, topk_idx = buffer.loopback_synthesise(t, h, k, e)
+    w = torch.rand((t, k), generator=torch.Generator().manual_seed(1)).cuda()
+    recv, count, handle, event, hook = buffer.low_latency_dispatch(x, topk_idx, t, e, use_fp8=use_fp8)
+    y = torch.randn((e // r, r * t, h), generator=torch.Generator().manual_seed(2)).bfloat16().cuda()
+    combined = buffer.low_latency_combine(y, topk_idx, w, handle)[0]
+    want = [v.clone() for v in (*(recv if use_fp8 else (recv,)), count, handle[0], handle[1], combined)]
+    run = buffer.runtime
+    for asynchronous in (False, True):
+        count.fill_(-1), handle[1].fill_(-1), combined.fill_(-1)
+        recv_x, scales, got_count, src_info, layout_range, event, hook = run.low_latency_dispatch(
+            x, topk_idx, None, None, t, e, use_fp8, False, False, asynchronous, asynchronous)
+        assert (event is not None) == asynchronous and (hook is not None) == asynchronous
+        got_combined, event, hook = run.low_latency_combine(y, topk_idx, w, src_info, layout_range, None, t, e, False,
+                                                            False, asynchronous, asynchronous, None)
+        assert (event is not None) == asynchronous and (hook is not None) == asynchronous
+        if asynchronous:
+            event.current_stream_wait(), hook()
+        torch.cuda.synchronize()
+        assert (scales is not None) == use_fp8
+        got = [*((recv_x, scales) if use_fp8 else (recv_x,)), got_count, src_info, layout_range, got_combined]
+        assert torch.equal(got[-4], want[-4]) and torch.equal(got[-2], want[-2]) and torch.equal(got[-1], want[-1])
+        for le, n in enumerate(want[-4].tolist()):
+            for a, b in zip(got[:-4] + got[-3:-2], want[:-4] + want[-3:-2]):
+                assert torch.equal(a[le, :n].view(torch.uint8), b[le, :n].view(torch.uint8))
+    buffer.destroy()
+
+
 def test_batches_that_change_from_call_to_call(deep_ep):
     """Uneven, skewed and balanced batches in turn through one buffer, each sized by the one before, give what a
     buffer of their own gives; they take the single launch and the index + copy form in both directions."""

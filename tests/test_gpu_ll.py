@@ -833,6 +833,17 @@ def test_exchange_metadata_through_the_host_module(rt):
         assert records[i, :n].cpu().tolist() == want[key][:n].tolist(), key
     with pytest.raises(RuntimeError, match="Assertion"):
         deep_ep_cpp.ll_exchange_metadata(routed, rank, m, cap)
+    for odd in (cap, cap + 3, 0):  # by name: the same launch, its records one by one
+        named = rt.ll.exchange_metadata(routed.cuda(), rank, m, odd)
+        whole = deep_ep_cpp.ll_exchange_metadata(routed.cuda(), rank, m, odd)
+        n = min(want["total_recv"], odd)
+        for got, key in zip(whole[:4] + whole[5:], ("send_counts", "recv_counts", "totals", "combine_remote_recv_offset",
+                                                    "num_recv_tokens", "tokens_per_expert")):
+            assert torch.equal(named[key], got), key
+        for i, key in enumerate(("source_rank", "source_offset", "padded_index", "combine_send_offset")):
+            assert named[key].shape == (odd,) and torch.equal(named[key][:n], whole[4][i, :n]), key
+    with pytest.raises(RuntimeError):
+        rt.ll.exchange_metadata(routed.cuda(), rank, m, -1)
 
 
 @pytest.mark.parametrize("hint", ["batch", "unknown", "huge"])
