@@ -609,7 +609,7 @@ __global__ __launch_bounds__(512) void pack_rows_kernel(PackArgs a) {
         int64_t first = 0;
         int skip = 0, size = 0;
         if (lane < a.num_ranks) {
-            first = a.cumsum[lane];
+            first = lane == 0 ? 0 : a.cumsum[lane];  // the list starts at its first row, whatever cumsum[0] is
             const int64_t n = a.cumsum[lane + 1] - first;
             skip = int((n * g) >> a.group_log2);
             size = int((n * (g + 1)) >> a.group_log2) - skip;

@@ -152,7 +152,8 @@ int deepep_pack_rows(const void* src, const void* scale_src, const int64_t* sort
 
 /* The same for a list that is known to be `num_ranks` ascending lists one after another, list r being rows
  * [send_cumsum[r], send_cumsum[r + 1]) (what deepep_moe_routing_sort writes): large packs then take the copies of
- * a token together, so that its row is read from HBM once.  num_rows_dev as above (send_cumsum + num_ranks). */
+ * a token together, so that its row is read from HBM once.  num_rows_dev as above (send_cumsum + num_ranks);
+ * send_cumsum[0] is taken as 0. */
 int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64_t* sorted_token_ids,
                              const int64_t* num_rows_dev, const int64_t* send_cumsum, int num_ranks,
                              int64_t max_rows, int num_src_rows, int row_bytes, int scale_row_bytes,

@@ -334,6 +334,21 @@ def test_pack_rows_by_rank(capi, rows, row_bytes, scale_bytes, r, odds, keep):
         assert torch.equal(dsc[:n].cpu(), sc[ids[:n]]) and (dsc[n:] == 0xEE).all()
 
 
+@pytest.mark.parametrize("rows", [1000, 4000])
+@pytest.mark.parametrize("first", [0, 1, 5, 8])
+def test_pack_rows_packs_the_whole_list(rows, first):
+    """Both sides of the size where the ranks' lists are merged; the row count is the last entry of send_cumsum, and
+    entries missing in front of it (the prefix of fewer, larger lists) leave no row out."""
+    from deepep_efa_amd import normal
+    g = torch.Generator().manual_seed(rows)
+    is_in = torch.rand((rows, 8), generator=g) < 0.7
+    x = torch.randint(0, 256, (rows, 2048), dtype=torch.uint8, generator=g)
+    ids, _, cumsum, _ = O.moe_routing_sort(is_in)
+    torch.full((ids.numel() * 2048,), 0xEE, dtype=torch.uint8, device="cuda")  # what the result's block held before
+    packed, none = normal.pack_rows(x.cuda(), None, ids.cuda(), cumsum[first:].contiguous().cuda())
+    assert none is None and torch.equal(packed.cpu(), x[ids])
+
+
 def run_cast(capi, x, fmt):
     lib = capi.load()
     m, n = x.shape
