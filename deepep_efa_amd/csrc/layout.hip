@@ -485,8 +485,8 @@ __global__ __launch_bounds__(1024) void channel_prefix_kernel(const uint8_t* __r
 
 // The same for a multiple of 8 ranks: one workgroup per 8 of them, so a wave reads the membership of eight ranks
 // with one 8-byte load per token, up to sixteen of them in flight, and adds the bool bytes up eight at a time.  The
-// bytes of a row that eight workgroups used to fetch for themselves are fetched once (12289 tokens, 8 ranks,
-// 10 channels: 8.7 us, two thirds of it waiting for loads).
+// bytes of a row that eight workgroups used to fetch for themselves are fetched once; the sums of eight ranks are
+// eight times the work of one's.
 template <int kAhead>  // loads in flight per lane: 4 for channels of up to 256 tokens, else 16
 __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64_t* __restrict__ is_token_in_rank,
                                                                     int num_tokens, int num_words, int num_channels,
@@ -786,7 +786,16 @@ int deepep_channel_prefix_matrix(const uint8_t* is_token_in_rank, int num_tokens
     EP_HOST_ASSERT(num_tokens == 0 || is_token_in_rank != nullptr);
     // one wave per channel, up to sixteen at a time
     const int threads = num_channels >= 16 ? 1024 : ((num_channels + 3) / 4) * 256;
-    if ((num_ranks & 7) == 0 && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 && num_channels <= 1024) {
+    // Eight ranks a workgroup pays once there is enough to fetch, and not for so many ranks that their workgroups fill
+    // the chip anyway.  Microseconds behind the launch that writes the matrix, against one rank a workgroup:
+    //   ranks                       8           16          32          64
+    //   131 tokens, 10 channels     2.4 / 2.4   2.7 / 2.4   2.8 / 2.6   3.0 / 2.7
+    //   1024, 24 channels           3.1 / 3.1   3.8 / 3.3   3.7 / 3.3   4.1 / 3.4
+    //   2048, 16 channels           2.7 / 2.7   2.8 / 2.8   3.1 / 3.3   4.1 / 4.0
+    //   4096, 24 channels           3.5 / 4.1   3.8 / 4.3   3.9 / 4.9   5.0 / 5.3
+    //   12289, 10 channels          5.7 / 7.9   6.0 / 8.0   7.7 / 8.9  11.2 / 10.1
+    const bool by_words = num_ranks == 8 || (num_ranks % 8 == 0 && num_ranks <= 32 && num_tokens >= 2048);
+    if (by_words && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 && num_channels <= 1024) {
 #define DEEPEP_LAUNCH_CHANNELS(AHEAD)                                                                              \
     channel_prefix_words_kernel<AHEAD><<<num_ranks / 8, threads, size_t(num_channels) * 32,                        \
                                          reinterpret_cast<hipStream_t>(stream)>>>(                                 \

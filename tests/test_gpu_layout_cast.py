@@ -165,6 +165,22 @@ def test_layout_sort_and_prefix_where_their_launch_forms_meet(t, r):
         assert torch.equal(normal.channel_prefix_matrix(is_in, c).cpu(), O.channel_prefix_matrix(want[3], c))
 
 
+@pytest.mark.parametrize("t", [511, 512, 513, 1023, 1024, 1025, 2047, 2048])
+@pytest.mark.parametrize("r,e", [(4, 64), (8, 64), (32, 128), (40, 280), (64, 256)])
+def test_layout_and_channel_prefix_either_side_of_their_lines(t, r, e):
+    from deepep_efa_amd import deep_ep_cpp, normal
+    topk = _topk(t, 6, e, seed=t + r, drop=3)
+    buffer = deep_ep_cpp.Buffer(r - 1, r, 0, 0, False, False, False, False)
+    buffer.sync([0], [None], None)
+    per_rank, per_node, per_expert, is_in, _ = buffer.get_dispatch_layout(topk.cuda(), e, None, False, False)
+    want = O.get_dispatch_layout(topk, e, r)
+    assert torch.equal(per_rank.cpu(), want[0]) and torch.equal(per_expert.cpu(), want[2])
+    assert torch.equal(is_in.cpu(), want[3])
+    assert per_node is None if r <= 8 else torch.equal(per_node.cpu(), want[1])
+    for c in (1, 10, 24, 33):
+        assert torch.equal(normal.channel_prefix_matrix(is_in, c).cpu(), O.channel_prefix_matrix(want[3], c))
+
+
 # every form of the sort: one workgroup a rank, one per 256 tokens, count + scan + scatter; no tokens at all
 SORT_FORMS = [(0, 8), (0, 9), (0, 72), (1, 9), (300, 24), (131, 16), (5000, 16), (8192, 64), (40000, 8), (9000, 12),
               (70000, 8), (3000, 72), (1, 130)]
