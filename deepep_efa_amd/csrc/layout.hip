@@ -9,9 +9,15 @@ namespace deepep {
 
 constexpr int kLayoutThreads = 256;
 constexpr int kMaxRankWords = 4;  // membership bitmask: up to 256 ranks
-// Up to here one workgroup of 1024 threads counts everything and no second launch adds up partial rows.
-constexpr int kLayoutOneBlockTokens = 2048;
 constexpr int kLayoutOneBlockThreads = 1024;
+// Up to here one workgroup counts everything and no second launch adds up partial rows: a token a thread, and half of
+// that past 32 ranks, whose ballots it takes one after another.  Microseconds of the one launch against the two:
+//   ranks        8            16           32            64
+//   400 tokens   3.2 / 4.6    3.7 / 5.1    4.6 / 5.9     6.9 / 7.7
+//   600          3.7 / 4.6    4.4 / 5.3    5.4 / 6.1     8.0 / 7.7
+//   1024         4.5 / 4.7    5.2 / 5.1    6.8 / 6.1    10.6 / 7.8    (the second launch takes the host 2 more)
+//   2048         6.7 / 4.8    7.6 / 5.4   10.5 / 6.2    17.8 / 8.1
+inline int layout_one_block_tokens(int num_ranks) { return num_ranks <= 32 ? 1024 : 512; }
 
 // Spreads the 8 bits of b into 8 bytes (byte i = bit i, value 0 or 1).
 __device__ __forceinline__ uint64_t bits_to_bool_bytes(uint32_t b) {
@@ -30,9 +36,9 @@ __device__ __forceinline__ uint64_t bits_to_bool_bytes(uint32_t b) {
 // Each workgroup writes a partial row [E | R | R/8]; with one workgroup the
 // partial row is the result, otherwise a second small kernel adds the rows.
 // What bounds it is latency and launches, not the few hundred KB it reads: hence
-// one workgroup while its two tokens a thread cost less than the second launch,
-// and a bitmask of as many words as there are ranks for (an index into a longer
-// one that the compiler cannot resolve goes through selects).
+// one workgroup while that costs less than the second launch, and a bitmask of
+// as many words as there are ranks for (an index into a longer one that the
+// compiler cannot resolve goes through selects).
 // Reference: csrc/kernels/layout.cu:9-121 (which re-reads topk_idx once per
 // 4 experts / 8 ranks).
 // ---------------------------------------------------------------------
@@ -657,7 +663,7 @@ int deepep_get_dispatch_layout(const int64_t* topk_idx, int num_tokens, int num_
     EP_HOST_ASSERT(size_t(width) * 4 <= 64 * 1024);
     const int partials = num_tokens == 0 ? 1 : (num_tokens + kLayoutThreads - 1) / kLayoutThreads;
     EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(partials) * width * 4);
-    const int blocks = num_tokens <= kLayoutOneBlockTokens ? 1 : partials;
+    const int blocks = num_tokens <= layout_one_block_tokens(num_ranks) ? 1 : partials;
     const int threads = blocks == 1 && num_tokens > kLayoutThreads ? kLayoutOneBlockThreads : kLayoutThreads;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     int32_t* partial = reinterpret_cast<int32_t*>(workspace);
