@@ -15,7 +15,8 @@ from . import deep_ep_cpp
 
 
 def moe_routing_sort(is_token_in_rank: torch.Tensor):
-    """[T, R] bool -> (sorted_token_ids [S] int64, send_counts [R] int32, send_cumsum [R+1] int64, S)."""
+    """[T, R] bool -> (sorted_token_ids [S] int64, send_counts [R] int32, send_cumsum [R+1] int64, S).
+    Waits for S, and with it for everything the sort writes: the results may be used from any stream."""
     return deep_ep_cpp.moe_routing_sort(is_token_in_rank)
 
 
