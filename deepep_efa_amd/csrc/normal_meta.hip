@@ -23,8 +23,8 @@ __device__ __forceinline__ int rank_of_row(const int64_t* cumsum, int num_ranks,
 // entries in the expert numbering of the destination rank; entries for
 // other ranks' experts become (-1, 0.0).  One thread per (row, k); the
 // R + 1 prefix lives in LDS.  A short list is a chain of memory round trips and
-// nothing else, so the token's number is asked for before the prefix has come
-// and its weight before its expert has.
+// nothing else, so a token's weight is asked for before its expert has come.  Its
+// number waits for the prefix: the list need not have entries past the total.
 // Reference: csrc/kernels/efa_kernels.cu:339-387.
 // ---------------------------------------------------------------------
 __global__ __launch_bounds__(kMetaThreads) void topk_remap_kernel(
@@ -33,18 +33,15 @@ __global__ __launch_bounds__(kMetaThreads) void topk_remap_kernel(
     int num_topk, int num_ranks, int num_local_experts, int64_t max_send, int64_t* __restrict__ remapped_topk,
     float* __restrict__ remapped_weights) {
     extern __shared__ int64_t cumsum[];  // [R + 1]
-    // rows of a step of the grid; all of max_send's rows have a list entry, valid or not
-    const int64_t step = int64_t(gridDim.x) * kMetaThreads;
-    int64_t idx = int64_t(blockIdx.x) * kMetaThreads + threadIdx.x;
-    auto row_of = [&](int64_t i) { return i < (int64_t(1) << 32) ? int64_t(uint32_t(i) / uint32_t(num_topk)) : i / num_topk; };
-    int64_t row = row_of(idx);
-    int64_t token = row < max_send ? sorted_token_ids[row] : -1;
     for (int r = threadIdx.x; r <= num_ranks; r += kMetaThreads) cumsum[r] = send_cumsum[r];
     lds_barrier();
     int64_t total = cumsum[num_ranks];
     if (total > max_send) total = max_send;
     const int64_t work = total * num_topk;
-    while (idx < work) {
+    for (int64_t idx = int64_t(blockIdx.x) * kMetaThreads + threadIdx.x; idx < work;
+         idx += int64_t(gridDim.x) * kMetaThreads) {
+        const int64_t row = idx < (int64_t(1) << 32) ? int64_t(uint32_t(idx) / uint32_t(num_topk)) : idx / num_topk;
+        const int64_t token = sorted_token_ids[row];
         int64_t out_e = -1;
         float out_w = 0.0f;
         if (token >= 0 && token < num_tokens) {
@@ -56,9 +53,6 @@ __global__ __launch_bounds__(kMetaThreads) void topk_remap_kernel(
         }
         remapped_topk[idx] = out_e;
         remapped_weights[idx] = out_w;
-        idx += step;
-        row = row_of(idx);
-        token = row < max_send ? sorted_token_ids[row] : -1;
     }
 }
 

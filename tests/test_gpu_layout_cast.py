@@ -485,6 +485,24 @@ def test_topk_remap(capi, t, k, e, r):
     assert (out_e[total:] == -99).all() and (out_w[total:] == -99.0).all()
 
 
+@pytest.mark.parametrize("t,room", [(1, 1 << 20), (131, 1), (131, 100000), (4096, 200000)])
+def test_topk_remap_with_room_for_more_rows_than_the_list_has(capi, t, room):
+    """max_send sizes the outputs; the list ends with its last row, and nothing behind it is used."""
+    lib, k, e, r = capi.load(), 8, 256, 8
+    topk, w, _, ids, _, cumsum, total = _normal_world(t, k, e, r, seed=t + room, drop=0)
+    want_e, want_w = O.topk_remap(topk, w, ids, cumsum, e // r)
+    cap = total + room
+    out_e = torch.full((cap, k), -99, dtype=torch.int64, device="cuda")
+    out_w = torch.full((cap, k), -99.0, dtype=torch.float32, device="cuda")
+    held = [v.cuda() for v in (topk, w, ids, cumsum)]
+    assert held[2].numel() == total
+    capi.check(lib.deepep_topk_remap(*[capi.ptr(v) for v in held], t, k, r, e // r, cap, capi.ptr(out_e),
+                                     capi.ptr(out_w), stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(out_e[:total].cpu(), want_e) and torch.equal(out_w[:total].cpu(), want_w)
+    assert (out_e[total:] == -99).all() and (out_w[total:] == -99.0).all()
+
+
 @pytest.mark.parametrize("r,local", [(8, 8), (32, 8), (17, 4), (1, 1)])
 def test_build_recv_src_meta(capi, r, local):
     lib = capi.load()
