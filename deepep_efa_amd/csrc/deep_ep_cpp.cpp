@@ -1272,8 +1272,6 @@ static std::tuple<torch::Tensor, std::optional<torch::Tensor>> pack_rows(const t
 // position, converted one by one.  pybind11's dispatcher takes 0.3 to 0.5 us of host time a call more, of the 4 to 5
 // that a call with its launch takes, and small steps are bound by that.
 // ---------------------------------------------------------------------------
-static PyObject* ep_exception_type = nullptr;  // set when the module is made
-
 static const torch::Tensor& tensor_argument(PyObject* v) {
     if (!THPVariable_Check(v)) throw pybind11::type_error("a torch.Tensor was expected");
     return THPVariable_Unpack(v);
@@ -1365,7 +1363,8 @@ static pybind11::object result_object(const std::tuple<T...>& v) {
         v);
 }
 
-// Runs f and turns what it throws into the Python error that pybind11 would raise.
+// Runs f and turns what it throws into the Python error that pybind11 raises for a bound function: its registered
+// translators, PyTorch's among them (torch.OutOfMemoryError, torch.AcceleratorError), have their say.
 template <typename F>
 static PyObject* as_python_call(Py_ssize_t got, Py_ssize_t wanted, F&& f) {
     try {
@@ -1373,12 +1372,8 @@ static PyObject* as_python_call(Py_ssize_t got, Py_ssize_t wanted, F&& f) {
         return f().release().ptr();
     } catch (pybind11::error_already_set& e) {
         e.restore();
-    } catch (const pybind11::builtin_exception& e) {
-        e.set_error();
-    } catch (const EPException& e) {
-        PyErr_SetString(ep_exception_type, e.what());
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (...) {
+        pybind11::detail::try_translate_exceptions();
     }
     return nullptr;
 }
@@ -1548,8 +1543,7 @@ static bool is_sm90_compiled() { return true; }  // FP8 paths are always built f
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "DeepEP dispatch/combine hot path for MI355X (gfx950): host module over libdeepep_hip.so";
 
-    deep_ep::ep_exception_type =
-        pybind11::register_exception<deep_ep::EPException>(m, "EPException", PyExc_RuntimeError).ptr();
+    pybind11::register_exception<deep_ep::EPException>(m, "EPException", PyExc_RuntimeError);
 
     pybind11::class_<deep_ep::Config>(m, "Config")
         .def(pybind11::init<int, int, int, int, int>(), py::arg("num_sms") = 20,

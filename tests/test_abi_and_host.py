@@ -133,6 +133,21 @@ def test_calls_refuse_what_is_not_their_object():
         deep_ep_cpp.a2a_dispatch_send(None, {}, x, idx)
 
 
+def test_plain_calls_raise_the_modules_exception():
+    from deepep_efa_amd import deep_ep_cpp
+    with pytest.raises(deep_ep_cpp.EPException, match=r"^Failed: Assertion error deep_ep_cpp.cpp:\d+ 'x.dim\(\) == 2"):
+        deep_ep_cpp.per_token_cast_to_fp8(torch.zeros(128, dtype=torch.bfloat16), False, False)
+    with pytest.raises(TypeError, match="wrong number of arguments"):
+        deep_ep_cpp.moe_routing_sort()
+    if not torch.cuda.is_available():  # PyTorch's own kinds come through
+        calls = deep_ep_cpp.AllToAllCalls(2, 0, 2, 1, 128, 2, 0)
+        state = dict.fromkeys(("send_rows", "send_count", "send_expert_prefix", "send_counts", "send_cumsum", "pair_slot",
+                               "workspace"), torch.zeros(1))
+        with pytest.raises(torch.AcceleratorError):
+            deep_ep_cpp.a2a_dispatch_send(calls, dict(state, send_capacity=8), torch.zeros((1, 128), dtype=torch.bfloat16),
+                                          torch.zeros((1, 2), dtype=torch.int64))
+
+
 def test_combine_reduce_takes_its_arguments_by_position_and_by_name():
     from deepep_efa_amd import deep_ep_cpp
     x = torch.zeros((1, 128), dtype=torch.bfloat16)  # refused for not being on a GPU once the arguments are sorted out

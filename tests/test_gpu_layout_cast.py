@@ -365,6 +365,15 @@ def test_pack_rows_packs_the_whole_list(rows, first):
     assert none is None and torch.equal(packed.cpu(), x[ids])
 
 
+def test_an_allocation_that_fails_is_pytorchs_error():
+    """A result that no card holds (1 TB): the exception is the one a program catches to make room and try again."""
+    from deepep_efa_amd import normal
+    x = torch.zeros((1, 1 << 20), dtype=torch.uint8, device="cuda")
+    ids, cumsum = torch.zeros(1 << 20, dtype=torch.int64, device="cuda"), torch.tensor([0, 1 << 20], device="cuda")
+    with pytest.raises(torch.OutOfMemoryError):
+        normal.pack_rows(x, None, ids, cumsum)
+
+
 def run_cast(capi, x, fmt):
     lib = capi.load()
     m, n = x.shape
