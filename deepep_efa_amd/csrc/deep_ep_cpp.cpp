@@ -1174,6 +1174,7 @@ struct AllToAllCalls {
         using namespace name;
         const Attributes s(state);
         const torch::Tensor* buf = recv.has_value() ? &recv.value() : s.tensor(recv_flat);
+        if (buf == nullptr) throw pybind11::type_error("recv is None and so is recv_flat");
         capi_call(
             &deepep_ll_combine_recv_flat,
             buf->data_ptr(), buf->size(0), recv_slot_rows, s.ptr<int32_t>(send_expert_prefix),

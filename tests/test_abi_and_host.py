@@ -148,6 +148,15 @@ def test_plain_calls_raise_the_modules_exception():
                                           torch.zeros((1, 2), dtype=torch.int64))
 
 
+def test_a_reduce_without_a_buffer_to_reduce_from_is_refused():
+    """recv_flat may be given up by a caller who always passes the transport's own buffer."""
+    from deepep_efa_amd import deep_ep_cpp
+    calls, t = deep_ep_cpp.AllToAllCalls(2, 0, 2, 1, 128, 2, 0), torch.zeros((1, 2))
+    state = dict(recv_flat=None, send_expert_prefix=t, pair_slot=t)
+    with pytest.raises(TypeError, match="recv_flat"):
+        deep_ep_cpp.a2a_combine_recv(calls, state, t.long(), t, t.bfloat16(), None, 0, False)
+
+
 def test_combine_reduce_takes_its_arguments_by_position_and_by_name():
     from deepep_efa_amd import deep_ep_cpp
     x = torch.zeros((1, 128), dtype=torch.bfloat16)  # refused for not being on a GPU once the arguments are sorted out
