@@ -936,20 +936,33 @@ static torch::Tensor build_recv_src_meta(const torch::Tensor& recv_counts, const
 }
 
 // ---------------------------------------------------------------------------
-// The calls of ll_runtime.AllToAllState.  A call is given the state's attribute dictionary and takes the tensors
-// out of it by interned name, so whatever the attributes hold at that moment is what the kernels get; through
-// ctypes the argument lists cost the host 5 us a call on top of the launch, and the ten results of the metadata
-// call 14 us more.
+// The calls of ll_runtime.AllToAllState.  A call is given the state and takes the tensors out of its attribute
+// dictionary by interned name, or asks the state where a subclass keeps one elsewhere (a property), so whatever the
+// attributes hold at that moment is what the kernels get; through ctypes the argument lists cost the host 5 us a call
+// on top of the launch, and the ten results of the metadata call 14 us more.
 // ---------------------------------------------------------------------------
 struct Attributes {
-    PyObject* dict;
+    PyObject* object;                            // null: a plain dictionary
+    pybind11::object dict;
+    mutable std::vector<pybind11::object> held;  // what came from elsewhere
 
-    explicit Attributes(const pybind11::dict& d) : dict(d.ptr()) {}
+    explicit Attributes(const pybind11::handle& v) {
+        object = PyDict_Check(v.ptr()) ? nullptr : v.ptr();
+        dict = object == nullptr ? pybind11::reinterpret_borrow<pybind11::object>(v)
+                                 : pybind11::reinterpret_steal<pybind11::object>(PyObject_GenericGetDict(object, nullptr));
+        if (!dict) PyErr_Clear();
+    }
     PyObject* get(PyObject* key) const {
-        PyObject* v = PyDict_GetItemWithError(dict, key);  // borrowed
+        PyObject* v = dict ? PyDict_GetItemWithError(dict.ptr(), key) : nullptr;  // borrowed
         if (v == nullptr) {
-            if (!PyErr_Occurred()) PyErr_SetObject(PyExc_AttributeError, key);
-            throw pybind11::error_already_set();
+            if (PyErr_Occurred()) throw pybind11::error_already_set();
+            if (object == nullptr) {
+                PyErr_SetObject(PyExc_AttributeError, key);
+                throw pybind11::error_already_set();
+            }
+            v = PyObject_GetAttr(object, key);
+            if (v == nullptr) throw pybind11::error_already_set();
+            held.push_back(pybind11::reinterpret_steal<pybind11::object>(v));
         }
         return v;
     }
@@ -1113,7 +1126,7 @@ static pybind11::dict exchange_metadata_dict(const torch::Tensor& all_num_routed
 struct AllToAllCalls {
     int num_ranks, rank, num_experts, max_tokens, hidden, num_topk, fmt;
 
-    void dispatch_send(const pybind11::dict& state, const torch::Tensor& x, const torch::Tensor& topk_idx) const {
+    void dispatch_send(const pybind11::handle& state, const torch::Tensor& x, const torch::Tensor& topk_idx) const {
         using namespace name;
         const Attributes s(state);
         capi_call(
@@ -1125,7 +1138,7 @@ struct AllToAllCalls {
             current_stream());
     }
 
-    void dispatch_recv_ordered(const pybind11::dict& state, const torch::Tensor& all_num_routed,
+    void dispatch_recv_ordered(const pybind11::handle& state, const torch::Tensor& all_num_routed,
                                const std::optional<torch::Tensor>& stats) const {
         using namespace name;
         const Attributes s(state);
@@ -1139,7 +1152,7 @@ struct AllToAllCalls {
             s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream());
     }
 
-    void dispatch_recv(const pybind11::dict& state, const pybind11::dict& meta,
+    void dispatch_recv(const pybind11::handle& state, const pybind11::dict& meta,
                        const std::optional<torch::Tensor>& stats) const {
         using namespace name;
         const Attributes s(state), m(meta);
@@ -1153,7 +1166,7 @@ struct AllToAllCalls {
             s.ptr(by_source_workspace), size_t(s.size_bytes(by_source_workspace)), current_stream());
     }
 
-    void combine_send(const pybind11::dict& state, const pybind11::dict& meta, const torch::Tensor& y,
+    void combine_send(const pybind11::handle& state, const pybind11::dict& meta, const torch::Tensor& y,
                       const std::optional<torch::Tensor>& peer_recv_flat,
                       const std::optional<torch::Tensor>& peer_recv_rows) const {
         using namespace name;
@@ -1168,7 +1181,7 @@ struct AllToAllCalls {
             current_stream());
     }
 
-    void combine_recv(const pybind11::dict& state, const torch::Tensor& topk_idx, const torch::Tensor& topk_weights,
+    void combine_recv(const pybind11::handle& state, const torch::Tensor& topk_idx, const torch::Tensor& topk_weights,
                       const torch::Tensor& out, const std::optional<torch::Tensor>& recv, int64_t recv_slot_rows,
                       bool accumulate) const {
         using namespace name;
@@ -1315,6 +1328,11 @@ struct Argument<std::optional<EventHandle>&> {
     explicit Argument(PyObject* v) {
         if (v != Py_None) value = object_argument<EventHandle>(v);
     }
+};
+template <>
+struct Argument<const pybind11::handle&> {
+    pybind11::handle value;
+    explicit Argument(PyObject* v) : value(v) {}
 };
 template <>
 struct Argument<const pybind11::dict&> {

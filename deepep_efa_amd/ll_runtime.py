@@ -222,7 +222,7 @@ class AllToAllState:
         self.expected_rows = m * k  # what a balanced world delivers; sizes grids, never the result
 
     def dispatch_send(self, x: torch.Tensor, topk_idx: torch.Tensor) -> None:
-        deep_ep_cpp.a2a_dispatch_send(self.calls, self.__dict__, x, topk_idx)
+        deep_ep_cpp.a2a_dispatch_send(self.calls, self, x, topk_idx)
 
     def exchange_metadata(self, all_num_routed: torch.Tensor) -> dict:
         """all_num_routed [R, E] int32: the ranks' send_count, as an all-gather leaves them everywhere."""
@@ -232,17 +232,17 @@ class AllToAllState:
     def dispatch_recv_ordered(self, all_num_routed: torch.Tensor, stats: torch.Tensor = None) -> None:
         """The receive for messages in this build's own order (what dispatch_send emits): places every row by
         arithmetic on the gathered counts, without the record list and without reading the rows' tails."""
-        deep_ep_cpp.a2a_dispatch_recv_ordered(self.calls, self.__dict__, all_num_routed, stats)
+        deep_ep_cpp.a2a_dispatch_recv_ordered(self.calls, self, all_num_routed, stats)
 
     def dispatch_recv(self, stats: torch.Tensor = None) -> None:
-        deep_ep_cpp.a2a_dispatch_recv(self.calls, self.__dict__, self.meta, stats)
+        deep_ep_cpp.a2a_dispatch_recv(self.calls, self, self.meta, stats)
 
     def combine_send(self, y: torch.Tensor, peer_recv_flat: torch.Tensor = None,
                      peer_recv_rows: torch.Tensor = None) -> None:
         """Rows owed to the other ranks into send_flat, or, with a table of the ranks' recv_flat addresses
         (int64 [R]) and their row counts, straight to their place in those buffers."""
-        deep_ep_cpp.a2a_combine_send(self.calls, self.__dict__, self.meta, y, peer_recv_flat, peer_recv_rows)
+        deep_ep_cpp.a2a_combine_send(self.calls, self, self.meta, y, peer_recv_flat, peer_recv_rows)
 
     def combine_recv(self, topk_idx: torch.Tensor, topk_weights: torch.Tensor, out: torch.Tensor,
                      recv: torch.Tensor = None, slot_rows: int = 0, accumulate: bool = False) -> None:
-        deep_ep_cpp.a2a_combine_recv(self.calls, self.__dict__, topk_idx, topk_weights, out, recv, slot_rows, accumulate)
+        deep_ep_cpp.a2a_combine_recv(self.calls, self, topk_idx, topk_weights, out, recv, slot_rows, accumulate)

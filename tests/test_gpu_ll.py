@@ -1648,3 +1648,39 @@ def test_all_to_all_calls_let_other_threads_run(rt):
             time.sleep(0.001)
         torch.cuda.synchronize()
         assert got_on, i
+
+
+def test_all_to_all_state_with_attributes_of_a_subclass(rt):
+    """A subclass may keep an attribute where it likes (a property with a setter): the calls get what it says."""
+    class Counting(rt.ll.AllToAllState):
+        asked = 0
+
+        @property
+        def expected_rows(self):
+            type(self).asked += 1
+            return self._rows
+
+        @expected_rows.setter
+        def expected_rows(self, rows):
+            self._rows = rows
+
+    r, rank, t, h, k, e = 2, 0, 16, 256, 2, 4
+    x_all, topk_all, w = make_world(r, t, h, k, e, seed=5)
+    x, topk, weights = x_all[rank].cuda(), topk_all[rank].cuda(), w[rank].cuda()
+    results = []
+    for kind in (rt.ll.AllToAllState, Counting):
+        me = kind(rt.ll.LLShape(r, rank, e, t, h, k, O.ROW_BF16))
+        me.dispatch_send(x, topk)
+        routed = torch.stack([me.send_count, torch.zeros_like(me.send_count)])
+        lo, hi = (int(v) for v in me.send_cumsum[rank:rank + 2].cpu())
+        me.recv_by_source[:hi - lo] = me.send_rows[lo:hi]
+        me.exchange_metadata(routed)
+        me.dispatch_recv_ordered(routed)
+        me.send_flat.zero_(), me.recv_flat.fill_(1)
+        me.combine_send(me.packed_recv_x)
+        out = torch.empty((t, h), dtype=torch.bfloat16, device="cuda")
+        me.combine_recv(topk, weights, out)
+        torch.cuda.synchronize()
+        results.append((me.packed_recv_count.clone(), me.send_flat.clone(), out))
+    assert Counting.asked == 2
+    assert all(torch.equal(a, b) for a, b in zip(*results)) and int(results[0][0].sum()) > 0
