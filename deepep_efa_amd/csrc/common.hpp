@@ -107,6 +107,29 @@ __device__ __forceinline__ void store_u32x4(uint8_t* p, u32x4 v) {
     if constexpr (kStream) __builtin_nontemporal_store(v, (global_u32x4*)(p));
     else *(global_u32x4*)(p) = v;
 }
+// Scalar values that have been asked for and must all be there from here on: their loads go out together, in front of
+// this, where the compiler would put each behind the branch that first uses it (a trip to memory each).
+__device__ __forceinline__ void await_scalars(uint32_t& a, uint32_t& b, uint32_t& c) {
+    asm volatile("" : "+s"(a), "+s"(b), "+s"(c));
+}
+__device__ __forceinline__ void await_scalars(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+    asm volatile("" : "+s"(a), "+s"(b), "+s"(c), "+s"(d));
+}
+
+// A row as a buffer: its address is the wave's, so a lane brings 32 bits of offset, and lanes past its end read zeros
+// and store nothing without a branch.  The row kernels' waves live for one or two trips to memory, so what stands in
+// front of the first one counts.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t row_buffer(const uint8_t* row, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(row), 0, bytes, 0x00020000);
+}
+template <bool kStream>
+__device__ __forceinline__ u32x4 load_row_u32x4(__amdgpu_buffer_rsrc_t row, int offset) {
+    return __builtin_amdgcn_raw_buffer_load_b128(row, offset, 0, kStream ? 2 : 0);  // 2: the non-temporal hint
+}
+template <bool kStream>
+__device__ __forceinline__ void store_row_u32x4(__amdgpu_buffer_rsrc_t row, int offset, u32x4 v) {
+    __builtin_amdgcn_raw_buffer_store_b128(v, row, offset, 0, kStream ? 2 : 0);
+}
 // Traffic above which a kernel streams (the memory-side cache holds 256 MB).
 inline int64_t stream_bytes() { return int64_t(192) << 20; }
 // The dispatch streams from 64 MB of traffic on (the send side's payload stores; in the single launch

@@ -6,6 +6,7 @@
 //   combine_staging     [E][M][H] bf16 — slot j of expert e holds the output
 //                       for this rank's pair whose dispatch slot was j
 //   combine_send_slots  [E_l][R][M][H] bf16 — rows owed to other ranks
+#include <algorithm>
 #include <cstdlib>
 
 #include "common.hpp"
@@ -324,62 +325,62 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
 // ranks below this one (combine_remote_recv_offset,
 // csrc/transport/ll_pipeline.cpp:1283-1295; the reference's peer stores:
 // coop_combine_send.cuh:205-246).  One workgroup per record, walked like the rows of ll_rows_flat_kernel: HBM
-// bounds it, and neighbouring records are neighbouring rows on both sides.  Against one vector a thread and
-// neighbouring records on eight XCDs: 16376 rows of 14336 bytes 95 -> 77 us (6.1 TB/s), 1024 rows 10.9 -> 7.9 us.
+// bounds it, and neighbouring records are neighbouring rows on both sides.  Up to 512 threads: with twice the trips in
+// front of a row that one has, 896 for a row of 14336 bytes are the slower form (16376 rows 77 us, 1024 rows 6.9).
+// 16376 rows of 14336 bytes 78.7 -> 75.4 us (6.2 TB/s), 1024 rows 7.7 -> 6.4, against two vectors a thread and the
+// record behind the number of records.
 // ---------------------------------------------------------------------
-struct CombineByDestArgs {
-    const uint8_t* x;
-    const int32_t* record_packed_row;
-    const uint32_t* source_rank;
-    const uint32_t* padded_index;
-    const uint32_t* combine_send_offset;
-    const uint32_t* num_recv_tokens;
-    int64_t row_capacity, x_rows;
-    int num_ranks, num_vec;
-    uint8_t* send_flat;
-    // direct delivery
-    uint8_t* const* peer_recv;  // [R] device pointers, or null
-    const int64_t* peer_rows;   // [R] rows each peer buffer holds
+struct CombineByDestPeers {  // direct delivery
+    uint8_t* const* peer_recv;   // [R] device pointers, or null
+    const int64_t* peer_rows;    // [R] rows each peer buffer holds
     const int32_t* recv_counts;
     const int64_t* remote_offset;
+    const uint32_t* source_rank;
+    int num_ranks;
 };
 
-template <bool kStream>
-__global__ __launch_bounds__(512) void ll_combine_send_by_dest_kernel(CombineByDestArgs a) {
-    const int lane = lane_id();
-    const int64_t row_bytes = int64_t(a.num_vec) * 16;
-    for (int64_t block = blockIdx.x;; block += gridDim.x) {
-        const int64_t i = flat_row_of_block(block);
-        // The record is fetched together with the number of records (both sides of the bound are memory the
-        // tables have), and padded_index[i] is i whenever the records come from deepep_ll_exchange_metadata, so
-        // the packed row is fetched for that guess as well and again only if the guess was wrong: one round trip
-        // in front of the row loads instead of three.
-        const int64_t at = i < a.row_capacity ? i : a.row_capacity - 1;
-        const uint32_t num_records = a.num_recv_tokens[1];
-        const uint32_t p = a.padded_index[at];
-        int64_t src_row = a.record_packed_row[at];
-        const int64_t offset = a.combine_send_offset[at];
-        const int64_t records = int64_t(num_records) < a.row_capacity ? int64_t(num_records) : a.row_capacity;
-        if (block >= flat_rounds_end(records)) break;
-        if (i >= records || int64_t(p) >= a.row_capacity) continue;
-        if (int64_t(p) != i) src_row = a.record_packed_row[p];
-        if (src_row < 0 || src_row >= a.x_rows) continue;  // the record has no row
-        uint8_t* dst;
-        if (a.peer_recv == nullptr) {
-            if (offset >= a.row_capacity) continue;
-            dst = a.send_flat + offset * row_bytes;
-        } else {
-            const uint32_t s = a.source_rank[i];
-            if (s >= uint32_t(a.num_ranks)) continue;
-            // the record's place among the rows of its source: offset minus the rows of the lower sources
-            int part = 0;
-            for (int r = lane; r < int(s); r += kWave) part += a.recv_counts[r] < 0 ? 0 : a.recv_counts[r];
-            const int64_t j = offset - __builtin_amdgcn_readlane(wave_inclusive_sum(part), kWave - 1);
-            const int64_t at_peer = a.remote_offset[s] + j;
-            if (j < 0 || j >= a.recv_counts[s] || at_peer < 0 || at_peer >= a.peer_rows[s]) continue;
-            dst = a.peer_recv[s] + at_peer * row_bytes;
+template <bool kStream, bool kPeers>
+__global__ __launch_bounds__(1024) void ll_combine_send_by_dest_kernel(
+    const uint32_t* __restrict__ num_recv_tokens, const uint32_t* __restrict__ padded_index,
+    const int32_t* __restrict__ record_packed_row, const uint32_t* __restrict__ combine_send_offset,
+    uint32_t row_capacity, uint32_t x_rows, const uint8_t* __restrict__ x, uint8_t* __restrict__ send_flat, int num_vec,
+    int threads, uint32_t grid, CombineByDestPeers peers) {
+    const uint64_t row_bytes = uint64_t(num_vec) * 16;
+    uint32_t block = blockIdx.x, i = flat_row_of_block(block);
+    // The record is fetched together with the number of records (both sides of the bound are memory the
+    // tables have), and padded_index[i] is i whenever the records come from deepep_ll_exchange_metadata, so
+    // the packed row is fetched for that guess as well and again only if the guess was wrong: one round trip
+    // in front of the row loads instead of three.
+    const uint32_t at = i < row_capacity ? i : row_capacity - 1;
+    uint32_t records = num_recv_tokens[1], p = padded_index[at], src_row = uint32_t(record_packed_row[at]);
+    uint32_t offset = combine_send_offset[at];
+    await_scalars(records, p, src_row, offset);
+    if (records > row_capacity) records = row_capacity;
+    for (;;) {
+        if (i < records && p < row_capacity) {
+            if (p != i) src_row = uint32_t(record_packed_row[p]);
+            uint8_t* dst = nullptr;
+            if constexpr (!kPeers) {
+                if (offset < row_capacity) dst = send_flat + offset * row_bytes;
+            } else {
+                const uint32_t s = peers.source_rank[i];
+                if (s < uint32_t(peers.num_ranks)) {
+                    // the record's place among the rows of its source: offset minus the rows of the lower sources
+                    const int lane = lane_id();
+                    int part = 0;
+                    for (int r = lane; r < int(s); r += kWave) part += peers.recv_counts[r] < 0 ? 0 : peers.recv_counts[r];
+                    const int64_t j = int64_t(offset) - __builtin_amdgcn_readlane(wave_inclusive_sum(part), kWave - 1);
+                    const int64_t at_peer = peers.remote_offset[s] + j;
+                    if (j >= 0 && j < peers.recv_counts[s] && at_peer >= 0 && at_peer < peers.peer_rows[s])
+                        dst = peers.peer_recv[s] + at_peer * row_bytes;
+                }
+            }
+            if (dst != nullptr && src_row < x_rows)  // < 0: the record has no row
+                block_copy_row<kStream>(x + src_row * row_bytes, dst, num_vec, threadIdx.x, threads);
         }
-        block_copy_row<kStream>(a.x + src_row * row_bytes, dst, a.num_vec, threadIdx.x, blockDim.x);
+        if (uint64_t(block) + grid >= flat_rounds_end(records)) break;
+        block += grid, i = flat_row_of_block(block);
+        if (i < records) p = padded_index[i], src_row = uint32_t(record_packed_row[i]), offset = combine_send_offset[i];
     }
 }
 
@@ -468,11 +469,10 @@ static int launch_combine_rows(const CombineIndexArgs& index, const void* x, int
                                void* combine_send_slots, int64_t expected_rows, hipStream_t hs) {
     const int num_experts = index.num_local_experts * index.num_ranks, num_vec = hidden * 2 / 16;
     const int64_t max_rows = int64_t(num_experts) * index.max_tokens;
-    ll_rows_flat_kernel<<<flat_grid_blocks(expected_rows, max_rows, index.max_tokens), flat_row_threads(num_vec), 0,
-                          hs>>>(index.flat_out, num_experts, index.desc, reinterpret_cast<const uint8_t*>(x),
-                                int64_t(hidden) * 2, num_vec, reinterpret_cast<uint8_t*>(combine_send_slots),
-                                reinterpret_cast<uint8_t*>(combine_staging), int64_t(hidden) * 2, 0, 0, nullptr, 0,
-                                nullptr, 0);
+    const int64_t rows = estimated_rows(expected_rows, num_experts, index.max_tokens);
+    launch_rows_flat(index.flat_out + num_experts, index.desc, max_rows,
+                     index.skip_own ? rows - rows / index.num_ranks : rows, x, int64_t(hidden) * 2, num_vec,
+                     combine_send_slots, combine_staging, int64_t(hidden) * 2, nullptr, hs);
     EP_LAUNCH_CHECK();
     return 0;
 }
@@ -584,25 +584,28 @@ int deepep_ll_combine_send_by_dest(const void* x, const int32_t* record_packed_r
                                combine_remote_recv_offset != nullptr && peer_recv_rows != nullptr));
     EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(x) & 15) == 0);
     EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(send_flat) & 15) == 0);
-    CombineByDestArgs a;
-    a.x = reinterpret_cast<const uint8_t*>(x);
-    a.record_packed_row = record_packed_row, a.source_rank = source_rank, a.padded_index = padded_index;
-    a.combine_send_offset = combine_send_offset, a.num_recv_tokens = num_recv_tokens;
-    a.row_capacity = row_capacity;
-    a.x_rows = int64_t(num_experts) * num_max_dispatch_tokens_per_rank;  // E_l * R * M rows of expert outputs
-    a.num_ranks = num_ranks, a.num_vec = hidden * 2 / 16;
-    a.send_flat = reinterpret_cast<uint8_t*>(send_flat);
-    a.peer_recv = reinterpret_cast<uint8_t* const*>(peer_recv_flat), a.peer_rows = peer_recv_rows;
-    a.recv_counts = recv_counts, a.remote_offset = combine_remote_recv_offset;
-    const int threads = flat_row_threads(a.num_vec);
+    CombineByDestPeers peers;
+    peers.peer_recv = reinterpret_cast<uint8_t* const*>(peer_recv_flat), peers.peer_rows = peer_recv_rows;
+    peers.recv_counts = recv_counts, peers.remote_offset = combine_remote_recv_offset;
+    peers.source_rank = source_rank, peers.num_ranks = num_ranks;
+    const int num_vec = hidden * 2 / 16, threads = flat_row_threads(num_vec, 512);
     // grid from the rows expected, not from the capacity (an idle workgroup is not free)
     const int64_t rows = expected_rows > 0 && expected_rows < row_capacity ? expected_rows : row_capacity;
-    const unsigned blocks = flat_grid_blocks(rows, row_capacity, num_max_dispatch_tokens_per_rank);
-    hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
-    if (2 * rows * hidden * 2 > stream_bytes())
-        ll_combine_send_by_dest_kernel<true><<<blocks, threads, 0, hs>>>(a);
-    else
-        ll_combine_send_by_dest_kernel<false><<<blocks, threads, 0, hs>>>(a);
+    const unsigned grid = flat_grid_blocks(rows, row_capacity);
+    const int64_t x_rows = std::min(int64_t(num_experts) * num_max_dispatch_tokens_per_rank, int64_t(1) << 31);
+#define DEEPEP_LAUNCH_BY_DEST(STREAM, PEERS)                                                                            \
+    ll_combine_send_by_dest_kernel<STREAM, PEERS><<<grid, threads, 0, reinterpret_cast<hipStream_t>(stream)>>>(         \
+        num_recv_tokens, padded_index, record_packed_row, combine_send_offset, uint32_t(row_capacity),                  \
+        uint32_t(x_rows), reinterpret_cast<const uint8_t*>(x),                                                          \
+        reinterpret_cast<uint8_t*>(send_flat), num_vec, threads, grid, peers)
+    if (2 * rows * hidden * 2 > stream_bytes()) {
+        if (peer_recv_flat != nullptr) DEEPEP_LAUNCH_BY_DEST(true, true);
+        else DEEPEP_LAUNCH_BY_DEST(true, false);
+    } else {
+        if (peer_recv_flat != nullptr) DEEPEP_LAUNCH_BY_DEST(false, true);
+        else DEEPEP_LAUNCH_BY_DEST(false, false);
+    }
+#undef DEEPEP_LAUNCH_BY_DEST
     EP_LAUNCH_CHECK();
     return 0;
 }

@@ -1252,15 +1252,15 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
         const int64_t data_bytes = row_data_bytes(hidden, row_format);
         const int64_t scale_bytes = row_scale_bytes(hidden, row_format);
         const int num_vec = int(data_bytes / 16);
-        const int threads = flat_row_threads(num_vec), extra = 64;  // one more wave for scales + source index
-        ll_rows_flat_kernel<<<flat_grid_blocks(expected_rows, max_rows, num_max_dispatch_tokens_per_rank),
-                              threads + extra, 0,
-                              hs>>>(flat, num_experts, desc, reinterpret_cast<const uint8_t*>(recv_staging),
-                                    row_stride_bytes(hidden, row_format), num_vec,
-                                    reinterpret_cast<uint8_t*>(packed_recv_x), nullptr, data_bytes,
-                                    int(scale_bytes / 4), align16(data_bytes),
-                                    scale_bytes > 0 ? reinterpret_cast<uint8_t*>(packed_recv_scales) : nullptr,
-                                    align16(data_bytes) + align16(scale_bytes), packed_recv_src_info, extra);
+        FlatTails tails;
+        tails.scale_dst = reinterpret_cast<uint8_t*>(packed_recv_scales), tails.src_info = packed_recv_src_info;
+        tails.scale_dwords = packed_recv_scales != nullptr ? uint32_t(scale_bytes / 4) : 0u;
+        tails.scale_off = uint32_t(align16(data_bytes));
+        tails.info_off = uint32_t(align16(data_bytes) + align16(scale_bytes));
+        // rows that are in place already are not described: of a balanced batch, one in num_ranks
+        const int64_t rows = estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank);
+        launch_rows_flat(flat + num_experts, desc, max_rows, own_rank >= 0 ? rows - rows / num_ranks : rows, recv_staging,
+                         row_stride_bytes(hidden, row_format), num_vec, packed_recv_x, nullptr, data_bytes, &tails, hs);
         EP_LAUNCH_CHECK();
         return 0;
     }

@@ -620,16 +620,13 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
     }
     if (row_capacity == 0) return 0;
     const int num_vec = int(data_bytes / 16);
-    const int threads = flat_row_threads(num_vec), extra = 64;  // one more wave for scales + source index
-    // the copy's grid follows the rows expected, not the capacity: a workgroup that finds no row still costs
-    // a fraction of a nanosecond, and a capacity of R slots is many times what a balanced world fills
-    const unsigned blocks = flat_grid_blocks(expected_rows > 0 ? expected_rows : row_capacity, row_capacity,
-                                             num_max_dispatch_tokens_per_rank);
-    ll_rows_flat_kernel<<<blocks, threads + extra, 0, hs>>>(
-        flat_total, 0, desc, rows_in, stride, num_vec,
-        reinterpret_cast<uint8_t*>(packed_recv_x), nullptr, data_bytes, int(scale_bytes / 4), align16(data_bytes),
-        scale_bytes > 0 ? reinterpret_cast<uint8_t*>(packed_recv_scales) : nullptr, tail_off, packed_recv_src_info,
-        extra);
+    FlatTails tails;
+    tails.scale_dst = reinterpret_cast<uint8_t*>(packed_recv_scales), tails.src_info = packed_recv_src_info;
+    tails.scale_dwords = packed_recv_scales != nullptr ? uint32_t(scale_bytes / 4) : 0u;
+    tails.scale_off = uint32_t(align16(data_bytes));
+    tails.info_off = uint32_t(tail_off);
+    launch_rows_flat(flat_total, desc, row_capacity, expected_rows > 0 ? expected_rows : row_capacity, rows_in,
+                     stride, num_vec, packed_recv_x, nullptr, data_bytes, &tails, hs);
     EP_LAUNCH_CHECK();
     return 0;
 }
@@ -702,14 +699,13 @@ int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_
     const int64_t data_bytes = row_data_bytes(hidden, row_format);
     const int64_t scale_bytes = row_scale_bytes(hidden, row_format);
     const int num_vec = int(data_bytes / 16);
-    const int threads = flat_row_threads(num_vec), extra = 64;  // one more wave for scales + source index
-    const unsigned blocks = flat_grid_blocks(expected_rows > 0 ? expected_rows : most_rows, most_rows,
-                                             num_max_dispatch_tokens_per_rank);
-    ll_rows_flat_kernel<<<blocks, threads + extra, 0, hs>>>(
-        flat_total, 0, desc, reinterpret_cast<const uint8_t*>(recv_by_source), row_stride_bytes(hidden, row_format),
-        num_vec, reinterpret_cast<uint8_t*>(packed_recv_x), nullptr, data_bytes, int(scale_bytes / 4),
-        align16(data_bytes), scale_bytes > 0 ? reinterpret_cast<uint8_t*>(packed_recv_scales) : nullptr,
-        align16(data_bytes) + align16(scale_bytes), packed_recv_src_info, extra);
+    FlatTails tails;
+    tails.scale_dst = reinterpret_cast<uint8_t*>(packed_recv_scales), tails.src_info = packed_recv_src_info;
+    tails.scale_dwords = packed_recv_scales != nullptr ? uint32_t(scale_bytes / 4) : 0u;
+    tails.scale_off = uint32_t(align16(data_bytes));
+    tails.info_off = uint32_t(align16(data_bytes) + align16(scale_bytes));
+    launch_rows_flat(flat_total, desc, most_rows, expected_rows > 0 ? expected_rows : most_rows, recv_by_source,
+                     row_stride_bytes(hidden, row_format), num_vec, packed_recv_x, nullptr, data_bytes, &tails, hs);
     EP_LAUNCH_CHECK();
     return 0;
 }

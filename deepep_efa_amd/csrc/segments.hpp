@@ -389,79 +389,90 @@ __device__ __forceinline__ void combine_index_block(const CombineIndexArgs& a, i
     }
 }
 
-// One workgroup per described row (looping only if there are more rows than workgroups).  Only batches too large
-// for the caches come here, so the payload streams, two 16-byte vectors a thread in flight.  HBM bounds it, and
-// beyond a few hundred MB address translation as well, which likes the rows in flight to be close together:
+// One workgroup per described row (looping only if there are more rows than workgroups).  Only batches too large for
+// the caches come here, so the payload streams, one 16-byte vector a thread: two workgroups of a 14336-byte row are
+// what a compute unit holds, and with as few rows as that in flight HBM serves them best, provided that a row's
+// address is there early.  Hence two trips to memory in front of the row and no more (the arguments; then descriptor and
+// number of rows together: left to the compiler it is four), buffer addressing, and no row that waits for another one.
+// Beyond a few hundred MB address translation bounds it as well, which likes the rows in flight to be close together:
 // workgroup i runs on XCD i % 8, and each XCD is given kFlatWindow rows in a row instead of every eighth one.
-// Measured with one vector a thread and neighbouring rows on eight XCDs against this: 28672 x 14336 bytes 134 ->
-// 131 us (6.3 TB/s), 160000 x 14336 785 -> 753 us, 160000 x 7168 384 -> 370 us.
+// Microseconds against two vectors a thread, four trips and a grid of one workgroup for two rows:
+//   28672 rows of 14336 bytes 131.3 -> 125.5 (6.55 TB/s), 7168 bytes and scales 67.8 -> 65.7;
+//   160000 of 14336 bytes 792 -> 712 (6.5 TB/s), 14300 of 7168 41.5 -> 39.8.
+// A bare copy of whole rows, nothing in front of it, reaches 6.7.  Workgroups that loop are slower however early they
+// fetch what comes next: 32768 x 14336 bytes 142.5 us with a row each, 145 with two, 153 with four, 164 with eight,
+// 165 to 175 with 512 workgroups that stay.
 constexpr int kFlatWindow = 32;
 constexpr int kFlatRound = 8 * kFlatWindow;
 
-__device__ __forceinline__ int64_t flat_row_of_block(int64_t block) {
-    const int in_round = int(block % kFlatRound);
-    return block - in_round + (in_round & 7) * kFlatWindow + (in_round >> 3);
+__device__ __forceinline__ uint32_t flat_row_of_block(uint32_t block) {
+    const uint32_t in_round = block % kFlatRound;
+    return block - in_round + in_round % 8 * kFlatWindow + in_round / 8;
 }
-__device__ __forceinline__ int64_t flat_rounds_end(int64_t rows) {
+__device__ __forceinline__ uint32_t flat_rounds_end(uint32_t rows) {
     return (rows + kFlatRound - 1) / kFlatRound * kFlatRound;
 }
 
-// Thread `tid` of `threads` moves its vectors of a row, two in flight.
+// Threads [0, threads) of a workgroup move a row, a vector each; wider rows go round.
 template <bool kStream>
 __device__ __forceinline__ void block_copy_row(const uint8_t* src, uint8_t* dst, int num_vec, int tid, int threads) {
-    for (int v = tid; v < num_vec; v += 2 * threads) {
-        const bool second = v + threads < num_vec;
-        const u32x4 r0 = load_u32x4<kStream>(src + int64_t(v) * 16);
-        u32x4 r1 = r0;
-        if (second) r1 = load_u32x4<kStream>(src + int64_t(v + threads) * 16);
-        store_u32x4<kStream>(dst + int64_t(v) * 16, r0);
-        if (second) store_u32x4<kStream>(dst + int64_t(v + threads) * 16, r1);
-    }
+    const auto from = row_buffer(src, num_vec * 16), to = row_buffer(dst, num_vec * 16);
+    store_row_u32x4<kStream>(to, tid * 16, load_row_u32x4<kStream>(from, tid * 16));
+    for (int v = threads; v < num_vec; v += threads)
+        store_row_u32x4<kStream>(to, (v + tid) * 16, load_row_u32x4<kStream>(from, (v + tid) * 16));
 }
 
+// What a row carries besides its payload (the dispatch's rows; all null for the combine's).
+struct FlatTails {
+    uint8_t* scale_dst;
+    int32_t* src_info;
+    uint32_t scale_dwords, scale_off, info_off;
+};
+
+template <bool kTails>
 static __global__ __launch_bounds__(1024) void ll_rows_flat_kernel(
-    const int32_t* __restrict__ flat, int num_segments, const RowDesc* __restrict__ desc,
-    const uint8_t* __restrict__ src, int64_t src_stride, int num_vec, uint8_t* __restrict__ dst_primary,
-    uint8_t* __restrict__ dst_secondary, int64_t dst_stride, int scale_dwords, int64_t src_scale_off,
-    uint8_t* __restrict__ scale_dst, int64_t tail_off, int32_t* __restrict__ src_info, int extra_threads) {
-    const int total = flat[num_segments];
-    const int64_t rounds_end = flat_rounds_end(total);
-    for (int64_t i = blockIdx.x; i < rounds_end; i += gridDim.x) {
-        const int64_t row = flat_row_of_block(i);
-        if (row >= total) continue;
-        const RowDesc d = desc[row];
-        if (d.src_row < 0) continue;  // a record that names no row
-        const uint8_t* s = src + int64_t(d.src_row) * src_stride;
-        uint8_t* o;
-        if (d.dst_row >= 0) {
-            if (dst_primary == nullptr) continue;
-            o = dst_primary + int64_t(d.dst_row) * dst_stride;
-        } else {
-            o = dst_secondary + int64_t(-(d.dst_row + 1)) * dst_stride;
-        }
-        // threads [0, data_threads) move the payload; when the launch carries extra threads beyond
-        // them, those move scales and the source index in the same pass instead of a second one
-        const int data_threads = int(blockDim.x) - extra_threads;
-        const int tid = threadIdx.x;
-        if (tid < data_threads) block_copy_row<true>(s, o, num_vec, tid, data_threads);
-        if (extra_threads == 0 || tid >= data_threads) {
-            const int t2 = extra_threads > 0 ? tid - data_threads : tid;
-            const int step = extra_threads > 0 ? extra_threads : int(blockDim.x);
-            if (scale_dst != nullptr) {
-                const uint32_t* s32 = reinterpret_cast<const uint32_t*>(s + src_scale_off);
-                uint32_t* d32 = reinterpret_cast<uint32_t*>(scale_dst + int64_t(d.dst_row) * scale_dwords * 4);
-                for (int v = t2; v < scale_dwords; v += step) d32[v] = s32[v];
+    const int32_t* __restrict__ total, const RowDesc* __restrict__ desc, uint32_t capacity, uint32_t grid,
+    const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, uint32_t src_stride, uint32_t dst_stride, int num_vec,
+    int data_threads, uint8_t* __restrict__ dst_own, FlatTails tails) {
+    const int tid = threadIdx.x;
+    uint32_t i = blockIdx.x, row = flat_row_of_block(i);
+    // the descriptor is fetched with the number of rows, not behind it: the table has `capacity` of them
+    const RowDesc* at = desc + (row < capacity ? row : capacity - 1);
+    uint32_t rows = uint32_t(*total), src_row = uint32_t(at->src_row), dst_row = uint32_t(at->dst_row);
+    await_scalars(rows, src_row, dst_row);
+    for (;;) {
+        if (row < rows && int32_t(src_row) >= 0) {  // < 0: a record that names no row
+            const uint8_t* s = src + uint64_t(src_row) * src_stride;
+            if constexpr (kTails) {
+                if (wave_in_block() * kWave < data_threads) {
+                    block_copy_row<true>(s, dst + uint64_t(dst_row) * dst_stride, num_vec, tid, data_threads);
+                } else {  // the last wave: scales and source index
+                    const int lane = lane_id();
+                    int32_t info = 0;
+                    if (lane == 0) info = *reinterpret_cast<const int32_t*>(s + tails.info_off);
+                    const uint32_t* from = reinterpret_cast<const uint32_t*>(s + tails.scale_off);
+                    uint32_t* to = reinterpret_cast<uint32_t*>(tails.scale_dst) +
+                                   uint64_t(dst_row) * tails.scale_dwords;
+                    for (uint32_t v = lane; v < tails.scale_dwords; v += kWave) to[v] = from[v];
+                    if (lane == 0) tails.src_info[dst_row] = info;
+                }
+            } else {
+                const bool own = int32_t(dst_row) < 0;
+                uint8_t* base = own ? dst_own : dst;
+                const uint32_t to = own ? ~dst_row : dst_row;
+                if (base != nullptr) block_copy_row<true>(s, base + uint64_t(to) * dst_stride, num_vec, tid, data_threads);
             }
-            if (src_info != nullptr && t2 == step - 1)
-                src_info[d.dst_row] = *reinterpret_cast<const int32_t*>(s + tail_off);
         }
+        if (uint64_t(i) + grid >= flat_rounds_end(rows)) break;
+        i += grid, row = flat_row_of_block(i);
+        if (row < rows) src_row = uint32_t(desc[row].src_row), dst_row = uint32_t(desc[row].dst_row);
     }
 }
 
-// Threads of the kernel above that move a row's payload: two vectors each.
-inline int flat_row_threads(int num_vec) {
-    const int threads = (num_vec / 2 + 63) / 64 * 64;
-    return threads < 64 ? 64 : (threads > 512 ? 512 : threads);
+// Threads that move a row's payload, a vector each, at most `most`: wider rows take whole trips of about equal size.
+inline int flat_row_threads(int num_vec, int most) {
+    const int trips = (num_vec + most - 1) / most;
+    return ((num_vec + trips - 1) / trips + 63) / 64 * 64;
 }
 
 __host__ __device__ inline int64_t segment_workspace_bytes(int num_experts, int max_tokens) {
@@ -479,15 +490,33 @@ inline int64_t estimated_rows(int64_t expected_rows, int64_t num_experts, int64_
     return expected_rows > 0 ? expected_rows : num_experts * max_tokens / 32;
 }
 
-inline unsigned flat_grid_blocks(int64_t expected_rows, int64_t max_rows, int max_tokens) {
-    int64_t want = expected_rows > 0 ? expected_rows : int64_t(max_tokens) * 8;
-    want += want / 8 + 64;
+// Workgroups for `rows` expected rows of at most max_rows.  One that finds no row costs what it takes to launch its
+// waves (a nanosecond for fourteen: 4 us for an eighth too many of 32768), one that finds a second row about 2 us at
+// the very end: a thirty-second more than expected.
+inline unsigned flat_grid_blocks(int64_t rows, int64_t max_rows) {
+    int64_t want = rows + rows / 32 + 64;
     if (want > max_rows) want = max_rows;
     if (want > (int64_t(1) << 22)) want = int64_t(1) << 22;
     if (want < 1) want = 1;
-    // beyond 64 workgroups per CU two rows per workgroup measured ~5 % faster than one; eight slower
-    if (want > 16384) want = want / 2 > 16384 ? want / 2 : 16384;
     return unsigned((want + kFlatRound - 1) / kFlatRound * kFlatRound);  // whole rounds over the XCDs
+}
+
+// The flat copy of the rows `desc` describes (*total of them, memory for max_rows); expected_rows sizes the grid.
+inline void launch_rows_flat(const int32_t* total, const RowDesc* desc, int64_t max_rows, int64_t expected_rows,
+                             const void* src, int64_t src_stride, int num_vec, void* dst, void* dst_own,
+                             int64_t dst_stride, const FlatTails* tails, hipStream_t stream) {
+    // many short rows: two a workgroup are 1 % faster (160000 x 7168 bytes 383 -> 378 us; 28672: 65.7 -> 66.3)
+    const bool pairs = expected_rows > 65536 && num_vec <= 512;
+    const unsigned grid = flat_grid_blocks(pairs ? expected_rows / 2 : expected_rows, max_rows);
+    const int others = tails != nullptr ? kWave : 0, threads = flat_row_threads(num_vec, 1024 - others);
+#define DEEPEP_LAUNCH_ROWS(TAILS)                                                                                     \
+    ll_rows_flat_kernel<TAILS><<<grid, threads + others, 0, stream>>>(                                                \
+        total, desc, uint32_t(max_rows), grid, reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst), \
+        uint32_t(src_stride), uint32_t(dst_stride), num_vec, threads, reinterpret_cast<uint8_t*>(dst_own),            \
+        tails != nullptr ? *tails : FlatTails{})
+    if (tails != nullptr) DEEPEP_LAUNCH_ROWS(true);
+    else DEEPEP_LAUNCH_ROWS(false);
+#undef DEEPEP_LAUNCH_ROWS
 }
 
 }  // namespace deepep

@@ -1579,6 +1579,40 @@ def test_return_by_destination_over_record_counts(rt, records, hidden):
     assert torch.equal(out.cpu(), want)
 
 
+@pytest.mark.parametrize("t,h,fmt,hint", [
+    (33, 128, O.ROW_FP8, 8193), (33, 15488, O.ROW_FP8, 8193),  # the grid is far larger than the rows; two trips a row
+    (40, 8320, O.ROW_BF16, 9000), (1300, 512, O.ROW_FP8_UE8M0, 8193),  # more rows than workgroups
+    (4700, 128, O.ROW_FP8, 65537),  # two rows a workgroup, and more than that
+])
+def test_row_copies_over_widths_and_hints(rt, t, h, fmt, hint):
+    """The flat row copy of both directions, every row and every byte around it."""
+    r, rank, k, e = 2, 1, 8, 16
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + h, drop=20)
+    st = rt.ll.LowLatencyState(rt.ll.LLShape(num_ranks=r, rank=rank, num_experts=e, max_tokens=t, hidden=h, num_topk=k,
+                                             fmt=fmt))
+    st.expected_rows = hint
+    st.segment_workspace = torch.empty(rt.capi.load().deepep_ll_segment_workspace_bytes(e, t), dtype=torch.uint8,
+                                       device="cuda")
+    world = rt.lb.LoopbackWorld(r, rank, seed=0)
+    world.set_inputs(x_all.cuda(), topk_all.cuda())
+    run_dispatch(st, world, *world.own_inputs())
+    want = O.ll_dispatch(list(x_all), list(topk_all), rank, e, t, fmt)
+    check_dispatch(st, want, fmt)
+    px = st.packed_recv_x.view(torch.uint8).view(e // r, r * t, -1)
+    for le, n in enumerate(st.packed_recv_count.tolist()):
+        assert bool((px[le, n:] == 0xEE).all())  # nothing behind the last row
+    y = torch.randn((e // r, r * t, h), device="cuda").bfloat16()
+    st.combine_send_slots.fill_(3.0)
+    st.combine_staging.fill_(3.0)
+    slots, staging = st.combine_send_slots.clone(), st.combine_staging.clone()
+    st.combine_send(y)
+    for le in range(e // r):
+        for s in range(r):
+            begin, n = int(want["packed_recv_layout_range"][le, s]) >> 32, int(want["packed_recv_layout_range"][le, s]) & 0xFFFFFFFF
+            (staging[rank * (e // r) + le] if s == rank else slots[le, s])[:n] = y[le, begin:begin + n]
+    assert torch.equal(st.combine_send_slots, slots) and torch.equal(st.combine_staging, staging)
+
+
 @pytest.mark.parametrize("t,k", [(1025, 8), (1100, 8)])
 def test_large_combine_moves_no_rows_of_a_malformed_range(rt, t, k):
     """Past 8192 rows the reduce's launch builds the row return's index; a segment whose range leaves its expert gets
