@@ -108,24 +108,37 @@ __global__ __launch_bounds__(kMetaThreads) void combine_positions_kernel(
 // lane r fetches rank r's membership byte and row index (one round of loads
 // for all ranks, neither waiting for the other), the rows and their weights are
 // then loaded eight at a time.
+// HBM bounds a large one.  A rank's rows of neighbouring tokens are neighbours, so a large one gives an XCD
+// kReduceWindow workgroups in a row, and a token's pieces to as few workgroups of about equal size as eight waves
+// allow: 12289 tokens of 14336 bytes at 8 ranks (1.1 GB) 184 -> 171 us (6.5 TB/s), 4096 61.0 -> 59.3, 9000 of 4096
+// bytes at 32 ranks 52.7 -> 50.6, against four waves in launch order; four waves in windows 175, whole tokens 174.  A
+// small one is latency and takes four waves wherever they run (131 tokens 4.6 us; seven waves in windows 5.6).
 // Reference: the zero_() + index_add_ of deep_ep/buffer.py:1542-1557, which
 // accumulates in bf16 through atomics in arrival order.
 // ---------------------------------------------------------------------
+constexpr int kReduceWindow = 32;
+constexpr int kReduceRound = 8 * kReduceWindow;
+
 template <bool kStream>  // the returned rows exceed what the caches hold: read them with the non-temporal hint
-__global__ __launch_bounds__(kMetaThreads) void combine_reduce_kernel(
+__global__ __launch_bounds__(512) void combine_reduce_kernel(
     const uint8_t* __restrict__ recv_x, const float* __restrict__ recv_w,
     const uint8_t* __restrict__ is_token_in_rank, const int32_t* __restrict__ row_of_pair,
-    const uint8_t* __restrict__ bias_0, const uint8_t* __restrict__ bias_1, int num_tokens, int hidden,
-    int num_topk, int num_ranks, int64_t max_rows, int pieces_per_row, uint8_t* __restrict__ out_x,
+    const uint8_t* __restrict__ bias_0, const uint8_t* __restrict__ bias_1, int num_tokens, int row_bytes,
+    int num_topk, int num_ranks, int max_rows, uint32_t pieces_per_row, uint32_t waves, uint8_t* __restrict__ out_x,
     float* __restrict__ out_w) {
     const int lane = lane_id();
-    const int64_t item = int64_t(blockIdx.x) * (kMetaThreads / kWave) + wave_in_block();
-    if (item >= int64_t(num_tokens) * pieces_per_row) return;
-    const int t = int(item / pieces_per_row);
-    const int piece = int(item - int64_t(t) * pieces_per_row);
-    const int64_t row_bytes = int64_t(hidden) * 2;
-    const int64_t off = int64_t(piece) * 1024 + lane * 16;
-    const bool lane_live = off < row_bytes;
+    uint32_t t, piece;
+    if constexpr (kStream) {  // workgroups of a token are neighbours on an XCD
+        const uint32_t in_round = blockIdx.x % kReduceRound, per_token = (pieces_per_row + waves - 1) / waves;
+        const uint32_t block = blockIdx.x - in_round + in_round % 8 * kReduceWindow + in_round / 8;
+        t = block / per_token, piece = (block - t * per_token) * waves + wave_in_block();
+        if (piece >= pieces_per_row) return;
+    } else {
+        const uint32_t item = blockIdx.x * waves + wave_in_block();
+        t = item / pieces_per_row, piece = item - t * pieces_per_row;
+    }
+    if (t >= uint32_t(num_tokens)) return;
+    const int off = int(piece) * 1024 + lane * 16;
 
     float acc[8];
 #pragma unroll
@@ -135,7 +148,7 @@ __global__ __launch_bounds__(kMetaThreads) void combine_reduce_kernel(
 
     for (int r0 = 0; r0 < num_ranks; r0 += kWave) {
         const int r = r0 + lane;
-        int64_t my_row = -1;
+        int my_row = -1;
         if (r < num_ranks) {
             const uint8_t member = is_token_in_rank[int64_t(t) * num_ranks + r];
             my_row = row_of_pair[int64_t(t) * num_ranks + r];  // means nothing for a rank the token is not sent to
@@ -145,50 +158,45 @@ __global__ __launch_bounds__(kMetaThreads) void combine_reduce_kernel(
         while (present != 0) {
             u32x4 v[8];
             float wv[8];
-            int rows[8];
             int n = 0;
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                rows[u] = -1;
                 if (present != 0) {
                     const int src_lane = __builtin_ctzll(present);
                     present &= present - 1;
-                    rows[u] = __builtin_amdgcn_readlane(int(my_row), src_lane);
-                    if (lane_live) v[u] = load_u32x4<kStream>(recv_x + int64_t(rows[u]) * row_bytes + off);
-                    if (weights_here && lane < num_topk) wv[u] = recv_w[int64_t(rows[u]) * num_topk + lane];
+                    const int row = __builtin_amdgcn_readlane(my_row, src_lane);
+                    const uint8_t* from = recv_x + uint64_t(uint32_t(row)) * uint32_t(row_bytes);
+                    v[u] = load_row_u32x4<kStream>(row_buffer(from, row_bytes), off);
+                    if (weights_here && lane < num_topk) wv[u] = recv_w[int64_t(row) * num_topk + lane];
                     n = u + 1;
                 }
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 if (u >= n) continue;
-                if (lane_live) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        acc[2 * i] += bf16_lo(v[u][i]);
-                        acc[2 * i + 1] += bf16_hi(v[u][i]);
-                    }
+                for (int i = 0; i < 4; ++i) {
+                    acc[2 * i] += bf16_lo(v[u][i]);
+                    acc[2 * i + 1] += bf16_hi(v[u][i]);
                 }
                 if (weights_here && lane < num_topk) w_acc += wv[u];
             }
         }
     }
-    if (lane_live) {
-        if (bias_0 != nullptr) {
-            const u32x4 b = load_global_u32x4(bias_0 + int64_t(t) * row_bytes + off);
+    if (bias_0 != nullptr) {
+        const u32x4 b = load_row_u32x4<false>(row_buffer(bias_0 + uint64_t(t) * uint32_t(row_bytes), row_bytes), off);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) acc[2 * i] += bf16_lo(b[i]), acc[2 * i + 1] += bf16_hi(b[i]);
-        }
-        if (bias_1 != nullptr) {
-            const u32x4 b = load_global_u32x4(bias_1 + int64_t(t) * row_bytes + off);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[2 * i] += bf16_lo(b[i]), acc[2 * i + 1] += bf16_hi(b[i]);
-        }
-        u32x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
-        store_u32x4<kStream>(out_x + int64_t(t) * row_bytes + off, o);
+        for (int i = 0; i < 4; ++i) acc[2 * i] += bf16_lo(b[i]), acc[2 * i + 1] += bf16_hi(b[i]);
     }
+    if (bias_1 != nullptr) {
+        const u32x4 b = load_row_u32x4<false>(row_buffer(bias_1 + uint64_t(t) * uint32_t(row_bytes), row_bytes), off);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[2 * i] += bf16_lo(b[i]), acc[2 * i + 1] += bf16_hi(b[i]);
+    }
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
+    store_row_u32x4<kStream>(row_buffer(out_x + uint64_t(t) * uint32_t(row_bytes), row_bytes), off, o);
     if (weights_here && lane < num_topk) out_w[int64_t(t) * num_topk + lane] = w_acc;
 }
 
@@ -275,14 +283,18 @@ int deepep_combine_reduce(const void* recv_x, const float* recv_topk_weights, co
         EP_LAUNCH_CHECK();
     }
     const int pieces = (hidden * 2 + 1023) / 1024;
-    const int64_t blocks = (int64_t(num_tokens) * pieces + (kMetaThreads / kWave) - 1) / (kMetaThreads / kWave);
-    EP_HOST_ASSERT(blocks < (int64_t(1) << 31));
-#define DEEPEP_LAUNCH_REDUCE(STREAM)                                                                          \
-    combine_reduce_kernel<STREAM><<<dim3(unsigned(blocks)), kMetaThreads, 0, hs>>>(                             \
+    const bool stream_rows = max_rows * hidden * 2 > stream_bytes();
+    const int per_token = (pieces + 7) / 8, waves = stream_rows ? (pieces + per_token - 1) / per_token : 4;
+    int64_t blocks = stream_rows ? int64_t(num_tokens) * per_token : (int64_t(num_tokens) * pieces + waves - 1) / waves;
+    if (stream_rows) blocks = (blocks + kReduceRound - 1) / kReduceRound * kReduceRound;
+    EP_HOST_ASSERT(blocks < (int64_t(1) << 31) && int64_t(num_tokens) * pieces < (int64_t(1) << 32));
+#define DEEPEP_LAUNCH_REDUCE(STREAM)                                                                             \
+    combine_reduce_kernel<STREAM><<<dim3(unsigned(blocks)), waves * kWave, 0, hs>>>(                              \
         reinterpret_cast<const uint8_t*>(recv_x), recv_topk_weights, is_token_in_rank, row_of_pair,               \
-        reinterpret_cast<const uint8_t*>(bias_0), reinterpret_cast<const uint8_t*>(bias_1), num_tokens, hidden,  \
-        num_topk, num_ranks, max_rows, pieces, reinterpret_cast<uint8_t*>(combined_x), combined_topk_weights)
-    if (max_rows * hidden * 2 > stream_bytes()) DEEPEP_LAUNCH_REDUCE(true);
+        reinterpret_cast<const uint8_t*>(bias_0), reinterpret_cast<const uint8_t*>(bias_1), num_tokens,          \
+        hidden * 2, num_topk, num_ranks, int(max_rows), uint32_t(pieces), uint32_t(waves),                       \
+        reinterpret_cast<uint8_t*>(combined_x), combined_topk_weights)
+    if (stream_rows) DEEPEP_LAUNCH_REDUCE(true);
     else DEEPEP_LAUNCH_REDUCE(false);
 #undef DEEPEP_LAUNCH_REDUCE
     EP_LAUNCH_CHECK();

@@ -568,6 +568,31 @@ def test_combine_reduce(capi, t, k, e, r, h, with_bias):
     assert torch.allclose(out_w.cpu().double(), ref_w, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("h", [8, 512, 4616, 7168, 9224])  # 1, 1, 10, 14 and 19 pieces: 1, 1, 2, 2 and 3 workgroups a token
+@pytest.mark.parametrize("t", [1, 37, 300])
+def test_combine_reduce_of_a_buffer_past_the_caches(capi, t, h):
+    """The streaming form, chosen by the size of the returned buffer: every token once, bit for bit."""
+    lib = capi.load()
+    k, r = 4, 8
+    topk, w, is_in, ids, counts, cumsum, total = _normal_world(t, k, 32, r, seed=t + h)
+    g = torch.Generator().manual_seed(6)
+    rows, rw = torch.randn((total, h), generator=g).to(torch.bfloat16), torch.rand((total, k), generator=g)
+    b0 = torch.randn((t, h), generator=g).to(torch.bfloat16)
+    max_rows = (192 << 20) // (2 * h) + 1
+    recv = torch.empty((max_rows, h), dtype=torch.bfloat16, device="cuda")
+    recv[:total] = rows.cuda()
+    out_x = torch.full((t + 1, h), 7.0, dtype=torch.bfloat16, device="cuda")
+    out_w = torch.full((t, k), float("nan"), dtype=torch.float32, device="cuda")
+    dev = [None if v is None else v.cuda() for v in (rw, ids, cumsum, is_in, b0)]
+    table = _want_row_of_pair(is_in, ids, cumsum).cuda()
+    capi.check(lib.deepep_combine_reduce(capi.ptr(recv), *[capi.ptr(v) for v in dev], None, t, h, k, r, max_rows,
+                                         capi.ptr(table), capi.ptr(out_x), capi.ptr(out_w), None, 0, stream()))
+    torch.cuda.synchronize()
+    chain_x, chain_w = O.combine_reduce_f32_chain(rows, rw, ids, cumsum, t, b0, None)
+    assert torch.equal(out_x[:t].cpu().view(torch.int16), chain_x.view(torch.int16)) and bool((out_x[t] == 7.0).all())
+    assert torch.equal(out_w.cpu(), chain_w)
+
+
 @pytest.mark.parametrize("seed", range(int(os.environ.get("DEEPEP_TEST_RANDOM_SHAPES", "16"))))
 def test_pack_remap_reduce_seeded_random_shapes(capi, seed):
     """Pack, top-k remap and the combine reduce on shapes nobody picked by hand: odd rank counts, ragged
