@@ -135,11 +135,11 @@ struct CombineSelection {
 // Issues the loads of selection `lane`'s (slot, expert, weight): one round of loads for the whole token.
 // Nothing here waits for them, so a caller can put other latency (the own-range lookup of the
 // single-launch combine) behind the same round trip.
-__device__ __forceinline__ CombineSelection combine_load_selection(const CombineRecvArgs& a, int64_t item) {
+__device__ __forceinline__ CombineSelection combine_load_selection(const CombineRecvArgs& a, uint32_t t) {
     CombineSelection s = {-1, -1, 0.0f};
     const int lane = lane_id();
-    if (item < int64_t(a.num_tokens) * a.pieces_per_row && lane < a.num_topk) {
-        const int64_t idx = (item / a.pieces_per_row) * a.num_topk + lane;
+    if (t < uint32_t(a.num_tokens) && lane < a.num_topk) {
+        const int64_t idx = int64_t(t) * a.num_topk + lane;
         s.slot = a.pair_slot[idx];
         s.expert = a.topk_idx[idx];
         s.weight = a.topk_weights[idx];
@@ -148,18 +148,16 @@ __device__ __forceinline__ CombineSelection combine_load_selection(const Combine
 }
 
 template <bool kStream>
-__device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, int64_t item, const CombineSelection& sel,
-                                                   const uint8_t* own_x, const int32_t* own_begin,
-                                                   int own_first_expert, int num_local_experts,
-                                                   int64_t slots_per_expert) {
+__device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, uint32_t t, uint32_t piece,
+                                                   const CombineSelection& sel, const uint8_t* own_x,
+                                                   const int32_t* own_begin, int own_first_expert,
+                                                   int num_local_experts, int64_t slots_per_expert) {
     const int lane = lane_id();
-    if (item >= int64_t(a.num_tokens) * a.pieces_per_row) return;
-    const int t = int(item / a.pieces_per_row);
-    const int piece = int(item - int64_t(t) * a.pieces_per_row);
+    if (t >= uint32_t(a.num_tokens)) return;
     const int64_t row_bytes = int64_t(a.hidden) * 2;
-    const int64_t off = int64_t(piece) * 1024 + lane * 16;
-    const bool lane_live = off < row_bytes;
+    const int off = int(piece) * 1024 + lane * 16;  // lanes past the row's end read zeros and store nothing
     const int num_topk = a.num_topk;
+    const auto out = row_buffer(a.out + int64_t(t) * row_bytes, int(row_bytes));
 
     DEEPEP_PHASE(0);
     // Lane k works out where selection k's row is; the loop below reads the results back lane by
@@ -202,8 +200,8 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, int
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-    if (a.accumulate != 0 && lane_live) {  // reference: csrc/kernels/coop_combine_recv.cuh:174-179
-        const u32x4 prev = load_global_u32x4(a.out + int64_t(t) * row_bytes + off);
+    if (a.accumulate != 0) {  // reference: csrc/kernels/coop_combine_recv.cuh:174-179
+        const u32x4 prev = load_row_u32x4<false>(out, off);
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[2 * i] = bf16_lo(prev[i]), acc[2 * i + 1] = bf16_hi(prev[i]);
     }
@@ -222,13 +220,13 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, int
                 const uint32_t hi32 = __builtin_amdgcn_readlane(uint32_t(my_row >> 32), k);
                 wgt[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_weight), k));
                 const uint8_t* row = reinterpret_cast<const uint8_t*>((uint64_t(hi32) << 32) | lo32);
-                if (lane_live) v[u] = load_u32x4<kStream>(row + off);
+                v[u] = load_row_u32x4<kStream>(row_buffer(row, int(row_bytes)), off);
             }
         }
         DEEPEP_PHASE(1);
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            if (!live[u] || !lane_live) continue;
+            if (!live[u]) continue;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 acc[2 * i] = __builtin_fmaf(bf16_lo(v[u][i]), wgt[u], acc[2 * i]);
@@ -237,12 +235,10 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, int
         }
     }
     DEEPEP_PHASE(2);
-    if (lane_live) {
-        u32x4 o;
+    u32x4 o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
-        store_u32x4<kStream>(a.out + int64_t(t) * row_bytes + off, o);
-    }
+    for (int i = 0; i < 4; ++i) o[i] = pack_bf16x2(acc[2 * i], acc[2 * i + 1]);
+    store_row_u32x4<kStream>(out, off, o);
     DEEPEP_PHASE(3);
 }
 
@@ -251,10 +247,12 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, int
 // the expert-output tensor directly (layout_range says where each own segment begins).
 // index_blocks > 0: that many workgroups in front of the reduce's build the index of the row return that follows
 // (a launch of its own took 3 to 5 us of a large combine).
+// Streaming, a workgroup is one wave: nothing holds a wave's slot once it is done (4096 tokens, eight rows of 14336
+// bytes each, 90.5 -> 88.7 us, 6.0 TB/s; two to fourteen waves 91 to 95, neighbouring tokens on one XCD no gain).
 template <bool kStream>
 __global__ __launch_bounds__(256) void ll_combine_recv_kernel(CombineRecvArgs a, const uint8_t* own_x,
                                                               const int64_t* layout_range, int rank,
-                                                              int num_local_experts, int num_ranks,
+                                                              int num_local_experts, int num_ranks, uint32_t waves,
                                                               CombineIndexArgs index, int index_blocks) {
     extern __shared__ int32_t own_begin[];  // [E_l], with own_x only; index workgroups: [segments + 1]
     __shared__ int32_t index_wave_totals[kMaxBlockWaves];
@@ -262,16 +260,17 @@ __global__ __launch_bounds__(256) void ll_combine_recv_kernel(CombineRecvArgs a,
         combine_index_block(index, blockIdx.x, own_begin, index_wave_totals);
         return;
     }
-    const int64_t item = (int64_t(blockIdx.x) - index_blocks) * (blockDim.x >> 6) + wave_in_block();
-    const CombineSelection sel = combine_load_selection(a, item);  // in flight while the own ranges are fetched
+    const uint32_t item = (blockIdx.x - index_blocks) * waves + wave_in_block(), pieces = a.pieces_per_row;
+    const uint32_t t = item / pieces, piece = item - t * pieces;
+    const CombineSelection sel = combine_load_selection(a, t);  // in flight while the own ranges are fetched
     if (own_x != nullptr) {
-        for (int le = threadIdx.x; le < num_local_experts; le += blockDim.x) {
+        for (int le = threadIdx.x; le < num_local_experts; le += int(waves) * kWave) {
             const int64_t lr = layout_range[le * num_ranks + rank];
             own_begin[le] = (lr & 0xffffffffll) > 0 ? int(lr >> 32) : 0;
         }
         lds_barrier();
     }
-    combine_recv_piece<kStream>(a, item, sel, own_x, own_x != nullptr ? own_begin : nullptr, rank * num_local_experts,
+    combine_recv_piece<kStream>(a, t, piece, sel, own_x, own_x != nullptr ? own_begin : nullptr, rank * num_local_experts,
                                 num_local_experts, int64_t(a.max_tokens) * num_ranks);
 }
 
@@ -298,14 +297,15 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
     if (block < num_recv_blocks) {
         // the token's index loads and the own-range loads go out together: one memory round trip
         // before the row loads instead of two
-        const int64_t item = int64_t(block) * 4 + wave_in_block();
-        const CombineSelection sel = combine_load_selection(ra, item);
-        for (int le = threadIdx.x; le < sa.num_local_experts; le += blockDim.x) {
+        const uint32_t item = uint32_t(block) * 4 + wave_in_block(), pieces = ra.pieces_per_row;
+        const uint32_t t = item / pieces, piece = item - t * pieces;
+        const CombineSelection sel = combine_load_selection(ra, t);
+        for (int le = threadIdx.x; le < sa.num_local_experts; le += 256) {
             const int64_t lr = sa.layout_range[le * sa.num_ranks + sa.rank];
             dyn_lds[le] = (lr & 0xffffffffll) > 0 ? int(lr >> 32) : 0;
         }
         lds_barrier();
-        combine_recv_piece<kStream>(ra, item, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
+        combine_recv_piece<kStream>(ra, t, piece, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
                                     sa.num_local_experts, int64_t(sa.max_tokens) * sa.num_ranks);
     } else {
         combine_send_rows<kStream>(sa, block - num_recv_blocks, int(gridDim.x) - num_recv_blocks, true);
@@ -440,7 +440,7 @@ static int check_combine_recv_args(const void* combine_staging, const int64_t* t
                    pair_slot != nullptr && out != nullptr);
     EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(combine_staging) & 15) == 0);
     EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(out) & 15) == 0);
-    EP_HOST_ASSERT((int64_t(num_tokens) * ((hidden * 2 + 1023) / 1024) + 3) / 4 < (int64_t(1) << 31));
+    EP_HOST_ASSERT(int64_t(num_tokens) * ((hidden * 2 + 1023) / 1024) < (int64_t(1) << 31));
     return 0;
 }
 
@@ -520,17 +520,18 @@ int deepep_ll_combine_send(const void* x, const int64_t* layout_range, int hidde
 
 static void launch_reduce(const CombineRecvArgs& ra, const uint8_t* own, const int64_t* layout_range, int rank,
                           int num_local_experts, int num_ranks, const CombineIndexArgs* index, hipStream_t hs) {
-    const int waves = 4;  // block shape makes no measurable difference (1..16 waves: within 5 %)
+    const bool stream_rows = int64_t(ra.num_tokens) * ra.num_topk * ra.hidden * 2 > stream_bytes();
+    const int waves = stream_rows ? 1 : 4;
     const int index_blocks = index != nullptr ? index->num_local_experts * index->num_ranks : 0;
     const CombineIndexArgs ia = index != nullptr ? *index : CombineIndexArgs{};
     const int64_t blocks = index_blocks + (int64_t(ra.num_tokens) * ra.pieces_per_row + waves - 1) / waves;
     const size_t lds = size_t(index_blocks > 0 ? index_blocks + 1 : num_local_experts) * sizeof(int32_t);
-    if (int64_t(ra.num_tokens) * ra.num_topk * ra.hidden * 2 > stream_bytes())
+    if (stream_rows)
         ll_combine_recv_kernel<true><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(
-            ra, own, layout_range, rank, num_local_experts, num_ranks, ia, index_blocks);
+            ra, own, layout_range, rank, num_local_experts, num_ranks, uint32_t(waves), ia, index_blocks);
     else
         ll_combine_recv_kernel<false><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(
-            ra, own, layout_range, rank, num_local_experts, num_ranks, ia, index_blocks);
+            ra, own, layout_range, rank, num_local_experts, num_ranks, uint32_t(waves), ia, index_blocks);
 }
 
 // own_x != null: the answers of this rank's own experts are read from own_x at the positions
