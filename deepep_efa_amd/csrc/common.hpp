@@ -130,6 +130,27 @@ template <bool kStream>
 __device__ __forceinline__ void store_row_u32x4(__amdgpu_buffer_rsrc_t row, int offset, u32x4 v) {
     __builtin_amdgcn_raw_buffer_store_b128(v, row, offset, 0, kStream ? 2 : 0);
 }
+// Threads [0, threads) of a workgroup move a row, kVecs vectors of each in flight; wider rows go round.
+template <int kVecs, bool kStreamLoad, bool kStreamStore>
+__device__ __forceinline__ void block_copy_row(const uint8_t* src, uint8_t* dst, int num_vec, int tid, int threads) {
+    const auto from = row_buffer(src, num_vec * 16), to = row_buffer(dst, num_vec * 16);
+    int v = 0;
+    for (;;) {
+        u32x4 r[kVecs];
+#pragma unroll
+        for (int u = 0; u < kVecs; ++u) r[u] = load_row_u32x4<kStreamLoad>(from, (v + u * threads + tid) * 16);
+#pragma unroll
+        for (int u = 0; u < kVecs; ++u) store_row_u32x4<kStreamStore>(to, (v + u * threads + tid) * 16, r[u]);
+        v += kVecs * threads;
+        if (v >= num_vec) break;
+    }
+}
+// Threads that move a row's payload, a vector each, at most `most`: wider rows take whole trips of about equal size.
+inline int flat_row_threads(int num_vec, int most) {
+    const int trips = (num_vec + most - 1) / most;
+    return ((num_vec + trips - 1) / trips + 63) / 64 * 64;
+}
+
 // Traffic above which a kernel streams (the memory-side cache holds 256 MB).
 inline int64_t stream_bytes() { return int64_t(192) << 20; }
 // The dispatch streams from 64 MB of traffic on (the send side's payload stores; in the single launch

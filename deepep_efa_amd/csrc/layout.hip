@@ -561,75 +561,77 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 //    39 MB  10.0 / 8.9    25.6 / 29.5     129 MB  40.4 / 23.2   83.8 / 85.6
 //    78 MB  24.0 / 15.3   48.8 / 54.2     140 MB  42.0 / 25.3   93.9 / 91.4
 //    97 MB  29.3 / 18.4   59.8 / 65.7     155 MB  48.5 / 27.4  107.2 / 102.5    311 MB  88.7 / 54.6  209 / 197
-// Grouping and hint against list order and ordinary stores: 12289 x 14336 bytes (934 MB) 305 -> 211 us (5.2 TB/s on
-// the bytes that have to move), 4096 x 7168 (155 MB) 48.1 -> 27.3 us (6.7).
-// Half the threads with two vectors each against all with one: 260 -> 211 us.
+// Grouping and hint against list order and ordinary stores: 12289 x 14336 bytes (934 MB) 305 -> 211 us, 4096 x 7168
+// (155 MB) 48.1 -> 27.3.  Rows as buffers and the scales in a wave of their own (a wave that stores its payload first
+// waits for that before its scales are there): 202 -> 188 us (5.9 TB/s on the bytes that have to move), 9000 x 10240 to
+// 32 ranks 151 -> 136, 4096 x 7168 27.4 -> 27.2.  Four trips to memory stand in front of a row here, which takes more
+// rows in flight to hide than the copies of described rows need: two vectors a thread against one, 205 and 273 us for
+// 512 threads and for whole rows; three or four 186 to 195, and 28.4 and 29.5 for rows of 7168 bytes.
+// Groups of 6, 12, 24 and 48 MB: 230, 215, 211 and 207 us, but from 36 MB on 5 us are lost where their source rows
+// no longer fit an L2 (4 MB); fewer than two groups an XCD lose a tenth.  The groups' rows drift apart by some fifty
+// tokens, so a group reads half as much again as its share of the source.
+// Up to 256 threads while the rows stay in the caches: 600 x 14336 10.7 -> 10.1 us.
 // ---------------------------------------------------------------------
 constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of a group: about 2 MB of source rows
 constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
 
 struct PackArgs {
     const uint8_t* src;
-    const uint8_t* scale_src;
-    const int64_t* ids;
-    const int64_t* num_rows_dev;
-    const int64_t* cumsum;  // [R + 1], grouped only
-    int num_ranks, group_log2, slots;
-    int64_t max_rows;
-    int num_src_rows, row_bytes, scale_row_bytes;
     uint8_t* dst;
+    int num_src_rows, row_bytes, threads;  // threads that move a row; with scales another wave
+    const uint8_t* scale_src;
     uint8_t* scale_dst;
+    int scale_row_bytes;
 };
 
 template <bool kStream>
-__device__ __forceinline__ void pack_row(const PackArgs& a, int64_t row) {
-    const int64_t id = a.ids[row];
+__device__ __forceinline__ void pack_row(const PackArgs& a, const int64_t* __restrict__ ids, int64_t row) {
+    const int64_t id = ids[row];
     if (id < 0 || id >= a.num_src_rows) return;
-    const int tid = threadIdx.x, threads = blockDim.x, num_vec = a.row_bytes / 16;
-    const uint8_t* s = a.src + id * a.row_bytes;
-    uint8_t* d = a.dst + row * a.row_bytes;
-    for (int v = tid; v < num_vec; v += 2 * threads) {
-        const bool second = v + threads < num_vec;
-        u32x4 r0 = load_u32x4<false>(s + int64_t(v) * 16), r1 = r0;
-        if (second) r1 = load_u32x4<false>(s + int64_t(v + threads) * 16);
-        store_u32x4<kStream>(d + int64_t(v) * 16, r0);
-        if (second) store_u32x4<kStream>(d + int64_t(v + threads) * 16, r1);
-    }
-    if (a.scale_src != nullptr) {
-        const uint32_t* ss = reinterpret_cast<const uint32_t*>(a.scale_src + id * a.scale_row_bytes);
-        uint32_t* sd = reinterpret_cast<uint32_t*>(a.scale_dst + row * a.scale_row_bytes);
-        for (int v = tid; v < a.scale_row_bytes / 4; v += threads) sd[v] = ss[v];
+    if (wave_in_block() * kWave < a.threads) {
+        block_copy_row<2, false, kStream>(a.src + id * a.row_bytes, a.dst + row * a.row_bytes,
+                                          a.row_bytes / 16, threadIdx.x, a.threads);
+    } else {
+        const uint32_t* from = reinterpret_cast<const uint32_t*>(a.scale_src + id * a.scale_row_bytes);
+        uint32_t* to = reinterpret_cast<uint32_t*>(a.scale_dst + row * a.scale_row_bytes);
+        for (int v = lane_id(); v < a.scale_row_bytes / 4; v += kWave) to[v] = from[v];
     }
 }
 
-template <bool kGrouped, bool kStream>
-__global__ __launch_bounds__(512) void pack_rows_kernel(PackArgs a) {
-    if constexpr (!kGrouped) {
-        int64_t num_rows = *a.num_rows_dev;
-        if (num_rows > a.max_rows) num_rows = a.max_rows;
-        for (int64_t i = blockIdx.x; i < num_rows; i += gridDim.x) pack_row<kStream>(a, i);
-    } else {
-        const int lane = lane_id(), xcd = int(blockIdx.x) & 7, i = int(blockIdx.x) >> 3;
-        const int g = (i / a.slots) * 8 + xcd;
-        // lane r: the part of rank r's list that is in the group
-        int64_t first = 0;
-        int skip = 0, size = 0;
-        if (lane < a.num_ranks) {
-            first = lane == 0 ? 0 : a.cumsum[lane];  // the list starts at its first row, whatever cumsum[0] is
-            const int64_t n = a.cumsum[lane + 1] - first;
-            skip = int((n * g) >> a.group_log2);
-            size = int((n * (g + 1)) >> a.group_log2) - skip;
-        }
-        const int incl = wave_inclusive_sum(size);
-        const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
-        const int64_t begin = first + skip - (incl - size);  // list row of slot s of the group: begin + s
-        for (int slot = i % a.slots; slot < total; slot += a.slots) {
-            const int r = __popcll(__ballot(incl <= slot));  // lanes past the ranks hold the total
-            const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(begin), r);
-            const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(begin >> 32), r);
-            const int64_t row = int64_t((uint64_t(hi) << 32) | lo) + slot;
-            if (row >= 0 && row < a.max_rows) pack_row<kStream>(a, row);
-        }
+template <bool kStream>
+__global__ __launch_bounds__(1024) void pack_rows_kernel(const int64_t* __restrict__ num_rows_dev,
+                                                         const int64_t* __restrict__ ids, int64_t max_rows,
+                                                         uint32_t grid, PackArgs a) {
+    int64_t num_rows = *num_rows_dev;
+    if (num_rows > max_rows) num_rows = max_rows;
+    for (int64_t i = blockIdx.x; i < num_rows; i += grid) pack_row<kStream>(a, ids, i);
+}
+
+template <bool kStream>
+__global__ __launch_bounds__(1024) void pack_groups_kernel(const int64_t* __restrict__ cumsum,
+                                                           const int64_t* __restrict__ ids, int64_t max_rows,
+                                                           int num_ranks, int group_log2, uint32_t slots, PackArgs a) {
+    const int lane = lane_id();
+    const uint32_t xcd = blockIdx.x & 7, i = blockIdx.x >> 3;
+    const uint32_t g = i / slots * 8 + xcd;
+    // lane r: the part of rank r's list that is in the group
+    int64_t first = 0;
+    int skip = 0, size = 0;
+    if (lane < num_ranks) {
+        first = lane == 0 ? 0 : cumsum[lane];  // the list starts at its first row, whatever cumsum[0] is
+        const int64_t n = cumsum[lane + 1] - first;
+        skip = int((n * g) >> group_log2);
+        size = int((n * (g + 1)) >> group_log2) - skip;
+    }
+    const int incl = wave_inclusive_sum(size);
+    const int total = __builtin_amdgcn_readlane(incl, kWave - 1);
+    const int64_t begin = first + skip - (incl - size);  // list row of slot s of the group: begin + s
+    for (int slot = i % slots; slot < total; slot += slots) {
+        const int r = __popcll(__ballot(incl <= slot));  // lanes past the ranks hold the total
+        const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(begin), r);
+        const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(begin >> 32), r);
+        const int64_t row = int64_t((uint64_t(hi) << 32) | lo) + slot;
+        if (row >= 0 && row < max_rows) pack_row<kStream>(a, ids, row);
     }
 }
 
@@ -834,29 +836,36 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
     EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(scale_src) & 3) == 0 && (reinterpret_cast<uintptr_t>(scale_dst) & 3) == 0);
     PackArgs a;
     a.src = reinterpret_cast<const uint8_t*>(src), a.scale_src = reinterpret_cast<const uint8_t*>(scale_src);
-    a.ids = sorted_token_ids, a.num_rows_dev = num_rows_dev, a.cumsum = send_cumsum, a.num_ranks = num_ranks;
-    a.max_rows = max_rows, a.num_src_rows = num_src_rows, a.row_bytes = row_bytes, a.scale_row_bytes = scale_row_bytes;
+    a.num_src_rows = num_src_rows, a.row_bytes = row_bytes, a.scale_row_bytes = scale_row_bytes;
     a.dst = reinterpret_cast<uint8_t*>(dst), a.scale_dst = reinterpret_cast<uint8_t*>(scale_dst);
-    a.group_log2 = 3, a.slots = 1;
-    int threads = (row_bytes / 32 + 63) / 64 * 64;  // two vectors a thread
-    threads = threads < 64 ? 64 : (threads > 512 ? 512 : threads);
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     const bool stream_rows = max_rows * row_bytes > kPackStreamBytes;
+    a.threads = flat_row_threads((row_bytes / 16 + 1) / 2, stream_rows ? 512 : 256);
+    const int threads = a.threads + (scale_src != nullptr ? kWave : 0);
     // Below a group's worth of packed rows everything stays in the caches and the grouping's lookup is one more
     // round trip in front of the rows: 6.5 MB 2.9 us against 3.4, 12 MB 3.9 either way, 22 MB 6.7 against 5.0.
     // A wave holds the ranks' parts one a lane, hence the 64.
     if (send_cumsum != nullptr && num_ranks > 1 && num_ranks <= kWave && max_rows * row_bytes > kPackGroupBytes) {
-        while (((max_rows * row_bytes) >> a.group_log2) > kPackGroupBytes && a.group_log2 < 16) ++a.group_log2;
+        int group_log2 = 3;  // two groups an XCD before a group may be larger
+        while (((max_rows * row_bytes) >> group_log2) > (group_log2 == 3 ? kPackGroupBytes : 2 * kPackGroupBytes) &&
+               group_log2 < 16)
+            ++group_log2;
         // rounding down the parts of every rank's list can put one more row per rank into a group
-        const int64_t slots = ((max_rows + (int64_t(1) << a.group_log2) - 1) >> a.group_log2) + num_ranks;
-        a.slots = int(slots < (1 << 14) ? slots : (1 << 14));  // the kernel goes round for the rest
-        const int64_t blocks = int64_t(a.slots) << a.group_log2;
-        if (stream_rows) pack_rows_kernel<true, true><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
-        else pack_rows_kernel<true, false><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
+        const int64_t needed = ((max_rows + (int64_t(1) << group_log2) - 1) >> group_log2) + num_ranks;
+        const uint32_t slots = uint32_t(needed < (1 << 14) ? needed : (1 << 14));  // the kernel goes round for the rest
+        const unsigned blocks = slots << group_log2;
+        if (stream_rows)
+            pack_groups_kernel<true><<<blocks, threads, 0, hs>>>(send_cumsum, sorted_token_ids, max_rows, num_ranks,
+                                                                 group_log2, slots, a);
+        else
+            pack_groups_kernel<false><<<blocks, threads, 0, hs>>>(send_cumsum, sorted_token_ids, max_rows, num_ranks,
+                                                                  group_log2, slots, a);
     } else {
-        const int64_t blocks = max_rows < (int64_t(1) << 22) ? max_rows : int64_t(1) << 22;
-        if (stream_rows) pack_rows_kernel<false, true><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
-        else pack_rows_kernel<false, false><<<dim3(unsigned(blocks)), threads, 0, hs>>>(a);
+        const unsigned blocks = unsigned(max_rows < (int64_t(1) << 22) ? max_rows : int64_t(1) << 22);
+        if (stream_rows)
+            pack_rows_kernel<true><<<blocks, threads, 0, hs>>>(num_rows_dev, sorted_token_ids, max_rows, blocks, a);
+        else
+            pack_rows_kernel<false><<<blocks, threads, 0, hs>>>(num_rows_dev, sorted_token_ids, max_rows, blocks, a);
     }
     EP_LAUNCH_CHECK();
     return 0;

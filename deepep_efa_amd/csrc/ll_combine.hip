@@ -376,7 +376,7 @@ __global__ __launch_bounds__(1024) void ll_combine_send_by_dest_kernel(
                 }
             }
             if (dst != nullptr && src_row < x_rows)  // < 0: the record has no row
-                block_copy_row<kStream>(x + src_row * row_bytes, dst, num_vec, threadIdx.x, threads);
+                block_copy_row<1, kStream, kStream>(x + src_row * row_bytes, dst, num_vec, threadIdx.x, threads);
         }
         if (uint64_t(block) + grid >= flat_rounds_end(records)) break;
         block += grid, i = flat_row_of_block(block);

@@ -413,15 +413,6 @@ __device__ __forceinline__ uint32_t flat_rounds_end(uint32_t rows) {
     return (rows + kFlatRound - 1) / kFlatRound * kFlatRound;
 }
 
-// Threads [0, threads) of a workgroup move a row, a vector each; wider rows go round.
-template <bool kStream>
-__device__ __forceinline__ void block_copy_row(const uint8_t* src, uint8_t* dst, int num_vec, int tid, int threads) {
-    const auto from = row_buffer(src, num_vec * 16), to = row_buffer(dst, num_vec * 16);
-    store_row_u32x4<kStream>(to, tid * 16, load_row_u32x4<kStream>(from, tid * 16));
-    for (int v = threads; v < num_vec; v += threads)
-        store_row_u32x4<kStream>(to, (v + tid) * 16, load_row_u32x4<kStream>(from, (v + tid) * 16));
-}
-
 // What a row carries besides its payload (the dispatch's rows; all null for the combine's).
 struct FlatTails {
     uint8_t* scale_dst;
@@ -445,7 +436,7 @@ static __global__ __launch_bounds__(1024) void ll_rows_flat_kernel(
             const uint8_t* s = src + uint64_t(src_row) * src_stride;
             if constexpr (kTails) {
                 if (wave_in_block() * kWave < data_threads) {
-                    block_copy_row<true>(s, dst + uint64_t(dst_row) * dst_stride, num_vec, tid, data_threads);
+                    block_copy_row<1, true, true>(s, dst + uint64_t(dst_row) * dst_stride, num_vec, tid, data_threads);
                 } else {  // the last wave: scales and source index
                     const int lane = lane_id();
                     int32_t info = 0;
@@ -460,19 +451,13 @@ static __global__ __launch_bounds__(1024) void ll_rows_flat_kernel(
                 const bool own = int32_t(dst_row) < 0;
                 uint8_t* base = own ? dst_own : dst;
                 const uint32_t to = own ? ~dst_row : dst_row;
-                if (base != nullptr) block_copy_row<true>(s, base + uint64_t(to) * dst_stride, num_vec, tid, data_threads);
+                if (base != nullptr) block_copy_row<1, true, true>(s, base + uint64_t(to) * dst_stride, num_vec, tid, data_threads);
             }
         }
         if (uint64_t(i) + grid >= flat_rounds_end(rows)) break;
         i += grid, row = flat_row_of_block(i);
         if (row < rows) src_row = uint32_t(desc[row].src_row), dst_row = uint32_t(desc[row].dst_row);
     }
-}
-
-// Threads that move a row's payload, a vector each, at most `most`: wider rows take whole trips of about equal size.
-inline int flat_row_threads(int num_vec, int most) {
-    const int trips = (num_vec + most - 1) / most;
-    return ((num_vec + trips - 1) / trips + 63) / 64 * 64;
 }
 
 __host__ __device__ inline int64_t segment_workspace_bytes(int num_experts, int max_tokens) {
