@@ -130,6 +130,69 @@ template <bool kStream>
 __device__ __forceinline__ void store_row_u32x4(__amdgpu_buffer_rsrc_t row, int offset, u32x4 v) {
     __builtin_amdgcn_raw_buffer_store_b128(v, row, offset, 0, kStream ? 2 : 0);
 }
+__device__ __forceinline__ float bf16_bits_to_f32(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
+__device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_float(packed & 0xffff0000u); }
+
+// The next kRows rows that `live` names, for the 8 channels at byte `off` of each: lane i holds row i's address and
+// weight.
+template <int kRows>
+struct RowsInFlight {
+    u32x4 v[kRows];
+    float w[kRows];
+    template <bool kStream, bool kWeighted>
+    __device__ __forceinline__ void load(uint64_t address, float weight, uint64_t& live, int off, int row_bytes) {
+#pragma unroll
+        for (int u = 0; u < kRows; ++u) {
+            const int k = __builtin_ctzll(live);
+            live &= ~(uint64_t(1) << k);
+            const uint32_t lo = __builtin_amdgcn_readlane(int(uint32_t(address)), k);
+            const uint32_t hi = __builtin_amdgcn_readlane(int(uint32_t(address >> 32)), k);
+            if constexpr (kWeighted) w[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), k));
+            const uint8_t* row = reinterpret_cast<const uint8_t*>((uint64_t(hi) << 32) | lo);
+            v[u] = load_row_u32x4<kStream>(row_buffer(row, row_bytes), off);
+        }
+    }
+    template <bool kWeighted>
+    __device__ __forceinline__ void add(float (&acc)[8]) const {
+#pragma unroll
+        for (int u = 0; u < kRows; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (kWeighted) {
+                    acc[2 * i] = __builtin_fmaf(bf16_lo(v[u][i]), w[u], acc[2 * i]);
+                    acc[2 * i + 1] = __builtin_fmaf(bf16_hi(v[u][i]), w[u], acc[2 * i + 1]);
+                } else {
+                    acc[2 * i] += bf16_lo(v[u][i]), acc[2 * i + 1] += bf16_hi(v[u][i]);
+                }
+            }
+    }
+};
+
+// acc += weight * row (or row) over the rows that `live` names, in ascending order.  Eight rows are in flight, then what
+// is left of eight together; without a branch for each row, which costs a wave as much as the row's arithmetic.
+template <bool kStream, bool kWeighted>
+__device__ __forceinline__ void add_rows(uint64_t address, float weight, uint64_t live, int off, int row_bytes,
+                                         float (&acc)[8]) {
+    int n = __popcll(live);
+    for (; n >= 8; n -= 8) {
+        RowsInFlight<8> rows;
+        rows.load<kStream, kWeighted>(address, weight, live, off, row_bytes);
+        __builtin_amdgcn_sched_barrier(0);  // no row's arithmetic, and so its wait, in front of another's load
+        rows.add<kWeighted>(acc);
+    }
+    RowsInFlight<4> four;
+    RowsInFlight<2> two;
+    RowsInFlight<1> one;
+    if ((n & 4) != 0) four.load<kStream, kWeighted>(address, weight, live, off, row_bytes);
+    if ((n & 2) != 0) two.load<kStream, kWeighted>(address, weight, live, off, row_bytes);
+    if ((n & 1) != 0) one.load<kStream, kWeighted>(address, weight, live, off, row_bytes);
+    __builtin_amdgcn_sched_barrier(0);
+    if ((n & 4) != 0) four.add<kWeighted>(acc);
+    if ((n & 2) != 0) two.add<kWeighted>(acc);
+    if ((n & 1) != 0) one.add<kWeighted>(acc);
+}
+
 // Threads [0, threads) of a workgroup move a row, kVecs vectors of each in flight; wider rows go round.
 template <int kVecs, bool kStreamLoad, bool kStreamStore>
 __device__ __forceinline__ void block_copy_row(const uint8_t* src, uint8_t* dst, int num_vec, int tid, int threads) {
@@ -178,19 +241,12 @@ __device__ __forceinline__ uint64_t wave_uniform_u64(uint64_t v) {
 
 __device__ __forceinline__ uint64_t lanes_below(int lane) { return (uint64_t(1) << lane) - 1; }
 
-__device__ __forceinline__ float bf16_bits_to_f32(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
-__device__ __forceinline__ float bf16_lo(uint32_t packed) { return __uint_as_float(packed << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_float(packed & 0xffff0000u); }
-
-// float32 -> bf16 bits, round to nearest even (NaN kept quiet).
-__device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return u >> 16;
-}
+// Two float32 -> bf16, round to nearest even, NaN kept quiet: one instruction.
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+    typedef float float2_ __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const float2_ v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
 }
 
 // max over the 8 lanes that share one 128-channel group (lanes 8i..8i+7):

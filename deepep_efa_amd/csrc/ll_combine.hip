@@ -206,34 +206,8 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, uin
         for (int i = 0; i < 4; ++i) acc[2 * i] = bf16_lo(prev[i]), acc[2 * i + 1] = bf16_hi(prev[i]);
     }
 
-    for (int k0 = 0; k0 < num_topk; k0 += 8) {
-        u32x4 v[8];
-        float wgt[8];
-        bool live[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int k = k0 + u;
-            live[u] = k < num_topk && ((live_mask >> k) & 1) != 0;
-            wgt[u] = 0.0f;
-            if (live[u]) {
-                const uint32_t lo32 = __builtin_amdgcn_readlane(uint32_t(my_row), k);
-                const uint32_t hi32 = __builtin_amdgcn_readlane(uint32_t(my_row >> 32), k);
-                wgt[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_weight), k));
-                const uint8_t* row = reinterpret_cast<const uint8_t*>((uint64_t(hi32) << 32) | lo32);
-                v[u] = load_row_u32x4<kStream>(row_buffer(row, int(row_bytes)), off);
-            }
-        }
-        DEEPEP_PHASE(1);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            if (!live[u]) continue;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                acc[2 * i] = __builtin_fmaf(bf16_lo(v[u][i]), wgt[u], acc[2 * i]);
-                acc[2 * i + 1] = __builtin_fmaf(bf16_hi(v[u][i]), wgt[u], acc[2 * i + 1]);
-            }
-        }
-    }
+    DEEPEP_PHASE(1);
+    add_rows<kStream, true>(my_row, my_weight, live_mask, off, int(row_bytes), acc);
     DEEPEP_PHASE(2);
     u32x4 o;
 #pragma unroll

@@ -148,12 +148,11 @@ __global__ __launch_bounds__(512) void combine_reduce_kernel(
 
     for (int r0 = 0; r0 < num_ranks; r0 += kWave) {
         const int r = r0 + lane;
-        int my_row = -1;
-        if (r < num_ranks) {
-            const uint8_t member = is_token_in_rank[int64_t(t) * num_ranks + r];
-            my_row = row_of_pair[int64_t(t) * num_ranks + r];  // means nothing for a rank the token is not sent to
-            if (member == 0 || my_row < 0 || my_row >= max_rows) my_row = -1;
-        }
+        const int64_t pair = int64_t(t) * num_ranks + (r < num_ranks ? r : 0);
+        int member = is_token_in_rank[pair];
+        int my_row = row_of_pair[pair];  // means nothing for a rank the token is not sent to
+        asm volatile("" : "+v"(member), "+v"(my_row));  // one trip: left alone, the second waits for the first
+        if (r >= num_ranks || member == 0 || my_row < 0 || my_row >= max_rows) my_row = -1;
         uint64_t present = __ballot(my_row >= 0);
         while (present != 0) {
             u32x4 v[8];
