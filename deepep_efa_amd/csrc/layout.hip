@@ -562,11 +562,12 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 //    78 MB  24.0 / 15.3   48.8 / 54.2     140 MB  42.0 / 25.3   93.9 / 91.4
 //    97 MB  29.3 / 18.4   59.8 / 65.7     155 MB  48.5 / 27.4  107.2 / 102.5    311 MB  88.7 / 54.6  209 / 197
 // Grouping and hint against list order and ordinary stores: 12289 x 14336 bytes (934 MB) 305 -> 211 us, 4096 x 7168
-// (155 MB) 48.1 -> 27.3.  Rows as buffers and the scales in a wave of their own (a wave that stores its payload first
-// waits for that before its scales are there): 202 -> 188 us (5.9 TB/s on the bytes that have to move), 9000 x 10240 to
-// 32 ranks 151 -> 136, 4096 x 7168 27.4 -> 27.2.  Four trips to memory stand in front of a row here, which takes more
-// rows in flight to hide than the copies of described rows need: two vectors a thread against one, 205 and 273 us for
-// 512 threads and for whole rows; three or four 186 to 195, and 28.4 and 29.5 for rows of 7168 bytes.
+// (155 MB) 48.1 -> 27.3.  Rows as buffers, and the scales fetched with the payload instead of behind its stores (a wave
+// of their own takes the place of payload: 28.6 -> 30.5 us for 4096 x 7168): 202 -> 188 us (5.9 TB/s on the bytes that
+// have to move), 9000 x 10240 to 32 ranks 151 -> 136, 4096 x 7168 27.4 -> 27.1.  Four trips to memory stand in front of a
+// row here, which takes more rows in flight to hide than the copies of described rows need: two vectors a thread
+// against one, 205 and 273 us for 512 threads and for whole rows; three or four 186 to 195, and 28.4 and 29.5 for rows
+// of 7168 bytes.
 // Groups of 6, 12, 24 and 48 MB: 230, 215, 211 and 207 us, but from 36 MB on 5 us are lost where their source rows
 // no longer fit an L2 (4 MB); fewer than two groups an XCD lose a tenth.  The groups' rows drift apart by some fifty
 // tokens, so a group reads half as much again as its share of the source.
@@ -578,7 +579,7 @@ constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
 struct PackArgs {
     const uint8_t* src;
     uint8_t* dst;
-    int num_src_rows, row_bytes, threads;  // threads that move a row; with scales another wave
+    int num_src_rows, row_bytes, threads;
     const uint8_t* scale_src;
     uint8_t* scale_dst;
     int scale_row_bytes;
@@ -588,14 +589,15 @@ template <bool kStream>
 __device__ __forceinline__ void pack_row(const PackArgs& a, const int64_t* __restrict__ ids, int64_t row) {
     const int64_t id = ids[row];
     if (id < 0 || id >= a.num_src_rows) return;
-    if (wave_in_block() * kWave < a.threads) {
-        block_copy_row<2, false, kStream>(a.src + id * a.row_bytes, a.dst + row * a.row_bytes,
-                                          a.row_bytes / 16, threadIdx.x, a.threads);
-    } else {
-        const uint32_t* from = reinterpret_cast<const uint32_t*>(a.scale_src + id * a.scale_row_bytes);
-        uint32_t* to = reinterpret_cast<uint32_t*>(a.scale_dst + row * a.scale_row_bytes);
-        for (int v = lane_id(); v < a.scale_row_bytes / 4; v += kWave) to[v] = from[v];
-    }
+    const int tid = threadIdx.x;
+    const uint32_t* scales = reinterpret_cast<const uint32_t*>(a.scale_src + id * a.scale_row_bytes);
+    uint32_t* scales_to = reinterpret_cast<uint32_t*>(a.scale_dst + row * a.scale_row_bytes);
+    const int num_scales = a.scale_src != nullptr ? a.scale_row_bytes / 4 : 0;
+    uint32_t scale = 0;
+    if (tid < num_scales) scale = scales[tid];  // in flight with the payload, not behind its stores
+    block_copy_row<2, false, kStream>(a.src + id * a.row_bytes, a.dst + row * a.row_bytes, a.row_bytes / 16, tid, a.threads);
+    if (tid < num_scales) scales_to[tid] = scale;
+    for (int v = tid + a.threads; v < num_scales; v += a.threads) scales_to[v] = scales[v];
 }
 
 template <bool kStream>
@@ -841,7 +843,7 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     const bool stream_rows = max_rows * row_bytes > kPackStreamBytes;
     a.threads = flat_row_threads((row_bytes / 16 + 1) / 2, stream_rows ? 512 : 256);
-    const int threads = a.threads + (scale_src != nullptr ? kWave : 0);
+    const int threads = a.threads;
     // Below a group's worth of packed rows everything stays in the caches and the grouping's lookup is one more
     // round trip in front of the rows: 6.5 MB 2.9 us against 3.4, 12 MB 3.9 either way, 22 MB 6.7 against 5.0.
     // A wave holds the ranks' parts one a lane, hence the 64.
