@@ -26,6 +26,7 @@ struct CombineSendArgs {
     const uint8_t* x;
     const int64_t* layout_range;
     int hidden, num_local_experts, num_ranks, rank, max_tokens, parts_log2;
+    RankDivider expert_of;
     uint8_t* combine_staging;
     uint8_t* combine_send_slots;
 };
@@ -48,14 +49,14 @@ __device__ __forceinline__ void combine_send_rows_impl(const CombineSendArgs& a,
         const int s = lane * kPer + u;
         int c = int(ranges[u] & 0xffffffffll);
         c = c < 0 ? 0 : (c > max_tokens ? max_tokens : c);
-        if (skip_own && s % num_ranks == a.rank) c = 0;
+        if (skip_own && s - a.expert_of(s) * num_ranks == a.rank) c = 0;
         seg_table.cnt[u] = c;
         seg_table.aux[u] = int(ranges[u] >> 32);
     }
     wave_segments_finish(seg_table);
     DEEPEP_PHASE(1);
 
-    const int64_t row_bytes = int64_t(a.hidden) * 2;
+    const uint32_t row_bytes = uint32_t(a.hidden) * 2;
     const int num_vec = int(row_bytes / 16);
     const int64_t slots_per_expert = int64_t(max_tokens) * num_ranks;
     const int waves_total = num_blocks * waves;
@@ -67,20 +68,22 @@ __device__ __forceinline__ void combine_send_rows_impl(const CombineSendArgs& a,
         int seg_first, b;
         const int seg = wave_segments_find(seg_table, row, seg_first, b);
         const int j = row - seg_first;
-        const int le = seg / num_ranks;
+        const int le = a.expert_of(seg);
         const int s = seg - le * num_ranks;
         if (b < 0 || int64_t(b) + j >= slots_per_expert) continue;  // malformed range: never read past the expert
-        const uint8_t* src = a.x + (int64_t(le) * slots_per_expert + b + j) * row_bytes;
+        const uint8_t* src = a.x + uint64_t(uint32_t(le * slots_per_expert) + uint32_t(b + j)) * row_bytes;
         uint8_t* dst;
         if (s == a.rank)
-            dst = a.combine_staging + ((int64_t(a.rank) * a.num_local_experts + le) * max_tokens + j) * row_bytes;
+            dst = a.combine_staging + uint64_t(uint32_t((a.rank * a.num_local_experts + le) * max_tokens + j)) * row_bytes;
         else if (a.combine_send_slots != nullptr)
-            dst = a.combine_send_slots + (int64_t(seg) * max_tokens + j) * row_bytes;
+            dst = a.combine_send_slots + uint64_t(uint32_t(seg * max_tokens + j)) * row_bytes;
         else
             continue;
         int v_begin, v_end;
-        row_part_range(num_vec, parts, part, v_begin, v_end);
-        wave_copy_vec16<4, kStream>(src, dst, v_begin, v_end, lane);
+        row_part_range(num_vec, a.parts_log2, part, v_begin, v_end);
+        RowPart<4, kStream> piece;
+        piece.load(src, v_begin, v_end, lane);
+        piece.store(dst, v_begin, lane);
     }
     DEEPEP_PHASE(2);
 }
@@ -365,6 +368,7 @@ static CombineSendArgs make_combine_send_args(const void* x, const int64_t* layo
     sa.x = reinterpret_cast<const uint8_t*>(x);
     sa.layout_range = layout_range;
     sa.hidden = hidden, sa.num_local_experts = num_experts / num_ranks, sa.num_ranks = num_ranks, sa.rank = rank;
+    sa.expert_of = make_rank_divider(num_ranks);
     sa.max_tokens = max_tokens;
     sa.parts_log2 = choose_row_parts_log2(estimated_rows(expected_rows, num_experts, max_tokens), int64_t(hidden) * 2);
     sa.combine_staging = reinterpret_cast<uint8_t*>(combine_staging);

@@ -539,6 +539,7 @@ struct RecvArgs {
     const uint8_t* recv_staging;
     const int32_t* recv_count;
     int hidden, num_local_experts, num_ranks, max_tokens, fmt, parts_log2;
+    RankDivider expert_of;
     uint8_t* packed_x;
     uint8_t* packed_scales;
     int32_t* src_info;
@@ -601,15 +602,19 @@ __device__ __forceinline__ void own_row_counts_finish(const RecvArgs& a, const i
     lds_barrier();
 }
 
+constexpr int kRecvDepth = 4;  // 16-byte loads in flight per lane
+
 // One unit of the copying waves' work: a run of 16-byte vectors of one staged row.
+template <bool kStream>
 struct RecvItem {
     const uint8_t* src;
     int le, source, slot;  // slot: the row's place among the rows copied for the expert, own rows not counted
-    int v_begin, v_end;
+    int v_begin;
     bool carries_tail;  // also moves the row's scales and source index
+    RowPart<kRecvDepth, kStream> payload;
+    uint32_t scale;  // a lane's scale word, with the tail
+    int32_t info;
 };
-
-constexpr int kRecvDepth = 4;  // 16-byte loads in flight per lane
 
 // Workgroups [0, num_copy_blocks) copy rows; workgroup num_copy_blocks writes layout_range,
 // packed_count and stats and copies nothing.  A copying wave builds the segment prefix in its own
@@ -667,7 +672,7 @@ __device__ __forceinline__ void recv_rows_impl(const RecvArgs& a, int block, int
         seg_table.cnt[u] = clamp_count(seg_table.cnt[u], max_tokens);
     }
     if (own_placed) {  // the own segments (le * R + own_rank) hold nothing to copy
-        int source = (lane * kPer) % num_ranks;  // source rank of this lane's first segment
+        int source = lane * kPer - a.expert_of(lane * kPer) * num_ranks;  // source rank of this lane's first segment
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
             if (source == own_rank) seg_table.cnt[u] = 0;
@@ -677,86 +682,71 @@ __device__ __forceinline__ void recv_rows_impl(const RecvArgs& a, int block, int
     wave_segments_finish(seg_table);
     DEEPEP_PHASE(1);
 
-    const int64_t data_bytes = row_data_bytes(a.hidden, a.fmt);
-    const int64_t data_pad = align16(data_bytes);
-    const int64_t scale_bytes = row_scale_bytes(a.hidden, a.fmt);
-    const int64_t stride = row_stride_bytes(a.hidden, a.fmt);
-    const int64_t slots_per_expert = int64_t(max_tokens) * num_ranks;
+    const uint32_t data_bytes = uint32_t(row_data_bytes(a.hidden, a.fmt));
+    const uint32_t data_pad = uint32_t(align16(data_bytes));
+    const uint32_t scale_bytes = uint32_t(row_scale_bytes(a.hidden, a.fmt));
+    const uint32_t stride = uint32_t(row_stride_bytes(a.hidden, a.fmt));
+    const int slots_per_expert = max_tokens * num_ranks;
     const int waves_total = num_copy_blocks * waves;
     const int num_vec = int(data_bytes / 16);
     const int parts = 1 << a.parts_log2;
     const int num_items = seg_table.total << a.parts_log2;
 
-    auto decode = [&](int item, RecvItem& it) {
-        const int row = item >> a.parts_log2, part = item & (parts - 1);
-        int seg_first, unused;
-        const int seg = wave_segments_find(seg_table, row, seg_first, unused);
-        it.le = seg / num_ranks;
-        it.source = seg - it.le * num_ranks;
-        it.slot = row - wave_segments_prefix(seg_table, it.le * num_ranks);
-        it.src = a.recv_staging + (int64_t(seg) * max_tokens + (row - seg_first)) * stride;
-        row_part_range(num_vec, parts, part, it.v_begin, it.v_end);
-        it.carries_tail = part == parts - 1;  // the last part is the shortest
-    };
     // What the tail-carrying part of a row moves besides payload: one scale word per lane (the first 64;
     // a wider row's remainder is copied after the stores) and, in lane 0, the source index.  They are
     // loaded with the payload, not behind its stores: one round trip per row instead of two.
     const int scale_dwords = int(scale_bytes / 4);
     const bool has_scales = a.packed_scales != nullptr && scale_dwords > 0;
-    uint32_t tail_scale = 0;
-    int32_t tail_info = 0;
-    auto load_first = [&](const RecvItem& it, u32x4 (&r)[kRecvDepth]) {
-#pragma unroll
-        for (int u = 0; u < kRecvDepth; ++u) {
-            const int v = it.v_begin + u * kWave + lane;
-            if (v < it.v_end) r[u] = load_u32x4<kStream>(it.src + int64_t(v) * 16);
-        }
+    auto load_first = [&](int item, RecvItem<kStream>& it) {
+        const int row = item >> a.parts_log2, part = item & (parts - 1);
+        int seg_first, unused, v_end;
+        const int seg = wave_segments_find(seg_table, row, seg_first, unused);
+        it.le = a.expert_of(seg);
+        it.source = seg - it.le * num_ranks;
+        it.src = a.recv_staging + uint64_t(uint32_t(seg * max_tokens + (row - seg_first))) * stride;
+        row_part_range(num_vec, a.parts_log2, part, it.v_begin, v_end);
+        it.payload.load(it.src, it.v_begin, v_end, lane);
+        it.carries_tail = part == parts - 1;  // the last part is the shortest
+        it.scale = 0, it.info = 0;
         if (it.carries_tail) {
-            if (has_scales && lane < scale_dwords) tail_scale = reinterpret_cast<const uint32_t*>(it.src + data_pad)[lane];
-            if (lane == 0) tail_info = *reinterpret_cast<const int32_t*>(it.src + data_pad + align16(scale_bytes));
+            if (has_scales && lane < scale_dwords) it.scale = reinterpret_cast<const uint32_t*>(it.src + data_pad)[lane];
+            if (lane == 0) it.info = *reinterpret_cast<const int32_t*>(it.src + data_pad + uint32_t(align16(scale_bytes)));
         }
+        it.slot = row - wave_segments_prefix(seg_table, it.le * num_ranks);
     };
-    auto finish = [&](const RecvItem& it, const u32x4 (&r)[kRecvDepth]) {
+    auto finish = [&](RecvItem<kStream>& it) {
         int slot = it.slot;
-        if (own_placed && it.source > own_rank) slot += clamp_count(own_cnt[it.le], max_tokens);
-        const int64_t out_row = int64_t(it.le) * slots_per_expert + slot;
-        uint8_t* dst = a.packed_x + out_row * data_bytes;
-#pragma unroll
-        for (int u = 0; u < kRecvDepth; ++u) {
-            const int v = it.v_begin + u * kWave + lane;
-            if (v < it.v_end) store_u32x4<kStream>(dst + int64_t(v) * 16, r[u]);
-        }
-        wave_copy_vec16<kRecvDepth, kStream>(it.src, dst, it.v_begin + kRecvDepth * kWave, it.v_end, lane);
+        if (own_placed && it.source > own_rank)
+            slot += clamp_count(__builtin_amdgcn_readfirstlane(own_cnt[it.le]), max_tokens);
+        const uint32_t out_row = uint32_t(it.le * slots_per_expert + slot);
+        it.payload.store(a.packed_x + uint64_t(out_row) * data_bytes, it.v_begin, lane);
         if (!it.carries_tail) return;
         if (has_scales) {
             const uint32_t* s32 = reinterpret_cast<const uint32_t*>(it.src + data_pad);
-            uint32_t* d32 = reinterpret_cast<uint32_t*>(a.packed_scales + out_row * scale_bytes);
-            if (lane < scale_dwords) d32[lane] = tail_scale;
+            uint32_t* d32 = reinterpret_cast<uint32_t*>(a.packed_scales + uint64_t(out_row) * scale_bytes);
+            if (lane < scale_dwords) d32[lane] = it.scale;
             for (int v = kWave + lane; v < scale_dwords; v += kWave) d32[v] = s32[v];
         }
-        if (lane == 0) a.src_info[out_row] = tail_info;
+        if (lane == 0) a.src_info[out_row] = it.info;
     };
 
-    RecvItem it;
-    u32x4 r[kRecvDepth];
+    RecvItem<kStream> it;
     int item = block * waves + w;
     const bool have_first = item < num_items;
     if (have_first) {
-        decode(item, it);
         DEEPEP_PHASE(2);
-        load_first(it, r);
+        load_first(item, it);
     }
     // every wave of the workgroup passes here, with or without rows to copy
     if (own_placed) own_row_counts_finish(a, own_topk, own_entries, own_rank, own_cnt, own_loads);
     if (have_first) {
-        finish(it, r);
+        finish(it);
         DEEPEP_PHASE(3);
         item += waves_total;
     }
     for (; item < num_items; item += waves_total) {
-        decode(item, it);
-        load_first(it, r);
-        finish(it, r);
+        load_first(item, it);
+        finish(it);
     }
 }
 
@@ -1204,7 +1194,7 @@ static RecvArgs make_recv_args(const void* recv_staging, const int32_t* recv_cou
     ra.recv_staging = reinterpret_cast<const uint8_t*>(recv_staging);
     ra.recv_count = recv_count;
     ra.hidden = hidden, ra.num_local_experts = num_experts / num_ranks, ra.num_ranks = num_ranks;
-    ra.max_tokens = max_tokens, ra.fmt = row_format;
+    ra.max_tokens = max_tokens, ra.fmt = row_format, ra.expert_of = make_rank_divider(num_ranks);
     const int64_t rows = estimated_rows(expected_rows, num_experts, max_tokens), row_bytes = row_data_bytes(hidden, row_format);
     ra.parts_log2 = choose_row_parts_log2(rows, row_bytes);
     // A row of up to 4 KiB is what a wave loads at once (kRecvDepth): with enough rows to occupy the chip a wave

@@ -374,6 +374,7 @@ struct OrderedRecvArgs {
     const int32_t* all_num_routed;  // [R, E]
     int num_experts, num_local_experts, num_ranks, rank, max_tokens;
     int hidden, fmt, parts_log2;
+    RankDivider expert_of;
     int64_t slot_rows, row_capacity;
     uint8_t* packed_x;
     uint8_t* packed_scales;
@@ -402,13 +403,13 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
     // sent / first / kept of every pair, pairs in (expert, source) order: one global load per pair,
     // the sums over the lower experts from LDS
     for (int seg = tid; seg < num_segments; seg += threads) {
-        const int le = seg / num_ranks, src = seg - le * num_ranks;
+        const int le = a.expert_of(seg), src = seg - le * num_ranks;
         const int c = a.all_num_routed[int64_t(src) * a.num_experts + a.rank * num_local + le];
         sent[seg] = c < 0 ? 0 : (c > max_tokens ? max_tokens : c);
     }
     lds_barrier();
     for (int seg = tid; seg < num_segments; seg += threads) {
-        const int le = seg / num_ranks, src = seg - le * num_ranks;
+        const int le = a.expert_of(seg), src = seg - le * num_ranks;
         int before = 0;
         for (int e2 = 0; e2 < le; ++e2) before += sent[e2 * num_ranks + src];
         const int64_t room = a.slot_rows - before;
@@ -424,7 +425,7 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
         lds_barrier();
         block_exclusive_scan(place, num_segments, wave_totals);
         for (int seg = tid; seg < num_segments; seg += threads) {
-            const int le = seg / num_ranks;
+            const int le = a.expert_of(seg);
             const int64_t begin = place[seg] - place[le * num_ranks];
             a.layout_range[seg] = kept[seg] > 0 ? ((begin << 32) | int64_t(kept[seg])) : 0;
         }
@@ -446,10 +447,10 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
     }
     wave_segments_finish(seg_table);
 
-    const int64_t data_bytes = row_data_bytes(a.hidden, a.fmt);
-    const int64_t data_pad = align16(data_bytes);
-    const int64_t scale_bytes = row_scale_bytes(a.hidden, a.fmt);
-    const int64_t stride = row_stride_bytes(a.hidden, a.fmt);
+    const uint32_t data_bytes = uint32_t(row_data_bytes(a.hidden, a.fmt));
+    const uint32_t data_pad = uint32_t(align16(data_bytes));
+    const uint32_t scale_bytes = uint32_t(row_scale_bytes(a.hidden, a.fmt));
+    const uint32_t stride = uint32_t(row_stride_bytes(a.hidden, a.fmt));
     const int num_vec = int(data_bytes / 16);
     const int parts = 1 << a.parts_log2;
     const int num_items = seg_table.total << a.parts_log2;
@@ -459,38 +460,29 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
 
     for (int item = block * waves + w; item < num_items; item += waves_total) {
         const int row = item >> a.parts_log2, part = item & (parts - 1);
-        int seg_first, in_message;
+        int seg_first, in_message, v_begin, v_end;
         const int seg = wave_segments_find(seg_table, row, seg_first, in_message);
-        const int le = seg / num_ranks, src = seg - le * num_ranks;
+        const int le = a.expert_of(seg), src = seg - le * num_ranks;
         const int j = row - seg_first;
-        const uint8_t* from = a.rows + (int64_t(src) * a.slot_rows + in_message + j) * stride;
-        const int64_t out_row = int64_t(le) * slots_per_expert + (row - wave_segments_prefix(seg_table, le * num_ranks));
-        uint8_t* to = a.packed_x + out_row * data_bytes;
-        int v_begin, v_end;
-        row_part_range(num_vec, parts, part, v_begin, v_end);
+        const uint8_t* from = a.rows + uint64_t(uint32_t(src * int(a.slot_rows) + in_message + j)) * stride;
+        row_part_range(num_vec, a.parts_log2, part, v_begin, v_end);
+        RowPart<kOrderedDepth, false> payload;
+        payload.load(from, v_begin, v_end, lane);
         const bool carries_tail = part == parts - 1;  // the last part is the shortest
-        u32x4 r[kOrderedDepth];
-#pragma unroll
-        for (int u = 0; u < kOrderedDepth; ++u) {
-            const int v = v_begin + u * kWave + lane;
-            if (v < v_end) r[u] = load_u32x4<false>(from + int64_t(v) * 16);
-        }
         uint32_t tail_scale = 0;
         int32_t tail_info = 0;
         if (carries_tail) {  // scales and source index travel with the payload: one round trip per row
             if (has_scales && lane < scale_dwords) tail_scale = reinterpret_cast<const uint32_t*>(from + data_pad)[lane];
-            if (lane == 0) tail_info = *reinterpret_cast<const int32_t*>(from + data_pad + align16(scale_bytes));
+            if (lane == 0)
+                tail_info = *reinterpret_cast<const int32_t*>(from + data_pad + uint32_t(align16(scale_bytes)));
         }
-#pragma unroll
-        for (int u = 0; u < kOrderedDepth; ++u) {
-            const int v = v_begin + u * kWave + lane;
-            if (v < v_end) store_u32x4<false>(to + int64_t(v) * 16, r[u]);
-        }
-        wave_copy_vec16<kOrderedDepth, false>(from, to, v_begin + kOrderedDepth * kWave, v_end, lane);
+        const uint32_t out_row =
+            uint32_t(le * slots_per_expert) + uint32_t(row - wave_segments_prefix(seg_table, le * num_ranks));
+        payload.store(a.packed_x + uint64_t(out_row) * data_bytes, v_begin, lane);
         if (!carries_tail) continue;
         if (has_scales) {
             const uint32_t* s32 = reinterpret_cast<const uint32_t*>(from + data_pad);
-            uint32_t* d32 = reinterpret_cast<uint32_t*>(a.packed_scales + out_row * scale_bytes);
+            uint32_t* d32 = reinterpret_cast<uint32_t*>(a.packed_scales + uint64_t(out_row) * scale_bytes);
             if (lane < scale_dwords) d32[lane] = tail_scale;
             for (int v = kWave + lane; v < scale_dwords; v += kWave) d32[v] = s32[v];
         }
@@ -504,7 +496,7 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
     // not), then the source's rows for the lower experts, then j.
     if (a.record_packed_row == nullptr) return;
     for (int seg = waves_total - 1 - (block * waves + w); seg < num_segments; seg += waves_total) {
-        const int le = seg / num_ranks, src = seg - le * num_ranks;
+        const int le = a.expert_of(seg), src = seg - le * num_ranks;
         int lower = 0;  // rows the lower sources sent, all experts
         for (int r = lane; r < src; r += kWave)
             for (int e2 = 0; e2 < num_local; ++e2) lower += sent[e2 * num_ranks + r];
@@ -674,7 +666,7 @@ int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_
         oa.rank = rank, oa.max_tokens = num_max_dispatch_tokens_per_rank;
         oa.hidden = hidden, oa.fmt = row_format;
         oa.parts_log2 = choose_row_parts_log2(expected, row_data_bytes(hidden, row_format));
-        oa.slot_rows = slot_rows, oa.row_capacity = row_capacity;
+        oa.slot_rows = slot_rows, oa.row_capacity = row_capacity, oa.expert_of = make_rank_divider(num_ranks);
         oa.packed_x = reinterpret_cast<uint8_t*>(packed_recv_x);
         oa.packed_scales = row_format == kRowBF16 ? nullptr : reinterpret_cast<uint8_t*>(packed_recv_scales);
         oa.src_info = packed_recv_src_info, oa.layout_range = packed_recv_layout_range;

@@ -61,10 +61,21 @@ struct WaveSegments {
 };
 
 // Lane l's kPer consecutive values p[l * kPer + u] (0 beyond n), as 16-byte loads where a whole
-// vector lies inside the array.  p must be 16-byte aligned.
+// vector lies inside the array.  p must be 16-byte aligned.  Arrays of whole vectors are read as a
+// buffer, whose loads past the end give zeros without a branch for each of them.
 template <int kPer>
 __device__ __forceinline__ void wave_load_int32(const int32_t* __restrict__ p, int n, int lane, int (&out)[kPer]) {
     static_assert(kPer % 4 == 0, "whole 16-byte vectors per lane");
+    if (n % 4 == 0) {
+        const auto all = row_buffer(reinterpret_cast<const uint8_t*>(p), n * 4);
+#pragma unroll
+        for (int v = 0; v < kPer / 4; ++v) {
+            const u32x4 q = load_row_u32x4<false>(all, lane * kPer * 4 + v * 16);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[v * 4 + i] = int(q[i]);
+        }
+        return;
+    }
 #pragma unroll
     for (int v = 0; v < kPer / 4; ++v) {
         const int s0 = lane * kPer + v * 4;
@@ -83,6 +94,16 @@ template <int kPer>
 __device__ __forceinline__ void wave_load_int64(const int64_t* __restrict__ p, int n, int lane,
                                                 int64_t (&out)[kPer]) {
     static_assert(kPer % 2 == 0, "whole 16-byte vectors per lane");
+    if (n % 2 == 0) {
+        const auto all = row_buffer(reinterpret_cast<const uint8_t*>(p), n * 8);
+#pragma unroll
+        for (int v = 0; v < kPer / 2; ++v) {
+            const u32x4 q = load_row_u32x4<false>(all, lane * kPer * 8 + v * 16);
+            out[v * 2] = int64_t((uint64_t(q[1]) << 32) | q[0]);
+            out[v * 2 + 1] = int64_t((uint64_t(q[3]) << 32) | q[2]);
+        }
+        return;
+    }
 #pragma unroll
     for (int v = 0; v < kPer / 2; ++v) {
         const int s0 = lane * kPer + v * 2;
@@ -139,32 +160,48 @@ __device__ __forceinline__ int wave_segments_find(const WaveSegments<kPer>& t, i
     return owner * kPer + __builtin_amdgcn_readlane(found, owner);
 }
 
-// Copies 16-byte vectors [v_begin, v_end) of a row with one wave, kDepth loads in flight per lane.
-template <int kDepth, bool kStream = false>
-__device__ __forceinline__ void wave_copy_vec16(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
-                                                int v_begin, int v_end, int lane) {
-    for (int base = v_begin; base < v_end; base += kWave * kDepth) {
-        u32x4 r[kDepth];
-#pragma unroll
-        for (int u = 0; u < kDepth; ++u) {
-            const int v = base + u * kWave + lane;
-            if (v < v_end) r[u] = load_u32x4<kStream>(src + int64_t(v) * 16);
-        }
-#pragma unroll
-        for (int u = 0; u < kDepth; ++u) {
-            const int v = base + u * kWave + lane;
-            if (v < v_end) store_u32x4<kStream>(dst + int64_t(v) * 16, r[u]);
-        }
-    }
+// Segments, in (expert, source) order, to experts: n / num_ranks for n below 2^16 by one multiplication.
+struct RankDivider {
+    uint32_t magic;  // 0: one rank
+    __device__ __forceinline__ int operator()(int n) const { return magic != 0 ? int(__umulhi(uint32_t(n), magic)) : n; }
+};
+inline RankDivider make_rank_divider(int num_ranks) {
+    return RankDivider{num_ranks == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + num_ranks - 1) / num_ranks)};
 }
 
-// A row of num_vec vectors cut into `parts` runs of whole 64-vector (1 KiB) chunks.
-__device__ __forceinline__ void row_part_range(int num_vec, int parts, int part, int& v_begin, int& v_end) {
+// A row of num_vec vectors cut into 2^parts_log2 runs of whole 64-vector (1 KiB) chunks.
+__device__ __forceinline__ void row_part_range(int num_vec, int parts_log2, int part, int& v_begin, int& v_end) {
     const int chunks = (num_vec + kWave - 1) / kWave;
-    const int per = (chunks + parts - 1) / parts;
+    const int per = (chunks + (1 << parts_log2) - 1) >> parts_log2;
     v_begin = min(part * per * kWave, num_vec);
     v_end = min(v_begin + per * kWave, num_vec);
 }
+
+// Vectors [v_begin, v_end) of a row, moved by one wave, kDepth KiB of it in flight: the first of them in `r` between
+// load() and store(), which moves the others too.
+template <int kDepth, bool kStream>
+struct RowPart {
+    u32x4 r[kDepth];
+    const uint8_t* src;
+    int bytes;
+    __device__ __forceinline__ void load(const uint8_t* row, int v_begin, int v_end, int lane) {
+        src = row + v_begin * 16, bytes = (v_end - v_begin) * 16;
+        const auto from = row_buffer(src, bytes);
+#pragma unroll
+        for (int u = 0; u < kDepth; ++u) r[u] = load_row_u32x4<kStream>(from, lane * 16 + u * 1024);
+    }
+    __device__ __forceinline__ void store(uint8_t* row, int v_begin, int lane) {
+        const auto from = row_buffer(src, bytes), to = row_buffer(row + v_begin * 16, bytes);
+        for (int base = lane * 16;;) {
+#pragma unroll
+            for (int u = 0; u < kDepth; ++u) store_row_u32x4<kStream>(to, base + u * 1024, r[u]);
+            base += kDepth * 1024;
+            if (base - lane * 16 >= bytes) return;
+#pragma unroll
+            for (int u = 0; u < kDepth; ++u) r[u] = load_row_u32x4<kStream>(from, base + u * 1024);
+        }
+    }
+};
 
 // Host-side choice of the row split (log2 of the parts): small problems cannot fill the chip with
 // one wave per row.
