@@ -105,13 +105,12 @@ __device__ __forceinline__ void emit_expert_count(int e, int total, int num_expe
 // expert (reference: the serial scan of csrc/kernels/efa_kernels.cu:617-637 and
 // token_offset / expert_offsets of csrc/kernels/coop_dispatch_send.cuh:360-420).
 // The workgroup counts them itself: while the row loads are in flight every
-// thread fetches up to four entries that precede the token (more in a loop);
-// each wave counts, per selection, its entries naming that selection's expert
-// with a ballot and a popcount, and wave 0 adds the waves' counts.  Up to 8192
+// thread fetches up to four entries that precede the token (more in a loop) and
+// adds them to a histogram by expert in LDS.  Up to 8192
 // entries the sweep covers every earlier entry; beyond, it covers the token's
 // own chunk of about 2048 entries and the chunks before it come from the
 // histograms of ll_chunk_hist_kernel.  The per-expert totals come from one extra
-// workgroup per source.  Deterministic: integer adds and ballots only.
+// workgroup per source.  Deterministic: integer adds only.
 // ---------------------------------------------------------------------
 constexpr int kMaxTopk = 64;
 constexpr int kFusedMaxEntries = 8192;     // send + receive in one launch up to here
@@ -159,10 +158,24 @@ struct DirectOut {
     int32_t* src_info;
 };
 
+// Top-k entries read two at a time, with zeros past the end of the list: 16-byte loads, which as buffer loads need no
+// more than the four-byte alignment that every list has.
+struct EntryPair {
+    u32x4 v;
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t list, int pair) { v = load_row_u32x4<false>(list, pair * 16); }
+    // Entry 0 or 1 as an expert below `limit` counted from `first`, if it names one.
+    __device__ __forceinline__ bool expert(int which, uint32_t first, uint32_t limit, uint32_t& e) const {
+        e = v[which * 2] - first;
+        return v[which * 2 + 1] == 0u && e < limit;
+    }
+};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t entry_list(const int64_t* topk_idx, int n) {
+    return row_buffer(reinterpret_cast<const uint8_t*>(topk_idx), n * 8);
+}
+
 struct alignas(16) SendLds {
-    int32_t wave_count[kMaxTopk][kSendMaxWaves];  // [k][wave]: the wave's earlier entries naming selection k's expert
-    uint64_t sel_row[kMaxTopk];                   // where selection k's payload goes (0: nowhere)
-    uint64_t sel_scale[kMaxTopk];                 // where its scales go
+    uint64_t sel_row[kMaxTopk];    // where selection k's payload goes (0: nowhere)
+    uint64_t sel_scale[kMaxTopk];  // where its scales go
 };
 
 // hist[e] (LDS, [E + 1]) = entries of topk_idx[0 .. n) naming expert e, clamped to max_tokens, then their
@@ -193,6 +206,25 @@ __device__ __forceinline__ void expert_prefix_in_lds(const int64_t* __restrict__
     }
     lds_barrier();
     block_exclusive_scan(hist, num_experts, wave_totals);
+}
+
+// For one wave: the rows of the experts before the lane's expert e (none: e < 0), an expert's entries -- the low half
+// of its word of hist (LDS) -- clamped to max_tokens.  Lane l adds up the l-th 64th of the experts.
+__device__ __forceinline__ int wave_expert_prefix(const int32_t* hist, int num_experts, int max_tokens, int e) {
+    const int per = (num_experts + kWave - 1) / kWave, lane = lane_id();
+    const auto rows_of = [&](int x) {
+        const int c = hist[x] & 0xffff;
+        return c < max_tokens ? c : max_tokens;
+    };
+    int sum = 0;
+    for (int j = 0; j < per; ++j)
+        if (lane * per + j < num_experts) sum += rows_of(lane * per + j);
+    const int base = wave_inclusive_sum(sum) - sum;
+    const int owner = e < 0 ? 0 : e / per;
+    int run = __shfl(base, owner, kWave);
+    for (int j = 0; j < per; ++j)
+        if (owner * per + j < e) run += rows_of(owner * per + j);
+    return run;
 }
 
 // The per-rank tables of the by-destination form from the prefix in LDS.
@@ -244,8 +276,7 @@ __device__ __forceinline__ void send_count_block(const SendArgs& a, int b, int32
 // scales and tails stored, the ordinary way: the hint measured slower on those (63 and 56 us).
 template <int kFmt, bool kStream>
 __device__ __forceinline__ void send_token_block(const SendArgs& a, const DirectOut& direct, int b, int t,
-                                                 int block_in_token, SendLds& lds, int32_t* lds_hist,
-                                                 int32_t* lds_wave_totals) {
+                                                 int block_in_token, SendLds& lds, int32_t* lds_hist) {
     const int lane = lane_id(), tid = threadIdx.x;
     const int num_topk = a.num_topk, num_experts = a.num_experts;
     const int n = a.num_tokens * num_topk;
@@ -268,39 +299,37 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
 
     DEEPEP_PHASE(0);
     // ---- issue this wave's row loads ------------------------------------
-    u32x4 lo = {0u, 0u, 0u, 0u}, hi = {0u, 0u, 0u, 0u};
-    bool lane_live;
+    const auto token_row = row_buffer(a.x + uint64_t(row_id) * (uint32_t(a.hidden) * 2), a.hidden * 2);
+    u32x4 lo, hi = {0u, 0u, 0u, 0u};  // zeros past the row's end
+    bool lane_live = wave_live;
     int group = 0;
     if constexpr (kFmt == kRowBF16) {
-        const int64_t off = int64_t(piece) * 1024 + lane * 16;
-        lane_live = wave_live && off < data_bytes;
-        if (lane_live) lo = load_u32x4<false>(a.x + row_id * data_bytes + off);
+        lo = load_row_u32x4<false>(token_row, piece * 1024 + lane * 16);
     } else {
         group = piece * 8 + (lane >> 3);
         lane_live = wave_live && group < a.hidden / kGroup;
-        if (lane_live) {
-            const uint8_t* src = a.x + (row_id * a.hidden + int64_t(group) * kGroup + (lane & 7) * 16) * 2;
-            lo = load_u32x4<false>(src);
-            hi = load_u32x4<false>(src + 16);
-        }
+        lo = load_row_u32x4<false>(token_row, piece * 2048 + lane * 32);
+        hi = load_row_u32x4<false>(token_row, piece * 2048 + lane * 32 + 16);
     }
 
     // ---- every index load of the ranking, issued before anything waits -----
     // The loads are unconditional (an index that is not wanted is clamped to one that exists and its
     // value dropped): without branches around them the compiler can count them, so the first wait of
     // wave 0 -- for the token's own selections -- does not also wait out a second round trip for the
-    // entries it sweeps.  The wave then has one memory round trip in front of its ballots, not two.
+    // entries it sweeps.
+    const int threads = blockDim.x;
     const int chunk = a.tokens_per_chunk > 0 ? t / a.tokens_per_chunk : 0;
     const int sweep_begin = chunk * a.tokens_per_chunk * num_topk;
-    constexpr int kSweepAhead = 4;
-    const int64_t own_v = my_topk[entry0 + (tid < num_topk ? tid : num_topk - 1)];     // threads 0..K-1: selection tid
-    const int64_t sel_v = my_topk[entry0 + (lane < num_topk ? lane : num_topk - 1)];   // lane k of every wave: selection k
-    int64_t ahead_v[kSweepAhead];
+    const int sweep_end = a.prefix_in_block ? n : entry0;
+    constexpr int kSweepAhead = 2;
+    const int64_t own_v = my_topk[entry0 + (tid < num_topk ? tid : num_topk - 1)];  // threads 0..K-1: selection tid
+    const auto list = entry_list(my_topk + sweep_begin, n - sweep_begin);
+    const int sweep_pairs = (sweep_end - sweep_begin + 1) >> 1;
+    EntryPair ahead[kSweepAhead];
 #pragma unroll
-    for (int r = 0; r < kSweepAhead; ++r) {
-        const int i = sweep_begin + tid + r * int(blockDim.x);
-        ahead_v[r] = my_topk[i < entry0 ? i : entry0];
-    }
+    for (int r = 0; r < kSweepAhead; ++r) ahead[r].load(list, tid + r * threads);
+    for (int e = tid; e < num_experts; e += threads) lds_hist[e] = 0;
+    lds_barrier();
 
     // ---- per-selection bookkeeping, once per token --------------------------
     int my_expert = -1, my_slot = -1, dst_rank = -1, local = 0;  // threads 0..K-1: selection k = tid
@@ -316,12 +345,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
         }
     }
     int dest_first = 0;  // by-destination form: where the expert's run of rows begins in the send buffer
-    if (a.prefix_in_block) {
-        expert_prefix_in_lds(my_topk, n, num_experts, a.max_tokens, lds_hist, lds_wave_totals, nullptr);
-        if (my_expert >= 0) dest_first = lds_hist[my_expert];
-    } else if (a.expert_prefix != nullptr && my_expert >= 0) {
-        dest_first = a.expert_prefix[my_expert];
-    }
+    if (a.expert_prefix != nullptr && !a.prefix_in_block && my_expert >= 0) dest_first = a.expert_prefix[my_expert];
     if (direct.packed_x != nullptr && tid < kWave) {
         // Rows for this rank's own experts go straight to the packed tensors, at the place the
         // reference's range builder gives them: behind the rows of the lower source ranks
@@ -357,61 +381,38 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     DEEPEP_PHASE(1);
     u32x4 payload = lo;  // quantised below, while the workgroup's bookkeeping is in flight
     uint32_t scale_bits = 0;
-    // Rank the selections.  Each thread takes every blockDim-th entry between the start of the sweep
-    // and this token (four fetched up front, so their latency overlaps the loads above); each wave
-    // counts, per selection, how many of its entries name that selection's expert (a ballot and a
-    // popcount, against the token's own entries read as wave-uniform values) and leaves the counts
-    // in LDS.
-    int ahead[kSweepAhead];  // -1: no entry
+    // Rank the selections: the entries between the start of the sweep and this token, counted by expert in LDS.  (A
+    // ballot for each selection and load instead cost every wave of the workgroup 130 instructions a round of four
+    // entries a thread: 128 tokens 7.7 -> 7.4 us, 300 tokens 15.9 -> 15.4, single entries read instead of pairs 16.1.)
+    // The by-destination form sweeps the whole batch: the low half of a word counts all entries, the high half those
+    // before the token, and wave 0 gets the experts' prefix from the same words (128 tokens 9.4 -> 7.8 us against a
+    // histogram of its own and a scan by the whole workgroup).
+    const auto count_pair = [&](int pair, const EntryPair& entries) {
+        if (pair >= sweep_pairs) return;
 #pragma unroll
-    for (int r = 0; r < kSweepAhead; ++r) {
-        const int i = sweep_begin + tid + r * int(blockDim.x);
-        const int64_t v = ahead_v[r];
-        ahead[r] = i < entry0 && v >= 0 && v < num_experts ? int(v) : -1;
-    }
-    // lane k of every wave holds the token's selection k (-2: none, matches no entry)
-    int sel = -2;
-    if (lane < num_topk && sel_v >= 0 && sel_v < num_experts) sel = int(sel_v);
-    const int w = wave_in_block();
-    int my_count = 0;  // lane k: this wave's entries naming selection k's expert
-    for (int k = 0; k < num_topk; ++k) {
-        const int e = __builtin_amdgcn_readlane(sel, k);
-        int count = 0;
-#pragma unroll
-        for (int r = 0; r < kSweepAhead; ++r) count += __popcll(__ballot(ahead[r] == e));
-        if (lane == k) my_count = count;
-    }
-    for (int base = sweep_begin + kSweepAhead * int(blockDim.x); base < entry0;
-         base += kSweepAhead * int(blockDim.x)) {
-        int more[kSweepAhead];  // the same again, four loads in flight per thread
-#pragma unroll
-        for (int r = 0; r < kSweepAhead; ++r) {
-            const int i = base + tid + r * int(blockDim.x);
-            const int64_t v = i < entry0 ? my_topk[i] : -1;
-            more[r] = v >= 0 && v < num_experts ? int(v) : -1;
+        for (int i = 0; i < 2; ++i) {
+            const int at = sweep_begin + pair * 2 + i;
+            uint32_t e;
+            if (entries.expert(i, 0, uint32_t(num_experts), e) && at < sweep_end)
+                atomicAdd(&lds_hist[e], a.prefix_in_block && at < entry0 ? 0x10001 : 1);
         }
-        for (int k = 0; k < num_topk; ++k) {
-            const int e = __builtin_amdgcn_readlane(sel, k);
-            int count = 0;
+    };
 #pragma unroll
-            for (int r = 0; r < kSweepAhead; ++r) count += __popcll(__ballot(more[r] == e));
-            if (lane == k) my_count += count;
-        }
+    for (int r = 0; r < kSweepAhead; ++r) count_pair(tid + r * threads, ahead[r]);
+    for (int base = kSweepAhead * threads; base < sweep_pairs; base += kSweepAhead * threads) {
+#pragma unroll
+        for (int r = 0; r < kSweepAhead; ++r) ahead[r].load(list, base + tid + r * threads);
+#pragma unroll
+        for (int r = 0; r < kSweepAhead; ++r) count_pair(base + tid + r * threads, ahead[r]);
     }
-    if (lane < num_topk) lds.wave_count[lane][w] = my_count;
     if constexpr (kFmt != kRowBF16) payload = quantise_16<kFmt>(lo, hi, scale_bits);
     lds_barrier();
     DEEPEP_PHASE(3);
     if (tid < kWave) {  // wave 0: lane k finishes selection k
-        const int waves = int(blockDim.x) >> 6;
-        int total = 0;
-        if (tid < num_topk) {  // one wide read of the row; entries of absent waves are never summed
-            static_assert(kSendMaxWaves == 16, "four 16-byte LDS reads");
-            u32x4 c[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) c[q] = reinterpret_cast<const u32x4*>(lds.wave_count[tid])[q];
-#pragma unroll
-            for (int w2 = 0; w2 < kSendMaxWaves; ++w2) total += w2 < waves ? int(c[w2 >> 2][w2 & 3]) : 0;
+        int total = my_expert >= 0 ? lds_hist[my_expert] : 0;
+        if (a.prefix_in_block) {
+            total = int(uint32_t(total) >> 16);
+            dest_first = wave_expert_prefix(lds_hist, num_experts, a.max_tokens, my_expert);
         }
         for (int k2 = 0; k2 < num_topk; ++k2) {  // the same expert named earlier in this token
             const int other = __builtin_amdgcn_readlane(my_expert, k2);
@@ -457,7 +458,10 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     if (!wave_live) return;
 
     // ---- one store per selection ----------------------------------------
-    const int64_t lane_off = int64_t(piece) * 1024 + lane * 16;
+    // Rows are addressed as buffers: lanes past a row's end and, with the scales, all but the first of eight store
+    // nothing without a mask of their own.
+    const int lane_off = piece * 1024 + lane * 16;
+    const int scale_off = lane_live && (lane & 7) == 0 ? (kFmt == kRowFP8UE8M0 ? group : group * 4) : 0x7fffffff;
     DEEPEP_PHASE(5);
     // lane k reads selection k's destinations once; the loop takes them back as wave-uniform values
     uint64_t my_row = 0, my_scale_row = 0;
@@ -466,20 +470,20 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
         my_scale_row = lds.sel_scale[lane];
     }
     for (int k = part; k < num_topk; k += split) {
-        uint8_t* row = reinterpret_cast<uint8_t*>(
+        const uint8_t* row = reinterpret_cast<const uint8_t*>(
             (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_row >> 32), k))) << 32) |
             uint32_t(__builtin_amdgcn_readlane(int(uint32_t(my_row)), k)));
         if (row == nullptr) continue;
-        if (lane_live) store_u32x4<kStream>(row + lane_off, payload);
+        store_row_u32x4<kStream>(row_buffer(row, int(data_bytes)), lane_off, payload);
         if constexpr (kFmt != kRowBF16) {
-            uint8_t* scale_row = reinterpret_cast<uint8_t*>(
+            const uint8_t* scale_row = reinterpret_cast<const uint8_t*>(
                 (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_scale_row >> 32), k))) << 32) |
                 uint32_t(__builtin_amdgcn_readlane(int(uint32_t(my_scale_row)), k)));
-            if constexpr (kFmt == kRowFP8UE8M0) {
-                if (lane_live && (lane & 7) == 0) store_global_byte(scale_row + group, uint8_t(scale_bits >> 23));
-            } else {
-                if (lane_live && (lane & 7) == 0) store_global(scale_row + int64_t(group) * 4, scale_bits);
-            }
+            const auto scales = row_buffer(scale_row, int(scale_bytes));
+            if constexpr (kFmt == kRowFP8UE8M0)
+                __builtin_amdgcn_raw_buffer_store_b8(uint8_t(scale_bits >> 23), scales, scale_off, 0, 0);
+            else
+                __builtin_amdgcn_raw_buffer_store_b32(scale_bits, scales, scale_off, 0, 0);
         }
     }
     DEEPEP_PHASE(6);
@@ -513,7 +517,7 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_send_kernel(SendArgs 
         }  // else: ll_by_dest_prefix_kernel ran first
         return;
     }
-    send_token_block<kFmt, kStream>(a, direct, blockIdx.z, y, blockIdx.x, lds, lds_hist, index_wave_totals);
+    send_token_block<kFmt, kStream>(a, direct, blockIdx.z, y, blockIdx.x, lds, lds_hist);
 }
 
 // ---------------------------------------------------------------------
@@ -556,21 +560,19 @@ __device__ __forceinline__ int clamp_count(int c, int max_tokens) {
 // own_cnt[e_l] (LDS, unclamped) = rows this rank sends to its own expert e_l, counted by the whole
 // workgroup in two steps so that other loads can be issued in between: `begin` issues the first index
 // loads and clears the counters, `finish` counts and ends with a barrier.
-constexpr int kOwnAhead = 4;  // index loads in flight per thread
+constexpr int kOwnAhead = 4;  // index loads in flight per thread, two entries each
 
 struct OwnCountLoads {
-    int64_t v[kOwnAhead];
+    EntryPair v[kOwnAhead];
 };
 
 __device__ __forceinline__ void own_row_counts_begin(const RecvArgs& a, const int64_t* own_topk, int own_entries,
                                                      int32_t* own_cnt, OwnCountLoads& loads) {
     const int tid = threadIdx.x, threads = blockDim.x;
     if (own_topk == nullptr) return;
+    const auto list = entry_list(own_topk, own_entries);
 #pragma unroll
-    for (int r = 0; r < kOwnAhead; ++r) {
-        const int i = tid + r * threads;
-        loads.v[r] = i < own_entries ? own_topk[i] : -1;
-    }
+    for (int r = 0; r < kOwnAhead; ++r) loads.v[r].load(list, tid + r * threads);
     for (int le = tid; le < a.num_local_experts; le += threads) own_cnt[le] = 0;
     lds_barrier();
 }
@@ -584,20 +586,22 @@ __device__ __forceinline__ void own_row_counts_finish(const RecvArgs& a, const i
         lds_barrier();
         return;
     }
-    const int64_t first = int64_t(own_rank) * a.num_local_experts;
-    for (int base = 0; base < own_entries; base += kOwnAhead * threads) {
-        int64_t next[kOwnAhead];
+    const auto list = entry_list(own_topk, own_entries);
+    const uint32_t first = uint32_t(own_rank) * a.num_local_experts;
+    for (int base = 0;;) {
 #pragma unroll
-        for (int r = 0; r < kOwnAhead; ++r) {
-            const int i = base + (kOwnAhead + r) * threads + tid;
-            next[r] = i < own_entries ? own_topk[i] : -1;
-        }
+        for (int r = 0; r < kOwnAhead; ++r)
 #pragma unroll
-        for (int r = 0; r < kOwnAhead; ++r) {
-            const int64_t d = loads.v[r] - first;
-            if (loads.v[r] >= 0 && d >= 0 && d < a.num_local_experts) atomicAdd(&own_cnt[int(d)], 1);
-            loads.v[r] = next[r];
-        }
+            for (int i = 0; i < 2; ++i) {
+                uint32_t le;
+                if (loads.v[r].expert(i, first, uint32_t(a.num_local_experts), le) &&
+                    (base + tid + r * threads) * 2 + i < own_entries)
+                    atomicAdd(&own_cnt[le], 1);
+            }
+        base += kOwnAhead * threads;
+        if (base * 2 >= own_entries) break;
+#pragma unroll
+        for (int r = 0; r < kOwnAhead; ++r) loads.v[r].load(list, base + tid + r * threads);
     }
     lds_barrier();
 }
@@ -789,8 +793,7 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_dispatch_fused_kernel
     const int block = blockIdx.x;
     if (block < num_send_blocks) {
         const DirectOut direct = {ra.packed_x, ra.packed_scales, ra.src_info};
-        send_token_block<kFmt, kStream>(sa, direct, 0, block / blocks_per_token, block % blocks_per_token, lds, dyn_lds,
-                                        wave_totals);
+        send_token_block<kFmt, kStream>(sa, direct, 0, block / blocks_per_token, block % blocks_per_token, lds, dyn_lds);
     } else if (block == num_send_blocks) {
         send_count_block(sa, 0, dyn_lds);
     } else {

@@ -138,6 +138,7 @@ def check_dispatch(st, want, fmt):
     (128, 77, 9, 512, 4, 128),   # many ranks, one expert each
     (256, 3, 5, 512, 2, 512),
     (512, 500, 3, 512, 2, 1024),  # the widest world the path takes
+    (3, 1, 801, 512, 5, 9),    # odd entries a token and in all: the sweeps read them in pairs; 9 segments, not whole vectors
 ])
 @ONE_CALL
 def test_dispatch_small_worlds(rt, fmt, r, rank, t, h, k, e, one_call):
@@ -1084,6 +1085,8 @@ def check_send_by_dest(st, want, t):
     (512, 500, 3, 512, 2, 1024),
     (4, 3, 256, 512, 8, 32),     # 2048 entries: the last batch whose tables are built inside the send launch
     (4, 3, 257, 512, 8, 32),     # 2056 entries: the first with a launch for them
+    (32, 7, 77, 512, 6, 288),    # five experts a lane, the last lanes without any; an odd number of entries before tokens
+    (3, 2, 67, 512, 5, 195),     # as many experts as no lane's share divides, tokens of an odd number of entries
 ])
 def test_send_by_dest(rt, fmt, r, rank, t, h, k, e):
     """One buffer, contiguous per destination rank, rows by expert and slot; counts, prefixes and every
