@@ -186,7 +186,7 @@ SORT_FORMS = [(0, 8), (0, 9), (0, 72), (1, 9), (300, 24), (131, 16), (5000, 16),
               (70000, 8), (3000, 72), (1, 130)]
 # either side of the lines between them, and every width of a token's row in words
 SORT_FORMS += [(2559, 8), (2560, 8), (4095, 16), (4096, 16), (4096, 24), (13107, 40), (13108, 40), (10922, 48),
-               (10923, 48), (4097, 56), (16385, 32)]
+               (10923, 48), (4097, 56), (16385, 32), (512, 16), (513, 16), (511, 64), (257, 5)]
 
 
 @pytest.mark.parametrize("t,r", SORT_FORMS)
