@@ -12,10 +12,11 @@ namespace deepep {
 constexpr int kExchangeThreads = 1024;
 constexpr int kExchangeMaxRanks = 1024;
 
-__device__ __forceinline__ int64_t wave_sum_i64(int64_t v) {
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) v += __shfl_xor(v, d, kWave);
-    return v;
+// Sum over the wave of 64-bit values below 2^48, in two parts whose sums fit 32 bits (DPP, no LDS).
+__device__ __forceinline__ int64_t wave_sum_u48(int64_t v) {
+    const uint32_t low = __builtin_amdgcn_readlane(wave_inclusive_sum(int(v & 0xffffff)), kWave - 1);
+    const uint32_t high = __builtin_amdgcn_readlane(wave_inclusive_sum(int(v >> 24)), kWave - 1);
+    return (int64_t(high) << 24) + low;
 }
 
 // Every workgroup derives the per-rank tables itself (the R x E counts once, from L2: one wave per
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(kExchangeThreads) void ll_exchange_meta_kernel(
                 else if (e < first_expert + experts_per_rank) to_me += int(v[u]);
             }
         }
-        below = wave_sum_i64(below);
+        below = wave_sum_u48(below);
         to_me = __builtin_amdgcn_readlane(wave_inclusive_sum(to_me), kWave - 1);
         if (lane == 0) below_of[r] = below, recv_of[r] = to_me;
     }
