@@ -33,7 +33,6 @@ namespace deepep {
 
 __host__ __device__ inline int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
-constexpr int kByDestInBlockEntries = 2048;  // by-destination batches up to here build their tables in the send launch
 constexpr int kSweepChunkEntries = 2048;  // a token sweeps at most this many earlier entries itself
 
 // Tokens per sweep chunk: whole tokens, about kSweepChunkEntries entries.
@@ -73,6 +72,19 @@ __global__ __launch_bounds__(1024) void ll_chunk_hist_kernel(const int64_t* __re
     }
     lds_barrier();
     for (int e = tid; e < num_experts; e += blockDim.x) out[e] = hist_lds[e];
+}
+
+// Entries that name expert e, from the chunk histograms.
+__device__ __forceinline__ int chunk_total(const int32_t* __restrict__ hists, int num_chunks, int num_experts, int e) {
+    int total = 0;
+    for (int c0 = 0; c0 < num_chunks; c0 += 8) {  // eight loads in flight
+        int v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = c0 + u < num_chunks ? hists[int64_t(c0 + u) * num_experts + e] : 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) total += v[u];
+    }
+    return total;
 }
 
 // Writes the per-expert totals where the receivers look for them.
@@ -141,9 +153,8 @@ struct SendArgs {
     // By-destination form: send_slots is one buffer of rows, contiguous per destination rank, and every
     // row (the rank's own included) goes to row expert_prefix[expert] + slot of it.  Null: per-expert slots.
     const int32_t* expert_prefix;
-    // Small by-destination batches: no launch builds the tables first.  Every token's workgroup counts
-    // the batch's entries per expert itself and scans them in LDS (a few barriers beside its row loads,
-    // cheaper than a launch), and the counting row writes the tables out.
+    // By-destination batches for which no launch builds the tables first: every token's workgroup gets
+    // the batch's entries per expert itself, and the counting row writes the tables out.
     int prefix_in_block;
     ByDestTables by_dest;
 };
@@ -180,29 +191,37 @@ struct alignas(16) SendLds {
 
 // hist[e] (LDS, [E + 1]) = entries of topk_idx[0 .. n) naming expert e, clamped to max_tokens, then their
 // exclusive prefix over the experts with the total in hist[E]; the whole workgroup takes part.
-// counts_out (may be null): the clamped counts.
+// chunk_hist (may be null): the chunk histograms to take the entries from.  counts_out: the clamped counts.
 __device__ __forceinline__ void expert_prefix_in_lds(const int64_t* __restrict__ topk_idx, int n, int num_experts,
-                                                     int max_tokens, int32_t* hist, int32_t* wave_totals,
+                                                     int max_tokens, const int32_t* __restrict__ chunk_hist,
+                                                     int num_chunks, int32_t* hist, int32_t* wave_totals,
                                                      int32_t* counts_out) {
     const int tid = threadIdx.x, threads = blockDim.x;
-    for (int e = tid; e < num_experts; e += threads) hist[e] = 0;
-    lds_barrier();
-    for (int base = 0; base < n; base += 4 * threads) {  // four loads in flight per thread
-        int64_t v[4];
+    if (chunk_hist == nullptr) {
+        for (int e = tid; e < num_experts; e += threads) hist[e] = 0;
+        lds_barrier();
+        constexpr int kAhead = 4;  // pairs of entries in flight per thread
+        const auto list = entry_list(topk_idx, n);
+        for (int base = tid; base * 2 < n; base += kAhead * threads) {
+            EntryPair ahead[kAhead];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = base + u * threads + tid;
-            v[u] = i < n ? topk_idx[i] : -1;
+            for (int u = 0; u < kAhead; ++u) ahead[u].load(list, base + u * threads);
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    uint32_t e;
+                    if (ahead[u].expert(i, 0, uint32_t(num_experts), e) && (base + u * threads) * 2 + i < n)
+                        atomicAdd(&hist[e], 1);
+                }
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (v[u] >= 0 && v[u] < num_experts) atomicAdd(&hist[int(v[u])], 1);
+        lds_barrier();
     }
-    lds_barrier();
     for (int e = tid; e < num_experts; e += threads) {
-        const int c = hist[e] < max_tokens ? hist[e] : max_tokens;
+        const int total = chunk_hist != nullptr ? chunk_total(chunk_hist, num_chunks, num_experts, e) : hist[e];
+        const int c = total < max_tokens ? total : max_tokens;
         hist[e] = c;
-        if (counts_out != nullptr) counts_out[e] = c;
+        counts_out[e] = c;
     }
     lds_barrier();
     block_exclusive_scan(hist, num_experts, wave_totals);
@@ -250,8 +269,7 @@ __device__ __forceinline__ void send_count_block(const SendArgs& a, int b, int32
         const int32_t* hist = reinterpret_cast<const int32_t*>(a.scratch_base + int64_t(b) * a.scratch_stride);
         const int chunks = (a.num_tokens + a.tokens_per_chunk - 1) / a.tokens_per_chunk;
         for (int e = tid; e < a.num_experts; e += blockDim.x) {
-            int total = 0;
-            for (int c = 0; c < chunks; ++c) total += hist[int64_t(c) * a.num_experts + e];
+            const int total = chunk_total(hist, chunks, a.num_experts, e);
             emit_expert_count(e, total, a.num_experts, a.num_ranks, a.rank, src_rank, a.max_tokens, a.recv_count,
                               a.send_count);
         }
@@ -274,7 +292,8 @@ __device__ __forceinline__ void send_count_block(const SendArgs& a, int b, int32
 // destinations in HBM, that takes the send from 73 to 53 us (a row stored the ordinary way is first
 // allocated in the memory-side cache and written back later).  The token rows are read, and the
 // scales and tails stored, the ordinary way: the hint measured slower on those (63 and 56 us).
-template <int kFmt, bool kStream>
+// kTables: the launch may be one that makes the by-destination tables.
+template <int kFmt, bool kStream, bool kTables>
 __device__ __forceinline__ void send_token_block(const SendArgs& a, const DirectOut& direct, int b, int t,
                                                  int block_in_token, SendLds& lds, int32_t* lds_hist) {
     const int lane = lane_id(), tid = threadIdx.x;
@@ -320,7 +339,9 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     const int threads = blockDim.x;
     const int chunk = a.tokens_per_chunk > 0 ? t / a.tokens_per_chunk : 0;
     const int sweep_begin = chunk * a.tokens_per_chunk * num_topk;
-    const int sweep_end = a.prefix_in_block ? n : entry0;
+    const bool prefix_in_block = kTables && a.prefix_in_block;
+    const bool count_all = prefix_in_block && a.tokens_per_chunk == 0;
+    const int sweep_end = count_all ? n : entry0;
     constexpr int kSweepAhead = 2;
     const int64_t own_v = my_topk[entry0 + (tid < num_topk ? tid : num_topk - 1)];  // threads 0..K-1: selection tid
     const auto list = entry_list(my_topk + sweep_begin, n - sweep_begin);
@@ -345,7 +366,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
         }
     }
     int dest_first = 0;  // by-destination form: where the expert's run of rows begins in the send buffer
-    if (a.expert_prefix != nullptr && !a.prefix_in_block && my_expert >= 0) dest_first = a.expert_prefix[my_expert];
+    if (a.expert_prefix != nullptr && !prefix_in_block && my_expert >= 0) dest_first = a.expert_prefix[my_expert];
     if (direct.packed_x != nullptr && tid < kWave) {
         // Rows for this rank's own experts go straight to the packed tensors, at the place the
         // reference's range builder gives them: behind the rows of the lower source ranks
@@ -384,9 +405,17 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     // Rank the selections: the entries between the start of the sweep and this token, counted by expert in LDS.  (A
     // ballot for each selection and load instead cost every wave of the workgroup 130 instructions a round of four
     // entries a thread: 128 tokens 7.7 -> 7.4 us, 300 tokens 15.9 -> 15.4, single entries read instead of pairs 16.1.)
-    // The by-destination form sweeps the whole batch: the low half of a word counts all entries, the high half those
-    // before the token, and wave 0 gets the experts' prefix from the same words (128 tokens 9.4 -> 7.8 us against a
-    // histogram of its own and a scan by the whole workgroup).
+    // With prefix_in_block the low half of a word counts all of the batch's entries and the high half those before
+    // the token, and wave 0 gets the prefix from the same words (128 tokens 9.4 -> 7.8 us against a histogram of its
+    // own and a scan by the whole workgroup).  The sweep then goes through the whole batch, or, where there are chunk
+    // histograms, through the token's chunk as ever, and their column sums make the low halves.
+    const int before = prefix_in_block ? (count_all ? 0x10001 : 0x10000) : 1;
+    if (prefix_in_block && !count_all) {
+        const int32_t* hist = reinterpret_cast<const int32_t*>(a.scratch_base);
+        const int chunks = (a.num_tokens + a.tokens_per_chunk - 1) / a.tokens_per_chunk;
+        for (int e = tid; e < num_experts; e += threads)
+            atomicAdd(&lds_hist[e], chunk_total(hist, chunks, num_experts, e));
+    }
     const auto count_pair = [&](int pair, const EntryPair& entries) {
         if (pair >= sweep_pairs) return;
 #pragma unroll
@@ -394,7 +423,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
             const int at = sweep_begin + pair * 2 + i;
             uint32_t e;
             if (entries.expert(i, 0, uint32_t(num_experts), e) && at < sweep_end)
-                atomicAdd(&lds_hist[e], a.prefix_in_block && at < entry0 ? 0x10001 : 1);
+                atomicAdd(&lds_hist[e], at < entry0 ? before : 1);
         }
     };
 #pragma unroll
@@ -410,7 +439,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     DEEPEP_PHASE(3);
     if (tid < kWave) {  // wave 0: lane k finishes selection k
         int total = my_expert >= 0 ? lds_hist[my_expert] : 0;
-        if (a.prefix_in_block) {
+        if (prefix_in_block) {
             total = int(uint32_t(total) >> 16);
             dest_first = wave_expert_prefix(lds_hist, num_experts, a.max_tokens, my_expert);
         }
@@ -508,16 +537,18 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_send_kernel(SendArgs 
     }
     if (y == a.num_tokens) {  // the counting row of the grid
         if (blockIdx.x != 0) return;
-        if (a.prefix_in_block) {  // small by-destination batch: this workgroup writes the tables out
-            expert_prefix_in_lds(a.topk_idx, a.num_tokens * a.num_topk, a.num_experts, a.max_tokens, lds_hist,
-                                 index_wave_totals, a.send_count);
+        if (a.prefix_in_block) {  // this workgroup writes the tables out
+            const int tpc = a.tokens_per_chunk;
+            expert_prefix_in_lds(a.topk_idx, a.num_tokens * a.num_topk, a.num_experts, a.max_tokens,
+                                 tpc > 0 ? reinterpret_cast<const int32_t*>(a.scratch_base) : nullptr,
+                                 tpc > 0 ? (a.num_tokens + tpc - 1) / tpc : 0, lds_hist, index_wave_totals, a.send_count);
             by_dest_tables_out(lds_hist, a.num_experts, a.num_ranks, a.by_dest);
         } else if (a.expert_prefix == nullptr) {
             send_count_block(a, blockIdx.z, lds_hist);
         }  // else: ll_by_dest_prefix_kernel ran first
         return;
     }
-    send_token_block<kFmt, kStream>(a, direct, blockIdx.z, y, blockIdx.x, lds, lds_hist);
+    send_token_block<kFmt, kStream, true>(a, direct, blockIdx.z, y, blockIdx.x, lds, lds_hist);
 }
 
 // ---------------------------------------------------------------------
@@ -793,7 +824,8 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_dispatch_fused_kernel
     const int block = blockIdx.x;
     if (block < num_send_blocks) {
         const DirectOut direct = {ra.packed_x, ra.packed_scales, ra.src_info};
-        send_token_block<kFmt, kStream>(sa, direct, 0, block / blocks_per_token, block % blocks_per_token, lds, dyn_lds);
+        send_token_block<kFmt, kStream, false>(sa, direct, 0, block / blocks_per_token, block % blocks_per_token, lds,
+                                               dyn_lds);
     } else if (block == num_send_blocks) {
         send_count_block(sa, 0, dyn_lds);
     } else {
@@ -804,13 +836,12 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_dispatch_fused_kernel
 
 // ---------------------------------------------------------------------
 // By-destination send (what an all-to-all ships: one contiguous message per
-// peer).  Before the send kernel runs (batches of more than kByDestInBlockEntries entries;
-// smaller ones build the same tables inside the send launch, every token's workgroup
-// for itself), one workgroup turns the route counts into
-// the tables the rows are placed by: send_count[e] (clamped to the M slots of a
-// pair), its exclusive prefix over the experts -- the first row of every expert's
-// run, experts ascending, hence destination ranks ascending -- and the per-rank
-// counts and prefix the transport cuts the buffer by.
+// peer).  The rows are placed by tables made of the route counts: send_count[e]
+// (clamped to the M slots of a pair), its exclusive prefix over the experts --
+// the first row of every expert's run, experts ascending, hence destination ranks
+// ascending -- and the per-rank counts and prefix the transport cuts the buffer
+// by.  Batches that by_dest_tables_in_send() leaves to it get them from this one
+// workgroup before the send kernel runs.
 // Reference: the count + prefix phases of ll_dispatch_route_and_pack_v3
 // (csrc/kernels/efa_kernels.cu:2358-2371: ll_dispatch_count_kernel, prefix_sum_kernel).
 // ---------------------------------------------------------------------
@@ -820,43 +851,25 @@ __global__ __launch_bounds__(1024) void ll_by_dest_prefix_kernel(const int64_t* 
                                                                  int32_t* __restrict__ send_count, ByDestTables out) {
     extern __shared__ int32_t hist[];  // [E + 1]
     __shared__ int32_t wave_totals[kMaxBlockWaves];
-    const int tid = threadIdx.x, threads = blockDim.x;
-    if (chunk_hist != nullptr) {  // the column sums of the chunk histograms
-        for (int e = tid; e < num_experts; e += threads) {
-            int total = 0;
-            for (int c0 = 0; c0 < num_chunks; c0 += 8) {  // eight loads in flight
-                int v[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) v[u] = c0 + u < num_chunks ? chunk_hist[int64_t(c0 + u) * num_experts + e] : 0;
-#pragma unroll
-                for (int u = 0; u < 8; ++u) total += v[u];
-            }
-            hist[e] = total;
-        }
-    } else {
-        for (int e = tid; e < num_experts; e += threads) hist[e] = 0;
-        lds_barrier();
-        for (int base = 0; base < n; base += 4 * threads) {  // four loads in flight per thread
-            int64_t v[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i = base + u * threads + tid;
-                v[u] = i < n ? topk_idx[i] : -1;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (v[u] >= 0 && v[u] < num_experts) atomicAdd(&hist[int(v[u])], 1);
-        }
-    }
-    lds_barrier();
-    for (int e = tid; e < num_experts; e += threads) {
-        const int c = hist[e] < max_tokens ? hist[e] : max_tokens;
-        hist[e] = c;
-        send_count[e] = c;
-    }
-    lds_barrier();
-    block_exclusive_scan(hist, num_experts, wave_totals);
+    expert_prefix_in_lds(topk_idx, n, num_experts, max_tokens, chunk_hist, num_chunks, hist, wave_totals, send_count);
     by_dest_tables_out(hist, num_experts, num_ranks, out);
+}
+
+// Whether the send launch makes the by-destination tables, every token's workgroup for itself, instead of a launch before
+// it.  Without chunk histograms (chunks 0: up to 8192 entries) each workgroup goes through the whole batch instead of half
+// of it, and one wave through the experts: up to 1024 experts that costs less than the launch, past them only for batches
+// of up to 2048 entries.  With histograms it adds up their columns, which pays up to 2048 words.  Microseconds of the send
+// with the tables made by itself against the launch before it, top-8, fp8:
+//   300 tokens, 64 experts, hidden 7168      10.7 / 13.5        2047 tokens,  64 experts ( 512 words)  15.5 / 17.5
+//   1024 tokens, 64 experts, hidden 7168     18.2 / 19.5        8000 tokens,  64 experts (2048 words)  24.3 / 25.5
+//   300 tokens, 256 experts, hidden 2048      6.0 /  8.6        2047 tokens, 256 experts (2048 words)  16.7 / 17.7
+//   1000 tokens, 1024 experts, hidden 2048   12.1 / 14.3        2047 tokens, 512 experts (4096 words)  18.0 / 18.0
+//   1000 tokens, 4096 experts, hidden 2048   20.1 / 15.3        4000 tokens, 256 experts (4096 words)  24.2 / 23.8
+// Both counts of an expert share a 32-bit word: fewer than 2^16 entries.
+constexpr int kByDestInBlockExperts = 1024, kByDestInBlockEntries = 2048, kByDestInBlockWords = 2048;
+static bool by_dest_tables_in_send(int n, int num_experts, int chunks) {
+    if (chunks == 0) return num_experts <= kByDestInBlockExperts || n <= kByDestInBlockEntries;
+    return n < 65536 && int64_t(chunks) * num_experts <= kByDestInBlockWords;
 }
 
 // ---------------------------------------------------------------------
@@ -892,18 +905,15 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     // How slots get ranked: up to kSelfRankMaxEntries entries the send kernel sweeps every earlier
     // entry itself; beyond, it sweeps its own chunk on top of the per-chunk histograms.
     const int tpc = n <= kSelfRankMaxEntries || fused_recv != nullptr ? 0 : sweep_chunk_tokens(num_topk);
+    const int chunks = tpc > 0 ? (num_tokens + tpc - 1) / tpc : 0;
     if (tpc > 0) {
-        const int chunks = (num_tokens + tpc - 1) / tpc;
         ll_chunk_hist_kernel<<<dim3(chunks, num_src), 1024, size_t(num_experts) * sizeof(int32_t), stream>>>(
             topk_idx, n, tpc * num_topk, num_experts, scratch_bytes, ws);
         EP_LAUNCH_CHECK();
     }
-    // A small by-destination batch needs no launch for its tables: every token's workgroup counts the
-    // batch itself (kByDestInBlockEntries entries are a few loads per thread).
-    const bool prefix_in_block = by_dest != nullptr && tpc == 0 && n <= kByDestInBlockEntries;
+    const bool prefix_in_block = by_dest != nullptr && by_dest_tables_in_send(n, num_experts, chunks);
     if (by_dest != nullptr && !prefix_in_block) {  // the tables the by-destination rows are placed by
         EP_HOST_ASSERT(num_src == 1 && src_ranks == nullptr && fused_recv == nullptr && own_rows_direct == nullptr);
-        const int chunks = tpc > 0 ? (num_tokens + tpc - 1) / tpc : 0;
         ll_by_dest_prefix_kernel<<<1, 1024, size_t(num_experts + 1) * sizeof(int32_t), stream>>>(
             topk_idx, n, num_experts, num_ranks, max_tokens, tpc > 0 ? reinterpret_cast<const int32_t*>(ws) : nullptr,
             chunks, send_count, *by_dest);

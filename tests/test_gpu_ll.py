@@ -1083,8 +1083,15 @@ def check_send_by_dest(st, want, t):
     (1, 0, 16, 512, 2, 4),       # a world of one rank
     (4, 2, 24, 1536, 4, 16),     # hidden not a multiple of 1024
     (512, 500, 3, 512, 2, 1024),
-    (4, 3, 256, 512, 8, 32),     # 2048 entries: the last batch whose tables are built inside the send launch
-    (4, 3, 257, 512, 8, 32),     # 2056 entries: the first with a launch for them
+    (4, 3, 256, 512, 8, 32),     # 2048 entries: the last batch whose tables are built inside the send launch past 1024 experts
+    (4, 3, 257, 512, 8, 32),     # 2056 entries
+    (16, 9, 257, 512, 8, 1024),  # the most experts whose tables the send launch makes past 2048 entries
+    (16, 9, 257, 512, 8, 1040),  # and the first with a launch for them
+    (2, 1, 1024, 512, 8, 32),    # 8192 entries: the last without chunk histograms
+    (8, 5, 1030, 512, 8, 408),   # five chunk histograms of 2040 words: the send launch makes the tables
+    (8, 5, 1030, 512, 8, 416),   # 2080 words: a launch for them
+    (4, 3, 8191, 512, 8, 8),     # the last batch whose entries a half word counts
+    (4, 3, 8192, 512, 8, 8),
     (32, 7, 77, 512, 6, 288),    # five experts a lane, the last lanes without any; an odd number of entries before tokens
     (3, 2, 67, 512, 5, 195),     # as many experts as no lane's share divides, tokens of an odd number of entries
 ])
