@@ -341,6 +341,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     const int sweep_begin = chunk * a.tokens_per_chunk * num_topk;
     const bool prefix_in_block = kTables && a.prefix_in_block;
     const bool count_all = prefix_in_block && a.tokens_per_chunk == 0;
+    const bool count_chunks = prefix_in_block && a.tokens_per_chunk > 0;
     const int sweep_end = count_all ? n : entry0;
     constexpr int kSweepAhead = 2;
     const int64_t own_v = my_topk[entry0 + (tid < num_topk ? tid : num_topk - 1)];  // threads 0..K-1: selection tid
@@ -349,6 +350,19 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     EntryPair ahead[kSweepAhead];
 #pragma unroll
     for (int r = 0; r < kSweepAhead; ++r) ahead[r].load(list, tid + r * threads);
+    // the first eight words of a thread's column of the chunk histograms, zeros past the last chunk
+    uint32_t column[8];
+    int chunks = 0;
+    const auto load_column = [&](int e, int c0) {
+        const auto hists = row_buffer(a.scratch_base, chunks * num_experts * 4);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            column[u] = __builtin_amdgcn_raw_buffer_load_b32(hists, ((c0 + u) * num_experts + e) * 4, 0, 0);
+    };
+    if (count_chunks) {
+        chunks = (a.num_tokens + a.tokens_per_chunk - 1) / a.tokens_per_chunk;
+        if (tid < num_experts) load_column(tid, 0);
+    }
     for (int e = tid; e < num_experts; e += threads) lds_hist[e] = 0;
     lds_barrier();
 
@@ -389,7 +403,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     // Medium and large batches: the token sweeps only the earlier entries of its own chunk; what the
     // chunks before it hold of each selection's expert comes from their histograms.
     int chunk_base = 0;
-    if (chunk > 0 && tid < num_topk && my_expert >= 0) {
+    if (chunk > 0 && !count_chunks && tid < num_topk && my_expert >= 0) {
         const int32_t* hist = reinterpret_cast<const int32_t*>(a.scratch_base + int64_t(b) * a.scratch_stride);
         for (int c0 = 0; c0 < chunk; c0 += 8) {  // eight loads in flight
             int c[8];
@@ -408,13 +422,18 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     // With prefix_in_block the low half of a word counts all of the batch's entries and the high half those before
     // the token, and wave 0 gets the prefix from the same words (128 tokens 9.4 -> 7.8 us against a histogram of its
     // own and a scan by the whole workgroup).  The sweep then goes through the whole batch, or, where there are chunk
-    // histograms, through the token's chunk as ever, and their column sums make the low halves.
-    const int before = prefix_in_block ? (count_all ? 0x10001 : 0x10000) : 1;
-    if (prefix_in_block && !count_all) {
-        const int32_t* hist = reinterpret_cast<const int32_t*>(a.scratch_base);
-        const int chunks = (a.num_tokens + a.tokens_per_chunk - 1) / a.tokens_per_chunk;
-        for (int e = tid; e < num_experts; e += threads)
-            atomicAdd(&lds_hist[e], chunk_total(hist, chunks, num_experts, e));
+    // histograms, through the token's chunk as ever, and their columns, a thread an expert, make the rest of both halves.
+    const int before = count_chunks ? 0x10000 : (count_all ? 0x10001 : 1);
+    if (count_chunks) {
+        for (int e = tid; e < num_experts; e += threads) {
+            uint32_t sums = 0;
+            for (int c0 = 0; c0 < chunks; c0 += 8) {
+                if (c0 > 0 || e != tid) load_column(e, c0);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) sums += column[u] * (c0 + u < chunk ? 0x10001u : 1u);
+            }
+            atomicAdd(&lds_hist[e], int(sums));
+        }
     }
     const auto count_pair = [&](int pair, const EntryPair& entries) {
         if (pair >= sweep_pairs) return;
@@ -858,15 +877,15 @@ __global__ __launch_bounds__(1024) void ll_by_dest_prefix_kernel(const int64_t* 
 // Whether the send launch makes the by-destination tables, every token's workgroup for itself, instead of a launch before
 // it.  Without chunk histograms (chunks 0: up to 8192 entries) each workgroup goes through the whole batch instead of half
 // of it, and one wave through the experts: up to 1024 experts that costs less than the launch, past them only for batches
-// of up to 2048 entries.  With histograms it adds up their columns, which pays up to 2048 words.  Microseconds of the send
-// with the tables made by itself against the launch before it, top-8, fp8:
-//   300 tokens, 64 experts, hidden 7168      10.7 / 13.5        2047 tokens,  64 experts ( 512 words)  15.5 / 17.5
-//   1024 tokens, 64 experts, hidden 7168     18.2 / 19.5        8000 tokens,  64 experts (2048 words)  24.3 / 25.5
-//   300 tokens, 256 experts, hidden 2048      6.0 /  8.6        2047 tokens, 256 experts (2048 words)  16.7 / 17.7
-//   1000 tokens, 1024 experts, hidden 2048   12.1 / 14.3        2047 tokens, 512 experts (4096 words)  18.0 / 18.0
-//   1000 tokens, 4096 experts, hidden 2048   20.1 / 15.3        4000 tokens, 256 experts (4096 words)  24.2 / 23.8
+// of up to 2048 entries.  With histograms it adds up their columns, loaded with the first entries, which pays up to 4096
+// words.  Microseconds of the send with the tables made by itself against the launch before it, top-8, fp8:
+//   300 tokens, 64 experts, hidden 7168      10.7 / 13.5        2047 tokens,  64 experts ( 512 words)  14.9 / 17.5
+//   1024 tokens, 64 experts, hidden 7168     18.2 / 19.5        8000 tokens,  64 experts (2048 words)  23.0 / 25.5
+//   300 tokens, 256 experts, hidden 2048      6.0 /  8.6        2047 tokens, 256 experts (2048 words)  16.3 / 17.7
+//   1000 tokens, 1024 experts, hidden 2048   12.1 / 14.3        4000 tokens, 256 experts (4096 words)  23.6 / 24.0
+//   1000 tokens, 4096 experts, hidden 2048   20.1 / 15.3        2047 tokens, 1024 experts (8192 words) 21.0 / 18.3
 // Both counts of an expert share a 32-bit word: fewer than 2^16 entries.
-constexpr int kByDestInBlockExperts = 1024, kByDestInBlockEntries = 2048, kByDestInBlockWords = 2048;
+constexpr int kByDestInBlockExperts = 1024, kByDestInBlockEntries = 2048, kByDestInBlockWords = 4096;
 static bool by_dest_tables_in_send(int n, int num_experts, int chunks) {
     if (chunks == 0) return num_experts <= kByDestInBlockExperts || n <= kByDestInBlockEntries;
     return n < 65536 && int64_t(chunks) * num_experts <= kByDestInBlockWords;

@@ -1088,8 +1088,8 @@ def check_send_by_dest(st, want, t):
     (16, 9, 257, 512, 8, 1024),  # the most experts whose tables the send launch makes past 2048 entries
     (16, 9, 257, 512, 8, 1040),  # and the first with a launch for them
     (2, 1, 1024, 512, 8, 32),    # 8192 entries: the last without chunk histograms
-    (8, 5, 1030, 512, 8, 408),   # five chunk histograms of 2040 words: the send launch makes the tables
-    (8, 5, 1030, 512, 8, 416),   # 2080 words: a launch for them
+    (8, 5, 1030, 512, 8, 816),   # five chunk histograms of 4080 words: the send launch makes the tables
+    (8, 5, 1030, 512, 8, 824),   # 4120 words: a launch for them
     (4, 3, 8191, 512, 8, 8),     # the last batch whose entries a half word counts
     (4, 3, 8192, 512, 8, 8),
     (32, 7, 77, 512, 6, 288),    # five experts a lane, the last lanes without any; an odd number of entries before tokens
