@@ -258,7 +258,7 @@ __global__ __launch_bounds__(256) void ll_combine_index_kernel(CombineIndexArgs 
 }
 
 // ---------------------------------------------------------------------
-// Single-launch combine for small batches (at most 8192 expected rows): the reduce workgroups
+// Single-launch combine (combine_in_one_launch() says for which batches): the reduce workgroups
 // and the row-return workgroups of the two kernels above in one grid.  No
 // workgroup waits on another: the reduce reads the answers of this rank's own
 // experts straight from x (layout_range says where each segment begins), so the
@@ -613,6 +613,23 @@ int deepep_ll_combine_recv_flat(const void* recv_flat, int64_t recv_flat_rows, i
     return 0;
 }
 
+// Whether a combine whose rows are to be returned runs as one launch.  Up to kLargeBatchRows rows always.  Beyond, while
+// the rows returned and the tokens' rows stay within 220 MB: there the rows are moved beside the reduce's loads and the
+// step has one launch less.  Not where far more rows come in than the tokens send out (the hottest experts' rank: the
+// flat copy is the faster one, and the reduce too short to hide anything), nor for many rows of less than 2 KB.
+// Microseconds of a dispatch and a combine, one launch against two (rows, row size; 8 ranks x 8 experts unless given):
+//    8720 of  4 KB  55.2 /  57.4     13122 of 14 KB (2 ranks) 123.3 / 131.9      31786 of 2 KB     82.0 /  85.5
+//   11985 of  8 KB  97.1 / 107.5     11934 of 14 KB (top-4)   158.8 / 166.3      31786 of 1 KB     59.6 /  57.9
+//   19860 of  8 KB 146.3 / 155.5     13541 of 14 KB           170.0 / 175.8      31786 of 256 B    47.9 /  45.5
+//   47736 of  3 KB 134.8 / 152.4     15139 of 14 KB           179.3 / 172.1      10358 of 1 KB     33.5 /  34.5
+//   23888 of  8 KB 169.8 / 176.1     23877 of 10 KB           200.9 / 193.1
+//   skewed, 64 ranks: 10324 rows for 7200 selections 130.8 / 137.8, 13638 for 1600 130.0 / 119.8
+static bool combine_in_one_launch(int64_t rows, int num_tokens, int num_topk, int64_t row_bytes) {
+    if (rows <= kLargeBatchRows) return true;
+    return rows <= 2 * int64_t(num_tokens) * num_topk && (rows + num_tokens) * row_bytes <= (int64_t(220) << 20) &&
+           (row_bytes >= 2048 || rows <= 12288);
+}
+
 int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t* topk_idx, const float* topk_weights,
                       const int32_t* pair_slot, int num_tokens, int hidden, int num_topk, int num_experts,
                       int num_ranks, int rank, int num_max_dispatch_tokens_per_rank, int accumulate,
@@ -620,9 +637,10 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
                       void* workspace, size_t workspace_bytes, void* stream) {
     clear_error();
     const int64_t max_rows = int64_t(num_experts) * num_max_dispatch_tokens_per_rank;
-    // measured as whole calls the single launch wins up to this bound (512 tokens: 36 us against 40 for
-    // the phases back to back), although each phase timed alone on cache-warm data suggests otherwise
-    if (estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank) > kLargeBatchRows) {
+    const int64_t estimated = estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank);
+    const bool large = estimated > kLargeBatchRows;
+    if (large && (combine_send_slots == nullptr ||
+                  !combine_in_one_launch(estimated, num_tokens, num_topk, int64_t(hidden) * 2))) {
         // the two phases back to back, with the single launch's shortcut: the rows owed to this rank
         // itself are not moved, the reduce reads them from x.  Without send slots (zero copy: the transport
         // sends layout_range's ranges straight from x) there is nothing to return.
@@ -657,6 +675,12 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     if (int rc = check_combine_recv_args(combine_staging, topk_idx, topk_weights, pair_slot, num_tokens, hidden,
                                          num_topk, num_experts, num_max_dispatch_tokens_per_rank, out))
         return rc;
+    if (large && workspace != nullptr) {  // not needed in one launch: held to the same rules
+        CombineIndexArgs index;
+        if (int rc = make_combine_index(layout_range, num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank,
+                                        true, workspace, workspace_bytes, index))
+            return rc;
+    }
     const CombineSendArgs sa = make_combine_send_args(x, layout_range, hidden, num_experts, num_ranks, rank,
                                                       num_max_dispatch_tokens_per_rank, combine_staging,
                                                       combine_send_slots, expected_rows);
@@ -674,9 +698,10 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     if (send_blocks > 16384) send_blocks = 16384;
     if (recv_blocks + send_blocks == 0) return 0;
     const size_t lds = size_t(sa.num_local_experts) * sizeof(int32_t);
-    // rows returned (read + written) plus rows gathered: past what the caches hold, stream
+    // rows returned (read + written) plus rows gathered: past what the caches hold, stream.  Beside more than
+    // kLargeBatchRows rows it always pays (11946 of 4 KB, 61.2 -> 57.5 us a step).
     const int64_t traffic = (2 * rows + int64_t(num_tokens) * num_topk) * hidden * 2;
-    if (traffic > stream_bytes())
+    if (large || traffic > stream_bytes())
         ll_combine_fused_kernel<true><<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds,
                                         reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks));
     else

@@ -1656,6 +1656,35 @@ def test_large_combine_moves_no_rows_of_a_malformed_range(rt, t, k):
     assert torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("h,hints", [
+    (1024, (8192, 8193, 16400, 16401)),  # one launch, one that streams, the last before twice the selections, two launches
+    (512, (12288, 12289)),  # rows below 2 KB: one launch, two
+])
+def test_combine_in_one_launch_and_in_two(rt, h, hints):
+    """A combine's rows and its sums do not depend on which launches the expected rows choose."""
+    r, rank, t, k, e = 8, 3, 1025, 8, 16
+    x_all, topk_all, w = make_world(r, t, h, k, e, seed=h, drop=30)
+    st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, t, O.ROW_BF16, one_call=True)
+    y = torch.randn(st.packed_recv_x.shape, generator=torch.Generator().manual_seed(h)).bfloat16().cuda()
+    world.combine_from_peers(st, mode=1, seed=5)
+    ranges, slots = st.packed_recv_layout_range.cpu(), torch.full((e // r, r, t, h), 0x7FC0, dtype=torch.int16)
+    for le in range(e // r):
+        for s in range(r):
+            n, begin = int(ranges[le, s] & 0xffffffff), int(ranges[le, s] >> 32)
+            if s != rank:
+                slots[le, s, :n] = y[le, begin:begin + n].view(torch.int16).cpu()
+    sums = []
+    for hint in hints:
+        st.expected_rows = hint
+        st.combine_send_slots.view(torch.int16).fill_(0x7FC0)
+        out = torch.zeros((t, h), dtype=torch.bfloat16, device="cuda")
+        st.combine(y, topk_all[rank].cuda(), w[rank].cuda(), out)
+        torch.cuda.synchronize()
+        assert torch.equal(st.combine_send_slots.view(torch.int16).view(e // r, r, t, h).cpu(), slots)
+        sums.append(out.cpu())
+    assert all(torch.equal(sums[0], o) for o in sums[1:])
+
+
 def test_all_to_all_calls_let_other_threads_run(rt):
     """A launch of the all-to-all surface releases the GIL.  The interpreter is told never to take it away from a
     running thread, and nothing else in the loop gives it up, so the second thread gets on only through the calls."""
