@@ -360,8 +360,8 @@ __global__ __launch_bounds__(kIndexThreads) void ll_by_source_ordered_index_kern
 }
 
 // ---------------------------------------------------------------------
-// The ordered receive for small batches (at most kLargeBatchRows rows expected): index and copy in one
-// launch, like the staged receive's ll_recv_kernel.  Every workgroup works out the (expert, source)
+// The ordered receive for small batches (ordered_in_one_launch()): index and copy in one launch,
+// like the staged receive's ll_recv_kernel.  Every workgroup works out the (expert, source)
 // pairs' numbers for itself in LDS -- sent(e, s) from the gathered counts, first(e, s) (where the pair
 // starts in its source's message) and kept(e, s) -- one thread per pair; a copying wave then holds kept
 // and first in its registers (WaveSegments) and walks the flat index space of the rows kept, one wave
@@ -623,6 +623,15 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
     return 0;
 }
 
+// Past 52 MB the flat copy gains more than the index's launch costs.  Microseconds of the five calls of an exchange, 8
+// ranks x 8 experts, one launch against two:
+//   3600 rows of 14 KB (50 MB)  84.2 / 85.3     4400 (60 MB)  96.8 / 95.2     5600  116.3 / 113.3     8000  153.5 / 146.4
+//   6800 rows of  7 KB (46 MB) 108.5 / 109.5    8000 (55 MB) 119.8 / 118.2    8800  129.8 / 126.8
+//   6400 rows of  8 KB (50 MB)  86.2 / 87.0     8000 (62 MB)  93.9 / 93.0
+static bool ordered_in_one_launch(int64_t rows, int64_t row_bytes) {
+    return rows <= kLargeBatchRows && rows * row_bytes <= (int64_t(52) << 20);
+}
+
 int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_t slot_rows,
                                               const int32_t* all_num_routed, int hidden, int num_experts,
                                               int num_ranks, int rank, int num_max_dispatch_tokens_per_rank,
@@ -658,7 +667,7 @@ int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_
     const int num_local_experts = num_experts / num_ranks;
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     const int64_t expected = expected_rows > 0 ? expected_rows : most_rows;
-    if (expected <= kLargeBatchRows) {  // one launch: every workgroup indexes for itself
+    if (ordered_in_one_launch(expected, row_data_bytes(hidden, row_format))) {  // every workgroup indexes for itself
         OrderedRecvArgs oa;
         oa.rows = reinterpret_cast<const uint8_t*>(recv_by_source);
         oa.all_num_routed = all_num_routed;

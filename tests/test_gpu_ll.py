@@ -1656,6 +1656,27 @@ def test_large_combine_moves_no_rows_of_a_malformed_range(rt, t, k):
     assert torch.equal(got[0][1], got[1][1])
 
 
+@pytest.mark.parametrize("fmt,h,hints", [(O.ROW_BF16, 4096, (6656, 6657)), (O.ROW_FP8, 7168, (7606, 7607, 8193))])
+def test_ordered_receive_in_one_launch_and_in_two(rt, fmt, h, hints):
+    """On either side of the 52 MB of expected rows the ordered receive gives the oracle's rows and records."""
+    r, rank, t, k, e = 3, 1, 40, 4, 24
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=h, drop=9)
+    states = [rt.ll.AllToAllState(rt.ll.LLShape(r, s, e, t, h, k, fmt)) for s in range(r)]
+    for s, st in enumerate(states):
+        st.dispatch_send(x_all[s].cuda(), topk_all[s].cuda())
+    torch.cuda.synchronize()
+    routed, st = all_to_all_dispatch(states, fmt), states[rank]
+    want, rec = O.ll_dispatch(list(x_all), list(topk_all), rank, e, t, fmt), O.ll_record_packed_rows(list(topk_all), rank, e, t)
+    for hint in hints:
+        poison_outputs_keep_pair_slot(st)
+        st.record_packed_row.fill_(-7)
+        st.expected_rows = hint
+        st.dispatch_recv_ordered(routed)
+        torch.cuda.synchronize()
+        check_dispatch(st, want, fmt)
+        assert torch.equal(st.record_packed_row[:rec.numel()].cpu().long(), rec)
+
+
 @pytest.mark.parametrize("h,hints", [
     (1024, (8192, 8193, 16400, 16401)),  # one launch, one that streams, the last before twice the selections, two launches
     (512, (12288, 12289)),  # rows below 2 KB: one launch, two
