@@ -546,7 +546,7 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 
 // ---------------------------------------------------------------------
 // pack_rows: dst[i] = src[ids[i]].  One workgroup per output row, two 16-byte
-// vectors per thread in flight (rows wider than 1024 vectors loop).  The row
+// vectors per thread in flight (wider rows loop).  The row
 // count is read from device memory so no host sync is needed.
 // Reference: deep_ep/buffer.py:877,917 (torch advanced-index gathers).
 //
@@ -576,7 +576,9 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // Groups of 6, 12, 24 and 48 MB: 230, 215, 211 and 207 us, but from 36 MB on 5 us are lost where their source rows
 // no longer fit an L2 (4 MB); fewer than two groups an XCD lose a tenth.  The groups' rows drift apart by some fifty
 // tokens, so a group reads half as much again as its share of the source.
-// Up to 256 threads while the rows stay in the caches: 600 x 14336 10.7 -> 10.1 us.
+// Up to 256 threads while the rows stay in the caches: 600 x 14336 10.7 -> 10.1 us.  In list order, past them, one vector
+// a thread, up to 512 threads: two trips to memory stand in front of a row there.  4096 x 14336 87.3 us against 96.1 with
+// two vectors and 88.7 with 1024 threads, 4096 x 7168 46.0 and 47.9, 12289 x 14336 258 and 267.
 // ---------------------------------------------------------------------
 constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of a group: about 2 MB of source rows
 constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
@@ -590,7 +592,7 @@ struct PackArgs {
     int scale_row_bytes;
 };
 
-template <bool kStream>
+template <bool kStream, int kVecs>
 __device__ __forceinline__ void pack_row(const PackArgs& a, const int64_t* __restrict__ ids, int64_t row) {
     const int64_t id = ids[row];
     if (id < 0 || id >= a.num_src_rows) return;
@@ -600,7 +602,7 @@ __device__ __forceinline__ void pack_row(const PackArgs& a, const int64_t* __res
     const int num_scales = a.scale_src != nullptr ? a.scale_row_bytes / 4 : 0;
     uint32_t scale = 0;
     if (tid < num_scales) scale = scales[tid];  // in flight with the payload, not behind its stores
-    block_copy_row<2, false, kStream>(a.src + id * a.row_bytes, a.dst + row * a.row_bytes, a.row_bytes / 16, tid, a.threads);
+    block_copy_row<kVecs, false, kStream>(a.src + id * a.row_bytes, a.dst + row * a.row_bytes, a.row_bytes / 16, tid, a.threads);
     if (tid < num_scales) scales_to[tid] = scale;
     for (int v = tid + a.threads; v < num_scales; v += a.threads) scales_to[v] = scales[v];
 }
@@ -611,7 +613,7 @@ __global__ __launch_bounds__(1024) void pack_rows_kernel(const int64_t* __restri
                                                          uint32_t grid, PackArgs a) {
     int64_t num_rows = *num_rows_dev;
     if (num_rows > max_rows) num_rows = max_rows;
-    for (int64_t i = blockIdx.x; i < num_rows; i += grid) pack_row<kStream>(a, ids, i);
+    for (int64_t i = blockIdx.x; i < num_rows; i += grid) pack_row<kStream, kStream ? 1 : 2>(a, ids, i);
 }
 
 template <bool kStream>
@@ -638,7 +640,7 @@ __global__ __launch_bounds__(1024) void pack_groups_kernel(const int64_t* __rest
         const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(begin), r);
         const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(begin >> 32), r);
         const int64_t row = int64_t((uint64_t(hi) << 32) | lo) + slot;
-        if (row >= 0 && row < max_rows) pack_row<kStream>(a, ids, row);
+        if (row >= 0 && row < max_rows) pack_row<kStream, 2>(a, ids, row);
     }
 }
 
@@ -850,12 +852,15 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
     a.dst = reinterpret_cast<uint8_t*>(dst), a.scale_dst = reinterpret_cast<uint8_t*>(scale_dst);
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     const bool stream_rows = max_rows * row_bytes > kPackStreamBytes;
-    a.threads = flat_row_threads((row_bytes / 16 + 1) / 2, stream_rows ? 512 : 256);
-    const int threads = a.threads;
     // Below a group's worth of packed rows everything stays in the caches and the grouping's lookup is one more
     // round trip in front of the rows: 6.5 MB 2.9 us against 3.4, 12 MB 3.9 either way, 22 MB 6.7 against 5.0.
     // A wave holds the ranks' parts one a lane, hence the 64.
-    if (send_cumsum != nullptr && num_ranks > 1 && num_ranks <= kWave && max_rows * row_bytes > kPackGroupBytes) {
+    const bool grouped =
+        send_cumsum != nullptr && num_ranks > 1 && num_ranks <= kWave && max_rows * row_bytes > kPackGroupBytes;
+    a.threads = stream_rows && !grouped ? flat_row_threads(row_bytes / 16, 512)
+                                        : flat_row_threads((row_bytes / 16 + 1) / 2, stream_rows ? 512 : 256);
+    const int threads = a.threads;
+    if (grouped) {
         int group_log2 = 3;  // two groups an XCD before a group may be larger
         while (((max_rows * row_bytes) >> group_log2) > (group_log2 == 3 ? kPackGroupBytes : 2 * kPackGroupBytes) &&
                group_log2 < 16)
