@@ -576,9 +576,9 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // Groups of 6, 12, 24 and 48 MB: 230, 215, 211 and 207 us, but from 36 MB on 5 us are lost where their source rows
 // no longer fit an L2 (4 MB); fewer than two groups an XCD lose a tenth.  The groups' rows drift apart by some fifty
 // tokens, so a group reads half as much again as its share of the source.
-// Up to 256 threads while the rows stay in the caches: 600 x 14336 10.7 -> 10.1 us.  In list order, past them, one vector
-// a thread, up to 512 threads: two trips to memory stand in front of a row there.  4096 x 14336 87.3 us against 96.1 with
-// two vectors and 88.7 with 1024 threads, 4096 x 7168 46.0 and 47.9, 12289 x 14336 258 and 267.
+// Up to 256 threads while the rows stay in the caches: 600 x 14336 10.7 -> 10.1 us.  In list order, past them, the same
+// threads move one vector at a time: two trips to memory stand in front of a row there.  4096 x 14336 88.5 us against 96.1
+// with two vectors in flight, 4096 x 7168 45.5 and 47.9 (46.0 to 48 with twice the threads), 12289 x 14336 258 and 267.
 // ---------------------------------------------------------------------
 constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of a group: about 2 MB of source rows
 constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
@@ -857,8 +857,7 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
     // A wave holds the ranks' parts one a lane, hence the 64.
     const bool grouped =
         send_cumsum != nullptr && num_ranks > 1 && num_ranks <= kWave && max_rows * row_bytes > kPackGroupBytes;
-    a.threads = stream_rows && !grouped ? flat_row_threads(row_bytes / 16, 512)
-                                        : flat_row_threads((row_bytes / 16 + 1) / 2, stream_rows ? 512 : 256);
+    a.threads = flat_row_threads((row_bytes / 16 + 1) / 2, stream_rows ? 512 : 256);
     const int threads = a.threads;
     if (grouped) {
         int group_log2 = 3;  // two groups an XCD before a group may be larger
