@@ -326,6 +326,7 @@ def test_pack_rows(capi, rows, row_bytes, scale_bytes):
     (9000, 4096, 4, 8, 0.5, 1.0),      # past 128 MB of packed rows, where they are stored past the caches
     (5500, 4112, 0, 72, 0.1, 1.0),     # the same in list order
     (9000, 8192, 516, 8, 0.72, 1.0),   # more than two groups an XCD; scales wider than a wave
+    (9000, 8192, 516, 8, 0.3, 1.0),  # few copies a row: the groups are bound by their source rows
 ])
 def test_pack_rows_by_rank(capi, rows, row_bytes, scale_bytes, r, odds, keep):
     lib = capi.load()
