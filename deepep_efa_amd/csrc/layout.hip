@@ -576,13 +576,14 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // Groups of 6, 12, 24 and 48 MB: 230, 215, 211 and 207 us, but much is lost where their source rows no longer fit an L2
 // (4 MB): a whole prefill of 9000 x 7168 in fp8 to 8 ranks 262 us with 4.0 MB of source a group and 250 with 2.0, of 6000 x
 // 14336 at top-6 188 and 173 with 5.4 and 2.7, of 7000 x 8192 127.3 and 125 with 3.4 and 1.7; 2.9 at 32 ranks gains (308
-// -> 302 against half).  Fewer than two groups an XCD lose a tenth.  The groups' rows drift apart by some fifty
+// -> 302 against half).  Fewer than two groups an XCD lose a tenth, and two of more than 16 MB some: the pack of 7000 x 7168
+// in fp8 to 32 ranks behind its cast 68.5 us with 16 groups of 22 MB, 63.6 with 32.  The groups' rows drift apart by some fifty
 // tokens, so a group reads half as much again as its share of the source.
 // Up to 256 threads while the rows stay in the caches: 600 x 14336 10.7 -> 10.1 us.  In list order, past them, the same
 // threads move one vector at a time: two trips to memory stand in front of a row there.  4096 x 14336 88.5 us against 96.1
 // with two vectors in flight, 4096 x 7168 45.5 and 47.9 (46.0 to 48 with twice the threads), 12289 x 14336 258 and 267.
 // ---------------------------------------------------------------------
-constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of a group, twice that from 16 groups on
+constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of one of 8 groups; 16 MB of 16, 24 MB of more
 constexpr int64_t kPackSourceBytes = int64_t(3) << 20;  // source bytes of a group
 constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
 
@@ -863,8 +864,8 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
     a.threads = flat_row_threads((row_bytes / 16 + 1) / 2, stream_rows ? 512 : 256);
     const int threads = a.threads;
     if (grouped) {
-        int group_log2 = 3;  // two groups an XCD before a group may be larger, and its source rows no larger than its L2
-        while (((max_rows * row_bytes) >> group_log2) > (group_log2 == 3 ? kPackGroupBytes : 2 * kPackGroupBytes) ||
+        int group_log2 = 3;  // the fewer groups an XCD, the smaller, and no group's source rows larger than fit its L2
+        while (((max_rows * row_bytes) >> group_log2) > kPackGroupBytes * (group_log2 < 5 ? group_log2 : 6) / 3 ||
                ((int64_t(num_src_rows) * row_bytes) >> group_log2) > kPackSourceBytes)
             if (++group_log2 == 16) break;
         // rounding down the parts of every rank's list can put one more row per rank into a group

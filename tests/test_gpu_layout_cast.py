@@ -327,6 +327,7 @@ def test_pack_rows(capi, rows, row_bytes, scale_bytes):
     (5500, 4112, 0, 72, 0.1, 1.0),     # the same in list order
     (9000, 8192, 516, 8, 0.72, 1.0),   # more than two groups an XCD; scales wider than a wave
     (9000, 8192, 516, 8, 0.3, 1.0),  # few copies a row: the groups are bound by their source rows
+    (9000, 8192, 0, 8, 0.5, 1.0),  # more than 16 groups for their size alone
 ])
 def test_pack_rows_by_rank(capi, rows, row_bytes, scale_bytes, r, odds, keep):
     lib = capi.load()
