@@ -514,13 +514,15 @@ inline int64_t estimated_rows(int64_t expected_rows, int64_t num_experts, int64_
 
 // Workgroups for `rows` expected rows of at most max_rows.  One that finds no row costs what it takes to launch its
 // waves (a nanosecond for fourteen: 4 us for an eighth too many of 32768), one that finds a second row about 2 us at
-// the very end: a thirty-second more than expected.
-inline unsigned flat_grid_blocks(int64_t rows, int64_t max_rows) {
+// the very end: a thirty-second more than expected.  No more than a launch takes, which is 2^32 - 1 threads.
+inline unsigned flat_grid_blocks(int64_t rows, int64_t max_rows, int threads) {
     int64_t want = rows + rows / 32 + 64;
     if (want > max_rows) want = max_rows;
     if (want > (int64_t(1) << 22)) want = int64_t(1) << 22;
     if (want < 1) want = 1;
-    return unsigned((want + kFlatRound - 1) / kFlatRound * kFlatRound);  // whole rounds over the XCDs
+    want = (want + kFlatRound - 1) / kFlatRound * kFlatRound;  // whole rounds over the XCDs
+    const int64_t most = 0xffffffffll / threads / kFlatRound * kFlatRound;
+    return unsigned(want < most ? want : most);
 }
 
 // The flat copy of the rows `desc` describes (*total of them, memory for max_rows); expected_rows sizes the grid.
@@ -529,8 +531,8 @@ inline void launch_rows_flat(const int32_t* total, const RowDesc* desc, int64_t 
                              int64_t dst_stride, const FlatTails* tails, hipStream_t stream) {
     // many short rows: two a workgroup are 1 % faster (160000 x 7168 bytes 383 -> 378 us; 28672: 65.7 -> 66.3)
     const bool pairs = expected_rows > 65536 && num_vec <= 512;
-    const unsigned grid = flat_grid_blocks(pairs ? expected_rows / 2 : expected_rows, max_rows);
     const int others = tails != nullptr ? kWave : 0, threads = flat_row_threads(num_vec, 1024 - others);
+    const unsigned grid = flat_grid_blocks(pairs ? expected_rows / 2 : expected_rows, max_rows, threads + others);
 #define DEEPEP_LAUNCH_ROWS(TAILS)                                                                                     \
     ll_rows_flat_kernel<TAILS><<<grid, threads + others, 0, stream>>>(                                                \
         total, desc, uint32_t(max_rows), grid, reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst), \

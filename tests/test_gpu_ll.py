@@ -1623,6 +1623,53 @@ def test_row_copies_over_widths_and_hints(rt, t, h, fmt, hint):
     assert torch.equal(st.combine_send_slots, slots) and torch.equal(st.combine_staging, staging)
 
 
+def test_row_return_sized_for_more_rows_than_a_launch_has_threads(rt):
+    """4.2 million expected rows of 1024 vectors, a workgroup of 1024 threads each, would be 2^32 threads, which a
+    launch refuses; the six rows that are there are moved all the same."""
+    r, m, h, n = 1024, 4096, 8192, 3
+    lib = rt.capi.load()
+    x = torch.randn((2 * n, h), generator=torch.Generator().manual_seed(1)).bfloat16().cuda()
+    ranges = torch.zeros((1, r), dtype=torch.int64)
+    ranges[0, 0], ranges[0, 1] = n, (n << 32) | n  # this rank's own rows and those owed to rank 1
+    ranges = ranges.cuda()
+    staging = torch.full((n + 1, h), 3.0, dtype=torch.bfloat16, device="cuda")
+    slots = torch.full((m + n + 1, h), 3.0, dtype=torch.bfloat16, device="cuda")
+    ws = torch.empty(lib.deepep_ll_segment_workspace_bytes(r, m), dtype=torch.uint8, device="cuda")
+    rt.capi.check(lib.deepep_ll_combine_send(
+        rt.capi.ptr(x), rt.capi.ptr(ranges), h, r, r, 0, m, rt.capi.ptr(staging), rt.capi.ptr(slots), r * m,
+        rt.capi.ptr(ws), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(staging[:n], x[:n]) and torch.equal(slots[m:m + n], x[n:])
+    assert bool((staging[n:] == 3.0).all()) and bool((slots[:m] == 3.0).all()) and bool((slots[m + n:] == 3.0).all())
+
+
+@pytest.mark.parametrize("hint", [0, 1024 * 4096])
+def test_ordered_receive_sized_for_more_rows_than_a_launch_has_threads(rt, hint):
+    """The same for rows whose payload takes 960 threads and whose scales take a wave more, by a hint and by capacity."""
+    r, m, h, n = 1024, 4096, 15360, 3
+    lib = rt.capi.load()
+    stride, payload = lib.deepep_ll_row_stride(h, O.ROW_FP8), lib.deepep_ll_row_payload_bytes(h, O.ROW_FP8)
+    rows = torch.randint(0, 256, (m + n, stride), dtype=torch.uint8, generator=torch.Generator().manual_seed(2)).cuda()
+    routed = torch.zeros((r, r), dtype=torch.int32)
+    routed[:2, 0] = n  # sources 0 and 1 send three rows each to this rank's expert
+    routed = routed.cuda()
+    i32 = dict(dtype=torch.int32, device="cuda")
+    px = torch.full((2 * n + 1, h), 7, dtype=torch.uint8, device="cuda")
+    scales, info = torch.full((2 * n + 1, h // 128), 7, **i32), torch.full((2 * n + 1,), 7, **i32)
+    ranges, count = torch.empty((1, r), dtype=torch.int64, device="cuda"), torch.empty(1, **i32)
+    ws = torch.empty(256 + r * m * 8, dtype=torch.uint8, device="cuda")
+    rt.capi.check(lib.deepep_ll_dispatch_recv_by_source_ordered(
+        rt.capi.ptr(rows), m, rt.capi.ptr(routed), h, r, r, 0, m, O.ROW_FP8, rt.capi.ptr(px), rt.capi.ptr(scales),
+        rt.capi.ptr(info), rt.capi.ptr(ranges), rt.capi.ptr(count), None, None, None, r * m, hint, rt.capi.ptr(ws),
+        ws.numel(), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    want = torch.cat([rows[:n], rows[m:]])
+    assert count.tolist() == [2 * n]
+    assert torch.equal(px[:2 * n], want[:, :h]) and bool((px[2 * n] == 7).all())
+    assert torch.equal(scales[:2 * n], want[:, h:h + h // 32].contiguous().view(torch.int32)) and bool((scales[2 * n] == 7).all())
+    assert torch.equal(info[:2 * n], want[:, payload - 16:payload - 12].contiguous().view(torch.int32).view(-1)) and int(info[2 * n]) == 7
+
+
 @pytest.mark.parametrize("t,k", [(1025, 8), (1100, 8)])
 def test_large_combine_moves_no_rows_of_a_malformed_range(rt, t, k):
     """Past 8192 rows the reduce's launch builds the row return's index; a segment whose range leaves its expert gets
