@@ -570,7 +570,7 @@ int deepep_ll_combine_send_by_dest(const void* x, const int32_t* record_packed_r
     const int num_vec = hidden * 2 / 16, threads = flat_row_threads(num_vec, 512);
     // grid from the rows expected, not from the capacity (an idle workgroup is not free)
     const int64_t rows = expected_rows > 0 && expected_rows < row_capacity ? expected_rows : row_capacity;
-    const unsigned grid = flat_grid_blocks(rows, row_capacity, threads);
+    const unsigned grid = flat_grid_blocks(flat_rows_expected(expected_rows, row_capacity), row_capacity, threads);
     const int64_t x_rows = std::min(int64_t(num_experts) * num_max_dispatch_tokens_per_rank, int64_t(1) << 31);
 #define DEEPEP_LAUNCH_BY_DEST(STREAM, PEERS)                                                                            \
     ll_combine_send_by_dest_kernel<STREAM, PEERS><<<grid, threads, 0, reinterpret_cast<hipStream_t>(stream)>>>(         \

@@ -617,7 +617,7 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
     tails.scale_dwords = packed_recv_scales != nullptr ? uint32_t(scale_bytes / 4) : 0u;
     tails.scale_off = uint32_t(align16(data_bytes));
     tails.info_off = uint32_t(tail_off);
-    launch_rows_flat(flat_total, desc, row_capacity, expected_rows > 0 ? expected_rows : row_capacity, rows_in,
+    launch_rows_flat(flat_total, desc, row_capacity, flat_rows_expected(expected_rows, row_capacity), rows_in,
                      stride, num_vec, packed_recv_x, nullptr, data_bytes, &tails, hs);
     EP_LAUNCH_CHECK();
     return 0;
@@ -705,7 +705,7 @@ int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_
     tails.scale_dwords = packed_recv_scales != nullptr ? uint32_t(scale_bytes / 4) : 0u;
     tails.scale_off = uint32_t(align16(data_bytes));
     tails.info_off = uint32_t(align16(data_bytes) + align16(scale_bytes));
-    launch_rows_flat(flat_total, desc, most_rows, expected_rows > 0 ? expected_rows : most_rows, recv_by_source,
+    launch_rows_flat(flat_total, desc, most_rows, flat_rows_expected(expected_rows, most_rows), recv_by_source,
                      row_stride_bytes(hidden, row_format), num_vec, packed_recv_x, nullptr, data_bytes, &tails, hs);
     EP_LAUNCH_CHECK();
     return 0;

@@ -394,8 +394,10 @@ size_t deepep_ll_by_source_workspace_bytes(int num_experts, int64_t row_capacity
  *                   expert in its tail, past its pair's M rows) -- the reference's recv_expert_ids /
  *                   recv_expert_pos (csrc/kernels/efa_kernels.cu:2121-2231), which the combine needs to
  *                   return the rows in arrival order (deepep_ll_combine_send_by_dest)
- *   expected_rows   rows the caller expects to receive (0 = unknown: row_capacity is assumed); it only
- *                   sizes the copy's grid, and any value gives the same result
+ *   expected_rows   rows the caller expects to receive (0 = unknown: row_capacity is assumed, but the copy's
+ *                   grid is no larger than for 16384 rows); it sizes the grid and picks between equivalent
+ *                   kernels, and any value gives the same result.  Too large a value costs more than too small
+ *                   a one: a nanosecond for every row that is not there, against a seventh of the copy's time
  *   workspace       deepep_ll_by_source_workspace_bytes(E, row_capacity) bytes
  * An (expert, source) pair takes at most M rows, as a segment of the staged form does.
  * Replaces ll_recv_unpack_v2 on its flat / slotted input (csrc/kernels/efa_kernels.cu:2121-2231,
@@ -501,7 +503,7 @@ int deepep_ll_combine_recv(const void* combine_staging, const int64_t* topk_idx,
  * being the record's place among the rows of source s = source_rank[i].
  *   recv_counts                 [R] int32     } outputs of deepep_ll_exchange_metadata
  *   combine_remote_recv_offset  [R] int64     }
- *   expected_rows   rows the caller expects to return (0 = unknown: row_capacity); sizes the grid only
+ *   expected_rows   rows the caller expects to return (0 = unknown), as for deepep_ll_dispatch_recv_by_source
  *   peer_recv_flat  [R] device array of pointers to the ranks' receive buffers (the buffer
  *                   deepep_ll_combine_recv_flat reads, flat form), peer_recv_rows [R] int64 their rows
  * Replaces the gather + un-sort of deep_ep/buffer.py:2601-2608 and a2a_combine_send

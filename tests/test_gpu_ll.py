@@ -1589,6 +1589,39 @@ def test_return_by_destination_over_record_counts(rt, records, hidden):
     assert torch.equal(out.cpu(), want)
 
 
+@pytest.mark.parametrize("records", [1000, 16384 + 256, 20000])
+def test_return_by_destination_with_room_for_a_million_records_and_no_hint(rt, records):
+    """Every record is moved, also those past the 16384 workgroups, and none of the room is paid for: 820 us for 1000
+    rows with a workgroup for each record there is room for, 17 with 16384 of them, 5 with the rows as a hint."""
+    h, e, m, capacity = 7168, 64, 16384, 1 << 20
+    lib = rt.capi.load()
+    x = torch.randn((records, h), generator=torch.Generator().manual_seed(records)).bfloat16().cuda()
+    out = torch.full((records, h), 3.0, dtype=torch.bfloat16, device="cuda")  # no record names a row past it
+    index = torch.arange(capacity, dtype=torch.int32, device="cuda")
+    num = torch.tensor([records, records], dtype=torch.int32, device="cuda")
+
+    def move(hint):
+        rt.capi.check(lib.deepep_ll_combine_send_by_dest(
+            rt.capi.ptr(x), rt.capi.ptr(index), None, rt.capi.ptr(index), rt.capi.ptr(index), rt.capi.ptr(num), capacity, h, e,
+            8, m, rt.capi.ptr(out), None, None, None, None, hint, torch.cuda.current_stream().cuda_stream))
+
+    def best(hint):
+        times = []
+        for _ in range(10):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            move(hint)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end) * 1000)
+        return min(times)
+
+    move(0)
+    torch.cuda.synchronize()
+    assert torch.equal(out, x)
+    assert best(0) < best(records) + 150
+
+
 @pytest.mark.parametrize("t,h,fmt,hint", [
     (33, 128, O.ROW_FP8, 8193), (33, 15488, O.ROW_FP8, 8193),  # the grid is far larger than the rows; two trips a row
     (40, 8320, O.ROW_BF16, 9000), (1300, 512, O.ROW_FP8_UE8M0, 8193),  # more rows than workgroups
