@@ -44,6 +44,7 @@ PROTOTYPES = {
     "deepep_ll_dispatch_observed": (_I, [_VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP,
                                          _VP, _VP, _VP, _I64, _VP, _SZ, _VP, _SZ, _VP, _VP]),
     "deepep_ll_expected_rows": (_I64, [_I, _I, _I, _I, _c.c_uint64]),
+    "deepep_ll_expected_rows_of_two": (_I64, [_I, _I, _I, _I, _c.c_uint64, _c.c_uint64]),
     "deepep_ll_combine": (_I, [_VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I, _VP, _VP, _VP, _I64, _VP, _SZ,
                                _VP]),
     "deepep_topk_remap": (_I, [_VP, _VP, _VP, _VP, _I, _I, _I, _I, _I64, _VP, _VP, _VP]),

@@ -217,8 +217,8 @@ static int row_format_of(bool use_fp8, bool round_scale, bool use_ue8m0) {
 }
 
 // Row-count words (Buffer::observed) of buffers dropped without destroy().  Kernels may still store to them, and the
-// garbage collector may drop a buffer during a capture, where nothing can be waited for: such a word stays what it
-// is and goes to the next buffer of the device, for which a late count is a poor hint and no more.  So there are
+// garbage collector may drop a buffer during a capture, where nothing can be waited for: such words stay what they
+// are and go to the next buffer of the device, for which a late count is a poor hint and no more.  So there are
 // never more of them than buffers were alive at a time.
 struct RetiredWords {
     std::mutex mutex;
@@ -264,11 +264,12 @@ struct Buffer {
     LowLatencyCache ll;
     std::vector<torch::Tensor> combine_input_buffers;
     int combine_buffer_idx = 0;
-    // What the last dispatch that has run received, stored there by its kernel as (tokens << 32) | rows: the next
-    // call is sized by it.  Under skewed routing a rank can receive many times num_tokens * num_topk rows, and
-    // kernels sized for a balanced world walk such a batch in a slow loop.
+    // What the last two dispatches that have run received, stored there in turn by their kernels as
+    // (tokens << 32) | rows: the next call is sized by them.  Under skewed routing a rank can receive many times
+    // num_tokens * num_topk rows, and kernels sized for a balanced world walk such a batch in a slow loop.
     at::DataPtr observed_memory;
-    std::atomic<uint64_t>* observed = nullptr;
+    std::atomic<uint64_t>* observed = nullptr;  // [2]
+    unsigned num_reporting = 0;
     // loopback world
     std::optional<torch::Tensor> world_x, world_topk_idx;
     torch::Tensor ranks_below, ranks_above, peer_workspace;
@@ -530,10 +531,12 @@ struct Buffer {
         return ll;
     }
 
-    // Rows a batch of num_tokens probably receives, from what the last one did.
+    // Rows a batch of num_tokens probably receives, from what the last two did.
     int64_t rows_expected(int num_tokens, int num_topk, int num_experts, int max_tokens) const {
-        return deepep_ll_expected_rows(num_tokens, num_topk, num_experts, max_tokens,
-                                       observed != nullptr ? observed->load(std::memory_order_relaxed) : 0);
+        if (observed == nullptr) return deepep_ll_expected_rows(num_tokens, num_topk, num_experts, max_tokens, 0);
+        return deepep_ll_expected_rows_of_two(num_tokens, num_topk, num_experts, max_tokens,
+                                              observed[0].load(std::memory_order_relaxed),
+                                              observed[1].load(std::memory_order_relaxed));
     }
 
     void stage_peer_rows(LowLatencyCache& c) {
@@ -597,8 +600,9 @@ struct Buffer {
         const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
         if (observed == nullptr and not capturing) {
             observed_memory = RetiredWords::take(device_id);
-            if (!observed_memory) observed_memory = at::getHostAllocator(at::kCUDA)->allocate(sizeof(uint64_t));
-            observed = new (observed_memory.get()) std::atomic<uint64_t>(0);
+            if (!observed_memory) observed_memory = at::getHostAllocator(at::kCUDA)->allocate(2 * sizeof(uint64_t));
+            observed = static_cast<std::atomic<uint64_t>*>(observed_memory.get());
+            for (int i = 0; i < 2; ++i) new (observed + i) std::atomic<uint64_t>(0);
         }
         // send and receive phase in one call (one kernel launch for decode-sized batches)
         abi_check(deepep_ll_dispatch_observed(
@@ -611,7 +615,7 @@ struct Buffer {
             cumulative_local_expert_recv_stats != nullptr ? cumulative_local_expert_recv_stats->data_ptr<int>() : nullptr,
             rows_expected(num_tokens, num_topk, num_experts, num_max_dispatch_tokens_per_rank), c.workspace.data_ptr(),
             size_t(c.workspace.numel()), c.segment_workspace.data_ptr(), size_t(c.segment_workspace.numel()),
-            capturing ? nullptr : reinterpret_cast<uint64_t*>(observed), stream));
+            capturing ? nullptr : reinterpret_cast<uint64_t*>(observed + (num_reporting++ & 1)), stream));
         c.dispatched = true;
         return c;
     }

@@ -596,6 +596,12 @@ int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx,
 int64_t deepep_ll_expected_rows(int num_tokens, int num_topk, int num_experts, int num_max_dispatch_tokens_per_rank,
                                 uint64_t observed);
 
+/* The same from the words of two dispatches, for calls whose batches differ from one to the next (layers that share
+ * the words): the geometric mean of what either leads to expect.  A word of 0, or of a batch with fewer tokens than
+ * this one when the other has as many, does not count. */
+int64_t deepep_ll_expected_rows_of_two(int num_tokens, int num_topk, int num_experts,
+                                       int num_max_dispatch_tokens_per_rank, uint64_t observed_a, uint64_t observed_b);
+
 /* deepep_ll_combine_send followed by deepep_ll_combine_recv, for a caller
  * whose remote experts' answers are already in combine_staging when the call
  * is made (the reference: Buffer::low_latency_combine,

@@ -101,6 +101,26 @@ def test_rows_expected_of_a_batch_follow_the_last_one(tokens, seen_tokens, seen_
         assert lib.deepep_ll_dispatch_is_single_launch(tokens, 8, 256, 128, got) == 1
 
 
+@pytest.mark.parametrize("tokens,a,b,want", [
+    (1000, (0, 0), (0, 0), 8000),
+    (1000, (1000, 160000), (0, 0), 160000),           # one report so far
+    (1000, (0, 0), (1000, 160000), 160000),
+    (1000, (1000, 160000), (1000, 160000), 160000),   # the same layer again
+    (1000, (1000, 160000), (1000, 10000), 40000),     # a hot layer and a cold one in turn: neither sizes the other
+    (1000, (1000, 10000), (1000, 160000), 40000),
+    (1000, (1000, 160000), (1000, 500), 35777),       # less than balanced is balanced
+    (1000, (1000, 160000), (3, 500), 160000),         # a smaller batch says nothing of a larger one
+    (1000, (3, 500), (1000, 160000), 160000),
+    (1000, (3, 500), (4, 50000), 20000),              # unless there is nothing else
+    (4, (1000, 60000), (1000, 60000), 240),           # the decode step behind a prefill
+    (4, (1000, 60000), (4, 60), 120),
+])
+def test_rows_expected_of_a_batch_lie_between_the_last_two(tokens, a, b, want):
+    from deepep_efa_amd import _capi
+    got = _capi.load().deepep_ll_expected_rows_of_two(tokens, 8, 256, 1024, a[0] << 32 | a[1], b[0] << 32 | b[1])
+    assert got == want
+
+
 @pytest.mark.parametrize("flag,taken", [
     (True, True), (False, True), (None, True), (1, True), (np.bool_(False), True), (0.0, True),
     ("False", False), ([], False), ((1,), False), ({}, False)])
