@@ -539,8 +539,11 @@ inline int64_t flat_rows_expected(int64_t expected_rows, int64_t max_rows) {
 inline void launch_rows_flat(const int32_t* total, const RowDesc* desc, int64_t max_rows, int64_t expected_rows,
                              const void* src, int64_t src_stride, int num_vec, void* dst, void* dst_own,
                              int64_t dst_stride, const FlatTails* tails, hipStream_t stream) {
-    // many short rows: two a workgroup are 1 % faster (160000 x 7168 bytes 383 -> 378 us; 28672: 65.7 -> 66.3)
-    const bool pairs = expected_rows > 65536 && num_vec <= 512;
+    // Many rows of up to 4 KB with scales and a source index: two a workgroup, where the descriptor and the tail are as
+    // many instructions as the payload.  Microseconds, one a workgroup / two, in two processes: 160000 x 2048 bytes 114.3 /
+    // 106.9 and 115.9 / 110.7, 4096 bytes 215.6 / 209.5 and 215.6 / 208.5; 20000 x 4096 32.4 / 32.0.  7168 bytes 348.0 / 343.7
+    // in one process, 345.8 / 353.5 in the other.  Without tails no width gains: 7168 bytes 348.3 / 355.5 and 342.5 / 353.1.
+    const bool pairs = tails != nullptr && expected_rows > 65536 && num_vec <= 256;
     const int others = tails != nullptr ? kWave : 0, threads = flat_row_threads(num_vec, 1024 - others);
     const unsigned grid = flat_grid_blocks(pairs ? expected_rows / 2 : expected_rows, max_rows, threads + others);
 #define DEEPEP_LAUNCH_ROWS(TAILS)                                                                                     \
