@@ -303,7 +303,10 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
 // csrc/transport/ll_pipeline.cpp:1283-1295; the reference's peer stores:
 // coop_combine_send.cuh:205-246).  One workgroup per record, walked like the rows of ll_rows_flat_kernel: HBM
 // bounds it, and neighbouring records are neighbouring rows on both sides.  Up to 512 threads: with twice the trips in
-// front of a row that one has, 896 for a row of 14336 bytes are the slower form (16376 rows 77 us, 1024 rows 6.9).
+// front of a row that a described one has, 896 for a row of 14336 bytes are the slower form behind an ordered receive
+// (16376 rows 77 us against 75.4, 1024 rows 6.9 against 6.4), until the rows are so many that a vector a thread pays as it
+// does there: 40000 rows 176 us with up to 512 threads and 171.6 with 896, 160000 746 and 693 (two vectors a thread 755),
+// 320000 1537 and 1399.
 // 16376 rows of 14336 bytes 78.7 -> 75.4 us (6.2 TB/s), 1024 rows 7.7 -> 6.4, against two vectors a thread and the
 // record behind the number of records.
 // ---------------------------------------------------------------------
@@ -567,10 +570,11 @@ int deepep_ll_combine_send_by_dest(const void* x, const int32_t* record_packed_r
     peers.peer_recv = reinterpret_cast<uint8_t* const*>(peer_recv_flat), peers.peer_rows = peer_recv_rows;
     peers.recv_counts = recv_counts, peers.remote_offset = combine_remote_recv_offset;
     peers.source_rank = source_rank, peers.num_ranks = num_ranks;
-    const int num_vec = hidden * 2 / 16, threads = flat_row_threads(num_vec, 512);
     // grid from the rows expected, not from the capacity (an idle workgroup is not free)
     const int64_t rows = expected_rows > 0 && expected_rows < row_capacity ? expected_rows : row_capacity;
-    const unsigned grid = flat_grid_blocks(flat_rows_expected(expected_rows, row_capacity), row_capacity, threads);
+    const int64_t sized_for = flat_rows_expected(expected_rows, row_capacity);
+    const int num_vec = hidden * 2 / 16, threads = flat_row_threads(num_vec, sized_for > 32768 ? 1024 : 512);
+    const unsigned grid = flat_grid_blocks(sized_for, row_capacity, threads);
     const int64_t x_rows = std::min(int64_t(num_experts) * num_max_dispatch_tokens_per_rank, int64_t(1) << 31);
 #define DEEPEP_LAUNCH_BY_DEST(STREAM, PEERS)                                                                            \
     ll_combine_send_by_dest_kernel<STREAM, PEERS><<<grid, threads, 0, reinterpret_cast<hipStream_t>(stream)>>>(         \

@@ -1589,6 +1589,27 @@ def test_return_by_destination_over_record_counts(rt, records, hidden):
     assert torch.equal(out.cpu(), want)
 
 
+@pytest.mark.parametrize("hidden", [8192, 16512])  # a round of 1024 threads, and more than two
+@pytest.mark.parametrize("records,hint", [(700, 32768), (700, 32769), (33792 + 257, 32769)])  # the last has more than workgroups
+def test_return_by_destination_of_many_records(rt, records, hidden, hint):
+    """Past 32768 expected records a row takes up to 1024 threads instead of 512."""
+    e, r, capacity = 8, 4, 34400
+    g = torch.Generator(device="cuda").manual_seed(records + hidden)
+    x = torch.randint(-2 ** 15, 2 ** 15, (capacity, hidden), dtype=torch.int16, device="cuda", generator=g)
+    packed, padded, offset = (torch.randperm(capacity, device="cuda", generator=g).int() for _ in range(3))
+    packed[::5] = -1
+    out = torch.full((capacity, hidden), 3, dtype=torch.int16, device="cuda")
+    num = torch.tensor([records, records], dtype=torch.int32, device="cuda")
+    rt.capi.check(rt.capi.load().deepep_ll_combine_send_by_dest(
+        rt.capi.ptr(x), rt.capi.ptr(packed), None, rt.capi.ptr(padded), rt.capi.ptr(offset), rt.capi.ptr(num), capacity, hidden, e,
+        r, capacity // e, rt.capi.ptr(out), None, None, None, None, hint, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    rows, to = packed[padded[:records].long()].long(), offset[:records].long()
+    want = torch.full_like(out, 3)
+    want[to[rows >= 0]] = x[rows[rows >= 0]]
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("records", [1000, 16384 + 256, 20000])
 def test_return_by_destination_with_room_for_a_million_records_and_no_hint(rt, records):
     """Every record is moved, also those past the 16384 workgroups, and none of the room is paid for: 820 us for 1000
