@@ -539,11 +539,12 @@ inline int64_t flat_rows_expected(int64_t expected_rows, int64_t max_rows) {
 inline void launch_rows_flat(const int32_t* total, const RowDesc* desc, int64_t max_rows, int64_t expected_rows,
                              const void* src, int64_t src_stride, int num_vec, void* dst, void* dst_own,
                              int64_t dst_stride, const FlatTails* tails, hipStream_t stream) {
-    // Many rows of up to 4 KB with scales and a source index: two a workgroup, where the descriptor and the tail are as
-    // many instructions as the payload.  Microseconds, one a workgroup / two, in two processes: 160000 x 2048 bytes 114.3 /
-    // 106.9 and 115.9 / 110.7, 4096 bytes 215.6 / 209.5 and 215.6 / 208.5; 20000 x 4096 32.4 / 32.0.  7168 bytes 348.0 / 343.7
-    // in one process, 345.8 / 353.5 in the other.  Without tails no width gains: 7168 bytes 348.3 / 355.5 and 342.5 / 353.1.
-    const bool pairs = tails != nullptr && expected_rows > 65536 && num_vec <= 256;
+    // Past 65536 rows that carry a source index (and scales), two a workgroup while they are up to 10 KB.  Microseconds of
+    // a skewed dispatch of 166336 rows, one a workgroup / two, in three processes: 2048 bytes 136 to 138 / 126 to 129,
+    // 4096 263 to 266 / 243 to 249, 7168 404 to 411 / 397 to 406, bf16 10240 557 to 564 / 538 to 555, but 14336 747 to 755 /
+    // 739 to 773; of 83055 rows 74 / 70, 129 / 123, 205 / 207, 284 / 276, 378 / 388.  Without tails two gain nothing (the
+    // return of 4096 bytes 221.5 / 224, 8192 430 / 443, 14336 745 / 753).
+    const bool pairs = tails != nullptr && expected_rows > 65536 && num_vec <= 640;
     const int others = tails != nullptr ? kWave : 0, threads = flat_row_threads(num_vec, 1024 - others);
     const unsigned grid = flat_grid_blocks(pairs ? expected_rows / 2 : expected_rows, max_rows, threads + others);
 #define DEEPEP_LAUNCH_ROWS(TAILS)                                                                                     \
