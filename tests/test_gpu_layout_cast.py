@@ -596,6 +596,30 @@ def test_combine_reduce_of_a_buffer_past_the_caches(capi, t, h):
     assert torch.equal(out_w.cpu(), chain_w)
 
 
+# 10, 19 and 2 pieces: 3, 5 and 1 workgroups of four waves a token up to 3.5 rows of it, 2, 3 and 1 larger ones above
+@pytest.mark.parametrize("t,h", [(7000, 4616), (3600, 9224), (60000, 520)])
+@pytest.mark.parametrize("copies", [3.5, 3.51])
+def test_combine_reduce_past_the_caches_by_copies_a_token(capi, t, h, copies):
+    lib = capi.load()
+    r, rows = 8, int(t * copies)
+    g = torch.Generator(device="cuda").manual_seed(t)
+    recv = torch.randn((rows, h), device="cuda", generator=g).bfloat16()
+    assert rows * h * 2 > 192 << 20
+    table = torch.full((t, r), -1, dtype=torch.int32, device="cuda")  # row_of_pair; 3 rows a token, none for every 50th
+    for i in range(3):
+        table[:, (5 * i + 1) % r] = torch.randperm(t, device="cuda", generator=g).int() + i * (rows // 3 - t)
+    table[::50] = -1
+    is_in, some = table >= 0, torch.zeros(r + 1, dtype=torch.int64, device="cuda")
+    out = torch.full((t + 1, h), 7.0, dtype=torch.bfloat16, device="cuda")
+    capi.check(lib.deepep_combine_reduce(capi.ptr(recv), None, capi.ptr(some), capi.ptr(some), capi.ptr(is_in), None, None, t, h,
+                                         0, r, rows, capi.ptr(table), capi.ptr(out), None, None, 0, stream()))
+    torch.cuda.synchronize()
+    want = torch.zeros((t, h), device="cuda")
+    for i in range(r):  # float32, ranks ascending, rounded once
+        want += torch.where(is_in[:, i:i + 1], recv[table[:, i].clamp(min=0).long()].float(), 0.0)
+    assert torch.equal(out[:t], want.bfloat16()) and bool((out[t] == 7.0).all())
+
+
 @pytest.mark.parametrize("seed", range(int(os.environ.get("DEEPEP_TEST_RANDOM_SHAPES", "16"))))
 def test_pack_remap_reduce_seeded_random_shapes(capi, seed):
     """Pack, top-k remap and the combine reduce on shapes nobody picked by hand: odd rank counts, ragged
