@@ -574,10 +574,14 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // against one, 205 and 273 us for 512 threads and for whole rows; three or four 186 to 195, and 28.4 and 29.5 for rows
 // of 7168 bytes.
 // Groups of 6, 12, 24 and 48 MB: 230, 215, 211 and 207 us, but much is lost where their source rows no longer fit an L2
-// (4 MB): a whole prefill of 9000 x 7168 in fp8 to 8 ranks 262 us with 4.0 MB of source a group and 250 with 2.0, of 6000 x
+// (4 MB; of a source larger than what is packed, no more than that is read: 896 rows out of 3.1 GB 7.5 -> 5.9 us, 20000
+// 86 -> 83): a whole prefill of 9000 x 7168 in fp8 to 8 ranks 262 us with 4.0 MB of source a group and 250 with 2.0, of 6000 x
 // 14336 at top-6 188 and 173 with 5.4 and 2.7, of 7000 x 8192 127.3 and 125 with 3.4 and 1.7; 2.9 at 32 ranks gains (308
 // -> 302 against half).  Fewer than two groups an XCD lose a tenth, and two of more than 16 MB some: the pack of 7000 x 7168
-// in fp8 to 32 ranks behind its cast 68.5 us with 16 groups of 22 MB, 63.6 with 32.  The groups' rows drift apart by some fifty
+// in fp8 to 32 ranks behind its cast 68.5 us with 16 groups of 22 MB, 63.6 with 32.  Against 8 to 128 groups by force, 1500
+// to 12000 rows of 2 to 14 KB, 3.3 to 7.3 copies: past 128 MB these bounds are within 2 % of the best everywhere; below,
+// on four sets of tensors in turn, 8 groups are up to 96 MB (7168 x 8 ranks: 72 MB 17.4 us and 18.6 with 16, 88 MB 21.7 and
+// 22.6) and lose beyond (112 MB 30.5 and 28.0).  The groups' rows drift apart by some fifty
 // tokens, so a group reads half as much again as its share of the source.
 // Up to 256 threads while the rows stay in the caches: 600 x 14336 10.7 -> 10.1 us.  In list order, past them, the same
 // threads move one vector at a time: two trips to memory stand in front of a row there.  4096 x 14336 88.5 us against 96.1
@@ -865,8 +869,9 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
     const int threads = a.threads;
     if (grouped) {
         int group_log2 = 3;  // the fewer groups an XCD, the smaller, and no group's source rows larger than fit its L2
+        const int64_t source_rows = max_rows < num_src_rows ? max_rows : num_src_rows;  // that can be read
         while (((max_rows * row_bytes) >> group_log2) > kPackGroupBytes * (group_log2 < 5 ? group_log2 : 6) / 3 ||
-               ((int64_t(num_src_rows) * row_bytes) >> group_log2) > kPackSourceBytes)
+               ((source_rows * row_bytes) >> group_log2) > kPackSourceBytes)
             if (++group_log2 == 16) break;
         // rounding down the parts of every rank's list can put one more row per rank into a group
         const int64_t needed = ((max_rows + (int64_t(1) << group_log2) - 1) >> group_log2) + num_ranks;

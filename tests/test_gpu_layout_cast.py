@@ -353,6 +353,23 @@ def test_pack_rows_by_rank(capi, rows, row_bytes, scale_bytes, r, odds, keep):
         assert torch.equal(dsc[:n].cpu(), sc[ids[:n]]) and (dsc[n:] == 0xEE).all()
 
 
+@pytest.mark.parametrize("r,per_rank", [(8, 100), (8, 113), (64, 13), (3, 3000)])  # below one group's worth, then grouped
+def test_pack_few_rows_of_a_large_source(capi, r, per_rank):
+    """The groups are bound by the rows that are packed, not by the tensor they come from."""
+    lib = capi.load()
+    rows, row_bytes, n = 40000, 16384, r * per_rank
+    g = torch.Generator(device="cuda").manual_seed(n)
+    src = torch.randint(-2 ** 31, 2 ** 31 - 1, (rows, row_bytes // 4), dtype=torch.int32, device="cuda", generator=g)
+    ids = torch.cat([torch.randperm(rows, device="cuda", generator=g)[:per_rank].sort()[0] for _ in range(r)])
+    cumsum = torch.arange(r + 1, device="cuda") * per_rank
+    dst = torch.full((n + 1, row_bytes // 4), 7, dtype=torch.int32, device="cuda")
+    capi.check(lib.deepep_pack_rows_by_rank(
+        capi.ptr(src), None, capi.ptr(ids), cumsum.data_ptr() + 8 * r, capi.ptr(cumsum), r, n, rows, row_bytes, 0, capi.ptr(dst),
+        None, stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(dst[:n], src[ids]) and bool((dst[n] == 7).all())
+
+
 @pytest.mark.parametrize("rows", [1000, 4000])
 @pytest.mark.parametrize("first", [0, 1, 5, 8])
 def test_pack_rows_packs_the_whole_list(rows, first):
