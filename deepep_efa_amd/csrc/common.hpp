@@ -136,6 +136,10 @@ __device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_flo
 
 // The next kRows rows that `live` names, for the 8 channels at byte `off` of each: lane i holds row i's address and
 // weight.
+// add() takes one row after the other: left to itself the compiler widens all of them ahead of the sums, 32 registers more
+// than the rows hold (ll_combine_recv_kernel 78 against 50, ll_combine_fused_kernel 76 against 57), and six waves fit a
+// SIMD instead of eight.  A combine of 128 tokens no longer fits the chip then: its last workgroups start 4.9 us into a
+// kernel of 5.9, against 1.7 (the kernel takes 10.3 us either way; 9.4 -> 9.0 for 509 tokens).
 template <int kRows>
 struct RowsInFlight {
     u32x4 v[kRows];
@@ -156,7 +160,7 @@ struct RowsInFlight {
     template <bool kWeighted>
     __device__ __forceinline__ void add(float (&acc)[8]) const {
 #pragma unroll
-        for (int u = 0; u < kRows; ++u)
+        for (int u = 0; u < kRows; ++u) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if constexpr (kWeighted) {
@@ -166,6 +170,8 @@ struct RowsInFlight {
                     acc[2 * i] += bf16_lo(v[u][i]), acc[2 * i + 1] += bf16_hi(v[u][i]);
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 };
 

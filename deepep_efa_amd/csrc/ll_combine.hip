@@ -44,12 +44,13 @@ __device__ __forceinline__ void combine_send_rows_impl(const CombineSendArgs& a,
     int64_t ranges[kPer];
     DEEPEP_PHASE(0);
     wave_load_int64<kPer>(a.layout_range, num_segments, lane, ranges);
+    int source = lane * kPer - a.expert_of(lane * kPer) * num_ranks;  // of segment lane * kPer + u
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-        const int s = lane * kPer + u;
         int c = int(ranges[u] & 0xffffffffll);
         c = c < 0 ? 0 : (c > max_tokens ? max_tokens : c);
-        if (skip_own && s - a.expert_of(s) * num_ranks == a.rank) c = 0;
+        if (skip_own && source == a.rank) c = 0;
+        source = source + 1 == num_ranks ? 0 : source + 1;
         seg_table.cnt[u] = c;
         seg_table.aux[u] = int(ranges[u] >> 32);
     }

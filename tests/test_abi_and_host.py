@@ -80,6 +80,27 @@ def test_host_argument_checks_without_a_gpu():
         _capi.check(rc)
 
 
+def _kernel_metadata():
+    """name -> metadata of every kernel in the built library: the msgpack notes of its code objects."""
+    msgpack = pytest.importorskip("msgpack")
+    blob = open(os.path.join(ROOT, "deepep_efa_amd", "libdeepep_hip.so"), "rb").read()
+    kernels = {}
+    for m in re.finditer(rb"\x07\0\0\0(....)\x20\0\0\0AMDGPU\0\0", blob, re.S):  # note: name size, data size, type 32, name
+        note = blob[m.end():m.end() + int.from_bytes(m.group(1), "little")]
+        for k in msgpack.unpackb(note, strict_map_key=False)["amdhsa.kernels"]:
+            kernels[k[".name"]] = k
+    return kernels
+
+
+@pytest.mark.parametrize("kernel", ["ll_combine_fused_kernel", "ll_combine_recv_kernel", "combine_reduce_kernel"])
+def test_reduces_leave_room_for_eight_waves_a_simd(kernel):
+    """512 registers a lane and SIMD, eight waves: 64 each, and none kept in memory instead."""
+    found = [k for name, k in _kernel_metadata().items() if kernel in name]
+    assert len(found) == 2
+    for k in found:
+        assert k[".vgpr_count"] <= 64 and k[".private_segment_fixed_size"] == 0, k[".name"]
+
+
 @pytest.mark.parametrize("tokens,seen_tokens,seen_rows,want", [
     (128, 0, 0, 1024),          # nothing seen yet: what a balanced world sends
     (0, 0, 0, 8),
