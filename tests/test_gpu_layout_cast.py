@@ -613,6 +613,32 @@ def test_combine_reduce_of_a_buffer_past_the_caches(capi, t, h):
     assert torch.equal(out_w.cpu(), chain_w)
 
 
+def test_combine_reduce_of_ties_infinities_and_nan(capi):
+    """Every pair of special values as the sum of two ranks' rows: zeros, subnormals, half a step beside 1 and beside the
+    largest value, infinities, quiet and signalling NaN."""
+    lib = capi.load()
+    special = [0x0000, 0x8000, 0x0001, 0x8001, 0x007F, 0x0080, 0x3F80, 0xBF80, 0x3F81, 0x3F82, 0x3B80, 0xBB80, 0x7F7F, 0xFF7F,
+               0x7B00, 0xFB00, 0x7F80, 0xFF80, 0x7FC0, 0x7F81, 0xFFFF]
+    v = torch.tensor(special, dtype=torch.int32).short().view(torch.bfloat16)
+    a, b = (m.reshape(-1) for m in torch.meshgrid(v, v, indexing="ij"))
+    h = 448
+    rows = torch.zeros((2, h), dtype=torch.bfloat16)
+    rows[0, :a.numel()], rows[1, :a.numel()] = a, b
+    dev = [rows.cuda(), torch.tensor([0, 0]).cuda(), torch.tensor([0, 1, 2]).cuda(), torch.ones((1, 2), dtype=torch.bool).cuda()]
+    table = torch.tensor([[0, 1]], dtype=torch.int32).cuda()
+    out = torch.empty((1, h), dtype=torch.bfloat16, device="cuda")
+    capi.check(lib.deepep_combine_reduce(capi.ptr(dev[0]), None, *[capi.ptr(d) for d in dev[1:]], None, None, 1, h, 0, 2, 2,
+                                         capi.ptr(table), capi.ptr(out), None, None, 0, stream()))
+    torch.cuda.synchronize()
+    want = (rows[0].float() + 0.0) + rows[1].float()
+    bits = want.view(torch.int32).long() & 0xFFFFFFFF
+    bits = (bits + 0x7FFF + ((bits >> 16) & 1)) >> 16  # to nearest, ties to even
+    got = out[0].cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    number = ~want.isnan()
+    assert torch.equal(got.view(torch.int16)[number].long() & 0xFFFF, bits[number])
+
+
 # 10, 19 and 2 pieces: 3, 5 and 1 workgroups of four waves a token up to 3.5 rows of it, 2, 3 and 1 larger ones above
 @pytest.mark.parametrize("t,h", [(7000, 4616), (3600, 9224), (60000, 520)])
 @pytest.mark.parametrize("copies", [3.5, 3.51])

@@ -607,6 +607,70 @@ def test_combine_random_expert_outputs(rt, oracle_c, r, rank, t, h, k, e, one_ca
 
 
 @ONE_CALL
+def bf16_bits_of(x):
+    """float32 -> bf16 bits by integer arithmetic, to nearest with ties to even; any NaN as 0x7FC0."""
+    b = x.contiguous().view(torch.int32).long() & 0xFFFFFFFF
+    r = (b + 0x7FFF + ((b >> 16) & 1)) >> 16
+    return torch.where(x.isnan(), torch.full_like(r, 0x7FC0), r).int()
+
+
+def bf16_bits(x):
+    return torch.where(x.isnan(), torch.full(x.shape, 0x7FC0, dtype=torch.int32, device=x.device), x.view(torch.int16).int() & 0xFFFF)
+
+
+def reduce_rows(rt, staging, topk_weights, out):
+    """combine_recv of one expert's rows: token t adds up weight * row over the selections, rows 0, 1, .. in turn."""
+    t, k = topk_weights.shape
+    slot = torch.arange(k, dtype=torch.int32, device="cuda").repeat(t, 1).contiguous()
+    expert = torch.zeros((t, k), dtype=torch.int64, device="cuda")
+    rt.capi.check(rt.capi.load().deepep_ll_combine_recv(
+        rt.capi.ptr(staging), rt.capi.ptr(expert), rt.capi.ptr(topk_weights), rt.capi.ptr(slot), t, staging.shape[1], k, 1,
+        staging.shape[0], 0, rt.capi.ptr(out), torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+
+
+def test_combine_rounds_every_float_to_the_nearest_bf16(rt):
+    """Sums that take every float32 value of a normal size: each is three bf16 values added without a rounding.  The values
+    too small for that, infinities and NaN follow as weights of a row of ones, one lower half for each way to round."""
+    n = 1 << 24
+    one, low = torch.ones((1, 3), device="cuda"), torch.arange(n, dtype=torch.int64, device="cuda")
+    out = torch.empty((1, n), dtype=torch.bfloat16, device="cuda")
+    for top in range(256):
+        bits = (low + (top << 24))
+        exponent = (bits >> 23) & 255
+        bits = torch.where((exponent >= 24) & (exponent < 255), bits, 0x3F800000 + (bits & 0x7FFFFF))
+        x = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).int().view(torch.float32)
+        high = (x.view(torch.int32) & -65536).view(torch.float32)
+        middle = ((x - high).view(torch.int32) & -65536).view(torch.float32)
+        rows = torch.stack([v.view(torch.int32) >> 16 for v in (high, middle, x - high - middle)]).short().view(torch.bfloat16)
+        reduce_rows(rt, rows, one, out)
+        assert torch.equal(bf16_bits(out[0]), bf16_bits_of(x)), hex(top)
+    upper = torch.arange(65536, dtype=torch.int64, device="cuda").view(-1, 1) << 16
+    bits = (upper + torch.tensor([0, 1, 0x7FFF, 0x8000, 0x8001, 0xFFFF], device="cuda")).view(-1, 1)
+    w = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).int().view(torch.float32)
+    out = torch.empty((w.shape[0], 128), dtype=torch.bfloat16, device="cuda")
+    reduce_rows(rt, torch.ones((1, 128), dtype=torch.bfloat16, device="cuda"), w, out)
+    want = bf16_bits_of(torch.where(w == 0, 0.0, w))  # +0 + -0 is +0
+    assert torch.equal(bf16_bits(out), want.expand(-1, 128))
+
+
+# zeros, the smallest and largest subnormal, the smallest normal, 1, the next two and half a step, the largest and half a
+# step of it, infinities, a quiet and two signalling NaN
+SPECIAL = [0x0000, 0x8000, 0x0001, 0x8001, 0x007F, 0x0080, 0x3F80, 0xBF80, 0x3F81, 0x3F82, 0x3B80, 0xBB80, 0x7F7F, 0xFF7F, 0x7B00,
+           0xFB00, 0x7F80, 0xFF80, 0x7FC0, 0x7F81, 0xFFFF]
+
+
+def test_combine_of_ties_infinities_and_nan(rt):
+    """Every pair of special values as one sum of two rows."""
+    v = torch.tensor(SPECIAL, dtype=torch.int32).short().view(torch.bfloat16)
+    a, b = (m.reshape(-1) for m in torch.meshgrid(v, v, indexing="ij"))
+    rows = torch.zeros((2, 512), dtype=torch.bfloat16)
+    rows[0, :a.numel()], rows[1, :a.numel()] = a, b
+    out = torch.empty((1, 512), dtype=torch.bfloat16, device="cuda")
+    reduce_rows(rt, rows.cuda(), torch.ones((1, 2), device="cuda"), out)
+    assert torch.equal(bf16_bits(out[0]).cpu(), bf16_bits_of((rows[0].float() + 0.0) + rows[1].float()))
+
+
 @pytest.mark.parametrize("e,rank", [(256, 11), (288, 7)])  # 288 experts: the reference's own LL test, nine per rank
 def test_ll_config_full_size(rt, one_call, e, rank):
     """One GPU's share of EP=32 at 128 tokens x 7168, top-8 of 256 (or 288) experts, seeded world."""
