@@ -606,7 +606,6 @@ def test_combine_random_expert_outputs(rt, oracle_c, r, rank, t, h, k, e, one_ca
     assert O.calc_diff(got, ref) < 1e-5
 
 
-@ONE_CALL
 def bf16_bits_of(x):
     """float32 -> bf16 bits by integer arithmetic, to nearest with ties to even; any NaN as 0x7FC0."""
     b = x.contiguous().view(torch.int32).long() & 0xFFFFFFFF
@@ -671,6 +670,7 @@ def test_combine_of_ties_infinities_and_nan(rt):
     assert torch.equal(bf16_bits(out[0]).cpu(), bf16_bits_of((rows[0].float() + 0.0) + rows[1].float()))
 
 
+@ONE_CALL
 @pytest.mark.parametrize("e,rank", [(256, 11), (288, 7)])  # 288 experts: the reference's own LL test, nine per rank
 def test_ll_config_full_size(rt, one_call, e, rank):
     """One GPU's share of EP=32 at 128 tokens x 7168, top-8 of 256 (or 288) experts, seeded world."""
