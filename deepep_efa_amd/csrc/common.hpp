@@ -136,10 +136,9 @@ __device__ __forceinline__ float bf16_hi(uint32_t packed) { return __uint_as_flo
 
 // The next kRows rows that `live` names, for the 8 channels at byte `off` of each: lane i holds row i's address and
 // weight.
-// add() takes one row after the other: left to itself the compiler widens all of them ahead of the sums, 32 registers more
-// than the rows hold (ll_combine_recv_kernel 78 against 50, ll_combine_fused_kernel 76 against 57), and six waves fit a
-// SIMD instead of eight.  A combine of 128 tokens no longer fits the chip then: its last workgroups start 4.9 us into a
-// kernel of 5.9, against 1.7 (the kernel takes 10.3 us either way; 9.4 -> 9.0 for 509 tokens).
+// kInTurn: add() widens one row after the other.  Left to itself the compiler widens all of them ahead of the sums, 32
+// registers more than the rows hold (ll_combine_recv_kernel 78 against 50, ll_combine_fused_kernel 76 against 57), and six
+// waves fit a SIMD instead of eight.
 template <int kRows>
 struct RowsInFlight {
     u32x4 v[kRows];
@@ -157,7 +156,7 @@ struct RowsInFlight {
             v[u] = load_row_u32x4<kStream>(row_buffer(row, row_bytes), off);
         }
     }
-    template <bool kWeighted>
+    template <bool kInTurn, bool kWeighted>
     __device__ __forceinline__ void add(float (&acc)[8]) const {
 #pragma unroll
         for (int u = 0; u < kRows; ++u) {
@@ -170,14 +169,14 @@ struct RowsInFlight {
                     acc[2 * i] += bf16_lo(v[u][i]), acc[2 * i + 1] += bf16_hi(v[u][i]);
                 }
             }
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (kInTurn) __builtin_amdgcn_sched_barrier(0);
         }
     }
 };
 
 // acc += weight * row (or row) over the rows that `live` names, in ascending order.  Eight rows are in flight, then what
 // is left of eight together; without a branch for each row, which costs a wave as much as the row's arithmetic.
-template <bool kStream, bool kWeighted>
+template <bool kStream, bool kWeighted, bool kInTurn>
 __device__ __forceinline__ void add_rows(uint64_t address, float weight, uint64_t live, int off, int row_bytes,
                                          float (&acc)[8]) {
     int n = __popcll(live);
@@ -185,7 +184,7 @@ __device__ __forceinline__ void add_rows(uint64_t address, float weight, uint64_
         RowsInFlight<8> rows;
         rows.load<kStream, kWeighted>(address, weight, live, off, row_bytes);
         __builtin_amdgcn_sched_barrier(0);  // no row's arithmetic, and so its wait, in front of another's load
-        rows.add<kWeighted>(acc);
+        rows.add<kInTurn, kWeighted>(acc);
     }
     RowsInFlight<4> four;
     RowsInFlight<2> two;
@@ -194,9 +193,9 @@ __device__ __forceinline__ void add_rows(uint64_t address, float weight, uint64_
     if ((n & 2) != 0) two.load<kStream, kWeighted>(address, weight, live, off, row_bytes);
     if ((n & 1) != 0) one.load<kStream, kWeighted>(address, weight, live, off, row_bytes);
     __builtin_amdgcn_sched_barrier(0);
-    if ((n & 4) != 0) four.add<kWeighted>(acc);
-    if ((n & 2) != 0) two.add<kWeighted>(acc);
-    if ((n & 1) != 0) one.add<kWeighted>(acc);
+    if ((n & 4) != 0) four.add<kInTurn, kWeighted>(acc);
+    if ((n & 2) != 0) two.add<kInTurn, kWeighted>(acc);
+    if ((n & 1) != 0) one.add<kInTurn, kWeighted>(acc);
 }
 
 // Threads [0, threads) of a workgroup move a row, kVecs vectors of each in flight; wider rows go round.

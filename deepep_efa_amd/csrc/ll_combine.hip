@@ -151,7 +151,7 @@ __device__ __forceinline__ CombineSelection combine_load_selection(const Combine
     return s;
 }
 
-template <bool kStream>
+template <bool kStream, bool kInTurn>
 __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, uint32_t t, uint32_t piece,
                                                    const CombineSelection& sel, const uint8_t* own_x,
                                                    const int32_t* own_begin, int own_first_expert,
@@ -211,7 +211,7 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, uin
     }
 
     DEEPEP_PHASE(1);
-    add_rows<kStream, true>(my_row, my_weight, live_mask, off, int(row_bytes), acc);
+    add_rows<kStream, true, kInTurn>(my_row, my_weight, live_mask, off, int(row_bytes), acc);
     DEEPEP_PHASE(2);
     u32x4 o;
 #pragma unroll
@@ -227,6 +227,8 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, uin
 // (a launch of its own took 3 to 5 us of a large combine).
 // Streaming, a workgroup is one wave: nothing holds a wave's slot once it is done (4096 tokens, eight rows of 14336
 // bytes each, 90.5 -> 88.7 us, 6.0 TB/s; two to fourteen waves 91 to 95, neighbouring tokens on one XCD no gain).
+// Eight waves a SIMD while the rows stay in the caches: 820 to 1000 tokens of 5120 at top-4 4 % less than with six, else the
+// same.  Streaming, six serve HBM as well or better (87.5 us against 87.8 at 4096 tokens).
 template <bool kStream>
 __global__ __launch_bounds__(256) void ll_combine_recv_kernel(CombineRecvArgs a, const uint8_t* own_x,
                                                               const int64_t* layout_range, int rank,
@@ -248,8 +250,8 @@ __global__ __launch_bounds__(256) void ll_combine_recv_kernel(CombineRecvArgs a,
         }
         lds_barrier();
     }
-    combine_recv_piece<kStream>(a, t, piece, sel, own_x, own_x != nullptr ? own_begin : nullptr, rank * num_local_experts,
-                                num_local_experts, int64_t(a.max_tokens) * num_ranks);
+    combine_recv_piece<kStream, !kStream>(a, t, piece, sel, own_x, own_x != nullptr ? own_begin : nullptr,
+                                          rank * num_local_experts, num_local_experts, int64_t(a.max_tokens) * num_ranks);
 }
 
 __global__ __launch_bounds__(256) void ll_combine_index_kernel(CombineIndexArgs index) {
@@ -266,8 +268,15 @@ __global__ __launch_bounds__(256) void ll_combine_index_kernel(CombineIndexArgs 
 // row return only has to move the rows owed to other ranks.
 // (The reference's combine is one kernel with a send and a receive phase as
 // well: csrc/kernels/coop_combine_send.cuh:37, coop_combine_recv.cuh:72.)
+// kInTurn: eight waves a SIMD, for grids that the chip then holds at once.  128 tokens are 1616 to 1646 workgroups: with
+// six the last row returns start 4.9 us into a kernel of 5.9 (7.7 of 8.7 after a flush), with eight 1.7 (1.5).  A step of
+// 128 tokens takes the same, of 280 x 5120 at top-4 14.7 -> 14.0 us, 200 x 5120 at top-6 17.5 -> 16.4, 280 x 4096 21.2 -> 20.6,
+// 160 x 7168 to 32 ranks 20.7 -> 20.1.  Beyond one round it depends on how full the last one is: 1.1 to 1.5 rounds of eight
+// gain 2 to 4 %, 1.7 to 2.05 lose as much (577 x 5120 at top-4 29.1 -> 30.2), more than three lose 0 to 1 %: six there.
 // ---------------------------------------------------------------------
-template <bool kStream>
+constexpr int64_t kWorkgroupsAtOnce = 256 * 8;  // compute units, workgroups of four waves on each
+
+template <bool kStream, bool kInTurn>
 __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs sa, CombineRecvArgs ra,
                                                                int num_recv_blocks) {
     extern __shared__ int32_t dyn_lds[];  // reduce workgroups: own_begin[E_l]
@@ -283,8 +292,8 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
             dyn_lds[le] = (lr & 0xffffffffll) > 0 ? int(lr >> 32) : 0;
         }
         lds_barrier();
-        combine_recv_piece<kStream>(ra, t, piece, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
-                                    sa.num_local_experts, int64_t(sa.max_tokens) * sa.num_ranks);
+        combine_recv_piece<kStream, kInTurn>(ra, t, piece, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
+                                             sa.num_local_experts, int64_t(sa.max_tokens) * sa.num_ranks);
     } else {
         combine_send_rows<kStream>(sa, block - num_recv_blocks, int(gridDim.x) - num_recv_blocks, true);
     }
@@ -706,12 +715,13 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     // rows returned (read + written) plus rows gathered: past what the caches hold, stream.  Beside more than
     // kLargeBatchRows rows it always pays (11946 of 4 KB, 61.2 -> 57.5 us a step).
     const int64_t traffic = (2 * rows + int64_t(num_tokens) * num_topk) * hidden * 2;
-    if (large || traffic > stream_bytes())
-        ll_combine_fused_kernel<true><<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds,
-                                        reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks));
-    else
-        ll_combine_fused_kernel<false><<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds,
-                                         reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks));
+#define DEEPEP_LAUNCH_FUSED(STREAM, IN_TURN)                                                           \
+    ll_combine_fused_kernel<STREAM, IN_TURN><<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds,     \
+                                               reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks))
+    if (large || traffic > stream_bytes()) DEEPEP_LAUNCH_FUSED(true, false);
+    else if (recv_blocks + send_blocks <= kWorkgroupsAtOnce) DEEPEP_LAUNCH_FUSED(false, true);
+    else DEEPEP_LAUNCH_FUSED(false, false);
+#undef DEEPEP_LAUNCH_FUSED
     EP_LAUNCH_CHECK();
     return 0;
 }
