@@ -112,7 +112,7 @@ __global__ __launch_bounds__(kMetaThreads) void combine_positions_kernel(
 // kReduceWindow workgroups in a row, and a token's pieces to as few workgroups of about equal size as eight waves
 // allow: 12289 tokens of 14336 bytes at 8 ranks (1.1 GB) 184 -> 171 us (6.5 TB/s), 4096 61.0 -> 59.3, 9000 of 4096
 // bytes at 32 ranks 52.7 -> 50.6, against four waves in launch order; four waves in windows 175, whole tokens 174.  With
-// few copies a token a wave has few loads in flight and its workgroup's other waves wait for it less: four waves there.
+// few copies a token a wave has few loads in flight, and four waves at most are the better size.
 // 12000 tokens of 5120 channels, whole tokens / four waves, by the copies: 1.9 64.7 / 58.7 us, 2.65 74.4 / 70.4, 3.3
 // 84.0 / 82.3, 3.9 93.8 / 94.2, 4.4 103.5 / 106.7, 5.3 122 / 126; of 6144 3.3 99.4 / 99.0, 3.9 112 / 116; of 7168 1.0
 // 78.3 / 75.0, 1.9 86.4 / 83.7, 3.3 116.2 / 115.8, 3.9 130.3 / 129.9.  A
@@ -287,10 +287,9 @@ int deepep_combine_reduce(const void* recv_x, const float* recv_topk_weights, co
     }
     const int pieces = (hidden * 2 + 1023) / 1024;
     const bool stream_rows = max_rows * hidden * 2 > stream_bytes();
-    // a token's pieces over workgroups of equal size, or, up to 3.5 copies a token, of four waves
-    const bool whole = stream_rows && 2 * max_rows > 7 * int64_t(num_tokens);
-    const int fewest = (pieces + 7) / 8, waves = whole ? (pieces + fewest - 1) / fewest : 4;
-    const int per_token = (pieces + waves - 1) / waves;
+    // a token's pieces over as few workgroups of about equal size as eight waves allow, or, up to 3.5 copies, four
+    const int most = 2 * max_rows > 7 * int64_t(num_tokens) ? 8 : 4;
+    const int per_token = (pieces + most - 1) / most, waves = stream_rows ? (pieces + per_token - 1) / per_token : 4;
     int64_t blocks = stream_rows ? int64_t(num_tokens) * per_token : (int64_t(num_tokens) * pieces + waves - 1) / waves;
     if (stream_rows) blocks = (blocks + kReduceRound - 1) / kReduceRound * kReduceRound;
     EP_HOST_ASSERT(blocks < (int64_t(1) << 31) && int64_t(num_tokens) * pieces < (int64_t(1) << 32));

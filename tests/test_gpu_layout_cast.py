@@ -639,7 +639,7 @@ def test_combine_reduce_of_ties_infinities_and_nan(capi):
     assert torch.equal(got.view(torch.int16)[number].long() & 0xFFFF, bits[number])
 
 
-# 10, 19 and 2 pieces: 3, 5 and 1 workgroups of four waves a token up to 3.5 rows of it, 2, 3 and 1 larger ones above
+# 10, 19 and 2 pieces: 3, 5 and 1 workgroups of up to four waves a token up to 3.5 rows of it, 2, 3 and 1 of up to eight above
 @pytest.mark.parametrize("t,h", [(7000, 4616), (3600, 9224), (60000, 520)])
 @pytest.mark.parametrize("copies", [3.5, 3.51])
 def test_combine_reduce_past_the_caches_by_copies_a_token(capi, t, h, copies):
