@@ -539,12 +539,13 @@ inline int64_t flat_rows_expected(int64_t expected_rows, int64_t max_rows) {
 inline void launch_rows_flat(const int32_t* total, const RowDesc* desc, int64_t max_rows, int64_t expected_rows,
                              const void* src, int64_t src_stride, int num_vec, void* dst, void* dst_own,
                              int64_t dst_stride, const FlatTails* tails, hipStream_t stream) {
-    // Past 65536 rows that carry a source index (and scales), two a workgroup while they are up to 10 KB.  Microseconds of
+    // Past 65536 rows two a workgroup, while they carry a source index (and scales) and are up to 10 KB.  Microseconds of
     // a skewed dispatch of 166336 rows, one a workgroup / two, in three processes: 2048 bytes 136 to 138 / 126 to 129,
     // 4096 263 to 266 / 243 to 249, 7168 404 to 411 / 397 to 406, bf16 10240 557 to 564 / 538 to 555, but 14336 747 to 755 /
-    // 739 to 773; of 83055 rows 74 / 70, 129 / 123, 205 / 207, 284 / 276, 378 / 388.  Without tails two gain nothing (the
-    // return of 4096 bytes 221.5 / 224, 8192 430 / 443, 14336 745 / 753).
-    const bool pairs = tails != nullptr && expected_rows > 65536 && num_vec <= 640;
+    // 739 to 773; of 83055 rows 74 / 70, 129 / 123, 205 / 207, 284 / 276, 378 / 388.  Without tails below 2 KB (160000
+    // rows of 256 bytes 40.2 / 29.6, 512 40.3 / 34.2, 1024 55.8 / 55.7, 1280 74.6 / 69.0); two gain nothing beyond (2048 104.0 /
+    // 104.4, 4096 221.5 / 224, 8192 430 / 443, 14336 745 / 753).
+    const bool pairs = expected_rows > 65536 && num_vec <= (tails != nullptr ? 640 : 127);
     const int others = tails != nullptr ? kWave : 0, threads = flat_row_threads(num_vec, 1024 - others);
     const unsigned grid = flat_grid_blocks(pairs ? expected_rows / 2 : expected_rows, max_rows, threads + others);
 #define DEEPEP_LAUNCH_ROWS(TAILS)                                                                                     \

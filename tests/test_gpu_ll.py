@@ -1711,6 +1711,7 @@ def test_return_by_destination_with_room_for_a_million_records_and_no_hint(rt, r
     (33, 128, O.ROW_FP8, 8193), (33, 15488, O.ROW_FP8, 8193),  # the grid is far larger than the rows; two trips a row
     (40, 8320, O.ROW_BF16, 9000), (1300, 512, O.ROW_FP8_UE8M0, 8193),  # more rows than workgroups
     (4700, 128, O.ROW_FP8, 65537),  # two rows a workgroup, and more than that
+    (300, 1024, O.ROW_BF16, 65537), (300, 5120, O.ROW_BF16, 65537), (300, 5248, O.ROW_BF16, 65537),  # where one and two meet
 ])
 def test_row_copies_over_widths_and_hints(rt, t, h, fmt, hint):
     """The flat row copy of both directions, every row and every byte around it."""
