@@ -583,17 +583,18 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // on four sets of tensors in turn, 8 groups are up to 96 MB (7168 x 8 ranks: 72 MB 17.4 us and 18.6 with 16, 88 MB 21.7 and
 // 22.6) and lose beyond (112 MB 30.5 and 28.0).  The groups' rows drift apart by some fifty
 // tokens, so a group reads half as much again as its share of the source.
-// Up to 256 threads up to 40 MB of packed rows, then 512.  Rows of 14336 bytes to 8 ranks, four sets of tensors in turn, 512
+// Up to 256 threads up to 50 MB of packed rows, then 512.  Rows of 14336 bytes to 8 ranks, four sets of tensors in turn, 512
 // / 256 threads, and the same with a copy of the packed rows behind it: 36 MB 9.0 / 8.7 us, 21.7 / 22.8; 45 MB 10.6 / 10.2,
-// 26.3 / 27.5; 60 MB 13.9 / 15.4, 33.6 / 34.5; 80 MB 18.9 / 19.7, 44.0 / 44.2; 95 MB 23.5 / 24.0, 54.6 / 53.3; 111 MB 27.1 / 28.5,
-// 65.1 / 63.4; rows of 10240 alike, narrower ones have 256 either way.  In list order, past 128 MB, the
+// 26.3 / 27.5; 54 MB 11.6 / 12.9; 60 MB 13.7 / 15.5, 33.4 / 34.7; 80 MB 18.8 / 19.7, 43.7 / 44.3; 95 MB 23.7 / 24.2, 54.8 / 53.0;
+// 111 MB 27.1 / 28.2, 65.0 / 63.3; rows of 8704 to 28672 bytes alike (51 MB of 8704 11.3 / 10.2, 54 MB 12.6 / 12.7), narrower ones have
+// 256 either way.  In list order, past 128 MB, the
 // same threads move one vector at a time: two trips to memory stand in front of a row there.  4096 x 14336 88.5 us against 96.1
 // with two vectors in flight, 4096 x 7168 45.5 and 47.9 (46.0 to 48 with twice the threads), 12289 x 14336 258 and 267.
 // ---------------------------------------------------------------------
 constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of one of 8 groups; 16 MB of 16, 24 MB of more
 constexpr int64_t kPackSourceBytes = int64_t(3) << 20;  // source bytes of a group
 constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
-constexpr int64_t kPackSmallBytes = int64_t(40) << 20;
+constexpr int64_t kPackSmallBytes = int64_t(50) << 20;
 
 struct PackArgs {
     const uint8_t* src;
