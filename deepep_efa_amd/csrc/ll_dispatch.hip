@@ -34,48 +34,30 @@ namespace deepep {
 
 __host__ __device__ inline int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
-constexpr int kSweepChunkEntries = 2048;  // a token sweeps at most this many earlier entries itself
+constexpr int kRankChunkEntries = 2048;  // entries ranked by one workgroup, at most
+constexpr int kSendColumns = 32;         // chunks whose histograms the waves that store the rows add up themselves
+// The send kernel ranks its own slots up to here, which costs its rows less than a launch ahead of them costs the stream.
+constexpr int kSelfRankMaxEntries = 8192;
 
-// Tokens per sweep chunk: whole tokens, about kSweepChunkEntries entries.
-inline int sweep_chunk_tokens(int num_topk) {
-    const int t = kSweepChunkEntries / num_topk;
+// Tokens of a chunk: whole ones, about kRankChunkEntries entries.
+inline int rank_chunk_tokens(int num_topk) {
+    const int t = kRankChunkEntries / num_topk;
     return t < 1 ? 1 : t;
 }
 
-// Per source: the chunk histograms, int32 [chunks][E].
-static int64_t route_scratch_bytes(int num_tokens, int num_topk, int num_experts) {
-    const int tpc = sweep_chunk_tokens(num_topk);
+// The chunk histograms, int32 [chunks][E].
+static int64_t chunk_hist_bytes(int num_tokens, int num_topk, int num_experts) {
+    const int tpc = rank_chunk_tokens(num_topk);
     const int64_t chunks = (num_tokens + tpc - 1) / tpc;
     return align256((chunks < 1 ? 1 : chunks) * num_experts * 4);
 }
-
-// ---------------------------------------------------------------------
-// Per-chunk expert histograms for medium and large batches: workgroup c counts the
-// entries of tokens [c * tpc, (c + 1) * tpc) per expert.  The send kernel then
-// ranks a pair as (entries of earlier chunks naming its expert, summed from these
-// rows) + (earlier entries of its own chunk, which it sweeps itself).
-// ---------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void ll_chunk_hist_kernel(const int64_t* __restrict__ topk_idx, int n,
-                                                             int entries_per_chunk, int num_experts,
-                                                             int64_t scratch_stride,
-                                                             uint8_t* __restrict__ scratch_base) {
-    extern __shared__ int32_t hist_lds[];  // [E]
-    const int c = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-    const int64_t* my_topk = topk_idx + int64_t(b) * n;
-    int32_t* out = reinterpret_cast<int32_t*>(scratch_base + int64_t(b) * scratch_stride) + int64_t(c) * num_experts;
-    for (int e = tid; e < num_experts; e += blockDim.x) hist_lds[e] = 0;
-    lds_barrier();
-    const int begin = c * entries_per_chunk;
-    const int end = begin + entries_per_chunk < n ? begin + entries_per_chunk : n;
-    for (int i = begin + tid; i < end; i += blockDim.x) {
-        const int64_t v = my_topk[i];
-        if (v >= 0 && v < num_experts) atomicAdd(&hist_lds[int(v)], 1);
-    }
-    lds_barrier();
-    for (int e = tid; e < num_experts; e += blockDim.x) out[e] = hist_lds[e];
+// Per source: the chunk histograms, where an own expert's rows begin, int32 [E], and slots, int32 [T][K].
+static int64_t route_scratch_bytes(int num_tokens, int num_topk, int num_experts) {
+    return chunk_hist_bytes(num_tokens, num_topk, num_experts) + align256(int64_t(num_experts) * 4) +
+           align256(int64_t(num_tokens) * num_topk * 4);
 }
 
-// Entries that name expert e, from the chunk histograms.
+// Entries that name expert e in the first num_chunks chunk histograms.
 __device__ __forceinline__ int chunk_total(const int32_t* __restrict__ hists, int num_chunks, int num_experts, int e) {
     int total = 0;
     for (int c0 = 0; c0 < num_chunks; c0 += 8) {  // eight loads in flight
@@ -117,17 +99,14 @@ __device__ __forceinline__ void emit_expert_count(int e, int total, int num_expe
 // The slot of a selection is the number of earlier (token,k) entries naming its
 // expert (reference: the serial scan of csrc/kernels/efa_kernels.cu:617-637 and
 // token_offset / expert_offsets of csrc/kernels/coop_dispatch_send.cuh:360-420).
-// The workgroup counts them itself: while the row loads are in flight every
-// thread fetches up to four entries that precede the token (more in a loop) and
-// adds them to a histogram by expert in LDS.  Up to 8192
-// entries the sweep covers every earlier entry; beyond, it covers the token's
-// own chunk of about 2048 entries and the chunks before it come from the
-// histograms of ll_chunk_hist_kernel.  The per-expert totals come from one extra
-// workgroup per source.  Deterministic: integer adds only.
+// Up to 8192 entries the workgroup counts them itself: while the row loads are in
+// flight every thread fetches up to four entries that precede the token (more in a
+// loop) and adds them to a histogram by expert in LDS; the per-expert totals come
+// from one extra workgroup per source.  Larger batches get their slots from
+// ll_rank_chunk_kernel, one launch ahead.  Deterministic: integer adds only.
 // ---------------------------------------------------------------------
 constexpr int kMaxTopk = 64;
 constexpr int kFusedMaxEntries = 8192;     // send + receive in one launch up to here
-constexpr int kSelfRankMaxEntries = 8192;  // the send kernel ranks its own slots, unaided, up to here
 constexpr int kSendMaxWaves = 16;
 
 struct ByDestTables {
@@ -143,9 +122,6 @@ struct SendArgs {
     int num_tokens, hidden, num_topk, num_experts, num_ranks, rank, max_tokens;
     int pieces_per_row, split_log2;
     uint32_t rank_of_expert_magic;
-    int tokens_per_chunk;  // > 0: scratch holds the per-chunk expert histograms of ll_chunk_hist_kernel
-    int64_t scratch_stride;
-    const uint8_t* scratch_base;
     uint8_t* recv_staging;
     uint8_t* send_slots;
     int32_t* pair_slot;
@@ -154,10 +130,21 @@ struct SendArgs {
     // By-destination form: send_slots is one buffer of rows, contiguous per destination rank, and every
     // row (the rank's own included) goes to row expert_prefix[expert] + slot of it.  Null: per-expert slots.
     const int32_t* expert_prefix;
-    // By-destination batches for which no launch builds the tables first: every token's workgroup gets
-    // the batch's entries per expert itself, and the counting row writes the tables out.
+    // By-destination batches that rank themselves: every token's workgroup gets the batch's entries per
+    // expert itself, and the counting row writes the tables out.
     int prefix_in_block;
     ByDestTables by_dest;
+};
+
+// A batch ranked ahead of its rows, a chunk of tokens at a time.
+struct RankedBatch {
+    int num_chunks, tokens_per_chunk;
+    RankDivider chunk_of;       // a token's chunk
+    const int32_t* hists;       // [chunks][E] entries of a chunk that name an expert
+    int32_t* slots;             // [T][K] slots, counted within the chunk or, in_full, within the batch
+    int64_t stride;             // of both from a source to the next, in ints
+    int in_full;
+    int32_t* own_first;         // [E_l] where the rank's own rows begin (null: nobody asks)
 };
 
 // Final destination of the rows a rank sends to its own experts, used by the
@@ -178,7 +165,7 @@ struct EntryPair {
     // Entry 0 or 1 as an expert below `limit` counted from `first`, if it names one.
     __device__ __forceinline__ bool expert(int which, uint32_t first, uint32_t limit, uint32_t& e) const {
         e = v[which * 2] - first;
-        return v[which * 2 + 1] == 0u && e < limit;
+        return (v[which * 2 + 1] == 0u) & (e < limit);
     }
 };
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t entry_list(const int64_t* topk_idx, int n) {
@@ -192,35 +179,31 @@ struct alignas(16) SendLds {
 
 // hist[e] (LDS, [E + 1]) = entries of topk_idx[0 .. n) naming expert e, clamped to max_tokens, then their
 // exclusive prefix over the experts with the total in hist[E]; the whole workgroup takes part.
-// chunk_hist (may be null): the chunk histograms to take the entries from.  counts_out: the clamped counts.
+// counts_out: the clamped counts.
 __device__ __forceinline__ void expert_prefix_in_lds(const int64_t* __restrict__ topk_idx, int n, int num_experts,
-                                                     int max_tokens, const int32_t* __restrict__ chunk_hist,
-                                                     int num_chunks, int32_t* hist, int32_t* wave_totals,
+                                                     int max_tokens, int32_t* hist, int32_t* wave_totals,
                                                      int32_t* counts_out) {
     const int tid = threadIdx.x, threads = blockDim.x;
-    if (chunk_hist == nullptr) {
-        for (int e = tid; e < num_experts; e += threads) hist[e] = 0;
-        lds_barrier();
-        constexpr int kAhead = 4;  // pairs of entries in flight per thread
-        const auto list = entry_list(topk_idx, n);
-        for (int base = tid; base * 2 < n; base += kAhead * threads) {
-            EntryPair ahead[kAhead];
+    for (int e = tid; e < num_experts; e += threads) hist[e] = 0;
+    lds_barrier();
+    constexpr int kAhead = 4;  // pairs of entries in flight per thread
+    const auto list = entry_list(topk_idx, n);
+    for (int base = tid; base * 2 < n; base += kAhead * threads) {
+        EntryPair ahead[kAhead];
 #pragma unroll
-            for (int u = 0; u < kAhead; ++u) ahead[u].load(list, base + u * threads);
+        for (int u = 0; u < kAhead; ++u) ahead[u].load(list, base + u * threads);
 #pragma unroll
-            for (int u = 0; u < kAhead; ++u)
+        for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    uint32_t e;
-                    if (ahead[u].expert(i, 0, uint32_t(num_experts), e) && (base + u * threads) * 2 + i < n)
-                        atomicAdd(&hist[e], 1);
-                }
-        }
-        lds_barrier();
+            for (int i = 0; i < 2; ++i) {
+                uint32_t e;
+                if (ahead[u].expert(i, 0, uint32_t(num_experts), e) && (base + u * threads) * 2 + i < n)
+                    atomicAdd(&hist[e], 1);
+            }
     }
+    lds_barrier();
     for (int e = tid; e < num_experts; e += threads) {
-        const int total = chunk_hist != nullptr ? chunk_total(chunk_hist, num_chunks, num_experts, e) : hist[e];
-        const int c = total < max_tokens ? total : max_tokens;
+        const int c = hist[e] < max_tokens ? hist[e] : max_tokens;
         hist[e] = c;
         counts_out[e] = c;
     }
@@ -266,16 +249,6 @@ __device__ __forceinline__ void send_count_block(const SendArgs& a, int b, int32
     const int n = a.num_tokens * a.num_topk;
     const int src_rank = a.src_ranks != nullptr ? a.src_ranks[b] : a.rank;
     const int64_t* my_topk = a.topk_idx + int64_t(b) * n;
-    if (a.tokens_per_chunk > 0) {  // the totals are the column sums of the chunk histograms
-        const int32_t* hist = reinterpret_cast<const int32_t*>(a.scratch_base + int64_t(b) * a.scratch_stride);
-        const int chunks = (a.num_tokens + a.tokens_per_chunk - 1) / a.tokens_per_chunk;
-        for (int e = tid; e < a.num_experts; e += blockDim.x) {
-            const int total = chunk_total(hist, chunks, a.num_experts, e);
-            emit_expert_count(e, total, a.num_experts, a.num_ranks, a.rank, src_rank, a.max_tokens, a.recv_count,
-                              a.send_count);
-        }
-        return;
-    }
     for (int j = tid; j < a.num_experts; j += blockDim.x) lds_hist[j] = 0;
     lds_barrier();
     for (int i = tid; i < n; i += blockDim.x) {
@@ -286,6 +259,31 @@ __device__ __forceinline__ void send_count_block(const SendArgs& a, int b, int32
     for (int e = tid; e < a.num_experts; e += blockDim.x)
         emit_expert_count(e, lds_hist[e], a.num_experts, a.num_ranks, a.rank, src_rank, a.max_tokens, a.recv_count,
                           a.send_count);
+}
+
+// A wave's stores of its piece, one a selection of its part: lane k holds selection k's row and scales (0: nowhere), which
+// the loop takes back as wave-uniform values.
+template <int kFmt, bool kStream>
+__device__ __forceinline__ void store_selections(uint64_t my_row, uint64_t my_scale_row, int num_topk, int part, int split,
+                                                 int data_bytes, int scale_bytes, int lane_off, u32x4 payload,
+                                                 int scale_off, uint32_t scale_bits) {
+    for (int k = part; k < num_topk; k += split) {
+        const uint8_t* row = reinterpret_cast<const uint8_t*>(
+            (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_row >> 32), k))) << 32) |
+            uint32_t(__builtin_amdgcn_readlane(int(uint32_t(my_row)), k)));
+        if (row == nullptr) continue;
+        store_row_u32x4<kStream>(row_buffer(row, data_bytes), lane_off, payload);
+        if constexpr (kFmt != kRowBF16) {
+            const uint8_t* scale_row = reinterpret_cast<const uint8_t*>(
+                (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_scale_row >> 32), k))) << 32) |
+                uint32_t(__builtin_amdgcn_readlane(int(uint32_t(my_scale_row)), k)));
+            const auto scales = row_buffer(scale_row, scale_bytes);
+            if constexpr (kFmt == kRowFP8UE8M0)
+                __builtin_amdgcn_raw_buffer_store_b8(uint8_t(scale_bits >> 23), scales, scale_off, 0, 0);
+            else
+                __builtin_amdgcn_raw_buffer_store_b32(scale_bits, scales, scale_off, 0, 0);
+        }
+    }
 }
 
 // One workgroup's share of token t of source b.  kStream (64 MB of traffic and more): the payload of
@@ -338,32 +336,15 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     // wave 0 -- for the token's own selections -- does not also wait out a second round trip for the
     // entries it sweeps.
     const int threads = blockDim.x;
-    const int chunk = a.tokens_per_chunk > 0 ? t / a.tokens_per_chunk : 0;
-    const int sweep_begin = chunk * a.tokens_per_chunk * num_topk;
     const bool prefix_in_block = kTables && a.prefix_in_block;
-    const bool count_all = prefix_in_block && a.tokens_per_chunk == 0;
-    const bool count_chunks = prefix_in_block && a.tokens_per_chunk > 0;
-    const int sweep_end = count_all ? n : entry0;
+    const int sweep_end = prefix_in_block ? n : entry0;
     constexpr int kSweepAhead = 2;
     const int64_t own_v = my_topk[entry0 + (tid < num_topk ? tid : num_topk - 1)];  // threads 0..K-1: selection tid
-    const auto list = entry_list(my_topk + sweep_begin, n - sweep_begin);
-    const int sweep_pairs = (sweep_end - sweep_begin + 1) >> 1;
+    const auto list = entry_list(my_topk, n);
+    const int sweep_pairs = (sweep_end + 1) >> 1;
     EntryPair ahead[kSweepAhead];
 #pragma unroll
     for (int r = 0; r < kSweepAhead; ++r) ahead[r].load(list, tid + r * threads);
-    // the first eight words of a thread's column of the chunk histograms, zeros past the last chunk
-    uint32_t column[8];
-    int chunks = 0;
-    const auto load_column = [&](int e, int c0) {
-        const auto hists = row_buffer(a.scratch_base, chunks * num_experts * 4);
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            column[u] = __builtin_amdgcn_raw_buffer_load_b32(hists, ((c0 + u) * num_experts + e) * 4, 0, 0);
-    };
-    if (count_chunks) {
-        chunks = (a.num_tokens + a.tokens_per_chunk - 1) / a.tokens_per_chunk;
-        if (tid < num_experts) load_column(tid, 0);
-    }
     for (int e = tid; e < num_experts; e += threads) lds_hist[e] = 0;
     lds_barrier();
 
@@ -381,7 +362,6 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
         }
     }
     int dest_first = 0;  // by-destination form: where the expert's run of rows begins in the send buffer
-    if (a.expert_prefix != nullptr && !prefix_in_block && my_expert >= 0) dest_first = a.expert_prefix[my_expert];
     if (direct.packed_x != nullptr && tid < kWave) {
         // Rows for this rank's own experts go straight to the packed tensors, at the place the
         // reference's range builder gives them: behind the rows of the lower source ranks
@@ -401,46 +381,21 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
             if (lane == k) direct_begin = sum;
         }
     }
-    // Medium and large batches: the token sweeps only the earlier entries of its own chunk; what the
-    // chunks before it hold of each selection's expert comes from their histograms.
-    int chunk_base = 0;
-    if (chunk > 0 && !count_chunks && tid < num_topk && my_expert >= 0) {
-        const int32_t* hist = reinterpret_cast<const int32_t*>(a.scratch_base + int64_t(b) * a.scratch_stride);
-        for (int c0 = 0; c0 < chunk; c0 += 8) {  // eight loads in flight
-            int c[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) c[u] = c0 + u < chunk ? hist[int64_t(c0 + u) * num_experts + my_expert] : 0;
-#pragma unroll
-            for (int u = 0; u < 8; ++u) chunk_base += c[u];
-        }
-    }
     DEEPEP_PHASE(1);
     u32x4 payload = lo;  // quantised below, while the workgroup's bookkeeping is in flight
     uint32_t scale_bits = 0;
     // Rank the selections: the entries between the start of the sweep and this token, counted by expert in LDS.  (A
     // ballot for each selection and load instead cost every wave of the workgroup 130 instructions a round of four
     // entries a thread: 128 tokens 7.7 -> 7.4 us, 300 tokens 15.9 -> 15.4, single entries read instead of pairs 16.1.)
-    // With prefix_in_block the low half of a word counts all of the batch's entries and the high half those before
-    // the token, and wave 0 gets the prefix from the same words (128 tokens 9.4 -> 7.8 us against a histogram of its
-    // own and a scan by the whole workgroup).  The sweep then goes through the whole batch, or, where there are chunk
-    // histograms, through the token's chunk as ever, and their columns, a thread an expert, make the rest of both halves.
-    const int before = count_chunks ? 0x10000 : (count_all ? 0x10001 : 1);
-    if (count_chunks) {
-        for (int e = tid; e < num_experts; e += threads) {
-            uint32_t sums = 0;
-            for (int c0 = 0; c0 < chunks; c0 += 8) {
-                if (c0 > 0 || e != tid) load_column(e, c0);
-#pragma unroll
-                for (int u = 0; u < 8; ++u) sums += column[u] * (c0 + u < chunk ? 0x10001u : 1u);
-            }
-            atomicAdd(&lds_hist[e], int(sums));
-        }
-    }
+    // With prefix_in_block the sweep goes through the whole batch: the low half of a word counts all of its entries and
+    // the high half those before the token, and wave 0 gets the prefix from the same words (128 tokens 9.4 -> 7.8 us
+    // against a histogram of its own and a scan by the whole workgroup).
+    const int before = prefix_in_block ? 0x10001 : 1;
     const auto count_pair = [&](int pair, const EntryPair& entries) {
         if (pair >= sweep_pairs) return;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int at = sweep_begin + pair * 2 + i;
+            const int at = pair * 2 + i;
             uint32_t e;
             if (entries.expert(i, 0, uint32_t(num_experts), e) && at < sweep_end)
                 atomicAdd(&lds_hist[e], at < entry0 ? before : 1);
@@ -467,7 +422,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
             const int other = __builtin_amdgcn_readlane(my_expert, k2);
             if (k2 < tid && other == my_expert) total += 1;
         }
-        if (tid < num_topk && my_expert >= 0) my_slot = total + chunk_base;
+        if (tid < num_topk && my_expert >= 0) my_slot = total;
     }
     if (tid < num_topk) {
         if (my_slot >= a.max_tokens) my_slot = -1;
@@ -512,63 +467,329 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     const int lane_off = piece * 1024 + lane * 16;
     const int scale_off = lane_live && (lane & 7) == 0 ? (kFmt == kRowFP8UE8M0 ? group : group * 4) : 0x7fffffff;
     DEEPEP_PHASE(5);
-    // lane k reads selection k's destinations once; the loop takes them back as wave-uniform values
+    // lane k reads selection k's destinations once
     uint64_t my_row = 0, my_scale_row = 0;
     if (lane < num_topk) {
         my_row = lds.sel_row[lane];
         my_scale_row = lds.sel_scale[lane];
     }
-    for (int k = part; k < num_topk; k += split) {
-        const uint8_t* row = reinterpret_cast<const uint8_t*>(
-            (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_row >> 32), k))) << 32) |
-            uint32_t(__builtin_amdgcn_readlane(int(uint32_t(my_row)), k)));
-        if (row == nullptr) continue;
-        store_row_u32x4<kStream>(row_buffer(row, int(data_bytes)), lane_off, payload);
-        if constexpr (kFmt != kRowBF16) {
-            const uint8_t* scale_row = reinterpret_cast<const uint8_t*>(
-                (uint64_t(uint32_t(__builtin_amdgcn_readlane(int(my_scale_row >> 32), k))) << 32) |
-                uint32_t(__builtin_amdgcn_readlane(int(uint32_t(my_scale_row)), k)));
-            const auto scales = row_buffer(scale_row, int(scale_bytes));
-            if constexpr (kFmt == kRowFP8UE8M0)
-                __builtin_amdgcn_raw_buffer_store_b8(uint8_t(scale_bits >> 23), scales, scale_off, 0, 0);
-            else
-                __builtin_amdgcn_raw_buffer_store_b32(scale_bits, scales, scale_off, 0, 0);
-        }
-    }
+    store_selections<kFmt, kStream>(my_row, my_scale_row, num_topk, part, split, int(data_bytes), int(scale_bytes), lane_off,
+                                    payload, scale_off, scale_bits);
     DEEPEP_PHASE(6);
 }
 
+template <int kFmt, bool kStream>
+__global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_send_kernel(SendArgs a) {
+    extern __shared__ int32_t lds_hist[];  // [E + 1]
+    __shared__ SendLds lds;
+    __shared__ int32_t wave_totals[kMaxBlockWaves];
+    if (int(blockIdx.y) == a.num_tokens) {  // the counting row of the grid
+        if (blockIdx.x != 0) return;
+        if (a.prefix_in_block) {  // this workgroup writes the tables out
+            expert_prefix_in_lds(a.topk_idx, a.num_tokens * a.num_topk, a.num_experts, a.max_tokens, lds_hist, wave_totals,
+                                 a.send_count);
+            by_dest_tables_out(lds_hist, a.num_experts, a.num_ranks, a.by_dest);
+        } else {
+            send_count_block(a, blockIdx.z, lds_hist);
+        }
+        return;
+    }
+    send_token_block<kFmt, kStream, true>(a, DirectOut{nullptr, nullptr, nullptr}, blockIdx.z, blockIdx.y, blockIdx.x, lds,
+                                          lds_hist);
+}
+
+// ---------------------------------------------------------------------
+// Large batches: the entries are ranked one launch ahead of the rows, a workgroup a chunk.  A wave matches 64 entries
+// at a time against one another, a ballot for each bit of the expert, and keeps how many it has seen of an expert in a
+// byte of LDS; an entry's place in its chunk is what the waves before its own have of its expert, what its wave had
+// before, and the lanes before it.  The sums of the bytes are the chunk's histogram, and what the chunks before an
+// entry's have of its expert is added by whoever reads the place.  Nothing is read twice: one compute unit takes 18 bytes
+// a cycle of a list that is not in its L2, so workgroups that went through all entries before their own took 4.6 us for
+// 16376 entries and 7.7 for 32768, and this takes 2.7 (an empty kernel 2.4).
+// The first workgroup also writes where the rank's own rows of each local expert begin, behind those of the lower
+// source ranks (csrc/kernels/efa_kernels.cu:991-1010).
+// ---------------------------------------------------------------------
+constexpr int kRankWaves = 16;
+
+__global__ __launch_bounds__(kRankWaves* kWave) void ll_rank_chunk_kernel(
+    const int64_t* __restrict__ topk_idx, int n, int num_topk, int num_experts, int32_t* __restrict__ hists,
+    RankedBatch batch, const int32_t* __restrict__ recv_count, int num_ranks, int rank, int max_tokens) {
+    extern __shared__ u32x4 rank_lds[];  // bytes [E][waves]
+    static_assert(kRankWaves == 16 && kRankChunkEntries <= 2 * kRankWaves * kWave, "a vector of bytes, two entries a lane");
+    uint8_t* counts = reinterpret_cast<uint8_t*>(rank_lds);
+    const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block(), b = blockIdx.y;
+    const int per_chunk = batch.tokens_per_chunk * num_topk;
+    const int begin = int(blockIdx.x) * per_chunk, end = min(begin + per_chunk, n);
+    const auto list = entry_list(topk_idx + int64_t(b) * n, n);
+    const int first = begin + w * 2 * kWave + lane;
+    u32x2 entry[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) entry[i] = __builtin_amdgcn_raw_buffer_load_b64(list, (first + i * kWave) * 8, 0, 0);
+    int own_rows = 0;
+    const bool own_wanted = blockIdx.x == 0 && batch.own_first != nullptr;
+    if (own_wanted) {  // a wave an expert, as far as there are waves
+        for (int s = lane; s < rank && w < num_experts / num_ranks; s += kWave) {
+            const int c = recv_count[w * num_ranks + s];
+            own_rows += c < 0 ? 0 : (c > max_tokens ? max_tokens : c);
+        }
+    }
+    for (int e = tid; e < num_experts; e += kRankWaves * kWave) rank_lds[e] = u32x4{0u, 0u, 0u, 0u};
+    lds_barrier();
+    int before[2];
+    bool live[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uint32_t e = entry[i][0];
+        live[i] = first + i * kWave < end && entry[i][1] == 0u && e < uint32_t(num_experts);
+        uint64_t same = __ballot(live[i]);
+        for (int bit = 1; bit < num_experts; bit <<= 1) {
+            const bool set = (e & uint32_t(bit)) != 0u;
+            const uint64_t votes = __ballot(set);
+            same &= set ? votes : ~votes;
+        }
+        const int lower = __popcll(same & lanes_below(lane));
+        const int had = live[i] ? counts[e * kRankWaves + w] : 0;  // LDS serves a wave in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (live[i] && lower == 0) counts[e * kRankWaves + w] = uint8_t(had + __popcll(same));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        before[i] = had + lower;
+    }
+    lds_barrier();
+    const auto count_of_waves = [&](uint32_t e, int waves) {  // what the waves before `waves` have of e
+        const u32x4 of = rank_lds[e];
+        uint32_t sum = 0;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const int n_bytes = waves - d * 4;
+            sum = __builtin_amdgcn_sad_u8(of[d] & (n_bytes <= 0 ? 0u : (n_bytes >= 4 ? ~0u : (1u << (n_bytes * 8)) - 1)), 0u, sum);
+        }
+        return int(sum);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (first + i * kWave < end)
+            batch.slots[int64_t(b) * batch.stride + first + i * kWave] =
+                live[i] ? before[i] + count_of_waves(entry[i][0], w) : -1;
+    int32_t* out = hists + int64_t(b) * batch.stride + int64_t(blockIdx.x) * num_experts;
+    for (int e = tid; e < num_experts; e += kRankWaves * kWave) out[e] = count_of_waves(uint32_t(e), kRankWaves);
+    if (own_wanted) {
+        for (int le = w;;) {
+            own_rows = wave_inclusive_sum(own_rows);
+            if (lane == kWave - 1 && le < num_experts / num_ranks) batch.own_first[le] = own_rows;
+            le += kRankWaves;
+            if (le >= num_experts / num_ranks) break;
+            own_rows = 0;
+            for (int s = lane; s < rank; s += kWave) {
+                const int c = recv_count[le * num_ranks + s];
+                own_rows += c < 0 ? 0 : (c > max_tokens ? max_tokens : c);
+            }
+        }
+    }
+}
+
+// The counts of a ranked batch, by one workgroup: columns of the chunk histograms.  By destination, the tables.
+__device__ __forceinline__ void ranked_counts(const SendArgs& a, const RankedBatch& batch, int b, int32_t* lds,
+                                              int32_t* wave_totals) {
+    const int32_t* hists = batch.hists + int64_t(b) * batch.stride;
+    const int src_rank = a.src_ranks != nullptr ? a.src_ranks[b] : a.rank;
+    for (int e = threadIdx.x; e < a.num_experts; e += blockDim.x) {
+        const int total = chunk_total(hists, batch.num_chunks, a.num_experts, e);
+        if (a.expert_prefix == nullptr) {
+            emit_expert_count(e, total, a.num_experts, a.num_ranks, a.rank, src_rank, a.max_tokens, a.recv_count,
+                              a.send_count);
+        } else {
+            lds[e] = total < a.max_tokens ? total : a.max_tokens;
+            a.send_count[e] = lds[e];
+        }
+    }
+    if (a.expert_prefix == nullptr) return;
+    lds_barrier();
+    block_exclusive_scan(lds, a.num_experts, wave_totals);
+    by_dest_tables_out(lds, a.num_experts, a.num_ranks, a.by_dest);
+}
+
+// Slots within the batch, for batches of many chunks and by-destination ones of many experts: workgroup c adds what the
+// chunks before c hold, the last one writes the counts.
+__global__ __launch_bounds__(1024) void ll_rank_finish_kernel(SendArgs a, RankedBatch batch) {
+    extern __shared__ int32_t before[];  // [E + 1]
+    __shared__ int32_t wave_totals[kMaxBlockWaves];
+    const int tid = threadIdx.x, threads = blockDim.x, c = blockIdx.x, b = blockIdx.y;
+    if (c == batch.num_chunks) {
+        ranked_counts(a, batch, b, before, wave_totals);
+        return;
+    }
+    const int32_t* hists = batch.hists + int64_t(b) * batch.stride;
+    for (int e = tid; e < a.num_experts; e += threads) before[e] = chunk_total(hists, c, a.num_experts, e);
+    lds_barrier();
+    const int per_chunk = batch.tokens_per_chunk * a.num_topk, n = a.num_tokens * a.num_topk;
+    const int end = min((c + 1) * per_chunk, n);
+    int32_t* slots = batch.slots + int64_t(b) * batch.stride;
+    for (int i = c * per_chunk + tid; i < end; i += threads) {
+        int slot = slots[i];
+        if (slot < 0) continue;
+        slot += before[int(a.topk_idx[int64_t(b) * n + i])];
+        slots[i] = slot < a.max_tokens ? slot : -1;
+    }
+}
+
+// For one wave, from the chunk histograms: the rows of the experts before the lane's `expert` (`first`: an expert's entries
+// are clamped to max_tokens) and the entries of the chunks before `chunk` that name it.  Lane l adds up the columns of the
+// kPer experts from l * kPer on, whole vectors of them.
+template <int kPer>
+__device__ __forceinline__ void columns_by_dest(__amdgpu_buffer_rsrc_t hists, int num_chunks, int chunk, int num_experts,
+                                                int max_tokens, int expert, int& first, int& below) {
+    static_assert(kPer == 1 || kPer == 4, "a word or a vector");
+    const int lane = lane_id();
+    const bool mine = lane * kPer < num_experts;
+    int total[kPer] = {}, lower[kPer] = {};
+    constexpr int kAhead = kPer == 1 ? 8 : 4;  // of vectors no more than eight waves a SIMD have registers for
+    for (int c0 = 0; c0 < num_chunks; c0 += kAhead) {
+        u32x4 v[kAhead];  // zeros past the last histogram
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int at = mine ? ((c0 + u) * num_experts + lane * kPer) * 4 : 0x7ffffff0;
+            if constexpr (kPer == 1) v[u][0] = __builtin_amdgcn_raw_buffer_load_b32(hists, at, 0, 0);
+            else v[u] = load_row_u32x4<false>(hists, at);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) total[i] += int(v[u][i]), lower[i] += c0 + u < chunk ? int(v[u][i]) : 0;
+    }
+    int sum = 0;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) total[i] = total[i] < max_tokens ? total[i] : max_tokens, sum += total[i];
+    int run = wave_inclusive_sum(sum) - sum;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const int run_of = __shfl(run, expert / kPer, kWave), lower_of = __shfl(lower[i], expert / kPer, kWave);
+        if (i == 0 || i <= expert % kPer) first = run_of, below = lower_of;
+        run += total[i];
+    }
+}
+
+// The rows of a ranked batch: a wave's share is a 1 KiB piece as in ll_send_kernel, but nothing is left to be worked out
+// by the workgroup, so no wave waits for another.  Selections, places and row are fetched together; behind them, beside
+// the row, the columns of the chunks before the token's, shared among the lanes, and a table (the by-destination prefix,
+// which without a table are the sums of all columns, or where own rows begin).
+// HBM bounds it: 4096 tokens of hidden 7168, top-8, fp8 (302 MB) 50 us, 6.0 TB/s, where workgroups that went through the
+// entries of their chunk and shared what they counted, three barriers ahead of the stores, took 61.  Both launches of a
+// send against histograms and that kernel: by destination to 8 ranks 4096 tokens 65 -> 59 us, of hidden 1024 23.4 -> 20.7,
+// 2047 tokens of 7168 30.0 -> 29.6, of 4096 with 256 experts 26.3 -> 22.9, 1100 23.6 -> 22.5; a dispatch of 4096 tokens 133 -> 125,
+// 2047 70 -> 67.  Two waves a piece, half of the stores each: 55 us instead of 50.  With the register allocation left
+// open instead of bounded for eight waves a SIMD the same dispatch takes 127, 2047 tokens of 4096 24.4.
 // index_rows > 0: the grid has that many rows in front of the token rows whose workgroups build the
 // receive side's row index (one (local expert, source) segment each), so that a large one-call
 // dispatch needs no launch for it.
 template <int kFmt, bool kStream>
-__global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_send_kernel(SendArgs a, DirectOut direct, FusedIndexArgs index,
-                                                                       int index_rows) {
-    extern __shared__ int32_t lds_hist[];  // counting workgroups: [E]; index workgroups: [2 * (E + 1)]
-    __shared__ SendLds lds;
-    __shared__ int32_t index_wave_totals[kMaxBlockWaves];
-    // Grid rows: first the index rows (started first, so that their few microseconds of scans run beside
-    // the token rows instead of behind them), then one row per token, then the counting row.
-    const int y = int(blockIdx.y) - index_rows;
-    if (y < 0) {
+__global__ __launch_bounds__(kSendMaxWaves* kWave, 8) void ll_send_ranked_kernel(SendArgs a, DirectOut direct,
+                                                                                 RankedBatch batch, FusedIndexArgs index,
+                                                                                 int index_rows, int topk_log2) {
+    extern __shared__ int32_t ranked_lds[];  // index workgroups: [2 * (E + 1)]; the counting row: [E + 1]
+    __shared__ int32_t wave_totals[kMaxBlockWaves];
+    // First the index rows (started first, so that their few microseconds of scans run beside the token rows instead
+    // of behind them), then one row per token, then the counting row.
+    const int t = int(blockIdx.y) - index_rows, b = blockIdx.z;
+    if (t < 0) {
         const int seg = int(blockIdx.y) * int(gridDim.x) + int(blockIdx.x);
-        if (seg < index.num_local_experts * index.num_ranks) recv_index_block(index, seg, lds_hist, index_wave_totals);
+        if (seg < index.num_local_experts * index.num_ranks) recv_index_block(index, seg, ranked_lds, wave_totals);
         return;
     }
-    if (y == a.num_tokens) {  // the counting row of the grid
-        if (blockIdx.x != 0) return;
-        if (a.prefix_in_block) {  // this workgroup writes the tables out
-            const int tpc = a.tokens_per_chunk;
-            expert_prefix_in_lds(a.topk_idx, a.num_tokens * a.num_topk, a.num_experts, a.max_tokens,
-                                 tpc > 0 ? reinterpret_cast<const int32_t*>(a.scratch_base) : nullptr,
-                                 tpc > 0 ? (a.num_tokens + tpc - 1) / tpc : 0, lds_hist, index_wave_totals, a.send_count);
-            by_dest_tables_out(lds_hist, a.num_experts, a.num_ranks, a.by_dest);
-        } else if (a.expert_prefix == nullptr) {
-            send_count_block(a, blockIdx.z, lds_hist);
-        }  // else: ll_by_dest_prefix_kernel ran first
+    if (t == a.num_tokens) {
+        if (blockIdx.x == 0) ranked_counts(a, batch, b, ranked_lds, wave_totals);
         return;
     }
-    send_token_block<kFmt, kStream, true>(a, direct, blockIdx.z, y, blockIdx.x, lds, lds_hist);
+    const int lane = lane_id(), num_topk = a.num_topk, num_experts = a.num_experts;
+    const int item = int(blockIdx.x) * int(blockDim.x >> 6) + wave_in_block();
+    if (item >= (a.pieces_per_row << a.split_log2)) return;
+    const int split = 1 << a.split_log2, part = item & (split - 1), piece = item >> a.split_log2;
+    const int64_t row_id = int64_t(b) * a.num_tokens + t;
+    const auto token_row = row_buffer(a.x + uint64_t(row_id) * (uint32_t(a.hidden) * 2), a.hidden * 2);
+    u32x4 lo, hi = {0u, 0u, 0u, 0u};  // zeros past the row's end
+    if constexpr (kFmt == kRowBF16) {
+        lo = load_row_u32x4<false>(token_row, piece * 1024 + lane * 16);
+    } else {
+        lo = load_row_u32x4<false>(token_row, piece * 2048 + lane * 32);
+        hi = load_row_u32x4<false>(token_row, piece * 2048 + lane * 32 + 16);
+    }
+    // Selection k in the lanes k, k + 2^topk_log2, ...: 2^topk_log2 >= K, so that the lanes share a selection's columns.
+    const int k = lane & ((1 << topk_log2) - 1);
+    int expert = 0, slot = -1;
+    if (k < num_topk) {
+        slot = batch.slots[int64_t(b) * batch.stride + int64_t(t) * num_topk + k];
+        expert = int(a.topk_idx[row_id * num_topk + k]);
+    }
+    if (slot < 0) expert = 0;
+    int first = 0;  // by destination: where the expert's run of rows begins in the send buffer
+    const bool by_dest = a.expert_prefix != nullptr;
+    if (batch.in_full) {
+        if (by_dest) first = a.expert_prefix[expert];
+    } else {
+        const int chunk = batch.chunk_of(t);
+        const auto hists = row_buffer(reinterpret_cast<const uint8_t*>(batch.hists + int64_t(b) * batch.stride),
+                                      batch.num_chunks * num_experts * 4);
+        int below = 0;
+        if (by_dest) {
+            if (num_experts <= kWave) columns_by_dest<1>(hists, batch.num_chunks, chunk, num_experts, a.max_tokens, expert, first, below);
+            else columns_by_dest<4>(hists, batch.num_chunks, chunk, num_experts, a.max_tokens, expert, first, below);
+        } else {
+            const int step = kWave >> topk_log2;
+            for (int c = lane >> topk_log2; c - (lane >> topk_log2) < chunk; c += 4 * step) {
+                int v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    v[u] = int(__builtin_amdgcn_raw_buffer_load_b32(
+                        hists, c + u * step < chunk ? ((c + u * step) * num_experts + expert) * 4 : 0x7fffffff, 0, 0));
+#pragma unroll
+                for (int u = 0; u < 4; ++u) below += v[u];
+            }
+            for (int d = 1 << topk_log2; d < kWave; d <<= 1) below += __shfl_xor(below, d, kWave);
+        }
+        if (slot >= 0) slot += below;
+        if (slot >= a.max_tokens) slot = -1;
+        if (item == 0 && lane < num_topk && a.pair_slot != nullptr) a.pair_slot[int64_t(t) * num_topk + lane] = slot;
+    }
+    const int src_rank = a.src_ranks != nullptr ? a.src_ranks[b] : a.rank;
+    const int64_t data_bytes = row_data_bytes(a.hidden, kFmt), scale_bytes = row_scale_bytes(a.hidden, kFmt);
+    const int64_t stride = row_stride_bytes(a.hidden, kFmt);
+    uint8_t *row = nullptr, *scale_row = nullptr;
+    if (slot >= 0 && lane < num_topk) {
+        // expert / E_l by multiply-high; magic 0 stands for E_l == 1
+        const int dst_rank = a.rank_of_expert_magic != 0 ? int(__umulhi(uint32_t(expert), a.rank_of_expert_magic)) : expert;
+        const int local = expert - dst_rank * (num_experts / a.num_ranks);
+        if (by_dest) {
+            row = a.send_slots + (int64_t(first) + slot) * stride;
+        } else if (dst_rank != a.rank) {
+            if (a.send_slots != nullptr) row = a.send_slots + (int64_t(expert) * a.max_tokens + slot) * stride;
+        } else if (direct.packed_x == nullptr) {
+            row = a.recv_staging + ((int64_t(local) * a.num_ranks + src_rank) * a.max_tokens + slot) * stride;
+        }
+        if (row != nullptr) {
+            scale_row = row + align16(data_bytes);
+            if (item == 0) {
+                const u32x4 tail = {uint32_t(t), uint32_t(lane), uint32_t(src_rank), uint32_t(local)};
+                *reinterpret_cast<u32x4*>(scale_row + align16(scale_bytes)) = tail;
+            }
+        } else if (dst_rank == a.rank) {
+            const int64_t out_row = int64_t(local) * a.num_ranks * a.max_tokens + batch.own_first[local] + slot;
+            row = direct.packed_x + out_row * data_bytes;
+            scale_row = direct.packed_scales + out_row * scale_bytes;
+            if (item == 0) direct.src_info[out_row] = t;
+        }
+    }
+    u32x4 payload = lo;
+    uint32_t scale_bits = 0;
+    int scale_off = 0x7fffffff;
+    if constexpr (kFmt != kRowBF16) {
+        payload = quantise_16<kFmt>(lo, hi, scale_bits);
+        const int group = piece * 8 + (lane >> 3);
+        if ((lane & 7) == 0 && group < a.hidden / kGroup) scale_off = kFmt == kRowFP8UE8M0 ? group : group * 4;
+    }
+    store_selections<kFmt, kStream>(reinterpret_cast<uint64_t>(row), reinterpret_cast<uint64_t>(scale_row), num_topk, part,
+                                    split, int(data_bytes), int(scale_bytes), piece * 1024 + lane * 16, payload, scale_off,
+                                    scale_bits);
 }
 
 // ---------------------------------------------------------------------
@@ -854,42 +1075,25 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_dispatch_fused_kernel
     }
 }
 
-// ---------------------------------------------------------------------
-// By-destination send (what an all-to-all ships: one contiguous message per
-// peer).  The rows are placed by tables made of the route counts: send_count[e]
-// (clamped to the M slots of a pair), its exclusive prefix over the experts --
-// the first row of every expert's run, experts ascending, hence destination ranks
-// ascending -- and the per-rank counts and prefix the transport cuts the buffer
-// by.  Batches that by_dest_tables_in_send() leaves to it get them from this one
-// workgroup before the send kernel runs.
-// Reference: the count + prefix phases of ll_dispatch_route_and_pack_v3
-// (csrc/kernels/efa_kernels.cu:2358-2371: ll_dispatch_count_kernel, prefix_sum_kernel).
-// ---------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void ll_by_dest_prefix_kernel(const int64_t* __restrict__ topk_idx, int n,
-                                                                 int num_experts, int num_ranks, int max_tokens,
-                                                                 const int32_t* __restrict__ chunk_hist, int num_chunks,
-                                                                 int32_t* __restrict__ send_count, ByDestTables out) {
-    extern __shared__ int32_t hist[];  // [E + 1]
-    __shared__ int32_t wave_totals[kMaxBlockWaves];
-    expert_prefix_in_lds(topk_idx, n, num_experts, max_tokens, chunk_hist, num_chunks, hist, wave_totals, send_count);
-    by_dest_tables_out(hist, num_experts, num_ranks, out);
+// Experts whose columns a wave adds up: a word a lane, or a vector.
+static bool columns_by_dest_fit(int num_experts) {
+    return num_experts <= kWave || (num_experts <= 4 * kWave && num_experts % 4 == 0);
 }
 
-// Whether the send launch makes the by-destination tables, every token's workgroup for itself, instead of a launch before
-// it.  Without chunk histograms (chunks 0: up to 8192 entries) each workgroup goes through the whole batch instead of half
-// of it, and one wave through the experts: up to 1024 experts that costs less than the launch, past them only for batches
-// of up to 2048 entries.  With histograms it adds up their columns, loaded with the first entries, which pays up to 4096
-// words.  Microseconds of the send with the tables made by itself against the launch before it, top-8, fp8:
-//   300 tokens, 64 experts, hidden 7168      10.7 / 13.5        2047 tokens,  64 experts ( 512 words)  14.9 / 17.5
-//   1024 tokens, 64 experts, hidden 7168     18.2 / 19.5        8000 tokens,  64 experts (2048 words)  23.0 / 25.5
-//   300 tokens, 256 experts, hidden 2048      6.0 /  8.6        2047 tokens, 256 experts (2048 words)  16.3 / 17.7
-//   1000 tokens, 1024 experts, hidden 2048   12.1 / 14.3        4000 tokens, 256 experts (4096 words)  23.6 / 24.0
-//   1000 tokens, 4096 experts, hidden 2048   20.1 / 15.3        2047 tokens, 1024 experts (8192 words) 21.0 / 18.3
+// Whether a by-destination send (what an all-to-all ships: one contiguous message per peer) of up to 8192 entries makes
+// its tables itself -- send_count[e], clamped to the M slots of a pair, its exclusive prefix over the experts, which is the
+// first row of every expert's run, and the per-rank counts and prefix the transport cuts the buffer by; reference: the
+// count + prefix phases of ll_dispatch_route_and_pack_v3 (csrc/kernels/efa_kernels.cu:2358-2371: ll_dispatch_count_kernel,
+// prefix_sum_kernel).  Every token's workgroup then goes through the whole batch instead of half of it, and one wave
+// through the experts: up to 1024 experts that costs less than a launch ahead, past them only for batches of up to 2048
+// entries.  Microseconds of the send with the tables made by itself against a launch before it, top-8, fp8:
+//   300 tokens, 64 experts, hidden 7168      10.7 / 13.5        300 tokens, 256 experts, hidden 2048      6.0 /  8.6
+//   1024 tokens, 64 experts, hidden 7168     18.2 / 19.5        1000 tokens, 1024 experts, hidden 2048   12.1 / 14.3
+//   1000 tokens, 4096 experts, hidden 2048   20.1 / 15.3
 // Both counts of an expert share a 32-bit word: fewer than 2^16 entries.
-constexpr int kByDestInBlockExperts = 1024, kByDestInBlockEntries = 2048, kByDestInBlockWords = 4096;
-static bool by_dest_tables_in_send(int n, int num_experts, int chunks) {
-    if (chunks == 0) return num_experts <= kByDestInBlockExperts || n <= kByDestInBlockEntries;
-    return n < 65536 && int64_t(chunks) * num_experts <= kByDestInBlockWords;
+constexpr int kByDestInBlockExperts = 1024, kByDestInBlockEntries = 2048;
+static bool by_dest_tables_in_send(int n, int num_experts) {
+    return n <= kSelfRankMaxEntries && (num_experts <= kByDestInBlockExperts || n <= kByDestInBlockEntries);
 }
 
 // ---------------------------------------------------------------------
@@ -917,27 +1121,46 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
                             int64_t fused_recv_wave_items = 0, const DirectOut* own_rows_direct = nullptr,
                             const ByDestTables* by_dest = nullptr, FusedIndexArgs* fused_index = nullptr,
                             bool* index_was_fused = nullptr) {
-    const int64_t scratch_bytes = route_scratch_bytes(num_tokens, num_topk, num_experts);
-    EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(scratch_bytes) * size_t(num_src));
-    EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(workspace) & 15) == 0);
     const int n = num_tokens * num_topk;
+    // How slots get ranked: the launch that stores the rows does it for itself while it is the only one and has no more
+    // than kSelfRankMaxEntries entries to go through.
+    const bool prefix_in_block = by_dest != nullptr && by_dest_tables_in_send(n, num_experts);
+    const bool ranked = fused_recv == nullptr && (n > kSelfRankMaxEntries || own_rows_direct != nullptr ||
+                                                  (by_dest != nullptr && !prefix_in_block));
+    const int64_t hist_bytes = chunk_hist_bytes(num_tokens, num_topk, num_experts);
+    const int64_t first_bytes = own_rows_direct != nullptr ? align256(int64_t(num_experts) * 4) : 0;
+    const int64_t slot_bytes = align256(int64_t(n) * 4);
+    // What the chunks before a token's hold of its experts is added up by the waves that store its rows, up to
+    // kSendColumns of them and, by destination, up to 256 experts; otherwise, and without room for slots that nobody sees,
+    // by a launch between the two.
+    RankedBatch batch = {};
+    batch.tokens_per_chunk = rank_chunk_tokens(num_topk);
+    batch.num_chunks = (num_tokens + batch.tokens_per_chunk - 1) / batch.tokens_per_chunk;
+    batch.chunk_of = make_rank_divider(batch.tokens_per_chunk);
+    const bool room = workspace_bytes >= size_t(hist_bytes + first_bytes + slot_bytes) * size_t(num_src);
+    batch.in_full = batch.num_chunks > kSendColumns || (by_dest != nullptr && !columns_by_dest_fit(num_experts)) || !room;
+    const bool slots_in_scratch = !batch.in_full || pair_slot == nullptr;
+    const int64_t scratch_bytes = hist_bytes + first_bytes + (slots_in_scratch ? slot_bytes : 0);
+    EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(ranked ? scratch_bytes : hist_bytes) * size_t(num_src));
+    EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(workspace) & 15) == 0);
+    EP_HOST_ASSERT(by_dest == nullptr || (num_src == 1 && src_ranks == nullptr && fused_recv == nullptr &&
+                                          own_rows_direct == nullptr));
+    // own_rows_direct (the form of the one-call dispatch in more than one launch): as in the single launch, the rows
+    // for this rank's own experts go straight to their packed position behind the lower ranks' rows
+    EP_HOST_ASSERT(own_rows_direct == nullptr || (num_src == 1 && src_ranks == nullptr));
+    EP_HOST_ASSERT(num_tokens < 65535 && num_src <= 65535);
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
-    // How slots get ranked: up to kSelfRankMaxEntries entries the send kernel sweeps every earlier
-    // entry itself; beyond, it sweeps its own chunk on top of the per-chunk histograms.
-    const int tpc = n <= kSelfRankMaxEntries || fused_recv != nullptr ? 0 : sweep_chunk_tokens(num_topk);
-    const int chunks = tpc > 0 ? (num_tokens + tpc - 1) / tpc : 0;
-    if (tpc > 0) {
-        ll_chunk_hist_kernel<<<dim3(chunks, num_src), 1024, size_t(num_experts) * sizeof(int32_t), stream>>>(
-            topk_idx, n, tpc * num_topk, num_experts, scratch_bytes, ws);
-        EP_LAUNCH_CHECK();
-    }
-    const bool prefix_in_block = by_dest != nullptr && by_dest_tables_in_send(n, num_experts, chunks);
-    if (by_dest != nullptr && !prefix_in_block) {  // the tables the by-destination rows are placed by
-        EP_HOST_ASSERT(num_src == 1 && src_ranks == nullptr && fused_recv == nullptr && own_rows_direct == nullptr);
-        ll_by_dest_prefix_kernel<<<1, 1024, size_t(num_experts + 1) * sizeof(int32_t), stream>>>(
-            topk_idx, n, num_experts, num_ranks, max_tokens, tpc > 0 ? reinterpret_cast<const int32_t*>(ws) : nullptr,
-            chunks, send_count, *by_dest);
-        EP_LAUNCH_CHECK();
+    if (ranked) {
+        batch.hists = reinterpret_cast<int32_t*>(ws);
+        batch.own_first = own_rows_direct != nullptr ? reinterpret_cast<int32_t*>(ws + hist_bytes) : nullptr;
+        batch.slots = slots_in_scratch ? reinterpret_cast<int32_t*>(ws + hist_bytes + first_bytes) : pair_slot;
+        batch.stride = scratch_bytes / 4;
+        if (batch.num_chunks > 0) {
+            ll_rank_chunk_kernel<<<dim3(batch.num_chunks, num_src), kRankWaves * kWave, size_t(num_experts) * kRankWaves,
+                                   stream>>>(topk_idx, n, num_topk, num_experts, reinterpret_cast<int32_t*>(ws), batch,
+                                             recv_count, num_ranks, rank, max_tokens);
+            EP_LAUNCH_CHECK();
+        }
     }
 
     const int pieces = row_format == kRowBF16 ? (hidden * 2 + 1023) / 1024 : (hidden / kGroup + 7) / 8;
@@ -957,7 +1180,6 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     // Workgroups of four waves stay: with eight, 509 tokens of hidden 4096 took 19.1 us instead of 17.0.
     if (fused_recv != nullptr && n > 1536 && waves > 4) waves = 8;
     if (fused_recv != nullptr && waves < 4) waves = 4;  // the receive workgroups want a few waves each
-    EP_HOST_ASSERT(num_tokens < 65535 && num_src <= 65535);
     // floor(e / E_l) == umulhi(e, ceil(2^32 / E_l)) for every e below 2^16.
     const uint32_t experts_per_rank = uint32_t(num_experts / num_ranks);
     const uint32_t magic =
@@ -971,19 +1193,20 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     sa.num_ranks = num_ranks, sa.rank = rank, sa.max_tokens = max_tokens;
     sa.pieces_per_row = pieces, sa.split_log2 = split_log2;
     sa.rank_of_expert_magic = magic;
-    sa.scratch_stride = scratch_bytes, sa.scratch_base = ws;
-    sa.tokens_per_chunk = tpc;
     sa.recv_staging = reinterpret_cast<uint8_t*>(recv_staging);
     sa.send_slots = reinterpret_cast<uint8_t*>(send_slots);
     sa.pair_slot = pair_slot, sa.recv_count = recv_count, sa.send_count = send_count;
     sa.expert_prefix = by_dest != nullptr ? by_dest->expert_prefix : nullptr;
     sa.prefix_in_block = prefix_in_block ? 1 : 0;
     sa.by_dest = by_dest != nullptr ? *by_dest : ByDestTables{nullptr, nullptr, nullptr};
-    if (by_dest != nullptr)
-        EP_HOST_ASSERT(num_src == 1 && src_ranks == nullptr && fused_recv == nullptr && own_rows_direct == nullptr);
+    if (ranked && batch.in_full) {
+        ll_rank_finish_kernel<<<dim3(batch.num_chunks + 1, num_src), 1024, size_t(num_experts + 1) * sizeof(int32_t), stream>>>(
+            sa, batch);
+        EP_LAUNCH_CHECK();
+    }
 
     if (fused_recv != nullptr) {  // single launch: send workgroups, the counting workgroup, receive workgroups
-        EP_HOST_ASSERT(tpc == 0 && num_src == 1 && src_ranks == nullptr);
+        EP_HOST_ASSERT(num_src == 1 && src_ranks == nullptr);
         const int num_send_blocks = blocks_per_token * num_tokens;
         int64_t fused_recv_blocks = (fused_recv_wave_items + waves - 1) / waves;
         fused_recv_blocks = fused_recv_blocks < 1 ? 1 : (fused_recv_blocks > 1024 ? 1024 : fused_recv_blocks);
@@ -1020,31 +1243,39 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         return 0;
     }
 
-    // The receive index rides along when the chunk histograms exist (its own counts come from them)
+    // The receive index rides along with the rows of a ranked one-call dispatch
     FusedIndexArgs index = {};
     int index_rows = 0;
-    if (fused_index != nullptr && tpc > 0 && num_src == 1 && own_rows_direct != nullptr) {
+    if (fused_index != nullptr && ranked) {
         index = *fused_index;
-        index.chunk_hist = reinterpret_cast<const int32_t*>(ws);
-        index.num_chunks = (num_tokens + tpc - 1) / tpc;
+        index.chunk_hist = batch.hists, index.num_chunks = batch.num_chunks;
         index_rows = (num_experts + blocks_per_token - 1) / blocks_per_token;
         if (num_tokens + 1 + index_rows > 65535) index_rows = 0, index = FusedIndexArgs{};
     }
     if (index_was_fused != nullptr) *index_was_fused = index_rows > 0;
-    const dim3 grid(blocks_per_token, num_tokens + 1 + index_rows, num_src);  // + the counting row, + the index rows
-    const size_t lds = size_t(index_rows > 0 ? 2 * (num_experts + 1) : num_experts + 1) * sizeof(int32_t);
-    // own_rows_direct (the two-launch form of the one-call dispatch): as in the single launch, the rows
-    // for this rank's own experts go straight to their packed position behind the lower ranks' rows
-    EP_HOST_ASSERT(own_rows_direct == nullptr || (num_src == 1 && src_ranks == nullptr));
     const DirectOut direct = own_rows_direct != nullptr ? *own_rows_direct : DirectOut{nullptr, nullptr, nullptr};
     // rows read once and written K times (about that many: a dropped selection writes nothing)
     const int64_t traffic = int64_t(num_src) * num_tokens *
                             (int64_t(hidden) * 2 + int64_t(num_topk) * row_payload_bytes(hidden, row_format));
     const bool streams = traffic > send_stream_bytes();
-#define DEEPEP_LAUNCH_SEND(FMT)                                                           \
-    do {                                                                                  \
-        if (streams) ll_send_kernel<FMT, true><<<grid, waves * kWave, lds, stream>>>(sa, direct, index, index_rows);  \
-        else ll_send_kernel<FMT, false><<<grid, waves * kWave, lds, stream>>>(sa, direct, index, index_rows);         \
+    // + the index rows, + the counting row (ll_rank_finish_kernel has the counts)
+    const dim3 grid(blocks_per_token, index_rows + num_tokens + (ranked && batch.in_full ? 0 : 1), num_src);
+    if (grid.y == 0) return 0;
+    const size_t lds = size_t(index_rows > 0 ? 2 * (num_experts + 1) : num_experts + 1) * sizeof(int32_t);
+    int topk_log2 = 0;
+    while ((1 << topk_log2) < num_topk) ++topk_log2;
+#define DEEPEP_LAUNCH_SEND_AS(FMT, STREAM)                                                                             \
+    do {                                                                                                               \
+        if (ranked)                                                                                                    \
+            ll_send_ranked_kernel<FMT, STREAM><<<grid, waves * kWave, lds, stream>>>(sa, direct, batch, index,         \
+                                                                                     index_rows, topk_log2);           \
+        else                                                                                                           \
+            ll_send_kernel<FMT, STREAM><<<grid, waves * kWave, lds, stream>>>(sa);                                     \
+    } while (0)
+#define DEEPEP_LAUNCH_SEND(FMT)                            \
+    do {                                                   \
+        if (streams) DEEPEP_LAUNCH_SEND_AS(FMT, true);     \
+        else DEEPEP_LAUNCH_SEND_AS(FMT, false);            \
     } while (0)
     switch (row_format) {
         case kRowBF16: DEEPEP_LAUNCH_SEND(kRowBF16); break;
@@ -1053,6 +1284,7 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         default: DEEPEP_LAUNCH_SEND(kRowFP8UE8M0); break;
     }
 #undef DEEPEP_LAUNCH_SEND
+#undef DEEPEP_LAUNCH_SEND_AS
     EP_LAUNCH_CHECK();
     return 0;
 }
@@ -1129,7 +1361,7 @@ int deepep_ll_dispatch_send_static(const void* x, const int64_t* topk_idx, int n
     if (int rc = check_ll_shape(num_tokens, hidden, num_topk, num_experts, num_ranks, rank,
                                 num_max_dispatch_tokens_per_rank, row_format))
         return rc;
-    const size_t need = size_t(route_scratch_bytes(num_tokens, num_topk, num_experts));
+    const size_t need = size_t(chunk_hist_bytes(num_tokens, num_topk, num_experts));
     if (need > kStaticScratchBytes) {
         set_error("Assertion", __FILE_NAME__, __LINE__,
                   "batch too large for the static route scratch: ceil(num_tokens / floor(2048 / num_topk)) * "
@@ -1354,7 +1586,7 @@ int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx, int num_
         const DirectOut direct = {reinterpret_cast<uint8_t*>(packed_recv_x),
                                   reinterpret_cast<uint8_t*>(packed_recv_scales), packed_recv_src_info};
         // When the receive side will run as index + flat copy, the index is built by extra workgroups of
-        // the send launch: three launches (histograms, send + index, copy) instead of four.
+        // the send launch: three launches (slots, send + index, copy) instead of four.
         FusedIndexArgs index = {};
         const bool flat_copy =
             segment_workspace != nullptr && num_experts <= 1024 &&

@@ -1198,6 +1198,102 @@ def test_all_to_all_with_an_empty_batch(rt, receive):
     assert (st.send_flat.view(torch.int16) == 0x7FC0).all()
 
 
+@pytest.mark.parametrize("t,k,e", [(1025, 8, 64), (1171, 7, 96), (1100, 8, 66), (2400, 5, 256), (1025, 64, 260),
+                                   (8193, 1, 8), (8192, 8, 64), (8193, 8, 64), (13200, 5, 256), (1025, 8, 4096)])
+def test_slots_of_batches_ranked_ahead_of_their_rows(rt, t, k, e):
+    """Past 8192 entries a launch of its own ranks them, whole tokens of up to 2048 entries a workgroup, and what the
+    chunks before a token's hold is added by the waves that store its rows: for up to 32 chunks and, by destination, up to
+    64 experts or 256 in fours; beyond by a launch between the two.  With odd numbers of entries, experts named more than
+    once by a token, hot ones, and entries that name none."""
+    g = torch.Generator().manual_seed(t * 10 + e)
+    topk = torch.randint(0, e, (t, k), generator=g)
+    topk[torch.rand((t, k), generator=g) < 0.3] = e // 2
+    topk[torch.rand((t, k), generator=g) < 0.05] = -1
+    topk[3, 0], topk[t - 1, k - 1] = e, (1 << 32) + 1
+    live = (topk >= 0) & (topk < e)
+    flat = torch.where(live, topk, 0).view(-1).numpy()
+    ok = live.view(-1).numpy()
+    order = np.argsort(np.where(ok, flat, e), kind="stable")
+    total = np.bincount(flat[ok], minlength=e)
+    first = np.concatenate([[0], np.cumsum(total)])
+    slot = np.full(t * k, -1, dtype=np.int64)
+    mine = order[:int(ok.sum())]
+    slot[mine] = np.arange(mine.size) - first[flat[mine]]
+    m, h, r, rank = t, 128, 4 if e % 4 == 0 else 2, 1
+    slot[slot >= m] = -1
+    count = np.minimum(total, m)
+
+    x = torch.randn((t, h), generator=g).to(torch.bfloat16)
+    by_dest = send_by_dest_on_gpu(rt, x, topk, rank, r, e, m, O.ROW_BF16)
+    assert np.array_equal(by_dest.pair_slot.cpu().numpy().reshape(-1)[:t * k], slot)
+    assert np.array_equal(by_dest.send_count.cpu().numpy(), count)
+    prefix = np.concatenate([[0], np.cumsum(count)])
+    assert np.array_equal(by_dest.send_expert_prefix.cpu().numpy(), prefix)
+    stride = rt.capi.load().deepep_ll_row_stride(h, O.ROW_BF16)
+    rows = by_dest.send_rows.cpu().view(-1, stride)
+    pair = np.flatnonzero(slot >= 0)
+    at = torch.from_numpy(prefix[flat[pair]] + slot[pair])
+    token = torch.from_numpy(pair // k)
+    assert torch.equal(rows[at, :2 * h], x.view(torch.uint8)[token])
+    tail = rows[at, 2 * h:2 * h + 16].contiguous().view(torch.int32)
+    per_rank = e // r
+    expert = torch.from_numpy(flat[pair])
+    want = torch.stack([token, torch.from_numpy(pair % k), torch.full_like(token, rank), expert % per_rank], dim=1)
+    assert torch.equal(tail, want.to(torch.int32))
+
+    lib = rt.capi.load()
+    n_src = 2  # two sources at once, whose slots nobody asked for, and the slots alone
+    staging = torch.empty((e // r) * r * m * stride, dtype=torch.uint8, device="cuda")
+    recv_count = torch.full((e // r, r), -7, dtype=torch.int32, device="cuda")
+    ws = torch.empty(n_src * lib.deepep_ll_dispatch_workspace_bytes(t, k, e), dtype=torch.uint8, device="cuda")
+    both_x = torch.stack([x, x.flip(0)]).cuda()
+    both_topk = torch.stack([topk, topk]).cuda()
+    src = torch.tensor([0, r - 1], dtype=torch.int32, device="cuda")
+    if staging.numel() < 2 ** 32:
+        rt.capi.check(lib.deepep_loopback_dispatch_from_peers(
+            rt.capi.ptr(both_x), rt.capi.ptr(both_topk), rt.capi.ptr(src), n_src, t, h, k, e, r, rank, m, O.ROW_BF16,
+            rt.capi.ptr(staging), rt.capi.ptr(recv_count), rt.capi.ptr(ws), ws.numel(), rt.ll.current_stream_ptr()))
+        mine = torch.from_numpy(count[rank * per_rank:(rank + 1) * per_rank]).to(torch.int32)
+        assert torch.equal(recv_count[:, 0].cpu(), mine) and torch.equal(recv_count[:, r - 1].cpu(), mine)
+        assert (recv_count[:, 1:r - 1] == -7).all()
+        le = per_rank // 2
+        got = staging.view(per_rank, r, m, stride)[le, r - 1, :int(mine[le]), 2 * h:2 * h + 4].contiguous().view(torch.int32)
+        of_expert = (expert == rank * per_rank + le).numpy()
+        assert torch.equal(got.view(-1).cpu(), token[torch.from_numpy(of_expert)].to(torch.int32))
+        for name, scratch in (("deepep_ll_dispatch_send", (rt.capi.ptr(ws), ws.numel())), ("deepep_ll_dispatch_send_static", ())):
+            sent = torch.full((e,), -7, dtype=torch.int32, device="cuda")
+            pair_slot = torch.full((t, k), -7, dtype=torch.int32, device="cuda")
+            recv_count.fill_(-7)
+            rt.capi.check(getattr(lib, name)(
+                rt.capi.ptr(both_x), rt.capi.ptr(both_topk), t, h, k, e, r, rank, m, O.ROW_BF16, rt.capi.ptr(staging),
+                rt.capi.ptr(recv_count), None, rt.capi.ptr(sent), rt.capi.ptr(pair_slot), *scratch, rt.ll.current_stream_ptr()))
+            assert np.array_equal(pair_slot.cpu().numpy().reshape(-1), slot), name
+            assert np.array_equal(sent.cpu().numpy(), count), name
+            assert torch.equal(recv_count[:, rank].cpu(), mine), name
+
+
+@pytest.mark.parametrize("rank", [0, 5])
+def test_one_call_dispatch_of_few_entries_and_many_rows(rt, rank):
+    """Fewer than 8192 entries but more rows than a single launch takes: the slots ahead, the index beside the rows."""
+    r, t, h, k, e = 8, 300, 256, 8, 64
+    g = torch.Generator().manual_seed(77)
+    x_all = torch.randn((r, t, h), generator=g).to(torch.bfloat16)
+    topk = torch.topk(torch.rand((r, t, e), generator=g) + (torch.arange(e) // 8 == rank) * 0.6, k, dim=-1)[1]
+    topk[:, ::7, 2] = -1
+    want = O.ll_dispatch(x_all, topk.contiguous(), rank, e, t, O.ROW_FP8)
+    shape = rt.ll.LLShape(num_ranks=r, rank=rank, num_experts=e, max_tokens=t, hidden=h, num_topk=k, fmt=O.ROW_FP8)
+    st = rt.ll.LowLatencyState(shape)
+    st.expected_rows = 8193
+    st.segment_workspace = torch.empty(rt.capi.load().deepep_ll_segment_workspace_bytes(e, t), dtype=torch.uint8,
+                                       device="cuda")
+    world = rt.lb.LoopbackWorld(r, rank, seed=0)
+    world.set_inputs(x_all.cuda(), topk.contiguous().cuda())
+    x, own = world.own_inputs()
+    run_dispatch(st, world, x, own, None, True)
+    assert int(want["packed_recv_count"].sum()) > 8192
+    check_dispatch(st, want, O.ROW_FP8)
+
+
 def test_send_by_dest_with_repeated_experts_and_full_pairs(rt):
     """Tokens naming an expert more than once: pairs beyond a pair's M slots are dropped from the counts,
     the prefixes and the buffer alike."""
