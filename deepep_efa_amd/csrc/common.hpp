@@ -221,11 +221,13 @@ inline int flat_row_threads(int num_vec, int most) {
 
 // Traffic above which a kernel streams (the memory-side cache holds 256 MB).
 inline int64_t stream_bytes() { return int64_t(192) << 20; }
-// The dispatch streams from 64 MB of traffic on (the send side's payload stores; in the single launch
-// the receive side's row copies too): with clean caches the hint makes no difference from 512 to 2560
+// The dispatch streams from 64 MB of traffic on (its stores: the send side's payload and, in the single launch, the
+// received rows): with clean caches the hint makes no difference from 512 to 2560
 // tokens, with the caches full of another call's dirty lines the send is 18 to 24 % faster with it and
-// the single launch 11 to 16 %.  (The single-launch combine measured the other way: slower at 256 and
-// 512 tokens with the lower bound, so it keeps the 192 MB.)
+// the single launch 11 to 16 %.  The staged rows themselves, which a transport has just put there, are read the ordinary
+// way.  Dispatch of 700 tokens of hidden 4096 and 1000 of 7168, us, hint on the loads too / not: behind a step on other
+// buffers 17.4 / 13.5 and 34.4 / 31.0, behind a read of 512 MB 18.8 / 18.2 and 36.9 / 36.4, on the same buffers 17.2 / 12.6
+// and 34.6 / 29.4; behind a write of 512 MB, whose lines the rows then push out, 19.5 / 22.1 and 39.4 / 44.
 inline int64_t send_stream_bytes() { return int64_t(64) << 20; }
 
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every

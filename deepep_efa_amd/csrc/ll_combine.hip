@@ -32,7 +32,7 @@ struct CombineSendArgs {
 };
 
 // No LDS and no barrier: each wave holds the segment counts and begins in registers.
-template <int kPer, bool kStream>
+template <int kPer, bool kStreamLoad, bool kStreamStore>
 __device__ __forceinline__ void combine_send_rows_impl(const CombineSendArgs& a, int block, int num_blocks,
                                                        bool skip_own) {
     const int lane = lane_id(), w = wave_in_block();
@@ -82,24 +82,24 @@ __device__ __forceinline__ void combine_send_rows_impl(const CombineSendArgs& a,
             continue;
         int v_begin, v_end;
         row_part_range(num_vec, a.parts_log2, part, v_begin, v_end);
-        RowPart<4, kStream> piece;
+        RowPart<4, kStreamLoad, kStreamStore> piece;
         piece.load(src, v_begin, v_end, lane);
         piece.store(dst, v_begin, lane);
     }
     DEEPEP_PHASE(2);
 }
 
-template <bool kStream>
+template <bool kStreamLoad, bool kStreamStore>
 __device__ __forceinline__ void combine_send_rows(const CombineSendArgs& a, int block, int num_blocks, bool skip_own) {
     if (a.num_local_experts * a.num_ranks <= 4 * kWave)
-        combine_send_rows_impl<4, kStream>(a, block, num_blocks, skip_own);
+        combine_send_rows_impl<4, kStreamLoad, kStreamStore>(a, block, num_blocks, skip_own);
     else
-        combine_send_rows_impl<16, kStream>(a, block, num_blocks, skip_own);
+        combine_send_rows_impl<16, kStreamLoad, kStreamStore>(a, block, num_blocks, skip_own);
 }
 
 // skip_own: the rows owed to this rank itself stay where they are (the reduce reads them from x).
 __global__ __launch_bounds__(256) void ll_combine_send_kernel(CombineSendArgs a, bool skip_own) {
-    combine_send_rows<false>(a, blockIdx.x, gridDim.x, skip_own);
+    combine_send_rows<false, false>(a, blockIdx.x, gridDim.x, skip_own);
 }
 
 // ---------------------------------------------------------------------
@@ -275,8 +275,27 @@ __global__ __launch_bounds__(256) void ll_combine_index_kernel(CombineIndexArgs 
 // gain 2 to 4 %, 1.7 to 2.05 lose as much (577 x 5120 at top-4 29.1 -> 30.2), more than three lose 0 to 1 %: six there.
 // ---------------------------------------------------------------------
 constexpr int64_t kWorkgroupsAtOnce = 256 * 8;  // compute units, workgroups of four waves on each
+// Which accesses of the single-launch combine stream.  Past 48 MB of traffic its stores and the gathered rows, which
+// nobody touches again, while the rows to be returned, which the experts have just written, are read the ordinary way;
+// past 192 MB, where nothing survives from one kernel to the next, those too.  The hint keeps the combine from displacing
+// what its neighbours left, and from waiting for their dirty lines to be written back.  Microseconds of dispatch + combine
+// without it below 192 MB / with it, behind steps on other buffers (three in turn; the wider one, called from C++), and of
+// their kernels behind a read (R) and behind a write (W) of 512 MB each:
+//   150 x 7168 to 32 ranks     24.8 / 24.2    R 20.4 / 20.2    W 28.8 / 24.9
+//   256 x 4096                 25.1 / 23.1    R 20.2 / 19.4    W 26.9 / 22.4
+//   300 x 7168                 46.6 / 38.4    R 34.9 / 34.4    W 51.2 / 40.6
+//   500 x 2048                 26.6 / 24.0    R 21.5 / 20.9    W 28.4 / 24.1
+//   509 x 4096, no row return  28.9 / 25.1    R 23.7 / 22.8    W 33.4 / 25.8
+//   700 x 4096                 54.6 / 45.1    R 43.6 / 44.6    W 63.7 / 51.9    (the dispatch's own share: common.hpp)
+//   900 x 2048                 42.5 / 38.8    R 33.5 / 33.0    W 47.0 / 38.6
+// Replayed on one set of buffers, all of it still cached, it costs 150 to 180 tokens 5 to 7 %, 509 3 % and gains from 700 on.
+// Below, 128 x 7168 (46 MB) gains 3 % on other buffers and loses 2 % behind a read, 256 x 5120 at top-4 (33 MB) and 77 x 5120
+// lose 2 % both ways.  The hint on the rows to be returned as well: 128 and 150 tokens 3 % slower than without any, 256 x
+// 4096 24.3 us, 500 x 2048 25.8, 700 x 4096 45.7, but 300 x 7168 37.2 and behind a write another 8 to 13 % less.
+enum CombineHint : int { kHintNone = 0, kHintGather = 1, kHintAll = 2 };
+constexpr int64_t kGatherStreamBytes = int64_t(48) << 20;
 
-template <bool kStream, bool kInTurn>
+template <int kHint, bool kInTurn>
 __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs sa, CombineRecvArgs ra,
                                                                int num_recv_blocks) {
     extern __shared__ int32_t dyn_lds[];  // reduce workgroups: own_begin[E_l]
@@ -292,10 +311,11 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
             dyn_lds[le] = (lr & 0xffffffffll) > 0 ? int(lr >> 32) : 0;
         }
         lds_barrier();
-        combine_recv_piece<kStream, kInTurn>(ra, t, piece, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
+        combine_recv_piece<kHint >= kHintGather, kInTurn>(ra, t, piece, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
                                              sa.num_local_experts, int64_t(sa.max_tokens) * sa.num_ranks);
     } else {
-        combine_send_rows<kStream>(sa, block - num_recv_blocks, int(gridDim.x) - num_recv_blocks, true);
+        combine_send_rows<kHint >= kHintAll, kHint >= kHintGather>(sa, block - num_recv_blocks,
+                                                                  int(gridDim.x) - num_recv_blocks, true);
     }
 }
 
@@ -712,15 +732,16 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     if (send_blocks > 16384) send_blocks = 16384;
     if (recv_blocks + send_blocks == 0) return 0;
     const size_t lds = size_t(sa.num_local_experts) * sizeof(int32_t);
-    // rows returned (read + written) plus rows gathered: past what the caches hold, stream.  Beside more than
-    // kLargeBatchRows rows it always pays (11946 of 4 KB, 61.2 -> 57.5 us a step).
+    // rows returned (read + written) plus rows gathered: past what the caches hold, stream (CombineHint).  Beside more
+    // than kLargeBatchRows rows it always pays (11946 of 4 KB, 61.2 -> 57.5 us a step).
     const int64_t traffic = (2 * rows + int64_t(num_tokens) * num_topk) * hidden * 2;
-#define DEEPEP_LAUNCH_FUSED(STREAM, IN_TURN)                                                           \
-    ll_combine_fused_kernel<STREAM, IN_TURN><<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds,     \
+#define DEEPEP_LAUNCH_FUSED(HINT, IN_TURN)                                                             \
+    ll_combine_fused_kernel<HINT, IN_TURN><<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds,     \
                                                reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks))
-    if (large || traffic > stream_bytes()) DEEPEP_LAUNCH_FUSED(true, false);
-    else if (recv_blocks + send_blocks <= kWorkgroupsAtOnce) DEEPEP_LAUNCH_FUSED(false, true);
-    else DEEPEP_LAUNCH_FUSED(false, false);
+    if (large || traffic > stream_bytes()) DEEPEP_LAUNCH_FUSED(kHintAll, false);
+    else if (traffic > kGatherStreamBytes) DEEPEP_LAUNCH_FUSED(kHintGather, false);
+    else if (recv_blocks + send_blocks <= kWorkgroupsAtOnce) DEEPEP_LAUNCH_FUSED(kHintNone, true);
+    else DEEPEP_LAUNCH_FUSED(kHintNone, false);
 #undef DEEPEP_LAUNCH_FUSED
     EP_LAUNCH_CHECK();
     return 0;

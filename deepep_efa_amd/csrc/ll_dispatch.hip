@@ -887,7 +887,7 @@ struct RecvItem {
     int le, source, slot;  // slot: the row's place among the rows copied for the expert, own rows not counted
     int v_begin;
     bool carries_tail;  // also moves the row's scales and source index
-    RowPart<kRecvDepth, kStream> payload;
+    RowPart<kRecvDepth, false, kStream> payload;
     uint32_t scale;  // a lane's scale word, with the tail
     int32_t info;
 };

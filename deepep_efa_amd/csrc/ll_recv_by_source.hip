@@ -466,7 +466,7 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
         const int j = row - seg_first;
         const uint8_t* from = a.rows + uint64_t(uint32_t(src * int(a.slot_rows) + in_message + j)) * stride;
         row_part_range(num_vec, a.parts_log2, part, v_begin, v_end);
-        RowPart<kOrderedDepth, false> payload;
+        RowPart<kOrderedDepth, false, false> payload;
         payload.load(from, v_begin, v_end, lane);
         const bool carries_tail = part == parts - 1;  // the last part is the shortest
         uint32_t tail_scale = 0;

@@ -179,7 +179,7 @@ __device__ __forceinline__ void row_part_range(int num_vec, int parts_log2, int 
 
 // Vectors [v_begin, v_end) of a row, moved by one wave, kDepth KiB of it in flight: the first of them in `r` between
 // load() and store(), which moves the others too.
-template <int kDepth, bool kStream>
+template <int kDepth, bool kStreamLoad, bool kStreamStore>
 struct RowPart {
     u32x4 r[kDepth];
     const uint8_t* src;
@@ -188,17 +188,17 @@ struct RowPart {
         src = row + v_begin * 16, bytes = (v_end - v_begin) * 16;
         const auto from = row_buffer(src, bytes);
 #pragma unroll
-        for (int u = 0; u < kDepth; ++u) r[u] = load_row_u32x4<kStream>(from, lane * 16 + u * 1024);
+        for (int u = 0; u < kDepth; ++u) r[u] = load_row_u32x4<kStreamLoad>(from, lane * 16 + u * 1024);
     }
     __device__ __forceinline__ void store(uint8_t* row, int v_begin, int lane) {
         const auto from = row_buffer(src, bytes), to = row_buffer(row + v_begin * 16, bytes);
         for (int base = lane * 16;;) {
 #pragma unroll
-            for (int u = 0; u < kDepth; ++u) store_row_u32x4<kStream>(to, base + u * 1024, r[u]);
+            for (int u = 0; u < kDepth; ++u) store_row_u32x4<kStreamStore>(to, base + u * 1024, r[u]);
             base += kDepth * 1024;
             if (base - lane * 16 >= bytes) return;
 #pragma unroll
-            for (int u = 0; u < kDepth; ++u) r[u] = load_row_u32x4<kStream>(from, base + u * 1024);
+            for (int u = 0; u < kDepth; ++u) r[u] = load_row_u32x4<kStreamLoad>(from, base + u * 1024);
         }
     }
 };

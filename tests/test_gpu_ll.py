@@ -1968,6 +1968,30 @@ def test_combine_in_one_launch_and_in_two(rt, h, hints):
     assert all(torch.equal(sums[0], o) for o in sums[1:])
 
 
+@pytest.mark.parametrize("h,k,hints", [(7168, 8, (1404, 1405, 6085, 6086)),  # 48 and 192 MB: three forms of the launch
+                                       (640, 3, (4096, 8192))])
+def test_combine_whose_accesses_stream_in_part(rt, h, k, hints):
+    """Which accesses of the single-launch combine carry the streaming hint changes no row and no sum."""
+    r, rank, t, e = 8, 3, 40, 64
+    x_all, topk_all, w = make_world(r, t, h, k, e, seed=h, drop=9)
+    st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, 160, O.ROW_BF16, one_call=True)
+    y = torch.randn(st.packed_recv_x.shape, generator=torch.Generator().manual_seed(h)).bfloat16().cuda()
+    world.combine_from_peers(st, mode=1, seed=5)
+    topk, w, got = topk_all[rank].cuda(), w[rank].cuda(), []
+    for hint in (0,) + hints:
+        st.combine_send_slots.view(torch.int16).fill_(0x7FC0)
+        out = torch.zeros((t, h), dtype=torch.bfloat16, device="cuda")
+        if hint == 0:
+            st.combine_send(y)
+            st.combine_recv(topk, w, out)
+        else:
+            st.expected_rows = hint
+            st.combine(y, topk, w, out)
+        torch.cuda.synchronize()
+        got.append((st.combine_send_slots.view(torch.int16).clone(), out.view(torch.int16).clone()))
+    assert all(torch.equal(a, b) for other in got[1:] for a, b in zip(got[0], other))
+
+
 @pytest.mark.parametrize("t,h,k,e,hints", [
     (64, 4096, 8, 64, (3399, 3400)),  # 2048 workgroups, which the chip holds at once, and 2049
     (61, 1024, 3, 512, (3572, 3573)),  # the same with more than 256 segments
