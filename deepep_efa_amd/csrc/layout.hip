@@ -558,10 +558,11 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // each list ascends, and workgroups 8 apart -- on one XCD, sharing an L2 -- work
 // through one group, so a source row is read once and found in that L2 by the
 // other ranks.  Any routing gives the same result; a skewed one only shares less.
-// Past 128 MB the packed rows are stored with the non-temporal hint: otherwise they push the source rows, and
-// whatever the caches hold of others, out again.  Below that a transport that reads them next finds them in the
-// memory-side cache (256 MB), which is worth more to the two together than the hint is to the pack.  Microseconds of
-// pack and pack + copy of the packed rows, ordinary stores against the hint (R = 8, four sets of tensors in turn):
+// Past 48 MB the packed rows are stored with the non-temporal hint: otherwise they push the source rows, and
+// whatever the caches hold of others, out again.  What reads them next is a transport, at the rate of its links, to which
+// the memory-side cache (256 MB) is worth nothing; a copy on this GPU would find them there and take back what the hint
+// gives.  Microseconds of pack and pack + copy of the packed rows, ordinary stores against the hint (R = 8, four sets of
+// tensors in turn):
 //    19 MB   7.0 / 5.0    13.8 / 15.3     118 MB  35.7 / 21.7   72.4 / 78.0
 //    39 MB  10.0 / 8.9    25.6 / 29.5     129 MB  40.4 / 23.2   83.8 / 85.6
 //    78 MB  24.0 / 15.3   48.8 / 54.2     140 MB  42.0 / 25.3   93.9 / 91.4
@@ -587,13 +588,15 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // / 256 threads, and the same with a copy of the packed rows behind it: 36 MB 9.0 / 8.7 us, 21.7 / 22.8; 45 MB 10.6 / 10.2,
 // 26.3 / 27.5; 54 MB 11.6 / 12.9; 60 MB 13.7 / 15.5, 33.4 / 34.7; 80 MB 18.8 / 19.7, 43.7 / 44.3; 95 MB 23.7 / 24.2, 54.8 / 53.0;
 // 111 MB 27.1 / 28.2, 65.0 / 63.3; rows of 8704 to 28672 bytes alike (51 MB of 8704 11.3 / 10.2, 54 MB 12.6 / 12.7), narrower ones have
-// 256 either way.  In list order, past 128 MB, the
+// 256 either way.  A whole prefill on three sets of buffers in turn, hint past 128 MB / past 48: 1000 x 14336 bytes (72 MB)
+// 63.0 / 59.1 us, 2000 x 7168 (73 MB) 90.2 / 83.6 (with the reduce's), 4000 x 4096 to 16 ranks (98 MB) 80.8 / 77.9; past 24: the
+// same.  In list order, past 128 MB, the
 // same threads move one vector at a time: two trips to memory stand in front of a row there.  4096 x 14336 88.5 us against 96.1
 // with two vectors in flight, 4096 x 7168 45.5 and 47.9 (46.0 to 48 with twice the threads), 12289 x 14336 258 and 267.
 // ---------------------------------------------------------------------
 constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of one of 8 groups; 16 MB of 16, 24 MB of more
 constexpr int64_t kPackSourceBytes = int64_t(3) << 20;  // source bytes of a group
-constexpr int64_t kPackStreamBytes = int64_t(128) << 20;
+constexpr int64_t kPackStreamBytes = int64_t(48) << 20;
 constexpr int64_t kPackSmallBytes = int64_t(50) << 20;
 
 struct PackArgs {

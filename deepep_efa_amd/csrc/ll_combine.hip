@@ -229,6 +229,11 @@ __device__ __forceinline__ void combine_recv_piece(const CombineRecvArgs& a, uin
 // bytes each, 90.5 -> 88.7 us, 6.0 TB/s; two to fourteen waves 91 to 95, neighbouring tokens on one XCD no gain).
 // Eight waves a SIMD while the rows stay in the caches: 820 to 1000 tokens of 5120 at top-4 4 % less than with six, else the
 // same.  Streaming, six serve HBM as well or better (87.5 us against 87.8 at 4096 tokens).
+// It streams from 32 MB of rows on, which nobody reads again.  A whole exchange to 8 ranks on three sets of buffers in turn,
+// from 192 MB on / from 32: 700 tokens of 7168 93.6 / 90.5 us, 1000 of 4096 81.6 / 78.8, 1500 of 5120 at top-6 113.4 / 109.8,
+// 2047 of 4096 133.8 / 131.2, 400 of 7168 (44 MB) 55 from 48 MB on and 51.4 so; 256 of 7168 (28 MB) 38.6 / 39.5 with it.  Behind a
+// read of 512 MB the reduce alone 12.0 / 11.7 at 400 tokens and 19.1 / 19.0 at 700, behind a write 20.1 / 11.5 and 34.2 / 19.3.
+constexpr int64_t kReduceStreamBytes = int64_t(32) << 20;
 template <bool kStream>
 __global__ __launch_bounds__(256) void ll_combine_recv_kernel(CombineRecvArgs a, const uint8_t* own_x,
                                                               const int64_t* layout_range, int rank,
@@ -339,7 +344,14 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
 // 320000 1537 and 1399.
 // 16376 rows of 14336 bytes 78.7 -> 75.4 us (6.2 TB/s), 1024 rows 7.7 -> 6.4, against two vectors a thread and the
 // record behind the number of records.
+// From 24 MB on (both directions) its stores stream, from 48 MB the loads too.  A whole exchange on three sets of buffers
+// in turn, from 192 MB on / so, other lines alike: 128 tokens of 7168 to 8 ranks 26.6 / 24.9 us, 256 of 4096 to 32 30.5 / 29.1,
+// 256 of 7168 to 16 46.4 / 39.5, 400 to 8 62.4 / 59.0, 1500 of 5120 at top-6 113.4 / 109.4; stores alone also past 48 MB 42.4 for
+// the 256, 60.8 for the 400 and 87.7 instead of 81 for 700.  Alone behind a read of 512 MB 256 tokens 13.3 / 12.9, 400 18.5 /
+// 18.6, 128 7.4 / 7.6, behind a write 18.1 / 13.4, 27.9 / 19.1, 9.4 / 9.9; an exchange of 256 on one set of buffers 35.5 / 38.4.
 // ---------------------------------------------------------------------
+constexpr int64_t kReturnStreamBytes = int64_t(48) << 20, kReturnStreamStoreBytes = int64_t(24) << 20;
+
 struct CombineByDestPeers {  // direct delivery
     uint8_t* const* peer_recv;   // [R] device pointers, or null
     const int64_t* peer_rows;    // [R] rows each peer buffer holds
@@ -349,7 +361,7 @@ struct CombineByDestPeers {  // direct delivery
     int num_ranks;
 };
 
-template <bool kStream, bool kPeers>
+template <bool kStreamLoad, bool kStreamStore, bool kPeers>
 __global__ __launch_bounds__(1024) void ll_combine_send_by_dest_kernel(
     const uint32_t* __restrict__ num_recv_tokens, const uint32_t* __restrict__ padded_index,
     const int32_t* __restrict__ record_packed_row, const uint32_t* __restrict__ combine_send_offset,
@@ -386,7 +398,7 @@ __global__ __launch_bounds__(1024) void ll_combine_send_by_dest_kernel(
                 }
             }
             if (dst != nullptr && src_row < x_rows)  // < 0: the record has no row
-                block_copy_row<1, kStream, kStream>(x + src_row * row_bytes, dst, num_vec, threadIdx.x, threads);
+                block_copy_row<1, kStreamLoad, kStreamStore>(x + src_row * row_bytes, dst, num_vec, threadIdx.x, threads);
         }
         if (uint64_t(block) + grid >= flat_rounds_end(records)) break;
         block += grid, i = flat_row_of_block(block);
@@ -531,7 +543,7 @@ int deepep_ll_combine_send(const void* x, const int64_t* layout_range, int hidde
 
 static void launch_reduce(const CombineRecvArgs& ra, const uint8_t* own, const int64_t* layout_range, int rank,
                           int num_local_experts, int num_ranks, const CombineIndexArgs* index, hipStream_t hs) {
-    const bool stream_rows = int64_t(ra.num_tokens) * ra.num_topk * ra.hidden * 2 > stream_bytes();
+    const bool stream_rows = int64_t(ra.num_tokens) * ra.num_topk * ra.hidden * 2 > kReduceStreamBytes;
     const int waves = stream_rows ? 1 : 4;
     const int index_blocks = index != nullptr ? index->num_local_experts * index->num_ranks : 0;
     const CombineIndexArgs ia = index != nullptr ? *index : CombineIndexArgs{};
@@ -606,17 +618,21 @@ int deepep_ll_combine_send_by_dest(const void* x, const int32_t* record_packed_r
     const int num_vec = hidden * 2 / 16, threads = flat_row_threads(num_vec, sized_for > 32768 ? 1024 : 512);
     const unsigned grid = flat_grid_blocks(sized_for, row_capacity, threads);
     const int64_t x_rows = std::min(int64_t(num_experts) * num_max_dispatch_tokens_per_rank, int64_t(1) << 31);
-#define DEEPEP_LAUNCH_BY_DEST(STREAM, PEERS)                                                                            \
-    ll_combine_send_by_dest_kernel<STREAM, PEERS><<<grid, threads, 0, reinterpret_cast<hipStream_t>(stream)>>>(         \
+#define DEEPEP_LAUNCH_BY_DEST(LOAD, STORE, PEERS)                                                                       \
+    ll_combine_send_by_dest_kernel<LOAD, STORE, PEERS><<<grid, threads, 0, reinterpret_cast<hipStream_t>(stream)>>>(    \
         num_recv_tokens, padded_index, record_packed_row, combine_send_offset, uint32_t(row_capacity),                  \
         uint32_t(x_rows), reinterpret_cast<const uint8_t*>(x),                                                          \
         reinterpret_cast<uint8_t*>(send_flat), num_vec, threads, grid, peers)
-    if (2 * rows * hidden * 2 > stream_bytes()) {
-        if (peer_recv_flat != nullptr) DEEPEP_LAUNCH_BY_DEST(true, true);
-        else DEEPEP_LAUNCH_BY_DEST(true, false);
+    const int64_t traffic = 2 * rows * hidden * 2;
+    if (traffic > kReturnStreamBytes) {
+        if (peer_recv_flat != nullptr) DEEPEP_LAUNCH_BY_DEST(true, true, true);
+        else DEEPEP_LAUNCH_BY_DEST(true, true, false);
+    } else if (traffic > kReturnStreamStoreBytes) {
+        if (peer_recv_flat != nullptr) DEEPEP_LAUNCH_BY_DEST(false, true, true);
+        else DEEPEP_LAUNCH_BY_DEST(false, true, false);
     } else {
-        if (peer_recv_flat != nullptr) DEEPEP_LAUNCH_BY_DEST(false, true);
-        else DEEPEP_LAUNCH_BY_DEST(false, false);
+        if (peer_recv_flat != nullptr) DEEPEP_LAUNCH_BY_DEST(false, false, true);
+        else DEEPEP_LAUNCH_BY_DEST(false, false, false);
     }
 #undef DEEPEP_LAUNCH_BY_DEST
     EP_LAUNCH_CHECK();

@@ -122,6 +122,11 @@ __global__ __launch_bounds__(kMetaThreads) void combine_positions_kernel(
 // ---------------------------------------------------------------------
 constexpr int kReduceWindow = 32;
 constexpr int kReduceRound = 8 * kReduceWindow;
+// From here on it streams.  A whole prefill on three sets of buffers in turn, from 192 MB on / from 96: 2000 x 7168 (145 MB)
+// 90.0 -> 83.6 us, 3000 x 5120 at top-6 to 32 ranks 108.0 / 100.3, 4000 x 2048 to 16 (98 MB) 80.7 / 74.3; behind a write of 512
+// MB the reduce alone 60.4 / 31.4 at 2000 tokens, behind a read 32.4 / 31.1, on one set of buffers the prefill 81 / 84.
+// From 48 MB on: 1000 x 7168 (72 MB) no change, 1000 x 4096 to 16 ranks (50 MB) 53.4 -> 56.8.
+constexpr int64_t kReduceStreamBytes = int64_t(96) << 20;
 
 template <bool kStream>  // the returned rows exceed what the caches hold: read them with the non-temporal hint
 __global__ __launch_bounds__(512) void combine_reduce_kernel(
@@ -286,7 +291,7 @@ int deepep_combine_reduce(const void* recv_x, const float* recv_topk_weights, co
         EP_LAUNCH_CHECK();
     }
     const int pieces = (hidden * 2 + 1023) / 1024;
-    const bool stream_rows = max_rows * hidden * 2 > stream_bytes();
+    const bool stream_rows = max_rows * hidden * 2 > kReduceStreamBytes;
     // a token's pieces over as few workgroups of about equal size as eight waves allow, or, up to 3.5 copies, four
     const int most = 2 * max_rows > 7 * int64_t(num_tokens) ? 8 : 4;
     const int per_token = (pieces + most - 1) / most, waves = stream_rows ? (pieces + per_token - 1) / per_token : 4;

@@ -323,8 +323,11 @@ def test_pack_rows(capi, rows, row_bytes, scale_bytes):
     (6000, 2048, 0, 8, (1.0, 0.0, 0.02, 1.0, 0.5, 0.0, 0.9, 0.001), 1.0),  # lists of very different lengths
     (4000, 2048, 0, 8, 0.66, 0.6),     # a list cut off before its end
     (4000, 2048, 0, 8, 0.66, 1.5),     # room for more rows than there are
-    (9000, 4096, 4, 8, 0.5, 1.0),      # past 128 MB of packed rows, where they are stored past the caches
-    (5500, 4112, 0, 72, 0.1, 1.0),     # the same in list order
+    (3000, 4096, 4, 8, 0.5, 1.0),      # 49 MB of packed rows
+    (3200, 4096, 4, 8, 0.5, 1.0),      # 52, where they are stored past the caches
+    (2500, 4112, 0, 72, 0.1, 1.0),     # the same in list order
+    (9000, 4096, 4, 8, 0.5, 1.0),
+    (5500, 4112, 0, 72, 0.1, 1.0),
     (9000, 8192, 516, 8, 0.72, 1.0),   # more than two groups an XCD; scales wider than a wave
     (9000, 8192, 516, 8, 0.3, 1.0),  # few copies a row: the groups are bound by their source rows
     (9000, 8192, 0, 8, 0.5, 1.0),  # more than 16 groups for their size alone

@@ -1749,6 +1749,50 @@ def test_return_by_destination_over_record_counts(rt, records, hidden):
     assert torch.equal(out.cpu(), want)
 
 
+@pytest.mark.parametrize("hidden,hints", [(7168, (877, 878, 1755, 1756)), (8192, (768, 769, 1536, 1537))])
+def test_return_by_destination_whose_accesses_stream_in_part(rt, hidden, hints):
+    """24 and 48 MB of expected traffic: which accesses carry the streaming hint changes no row."""
+    r, e, m, capacity, records = 4, 8, 256, 2048, 300
+    g = torch.Generator().manual_seed(hidden)
+    x = torch.randn((e * m, hidden), generator=g).bfloat16().cuda()
+    packed = torch.randperm(e * m, generator=g)[:capacity].int()
+    offset = torch.randperm(capacity, generator=g).int()
+    num = torch.tensor([records, records], dtype=torch.int32, device="cuda")
+    on_gpu = [v.cuda() for v in (packed, torch.arange(capacity, dtype=torch.int32), offset)]
+    want = torch.full((capacity, hidden), 3.0, dtype=torch.bfloat16, device="cuda")
+    want[on_gpu[2][:records].long()] = x[on_gpu[0][:records].long()]
+    for hint in hints:
+        out = torch.full((capacity, hidden), 3.0, dtype=torch.bfloat16, device="cuda")
+        rt.capi.check(rt.capi.load().deepep_ll_combine_send_by_dest(
+            rt.capi.ptr(x), rt.capi.ptr(on_gpu[0]), None, rt.capi.ptr(on_gpu[1]), rt.capi.ptr(on_gpu[2]), rt.capi.ptr(num),
+            capacity, hidden, e, r, m, rt.capi.ptr(out), None, None, None, None, hint, torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(out, want), hint
+
+
+@pytest.mark.parametrize("t", [292, 293])  # 32 MB of gathered rows, and more
+def test_reduce_around_its_streaming_bound(rt, t):
+    """The reduce of a batch is the reduces of its tokens."""
+    h, k, e = 7168, 8, 16
+    g = torch.Generator().manual_seed(t)
+    topk = torch.topk(torch.rand((t, e), generator=g), k, dim=-1)[1]
+    topk[5, 3] = -1
+    slots = torch.arange(t, dtype=torch.int32).repeat_interleave(k).view(t, k)
+    slots[topk < 0] = -1
+    staging = torch.randn((e, t, h), generator=g).bfloat16().cuda()
+    w, topk, slots = torch.rand((t, k), generator=g).cuda(), topk.cuda(), slots.cuda()
+    lib = rt.capi.load()
+
+    def reduce(lo, hi):
+        out = torch.full((hi - lo + 1, h), 7.0, dtype=torch.bfloat16, device="cuda")
+        parts = [v[lo:hi].contiguous() for v in (topk, w, slots)]
+        rt.capi.check(lib.deepep_ll_combine_recv(rt.capi.ptr(staging), *[rt.capi.ptr(v) for v in parts], hi - lo, h, k, e, t, 0,
+                                                 rt.capi.ptr(out), torch.cuda.current_stream().cuda_stream))
+        assert (out[hi - lo] == 7.0).all()
+        return out[:hi - lo]
+
+    assert torch.equal(reduce(0, t), torch.cat([reduce(0, 100), reduce(100, t)]))
+
+
 @pytest.mark.parametrize("hidden", [8192, 16512])  # a round of 1024 threads, and more than two
 @pytest.mark.parametrize("records,hint", [(700, 32768), (700, 32769), (33792 + 257, 32769)])  # the last has more than workgroups
 def test_return_by_destination_of_many_records(rt, records, hidden, hint):
