@@ -175,15 +175,49 @@ static size_t get_low_latency_rdma_size_hint(int num_max_dispatch_tokens_per_ran
 // ---------------------------------------------------------------------------
 // EventHandle (reference: csrc/event.hpp:9-25)
 // ---------------------------------------------------------------------------
+static void hip_check(hipError_t e, int line) {
+    if (e != hipSuccess) throw EPException("HIP", "deep_ep_cpp.cpp", line, hipGetErrorString(e));
+}
+
+// An event that streams wait for, and nobody else: the handle cannot be queried, synchronised with or shared.
+// fence: whether the record makes what was written before it visible to the host and to other devices too, which writes
+// the caches back and invalidates them between two kernels.  Streams of one device need none: they see one another's
+// writes when the kernels that made them have ended (hipEventDisableSystemFence), and a host or another device that reads
+// behind one of them has the fence of that wait or copy.
+class DeviceEvent {
+    hipEvent_t event = nullptr;
+    const c10::Device device;
+
+public:
+    DeviceEvent(const HostStream& stream, bool fence) : device(stream.unwrap().device()) {
+        const c10::DeviceGuard guard(device);
+        hip_check(hipEventCreateWithFlags(&event, hipEventDisableTiming | (fence ? 0u : hipEventDisableSystemFence)),
+                  __LINE__);
+        const hipError_t e = hipEventRecord(event, stream.stream());
+        if (e != hipSuccess) (void)hipEventDestroy(event);
+        hip_check(e, __LINE__);
+    }
+    DeviceEvent(const DeviceEvent&) = delete;
+    ~DeviceEvent() {
+        try {
+            const c10::DeviceGuard guard(device);
+            (void)hipEventDestroy(event);
+        } catch (...) {  // the process is ending
+        }
+    }
+    void wait_on(const HostStream& waiter) const {
+        const c10::DeviceGuard guard(waiter.unwrap().device());
+        hip_check(hipStreamWaitEvent(waiter.stream(), event, 0), __LINE__);
+    }
+};
+
 struct EventHandle {
-    std::shared_ptr<torch::Event> event;
+    std::shared_ptr<DeviceEvent> event;
 
     EventHandle() : EventHandle(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()) {}
-    explicit EventHandle(const HostStream& stream) {
-        event = std::make_shared<torch::Event>(torch::kCUDA);
-        event->record(stream);
-    }
-    void stream_wait_for(const HostStream& waiter) const { waiter.unwrap().wait(*event); }
+    explicit EventHandle(const HostStream& stream, bool fence = true)
+        : event(std::make_shared<DeviceEvent>(stream, fence)) {}
+    void stream_wait_for(const HostStream& waiter) const { event->wait_on(waiter); }
     void current_stream_wait() const { stream_wait_for(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
 };
 
@@ -1451,8 +1485,14 @@ struct PlainCall<F> {
 // The event of a low-latency call, with or without async_finish.  It is recorded before the call returns: recorded
 // when somebody waits, it would also cover what the caller's stream was given in between, which takes away the
 // overlap with it and hangs where that work waits for the waiter.  A record takes the stream 3 us beside kernels of
-// 8 us and the host 2 (two launches and a record each: 24.3 us against 18.6 without); a step records two.
-static pybind11::object recorded_event() { return pybind11::cast(EventHandle()); }
+// 8 us, 1 without the fence, and the host 2; a step records two.  A dispatch's is without: what follows it are the experts,
+// on a stream of this device.  A combine's has the fence, which a wait for its stream then need not bring.  Microseconds
+// of a step, fences on both / on the combine's / on none, in a row and each waited for:
+//   1 token     13.5 / 11.8 / 10.3    22.3 / 20.8 / 23.8        128   23.0 / 20.9 / 18.9    32.0 / 30.3 / 33.4
+//   77 in bf16  17.4 / 15.5 / 13.7    26.2 / 24.5 / 27.5        509   25.3 / 24.0 / 22.0    33.9 / 33.0 / 35.3
+static pybind11::object recorded_event(bool fence) {
+    return pybind11::cast(EventHandle(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(), fence));
+}
 
 static pybind11::object hook_object(bool wanted) {
     if (!wanted) return pybind11::none();
@@ -1476,7 +1516,7 @@ static PyObject* low_latency_dispatch_call(PyObject*, PyObject* const* a, Py_ssi
                                                    c.num_experts);
         }
         (void)bool_argument(a[10]);
-        const pybind11::object count = result_object(c.packed_recv_count), event = recorded_event(),
+        const pybind11::object count = result_object(c.packed_recv_count), event = recorded_event(false),
                                hook = hook_object(bool_argument(a[11]));
         return pybind11::reinterpret_steal<pybind11::object>(
             PyTuple_Pack(5, c.recv_result.ptr(), count.ptr(), c.handle_result.ptr(), event.ptr(), hook.ptr()));
@@ -1498,7 +1538,7 @@ static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssiz
             tensor_argument(of_handle(1)), optional_tensor_argument(a[5]), int_argument(of_handle(2)),
             int_argument(of_handle(4)), bool_argument(a[6]), optional_tensor_argument(a[9]), bool_argument(a[10])));
         (void)bool_argument(a[7]);
-        const pybind11::object event = recorded_event(), hook = hook_object(bool_argument(a[8]));
+        const pybind11::object event = recorded_event(true), hook = hook_object(bool_argument(a[8]));
         return pybind11::reinterpret_steal<pybind11::object>(PyTuple_Pack(3, combined.ptr(), event.ptr(), hook.ptr()));
     });
 }

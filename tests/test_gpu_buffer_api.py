@@ -254,6 +254,55 @@ def test_another_stream_waits_on_the_returned_events(deep_ep, caller, async_fini
     buffer.destroy()
 
 
+def test_what_other_streams_read_behind_the_events(deep_ep):
+    """A kernel, a copy on the device and a copy to the host on another stream see everything a call wrote, call after
+    call over the same buffers, and the call sees what another stream's event was recorded behind."""
+    from deepep_efa_amd.deep_ep_cpp import EventHandle
+    num_ranks, rank, t, h, k, e = 8, 2, 64, 2048, 4, 64
+    buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=num_ranks,
+                            sim_rank=rank, sim_seed=17)
+    x, topk_idx = buffer.loopback_synthesise(t, h, k, e)
+    w = torch.rand((t, k), generator=torch.Generator().manual_seed(4)).cuda()
+    recv_x, _, handle, _, _ = buffer.low_latency_dispatch(x, topk_idx, t, e, use_fp8=False)
+    y = recv_x.clone()
+    buffer.low_latency_combine(y, topk_idx, w, handle)
+    buffer.loopback_clear_world()
+    rounds = 60
+    scale = [1.0 + 0.125 * (i % 7) for i in range(rounds)]
+
+    def call(i):
+        mine_x, mine_y = x * scale[i], y * scale[i]
+        recv_x, count, handle, dispatched, _ = buffer.low_latency_dispatch(mine_x, topk_idx, t, e, use_fp8=False)
+        combined, reduced, _ = buffer.low_latency_combine(mine_y, topk_idx, w, handle)
+        return recv_x, combined, dispatched, reduced
+
+    want = []
+    for i in range(7):
+        recv_x, combined, _, _ = call(i)
+        torch.cuda.synchronize()
+        want.append((recv_x.clone(), combined.clone()))
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+    got = []
+    torch.cuda.synchronize()
+    for i in range(rounds):
+        with torch.cuda.stream(mine):
+            recv_x, combined, dispatched, reduced = call(i)
+        with torch.cuda.stream(other):
+            reduced.current_stream_wait()
+            host = torch.empty(combined.shape, dtype=combined.dtype, pin_memory=True)
+            host.copy_(combined, non_blocking=True)
+            dispatched.current_stream_wait()
+            got.append((recv_x.clone(), combined + 0, host))
+            read = deep_ep.EventOverlap(EventHandle())
+        with torch.cuda.stream(mine):
+            read.current_stream_wait()  # the next call writes over what was read
+    other.synchronize()
+    for i, (recv_x, combined, host) in enumerate(got):
+        assert torch.equal(recv_x, want[i % 7][0]) and torch.equal(combined, want[i % 7][1])
+        assert torch.equal(host, want[i % 7][1].cpu()), i
+    buffer.destroy()
+
+
 def _step_with_events(deep_ep):
     """A buffer and a call that runs one small step on the current stream and returns its two events."""
     num_ranks, rank, t, h, k, e = 8, 2, 32, 1024, 4, 64
