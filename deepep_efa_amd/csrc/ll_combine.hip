@@ -297,13 +297,13 @@ constexpr int64_t kWorkgroupsAtOnce = 256 * 8;  // compute units, workgroups of 
 // Below, 128 x 7168 (46 MB) gains 3 % on other buffers and loses 2 % behind a read, 256 x 5120 at top-4 (33 MB) and 77 x 5120
 // lose 2 % both ways.  The hint on the rows to be returned as well: 128 and 150 tokens 3 % slower than without any, 256 x
 // 4096 24.3 us, 500 x 2048 25.8, 700 x 4096 45.7, but 300 x 7168 37.2 and behind a write another 8 to 13 % less.
-enum CombineHint : int { kHintNone = 0, kHintGather = 1, kHintAll = 2 };
 constexpr int64_t kGatherStreamBytes = int64_t(48) << 20;
 
-template <int kHint, bool kInTurn>
-__global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs sa, CombineRecvArgs ra,
-                                                               int num_recv_blocks) {
-    extern __shared__ int32_t dyn_lds[];  // reduce workgroups: own_begin[E_l]
+// kStream: stores and gathered rows; kStreamRows: the rows to be returned as well.
+template <bool kStream, bool kStreamRows, bool kInTurn>
+__device__ __forceinline__ void combine_fused_block(const CombineSendArgs& sa, const CombineRecvArgs& ra,
+                                                    int num_recv_blocks, int32_t* dyn_lds) {
+    // dyn_lds: reduce workgroups, own_begin[E_l]
     const int block = blockIdx.x;
     if (block < num_recv_blocks) {
         // the token's index loads and the own-range loads go out together: one memory round trip
@@ -316,12 +316,24 @@ __global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs s
             dyn_lds[le] = (lr & 0xffffffffll) > 0 ? int(lr >> 32) : 0;
         }
         lds_barrier();
-        combine_recv_piece<kHint >= kHintGather, kInTurn>(ra, t, piece, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
+        combine_recv_piece<kStream, kInTurn>(ra, t, piece, sel, sa.x, dyn_lds, sa.rank * sa.num_local_experts,
                                              sa.num_local_experts, int64_t(sa.max_tokens) * sa.num_ranks);
     } else {
-        combine_send_rows<kHint >= kHintAll, kHint >= kHintGather>(sa, block - num_recv_blocks,
-                                                                  int(gridDim.x) - num_recv_blocks, true);
+        combine_send_rows<kStreamRows, kStream>(sa, block - num_recv_blocks, int(gridDim.x) - num_recv_blocks, true);
     }
+}
+
+template <bool kStream, bool kInTurn>
+__global__ __launch_bounds__(256) void ll_combine_fused_kernel(CombineSendArgs sa, CombineRecvArgs ra,
+                                                               int num_recv_blocks) {
+    extern __shared__ int32_t dyn_lds[];
+    combine_fused_block<kStream, false, kInTurn>(sa, ra, num_recv_blocks, dyn_lds);
+}
+
+__global__ __launch_bounds__(256) void ll_combine_fused_past_caches_kernel(CombineSendArgs sa, CombineRecvArgs ra,
+                                                                           int num_recv_blocks) {
+    extern __shared__ int32_t dyn_lds[];
+    combine_fused_block<true, true, false>(sa, ra, num_recv_blocks, dyn_lds);
 }
 
 // ---------------------------------------------------------------------
@@ -748,16 +760,15 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     if (send_blocks > 16384) send_blocks = 16384;
     if (recv_blocks + send_blocks == 0) return 0;
     const size_t lds = size_t(sa.num_local_experts) * sizeof(int32_t);
-    // rows returned (read + written) plus rows gathered: past what the caches hold, stream (CombineHint).  Beside more
+    // rows returned (read + written) plus rows gathered: past what the caches hold, stream.  Beside more
     // than kLargeBatchRows rows it always pays (11946 of 4 KB, 61.2 -> 57.5 us a step).
     const int64_t traffic = (2 * rows + int64_t(num_tokens) * num_topk) * hidden * 2;
-#define DEEPEP_LAUNCH_FUSED(HINT, IN_TURN)                                                             \
-    ll_combine_fused_kernel<HINT, IN_TURN><<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds,     \
-                                               reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks))
-    if (large || traffic > stream_bytes()) DEEPEP_LAUNCH_FUSED(kHintAll, false);
-    else if (traffic > kGatherStreamBytes) DEEPEP_LAUNCH_FUSED(kHintGather, false);
-    else if (recv_blocks + send_blocks <= kWorkgroupsAtOnce) DEEPEP_LAUNCH_FUSED(kHintNone, true);
-    else DEEPEP_LAUNCH_FUSED(kHintNone, false);
+#define DEEPEP_LAUNCH_FUSED(KERNEL) \
+    KERNEL<<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds, reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks))
+    if (large || traffic > stream_bytes()) DEEPEP_LAUNCH_FUSED(ll_combine_fused_past_caches_kernel);
+    else if (traffic > kGatherStreamBytes) DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<true, false>));
+    else if (recv_blocks + send_blocks <= kWorkgroupsAtOnce) DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<false, true>));
+    else DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<false, false>));
 #undef DEEPEP_LAUNCH_FUSED
     EP_LAUNCH_CHECK();
     return 0;
