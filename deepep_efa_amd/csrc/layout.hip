@@ -590,9 +590,10 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
 // 111 MB 27.1 / 28.2, 65.0 / 63.3; rows of 8704 to 28672 bytes alike (51 MB of 8704 11.3 / 10.2, 54 MB 12.6 / 12.7), narrower ones have
 // 256 either way.  A whole prefill on three sets of buffers in turn, hint past 128 MB / past 48: 1000 x 14336 bytes (72 MB)
 // 63.0 / 59.1 us, 2000 x 7168 (73 MB) 90.2 / 83.6 (with the reduce's), 4000 x 4096 to 16 ranks (98 MB) 80.8 / 77.9; past 24: the
-// same.  In list order, past 128 MB, the
+// same.  In list order, where the rows stream, the
 // same threads move one vector at a time: two trips to memory stand in front of a row there.  4096 x 14336 88.5 us against 96.1
-// with two vectors in flight, 4096 x 7168 45.5 and 47.9 (46.0 to 48 with twice the threads), 12289 x 14336 258 and 267.
+// with two vectors in flight, 4096 x 7168 45.5 and 47.9 (46.0 to 48 with twice the threads), 12289 x 14336 258 and 267; against
+// two vectors and ordinary stores 60 MB 17.3 and 18.4, 80 MB 22.6 and 24.0, 110 MB 31.0 and 34.4.
 // ---------------------------------------------------------------------
 constexpr int64_t kPackGroupBytes = int64_t(12) << 20;  // packed bytes of one of 8 groups; 16 MB of 16, 24 MB of more
 constexpr int64_t kPackSourceBytes = int64_t(3) << 20;  // source bytes of a group

@@ -23,7 +23,7 @@
 
 #include "../../include/deepep_hip.h"
 
-// Route scratch (the chunk histograms of ll_chunk_hist_kernel) for deepep_ll_dispatch_send_static,
+// Route scratch (the chunk histograms of ll_rank_chunk_kernel) for deepep_ll_dispatch_send_static,
 // whose callers cannot allocate.  The array is part of the code object: every GPU the library runs
 // on holds its own copy, at its own address, until the process ends.  Host code never passes this
 // name to a kernel; it passes the device address hipGetSymbolAddress returns (static_route_scratch).
