@@ -83,6 +83,10 @@ __device__ __forceinline__ int lane_id() { return __builtin_amdgcn_mbcnt_hi(~0u,
 // stays in SGPRs and row addresses become scalar loads.
 __device__ __forceinline__ int wave_in_block() { return __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6); }
 
+// Threads of the workgroup, as a scalar.  No launch here has a partial workgroup, which blockDim.x allows for: where the
+// compiler does not see that it need not, that is a vector load, waited for, ahead of everything else a kernel does.
+__device__ __forceinline__ int block_threads() { return int(__builtin_amdgcn_workgroup_size_x()); }
+
 // Stores through a pointer the compiler cannot prove to be global memory (one rebuilt from
 // integers, say) are emitted as flat stores, which also tick the LDS counter; these say "global".
 typedef __attribute__((address_space(1))) u32x4 global_u32x4;

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(kLayoutOneBlockThreads) void layout_count_kernel(
     uint32_t rank_magic, int num_nodes, uint8_t* __restrict__ is_token_in_rank, int32_t* __restrict__ partial,
     int32_t* __restrict__ per_rank, int32_t* __restrict__ per_node, int32_t* __restrict__ per_expert) {
     extern __shared__ int32_t hist[];  // [E + R + nodes]
-    const int tid = threadIdx.x, lane = lane_id(), threads = blockDim.x;
+    const int tid = threadIdx.x, lane = lane_id(), threads = block_threads();
     const int width = num_experts + num_ranks + num_nodes;
     for (int j = tid; j < width; j += threads) hist[j] = 0;
     lds_barrier();
@@ -466,7 +466,7 @@ __global__ __launch_bounds__(1024) void channel_prefix_kernel(const uint8_t* __r
                                                               int32_t* __restrict__ cpm) {
     extern __shared__ int32_t per_channel[];  // [C]
     const int dst = blockIdx.x, lane = lane_id(), w = wave_in_block();
-    const int waves = int(blockDim.x) >> 6;
+    const int waves = block_threads() >> 6;
     const int per = (num_tokens + num_channels - 1) / num_channels;
     for (int ch = w; ch < num_channels; ch += waves) {
         const int begin = min(per * ch, num_tokens), end = min(begin + per, num_tokens);
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
                                                                     int32_t* __restrict__ cpm) {
     extern __shared__ int32_t per_channel[];  // [C][8]
     const int q = blockIdx.x, lane = lane_id(), w = wave_in_block();
-    const int waves = int(blockDim.x) >> 6;
+    const int waves = block_threads() >> 6;
     const int per = (num_tokens + num_channels - 1) / num_channels;
     for (int ch = w; ch < num_channels; ch += waves) {
         const int begin = min(per * ch, num_tokens), end = min(begin + per, num_tokens);

@@ -36,7 +36,7 @@ template <int kPer, bool kStreamLoad, bool kStreamStore>
 __device__ __forceinline__ void combine_send_rows_impl(const CombineSendArgs& a, int block, int num_blocks,
                                                        bool skip_own) {
     const int lane = lane_id(), w = wave_in_block();
-    const int waves = int(blockDim.x) >> 6;
+    const int waves = block_threads() >> 6;
     const int num_ranks = a.num_ranks, max_tokens = a.max_tokens;
     const int num_segments = a.num_local_experts * num_ranks;
 

@@ -183,7 +183,7 @@ struct alignas(16) SendLds {
 __device__ __forceinline__ void expert_prefix_in_lds(const int64_t* __restrict__ topk_idx, int n, int num_experts,
                                                      int max_tokens, int32_t* hist, int32_t* wave_totals,
                                                      int32_t* counts_out) {
-    const int tid = threadIdx.x, threads = blockDim.x;
+    const int tid = threadIdx.x, threads = block_threads();
     for (int e = tid; e < num_experts; e += threads) hist[e] = 0;
     lds_barrier();
     constexpr int kAhead = 4;  // pairs of entries in flight per thread
@@ -233,7 +233,7 @@ __device__ __forceinline__ int wave_expert_prefix(const int32_t* hist, int num_e
 // The per-rank tables of the by-destination form from the prefix in LDS.
 __device__ __forceinline__ void by_dest_tables_out(const int32_t* hist, int num_experts, int num_ranks,
                                                    const ByDestTables& out) {
-    const int tid = threadIdx.x, threads = blockDim.x;
+    const int tid = threadIdx.x, threads = block_threads();
     for (int e = tid; e <= num_experts; e += threads) out.expert_prefix[e] = hist[e];
     const int experts_per_rank = num_experts / num_ranks;
     for (int r = tid; r < num_ranks; r += threads) {
@@ -249,14 +249,14 @@ __device__ __forceinline__ void send_count_block(const SendArgs& a, int b, int32
     const int n = a.num_tokens * a.num_topk;
     const int src_rank = a.src_ranks != nullptr ? a.src_ranks[b] : a.rank;
     const int64_t* my_topk = a.topk_idx + int64_t(b) * n;
-    for (int j = tid; j < a.num_experts; j += blockDim.x) lds_hist[j] = 0;
+    for (int j = tid; j < a.num_experts; j += block_threads()) lds_hist[j] = 0;
     lds_barrier();
-    for (int i = tid; i < n; i += blockDim.x) {
+    for (int i = tid; i < n; i += block_threads()) {
         const int64_t v = my_topk[i];
         if (v >= 0 && v < a.num_experts) atomicAdd(&lds_hist[int(v)], 1);
     }
     lds_barrier();
-    for (int e = tid; e < a.num_experts; e += blockDim.x)
+    for (int e = tid; e < a.num_experts; e += block_threads())
         emit_expert_count(e, lds_hist[e], a.num_experts, a.num_ranks, a.rank, src_rank, a.max_tokens, a.recv_count,
                           a.send_count);
 }
@@ -301,7 +301,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     const int src_rank = a.src_ranks != nullptr ? a.src_ranks[b] : a.rank;
     const int64_t* my_topk = a.topk_idx + int64_t(b) * n;
 
-    const int item = block_in_token * int(blockDim.x >> 6) + wave_in_block();
+    const int item = block_in_token * (block_threads() >> 6) + wave_in_block();
     const int split = 1 << a.split_log2;
     const bool wave_live = item < (a.pieces_per_row << a.split_log2);
     const int part = item & (split - 1);
@@ -335,7 +335,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     // value dropped): without branches around them the compiler can count them, so the first wait of
     // wave 0 -- for the token's own selections -- does not also wait out a second round trip for the
     // entries it sweeps.
-    const int threads = blockDim.x;
+    const int threads = block_threads();
     const bool prefix_in_block = kTables && a.prefix_in_block;
     const int sweep_end = prefix_in_block ? n : entry0;
     constexpr int kSweepAhead = 2;
@@ -594,7 +594,7 @@ __device__ __forceinline__ void ranked_counts(const SendArgs& a, const RankedBat
                                               int32_t* wave_totals) {
     const int32_t* hists = batch.hists + int64_t(b) * batch.stride;
     const int src_rank = a.src_ranks != nullptr ? a.src_ranks[b] : a.rank;
-    for (int e = threadIdx.x; e < a.num_experts; e += blockDim.x) {
+    for (int e = threadIdx.x; e < a.num_experts; e += block_threads()) {
         const int total = chunk_total(hists, batch.num_chunks, a.num_experts, e);
         if (a.expert_prefix == nullptr) {
             emit_expert_count(e, total, a.num_experts, a.num_ranks, a.rank, src_rank, a.max_tokens, a.recv_count,
@@ -615,7 +615,7 @@ __device__ __forceinline__ void ranked_counts(const SendArgs& a, const RankedBat
 __global__ __launch_bounds__(1024) void ll_rank_finish_kernel(SendArgs a, RankedBatch batch) {
     extern __shared__ int32_t before[];  // [E + 1]
     __shared__ int32_t wave_totals[kMaxBlockWaves];
-    const int tid = threadIdx.x, threads = blockDim.x, c = blockIdx.x, b = blockIdx.y;
+    const int tid = threadIdx.x, threads = block_threads(), c = blockIdx.x, b = blockIdx.y;
     if (c == batch.num_chunks) {
         ranked_counts(a, batch, b, before, wave_totals);
         return;
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave, 8) void ll_send_ranked_kernel
         return;
     }
     const int lane = lane_id(), num_topk = a.num_topk, num_experts = a.num_experts;
-    const int item = int(blockIdx.x) * int(blockDim.x >> 6) + wave_in_block();
+    const int item = int(blockIdx.x) * (block_threads() >> 6) + wave_in_block();
     if (item >= (a.pieces_per_row << a.split_log2)) return;
     const int split = 1 << a.split_log2, part = item & (split - 1), piece = item >> a.split_log2;
     const int64_t row_id = int64_t(b) * a.num_tokens + t;
@@ -840,7 +840,7 @@ struct OwnCountLoads {
 
 __device__ __forceinline__ void own_row_counts_begin(const RecvArgs& a, const int64_t* own_topk, int own_entries,
                                                      int32_t* own_cnt, OwnCountLoads& loads) {
-    const int tid = threadIdx.x, threads = blockDim.x;
+    const int tid = threadIdx.x, threads = block_threads();
     if (own_topk == nullptr) return;
     const auto list = entry_list(own_topk, own_entries);
 #pragma unroll
@@ -851,7 +851,7 @@ __device__ __forceinline__ void own_row_counts_begin(const RecvArgs& a, const in
 
 __device__ __forceinline__ void own_row_counts_finish(const RecvArgs& a, const int64_t* own_topk, int own_entries,
                                                       int own_rank, int32_t* own_cnt, OwnCountLoads& loads) {
-    const int tid = threadIdx.x, threads = blockDim.x;
+    const int tid = threadIdx.x, threads = block_threads();
     if (own_topk == nullptr) {  // the send kernel has finished: recv_count holds the own counts
         for (int le = tid; le < a.num_local_experts; le += threads)
             own_cnt[le] = a.recv_count[le * a.num_ranks + own_rank];
@@ -903,7 +903,7 @@ __device__ __forceinline__ void recv_rows_impl(const RecvArgs& a, int block, int
                                                const int64_t* own_topk, int own_entries, int own_rank, int32_t* lds,
                                                int32_t* wave_totals) {
     const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block();
-    const int threads = blockDim.x, waves = threads >> 6;
+    const int threads = block_threads(), waves = threads >> 6;
     const int num_ranks = a.num_ranks, max_tokens = a.max_tokens;
     const int num_segments = a.num_local_experts * num_ranks;
     const bool own_placed = own_rank >= 0;

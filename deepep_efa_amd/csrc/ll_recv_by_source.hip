@@ -35,7 +35,7 @@ constexpr int kBySourceMaxLocalExperts = 1024;
 // records [prefix[s], prefix[s + 1]) belong to source s.  prefix has num_ranks + 1 entries.
 __device__ __forceinline__ void source_prefix(const int32_t* __restrict__ recv_counts, int num_ranks, int32_t* prefix,
                                               int32_t* scan_tmp) {
-    for (int r = threadIdx.x; r < num_ranks; r += blockDim.x) {
+    for (int r = threadIdx.x; r < num_ranks; r += block_threads()) {
         const int c = recv_counts[r];
         prefix[r] = c < 0 ? 0 : c;
     }
@@ -69,7 +69,7 @@ constexpr int kBySourceSmallRecords = 4096;  // up to here (record capacity) the
 // of the launch belongs to the source s with chunk_prefix[s] <= g < chunk_prefix[s + 1].
 __device__ __forceinline__ void source_chunk_prefix(const int32_t* prefix, int num_ranks, int64_t records,
                                                     int32_t* chunk_prefix, int32_t* scan_tmp) {
-    for (int r = threadIdx.x; r < num_ranks; r += blockDim.x) {
+    for (int r = threadIdx.x; r < num_ranks; r += block_threads()) {
         int64_t begin = prefix[r], end = prefix[r + 1];
         if (end > records) end = records;
         if (begin > end) begin = end;
@@ -392,7 +392,7 @@ template <int kPer>
 __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int block, int num_copy_blocks,
                                                   int32_t* lds, int32_t* wave_totals) {
     const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block();
-    const int threads = blockDim.x, waves = threads >> 6;
+    const int threads = block_threads(), waves = threads >> 6;
     const int num_ranks = a.num_ranks, max_tokens = a.max_tokens, num_local = a.num_local_experts;
     const int num_segments = num_local * num_ranks;
     int32_t* sent = lds;                       // [S]

@@ -18,7 +18,7 @@ constexpr int kMaxBlockWaves = 16;
 
 __device__ __forceinline__ void block_exclusive_scan(int32_t* data, int n, int32_t* wave_totals) {
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
-    const int threads = blockDim.x, waves = threads >> 6;
+    const int threads = block_threads(), waves = threads >> 6;
     const int per = (n + threads - 1) / threads;
     const int lo = tid * per;
     int sum = 0;
@@ -333,7 +333,7 @@ struct FusedIndexArgs {
 };
 
 __device__ __forceinline__ void recv_index_block(const FusedIndexArgs& a, int seg, int32_t* lds, int32_t* wave_totals) {
-    const int tid = threadIdx.x, threads = blockDim.x;
+    const int tid = threadIdx.x, threads = block_threads();
     const int num_ranks = a.num_ranks, max_tokens = a.max_tokens;
     const int num_segments = a.num_local_experts * num_ranks;
     int32_t* flat = lds;                      // prefix over the rows that get descriptors
@@ -402,7 +402,7 @@ struct CombineIndexArgs {
 
 __device__ __forceinline__ void combine_index_block(const CombineIndexArgs& a, int seg, int32_t* flat,
                                                     int32_t* wave_totals) {
-    const int tid = threadIdx.x, threads = blockDim.x;
+    const int tid = threadIdx.x, threads = block_threads();
     const int num_ranks = a.num_ranks, max_tokens = a.max_tokens;
     const int num_segments = a.num_local_experts * num_ranks;
     const int64_t begin = a.layout_range[seg] >> 32;
