@@ -499,32 +499,41 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_send_kernel(SendArgs 
 }
 
 // ---------------------------------------------------------------------
-// Large batches: the entries are ranked one launch ahead of the rows, a workgroup a chunk.  A wave matches 64 entries
-// at a time against one another, a ballot for each bit of the expert, and keeps how many it has seen of an expert in a
-// byte of LDS; an entry's place in its chunk is what the waves before its own have of its expert, what its wave had
-// before, and the lanes before it.  The sums of the bytes are the chunk's histogram, and what the chunks before an
-// entry's have of its expert is added by whoever reads the place.  Nothing is read twice: one compute unit takes 18 bytes
-// a cycle of a list that is not in its L2, so workgroups that went through all entries before their own took 4.6 us for
-// 16376 entries and 7.7 for 32768, and this takes 2.7 (an empty kernel 2.4).
+// Large batches: the entries are ranked one launch ahead of the rows, four workgroups a chunk, 512 entries each.  A wave
+// matches its 64 entries against one another, a ballot for each bit of the expert, and leaves how many it has of an expert
+// in a byte of LDS; an entry's place in its chunk is what the parts before its own hold of its expert, counted by LDS adds,
+// what the waves before its own do, and the lanes before it.  The last part has all it takes for the chunk's histogram,
+// and what the chunks before an entry's hold of its expert is added by whoever reads the place.  Latency and instructions
+// bound it: four SIMDs issue for the whole of a workgroup.  One workgroup a chunk, two entries a lane, took a microsecond
+// longer: both launches of a send by destination of 2047 tokens of 7168 30.5 us against 29.5, of 1100 20.2 and 19.4, of 2000
+// of 2048 with 256 experts 15.2 and 14.2.  Workgroups that went through all entries before their own took 4.6 us for 16376
+// entries and 7.7 for 32768, at the 18 bytes a cycle that a compute unit takes of a list that is not in its L2 (an empty
+// kernel 2.4).
 // The first workgroup also writes where the rank's own rows of each local expert begin, behind those of the lower
 // source ranks (csrc/kernels/efa_kernels.cu:991-1010).
 // ---------------------------------------------------------------------
-constexpr int kRankWaves = 16;
+constexpr int kRankWaves = 8, kRankParts = 4, kRankPart = kRankWaves * kWave;
 
-__global__ __launch_bounds__(kRankWaves* kWave) void ll_rank_chunk_kernel(
+__global__ __launch_bounds__(kRankPart) void ll_rank_chunk_kernel(
     const int64_t* __restrict__ topk_idx, int n, int num_topk, int num_experts, int32_t* __restrict__ hists,
     RankedBatch batch, const int32_t* __restrict__ recv_count, int num_ranks, int rank, int max_tokens) {
-    extern __shared__ u32x4 rank_lds[];  // bytes [E][waves]
-    static_assert(kRankWaves == 16 && kRankChunkEntries <= 2 * kRankWaves * kWave, "a vector of bytes, two entries a lane");
+    extern __shared__ u32x2 rank_lds[];  // bytes [E][waves]; int32 [E], what the parts before hold
+    static_assert(kRankWaves == 8 && kRankChunkEntries <= kRankParts * kRankPart, "two words of bytes, an entry a lane");
     uint8_t* counts = reinterpret_cast<uint8_t*>(rank_lds);
+    int32_t* of_parts = reinterpret_cast<int32_t*>(rank_lds + num_experts);
     const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block(), b = blockIdx.y;
+    const int chunk = int(blockIdx.x) / kRankParts, part = int(blockIdx.x) % kRankParts;
     const int per_chunk = batch.tokens_per_chunk * num_topk;
-    const int begin = int(blockIdx.x) * per_chunk, end = min(begin + per_chunk, n);
+    const int begin = chunk * per_chunk, end = min(begin + per_chunk, n);
+    const int first = begin + part * kRankPart + tid;
+    const bool writes_histogram = part == kRankParts - 1;
+    if (!writes_histogram && begin + part * kRankPart >= end) return;
     const auto list = entry_list(topk_idx + int64_t(b) * n, n);
-    const int first = begin + w * 2 * kWave + lane;
-    u32x2 entry[2];
+    const u32x2 entry = __builtin_amdgcn_raw_buffer_load_b64(list, first * 8, 0, 0);
+    u32x2 earlier[kRankParts - 1];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) entry[i] = __builtin_amdgcn_raw_buffer_load_b64(list, (first + i * kWave) * 8, 0, 0);
+    for (int u = 0; u < kRankParts - 1; ++u)
+        earlier[u] = __builtin_amdgcn_raw_buffer_load_b64(list, u < part ? (begin + u * kRankPart + tid) * 8 : 0x7ffffff0, 0, 0);
     int own_rows = 0;
     const bool own_wanted = blockIdx.x == 0 && batch.own_first != nullptr;
     if (own_wanted) {  // a wave an expert, as far as there are waves
@@ -533,47 +542,39 @@ __global__ __launch_bounds__(kRankWaves* kWave) void ll_rank_chunk_kernel(
             own_rows += c < 0 ? 0 : (c > max_tokens ? max_tokens : c);
         }
     }
-    for (int e = tid; e < num_experts; e += kRankWaves * kWave) rank_lds[e] = u32x4{0u, 0u, 0u, 0u};
+    for (int e = tid; e < num_experts; e += kRankPart) rank_lds[e] = u32x2{0u, 0u}, of_parts[e] = 0;
     lds_barrier();
-    int before[2];
-    bool live[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t e = entry[i][0];
-        live[i] = first + i * kWave < end && entry[i][1] == 0u && e < uint32_t(num_experts);
-        uint64_t same = __ballot(live[i]);
-        for (int bit = 1; bit < num_experts; bit <<= 1) {
-            const bool set = (e & uint32_t(bit)) != 0u;
-            const uint64_t votes = __ballot(set);
-            same &= set ? votes : ~votes;
-        }
-        const int lower = __popcll(same & lanes_below(lane));
-        const int had = live[i] ? counts[e * kRankWaves + w] : 0;  // LDS serves a wave in order
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (live[i] && lower == 0) counts[e * kRankWaves + w] = uint8_t(had + __popcll(same));
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        before[i] = had + lower;
+    const uint32_t e = entry[0];
+    const bool live = first < end && entry[1] == 0u && e < uint32_t(num_experts);
+    uint64_t same = __ballot(live);
+    for (int bit = 1; bit < num_experts; bit <<= 1) {
+        const bool set = (e & uint32_t(bit)) != 0u;
+        const uint64_t votes = __ballot(set);
+        same &= set ? votes : ~votes;
     }
-    lds_barrier();
-    const auto count_of_waves = [&](uint32_t e, int waves) {  // what the waves before `waves` have of e
-        const u32x4 of = rank_lds[e];
-        uint32_t sum = 0;
+    const int lower = __popcll(same & lanes_below(lane));
+    if (live && lower == 0) counts[e * kRankWaves + w] = uint8_t(__popcll(same));
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {
+    for (int u = 0; u < kRankParts - 1; ++u)
+        if (u < part && begin + u * kRankPart + tid < end && earlier[u][1] == 0u && earlier[u][0] < uint32_t(num_experts))
+            atomicAdd(&of_parts[earlier[u][0]], 1);
+    lds_barrier();
+    const auto count_before = [&](uint32_t of, int waves) {  // what the parts and waves before have of an expert
+        const u32x2 bytes = rank_lds[of];
+        uint32_t sum = uint32_t(of_parts[of]);
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
             const int n_bytes = waves - d * 4;
-            sum = __builtin_amdgcn_sad_u8(of[d] & (n_bytes <= 0 ? 0u : (n_bytes >= 4 ? ~0u : (1u << (n_bytes * 8)) - 1)), 0u, sum);
+            sum = __builtin_amdgcn_sad_u8(bytes[d] & (n_bytes <= 0 ? 0u : (n_bytes >= 4 ? ~0u : (1u << (n_bytes * 8)) - 1)), 0u, sum);
         }
         return int(sum);
     };
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        if (first + i * kWave < end)
-            batch.slots[int64_t(b) * batch.stride + first + i * kWave] =
-                live[i] ? before[i] + count_of_waves(entry[i][0], w) : -1;
-    int32_t* out = hists + int64_t(b) * batch.stride + int64_t(blockIdx.x) * num_experts;
-    for (int e = tid; e < num_experts; e += kRankWaves * kWave) out[e] = count_of_waves(uint32_t(e), kRankWaves);
+    if (first < end)
+        batch.slots[int64_t(b) * batch.stride + first] = live ? count_before(e, w) + lower : -1;
+    if (writes_histogram) {
+        int32_t* out = hists + int64_t(b) * batch.stride + int64_t(chunk) * num_experts;
+        for (int of = tid; of < num_experts; of += kRankPart) out[of] = count_before(uint32_t(of), kRankWaves);
+    }
     if (own_wanted) {
         for (int le = w;;) {
             own_rows = wave_inclusive_sum(own_rows);
@@ -676,9 +677,10 @@ __device__ __forceinline__ void columns_by_dest(__amdgpu_buffer_rsrc_t hists, in
 // which without a table are the sums of all columns, or where own rows begin).
 // HBM bounds it: 4096 tokens of hidden 7168, top-8, fp8 (302 MB) 50 us, 6.0 TB/s, where workgroups that went through the
 // entries of their chunk and shared what they counted, three barriers ahead of the stores, took 61.  Both launches of a
-// send against histograms and that kernel: by destination to 8 ranks 4096 tokens 65 -> 59 us, of hidden 1024 23.4 -> 20.7,
-// 2047 tokens of 7168 30.0 -> 29.6, of 4096 with 256 experts 26.3 -> 22.9, 1100 23.6 -> 22.5; a dispatch of 4096 tokens 133 -> 125,
-// 2047 70 -> 67.  Two waves a piece, half of the stores each: 55 us instead of 50.  With the register allocation left
+// send against histograms and that kernel (the ranking's own launch another microsecond slower than now): by destination to
+// 8 ranks 4096 tokens 65 -> 59 us, of hidden 1024 23.4 -> 20.7, 2047 tokens of 7168 30.0 -> 29.6, of 4096 with 256 experts
+// 26.3 -> 22.9, 1100 23.6 -> 22.5; a dispatch of 4096 tokens 133 -> 125, 2047 70 -> 67.  Two waves a piece, half of the
+// stores each: 55 us instead of 50.  With the register allocation left
 // open instead of bounded for eight waves a SIMD the same dispatch takes 127, 2047 tokens of 4096 24.4.
 // index_rows > 0: the grid has that many rows in front of the token rows whose workgroups build the
 // receive side's row index (one (local expert, source) segment each), so that a large one-call
@@ -1156,9 +1158,10 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         batch.slots = slots_in_scratch ? reinterpret_cast<int32_t*>(ws + hist_bytes + first_bytes) : pair_slot;
         batch.stride = scratch_bytes / 4;
         if (batch.num_chunks > 0) {
-            ll_rank_chunk_kernel<<<dim3(batch.num_chunks, num_src), kRankWaves * kWave, size_t(num_experts) * kRankWaves,
-                                   stream>>>(topk_idx, n, num_topk, num_experts, reinterpret_cast<int32_t*>(ws), batch,
-                                             recv_count, num_ranks, rank, max_tokens);
+            ll_rank_chunk_kernel<<<dim3(batch.num_chunks * kRankParts, num_src), kRankPart,
+                                   size_t(num_experts) * (kRankWaves + sizeof(int32_t)), stream>>>(
+                topk_idx, n, num_topk, num_experts, reinterpret_cast<int32_t*>(ws), batch, recv_count, num_ranks, rank,
+                max_tokens);
             EP_LAUNCH_CHECK();
         }
     }

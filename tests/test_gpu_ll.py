@@ -1199,10 +1199,11 @@ def test_all_to_all_with_an_empty_batch(rt, receive):
 
 
 @pytest.mark.parametrize("t,k,e", [(1025, 8, 64), (1171, 7, 96), (1100, 8, 66), (2400, 5, 256), (1025, 64, 260),
-                                   (8193, 1, 8), (8192, 8, 64), (8193, 8, 64), (13200, 5, 256), (1025, 8, 4096)])
+                                   (8193, 1, 8), (8192, 8, 64), (8193, 8, 64), (13200, 5, 256), (1025, 8, 4096),
+                                   (1088, 8, 64), (1089, 8, 128), (1240, 8, 128)])
 def test_slots_of_batches_ranked_ahead_of_their_rows(rt, t, k, e):
-    """Past 8192 entries a launch of its own ranks them, whole tokens of up to 2048 entries a workgroup, and what the
-    chunks before a token's hold is added by the waves that store its rows: for up to 32 chunks and, by destination, up to
+    """Past 8192 entries a launch of its own ranks them, whole tokens of up to 2048 entries a chunk and 512 a workgroup,
+    and what the chunks before a token's hold is added by the waves that store its rows: for up to 32 chunks and, by destination, up to
     64 experts or 256 in fours; beyond by a launch between the two.  With odd numbers of entries, experts named more than
     once by a token, hot ones, and entries that name none."""
     g = torch.Generator().manual_seed(t * 10 + e)
