@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "../../include/deepep_hip.h"
+#include "event.hpp"
 
 namespace deep_ep {
 
@@ -37,17 +38,6 @@ using topk_idx_t = int64_t;  // reference: csrc/kernels/configs.cuh:66-72 (TOPK_
 constexpr int kNumMaxNvlPeers = 8;            // reference: NUM_MAX_NVL_PEERS, csrc/kernels/configs.cuh:3
 constexpr int kNumBufferAlignmentBytes = 128;  // reference: csrc/kernels/configs.cuh:7
 constexpr int kSourceMetaBytes = 8;            // reference: internode::get_source_meta_bytes()
-
-class EPException : public std::exception {
-    std::string message;
-
-public:
-    EPException(const char* name, const char* file, int line, const std::string& error) {
-        message = std::string("Failed: ") + name + " error " + file + ":" + std::to_string(line) + " '" + error + "'";
-    }
-    explicit EPException(std::string text) : message(std::move(text)) {}
-    const char* what() const noexcept override { return message.c_str(); }
-};
 
 #define EP_HOST_ASSERT(cond)                                                          \
     do {                                                                              \
@@ -175,49 +165,13 @@ static size_t get_low_latency_rdma_size_hint(int num_max_dispatch_tokens_per_ran
 // ---------------------------------------------------------------------------
 // EventHandle (reference: csrc/event.hpp:9-25)
 // ---------------------------------------------------------------------------
-static void hip_check(hipError_t e, int line) {
-    if (e != hipSuccess) throw EPException("HIP", "deep_ep_cpp.cpp", line, hipGetErrorString(e));
-}
-
-// An event that streams wait for, and nobody else: the handle cannot be queried, synchronised with or shared.
-// fence: whether the record makes what was written before it visible to the host and to other devices too, which writes
-// the caches back and invalidates them between two kernels.  Streams of one device need none: they see one another's
-// writes when the kernels that made them have ended (hipEventDisableSystemFence), and a host or another device that reads
-// behind one of them has the fence of that wait or copy.
-class DeviceEvent {
-    hipEvent_t event = nullptr;
-    const c10::Device device;
-
-public:
-    DeviceEvent(const HostStream& stream, bool fence) : device(stream.unwrap().device()) {
-        const c10::DeviceGuard guard(device);
-        hip_check(hipEventCreateWithFlags(&event, hipEventDisableTiming | (fence ? 0u : hipEventDisableSystemFence)),
-                  __LINE__);
-        const hipError_t e = hipEventRecord(event, stream.stream());
-        if (e != hipSuccess) (void)hipEventDestroy(event);
-        hip_check(e, __LINE__);
-    }
-    DeviceEvent(const DeviceEvent&) = delete;
-    ~DeviceEvent() {
-        try {
-            const c10::DeviceGuard guard(device);
-            (void)hipEventDestroy(event);
-        } catch (...) {  // the process is ending
-        }
-    }
-    void wait_on(const HostStream& waiter) const {
-        const c10::DeviceGuard guard(waiter.unwrap().device());
-        hip_check(hipStreamWaitEvent(waiter.stream(), event, 0), __LINE__);
-    }
-};
-
 struct EventHandle {
     std::shared_ptr<DeviceEvent> event;
 
     EventHandle() : EventHandle(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()) {}
-    explicit EventHandle(const HostStream& stream, bool fence = true)
-        : event(std::make_shared<DeviceEvent>(stream, fence)) {}
-    void stream_wait_for(const HostStream& waiter) const { event->wait_on(waiter); }
+    explicit EventHandle(const HostStream& stream, DeviceEvent::Scope scope = DeviceEvent::kSystem)
+        : event(std::make_shared<DeviceEvent>(int(stream.device_index()), stream.stream(), scope)) {}
+    void stream_wait_for(const HostStream& waiter) const { event->wait_on(int(waiter.device_index()), waiter.stream()); }
     void current_stream_wait() const { stream_wait_for(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA()); }
 };
 
@@ -1486,12 +1440,12 @@ struct PlainCall<F> {
 // when somebody waits, it would also cover what the caller's stream was given in between, which takes away the
 // overlap with it and hangs where that work waits for the waiter.  A record takes the stream 3 us beside kernels of
 // 8 us, 1 without the fence, and the host 2; a step records two.  A dispatch's is without: what follows it are the experts,
-// on a stream of this device.  A combine's has the fence, which a wait for its stream then need not bring.  Microseconds
+// on a stream of this device (another's brings the fence when it waits: event.hpp).  A combine's has the fence, which a wait for its stream then need not bring.  Microseconds
 // of a step, fences on both / on the combine's / on none, in a row and each waited for:
 //   1 token     13.5 / 11.8 / 10.3    22.3 / 20.8 / 23.8        128   23.0 / 20.9 / 18.9    32.0 / 30.3 / 33.4
 //   77 in bf16  17.4 / 15.5 / 13.7    26.2 / 24.5 / 27.5        509   25.3 / 24.0 / 22.0    33.9 / 33.0 / 35.3
-static pybind11::object recorded_event(bool fence) {
-    return pybind11::cast(EventHandle(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(), fence));
+static pybind11::object recorded_event(DeviceEvent::Scope scope) {
+    return pybind11::cast(EventHandle(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(), scope));
 }
 
 static pybind11::object hook_object(bool wanted) {
@@ -1516,7 +1470,7 @@ static PyObject* low_latency_dispatch_call(PyObject*, PyObject* const* a, Py_ssi
                                                    c.num_experts);
         }
         (void)bool_argument(a[10]);
-        const pybind11::object count = result_object(c.packed_recv_count), event = recorded_event(false),
+        const pybind11::object count = result_object(c.packed_recv_count), event = recorded_event(DeviceEvent::kLocal),
                                hook = hook_object(bool_argument(a[11]));
         return pybind11::reinterpret_steal<pybind11::object>(
             PyTuple_Pack(5, c.recv_result.ptr(), count.ptr(), c.handle_result.ptr(), event.ptr(), hook.ptr()));
@@ -1538,7 +1492,7 @@ static PyObject* low_latency_combine_call(PyObject*, PyObject* const* a, Py_ssiz
             tensor_argument(of_handle(1)), optional_tensor_argument(a[5]), int_argument(of_handle(2)),
             int_argument(of_handle(4)), bool_argument(a[6]), optional_tensor_argument(a[9]), bool_argument(a[10])));
         (void)bool_argument(a[7]);
-        const pybind11::object event = recorded_event(true), hook = hook_object(bool_argument(a[8]));
+        const pybind11::object event = recorded_event(DeviceEvent::kSystem), hook = hook_object(bool_argument(a[8]));
         return pybind11::reinterpret_steal<pybind11::object>(PyTuple_Pack(3, combined.ptr(), event.ptr(), hook.ptr()));
     });
 }

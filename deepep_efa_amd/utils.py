@@ -3,8 +3,8 @@
 Same contract as the reference's wrapper (deep_ep/utils.py:10-61): holds an
 EventHandle recorded on a HIP stream; `current_stream_wait()` makes
 `torch.cuda.current_stream()` wait for it; usable as a `with` block that
-waits on exit.  The event of a low-latency dispatch orders streams of its
-device; a host that reads the results waits for one of them or for a copy.
+waits on exit.  It orders streams, of its device and of others; a host that
+reads the results waits for one of them or for a copy.
 """
 from typing import Any, Optional, Tuple
 

@@ -4,6 +4,7 @@ EPException text.  No kernel is launched here."""
 import decimal
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -256,3 +257,16 @@ def test_c_abi_library_needs_no_torch():
     header = open(os.path.join(ROOT, "include", "deepep_hip.h")).read()
     code = re.sub(r"/\*.*?\*/", "", header, flags=re.S)  # declarations only, comments cite the reference
     assert 'extern "C"' in code and "torch" not in code and "at::" not in code and "#include <hip" not in code
+
+
+def test_streams_of_another_device_wait_behind_the_system_scope_fence(tmp_path):
+    """An event recorded without the fence is not what they wait for.  Host code against a runtime that keeps a record."""
+    torch_dir = os.path.dirname(torch.__file__)
+    program = tmp_path / "events"
+    build = subprocess.run(
+        ["g++", "-O0", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+         f"-I{torch_dir}/include", "-I/opt/rocm/include", os.path.join(ROOT, "tests", "event_of_another_device.cpp"), "-o", str(program),
+         f"-L{torch_dir}/lib", "-lc10", f"-Wl,-rpath,{torch_dir}/lib"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert build.returncode == 0, build.stdout
+    ran = subprocess.run([str(program)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert ran.returncode == 0, ran.stdout
