@@ -255,52 +255,77 @@ def test_another_stream_waits_on_the_returned_events(deep_ep, caller, async_fini
 
 
 def test_what_other_streams_read_behind_the_events(deep_ep):
-    """A kernel, a copy on the device and a copy to the host on another stream see everything a call wrote, call after
-    call over the same buffers, and the call sees what another stream's event was recorded behind."""
+    """Kernels, copies on the device and copies to the host see everything a call wrote behind its event alone, a stream of
+    their own for each of the two events, call after call over the same buffers; and the call sees what another stream's
+    event was recorded behind."""
     from deepep_efa_amd.deep_ep_cpp import EventHandle
     num_ranks, rank, t, h, k, e = 8, 2, 64, 2048, 4, 64
     buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=num_ranks,
                             sim_rank=rank, sim_seed=17)
     x, topk_idx = buffer.loopback_synthesise(t, h, k, e)
+    topk_of = [topk_idx, topk_idx.flip(0).contiguous()]  # the same counts, other rows
     w = torch.rand((t, k), generator=torch.Generator().manual_seed(4)).cuda()
     recv_x, count, handle, _, _ = buffer.low_latency_dispatch(x, topk_idx, t, e, use_fp8=False)
     written = torch.arange(recv_x.shape[1], device="cuda") < count.view(-1, 1)  # what lies behind an expert's rows is anything
+    written_on_host = written.cpu()
     y = recv_x.clone()
     buffer.low_latency_combine(y, topk_idx, w, handle)
     buffer.loopback_clear_world()
-    rounds = 60
+    rounds = 28
     scale = [1.0 + 0.125 * (i % 7) for i in range(rounds)]
 
     def call(i):
-        mine_x, mine_y = x * scale[i], y * scale[i]
-        recv_x, count, handle, dispatched, _ = buffer.low_latency_dispatch(mine_x, topk_idx, t, e, use_fp8=False)
-        combined, reduced, _ = buffer.low_latency_combine(mine_y, topk_idx, w, handle)
-        return recv_x, combined, dispatched, reduced
+        mine_x, mine_y, topk = x * scale[i], y * scale[i], topk_of[i % 2]
+        recv_x, count, handle, dispatched, _ = buffer.low_latency_dispatch(mine_x, topk, t, e, use_fp8=False)
+        combined, reduced, _ = buffer.low_latency_combine(mine_y, topk, w, handle)
+        return (recv_x, count, handle[0], handle[1]), (combined,), dispatched, reduced
+
+    def pinned_copy(v):
+        host = torch.empty(v.shape, dtype=v.dtype, pin_memory=True)
+        host.copy_(v, non_blocking=True)
+        return host
 
     want = []
-    for i in range(7):
-        recv_x, combined, _, _ = call(i)
+    for i in range(14):
+        dispatch_out, combine_out, _, _ = call(i)
         torch.cuda.synchronize()
-        want.append((recv_x.clone(), combined.clone()))
-    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+        want.append([v.clone() for v in dispatch_out + combine_out])
+    assert not torch.equal(want[0][2][written], want[7][2][written])  # the source tokens of the two routings differ
+    for v in dispatch_out + combine_out:
+        v.zero_()
+    mine, readers = torch.cuda.Stream(), (torch.cuda.Stream(), torch.cuda.Stream())
     got = []
     torch.cuda.synchronize()
     for i in range(rounds):
         with torch.cuda.stream(mine):
-            recv_x, combined, dispatched, reduced = call(i)
-        with torch.cuda.stream(other):
-            reduced.current_stream_wait()
-            host = torch.empty(combined.shape, dtype=combined.dtype, pin_memory=True)
-            host.copy_(combined, non_blocking=True)
-            dispatched.current_stream_wait()
-            got.append((recv_x.clone(), combined + 0, host))
-            read = deep_ep.EventOverlap(EventHandle())
+            if i % 4 == 0:
+                torch.cuda._sleep(1_000_000)
+            dispatch_out, combine_out, dispatched, reduced = call(i)
+        by_kernel, by_copy, on_host, read = [], [], [], []
+        for reader, event, outputs in zip(readers, (dispatched, reduced), (dispatch_out, combine_out)):
+            with torch.cuda.stream(reader):
+                event.current_stream_wait()
+                host_first = i % 2 == 0
+                if host_first:
+                    on_host += [pinned_copy(v) for v in outputs]
+                by_kernel += [v + 0 for v in outputs]
+                by_copy += [v.clone() for v in outputs]
+                if not host_first:
+                    on_host += [pinned_copy(v) for v in outputs]
+                read.append(deep_ep.EventOverlap(EventHandle()))
+        got.append((by_kernel, by_copy, on_host))
         with torch.cuda.stream(mine):
-            read.current_stream_wait()  # the next call writes over what was read
-    other.synchronize()
-    for i, (recv_x, combined, host) in enumerate(got):
-        assert torch.equal(recv_x[written], want[i % 7][0][written]) and torch.equal(combined, want[i % 7][1]), i
-        assert torch.equal(host, want[i % 7][1].cpu()), i
+            for r in read:
+                r.current_stream_wait()  # the next call writes over what was read
+    for reader in readers:
+        reader.synchronize()
+    for i, kinds in enumerate(got):
+        for kind, outputs in enumerate(kinds):
+            mask = written_on_host if kind == 2 else written
+            for j, (v, w_) in enumerate(zip(outputs, want[i % 14])):
+                w_ = w_.cpu() if kind == 2 else w_
+                rows = j in (0, 2)  # rows and source tokens: what was written
+                assert torch.equal(v[mask] if rows else v, w_[mask] if rows else w_), (i, kind, j)
     buffer.destroy()
 
 
