@@ -1440,8 +1440,8 @@ struct PlainCall<F> {
 // when somebody waits, it would also cover what the caller's stream was given in between, which takes away the
 // overlap with it and hangs where that work waits for the waiter.  A record takes the stream 3 us beside kernels of
 // 8 us, 1 without the fence, and the host 2; a step records two.  A dispatch's is without: what follows it are the experts,
-// on a stream of this device (another's brings the fence when it waits: event.hpp).  A combine's has the fence, which a wait for its stream then need not bring.  Microseconds
-// of a step, fences on both / on the combine's / on none, in a row and each waited for:
+// on a stream of this device (another's brings the fence when it waits: event.hpp).  A combine's has the fence, which a wait
+// for its stream then need not bring.  Microseconds of a step, fences on both / on the combine's / on none, in a row and each waited for:
 //   1 token     13.5 / 11.8 / 10.3    22.3 / 20.8 / 23.8        128   23.0 / 20.9 / 18.9    32.0 / 30.3 / 33.4
 //   77 in bf16  17.4 / 15.5 / 13.7    26.2 / 24.5 / 27.5        509   25.3 / 24.0 / 22.0    33.9 / 33.0 / 35.3
 static pybind11::object recorded_event(DeviceEvent::Scope scope) {

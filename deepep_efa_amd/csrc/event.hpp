@@ -1,7 +1,9 @@
 // Events that streams wait for (reference: csrc/event.hpp:9-25).  Streams are named by their device and HIP handle.
 #pragma once
+#include <c10/core/impl/GPUTrace.h>
 #include <hip/hip_runtime_api.h>
 
+#include <cstdint>
 #include <mutex>
 #include <unordered_map>
 
@@ -24,7 +26,8 @@ public:
     }
 };
 
-// An event that streams wait for, and nobody else: the handle cannot be queried, synchronised with or shared.
+// An event that streams wait for, and nobody else: the handle cannot be queried, synchronised with or shared.  PyTorch's
+// event callbacks (torch.cuda._gpu_trace) hear of it as of PyTorch's own.
 // kLocal: recorded without the system-scope fence (hipEventDisableSystemFence), which writes the caches back and invalidates
 // them between two kernels and without which memory may not be visible to the host and other devices.  Streams of the
 // device need none, they see one another's writes when the kernels that made them have ended, and a host that reads behind
@@ -39,18 +42,31 @@ private:
     const int device;
     const Scope scope;
 
+    template <typename F>
+    static void trace(F report) {
+        if (const auto* interpreter = c10::impl::GPUTrace::get_trace()) report(**interpreter);
+    }
+    uintptr_t name() const { return reinterpret_cast<uintptr_t>(event); }
+    void destroy() {
+        trace([&](const auto& to) { to.trace_gpu_event_deletion(c10::kCUDA, name()); });
+        (void)hipEventDestroy(event);
+    }
+
     // The one stream of the current device on which events are recorded for other devices; kept until the process ends.
     // What several threads put there at once may wait for one another's events, never for anything that follows them.
     static hipStream_t relay_of(int device) {
         static std::mutex& mutex = *new std::mutex;
         static auto& streams = *new std::unordered_map<int, hipStream_t>;
-        const std::lock_guard<std::mutex> lock(mutex);
+        const std::lock_guard<std::mutex> lock(mutex);  // not held beyond: the callbacks below run Python
         hipStream_t& relay = streams[device];
         if (relay == nullptr) hip_check(hipStreamCreateWithFlags(&relay, hipStreamNonBlocking), "event.hpp", __LINE__);
         return relay;
     }
 
     void stream_waits(hipStream_t waiter) const {
+        trace([&](const auto& to) {
+            to.trace_gpu_event_wait(c10::kCUDA, name(), reinterpret_cast<uintptr_t>(waiter));
+        });
         hip_check(hipStreamWaitEvent(waiter, event, 0), "event.hpp", __LINE__);
     }
 
@@ -58,15 +74,22 @@ public:
     DeviceEvent(int device, hipStream_t stream, Scope scope) : device(device), scope(scope) {
         const ScopedDevice current(device);
         hip_check(hipEventCreateWithFlags(&event, hipEventDisableTiming | scope), "event.hpp", __LINE__);
-        const hipError_t e = hipEventRecord(event, stream);
-        if (e != hipSuccess) (void)hipEventDestroy(event);
-        hip_check(e, "event.hpp", __LINE__);
+        try {
+            trace([&](const auto& to) {
+                to.trace_gpu_event_creation(c10::kCUDA, name());
+                to.trace_gpu_event_record(c10::kCUDA, name(), reinterpret_cast<uintptr_t>(stream));
+            });
+            hip_check(hipEventRecord(event, stream), "event.hpp", __LINE__);
+        } catch (...) {
+            destroy();
+            throw;
+        }
     }
     DeviceEvent(const DeviceEvent&) = delete;
     ~DeviceEvent() {
         try {
             const ScopedDevice current(device);
-            (void)hipEventDestroy(event);
+            destroy();
         } catch (...) {  // the process is ending
         }
     }

@@ -1,7 +1,10 @@
 """GPU tests of the deep_ep.Buffer API, written after the reference's own drivers
 (tests/test_low_latency.py:38-193, tests/test_intranode.py:35-66) with the other ranks
 supplied by the loopback world instead of real processes."""
+import os
 import random
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -327,6 +330,47 @@ def test_what_other_streams_read_behind_the_events(deep_ep):
                 rows = j in (0, 2)  # rows and source tokens: what was written
                 assert torch.equal(v[mask] if rows else v, w_[mask] if rows else w_), (i, kind, j)
     buffer.destroy()
+
+
+_TRACED_STEP = """
+import torch
+torch.cuda.init()
+torch._C._activate_gpu_trace()
+from torch.cuda import _gpu_trace
+import deep_ep
+seen = {"creation": [], "record": [], "wait": [], "deletion": []}
+for kind, calls in seen.items():
+    getattr(_gpu_trace, "register_callback_for_event_" + kind)(lambda *of, calls=calls: calls.append(of))
+buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=8, sim_rank=2, sim_seed=13)
+x, topk_idx = buffer.loopback_synthesise(32, 1024, 4, 64)
+w = torch.ones((32, 4), device="cuda")
+mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+for calls in seen.values():
+    calls.clear()
+with torch.cuda.stream(mine):
+    y, _, handle, dispatched, _ = buffer.low_latency_dispatch(x, topk_idx, 32, 64, use_fp8=False)
+    _, reduced, _ = buffer.low_latency_combine(y, topk_idx, w, handle)
+with torch.cuda.stream(other):
+    for event in (dispatched, reduced):
+        event.current_stream_wait()
+del event, dispatched, reduced
+names = [name for name, in seen["creation"]]
+assert len(names) == 2, seen
+assert seen["record"] == [(name, mine.cuda_stream) for name in names], seen
+assert seen["wait"] == [(name, other.cuda_stream) for name in names], seen
+assert sorted(seen["deletion"]) == sorted((name,) for name in names), seen
+torch.cuda.synchronize()
+buffer.destroy()
+print("traced")
+"""
+
+
+def test_event_callbacks_hear_of_a_steps_events():
+    """Tools that follow the order of streams through PyTorch's callbacks; in a process of its own, which keeps them on."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    ran = subprocess.run([sys.executable, "-c", _TRACED_STEP], cwd=root, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                         timeout=100)
+    assert ran.returncode == 0 and "traced" in ran.stdout, ran.stdout
 
 
 def _step_with_events(deep_ep):
