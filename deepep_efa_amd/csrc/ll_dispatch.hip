@@ -145,6 +145,7 @@ struct RankedBatch {
     int64_t stride;             // of both from a source to the next, in ints
     int in_full;
     int32_t* own_first;         // [E_l] where the rank's own rows begin (null: nobody asks)
+    int first_in_finish;        // the launch between the two writes own_first, over the last chunk's histogram
 };
 
 // Final destination of the rows a rank sends to its own experts, used by the
@@ -535,7 +536,7 @@ __global__ __launch_bounds__(kRankPart) void ll_rank_chunk_kernel(
     for (int u = 0; u < kRankParts - 1; ++u)
         earlier[u] = __builtin_amdgcn_raw_buffer_load_b64(list, u < part ? (begin + u * kRankPart + tid) * 8 : 0x7ffffff0, 0, 0);
     int own_rows = 0;
-    const bool own_wanted = blockIdx.x == 0 && batch.own_first != nullptr;
+    const bool own_wanted = blockIdx.x == 0 && batch.own_first != nullptr && !batch.first_in_finish;
     if (own_wanted) {  // a wave an expert, as far as there are waves
         for (int s = lane; s < rank && w < num_experts / num_ranks; s += kWave) {
             const int c = recv_count[w * num_ranks + s];
@@ -619,6 +620,16 @@ __global__ __launch_bounds__(1024) void ll_rank_finish_kernel(SendArgs a, Ranked
     const int tid = threadIdx.x, threads = block_threads(), c = blockIdx.x, b = blockIdx.y;
     if (c == batch.num_chunks) {
         ranked_counts(a, batch, b, before, wave_totals);
+        if (!batch.first_in_finish || c == 0) return;
+        __syncthreads();  // the last chunk's histogram has been read; the other workgroups read those before it
+        for (int le = tid; le < a.num_experts / a.num_ranks; le += threads) {
+            int rows = 0;
+            for (int s = 0; s < a.rank; ++s) {
+                const int n = a.recv_count[le * a.num_ranks + s];
+                rows += n < 0 ? 0 : (n > a.max_tokens ? a.max_tokens : n);
+            }
+            batch.own_first[le] = rows;
+        }
         return;
     }
     const int32_t* hists = batch.hists + int64_t(b) * batch.stride;
@@ -1127,11 +1138,11 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     // How slots get ranked: the launch that stores the rows does it for itself while it is the only one and has no more
     // than kSelfRankMaxEntries entries to go through.
     const bool prefix_in_block = by_dest != nullptr && by_dest_tables_in_send(n, num_experts);
-    const bool ranked = fused_recv == nullptr && (n > kSelfRankMaxEntries || own_rows_direct != nullptr ||
-                                                  (by_dest != nullptr && !prefix_in_block));
+    bool ranked = fused_recv == nullptr && (n > kSelfRankMaxEntries || own_rows_direct != nullptr ||
+                                            (by_dest != nullptr && !prefix_in_block));
     const int64_t hist_bytes = chunk_hist_bytes(num_tokens, num_topk, num_experts);
-    const int64_t first_bytes = own_rows_direct != nullptr ? align256(int64_t(num_experts) * 4) : 0;
     const int64_t slot_bytes = align256(int64_t(n) * 4);
+    int64_t first_bytes = own_rows_direct != nullptr ? align256(int64_t(num_experts) * 4) : 0;
     // What the chunks before a token's hold of its experts is added up by the waves that store its rows, up to
     // kSendColumns of them and, by destination, up to 256 experts; otherwise, and without room for slots that nobody sees,
     // by a launch between the two.
@@ -1139,7 +1150,11 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     batch.tokens_per_chunk = rank_chunk_tokens(num_topk);
     batch.num_chunks = (num_tokens + batch.tokens_per_chunk - 1) / batch.tokens_per_chunk;
     batch.chunk_of = make_rank_divider(batch.tokens_per_chunk);
+    // A workspace may hold the histograms alone.  The slots then go where the caller wants them and where own rows begin over a
+    // histogram that has been read; sends whose slots nobody wants rank themselves, whatever that takes.
     const bool room = workspace_bytes >= size_t(hist_bytes + first_bytes + slot_bytes) * size_t(num_src);
+    if (!room && pair_slot == nullptr) ranked = false;
+    if (!room && own_rows_direct != nullptr) first_bytes = 0, batch.first_in_finish = 1;
     batch.in_full = batch.num_chunks > kSendColumns || (by_dest != nullptr && !columns_by_dest_fit(num_experts)) || !room;
     const bool slots_in_scratch = !batch.in_full || pair_slot == nullptr;
     const int64_t scratch_bytes = hist_bytes + first_bytes + (slots_in_scratch ? slot_bytes : 0);
@@ -1154,7 +1169,10 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     uint8_t* ws = reinterpret_cast<uint8_t*>(workspace);
     if (ranked) {
         batch.hists = reinterpret_cast<int32_t*>(ws);
-        batch.own_first = own_rows_direct != nullptr ? reinterpret_cast<int32_t*>(ws + hist_bytes) : nullptr;
+        if (batch.first_in_finish)
+            batch.own_first = reinterpret_cast<int32_t*>(ws) + int64_t(std::max(batch.num_chunks - 1, 0)) * num_experts;
+        else if (own_rows_direct != nullptr)
+            batch.own_first = reinterpret_cast<int32_t*>(ws + hist_bytes);
         batch.slots = slots_in_scratch ? reinterpret_cast<int32_t*>(ws + hist_bytes + first_bytes) : pair_slot;
         batch.stride = scratch_bytes / 4;
         if (batch.num_chunks > 0) {
@@ -1246,10 +1264,10 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         return 0;
     }
 
-    // The receive index rides along with the rows of a ranked one-call dispatch
+    // The receive index rides along with the rows of a ranked one-call dispatch, for whose own counts it reads all histograms
     FusedIndexArgs index = {};
     int index_rows = 0;
-    if (fused_index != nullptr && ranked) {
+    if (fused_index != nullptr && ranked && !batch.first_in_finish) {
         index = *fused_index;
         index.chunk_hist = batch.hists, index.num_chunks = batch.num_chunks;
         index_rows = (num_experts + blocks_per_token - 1) / blocks_per_token;

@@ -1295,6 +1295,67 @@ def test_one_call_dispatch_of_few_entries_and_many_rows(rt, rank):
     check_dispatch(st, want, O.ROW_FP8)
 
 
+@pytest.mark.parametrize("t,k,e,rows", [(300, 8, 64, 8193), (1100, 8, 64, 0), (1100, 8, 64, 9000), (1171, 7, 96, 9000),
+                                        (8300, 8, 64, 70000)])  # the last of more than 32 chunks
+def test_workspace_that_holds_the_chunk_histograms_alone(rt, t, k, e, rows):
+    """ceil(T / floor(2048 / K)) * E * 4 bytes, rounded up to 256, for each source: every send works with them."""
+    r, rank, h, fmt = 4, 2, 256, O.ROW_FP8
+    lib = rt.capi.load()
+    g = torch.Generator().manual_seed(t + e)
+    x_all = torch.randn((r, t, h), generator=g).to(torch.bfloat16).cuda()
+    topk = torch.randint(0, e, (r, t, k), generator=g)
+    topk[torch.rand((r, t, k), generator=g) < 0.05] = -1
+    topk = topk.cuda()
+    hist_bytes = (-(-t // (2048 // k)) * e * 4 + 255) // 256 * 256
+    assert hist_bytes < lib.deepep_ll_dispatch_workspace_bytes(t, k, e)
+    per_rank = e // r
+
+    def guarded(nbytes):
+        whole = torch.full((nbytes + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+        return whole[:nbytes], whole[nbytes:]
+
+    def dispatch(small):
+        st = rt.ll.LowLatencyState(rt.ll.LLShape(num_ranks=r, rank=rank, num_experts=e, max_tokens=t, hidden=h, num_topk=k, fmt=fmt))
+        st.expected_rows = rows
+        st.segment_workspace = (torch.empty(lib.deepep_ll_segment_workspace_bytes(e, t), dtype=torch.uint8, device="cuda")
+                                if rows > 0 else None)
+        world = rt.lb.LoopbackWorld(r, rank, seed=0)
+        world.set_inputs(x_all, topk)
+        x, own = world.own_inputs()
+        guard = torch.empty(0, device="cuda")
+        if small:
+            st.workspace, guard = guarded(hist_bytes)
+        st.recv_staging.fill_(0x5A)
+        st.send_slots.fill_(0)  # a row's padding is not written
+        stats = torch.zeros(per_rank, dtype=torch.int32, device="cuda")
+        run_dispatch(st, world, x, own, stats, True)
+        count = st.packed_recv_count
+        written = torch.arange(r * t, device="cuda") < count.view(-1, 1)
+        assert (guard == 0x5A).all()
+        own_staged = st.recv_staging.view(per_rank, r, -1)[:, rank]
+        assert (own_staged == 0x5A).all()
+        return [count, stats, st.recv_count, st.send_count, st.pair_slot, st.packed_recv_layout_range,
+                st.packed_recv_x.view(torch.uint8)[written], st.packed_recv_scales[written], st.packed_recv_src_info[written],
+                st.send_slots]
+
+    for i, (a, b) in enumerate(zip(dispatch(False), dispatch(True))):
+        assert torch.equal(a, b), i
+
+    src = torch.tensor([0, 3], dtype=torch.int32, device="cuda")
+    stride = lib.deepep_ll_row_stride(h, fmt)
+    staged = []
+    for size in (lib.deepep_ll_dispatch_workspace_bytes(t, k, e), hist_bytes):
+        ws, guard = guarded(2 * size)
+        staging = torch.zeros((per_rank, r, t, stride), dtype=torch.uint8, device="cuda")
+        recv_count = torch.zeros((per_rank, r), dtype=torch.int32, device="cuda")
+        rt.capi.check(lib.deepep_loopback_dispatch_from_peers(
+            rt.capi.ptr(x_all[[0, 3]].contiguous()), rt.capi.ptr(topk[[0, 3]].contiguous()), rt.capi.ptr(src), 2, t, h, k, e, r, rank, t,
+            fmt, rt.capi.ptr(staging), rt.capi.ptr(recv_count), rt.capi.ptr(ws), ws.numel(), rt.ll.current_stream_ptr()))
+        assert (guard == 0x5A).all()
+        staged.append((staging, recv_count))
+    assert all(torch.equal(a, b) for a, b in zip(*staged))
+
+
 def test_send_by_dest_with_repeated_experts_and_full_pairs(rt):
     """Tokens naming an expert more than once: pairs beyond a pair's M slots are dropped from the counts,
     the prefixes and the buffer alike."""
