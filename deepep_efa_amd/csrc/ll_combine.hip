@@ -290,14 +290,21 @@ constexpr int64_t kWorkgroupsAtOnce = 256 * 8;  // compute units, workgroups of 
 //   256 x 4096                 25.1 / 23.1    R 20.2 / 19.4    W 26.9 / 22.4
 //   300 x 7168                 46.6 / 38.4    R 34.9 / 34.4    W 51.2 / 40.6
 //   500 x 2048                 26.6 / 24.0    R 21.5 / 20.9    W 28.4 / 24.1
-//   509 x 4096, no row return  28.9 / 25.1    R 23.7 / 22.8    W 33.4 / 25.8
 //   700 x 4096                 54.6 / 45.1    R 43.6 / 44.6    W 63.7 / 51.9    (the dispatch's own share: common.hpp)
 //   900 x 2048                 42.5 / 38.8    R 33.5 / 33.0    W 47.0 / 38.6
-// Replayed on one set of buffers, all of it still cached, it costs 150 to 180 tokens 5 to 7 %, 509 3 % and gains from 700 on.
+// Replayed on one set of buffers, all of it still cached, it costs 150 to 180 tokens 5 to 7 % and gains from 700 on.
 // Below, 128 x 7168 (46 MB) gains 3 % on other buffers and loses 2 % behind a read, 256 x 5120 at top-4 (33 MB) and 77 x 5120
 // lose 2 % both ways.  The hint on the rows to be returned as well: 128 and 150 tokens 3 % slower than without any, 256 x
 // 4096 24.3 us, 500 x 2048 25.8, 700 x 4096 45.7, but 300 x 7168 37.2 and behind a write another 8 to 13 % less.
 constexpr int64_t kGatherStreamBytes = int64_t(48) << 20;
+// Without a row return the gathered rows are all there is, and the line lies at 18 MB of them.  Steps in microseconds without
+// the hint / with it, on three sets of buffers in turn and on one, and the combine alone behind a write of 512 MB (behind a read
+// the two differ by no more than two runs of one):
+//   128 x 7168 (15 MB)  15.7 / 16.4   15.1 / 15.4   14.5 /  8.9     256 x 7168 (29 MB)  23.7 / 22.9   21.1 / 22.6   18.9 / 11.2
+//   500 x 2048 (16 MB)  18.1 / 18.6   17.1 / 17.5   12.7 /  9.0     300 x 7168 (34 MB)  26.8 / 24.8   22.9 / 24.5   21.1 / 12.2
+//   150 x 7168 (17 MB)  16.8 / 17.7   16.0 / 16.8   14.0 /  9.8     509 x 4096 (33 MB)  28.3 / 24.6   22.4 / 23.2   17.6 / 11.8
+//   180 x 7168 (21 MB)  19.7 / 19.1   17.7 / 18.7   15.2 /  9.6     700 x 4096 (46 MB)  31.7 / 29.6   27.8 / 28.8   25.3 / 14.6
+constexpr int64_t kGatherAloneStreamBytes = int64_t(18) << 20;
 
 // kStream: stores and gathered rows; kStreamRows: the rows to be returned as well.
 template <bool kStream, bool kStreamRows, bool kInTurn>
@@ -762,11 +769,13 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     const size_t lds = size_t(sa.num_local_experts) * sizeof(int32_t);
     // rows returned (read + written) plus rows gathered: past what the caches hold, stream.  Beside more
     // than kLargeBatchRows rows it always pays (11946 of 4 KB, 61.2 -> 57.5 us a step).
-    const int64_t traffic = (2 * rows + int64_t(num_tokens) * num_topk) * hidden * 2;
+    const bool returns_rows = combine_send_slots != nullptr;
+    const int64_t traffic = ((returns_rows ? 2 * rows : 0) + int64_t(num_tokens) * num_topk) * hidden * 2;
+    const int64_t gather_streams = returns_rows ? kGatherStreamBytes : kGatherAloneStreamBytes;
 #define DEEPEP_LAUNCH_FUSED(KERNEL) \
     KERNEL<<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds, reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks))
     if (large || traffic > stream_bytes()) DEEPEP_LAUNCH_FUSED(ll_combine_fused_past_caches_kernel);
-    else if (traffic > kGatherStreamBytes) DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<true, false>));
+    else if (traffic > gather_streams) DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<true, false>));
     else if (recv_blocks + send_blocks <= kWorkgroupsAtOnce) DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<false, true>));
     else DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<false, false>));
 #undef DEEPEP_LAUNCH_FUSED

@@ -8,6 +8,7 @@ bit for bit and the float64 sum within 1e-2 relative.
 """
 import ctypes
 import os
+import re
 
 import numpy as np
 import pytest
@@ -2074,9 +2075,26 @@ def test_combine_in_one_launch_and_in_two(rt, h, hints):
     assert all(torch.equal(sums[0], o) for o in sums[1:])
 
 
+_FORMS = ("ll_combine_fused_kernelILb0", "ll_combine_fused_kernelILb1", "ll_combine_fused_past_caches_kernel")
+
+
+def combine_launched(call, tmp_path):
+    """The combine kernel of a call, by its node in a captured graph."""
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    graph.enable_debug_mode()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        call()
+    graph.debug_dump(str(tmp_path / "graph.dot"))
+    names = set(re.findall(r"ll_combine_\w*?kernel(?:I(?:Lb[01]E)+E)?", (tmp_path / "graph.dot").read_text()))
+    assert len(names) == 1
+    return names.pop()
+
+
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
 @pytest.mark.parametrize("h,k,hints", [(7168, 8, (1404, 1405, 6085, 6086)),  # 48 and 192 MB: three forms of the launch
-                                       (640, 3, (4096, 8192))])
-def test_combine_whose_accesses_stream_in_part(rt, h, k, hints):
+                                       (5504, 8, (1876, 1877, 7972, 7973))])  # rows with a last piece of three quarters
+def test_combine_whose_accesses_stream_in_part(rt, h, k, hints, tmp_path):
     """Which accesses of the single-launch combine carry the streaming hint changes no row and no sum."""
     r, rank, t, e = 8, 3, 40, 64
     x_all, topk_all, w = make_world(r, t, h, k, e, seed=h, drop=9)
@@ -2093,9 +2111,35 @@ def test_combine_whose_accesses_stream_in_part(rt, h, k, hints):
         else:
             st.expected_rows = hint
             st.combine(y, topk, w, out)
+            form = combine_launched(lambda: st.combine(y, topk, w, out), tmp_path)
+            assert form.startswith(_FORMS[(0, 1, 1, 2)[hints.index(hint)]]), hint
         torch.cuda.synchronize()
         got.append((st.combine_send_slots.view(torch.int16).clone(), out.view(torch.int16).clone()))
     assert all(torch.equal(a, b) for other in got[1:] for a, b in zip(got[0], other))
+
+
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
+@pytest.mark.parametrize("t,h,streams", [(164, 7168, 0), (165, 7168, 1), (214, 5504, 0), (215, 5504, 1)])
+def test_combine_without_row_return_streams_by_what_it_gathers(rt, t, h, streams, tmp_path):
+    """18 MB of gathered rows, whatever number of rows is expected; and the sums of the two phases."""
+    r, rank, k, e = 8, 3, 8, 64
+    x_all, topk_all, w = make_world(r, t, h, k, e, seed=t, drop=9)
+    st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, 256, O.ROW_BF16, one_call=True)
+    y = torch.randn(st.packed_recv_x.shape, generator=torch.Generator().manual_seed(h)).bfloat16().cuda()
+    world.combine_from_peers(st, mode=1, seed=5)
+    topk, w = topk_all[rank].cuda(), w[rank].cuda()
+    want = torch.zeros((t, h), dtype=torch.bfloat16, device="cuda")
+    st.combine_send(y)
+    st.combine_recv(topk, w, want)
+    st.combine_send_slots.view(torch.int16).fill_(0x7FC0)
+    for hint in (t * k, 8192):
+        st.expected_rows = hint
+        out = torch.zeros((t, h), dtype=torch.bfloat16, device="cuda")
+        st.combine(y, topk, w, out, zero_copy=True)
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), hint
+        form = combine_launched(lambda: st.combine(y, topk, w, out, zero_copy=True), tmp_path)
+        assert form.startswith(_FORMS[streams]), hint
+    assert (st.combine_send_slots.view(torch.int16) == 0x7FC0).all()
 
 
 @pytest.mark.parametrize("t,h,k,e,hints", [
