@@ -466,9 +466,11 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
         const int j = row - seg_first;
         const uint8_t* from = a.rows + uint64_t(uint32_t(src * int(a.slot_rows) + in_message + j)) * stride;
         row_part_range(num_vec, a.parts_log2, part, v_begin, v_end);
-        // Stored past the caches: an exchange of 128 tokens of hidden 7168 on three sets of buffers in turn 29.1 -> 27.7 us to
-        // 32 ranks and 27.4 -> 26.6 to 8 (the receive alone behind a read of 512 MB 6.6 -> 6.8).
-        RowPart<kOrderedDepth, false, true> payload;
+        // Stored the ordinary way, since the experts read the rows next.  Receive and a copy of its rows, ordinary stores / past
+        // the caches, on three sets of buffers in turn and behind a write of 512 MB: 128 tokens of hidden 7168 to 32 ranks (7 MB)
+        // 10.1 / 10.3 us and 12.9 / 14.1, 256 to 16 (15 MB) 14.7 / 16.3 and 20.5 / 23.0, 700 to 8 (41 MB) 35.6 / 38.7 and 43.5 /
+        // 50.8; 1000 of 4096 (33 MB) 31.8 / 34.1 and 38.9 / 42.7.  The receive alone 5.2 / 4.8, 8.2 / 8.1, 18.1 / 16.4, 14.8 / 14.5.
+        RowPart<kOrderedDepth, false, false> payload;
         payload.load(from, v_begin, v_end, lane);
         const bool carries_tail = part == parts - 1;  // the last part is the shortest
         uint32_t tail_scale = 0;
