@@ -274,8 +274,8 @@ int deepep_ll_dispatch_send(const void* x, const int64_t* topk_idx,
  * is for callers that cannot allocate: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  Same arguments, outputs and errors as
  * deepep_ll_dispatch_send otherwise.
- *   Limit: ceil(T / floor(2048 / K)) * E * 4 <= 1048576 (at K = 8, E = 256: T <= 262144); a larger batch
- *   fails with a message that says so.
+ *   Limit: ceil(T / floor(2048 / K)) * E * 4 <= 1048576 (at K = 8, E = 4096: T <= 16384); a larger batch
+ *   fails with a message that says so.  T < 65535 as in every send.
  *   `stream` must belong to the current device.  The array's address is looked up on the first
  *   call on each device (a host-side query, no device work).
  *   Every call on a GPU shares that GPU's array: two calls that overlap in time on one GPU (on

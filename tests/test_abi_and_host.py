@@ -101,6 +101,13 @@ def test_reduces_leave_room_for_eight_waves_a_simd(kernel):
     assert len(found) == 1 and found[0][".vgpr_count"] <= 64 and found[0][".private_segment_fixed_size"] == 0
 
 
+def test_ranked_send_leaves_room_for_eight_waves_a_simd():
+    """Every row format, streaming or not: the kernel has no other way to hide its trips to memory."""
+    found = [k for name, k in _kernel_metadata().items() if "ll_send_ranked_kernel" in name]
+    assert len(found) == 8
+    assert all(k[".vgpr_count"] <= 64 and k[".private_segment_fixed_size"] == 0 for k in found)
+
+
 @pytest.mark.parametrize("tokens,seen_tokens,seen_rows,want", [
     (128, 0, 0, 1024),          # nothing seen yet: what a balanced world sends
     (0, 0, 0, 8),
