@@ -470,6 +470,9 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
         // the caches, on three sets of buffers in turn and behind a write of 512 MB: 128 tokens of hidden 7168 to 32 ranks (7 MB)
         // 10.1 / 10.3 us and 12.9 / 14.1, 256 to 16 (15 MB) 14.7 / 16.3 and 20.5 / 23.0, 700 to 8 (41 MB) 35.6 / 38.7 and 43.5 /
         // 50.8; 1000 of 4096 (33 MB) 31.8 / 34.1 and 38.9 / 42.7.  The receive alone 5.2 / 4.8, 8.2 / 8.1, 18.1 / 16.4, 14.8 / 14.5.
+        // A whole exchange whose experts hand the rows on 47.9 / 50.3, 76.8 / 82.6, 180.8 / 198.6 and 150.8 / 167.3, one whose experts
+        // read 512 MB first 58.4 / 58.1, 90.2 / 89.3, 206 / 205 and 177.8 / 176.0, and one without experts 27.8 / 26.9, 40.5 / 39.2,
+        // 89.7 / 84.4 and 75.8 / 71.1.
         RowPart<kOrderedDepth, false, false> payload;
         payload.load(from, v_begin, v_end, lane);
         const bool carries_tail = part == parts - 1;  // the last part is the shortest
