@@ -686,9 +686,9 @@ __device__ __forceinline__ void columns_by_dest(__amdgpu_buffer_rsrc_t hists, in
 // by the workgroup, so no wave waits for another.  Selections, places and row are fetched together; behind them, beside
 // the row, the columns of the chunks before the token's, shared among the lanes, and a table (the by-destination prefix,
 // which without a table are the sums of all columns, or where own rows begin).
-// HBM bounds it: 4096 tokens of hidden 7168, top-8, fp8 (302 MB) 52 us in the kernel trace of a step, 5.8 TB/s, 49 at its
-// fastest, where workgroups that went through the entries of their chunk and shared what they counted, three barriers ahead
-// of the stores, took 62; both behind a launch of 4.2.  Called in a row, both launches of a
+// HBM bounds it: 4096 tokens of hidden 7168, top-8, fp8 (302 MB) 52 to 55 us in the kernel trace of a step (5.5 to 5.8 TB/s), 49
+// at its fastest, where workgroups that went through the entries of their chunk and shared what they counted, three barriers
+// ahead of the stores, took 62; both behind a launch of 4.2.  Called in a row, both launches of a
 // send against histograms and that kernel (the ranking's own launch another microsecond slower than now): by destination to
 // 8 ranks 4096 tokens 65 -> 59 us, of hidden 1024 23.4 -> 20.7, 2047 tokens of 7168 30.0 -> 29.6, of 4096 with 256 experts
 // 26.3 -> 22.9, 1100 23.6 -> 22.5; a dispatch of 4096 tokens 133 -> 125, 2047 70 -> 67.  Two waves a piece, half of the
