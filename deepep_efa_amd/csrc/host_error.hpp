@@ -1,4 +1,4 @@
-// The exception of the host module, with the reference's text (csrc/kernels/exception.cuh:14-45).
+// The exception of the host module, with the reference's text (csrc/kernels/exception.cuh:12-22).
 #pragma once
 #include <hip/hip_runtime_api.h>
 
