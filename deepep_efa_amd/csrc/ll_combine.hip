@@ -683,19 +683,20 @@ int deepep_ll_combine_recv_flat(const void* recv_flat, int64_t recv_flat_rows, i
 }
 
 // Whether a combine whose rows are to be returned runs as one launch.  Up to kLargeBatchRows rows always.  Beyond, while
-// the rows returned and the tokens' rows stay within 220 MB: there the rows are moved beside the reduce's loads and the
-// step has one launch less.  Not where far more rows come in than the tokens send out (the hottest experts' rank: the
-// flat copy is the faster one, and the reduce too short to hide anything), nor for many rows of less than 2 KB.
+// the rows returned and the tokens' rows stay within 132 MB: there the rows are moved beside the reduce's loads and the
+// step has one launch less, past it the flat copy's rate is worth more.  Not where far more rows come in than the tokens
+// send out (the hottest experts' rank: the reduce is too short to hide anything), nor for many rows of less than 2 KB.
 // Microseconds of a dispatch and a combine, one launch against two (rows, row size; 8 ranks x 8 experts unless given):
-//    8720 of  4 KB  55.2 /  57.4     13122 of 14 KB (2 ranks) 123.3 / 131.9      31786 of 2 KB     82.0 /  85.5
-//   11985 of  8 KB  97.1 / 107.5     11934 of 14 KB (top-4)   158.8 / 166.3      31786 of 1 KB     59.6 /  57.9
-//   19860 of  8 KB 146.3 / 155.5     13541 of 14 KB           170.0 / 175.8      31786 of 256 B    47.9 /  45.5
-//   47736 of  3 KB 134.8 / 152.4     15139 of 14 KB           179.3 / 172.1      10358 of 1 KB     33.5 /  34.5
-//   23888 of  8 KB 169.8 / 176.1     23877 of 10 KB           200.9 / 193.1
+//    8800 of  4 KB  45.3 /  46.9      8800 of 14 KB (142 MB)   109.4 / 106.7     31786 of 1 KB     59.6 /  57.9
+//   14400 of  4 KB  60.8 /  62.4     10400 of 14 KB (16 ranks) 127.3 / 125.5     31786 of 256 B    47.9 /  45.5
+//    8800 of  8 KB  70.3 /  71.4     12000 of 14 KB (194 MB)   140.9 / 138.1     10358 of 1 KB     33.5 /  34.5
+//   12800 of  8 KB  94.0 /  94.0      9200 of 14 KB (top-4)    114.6 / 114.2
+//   16800 of  8 KB 121.8 / 116.6      9000 of 10 KB (top-6)     88.1 /  89.7
+//   28000 of  4 KB 101.8 / 101.8     10000 of 10 KB (top-4)     93.6 /  94.6
 //   skewed, 64 ranks: 10324 rows for 7200 selections 130.8 / 137.8, 13638 for 1600 130.0 / 119.8
 static bool combine_in_one_launch(int64_t rows, int num_tokens, int num_topk, int64_t row_bytes) {
     if (rows <= kLargeBatchRows) return true;
-    return rows <= 2 * int64_t(num_tokens) * num_topk && (rows + num_tokens) * row_bytes <= (int64_t(220) << 20) &&
+    return rows <= 2 * int64_t(num_tokens) * num_topk && (rows + num_tokens) * row_bytes <= (int64_t(132) << 20) &&
            (row_bytes >= 2048 || rows <= 12288);
 }
 

@@ -203,10 +203,12 @@ struct RowPart {
     }
 };
 
-// Host-side choice of the row split (log2 of the parts): small problems cannot fill the chip with
-// one wave per row.
+// Host-side choice of the row split (log2 of the parts): small problems cannot fill the chip with one wave per row, and
+// in larger ones a wave that takes a whole row is what the launch ends up waiting for.  Microseconds of a dispatch and a
+// combine in one launch, rows whole / in parts: 8800 rows of 14 KB 112.5 / 109.4, 10400 of 8 KB 82.2 / 80.8, 14400 of 4 KB
+// 61.6 / 60.8, 21600 of 4 KB 85.2 / 82.8, 28000 of 4 KB 103.1 / 100.8, but of 3 KB 84.0 / 85.0, 32768 of 2 KB 69.4 / 71.5.
 inline int choose_row_parts_log2(int64_t estimated_rows, int64_t row_bytes) {
-    if (estimated_rows > 8192) return 0;
+    if (estimated_rows > (row_bytes < 4096 ? 16384 : 32768)) return 0;
     return row_bytes > 8192 ? 2 : 1;
 }
 

@@ -611,7 +611,7 @@ int64_t deepep_ll_expected_rows_of_two(int num_tokens, int num_topk, int num_exp
  * answers of this rank's own experts are read from x directly — the own
  * experts' part of combine_staging is neither written nor read.  When at most
  * 8192 rows are expected, or more that are not many more than the batch sends
- * (up to some 220 MB), both phases run as one kernel launch; other batches launch
+ * (up to some 132 MB), both phases run as one kernel launch; other batches launch
  * them back to back.  combine_send_slots may be NULL (the reference's
  * zero_copy, deep_ep/buffer.py:2831-2852: "the next combine kernel can skip the
  * copying"): no row is returned, the call is the reduce alone, and the caller's

@@ -2075,6 +2075,36 @@ def test_combine_in_one_launch_and_in_two(rt, h, hints):
     assert all(torch.equal(sums[0], o) for o in sums[1:])
 
 
+@pytest.mark.parametrize("r,e,h,hints", [
+    (8, 16, 1024, (8193, 16384, 16385)),  # rows of 2 KB: in two parts, the last hint that splits them, whole
+    (8, 16, 2048, (8193, 16384, 16385)),  # rows of 4 KB: in two parts throughout
+    (2, 16, 7168, (8192, 8193, 8629, 8630)),  # rows of 14 KB in four parts; 132 MB with the tokens' rows, two launches
+])
+def test_combine_past_8192_rows_in_parts(rt, r, e, h, hints):
+    """How the rows of a single-launch combine are cut, and whether it is one, changes no row and no sum."""
+    rank, t, k = 1, 1025, 8
+    x_all, topk_all, w = make_world(r, t, h, k, e, seed=h + r, drop=30)
+    st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, t, O.ROW_BF16, one_call=True)
+    y = torch.randn(st.packed_recv_x.shape, generator=torch.Generator().manual_seed(h)).bfloat16().cuda()
+    world.combine_from_peers(st, mode=1, seed=5)
+    topk, weights, got = topk_all[rank].cuda(), w[rank].cuda(), []
+    for hint in (0,) + hints:
+        st.combine_send_slots.view(torch.int16).fill_(0x7FC0)
+        out = torch.zeros((t, h), dtype=torch.bfloat16, device="cuda")
+        if hint == 0:  # the two calls, which also move the rank's own rows to the staging area
+            st.expected_rows = 8192
+            st.combine_send(y)
+            st.combine_recv(topk, weights, out)
+        else:
+            st.expected_rows = hint
+            st.combine(y, topk, weights, out)
+        torch.cuda.synchronize()
+        got.append((st.combine_send_slots.view(torch.int16).clone(), out))
+    assert not torch.equal(got[0][0], torch.full_like(got[0][0], 0x7FC0))
+    for slots, out in got[1:]:
+        assert torch.equal(slots, got[0][0]) and torch.equal(out, got[0][1])
+
+
 _FORMS = ("ll_combine_fused_kernelILb0", "ll_combine_fused_kernelILb1", "ll_combine_fused_past_caches_kernel")
 
 
