@@ -336,8 +336,10 @@ __global__ __launch_bounds__(kThreads) void routing_sort_single_kernel(
 // word up eight at a time, once over all tokens and once over those before its own: the first gives where every
 // rank's ids begin, the second where its own tokens' ids do.  Against one workgroup per rank, a token's row of
 // row_of_pair is written in one piece, and the loads are independent of one another; against three launches
-// (count, scan, scatter) it is one.  What bounds it is the sums over a wave, one for every two ranks and pass, which
-// small batches pay for as much as large ones.
+// (count, scan, scatter) it is one.  What bounds it are the instructions of sixteen waves on one compute unit, so what a
+// wave need not do by itself is shared: the lanes' counts of all waves are added up in LDS, and each wave sums a few of the
+// columns over the lanes (every wave for itself, two ranks at a time, took 12.2 us for 4096 tokens to 32 ranks); bytes are
+// taken for the 0 and 1 of a bool, which one test at the end confirms; only the waves that are asked count the own tokens.
 // ---------------------------------------------------------------------
 constexpr int kWideSortTokens = 256;  // tokens per workgroup
 constexpr int kWideSortThreads = 1024;
@@ -349,86 +351,115 @@ __device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {
     return v & 0x0101010101010101ull;
 }
 
+// A token's row of kWords words out of the matrix as a buffer: zeros past its end.
+template <int kWords>
+__device__ __forceinline__ void load_member_words(__amdgpu_buffer_rsrc_t matrix, int t, uint64_t (&row)[kWords]) {
+    const int at = t * (kWords * 8);
+#pragma unroll
+    for (int q = 0; q + 1 < kWords; q += 2) {
+        const u32x4 v = load_row_u32x4<false>(matrix, at + q * 8);
+        row[q] = (uint64_t(v[1]) << 32) | v[0], row[q + 1] = (uint64_t(v[3]) << 32) | v[2];
+    }
+    if constexpr (kWords % 2 != 0) {
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(matrix, at + (kWords - 1) * 8, 0, 0);
+        row[kWords - 1] = (uint64_t(v[1]) << 32) | v[0];
+    }
+}
+
+// all[q] (bytes) += the members among this thread's tokens tid, tid + 1024, ..., before[q] those among them in front of
+// token `begin`, a multiple of 256.  kBool: bytes are 0 or 1; returns whether they were.
+template <int kWords, bool kBool>
+__device__ __forceinline__ bool count_members(__amdgpu_buffer_rsrc_t matrix, int num_tokens, int begin,
+                                              uint64_t (&all)[kWords], uint64_t (&before)[kWords]) {
+    constexpr int kAhead = kWords <= 4 ? 4 : 2;  // tokens in flight
+    const int tid = threadIdx.x;
+    uint64_t bits = 0;
+#pragma unroll
+    for (int q = 0; q < kWords; ++q) all[q] = before[q] = 0;
+    for (int t0 = 0; t0 < num_tokens; t0 += kAhead * kWideSortThreads) {
+        uint64_t v[kAhead][kWords];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) load_member_words(matrix, t0 + u * kWideSortThreads + tid, v[u]);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int round = t0 + u * kWideSortThreads;
+            if constexpr (!kBool)
+#pragma unroll
+                for (int q = 0; q < kWords; ++q) v[u][q] = nonzero_bytes(v[u][q]);
+            if (round == begin / kWideSortThreads * kWideSortThreads)  // once: what came before it is all there
+#pragma unroll
+                for (int q = 0; q < kWords; ++q) before[q] = all[q] + (round + tid < begin ? v[u][q] : 0);
+#pragma unroll
+            for (int q = 0; q < kWords; ++q) {
+                all[q] += v[u][q];
+                if constexpr (kBool) bits |= v[u][q];
+            }
+        }
+    }
+    return __ballot((bits & 0xfefefefefefefefeull) != 0) == 0;
+}
+
 template <int kWords>  // 8-byte words of a token's row: ranks / 8
 __global__ __launch_bounds__(kWideSortThreads) void routing_sort_wide_kernel(
-    const uint64_t* __restrict__ is_token_in_rank, int num_tokens, int32_t* __restrict__ send_counts,
+    const uint8_t* __restrict__ is_token_in_rank, int num_tokens, int32_t* __restrict__ send_counts,
     int64_t* __restrict__ send_cumsum, int64_t* __restrict__ sorted_token_ids, int32_t* __restrict__ row_of_pair,
     int64_t* __restrict__ report) {
     constexpr int kThreads = kWideSortThreads;
-    constexpr int kRanks = kWords * 8, kWaves = kThreads / kWave, kAhead = kWords <= 2 ? 4 : 2;
+    constexpr int kRanks = kWords * 8, kWaves = kThreads / kWave;
     constexpr int kTokenWaves = kWideSortTokens / kWave, kRankShares = kWaves / kTokenWaves;
-    __shared__ int32_t wave_all[kWaves][kRanks], wave_before[kWaves][kRanks];
+    constexpr int kColumns = kWords * 2;  // even and odd bytes of a word, widened to 16 bits
+    __shared__ unsigned long long lane_counts[2][kColumns][kWave];  // over all tokens, and over those before
+    __shared__ int32_t rank_counts[2][kRanks];
     __shared__ int32_t start[kRanks];                // where the ids of this workgroup's tokens begin, per rank
     __shared__ int32_t chunk_cnt[kTokenWaves][kRanks];
     __shared__ int32_t total_of_all;
     const int tid = threadIdx.x, lane = lane_id(), w = wave_in_block();
     const int begin = blockIdx.x * kWideSortTokens;
+    const auto matrix = row_buffer(is_token_in_rank, num_tokens * kRanks);
     // this thread's own token, loaded with the rest: wave w has tokens (w % 4) * 64 + lane
     const int tw = w & (kTokenWaves - 1), share = w / kTokenWaves;
     const int own = begin + tw * kWave + lane;
     uint64_t own_row[kWords];
-#pragma unroll
-    for (int q = 0; q < kWords; ++q) {
-        own_row[q] = is_token_in_rank[int64_t(own < num_tokens ? own : num_tokens - 1) * kWords + q];
-        if (own >= num_tokens) own_row[q] = 0;
-    }
+    load_member_words(matrix, own, own_row);
+    for (int i = tid; i < 2 * kColumns * kWave; i += kThreads) (&lane_counts[0][0][0])[i] = 0;
+    lds_barrier();
     uint64_t all[kWords], before[kWords];
+    if (!count_members<kWords, true>(matrix, num_tokens, begin, all, before))
+        count_members<kWords, false>(matrix, num_tokens, begin, all, before);
 #pragma unroll
-    for (int q = 0; q < kWords; ++q) all[q] = before[q] = 0;
-    for (int t0 = tid; t0 < num_tokens; t0 += kAhead * kThreads) {
-        uint64_t v[kAhead][kWords];
+    for (int q = 0; q < kWords; ++q)
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) {  // unconditional loads, all in flight together
-            const int t = t0 + u * kThreads;
-#pragma unroll
-            for (int q = 0; q < kWords; ++q)
-                v[u][q] = is_token_in_rank[int64_t(t < num_tokens ? t : num_tokens - 1) * kWords + q];
+        for (int odd = 0; odd < 2; ++odd) {
+            atomicAdd(&lane_counts[0][q * 2 + odd][lane], (all[q] >> (8 * odd)) & 0x00ff00ff00ff00ffull);
+            if (begin > 0) atomicAdd(&lane_counts[1][q * 2 + odd][lane], (before[q] >> (8 * odd)) & 0x00ff00ff00ff00ffull);
         }
+    if (share == 0) {  // this workgroup's own tokens per rank and wave
+        int mine = 0;
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const int t = t0 + u * kThreads;
+        for (int q = 0; q < kWords; ++q)
 #pragma unroll
-            for (int q = 0; q < kWords; ++q) {
-                const uint64_t one = t < num_tokens ? nonzero_bytes(v[u][q]) : 0;
-                all[q] += one;
-                before[q] += t < begin ? one : 0;
+            for (int i = 0; i < 8; ++i) {
+                const int votes = __popcll(__ballot(((own_row[q] >> (8 * i)) & 0xff) != 0));
+                if (lane == q * 8 + i) mine = votes;
             }
+        if (lane < kRanks) chunk_cnt[tw][lane] = mine;
+    }
+    lds_barrier();
+#pragma unroll
+    for (int c = w; c < 2 * kColumns; c += kWaves) {
+        const int which = c / kColumns, column = c % kColumns;
+        const uint64_t counts = lane_counts[which][column][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int sum = wave_inclusive_sum(int((counts >> (16 * i)) & 0xffff));
+            if (lane == kWave - 1) rank_counts[which][column / 2 * 8 + 2 * i + column % 2] = sum;
         }
     }
-    // the wave's sums: bytes widened to 16 bits (64 lanes of at most 255 fit), four ranks in two words
-#pragma unroll
-    for (int q = 0; q < kWords; ++q)
-#pragma unroll
-        for (int half = 0; half < 2; ++half)
-#pragma unroll
-            for (int odd = 0; odd < 2; ++odd) {
-                const int a = int((uint32_t(all[q] >> (32 * half)) >> (8 * odd)) & 0x00ff00ffu);
-                const int b = int((uint32_t(before[q] >> (32 * half)) >> (8 * odd)) & 0x00ff00ffu);
-                const uint32_t sa = uint32_t(wave_inclusive_sum(a)), sb = uint32_t(wave_inclusive_sum(b));
-                if (lane == kWave - 1) {
-                    const int r = q * 8 + half * 4 + odd;
-                    wave_all[w][r] = int(sa & 0xffffu), wave_all[w][r + 2] = int(sa >> 16);
-                    wave_before[w][r] = int(sb & 0xffffu), wave_before[w][r + 2] = int(sb >> 16);
-                }
-            }
-    // this workgroup's own tokens per rank and wave
-    int mine = 0;
-#pragma unroll
-    for (int q = 0; q < kWords; ++q)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int votes = __popcll(__ballot(((own_row[q] >> (8 * i)) & 0xff) != 0));
-            if (lane == q * 8 + i) mine = votes;
-        }
-    if (share == 0 && lane < kRanks) chunk_cnt[tw][lane] = mine;
     lds_barrier();
     if (w == 0) {
-        int total = 0, ahead = 0;
-        if (lane < kRanks)
-#pragma unroll
-            for (int w2 = 0; w2 < kWaves; ++w2) total += wave_all[w2][lane], ahead += wave_before[w2][lane];
+        const int total = lane < kRanks ? rank_counts[0][lane] : 0;
         const int incl = wave_inclusive_sum(total);
-        if (lane < kRanks) start[lane] = incl - total + ahead;
+        if (lane < kRanks) start[lane] = incl - total + rank_counts[1][lane];
         if (lane == kRanks - 1) total_of_all = incl;
         if (blockIdx.x == 0) {
             if (lane == kRanks - 1) send_cumsum[kRanks] = incl;
@@ -438,6 +469,7 @@ __global__ __launch_bounds__(kWideSortThreads) void routing_sort_wide_kernel(
     lds_barrier();
     // wave (share, tw) writes its 64 tokens' places in its share of the ranks
     constexpr int kPerShare = kRanks / kRankShares;
+    int place[kPerShare];
 #pragma unroll
     for (int i = 0; i < kPerShare; ++i) {
         const int r = share * kPerShare + i;
@@ -451,7 +483,18 @@ __global__ __launch_bounds__(kWideSortThreads) void routing_sort_wide_kernel(
 #pragma unroll
         for (int t2 = 0; t2 < kTokenWaves - 1; ++t2) pos += t2 < tw ? chunk_cnt[t2][r] : 0;
         if (in) sorted_token_ids[pos] = own;
-        if (row_of_pair != nullptr && own < num_tokens) row_of_pair[int64_t(own) * kRanks + r] = in ? pos : -1;
+        place[i] = in ? pos : -1;
+    }
+    if (row_of_pair != nullptr) {
+        const auto places = row_buffer(reinterpret_cast<const uint8_t*>(row_of_pair), num_tokens * (kRanks * 4));
+        const int at = own * (kRanks * 4) + share * (kPerShare * 4);
+#pragma unroll
+        for (int i = 0; i + 3 < kPerShare; i += 4)
+            store_row_u32x4<false>(places, at + i * 4,
+                                   u32x4{uint32_t(place[i]), uint32_t(place[i + 1]), uint32_t(place[i + 2]), uint32_t(place[i + 3])});
+        if constexpr (kPerShare % 4 != 0)  // two
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{uint32_t(place[kPerShare - 2]), uint32_t(place[kPerShare - 1])}, places,
+                                                  at + (kPerShare - 2) * 4, 0, 0);
     }
     report_done(report, total_of_all);
 }
@@ -721,19 +764,20 @@ size_t deepep_routing_sort_workspace_bytes(int num_tokens, int num_ranks) {
 }
 
 // Which form sorts.  Microseconds of the wide form against one workgroup per rank, with row_of_pair:
-//   ranks       8            16           32            64
-//   131 tokens  3.4 / 3.1    4.9 / 3.3    8.0 / 3.5     15.0 / 4.1
-//   2048        4.5 / 4.3    6.7 / 4.7    10.9 / 6.0    20.9 / 12.6
-//   2560        4.5 / 4.8    6.7 / 5.6    11.5 / 7.9    22.0 / 14.7
-//   4096        4.5 / 6.0    6.9 / 7.2    12.0 / 12.7   23.2 / 23.3
-//   8192        5.2 / 10.0   8.0 / 15.0   14.3 / 23.2   27.7 / 41.7
-// 24, 40, 48 and 56 ranks meet at 4096 tokens too (9.3 / 9.4 to 20.1 / 20.4), and without row_of_pair nothing moves
-// the line by more than 1 us.  Upwards every workgroup reads the whole matrix: at 512 KB that still beats the three
-// launches (8 ranks, 20000 tokens 7.2 against 16.5; 24 ranks, 12289 12.7 against 34.2; 48 ranks, 9300 21.5 against
-// 76.9), past that its work grows with the square of the batch.
+//   ranks       8            16           24           32            48            64
+//   512 tokens  3.3 / 2.9    4.0 / 3.2    5.4 / 3.5    5.8 /  3.7     7.8 /  4.2     9.6 /  5.5
+//   1024        3.3 / 3.4    4.0 / 3.6    5.4 / 3.8    5.8 /  4.0     7.8 /  4.6     9.7 /  5.6
+//   1536        3.3 / 3.8    4.0 / 4.2    5.4 / 4.6    5.9 /  5.1     7.9 /  7.1    10.0 / 10.0
+//   2047        3.3 / 4.2    4.1 / 4.7    5.4 / 5.2    5.9 /  5.9     8.0 /  8.5    10.1 / 12.7
+//   3000        3.3 / 4.4    4.1 / 5.9    5.5 / 6.9    5.9 /  8.7     8.4 / 13.1    11.4 / 17.1
+//   8192        3.9 / 10.0   4.7 / 15.0   6.7 / 20     7.0 / 23.2                   15.8 / 41.7
+// Upwards every workgroup reads the whole matrix: at 512 KB that still beats the three launches (8 ranks, 20000 tokens
+// 7.2 against 16.5 before the wide form's own time was halved; 24 ranks, 12289 7.8 against 34.2), past that its work
+// grows with the square of the batch.
 static bool sort_is_wide(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks) {
+    const int from = num_ranks == 8 ? 1024 : num_ranks == 16 ? 1280 : 2048;
     return num_ranks % 8 == 0 && num_ranks <= 64 && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 &&
-           num_tokens >= (num_ranks == 8 ? 2560 : 4096) && int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
+           num_tokens >= from && int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
 }
 static bool sort_is_single(int num_tokens, int num_ranks) {
     return num_tokens <= kSortChunk * kSingleSortTokensPerThread && num_ranks <= 64;
@@ -759,11 +803,10 @@ int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_t
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (sort_is_wide(is_token_in_rank, num_tokens, num_ranks)) {
         const int blocks = (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
-        const uint64_t* rows = reinterpret_cast<const uint64_t*>(is_token_in_rank);
 #define DEEPEP_LAUNCH_SORT(WORDS)                                                                  \
     case WORDS:                                                                                    \
         routing_sort_wide_kernel<WORDS><<<blocks, kWideSortThreads, 0, s>>>(                       \
-            rows, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host); \
+            is_token_in_rank, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host); \
         break
         switch (num_ranks / 8) {
             DEEPEP_LAUNCH_SORT(1);

@@ -189,6 +189,31 @@ SORT_FORMS += [(2559, 8), (2560, 8), (4095, 16), (4096, 16), (4096, 24), (13107,
                (10923, 48), (4097, 56), (16385, 32), (512, 16), (513, 16), (511, 64), (257, 5)]
 
 
+@pytest.mark.parametrize("t,r", [(1023, 8), (1024, 8), (1279, 16), (1280, 16), (2047, 24), (2048, 24), (2049, 32),
+                                 (4096, 64), (20001, 8), (13107, 40), (10500, 48), (65536, 8)])
+@pytest.mark.parametrize("values", ["bool", "bytes", "all"])
+def test_routing_sort_eight_ranks_a_word(capi, t, r, values):
+    """Either side of the line from which the sort adds up eight ranks at a time: any byte but zero is a member, and
+    counts reach every token of the batch."""
+    lib = capi.load()
+    g = torch.Generator().manual_seed(t + r)
+    is_in = torch.ones((t, r), dtype=torch.bool) if values == "all" else torch.rand((t, r), generator=g) < 0.3
+    member = is_in.to(torch.uint8)
+    if values == "bytes":
+        member *= torch.tensor([1, 2, 16, 128, 255], dtype=torch.uint8)[torch.randint(5, (t, r), generator=g)]
+    dev = member.cuda()
+    ids, inverse = (torch.full((t * r,), -7, dtype=d, device="cuda") for d in (torch.int64, torch.int32))
+    counts = torch.full((r,), -1, dtype=torch.int32, device="cuda")
+    cumsum = torch.full((r + 1,), -1, dtype=torch.int64, device="cuda")
+    ws = torch.empty(max(256, lib.deepep_routing_sort_workspace_bytes(t, r)), dtype=torch.uint8, device="cuda")
+    capi.check(lib.deepep_moe_routing_sort(capi.ptr(dev), t, r, capi.ptr(ids), capi.ptr(counts), capi.ptr(cumsum),
+                                           capi.ptr(inverse), capi.ptr(ws), ws.numel(), stream()))
+    w_ids, w_counts, w_cumsum, total = O.moe_routing_sort(is_in)
+    assert torch.equal(counts.cpu(), w_counts) and torch.equal(cumsum.cpu(), w_cumsum)
+    assert torch.equal(ids[:total].cpu(), w_ids) and (ids[total:] == -7).all()
+    assert torch.equal(inverse.view(t, r).cpu(), _want_row_of_pair(is_in, w_ids, w_cumsum))
+
+
 @pytest.mark.parametrize("t,r", SORT_FORMS)
 def test_routing_sort_reports_every_workgroup(capi, t, r):
     """As many words as promised are set, the last to the total, and none beyond them."""
@@ -211,8 +236,8 @@ def test_routing_sort_reports_every_workgroup(capi, t, r):
 
 @pytest.mark.parametrize("t,r", [(1, 8), (131, 16), (2000, 64), (4096, 48)])
 def test_routing_sort_takes_the_form_measured_fastest(capi, t, r):
-    """One workgroup per rank up to 4095 tokens (2559 at 8 ranks), where the form that adds up eight ranks at a time
-    is up to four times as slow; a matrix whose address does not allow 8-byte loads never takes that form."""
+    """One workgroup per rank up to 2047 tokens (1023 at 8 ranks, 1279 at 16), where the form that adds up eight ranks at
+    a time is up to twice as slow; a matrix whose address does not allow 8-byte loads never takes that form."""
     lib = capi.load()
     assert lib.deepep_routing_sort_report_words(None, t, r) == (r if t < 4096 else (t + 255) // 256)
     assert lib.deepep_routing_sort_report_words(4, t, r) == r
