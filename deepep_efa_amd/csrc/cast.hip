@@ -64,9 +64,9 @@ extern "C" int deepep_per_token_cast_to_fp8(const void* x, int num_rows, int num
 #define DEEPEP_LAUNCH_CAST(FMT)                                                                                  \
     do {                                                                                                         \
         if (streams)                                                                                             \
-            per_token_cast_kernel<FMT, true><<<blocks, 256, 0, s>>>(xb, num_rows, num_cols, pieces, qb, sb);  \
+            launch(per_token_cast_kernel<FMT, true>, blocks, 256, 0, s, xb, num_rows, num_cols, pieces, qb, sb);  \
         else                                                                                                     \
-            per_token_cast_kernel<FMT, false><<<blocks, 256, 0, s>>>(xb, num_rows, num_cols, pieces, qb, sb); \
+            launch(per_token_cast_kernel<FMT, false>, blocks, 256, 0, s, xb, num_rows, num_cols, pieces, qb, sb); \
     } while (0)
     switch (row_format) {
         case kRowFP8: DEEPEP_LAUNCH_CAST(kRowFP8); break;

@@ -743,7 +743,7 @@ int deepep_get_dispatch_layout(const int64_t* topk_idx, int num_tokens, int num_
     const uint32_t rank_magic =
         experts_per_rank == 1 ? 0u : uint32_t(((uint64_t(1) << 32) + experts_per_rank - 1) / experts_per_rank);
 #define DEEPEP_LAUNCH_LAYOUT(WORDS)                                                                              \
-    layout_count_kernel<WORDS><<<blocks, threads, size_t(width) * 4, s>>>(                                        \
+    launch(layout_count_kernel<WORDS>, blocks, threads, size_t(width) * 4, s,                                         \
         topk_idx, num_tokens, num_topk, num_ranks, num_experts, rank_magic, num_nodes, is_token_in_rank, partial, \
         num_tokens_per_rank, num_tokens_per_rdma_rank, num_tokens_per_expert)
     if (num_ranks <= kWave) DEEPEP_LAUNCH_LAYOUT(1);
@@ -751,7 +751,7 @@ int deepep_get_dispatch_layout(const int64_t* topk_idx, int num_tokens, int num_
 #undef DEEPEP_LAUNCH_LAYOUT
     EP_LAUNCH_CHECK();
     if (blocks == 1) return 0;
-    layout_reduce_kernel<<<(width + kLayoutThreads - 1) / kLayoutThreads, kLayoutThreads, 0, s>>>(
+    launch(layout_reduce_kernel, (width + kLayoutThreads - 1) / kLayoutThreads, kLayoutThreads, 0, s,
         partial, blocks, num_experts, num_ranks, num_nodes, num_tokens_per_rank, num_tokens_per_rdma_rank,
         num_tokens_per_expert);
     EP_LAUNCH_CHECK();
@@ -805,7 +805,7 @@ int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_t
         const int blocks = (num_tokens + kWideSortTokens - 1) / kWideSortTokens;
 #define DEEPEP_LAUNCH_SORT(WORDS)                                                                  \
     case WORDS:                                                                                    \
-        routing_sort_wide_kernel<WORDS><<<blocks, kWideSortThreads, 0, s>>>(                       \
+        launch(routing_sort_wide_kernel<WORDS>, blocks, kWideSortThreads, 0, s,                        \
             is_token_in_rank, num_tokens, send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host); \
         break
         switch (num_ranks / 8) {
@@ -824,7 +824,7 @@ int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_t
     }
     if (sort_is_single(num_tokens, num_ranks)) {
 #define DEEPEP_LAUNCH_SORT(THREADS)                                                                            \
-    routing_sort_single_kernel<THREADS><<<num_ranks, THREADS, 0, s>>>(                                          \
+    launch(routing_sort_single_kernel<THREADS>, num_ranks, THREADS, 0, s,                                           \
         is_token_in_rank, num_tokens, num_ranks, num_tokens == 0 ? 1 : (num_tokens + THREADS - 1) / THREADS,    \
         send_counts, send_cumsum, sorted_token_ids, row_of_pair, report_host)
         if (num_tokens <= kSmallSortTokens) DEEPEP_LAUNCH_SORT(256);
@@ -835,15 +835,15 @@ int deepep_moe_routing_sort_reporting(const uint8_t* is_token_in_rank, int num_t
     }
     int32_t* table = reinterpret_cast<int32_t*>(workspace);
     const size_t lds = size_t(kSortChunk / kWave) * num_ranks * 4;
-    routing_sort_pass_kernel<false><<<chunks, kSortChunk, lds, s>>>(is_token_in_rank, num_tokens, num_ranks, table,
+    launch(routing_sort_pass_kernel<false>, chunks, kSortChunk, lds, s, is_token_in_rank, num_tokens, num_ranks, table,
                                                                     sorted_token_ids, nullptr, nullptr, nullptr);
     EP_LAUNCH_CHECK();
-    routing_sort_scan_kernel<<<1, 256, size_t(num_ranks + 1) * 8, s>>>(table, chunks, num_ranks, send_counts,
+    launch(routing_sort_scan_kernel, 1, 256, size_t(num_ranks + 1) * 8, s, table, chunks, num_ranks, send_counts,
                                                                        send_cumsum,
                                                                        num_tokens == 0 ? report_host : nullptr);
     EP_LAUNCH_CHECK();
     if (num_tokens > 0) {
-        routing_sort_pass_kernel<true><<<chunks, kSortChunk, lds, s>>>(is_token_in_rank, num_tokens, num_ranks,
+        launch(routing_sort_pass_kernel<true>, chunks, kSortChunk, lds, s, is_token_in_rank, num_tokens, num_ranks,
                                                                        table, sorted_token_ids, row_of_pair,
                                                                        send_cumsum + num_ranks, report_host);
         EP_LAUNCH_CHECK();
@@ -877,8 +877,8 @@ int deepep_channel_prefix_matrix(const uint8_t* is_token_in_rank, int num_tokens
     const bool by_words = num_ranks == 8 || (num_ranks % 8 == 0 && num_ranks <= 32 && num_tokens >= 2048);
     if (by_words && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 && num_channels <= 1024) {
 #define DEEPEP_LAUNCH_CHANNELS(AHEAD)                                                                              \
-    channel_prefix_words_kernel<AHEAD><<<num_ranks / 8, threads, size_t(num_channels) * 32,                        \
-                                         reinterpret_cast<hipStream_t>(stream)>>>(                                 \
+    launch(channel_prefix_words_kernel<AHEAD>, num_ranks / 8, threads, size_t(num_channels) * 32,                        \
+                                         reinterpret_cast<hipStream_t>(stream),                                  \
         reinterpret_cast<const uint64_t*>(is_token_in_rank), num_tokens, num_ranks / 8, num_channels,              \
         channel_prefix_matrix)
         if ((int64_t(num_tokens) + num_channels - 1) / num_channels <= 4 * kWave) DEEPEP_LAUNCH_CHANNELS(4);
@@ -887,7 +887,7 @@ int deepep_channel_prefix_matrix(const uint8_t* is_token_in_rank, int num_tokens
         EP_LAUNCH_CHECK();
         return 0;
     }
-    channel_prefix_kernel<<<num_ranks, threads, size_t(num_channels) * 4, reinterpret_cast<hipStream_t>(stream)>>>(
+    launch(channel_prefix_kernel, num_ranks, threads, size_t(num_channels) * 4, reinterpret_cast<hipStream_t>(stream),
         is_token_in_rank, num_tokens, num_ranks, num_channels, channel_prefix_matrix);
     EP_LAUNCH_CHECK();
     return 0;
@@ -930,17 +930,17 @@ int deepep_pack_rows_by_rank(const void* src, const void* scale_src, const int64
         const uint32_t slots = uint32_t(needed < (1 << 14) ? needed : (1 << 14));  // the kernel goes round for the rest
         const unsigned blocks = slots << group_log2;
         if (stream_rows)
-            pack_groups_kernel<true><<<blocks, threads, 0, hs>>>(send_cumsum, sorted_token_ids, max_rows, num_ranks,
+            launch(pack_groups_kernel<true>, blocks, threads, 0, hs, send_cumsum, sorted_token_ids, max_rows, num_ranks,
                                                                  group_log2, slots, a);
         else
-            pack_groups_kernel<false><<<blocks, threads, 0, hs>>>(send_cumsum, sorted_token_ids, max_rows, num_ranks,
+            launch(pack_groups_kernel<false>, blocks, threads, 0, hs, send_cumsum, sorted_token_ids, max_rows, num_ranks,
                                                                   group_log2, slots, a);
     } else {
         const unsigned blocks = unsigned(max_rows < (int64_t(1) << 22) ? max_rows : int64_t(1) << 22);
         if (stream_rows)
-            pack_rows_kernel<true><<<blocks, threads, 0, hs>>>(num_rows_dev, sorted_token_ids, max_rows, blocks, a);
+            launch(pack_rows_kernel<true>, blocks, threads, 0, hs, num_rows_dev, sorted_token_ids, max_rows, blocks, a);
         else
-            pack_rows_kernel<false><<<blocks, threads, 0, hs>>>(num_rows_dev, sorted_token_ids, max_rows, blocks, a);
+            launch(pack_rows_kernel<false>, blocks, threads, 0, hs, num_rows_dev, sorted_token_ids, max_rows, blocks, a);
     }
     EP_LAUNCH_CHECK();
     return 0;

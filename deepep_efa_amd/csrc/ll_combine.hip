@@ -535,7 +535,7 @@ static int launch_combine_send(const void* x, const int64_t* layout_range, int h
         if (int rc = make_combine_index(layout_range, num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank,
                                         skip_own, workspace, workspace_bytes, index))
             return rc;
-        ll_combine_index_kernel<<<num_experts, 256, size_t(num_experts + 1) * sizeof(int32_t), hs>>>(index);
+        launch(ll_combine_index_kernel, num_experts, 256, size_t(num_experts + 1) * sizeof(int32_t), hs, index);
         EP_LAUNCH_CHECK();
         return launch_combine_rows(index, x, hidden, combine_staging, combine_send_slots, expected_rows, hs);
     }
@@ -545,7 +545,7 @@ static int launch_combine_send(const void* x, const int64_t* layout_range, int h
     int64_t blocks = ((max_rows << sa.parts_log2) + 3) / 4;
     const int64_t cap = large ? 4096 : 1024;
     if (blocks > cap) blocks = cap;
-    ll_combine_send_kernel<<<dim3(unsigned(blocks)), 256, 0, hs>>>(sa, skip_own);
+    launch(ll_combine_send_kernel, dim3(unsigned(blocks)), 256, 0, hs, sa, skip_own);
     EP_LAUNCH_CHECK();
     return 0;
 }
@@ -569,10 +569,10 @@ static void launch_reduce(const CombineRecvArgs& ra, const uint8_t* own, const i
     const int64_t blocks = index_blocks + (int64_t(ra.num_tokens) * ra.pieces_per_row + waves - 1) / waves;
     const size_t lds = size_t(index_blocks > 0 ? index_blocks + 1 : num_local_experts) * sizeof(int32_t);
     if (stream_rows)
-        ll_combine_recv_kernel<true><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(
+        launch(ll_combine_recv_kernel<true>, dim3(unsigned(blocks)), waves * kWave, lds, hs,
             ra, own, layout_range, rank, num_local_experts, num_ranks, uint32_t(waves), ia, index_blocks);
     else
-        ll_combine_recv_kernel<false><<<dim3(unsigned(blocks)), waves * kWave, lds, hs>>>(
+        launch(ll_combine_recv_kernel<false>, dim3(unsigned(blocks)), waves * kWave, lds, hs,
             ra, own, layout_range, rank, num_local_experts, num_ranks, uint32_t(waves), ia, index_blocks);
 }
 
@@ -638,7 +638,7 @@ int deepep_ll_combine_send_by_dest(const void* x, const int32_t* record_packed_r
     const unsigned grid = flat_grid_blocks(sized_for, row_capacity, threads);
     const int64_t x_rows = std::min(int64_t(num_experts) * num_max_dispatch_tokens_per_rank, int64_t(1) << 31);
 #define DEEPEP_LAUNCH_BY_DEST(LOAD, STORE, PEERS)                                                                       \
-    ll_combine_send_by_dest_kernel<LOAD, STORE, PEERS><<<grid, threads, 0, reinterpret_cast<hipStream_t>(stream)>>>(    \
+    launch(ll_combine_send_by_dest_kernel<LOAD, STORE, PEERS>, grid, threads, 0, reinterpret_cast<hipStream_t>(stream),     \
         num_recv_tokens, padded_index, record_packed_row, combine_send_offset, uint32_t(row_capacity),                  \
         uint32_t(x_rows), reinterpret_cast<const uint8_t*>(x),                                                          \
         reinterpret_cast<uint8_t*>(send_flat), num_vec, threads, grid, peers)
@@ -774,7 +774,7 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     const int64_t traffic = ((returns_rows ? 2 * rows : 0) + int64_t(num_tokens) * num_topk) * hidden * 2;
     const int64_t gather_streams = returns_rows ? kGatherStreamBytes : kGatherAloneStreamBytes;
 #define DEEPEP_LAUNCH_FUSED(KERNEL) \
-    KERNEL<<<dim3(unsigned(recv_blocks + send_blocks)), 256, lds, reinterpret_cast<hipStream_t>(stream)>>>(sa, ra, int(recv_blocks))
+    launch(KERNEL, dim3(unsigned(recv_blocks + send_blocks)), 256, lds, reinterpret_cast<hipStream_t>(stream), sa, ra, int(recv_blocks))
     if (large || traffic > stream_bytes()) DEEPEP_LAUNCH_FUSED(ll_combine_fused_past_caches_kernel);
     else if (traffic > gather_streams) DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<true, false>));
     else if (recv_blocks + send_blocks <= kWorkgroupsAtOnce) DEEPEP_LAUNCH_FUSED((ll_combine_fused_kernel<false, true>));

@@ -1177,8 +1177,8 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         batch.slots = slots_in_scratch ? reinterpret_cast<int32_t*>(ws + hist_bytes + first_bytes) : pair_slot;
         batch.stride = scratch_bytes / 4;
         if (batch.num_chunks > 0) {
-            ll_rank_chunk_kernel<<<dim3(batch.num_chunks * kRankParts, num_src), kRankPart,
-                                   size_t(num_experts) * (kRankWaves + sizeof(int32_t)), stream>>>(
+            launch(ll_rank_chunk_kernel, dim3(batch.num_chunks * kRankParts, num_src), kRankPart,
+                                   size_t(num_experts) * (kRankWaves + sizeof(int32_t)), stream,
                 topk_idx, n, num_topk, num_experts, reinterpret_cast<int32_t*>(ws), batch, recv_count, num_ranks, rank,
                 max_tokens);
             EP_LAUNCH_CHECK();
@@ -1222,7 +1222,7 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     sa.prefix_in_block = prefix_in_block ? 1 : 0;
     sa.by_dest = by_dest != nullptr ? *by_dest : ByDestTables{nullptr, nullptr, nullptr};
     if (ranked && batch.in_full) {
-        ll_rank_finish_kernel<<<dim3(batch.num_chunks + 1, num_src), 1024, size_t(num_experts + 1) * sizeof(int32_t), stream>>>(
+        launch(ll_rank_finish_kernel, dim3(batch.num_chunks + 1, num_src), 1024, size_t(num_experts + 1) * sizeof(int32_t), stream,
             sa, batch);
         EP_LAUNCH_CHECK();
     }
@@ -1250,9 +1250,9 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
 #define DEEPEP_LAUNCH_FUSED(FMT)                                                                        \
     do {                                                                                                \
         if (fused_streams)                                                                              \
-            ll_dispatch_fused_kernel<FMT, true><<<dim3(unsigned(total)), waves * kWave, lds, stream>>>(sa, ra, blocks_per_token, num_send_blocks); \
+            launch(ll_dispatch_fused_kernel<FMT, true>, dim3(unsigned(total)), waves * kWave, lds, stream, sa, ra, blocks_per_token, num_send_blocks); \
         else                                                                                            \
-            ll_dispatch_fused_kernel<FMT, false><<<dim3(unsigned(total)), waves * kWave, lds, stream>>>(sa, ra, blocks_per_token, num_send_blocks); \
+            launch(ll_dispatch_fused_kernel<FMT, false>, dim3(unsigned(total)), waves * kWave, lds, stream, sa, ra, blocks_per_token, num_send_blocks); \
     } while (0)
         switch (row_format) {
             case kRowBF16: DEEPEP_LAUNCH_FUSED(kRowBF16); break;
@@ -1289,10 +1289,10 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
 #define DEEPEP_LAUNCH_SEND_AS(FMT, STREAM)                                                                             \
     do {                                                                                                               \
         if (ranked)                                                                                                    \
-            ll_send_ranked_kernel<FMT, STREAM><<<grid, waves * kWave, lds, stream>>>(sa, direct, batch, index,         \
+            launch(ll_send_ranked_kernel<FMT, STREAM>, grid, waves * kWave, lds, stream, sa, direct, batch, index,         \
                                                                                      index_rows, topk_log2);           \
         else                                                                                                           \
-            ll_send_kernel<FMT, STREAM><<<grid, waves * kWave, lds, stream>>>(sa);                                     \
+            launch(ll_send_kernel<FMT, STREAM>, grid, waves * kWave, lds, stream, sa);                                     \
     } while (0)
 #define DEEPEP_LAUNCH_SEND(FMT)                            \
     do {                                                   \
@@ -1521,7 +1521,7 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
         RowDesc* desc = reinterpret_cast<RowDesc*>(reinterpret_cast<uint8_t*>(workspace) +
                                                    (((int64_t(num_experts) + 1) * 4 + 255) & ~int64_t(255)));
         if (!index_done) {  // (a large one-call dispatch builds the index inside its send launch)
-            ll_segment_index_kernel<<<num_experts, kIndexThreads, 0, hs>>>(
+            launch(ll_segment_index_kernel, num_experts, kIndexThreads, 0, hs,
                 recv_count, num_local_experts, num_ranks, own_rank, num_max_dispatch_tokens_per_rank,
                 packed_recv_layout_range, packed_recv_count, cumulative_local_expert_recv_stats, flat, desc, observed);
             EP_LAUNCH_CHECK();
@@ -1549,7 +1549,7 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
     const int64_t cap = large ? 4096 : 1024;
     if (blocks > cap) blocks = cap;
     const size_t lds = size_t(num_experts + 1 + num_local_experts) * sizeof(int32_t);
-    ll_recv_kernel<<<dim3(unsigned(blocks) + 1), 256, lds, hs>>>(ra, nullptr, 0, own_rank);  // + the metadata workgroup
+    launch(ll_recv_kernel, dim3(unsigned(blocks) + 1), 256, lds, hs, ra, nullptr, 0, own_rank);  // + the metadata workgroup
     EP_LAUNCH_CHECK();
     return 0;
 }

@@ -159,7 +159,7 @@ extern "C" int deepep_ll_exchange_metadata(const int32_t* all_num_routed, int nu
                                          padded_index != nullptr && combine_send_offset != nullptr));
     int64_t blocks = (row_capacity + 4 * kExchangeThreads - 1) / (4 * kExchangeThreads);
     blocks = blocks < 1 ? 1 : (blocks > 64 ? 64 : blocks);
-    ll_exchange_meta_kernel<<<unsigned(blocks), kExchangeThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+    launch(ll_exchange_meta_kernel, unsigned(blocks), kExchangeThreads, 0, reinterpret_cast<hipStream_t>(stream),
         all_num_routed, num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank, row_capacity, send_counts,
         recv_counts, totals, combine_remote_recv_offset, source_rank, source_offset, padded_index,
         combine_send_offset, num_recv_tokens, tokens_per_expert);

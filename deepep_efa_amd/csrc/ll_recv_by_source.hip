@@ -596,7 +596,7 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
     // same result, and a buffer sized for its largest batch still takes the short form for a small one.
     const int64_t expected_records = expected_rows > 0 && expected_rows < row_capacity ? expected_rows : row_capacity;
     if (expected_records <= kBySourceSmallRecords) {
-        ll_by_source_index_kernel<false><<<num_ranks, kBySourceThreads, index_lds, hs>>>(
+        launch(ll_by_source_index_kernel<false>, num_ranks, kBySourceThreads, index_lds, hs,
             rows_in, stride, tail_off, buffer_rows, int(slot_rows), recv_counts, source_offset, num_recv_tokens,
             row_capacity, num_local_experts, num_ranks, num_max_dispatch_tokens_per_rank, nullptr,
             packed_recv_layout_range, packed_recv_count, cumulative_local_expert_recv_stats, tokens_per_expert,
@@ -606,11 +606,11 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
         // every source's records round up to whole chunks: at most ceil(capacity / 512) + R of them
         const int64_t chunks = (row_capacity + kBySourceThreads - 1) / kBySourceThreads + num_ranks;
         const size_t count_lds = size_t(2 * (num_ranks + 1) + num_local_experts) * sizeof(int32_t);
-        ll_by_source_count_kernel<<<unsigned(chunks), kBySourceThreads, count_lds, hs>>>(
+        launch(ll_by_source_count_kernel, unsigned(chunks), kBySourceThreads, count_lds, hs,
             rows_in, stride, tail_off, buffer_rows, int(slot_rows), recv_counts, source_offset, num_recv_tokens,
             row_capacity, num_local_experts, num_ranks, hist);
         EP_LAUNCH_CHECK();
-        ll_by_source_index_kernel<true><<<unsigned(chunks), kBySourceThreads, index_lds, hs>>>(
+        launch(ll_by_source_index_kernel<true>, unsigned(chunks), kBySourceThreads, index_lds, hs,
             rows_in, stride, tail_off, buffer_rows, int(slot_rows), recv_counts, source_offset, num_recv_tokens,
             row_capacity, num_local_experts, num_ranks, num_max_dispatch_tokens_per_rank, hist,
             packed_recv_layout_range, packed_recv_count, cumulative_local_expert_recv_stats, tokens_per_expert,
@@ -693,13 +693,13 @@ int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_
         int64_t blocks = ((rows << oa.parts_log2) + 3) / 4;
         blocks = blocks < 1 ? 1 : (blocks > 1024 ? 1024 : blocks);
         const size_t lds = size_t(4 * (num_experts + 1)) * sizeof(int32_t);
-        ll_recv_ordered_kernel<<<dim3(unsigned(blocks) + 1), 256, lds, hs>>>(oa);  // + the metadata workgroup
+        launch(ll_recv_ordered_kernel, dim3(unsigned(blocks) + 1), 256, lds, hs, oa);  // + the metadata workgroup
         EP_LAUNCH_CHECK();
         return 0;
     }
     int32_t* flat_total = reinterpret_cast<int32_t*>(workspace);
     RowDesc* desc = reinterpret_cast<RowDesc*>(reinterpret_cast<uint8_t*>(workspace) + by_source_head_bytes());
-    ll_by_source_ordered_index_kernel<<<num_experts, kIndexThreads, 0, hs>>>(
+    launch(ll_by_source_ordered_index_kernel, num_experts, kIndexThreads, 0, hs,
         all_num_routed, num_experts, num_local_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank,
         int(slot_rows), row_capacity, packed_recv_layout_range, packed_recv_count,
         cumulative_local_expert_recv_stats, tokens_per_expert, record_packed_row, flat_total, desc);

@@ -161,7 +161,7 @@ int deepep_synth_topk_idx(const uint32_t* expert_cdf, const int32_t* src_ranks, 
     EP_HOST_ASSERT(expert_cdf != nullptr && src_ranks != nullptr && topk_idx != nullptr);
     const int64_t blocks = (n + 255) / 256;
     EP_HOST_ASSERT(blocks < (int64_t(1) << 31));
-    synth_topk_kernel<<<dim3(unsigned(blocks)), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+    launch(synth_topk_kernel, dim3(unsigned(blocks)), 256, 0, reinterpret_cast<hipStream_t>(stream),
         expert_cdf, src_ranks, num_src, num_tokens, num_topk, num_experts, seed, topk_idx);
     EP_LAUNCH_CHECK();
     return 0;
@@ -178,7 +178,7 @@ int deepep_synth_bf16_rows(void* dst, int64_t num_rows, int hidden, int64_t row_
     EP_HOST_ASSERT(dst != nullptr && (reinterpret_cast<uintptr_t>(dst) & 15) == 0);
     int64_t blocks = (num_rows + 3) / 4;
     if (blocks > 16384) blocks = 16384;
-    synth_bf16_rows_kernel<<<dim3(unsigned(blocks)), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+    launch(synth_bf16_rows_kernel, dim3(unsigned(blocks)), 256, 0, reinterpret_cast<hipStream_t>(stream),
         reinterpret_cast<uint8_t*>(dst), num_rows, hidden, row_stride_bytes, row_keys, first_key, seed,
         outlier_period);
     EP_LAUNCH_CHECK();
@@ -202,7 +202,7 @@ int deepep_loopback_combine_from_peers(const void* send_slots, const int32_t* se
     const int64_t items = int64_t(num_experts) * num_max_dispatch_tokens_per_rank;
     const int64_t blocks = (items + 3) / 4;
     EP_HOST_ASSERT(blocks < (int64_t(1) << 31));
-    combine_from_peers_kernel<<<dim3(unsigned(blocks)), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+    launch(combine_from_peers_kernel, dim3(unsigned(blocks)), 256, 0, reinterpret_cast<hipStream_t>(stream),
         reinterpret_cast<const uint8_t*>(send_slots), send_count, hidden, num_experts, num_experts / num_ranks, rank,
         num_max_dispatch_tokens_per_rank, row_format, mode, seed, reinterpret_cast<uint8_t*>(combine_staging));
     EP_LAUNCH_CHECK();

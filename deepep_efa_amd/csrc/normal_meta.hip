@@ -232,8 +232,8 @@ int deepep_topk_remap(const int64_t* topk_idx, const float* topk_weights, const 
     if (max_send == 0) return 0;
     EP_HOST_ASSERT(topk_idx != nullptr && topk_weights != nullptr && sorted_token_ids != nullptr &&
                    send_cumsum != nullptr && remapped_topk != nullptr && remapped_weights != nullptr);
-    topk_remap_kernel<<<meta_grid(max_send * num_topk), kMetaThreads, size_t(num_ranks + 1) * sizeof(int64_t),
-                        reinterpret_cast<hipStream_t>(stream)>>>(
+    launch(topk_remap_kernel, meta_grid(max_send * num_topk), kMetaThreads, size_t(num_ranks + 1) * sizeof(int64_t),
+                        reinterpret_cast<hipStream_t>(stream),
         topk_idx, topk_weights, sorted_token_ids, send_cumsum, num_tokens, num_topk, num_ranks, num_local_experts,
         max_send, remapped_topk, remapped_weights);
     EP_LAUNCH_CHECK();
@@ -248,8 +248,8 @@ int deepep_build_recv_src_meta(const int64_t* recv_cumsum, int num_ranks, int nu
     if (max_recv_tokens == 0) return 0;
     EP_HOST_ASSERT(recv_cumsum != nullptr && recv_src_meta != nullptr);
     EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(recv_src_meta) & 7) == 0);
-    recv_src_meta_kernel<<<meta_grid(max_recv_tokens), kMetaThreads, size_t(num_ranks + 1) * sizeof(int64_t),
-                           reinterpret_cast<hipStream_t>(stream)>>>(recv_cumsum, num_ranks, num_local_ranks,
+    launch(recv_src_meta_kernel, meta_grid(max_recv_tokens), kMetaThreads, size_t(num_ranks + 1) * sizeof(int64_t),
+                           reinterpret_cast<hipStream_t>(stream), recv_cumsum, num_ranks, num_local_ranks,
                                                                     max_recv_tokens,
                                                                     reinterpret_cast<u32x2*>(recv_src_meta));
     EP_LAUNCH_CHECK();
@@ -286,7 +286,7 @@ int deepep_combine_reduce(const void* recv_x, const float* recv_topk_weights, co
     const int32_t* row_of_pair = row_of_pair_in;
     if (row_of_pair_in == nullptr) row_of_pair = reinterpret_cast<int32_t*>(workspace);
     if (max_rows > 0 && row_of_pair_in == nullptr) {
-        combine_positions_kernel<<<meta_grid(max_rows), kMetaThreads, size_t(num_ranks + 1) * sizeof(int64_t), hs>>>(
+        launch(combine_positions_kernel, meta_grid(max_rows), kMetaThreads, size_t(num_ranks + 1) * sizeof(int64_t), hs,
             sorted_token_ids, send_cumsum, num_tokens, num_ranks, max_rows, reinterpret_cast<int32_t*>(workspace));
         EP_LAUNCH_CHECK();
     }
@@ -299,7 +299,7 @@ int deepep_combine_reduce(const void* recv_x, const float* recv_topk_weights, co
     if (stream_rows) blocks = (blocks + kReduceRound - 1) / kReduceRound * kReduceRound;
     EP_HOST_ASSERT(blocks < (int64_t(1) << 31) && int64_t(num_tokens) * pieces < (int64_t(1) << 32));
 #define DEEPEP_LAUNCH_REDUCE(STREAM)                                                                             \
-    combine_reduce_kernel<STREAM><<<dim3(unsigned(blocks)), waves * kWave, 0, hs>>>(                              \
+    launch(combine_reduce_kernel<STREAM>, dim3(unsigned(blocks)), waves * kWave, 0, hs,                               \
         reinterpret_cast<const uint8_t*>(recv_x), recv_topk_weights, is_token_in_rank, row_of_pair,               \
         reinterpret_cast<const uint8_t*>(bias_0), reinterpret_cast<const uint8_t*>(bias_1), num_tokens,          \
         hidden * 2, num_topk, num_ranks, int(max_rows), uint32_t(pieces), uint32_t(waves),                       \

@@ -551,7 +551,7 @@ inline void launch_rows_flat(const int32_t* total, const RowDesc* desc, int64_t 
     const int others = tails != nullptr ? kWave : 0, threads = flat_row_threads(num_vec, 1024 - others);
     const unsigned grid = flat_grid_blocks(pairs ? expected_rows / 2 : expected_rows, max_rows, threads + others);
 #define DEEPEP_LAUNCH_ROWS(TAILS)                                                                                     \
-    ll_rows_flat_kernel<TAILS><<<grid, threads + others, 0, stream>>>(                                                \
+    launch(ll_rows_flat_kernel<TAILS>, grid, threads + others, 0, stream,                                                 \
         total, desc, uint32_t(max_rows), grid, reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst), \
         uint32_t(src_stride), uint32_t(dst_stride), num_vec, threads, reinterpret_cast<uint8_t*>(dst_own),            \
         tails != nullptr ? *tails : FlatTails{})
