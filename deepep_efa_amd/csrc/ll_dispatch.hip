@@ -109,6 +109,18 @@ constexpr int kMaxTopk = 64;
 constexpr int kFusedMaxEntries = 8192;     // send + receive in one launch up to here
 constexpr int kSendMaxWaves = 16;
 
+// A workgroup that ranks its own slots takes two or four tokens where it has waves for them, and one sweep through the
+// entries serves them all: while that leaves 240 workgroups of them, about one for every compute unit.  The sweeps are
+// instructions and LDS adds on every compute unit; so are the receive workgroups' for the own counts in the single-launch
+// dispatch, of which there are half as many then, 512 instead of 1024 (640 give 0.7 us of the first figure back).  There
+// it pays where a row has one or two pieces and four waves are more than a token takes.  Microseconds of a step or an
+// exchange, one token a workgroup / several:
+//   step, 1000 x 2048     39.2 / 36.3     exchange, 1000 x 2048  47.2 / 44.8     step, 509 x 4096  23.5 / 23.8 and 24.4 / 23.9
+//   700 x 2048            28.6 / 27.4     700 x 2048             38.4 / 36.8     400 x 4096, in 200 workgroups  28.6 / 30.2
+//   900 x 2048, top-6     31.2 / 29.7     1000 x 5120            91.1 / 87.6     700 x 4096        42.0 / 41.7
+//   500 x 2048            22.2 / 21.4     512 x 7168             65.5 / 64.4     1000 x 4096       57.5 / 57.4
+constexpr int kManyBlocks = 240;
+
 struct ByDestTables {
     int32_t* expert_prefix;  // [E + 1]
     int32_t* rank_counts;    // [R]
@@ -121,6 +133,8 @@ struct SendArgs {
     const int32_t* src_ranks;  // null: the rows are this rank's own
     int num_tokens, hidden, num_topk, num_experts, num_ranks, rank, max_tokens;
     int pieces_per_row, split_log2;
+    int tokens_per_block;  // 2 or 4: whole tokens, pieces_per_row << split_log2 waves each
+    RankDivider token_of;  // a workgroup's entry to the token among its own: division by K
     uint32_t rank_of_expert_magic;
     uint8_t* recv_staging;
     uint8_t* send_slots;
@@ -293,22 +307,28 @@ __device__ __forceinline__ void store_selections(uint64_t my_row, uint64_t my_sc
 // allocated in the memory-side cache and written back later).  The token rows are read, and the
 // scales and tails stored, the ordinary way: the hint measured slower on those (63 and 56 us).
 // kTables: the launch may be one that makes the by-destination tables.
-template <int kFmt, bool kStream, bool kTables>
+// kMany: the workgroup's share are the tokens_per_block tokens from t on, which are ranked by one sweep; lane i of wave 0
+// has the i-th of their selections.
+template <int kFmt, bool kStream, bool kTables, bool kMany>
 __device__ __forceinline__ void send_token_block(const SendArgs& a, const DirectOut& direct, int b, int t,
                                                  int block_in_token, SendLds& lds, int32_t* lds_hist) {
     const int lane = lane_id(), tid = threadIdx.x;
     const int num_topk = a.num_topk, num_experts = a.num_experts;
+    const int waves_per_token = a.pieces_per_row << a.split_log2;
     const int n = a.num_tokens * num_topk;
     const int src_rank = a.src_ranks != nullptr ? a.src_ranks[b] : a.rank;
     const int64_t* my_topk = a.topk_idx + int64_t(b) * n;
 
-    const int item = block_in_token * (block_threads() >> 6) + wave_in_block();
+    int item = block_in_token * (block_threads() >> 6) + wave_in_block(), token = 0;  // of the workgroup's, this wave's
+    if constexpr (kMany)
+        while (item >= waves_per_token && token + 1 < a.tokens_per_block) item -= waves_per_token, ++token;
     const int split = 1 << a.split_log2;
-    const bool wave_live = item < (a.pieces_per_row << a.split_log2);
+    const bool wave_live = item < waves_per_token && t + token < a.num_tokens;
     const int part = item & (split - 1);
     const int piece = item >> a.split_log2;
-    const int64_t row_id = int64_t(b) * a.num_tokens + t;
+    const int64_t row_id = int64_t(b) * a.num_tokens + (wave_live ? t + token : t);
     const int entry0 = t * num_topk;
+    const int selections = kMany ? min(a.tokens_per_block * num_topk, n - entry0) : num_topk;
 
     const int64_t data_bytes = row_data_bytes(a.hidden, kFmt);
     const int64_t data_pad = align16(data_bytes);
@@ -340,7 +360,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     const bool prefix_in_block = kTables && a.prefix_in_block;
     const int sweep_end = prefix_in_block ? n : entry0;
     constexpr int kSweepAhead = 2;
-    const int64_t own_v = my_topk[entry0 + (tid < num_topk ? tid : num_topk - 1)];  // threads 0..K-1: selection tid
+    const int64_t own_v = my_topk[entry0 + (tid < selections ? tid : selections - 1)];  // thread i: selection i
     const auto list = entry_list(my_topk, n);
     const int sweep_pairs = (sweep_end + 1) >> 1;
     EntryPair ahead[kSweepAhead];
@@ -350,9 +370,9 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     lds_barrier();
 
     // ---- per-selection bookkeeping, once per token --------------------------
-    int my_expert = -1, my_slot = -1, dst_rank = -1, local = 0;  // threads 0..K-1: selection k = tid
+    int my_expert = -1, my_slot = -1, dst_rank = -1, local = 0;  // thread i: selection i
     int direct_begin = 0;
-    if (tid < num_topk) {
+    if (tid < selections) {
         const int64_t v = own_v;
         if (v >= 0 && v < num_experts) {
             my_expert = int(v);
@@ -367,19 +387,30 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
         // Rows for this rank's own experts go straight to the packed tensors, at the place the
         // reference's range builder gives them: behind the rows of the lower source ranks
         // (csrc/kernels/efa_kernels.cu:991-1010).  For each such selection wave 0 adds up those
-        // ranks' counts of the expert.
+        // ranks' counts of the expert, kOwn of them at a time where there are several tokens'.
+        constexpr int kOwn = kMany ? 4 : 1;
         uint64_t to_own = __ballot(my_expert >= 0 && dst_rank == a.rank);
         while (to_own != 0) {
-            const int k = __builtin_ctzll(to_own);
-            to_own &= to_own - 1;
-            const int le = __builtin_amdgcn_readlane(local, k);
-            int part = 0;
-            for (int s = lane; s < a.rank; s += kWave) {
-                const int c = a.recv_count[le * a.num_ranks + s];
-                part += c < 0 ? 0 : (c > a.max_tokens ? a.max_tokens : c);
+            int k[kOwn], counts_at[kOwn], part[kOwn];
+#pragma unroll
+            for (int u = 0; u < kOwn; ++u) {
+                k[u] = to_own != 0 ? __builtin_ctzll(to_own) : (u > 0 ? k[u - 1] : 0);  // again the one before
+                to_own &= to_own - 1;
+                counts_at[u] = __builtin_amdgcn_readlane(local, k[u]) * a.num_ranks;
+                part[u] = 0;
             }
-            const int sum = __builtin_amdgcn_readlane(wave_inclusive_sum(part), kWave - 1);
-            if (lane == k) direct_begin = sum;
+            for (int s = lane; s < a.rank; s += kWave) {
+                int c[kOwn];
+#pragma unroll
+                for (int u = 0; u < kOwn; ++u) c[u] = a.recv_count[counts_at[u] + s];
+#pragma unroll
+                for (int u = 0; u < kOwn; ++u) part[u] += c[u] < 0 ? 0 : (c[u] > a.max_tokens ? a.max_tokens : c[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < kOwn; ++u) {
+                const int sum = __builtin_amdgcn_readlane(wave_inclusive_sum(part[u]), kWave - 1);
+                if (lane == k[u]) direct_begin = sum;
+            }
         }
     }
     DEEPEP_PHASE(1);
@@ -419,13 +450,23 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
             total = int(uint32_t(total) >> 16);
             dest_first = wave_expert_prefix(lds_hist, num_experts, a.max_tokens, my_expert);
         }
-        for (int k2 = 0; k2 < num_topk; ++k2) {  // the same expert named earlier in this token
-            const int other = __builtin_amdgcn_readlane(my_expert, k2);
-            if (k2 < tid && other == my_expert) total += 1;
+        if constexpr (kMany) {  // the same expert named earlier in these tokens
+            uint64_t same = __ballot(my_expert >= 0);
+            for (int bit = 1; bit < num_experts; bit <<= 1) {
+                const uint64_t votes = __ballot((my_expert & bit) != 0);
+                same &= (my_expert & bit) != 0 ? votes : ~votes;
+            }
+            total += __popcll(same & lanes_below(lane));
+        } else {
+            for (int k2 = 0; k2 < num_topk; ++k2) {  // the same expert named earlier in this token
+                const int other = __builtin_amdgcn_readlane(my_expert, k2);
+                if (k2 < tid && other == my_expert) total += 1;
+            }
         }
-        if (tid < num_topk && my_expert >= 0) my_slot = total;
+        if (tid < selections && my_expert >= 0) my_slot = total;
     }
-    if (tid < num_topk) {
+    if (tid < selections) {
+        const int of_token = kMany ? a.token_of(tid) : 0;
         if (my_slot >= a.max_tokens) my_slot = -1;
         uint8_t* row = nullptr;
         uint8_t* scale_row = nullptr;
@@ -438,7 +479,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
                 const int64_t out_row = int64_t(local) * a.num_ranks * a.max_tokens + direct_begin + my_slot;
                 row = direct.packed_x + out_row * data_bytes;
                 scale_row = direct.packed_scales + out_row * scale_bytes;
-                if (block_in_token == 0) direct.src_info[out_row] = t;
+                if (block_in_token == 0) direct.src_info[out_row] = t + of_token;
             } else if (dst_rank == a.rank) {
                 row = a.recv_staging + ((int64_t(local) * a.num_ranks + src_rank) * a.max_tokens + my_slot) * stride;
                 staged = true;
@@ -453,7 +494,7 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
         if (block_in_token == 0) {
             if (a.pair_slot != nullptr) a.pair_slot[entry0 + tid] = my_slot;
             if (staged) {
-                u32x4 tail = {uint32_t(t), uint32_t(tid), uint32_t(src_rank), uint32_t(local)};
+                u32x4 tail = {uint32_t(t + of_token), uint32_t(tid - of_token * num_topk), uint32_t(src_rank), uint32_t(local)};
                 *reinterpret_cast<u32x4*>(row + data_pad + scale_pad) = tail;
             }
         }
@@ -471,20 +512,20 @@ __device__ __forceinline__ void send_token_block(const SendArgs& a, const Direct
     // lane k reads selection k's destinations once
     uint64_t my_row = 0, my_scale_row = 0;
     if (lane < num_topk) {
-        my_row = lds.sel_row[lane];
-        my_scale_row = lds.sel_scale[lane];
+        my_row = lds.sel_row[token * num_topk + lane];
+        my_scale_row = lds.sel_scale[token * num_topk + lane];
     }
     store_selections<kFmt, kStream>(my_row, my_scale_row, num_topk, part, split, int(data_bytes), int(scale_bytes), lane_off,
                                     payload, scale_off, scale_bits);
     DEEPEP_PHASE(6);
 }
 
-template <int kFmt, bool kStream>
+template <int kFmt, bool kStream, bool kMany>
 __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_send_kernel(SendArgs a) {
     extern __shared__ int32_t lds_hist[];  // [E + 1]
     __shared__ SendLds lds;
     __shared__ int32_t wave_totals[kMaxBlockWaves];
-    if (int(blockIdx.y) == a.num_tokens) {  // the counting row of the grid
+    if (blockIdx.y + 1 == gridDim.y) {  // the counting row of the grid
         if (blockIdx.x != 0) return;
         if (a.prefix_in_block) {  // this workgroup writes the tables out
             expert_prefix_in_lds(a.topk_idx, a.num_tokens * a.num_topk, a.num_experts, a.max_tokens, lds_hist, wave_totals,
@@ -495,8 +536,8 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_send_kernel(SendArgs 
         }
         return;
     }
-    send_token_block<kFmt, kStream, true>(a, DirectOut{nullptr, nullptr, nullptr}, blockIdx.z, blockIdx.y, blockIdx.x, lds,
-                                          lds_hist);
+    send_token_block<kFmt, kStream, true, kMany>(a, DirectOut{nullptr, nullptr, nullptr}, blockIdx.z,
+                                                 int(blockIdx.y) * (kMany ? a.tokens_per_block : 1), blockIdx.x, lds, lds_hist);
 }
 
 // ---------------------------------------------------------------------
@@ -1070,7 +1111,7 @@ __global__ __launch_bounds__(256) void ll_recv_kernel(RecvArgs a, const int64_t*
 // (The reference's dispatch is one kernel with a send and a receive phase as
 // well: csrc/kernels/coop_dispatch_send.cuh:304, coop_dispatch_recv.cuh:42.)
 // ---------------------------------------------------------------------
-template <int kFmt, bool kStream>
+template <int kFmt, bool kStream, bool kMany>
 __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_dispatch_fused_kernel(SendArgs sa, RecvArgs ra, int blocks_per_token,
                                                                                  int num_send_blocks) {
     extern __shared__ int32_t dyn_lds[];  // counting: [E]; receive: [segments + 1 + E_l]
@@ -1079,8 +1120,11 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave) void ll_dispatch_fused_kernel
     const int block = blockIdx.x;
     if (block < num_send_blocks) {
         const DirectOut direct = {ra.packed_x, ra.packed_scales, ra.src_info};
-        send_token_block<kFmt, kStream, false>(sa, direct, 0, block / blocks_per_token, block % blocks_per_token, lds,
-                                               dyn_lds);
+        if constexpr (kMany)
+            send_token_block<kFmt, kStream, false, true>(sa, direct, 0, block * sa.tokens_per_block, 0, lds, dyn_lds);
+        else
+            send_token_block<kFmt, kStream, false, false>(sa, direct, 0, block / blocks_per_token, block % blocks_per_token,
+                                                          lds, dyn_lds);
     } else if (block == num_send_blocks) {
         send_count_block(sa, 0, dyn_lds);
     } else {
@@ -1199,9 +1243,15 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     // Every workgroup of the single launch goes through the batch's entries, the send ones for their slots and the
     // receive ones for the own counts: from some 1500 entries on the eighth wave that a 7168-wide row has no piece
     // for is worth its place (256 tokens, top-8 15.9 -> 15.1 us, 1024 tokens 40.9 -> 39.6; 128 tokens 8.0 -> 8.1).
-    // Workgroups of four waves stay: with eight, 509 tokens of hidden 4096 took 19.1 us instead of 17.0.
     if (fused_recv != nullptr && n > 1536 && waves > 4) waves = 8;
     if (fused_recv != nullptr && waves < 4) waves = 4;  // the receive workgroups want a few waves each
+    int tokens_per_block = 1;
+    if (!ranked && blocks_per_token == 1 && (fused_recv == nullptr || items <= 2))
+        while (tokens_per_block < 4 && 2 * tokens_per_block * items <= max_waves &&
+               2 * tokens_per_block * num_topk <= kWave && num_tokens >= 2 * tokens_per_block * kManyBlocks)
+            tokens_per_block *= 2;
+    const int token_blocks = (num_tokens + tokens_per_block - 1) / tokens_per_block;
+    if (tokens_per_block > 1) waves = std::max(waves, items * tokens_per_block);
     // floor(e / E_l) == umulhi(e, ceil(2^32 / E_l)) for every e below 2^16.
     const uint32_t experts_per_rank = uint32_t(num_experts / num_ranks);
     const uint32_t magic =
@@ -1214,6 +1264,7 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     sa.num_tokens = num_tokens, sa.hidden = hidden, sa.num_topk = num_topk, sa.num_experts = num_experts;
     sa.num_ranks = num_ranks, sa.rank = rank, sa.max_tokens = max_tokens;
     sa.pieces_per_row = pieces, sa.split_log2 = split_log2;
+    sa.tokens_per_block = tokens_per_block, sa.token_of = make_rank_divider(num_topk);
     sa.rank_of_expert_magic = magic;
     sa.recv_staging = reinterpret_cast<uint8_t*>(recv_staging);
     sa.send_slots = reinterpret_cast<uint8_t*>(send_slots);
@@ -1229,9 +1280,10 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
 
     if (fused_recv != nullptr) {  // single launch: send workgroups, the counting workgroup, receive workgroups
         EP_HOST_ASSERT(num_src == 1 && src_ranks == nullptr);
-        const int num_send_blocks = blocks_per_token * num_tokens;
+        const int num_send_blocks = blocks_per_token * token_blocks;
         int64_t fused_recv_blocks = (fused_recv_wave_items + waves - 1) / waves;
-        fused_recv_blocks = fused_recv_blocks < 1 ? 1 : (fused_recv_blocks > 1024 ? 1024 : fused_recv_blocks);
+        const int64_t most = tokens_per_block > 1 ? 512 : 1024;
+        fused_recv_blocks = fused_recv_blocks < 1 ? 1 : (fused_recv_blocks > most ? most : fused_recv_blocks);
         const int64_t total = int64_t(num_send_blocks) + 1 + fused_recv_blocks + 1;  // + counting, + metadata
         EP_HOST_ASSERT(total < (int64_t(1) << 31));
         const int num_segments = fused_recv->num_local_experts * fused_recv->num_ranks;
@@ -1247,12 +1299,18 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         const int64_t fused_traffic = int64_t(num_tokens) * (int64_t(hidden) * 2 + int64_t(num_topk) * payload) +
                                       2 * (fused_recv_wave_items >> ra.parts_log2) * payload;
         const bool fused_streams = fused_traffic > send_stream_bytes();
-#define DEEPEP_LAUNCH_FUSED(FMT)                                                                        \
-    do {                                                                                                \
-        if (fused_streams)                                                                              \
-            launch(ll_dispatch_fused_kernel<FMT, true>, dim3(unsigned(total)), waves * kWave, lds, stream, sa, ra, blocks_per_token, num_send_blocks); \
-        else                                                                                            \
-            launch(ll_dispatch_fused_kernel<FMT, false>, dim3(unsigned(total)), waves * kWave, lds, stream, sa, ra, blocks_per_token, num_send_blocks); \
+#define DEEPEP_LAUNCH_FUSED_AS(FMT, STREAM, MANY)                                                                    \
+    launch(ll_dispatch_fused_kernel<FMT, STREAM, MANY>, dim3(unsigned(total)), waves * kWave, lds, stream, sa, ra,    \
+           blocks_per_token, num_send_blocks)
+#define DEEPEP_LAUNCH_FUSED(FMT)                                                                                     \
+    do {                                                                                                             \
+        if (tokens_per_block > 1) {                                                                                  \
+            if (fused_streams) DEEPEP_LAUNCH_FUSED_AS(FMT, true, true);                                              \
+            else DEEPEP_LAUNCH_FUSED_AS(FMT, false, true);                                                           \
+        } else {                                                                                                     \
+            if (fused_streams) DEEPEP_LAUNCH_FUSED_AS(FMT, true, false);                                             \
+            else DEEPEP_LAUNCH_FUSED_AS(FMT, false, false);                                                          \
+        }                                                                                                            \
     } while (0)
         switch (row_format) {
             case kRowBF16: DEEPEP_LAUNCH_FUSED(kRowBF16); break;
@@ -1261,6 +1319,7 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
             default: DEEPEP_LAUNCH_FUSED(kRowFP8UE8M0); break;
         }
 #undef DEEPEP_LAUNCH_FUSED
+#undef DEEPEP_LAUNCH_FUSED_AS
         EP_LAUNCH_CHECK();
         return 0;
     }
@@ -1281,7 +1340,7 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
                             (int64_t(hidden) * 2 + int64_t(num_topk) * row_payload_bytes(hidden, row_format));
     const bool streams = traffic > send_stream_bytes();
     // + the index rows, + the counting row (ll_rank_finish_kernel has the counts)
-    const dim3 grid(blocks_per_token, index_rows + num_tokens + (ranked && batch.in_full ? 0 : 1), num_src);
+    const dim3 grid(blocks_per_token, index_rows + token_blocks + (ranked && batch.in_full ? 0 : 1), num_src);
     if (grid.y == 0) return 0;
     const size_t lds = size_t(index_rows > 0 ? 2 * (num_experts + 1) : num_experts + 1) * sizeof(int32_t);
     int topk_log2 = 0;
@@ -1291,8 +1350,10 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         if (ranked)                                                                                                    \
             launch(ll_send_ranked_kernel<FMT, STREAM>, grid, waves * kWave, lds, stream, sa, direct, batch, index,         \
                                                                                      index_rows, topk_log2);           \
+        else if (tokens_per_block > 1)                                                                                 \
+            launch(ll_send_kernel<FMT, STREAM, true>, grid, waves * kWave, lds, stream, sa);                           \
         else                                                                                                           \
-            launch(ll_send_kernel<FMT, STREAM>, grid, waves * kWave, lds, stream, sa);                                     \
+            launch(ll_send_kernel<FMT, STREAM, false>, grid, waves * kWave, lds, stream, sa);                          \
     } while (0)
 #define DEEPEP_LAUNCH_SEND(FMT)                            \
     do {                                                   \

@@ -1168,6 +1168,31 @@ def test_send_by_dest(rt, fmt, r, rank, t, h, k, e):
     check_send_by_dest(st, O.ll_send_by_dest(x_all[rank], topk_all[rank], rank, e, t, fmt, r), t)
 
 
+@pytest.mark.parametrize("t,k,h,fmt", [
+    (479, 8, 2048, O.ROW_FP8), (480, 8, 2048, O.ROW_FP8),  # one token a workgroup, two
+    (481, 16, 512, O.ROW_FP8_POW2), (511, 8, 4096, O.ROW_FP8_UE8M0),
+    (959, 8, 1024, O.ROW_BF16), (960, 8, 1024, O.ROW_BF16),  # two, four
+    (963, 5, 640, O.ROW_FP8), (1021, 7, 2048, O.ROW_FP8), (1024, 8, 512, O.ROW_FP8), (1024, 8, 4096, O.ROW_FP8)])
+def test_several_tokens_a_workgroup(rt, t, k, h, fmt):
+    """From 480 tokens on a workgroup that ranks its own slots has two or four of them: experts that its tokens share,
+    or one names twice, hot ones past a segment's room, entries that name none, and a last workgroup that is not full;
+    by destination and in the single-launch dispatch."""
+    r, rank, e, m = 4, 2, 20, t
+    g = torch.Generator().manual_seed(t * k)
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + k, drop=0)
+    topk_all[:] = torch.randint(0, e, topk_all.shape, generator=g)
+    topk_all[torch.rand(topk_all.shape, generator=g) < 0.2] = 11  # the rank's own, and more often than it has slots
+    topk_all[torch.rand(topk_all.shape, generator=g) < 0.05] = -1
+    topk_all[rank, 3, 0], topk_all[rank, t - 1, k - 1] = e, (1 << 32) + 1
+    live = (topk_all >= 0) & (topk_all < e)
+    topk = torch.where(live, topk_all, -1)  # the same to the oracle
+    st = send_by_dest_on_gpu(rt, x_all[rank], topk_all[rank], rank, r, e, m, fmt)
+    check_send_by_dest(st, O.ll_send_by_dest(x_all[rank], topk[rank], rank, e, m, fmt, r), t)
+    got, _ = dispatch_on_gpu(rt, x_all, topk_all, rank, e, m, fmt, one_call=True)
+    check_dispatch(got, O.ll_dispatch(list(x_all), list(topk), rank, e, m, fmt), fmt)
+    assert torch.equal(got.pair_slot.cpu().view(-1)[:t * k], st.pair_slot.cpu().view(-1)[:t * k])
+
+
 @pytest.mark.parametrize("receive", ["from_tails", "ordered"])
 def test_all_to_all_with_an_empty_batch(rt, receive):
     """No token anywhere: the tables are zeros, nothing is received, the records stay untouched, and the reduce of
