@@ -252,6 +252,36 @@ def test_exchange_metadata(rt, r, e, m, k, rank, capacity):
             assert torch.equal(out[key][:n], got[key][:n]), key
 
 
+@pytest.mark.parametrize("r,e,rank,capacity", [(1, 1, 0, 8), (1, 7, 0, 0), (3, 9, 2, 300), (2, 10, 1, 40), (5, 255, 4, 2100),
+                                               (7, 259, 3, 2049), (32, 256, 31, 4096), (4, 2048, 3, 70000),
+                                               (64, 1024, 1, 300000), (300, 300, 299, 500), (1024, 1024, 700, 20000)])
+def test_exchange_metadata_of_every_count(rt, r, e, rank, capacity):
+    """Lists of counts that end within a vector, pass a workgroup's loads, or name more experts than it has threads:
+    every count is added up, and one too large anywhere is seen."""
+    g = torch.Generator().manual_seed(r * 1000 + e)
+    m = 9
+    routed = torch.randint(0, m + 1, (r, e), generator=g, dtype=torch.int32)
+    routed[torch.rand((r, e), generator=g) > 8 * r / e] = 0  # no more in all than is possible
+    spots = [None, (0, 0), (r - 1, e - 1), (r // 2, e // 2), (r - 1, max(0, e - 2))]
+    for spot in spots:
+        mat = routed.clone()
+        if spot is not None:
+            mat[spot] = m + 1 if spot != (0, 0) else -5  # -5: 2^32 - 5 as the count that it is read as
+        want = O.ll_exchange_metadata(mat, rank, m)
+        out = rt.ll.exchange_metadata(mat.cuda(), rank, m, capacity)
+        torch.cuda.synchronize()
+        assert out["totals"].cpu().tolist() == [want["total_send"], want["total_recv"], int(spot is not None)]
+        assert out["send_counts"].cpu().tolist() == want["send_counts"].tolist()
+        assert out["recv_counts"].cpu().tolist() == want["recv_counts"].tolist()
+        first = rank * (e // r)
+        assert out["combine_remote_recv_offset"].cpu().tolist() == (mat[:, :first].long() & 0xffffffff).sum(1).tolist()
+        n = min(want["total_recv"], capacity)
+        assert out["num_recv_tokens"].cpu().tolist() == [want["total_recv"], n]
+        assert (out["tokens_per_expert"] == 0).all()
+        for key in ("source_rank", "source_offset", "padded_index", "combine_send_offset"):
+            assert out[key][:n].cpu().tolist() == want[key][:n].tolist(), key
+
+
 def test_exchange_metadata_hand_derived_world(rt):
     g, _, _ = load_tiny_world()
     routed = torch.tensor(g["all_num_routed"], dtype=torch.int32)
