@@ -10,14 +10,16 @@ namespace deepep {
 constexpr int kLayoutThreads = 256;
 constexpr int kMaxRankWords = 4;  // membership bitmask: up to 256 ranks
 constexpr int kLayoutOneBlockThreads = 1024;
-// Up to here one workgroup counts everything and no second launch adds up partial rows: a token a thread, and half of
-// that past 32 ranks, whose ballots it takes one after another.  Microseconds of the one launch against the two:
+// Up to here one workgroup counts everything and no second launch adds up partial rows: one or two tokens a thread.
+// Microseconds of the one launch against the two, in a row (the second also takes the host 2.3):
 //   ranks        8            16           32            64
-//   400 tokens   3.2 / 4.6    3.7 / 5.1    4.6 / 5.9     6.9 / 7.7
-//   600          3.7 / 4.6    4.4 / 5.3    5.4 / 6.1     8.0 / 7.7
-//   1024         4.5 / 4.7    5.2 / 5.1    6.8 / 6.1    10.6 / 7.8    (the second launch takes the host 2 more)
-//   2048         6.7 / 4.8    7.6 / 5.4   10.5 / 6.2    17.8 / 8.1
-inline int layout_one_block_tokens(int num_ranks) { return num_ranks <= 32 ? 1024 : 512; }
+//   400 tokens   2.9 / 4.1    3.3 / 4.4    3.8 / 4.8     4.8 / 5.4
+//   700          3.0 / 4.1    3.4 / 4.4    3.9 / 4.8     4.8 / 5.5
+//   1024         3.3 / 4.3    3.7 / 4.5    4.2 / 4.8     5.9 / 5.5
+//   1500         4.3 / 4.3    5.0 / 4.6    6.0 / 4.9    10.3 / 5.5
+//   2048         4.4 / 4.5    5.3 / 4.8    6.4 / 5.1    11.4 / 5.9
+//   3000         5.6 / 4.7    6.8 / 4.9    8.5 / 5.2    16.6 / 6.0
+inline int layout_one_block_tokens(int num_ranks) { return num_ranks <= 8 ? 2048 : num_ranks <= 32 ? 1024 : 768; }
 
 // Spreads the 8 bits of b into 8 bytes (byte i = bit i, value 0 or 1).
 __device__ __forceinline__ uint64_t bits_to_bool_bytes(uint32_t b) {
@@ -25,18 +27,35 @@ __device__ __forceinline__ uint64_t bits_to_bool_bytes(uint32_t b) {
     return ((x + 0x7f7f7f7f7f7f7f7full) >> 7) & 0x0101010101010101ull;
 }
 
+// 1 in every byte of v that is not zero.
+__device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {
+    v |= v >> 4, v |= v >> 2, v |= v >> 1;
+    return v & 0x0101010101010101ull;
+}
+
+// Sums over the wave of the eight bytes of v, which are 0 or 1, in its lanes first to first + 7: lane first + i gets byte i's;
+// the others get what they hand in.  Four bytes are added up by one sum over the lanes, no byte past 64.
+__device__ __forceinline__ int byte_sums_to_lanes(uint64_t v, int first, int otherwise) {
+    const uint32_t lo = __builtin_amdgcn_readlane(wave_inclusive_sum(int(uint32_t(v))), kWave - 1);
+    const uint32_t hi = __builtin_amdgcn_readlane(wave_inclusive_sum(int(uint32_t(v >> 32))), kWave - 1);
+    const int i = lane_id() - first;
+    return i >= 0 && i < 8 ? int((((i & 4) != 0 ? hi : lo) >> ((i & 3) * 8)) & 0xff) : otherwise;
+}
+
 // ---------------------------------------------------------------------
 // get_dispatch_layout: one pass over topk_idx, one token per lane.
 //   * per-expert pair counts: LDS histogram (integer adds — the result does
 //     not depend on their order);
 //   * per-rank and per-node distinct-token counts: each lane folds its K
-//     selections into a rank bitmask, then one 64-lane ballot + popcount per
-//     rank gives the wave's count;
-//   * is_token_in_rank: the bitmask expanded to bool bytes, 8 per store.
+//     selections into a rank bitmask, whose bits, spread to bytes, are added up
+//     over the wave, four ranks at a time (a ballot and a popcount for each
+//     rank: 64 tokens to 32 ranks 4.4 us, 1000 6.9);
+//   * is_token_in_rank: the same bytes, 8 per store.
 // Each workgroup writes a partial row [E | R | R/8]; with one workgroup the
 // partial row is the result, otherwise a second small kernel adds the rows.
-// What bounds it is latency and launches, not the few hundred KB it reads: hence
-// one workgroup while that costs less than the second launch, and a bitmask of
+// What bounds it is latency, launches and, in one workgroup, instructions, not the
+// few hundred KB it reads: hence one workgroup while that costs less than the
+// second launch, and a bitmask of
 // as many words as there are ranks for (an index into a longer one that the
 // compiler cannot resolve goes through selects).
 // Reference: csrc/kernels/layout.cu:9-121 (which re-reads topk_idx once per
@@ -53,55 +72,52 @@ __global__ __launch_bounds__(kLayoutOneBlockThreads) void layout_count_kernel(
     for (int j = tid; j < width; j += threads) hist[j] = 0;
     lds_barrier();
 
-    // whole waves go round together: the ballots below want every lane
+    // whole waves go round together: the sums below want every lane
     for (int t0 = blockIdx.x * threads; t0 < num_tokens; t0 += int(gridDim.x) * threads) {
         const int t = t0 + tid;
         uint64_t member[kRankWords];
 #pragma unroll
         for (int q = 0; q < kRankWords; ++q) member[q] = 0;
-        if (t < num_tokens) {
-            const int64_t* row = topk_idx + int64_t(t) * num_topk;
-            for (int k0 = 0; k0 < num_topk; k0 += 8) {
-                int64_t e[8];  // the eight loads of a round in flight before the first is used
+        // The round's rows as one buffer: 16-byte loads, two entries each, that need no more than four-byte alignment, and
+        // zeros past the last token.  (Entries one at a time: 1000 tokens 4.1 us, a line of cache a lane and load.)
+        const int tokens = num_tokens - t0 < threads ? num_tokens - t0 : threads;
+        const auto rows = row_buffer(reinterpret_cast<const uint8_t*>(topk_idx + int64_t(t0) * num_topk), tokens * num_topk * 8);
+        for (int k0 = 0; k0 < num_topk; k0 += 8) {
+            u32x4 two[4];  // all in flight before the first is used
 #pragma unroll
-                for (int u = 0; u < 8; ++u) e[u] = k0 + u < num_topk ? row[k0 + u] : -1;
+            for (int u = 0; u < 4; ++u) two[u] = load_row_u32x4<false>(rows, (tid * num_topk + k0 + 2 * u) * 8);
 #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    if (e[u] < 0 || e[u] >= num_experts) continue;
-                    atomicAdd(&hist[int(e[u])], 1);
-                    // e / E_l by multiply-high (exact below 2^16 experts); magic 0 stands for E_l == 1
-                    const int r = rank_magic != 0 ? int(__umulhi(uint32_t(e[u]), rank_magic)) : int(e[u]);
+            for (int u = 0; u < 8; ++u) {
+                const uint32_t e = two[u / 2][u % 2 * 2];
+                if (two[u / 2][u % 2 * 2 + 1] != 0u || e >= uint32_t(num_experts) || k0 + u >= num_topk || t >= num_tokens) continue;
+                atomicAdd(&hist[e], 1);
+                // e / E_l by multiply-high (exact below 2^16 experts); magic 0 stands for E_l == 1
+                const int r = rank_magic != 0 ? int(__umulhi(e, rank_magic)) : int(e);
 #pragma unroll
-                    for (int q = 0; q < kRankWords; ++q)
-                        if (kRankWords == 1 || (r >> 6) == q) member[q] |= uint64_t(1) << (r & 63);
-                }
-            }
-            uint8_t* out = is_token_in_rank + int64_t(t) * num_ranks;
-#pragma unroll
-            for (int q = 0; q < kRankWords; ++q) {
-                const int begin = q * kWave, end = num_ranks < begin + kWave ? num_ranks : begin + kWave;
-                if ((num_ranks & 7) == 0) {
-                    for (int r8 = begin; r8 < end; r8 += 8)
-                        *reinterpret_cast<uint64_t*>(out + r8) = bits_to_bool_bytes(uint32_t(member[q] >> (r8 - begin)));
-                } else {
-                    for (int r = begin; r < end; ++r) out[r] = uint8_t((member[q] >> (r - begin)) & 1);
-                }
+                for (int q = 0; q < kRankWords; ++q)
+                    if (kRankWords == 1 || (r >> 6) == q) member[q] |= uint64_t(1) << (r & 63);
             }
         }
         // lane r keeps rank (q * 64 + r)'s count of the wave, so that one atomic per lane adds them all
+        uint8_t* out = is_token_in_rank + int64_t(t) * num_ranks;
 #pragma unroll
         for (int q = 0; q < kRankWords; ++q) {
-            const int begin = q * kWave, n = num_ranks - begin < kWave ? num_ranks - begin : kWave;
+            const int begin = q * kWave, end = num_ranks < begin + kWave ? num_ranks : begin + kWave;
             int count = 0;
-            for (int r = 0; r < n; ++r) {
-                const int votes = __popcll(__ballot((member[q] >> r) & 1));
-                if (lane == r) count = votes;
+            for (int r8 = begin; r8 < end; r8 += 8) {
+                const uint64_t in = bits_to_bool_bytes(uint32_t(member[q] >> (r8 - begin)));
+                count = byte_sums_to_lanes(in, r8 - begin, count);
+                if (t >= num_tokens) continue;
+                if ((num_ranks & 7) == 0) {
+                    *reinterpret_cast<uint64_t*>(out + r8) = in;
+                } else {
+                    for (int i = 0; i < 8 && r8 + i < end; ++i) out[r8 + i] = uint8_t(in >> (8 * i));
+                }
             }
             if (count != 0) atomicAdd(&hist[num_experts + begin + lane], count);
-            // 8 ranks per node (reference: NUM_MAX_NVL_PEERS, csrc/kernels/configs.cuh:3)
-            for (int nd = 0; nd < 8 && q * 8 + nd < num_nodes; ++nd) {
-                const int votes = __popcll(__ballot((member[q] >> (nd * 8)) & 0xffull));
-                if (lane == 0 && votes != 0) atomicAdd(&hist[num_experts + num_ranks + q * 8 + nd], votes);
+            if (q * 8 < num_nodes) {  // 8 ranks per node (reference: NUM_MAX_NVL_PEERS, csrc/kernels/configs.cuh:3)
+                const int in_node = byte_sums_to_lanes(nonzero_bytes(member[q]), 0, 0);
+                if (in_node != 0) atomicAdd(&hist[num_experts + num_ranks + q * 8 + lane], in_node);
             }
         }
     }
@@ -345,12 +361,6 @@ constexpr int kWideSortTokens = 256;  // tokens per workgroup
 constexpr int kWideSortThreads = 1024;
 constexpr int64_t kWideSortMaxBytes = 512 * 1024;
 
-// 1 in every byte of v that is not zero.
-__device__ __forceinline__ uint64_t nonzero_bytes(uint64_t v) {
-    v |= v >> 4, v |= v >> 2, v |= v >> 1;
-    return v & 0x0101010101010101ull;
-}
-
 // A token's row of kWords words out of the matrix as a buffer: zeros past its end.
 template <int kWords>
 __device__ __forceinline__ void load_member_words(__amdgpu_buffer_rsrc_t matrix, int t, uint64_t (&row)[kWords]) {
@@ -541,6 +551,41 @@ __global__ __launch_bounds__(1024) void channel_prefix_kernel(const uint8_t* __r
 // with one 8-byte load per token, up to sixteen of them in flight, and adds the bool bytes up eight at a time.  The
 // bytes of a row that eight workgroups used to fetch for themselves are fetched once; the sums of eight ranks are
 // eight times the work of one's.
+// Instructions bound it where channels are long: the bytes are taken for the 0 and 1 of a bool, which one test a channel
+// confirms (4096 tokens 3.8 -> 3.4 us, 12000 5.6 -> 4.5).
+template <int kAhead, bool kBool>
+__device__ __forceinline__ bool count_channel(const uint64_t* __restrict__ is_token_in_rank, int begin, int end, int q,
+                                              int num_words, int (&count)[8]) {
+    const int lane = lane_id();
+    uint64_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) count[i] = 0;
+    for (int t0 = begin + lane; t0 - lane < end; t0 += kWave * kAhead) {
+        uint64_t v[kAhead], sum = 0;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int t = t0 + u * kWave;
+            v[u] = is_token_in_rank[int64_t(t < end ? t : end - 1) * num_words + q];
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const uint64_t one = t0 + u * kWave < end ? (kBool ? v[u] : nonzero_bytes(v[u])) : 0;
+            sum += one;
+            if constexpr (kBool) bits |= one;
+        }
+#pragma unroll
+        for (int half = 0; half < 2; ++half)  // bytes widened to 16 bits: 64 lanes of at most 16 fit
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd) {
+                const int part = int((uint32_t(sum >> (32 * half)) >> (8 * odd)) & 0x00ff00ffu);
+                const uint32_t all = uint32_t(__builtin_amdgcn_readlane(wave_inclusive_sum(part), kWave - 1));
+                count[half * 4 + odd] += int(all & 0xffffu);
+                count[half * 4 + odd + 2] += int(all >> 16);
+            }
+    }
+    return __ballot((bits & 0xfefefefefefefefeull) != 0) == 0;
+}
+
 template <int kAhead>  // loads in flight per lane: 4 for channels of up to 256 tokens, else 16
 __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64_t* __restrict__ is_token_in_rank,
                                                                     int num_tokens, int num_words, int num_channels,
@@ -552,27 +597,8 @@ __global__ __launch_bounds__(1024) void channel_prefix_words_kernel(const uint64
     for (int ch = w; ch < num_channels; ch += waves) {
         const int begin = min(per * ch, num_tokens), end = min(begin + per, num_tokens);
         int count[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) count[i] = 0;
-        for (int t0 = begin + lane; t0 - lane < end; t0 += kWave * kAhead) {
-            uint64_t v[kAhead], sum = 0;
-#pragma unroll
-            for (int u = 0; u < kAhead; ++u) {
-                const int t = t0 + u * kWave;
-                v[u] = is_token_in_rank[int64_t(t < end ? t : end - 1) * num_words + q];
-            }
-#pragma unroll
-            for (int u = 0; u < kAhead; ++u) sum += t0 + u * kWave < end ? nonzero_bytes(v[u]) : 0;
-#pragma unroll
-            for (int half = 0; half < 2; ++half)  // bytes widened to 16 bits: 64 lanes of at most 16 fit
-#pragma unroll
-                for (int odd = 0; odd < 2; ++odd) {
-                    const int part = int((uint32_t(sum >> (32 * half)) >> (8 * odd)) & 0x00ff00ffu);
-                    const uint32_t all = uint32_t(__builtin_amdgcn_readlane(wave_inclusive_sum(part), kWave - 1));
-                    count[half * 4 + odd] += int(all & 0xffffu);
-                    count[half * 4 + odd + 2] += int(all >> 16);
-                }
-        }
+        if (!count_channel<kAhead, true>(is_token_in_rank, begin, end, q, num_words, count))
+            count_channel<kAhead, false>(is_token_in_rank, begin, end, q, num_words, count);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
             if (lane == i) per_channel[ch * 8 + i] = count[i];

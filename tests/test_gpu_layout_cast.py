@@ -181,6 +181,50 @@ def test_layout_and_channel_prefix_either_side_of_their_lines(t, r, e):
         assert torch.equal(normal.channel_prefix_matrix(is_in, c).cpu(), O.channel_prefix_matrix(want[3], c))
 
 
+@pytest.mark.parametrize("t,r,e,k", [(767, 64, 256, 6), (768, 64, 256, 6), (769, 64, 256, 6), (2048, 8, 64, 8), (2049, 8, 64, 8),
+                                     (1024, 32, 256, 8), (1025, 32, 256, 8), (70, 9, 18, 9), (65, 72, 144, 5), (300, 256, 512, 17),
+                                     (1030, 200, 400, 3), (63, 24, 24, 1)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_layout_counts_ranks_and_nodes(capi, t, r, e, k, shift):
+    """Counts of ranks and nodes added up as bytes, entries read in pairs at any eight-byte address: either side of the
+    one-workgroup lines, tokens of an odd number of entries, ranks that fill no byte or several masks, entries that name
+    no expert, a wave whose tokens all go to one rank."""
+    topk = _topk(t, k, e, seed=t + r + k, drop=7)
+    topk[t // 2, 0], topk[0, k - 1] = e, (1 << 32) + 1
+    topk[:min(t, 64), 0] = e // 2
+    lib = capi.load()
+    dev = torch.full((t * k + 2,), 3, dtype=torch.int64, device="cuda")
+    dev[shift:shift + t * k] = topk.view(-1).cuda()
+    nodes = r // 8 if r > 8 and r % 8 == 0 else 0
+    per_rank, per_node, per_expert = (torch.full((n,), -1, dtype=torch.int32, device="cuda") for n in (r, max(1, nodes), e))
+    is_in = torch.full((t + 1, r), 7, dtype=torch.uint8, device="cuda")
+    ws = torch.empty(lib.deepep_layout_workspace_bytes(t, r, e), dtype=torch.uint8, device="cuda")
+    capi.check(lib.deepep_get_dispatch_layout(
+        dev.data_ptr() + 8 * shift, t, k, r, e, capi.ptr(per_rank), capi.ptr(per_node) if nodes else None,
+        capi.ptr(per_expert), capi.ptr(is_in), capi.ptr(ws), ws.numel(), stream()))
+    torch.cuda.synchronize()
+    want = O.get_dispatch_layout(torch.where((topk >= 0) & (topk < e), topk, -1), e, r)
+    assert torch.equal(per_rank.cpu(), want[0]) and torch.equal(per_expert.cpu(), want[2])
+    assert not nodes or torch.equal(per_node.cpu(), want[1])
+    assert torch.equal(is_in[:t].cpu(), want[3].to(torch.uint8)) and (is_in[t] == 7).all()
+
+
+@pytest.mark.parametrize("t,r,c", [(300, 8, 1), (4096, 8, 10), (12001, 16, 7), (5000, 32, 33), (2048, 24, 4)])
+@pytest.mark.parametrize("values", ["bytes", "all"])
+def test_channel_prefix_of_any_bytes(capi, t, r, c, values):
+    """Any byte but zero is a member, in every form of the prefix."""
+    g = torch.Generator().manual_seed(t + r + c)
+    is_in = torch.ones((t, r), dtype=torch.bool) if values == "all" else torch.rand((t, r), generator=g) < 0.4
+    member = is_in.to(torch.uint8)
+    if values == "bytes":
+        member *= torch.tensor([1, 2, 64, 128, 255], dtype=torch.uint8)[torch.randint(5, (t, r), generator=g)]
+    dev = member.cuda()
+    cpm = torch.full((r, c), -1, dtype=torch.int32, device="cuda")
+    capi.check(capi.load().deepep_channel_prefix_matrix(capi.ptr(dev), t, r, c, capi.ptr(cpm), stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(cpm.cpu(), O.channel_prefix_matrix(is_in, c))
+
+
 # every form of the sort: one workgroup a rank, one per 256 tokens, count + scan + scatter; no tokens at all
 SORT_FORMS = [(0, 8), (0, 9), (0, 72), (1, 9), (300, 24), (131, 16), (5000, 16), (8192, 64), (40000, 8), (9000, 12),
               (70000, 8), (3000, 72), (1, 130)]
