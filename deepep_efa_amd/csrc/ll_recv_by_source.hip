@@ -466,14 +466,16 @@ __device__ __forceinline__ void ordered_recv_impl(const OrderedRecvArgs& a, int 
         const int j = row - seg_first;
         const uint8_t* from = a.rows + uint64_t(uint32_t(src * int(a.slot_rows) + in_message + j)) * stride;
         row_part_range(num_vec, a.parts_log2, part, v_begin, v_end);
-        // Stored the ordinary way, since the experts read the rows next.  Receive and a copy of its rows, ordinary stores / past
-        // the caches, on three sets of buffers in turn and behind a write of 512 MB: 128 tokens of hidden 7168 to 32 ranks (7 MB)
-        // 10.1 / 10.3 us and 12.9 / 14.1, 256 to 16 (15 MB) 14.7 / 16.3 and 20.5 / 23.0, 700 to 8 (41 MB) 35.6 / 38.7 and 43.5 /
-        // 50.8; 1000 of 4096 (33 MB) 31.8 / 34.1 and 38.9 / 42.7.  The receive alone 5.2 / 4.8, 8.2 / 8.1, 18.1 / 16.4, 14.8 / 14.5.
-        // A whole exchange whose experts hand the rows on 47.9 / 50.3, 76.8 / 82.6, 180.8 / 198.6 and 150.8 / 167.3, one whose experts
-        // read 512 MB first 58.4 / 58.1, 90.2 / 89.3, 206 / 205 and 177.8 / 176.0, and one without experts 27.8 / 26.9, 40.5 / 39.2,
-        // 89.7 / 84.4 and 75.8 / 71.1.
-        RowPart<kOrderedDepth, false, false> payload;
+        // Read past the caches, since nobody reads the staged rows again, and stored the ordinary way, since the experts read
+        // the rows next.  Microseconds of whole exchanges to 8 ranks on three sets of buffers in turn, rows read the ordinary way /
+        // past the caches -- as they are; behind a copy that puts the rows there, and in front of one that takes them on:
+        //   256 x 7168   39.9 / 39.6    67.6 / 65.4      1000 x 2048  45.7 / 44.9    75.4 / 73.4
+        //   512          63.7 / 63.0   106.7 / 105.3     1000 x 4096  73.3 / 67.4   115.3 / 114.7
+        //   800          95.1 / 90.9   150.3 / 149.2     128 to 32 ranks 26.7 / 26.4   45.8 / 45.3
+        // and behind 512 MB that were written or read in between 0 to 2.5 % less.
+        // The stores past the caches too: 700 x 7168 whose experts hand the rows on 180.8 / 198.6, 1000 x 4096 150.8 / 167.3, with
+        // experts that read 512 MB first 206 / 205 and 177.8 / 176.0, without experts 89.7 / 84.4 and 75.8 / 71.1 (ordinary loads).
+        RowPart<kOrderedDepth, true, false> payload;
         payload.load(from, v_begin, v_end, lane);
         const bool carries_tail = part == parts - 1;  // the last part is the shortest
         uint32_t tail_scale = 0;
@@ -630,13 +632,15 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
     return 0;
 }
 
-// Past 52 MB the flat copy gains more than the index's launch costs.  Microseconds of the five calls of an exchange, 8
-// ranks x 8 experts, one launch against two:
-//   3600 rows of 14 KB (50 MB)  84.2 / 85.3     4400 (60 MB)  96.8 / 95.2     5600  116.3 / 113.3     8000  153.5 / 146.4
-//   6800 rows of  7 KB (46 MB) 108.5 / 109.5    8000 (55 MB) 119.8 / 118.2    8800  129.8 / 126.8
-//   6400 rows of  8 KB (50 MB)  86.2 / 87.0     8000 (62 MB)  93.9 / 93.0
+// Past 52 MB, or 40 past 8192 rows, the flat copy gains more than the index's launch costs; and past 8192 rows of less than
+// 2 KB.  Microseconds of the five calls of an exchange, 8 ranks x 8 experts, one launch against two:
+//   6400 rows of  7 KB (45 MB)  91.3 / 94.7      8800 rows of  2 KB (18 MB) 48.7 / 50.1     16376 rows of 2 KB (33 MB) 72.0 / 73.0
+//   7200 (52 MB)               101.4 / 98.1      8800 rows of  4 KB (36 MB) 74.6 / 77.0     16376 rows of 1 KB         50.2 / 47.5
+//   4000 rows of 14 KB (57 MB)  79.4 / 75.8     10000 rows of  4 KB (41 MB) 84.3 / 85.2     16376 rows of 512 B        38.1 / 36.5
+//   5600 (80 MB)               101.7 / 99.6     12000 rows of  4 KB (49 MB)101.3 / 97.6
 static bool ordered_in_one_launch(int64_t rows, int64_t row_bytes) {
-    return rows <= kLargeBatchRows && rows * row_bytes <= (int64_t(52) << 20);
+    if (rows <= kLargeBatchRows) return rows * row_bytes <= (int64_t(52) << 20);
+    return rows <= 2 * kLargeBatchRows && row_bytes >= 2048 && rows * row_bytes <= (int64_t(40) << 20);
 }
 
 int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_t slot_rows,

@@ -2101,6 +2101,29 @@ def test_ordered_receive_in_one_launch_and_in_two(rt, fmt, h, hints):
         assert torch.equal(st.record_packed_row[:rec.numel()].cpu().long(), rec)
 
 
+@pytest.mark.parametrize("fmt,h,hints", [
+    (O.ROW_BF16, 2048, (8192, 8193, 10240, 10241)),  # 40 MB past 8192 rows
+    (O.ROW_FP8, 2048, (16384, 16385)), (O.ROW_FP8, 1920, (8192, 8193))])  # the last rows, and too narrow ones
+def test_ordered_receive_past_8192_rows(rt, fmt, h, hints):
+    """One launch or two past 8192 expected rows: the oracle's rows and records either way."""
+    r, rank, t, k, e = 4, 3, 33, 5, 24
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=h, drop=9)
+    states = [rt.ll.AllToAllState(rt.ll.LLShape(r, s, e, t, h, k, fmt)) for s in range(r)]
+    for s, st in enumerate(states):
+        st.dispatch_send(x_all[s].cuda(), topk_all[s].cuda())
+    torch.cuda.synchronize()
+    routed, st = all_to_all_dispatch(states, fmt), states[rank]
+    want, rec = O.ll_dispatch(list(x_all), list(topk_all), rank, e, t, fmt), O.ll_record_packed_rows(list(topk_all), rank, e, t)
+    for hint in hints:
+        poison_outputs_keep_pair_slot(st)
+        st.record_packed_row.fill_(-7)
+        st.expected_rows = hint
+        st.dispatch_recv_ordered(routed)
+        torch.cuda.synchronize()
+        check_dispatch(st, want, fmt)
+        assert torch.equal(st.record_packed_row[:rec.numel()].cpu().long(), rec)
+
+
 @pytest.mark.parametrize("h,hints", [
     (1024, (8192, 8193, 16400, 16401)),  # one launch, one that streams, the last before twice the selections, two launches
     (512, (12288, 12289)),  # rows below 2 KB: one launch, two
