@@ -106,7 +106,7 @@ __device__ __forceinline__ void emit_expert_count(int e, int total, int num_expe
 // ll_rank_chunk_kernel, one launch ahead.  Deterministic: integer adds only.
 // ---------------------------------------------------------------------
 constexpr int kMaxTopk = 64;
-constexpr int kFusedMaxEntries = 8192;     // send + receive in one launch up to here
+constexpr int kFusedMaxEntries = 8192;     // send + receive in one launch up to here, whatever the rows
 constexpr int kSendMaxWaves = 16;
 
 // A workgroup that ranks its own slots takes two or four tokens where it has waves for them, and one sweep through the
@@ -1099,7 +1099,7 @@ __global__ __launch_bounds__(256) void ll_recv_kernel(RecvArgs a, const int64_t*
 }
 
 // ---------------------------------------------------------------------
-// Single-launch dispatch for small batches (T*K <= 8192, at most 8192 expected rows): the send
+// Single-launch dispatch for small batches (dispatch_in_one_launch()): the send
 // workgroups, the counting workgroup and the receive workgroups of the two
 // kernels above in one grid.  No workgroup waits on another: the receive
 // workgroups copy only the peers' rows (already in the staging area when the
@@ -1171,6 +1171,43 @@ static int check_ll_shape(int num_tokens, int hidden, int num_topk, int num_expe
     return 0;
 }
 
+// Waves that a token's row takes.
+static int row_pieces(int hidden, int row_format) {
+    return row_format == kRowBF16 ? (hidden * 2 + 1023) / 1024 : (hidden / kGroup + 7) / 8;
+}
+
+// Tokens of a workgroup that ranks its own slots, of `items` waves each (kManyBlocks says why).
+static int tokens_per_send_block(int items, int max_waves, int num_topk, int num_tokens) {
+    int tokens = 1;
+    while (tokens < 4 && 2 * tokens * items <= max_waves && 2 * tokens * num_topk <= kWave &&
+           num_tokens >= 2 * tokens * kManyBlocks)
+        tokens *= 2;
+    return tokens;
+}
+
+constexpr int kFusedMaxWaves = 8, kFusedManyPieces = 2;
+
+// Whether a one-call dispatch runs as one launch: up to 8192 entries and rows always.  Past them it saves a launch or two
+// (4 to 8 us) and pays with its workgroups' sweeps through the entries, fewer of them where a workgroup has several
+// tokens, and with copying waves that go round for more rows, which falls behind the flat copy once the rows are large in
+// all.  Microseconds of a step, top-8 unless said, fp8 unless said, three launches / one, by the millions of entries that
+// the send workgroups go through and the MB of rows expected:
+//   1100 x 2048   2.4   19   44.8 / 39.5     1100 x 2048 bf16   9.7   36   51.5 / 43.9     1100 x 7168  9.7   66  106.8 / 103.5
+//   2300 x 2048  10.6   39   73.3 / 66.3     2000 x 2048 bf16, top-6                       2000 x 4096  32    69  112.1 / 112.1
+//   3400 x 2048  23     58  100.1 / 99.5                       24    49   64.1 / 57.7      1500 x 7168  18    90  140.5 / 142.8
+//   4096 x 2048  33.5   70  115.4 / 114.0    3000 x 2048 bf16, top-6                       1500 x 5120 bf16
+//   1700 x 4096  23     58  100.7 / 94.0                       54    74   84.8 / 90.3                   18   123  127.7 / 140.0
+// The rank of the hottest of 256 experts on 64 ranks: 100 tokens of 4096 86.2 / 77.4, 200 of 2048 86.7 / 80.2.
+static bool dispatch_in_one_launch(int num_tokens, int num_topk, int num_experts, int max_tokens, int hidden,
+                                   int row_format, int64_t expected_rows) {
+    if (deepep_ll_dispatch_is_single_launch(num_tokens, num_topk, num_experts, max_tokens, expected_rows) != 0) return true;
+    const int pieces = row_pieces(hidden, row_format);
+    const int tokens = pieces <= kFusedManyPieces ? tokens_per_send_block(pieces, kFusedMaxWaves, num_topk, num_tokens) : 1;
+    const int64_t send_blocks = (num_tokens + tokens - 1) / tokens * int64_t((pieces + kFusedMaxWaves - 1) / kFusedMaxWaves);
+    return send_blocks * num_tokens * num_topk <= (int64_t(24) << 20) &&
+           estimated_rows(expected_rows, num_experts, max_tokens) * row_payload_bytes(hidden, row_format) <= (int64_t(72) << 20);
+}
+
 static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_t* src_ranks, int num_src,
                             int num_tokens, int hidden, int num_topk, int num_experts, int num_ranks, int rank,
                             int max_tokens, int row_format, void* recv_staging, int32_t* recv_count,
@@ -1229,7 +1266,7 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         }
     }
 
-    const int pieces = row_format == kRowBF16 ? (hidden * 2 + 1023) / 1024 : (hidden / kGroup + 7) / 8;
+    const int pieces = row_pieces(hidden, row_format);
     // A small batch cannot fill 1024 SIMDs with one wave per row piece: give a share of the
     // K stores of each piece to a second wave.
     int split_log2 = int64_t(num_src) * num_tokens * pieces < 4096 && num_topk > 1 ? 1 : 0;
@@ -1237,7 +1274,7 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     // workgroups small enough that two fit a compute unit.
     if (fused_recv != nullptr) split_log2 = 0;
     const int items = pieces << split_log2;  // waves per token
-    const int max_waves = fused_recv != nullptr ? 8 : kSendMaxWaves;
+    const int max_waves = fused_recv != nullptr ? kFusedMaxWaves : kSendMaxWaves;
     int waves = items < max_waves ? items : max_waves;
     const int blocks_per_token = (items + waves - 1) / waves;
     // Every workgroup of the single launch goes through the batch's entries, the send ones for their slots and the
@@ -1246,10 +1283,8 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     if (fused_recv != nullptr && n > 1536 && waves > 4) waves = 8;
     if (fused_recv != nullptr && waves < 4) waves = 4;  // the receive workgroups want a few waves each
     int tokens_per_block = 1;
-    if (!ranked && blocks_per_token == 1 && (fused_recv == nullptr || items <= 2))
-        while (tokens_per_block < 4 && 2 * tokens_per_block * items <= max_waves &&
-               2 * tokens_per_block * num_topk <= kWave && num_tokens >= 2 * tokens_per_block * kManyBlocks)
-            tokens_per_block *= 2;
+    if (!ranked && blocks_per_token == 1 && (fused_recv == nullptr || items <= kFusedManyPieces))
+        tokens_per_block = tokens_per_send_block(items, max_waves, num_topk, num_tokens);
     const int token_blocks = (num_tokens + tokens_per_block - 1) / tokens_per_block;
     if (tokens_per_block > 1) waves = std::max(waves, items * tokens_per_block);
     // floor(e / E_l) == umulhi(e, ceil(2^32 / E_l)) for every e below 2^16.
@@ -1648,11 +1683,18 @@ int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx, int num_
     EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(observed_host) & 7) == 0);
     const ObservedRows observed = {observed_host, uint32_t(num_tokens < 0 ? 0 : num_tokens)};
     const int64_t max_rows = int64_t(num_experts) * num_max_dispatch_tokens_per_rank;
-    const bool fused = deepep_ll_dispatch_is_single_launch(num_tokens, num_topk, num_experts,
-                                                           num_max_dispatch_tokens_per_rank, expected_rows) != 0;
     if (int rc = check_ll_shape(num_tokens, hidden, num_topk, num_experts, num_ranks, rank,
                                 num_max_dispatch_tokens_per_rank, row_format))
         return rc;
+    const bool fused = dispatch_in_one_launch(num_tokens, num_topk, num_experts, num_max_dispatch_tokens_per_rank, hidden,
+                                              row_format, expected_rows);
+    const bool large = segment_workspace != nullptr && num_experts <= 1024 &&
+                       estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank) > kLargeBatchRows;
+    if (large) {
+        EP_HOST_ASSERT(segment_workspace_bytes >=
+                       size_t(deepep::segment_workspace_bytes(num_experts, num_max_dispatch_tokens_per_rank)));
+        EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(segment_workspace) & 15) == 0);
+    }
     if (!fused) {
         // The two phases back to back, with the single launch's shortcut: the send side writes the
         // rows for this rank's own experts straight to their packed position behind the lower ranks'
@@ -1671,13 +1713,7 @@ int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx, int num_
         // When the receive side will run as index + flat copy, the index is built by extra workgroups of
         // the send launch: three launches (slots, send + index, copy) instead of four.
         FusedIndexArgs index = {};
-        const bool flat_copy =
-            segment_workspace != nullptr && num_experts <= 1024 &&
-            estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank) > kLargeBatchRows;
-        if (flat_copy) {
-            EP_HOST_ASSERT(segment_workspace_bytes >=
-                           size_t(deepep::segment_workspace_bytes(num_experts, num_max_dispatch_tokens_per_rank)));
-            EP_HOST_ASSERT((reinterpret_cast<uintptr_t>(segment_workspace) & 15) == 0);
+        if (large) {
             index.recv_count = recv_count;
             index.num_experts = num_experts, index.num_local_experts = num_experts / num_ranks;
             index.num_ranks = num_ranks, index.rank = rank, index.max_tokens = num_max_dispatch_tokens_per_rank;
@@ -1693,7 +1729,7 @@ int deepep_ll_dispatch_observed(const void* x, const int64_t* topk_idx, int num_
                                       rank, num_max_dispatch_tokens_per_rank, row_format, recv_staging, recv_count,
                                       send_slots, send_count, pair_slot, workspace, workspace_bytes,
                                       reinterpret_cast<hipStream_t>(stream), nullptr, 0, &direct, nullptr,
-                                      flat_copy ? &index : nullptr, &index_done))
+                                      large ? &index : nullptr, &index_done))
             return rc;
         return launch_recv_side(recv_staging, recv_count, hidden, num_experts, num_ranks,
                                 num_max_dispatch_tokens_per_rank, row_format, packed_recv_x, packed_recv_scales,

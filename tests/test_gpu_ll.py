@@ -1223,6 +1223,35 @@ def test_several_tokens_a_workgroup(rt, t, k, h, fmt):
     assert torch.equal(got.pair_slot.cpu().view(-1)[:t * k], st.pair_slot.cpu().view(-1)[:t * k])
 
 
+@pytest.mark.parametrize("t,k,h,fmt", [
+    (1024, 8, 2048, O.ROW_FP8), (1025, 8, 2048, O.ROW_FP8),  # 8192 entries, more
+    (1025, 8, 4096, O.ROW_BF16), (1291, 7, 640, O.ROW_FP8_POW2), (1100, 8, 3584, O.ROW_FP8_UE8M0),
+    (1773, 8, 2176, O.ROW_FP8), (1774, 8, 2176, O.ROW_FP8),  # 24 M entries for a token a workgroup to go through
+    (3546, 8, 512, O.ROW_BF16), (3547, 8, 512, O.ROW_BF16)])  # and for four tokens a workgroup
+def test_one_call_dispatch_past_8192_entries(rt, t, k, h, fmt):
+    """One launch or several, by entries, rows expected and what these hold in all: the oracle's rows either way, also
+    where far more or fewer of them arrive than were expected."""
+    r, rank, e, m = 4, 2, 20, t
+    g = torch.Generator().manual_seed(t * k)
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + k, drop=0)
+    topk_all[torch.rand(topk_all.shape, generator=g) < 0.1] = 11  # the rank's own, and more often than a token has slots for
+    topk_all[torch.rand(topk_all.shape, generator=g) < 0.05] = -1
+    most = (72 << 20) // rt.capi.load().deepep_ll_row_payload_bytes(h, fmt)
+    st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, m, fmt, one_call=True)
+    x, topk = world.own_inputs()
+    want = O.ll_dispatch(list(x_all), list(topk_all), rank, e, m, fmt)
+    check_dispatch(st, want, fmt)
+    slots = st.pair_slot.clone()
+    if st.segment_workspace is None:
+        st.segment_workspace = torch.empty(rt.capi.load().deepep_ll_segment_workspace_bytes(e, m), dtype=torch.uint8,
+                                           device="cuda")
+    for hint in (8192, 8193, most, most + 1):
+        st.expected_rows = hint
+        run_dispatch(st, world, x, topk, None, one_call=True)
+        check_dispatch(st, want, fmt)
+        assert torch.equal(st.pair_slot, slots)
+
+
 @pytest.mark.parametrize("receive", ["from_tails", "ordered"])
 def test_all_to_all_with_an_empty_batch(rt, receive):
     """No token anywhere: the tables are zeros, nothing is received, the records stay untouched, and the reduce of
