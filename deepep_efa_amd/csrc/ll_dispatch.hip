@@ -1185,7 +1185,7 @@ static int tokens_per_send_block(int items, int max_waves, int num_topk, int num
     return tokens;
 }
 
-constexpr int kFusedMaxWaves = 8, kFusedManyPieces = 2;
+constexpr int kFusedMaxWaves = 8, kFusedManyPieces = 2, kFusedEvenEntries = 1792;
 
 // Whether a one-call dispatch runs as one launch: up to 8192 entries and rows always.  Past them it saves a launch or two
 // (4 to 8 us) and pays with its workgroups' sweeps through the entries, fewer of them where a workgroup has several
@@ -1281,6 +1281,14 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     // receive ones for the own counts: from some 1500 entries on the eighth wave that a 7168-wide row has no piece
     // for is worth its place (256 tokens, top-8 15.9 -> 15.1 us, 1024 tokens 40.9 -> 39.6; 128 tokens 8.0 -> 8.1).
     if (fused_recv != nullptr && n > 1536 && waves > 4) waves = 8;
+    // A row of several workgroups is cut evenly in the single launch where that does without two waves or more of each: the
+    // waves that have no piece take others' places on the chip.  Past 1792 entries they pay for it with what they do for the
+    // sweeps.  Microseconds of a step in bf16, eight waves / five (six at hidden 6144), top-8 to 32 ranks:
+    //   100 x 5120 to 8    16.7 / 16.2    128 x 5120  21.8 / 20.6    180 to 16  28.0 / 26.3    220  30.6 / 29.5
+    //   190 x 4608 to 64   28.8 / 27.3    150 x 6144  27.6 / 26.6    16 and 60  12.2 and 14.4 either way
+    //   250 x 5120 to 64   28.1 / 28.7    400 to 8    39.0 / 39.9    1000 to 8  91.0 / 92.7; seven of eight, 128 x 7168 26.7 / 27.0
+    const int even_waves = (items + blocks_per_token - 1) / blocks_per_token;
+    if (fused_recv != nullptr && blocks_per_token > 1 && n <= kFusedEvenEntries && even_waves + 2 <= waves) waves = even_waves;
     if (fused_recv != nullptr && waves < 4) waves = 4;  // the receive workgroups want a few waves each
     int tokens_per_block = 1;
     if (!ranked && blocks_per_token == 1 && (fused_recv == nullptr || items <= kFusedManyPieces))

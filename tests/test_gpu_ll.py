@@ -1224,6 +1224,26 @@ def test_several_tokens_a_workgroup(rt, t, k, h, fmt):
 
 
 @pytest.mark.parametrize("t,k,h,fmt", [
+    (13, 8, 4608, O.ROW_BF16), (224, 8, 4608, O.ROW_BF16), (225, 8, 4608, O.ROW_BF16),  # 9 pieces: five waves of a workgroup, eight
+    (200, 6, 5120, O.ROW_BF16), (150, 8, 6144, O.ROW_BF16), (40, 8, 7168, O.ROW_BF16),  # 10, 12 and 14: five, six, eight
+    (100, 7, 9216, O.ROW_FP8), (31, 3, 8832, O.ROW_FP8_POW2), (20, 5, 17408, O.ROW_FP8_UE8M0)])  # fp8; three workgroups a row
+def test_rows_cut_evenly_between_workgroups(rt, t, k, h, fmt):
+    """A row of more pieces than a workgroup has waves, cut evenly up to 1792 entries: the oracle's rows, sent and kept."""
+    r, rank, e, m = 4, 2, 20, t
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + k, drop=5)
+    want = O.ll_dispatch(list(x_all), list(topk_all), rank, e, m, fmt)
+    (got, _), (two, _) = (dispatch_on_gpu(rt, x_all, topk_all, rank, e, m, fmt, one_call=c) for c in (True, False))
+    check_dispatch(got, want, fmt)
+    check_dispatch(two, want, fmt)
+    assert torch.equal(got.pair_slot, two.pair_slot) and torch.equal(got.send_count, two.send_count)
+    data, own = (2 * h if fmt == O.ROW_BF16 else h), e // r
+    for expert in range(e):  # rows to other ranks leave through the slots
+        n = min(m, int(got.send_count[expert])) if expert // own != rank else 0
+        a, b = (s.send_slots.view(torch.uint8).view(e, m, s.stride)[expert, :n, :data] for s in (got, two))
+        assert torch.equal(a, b), f"rows sent to expert {expert}"
+
+
+@pytest.mark.parametrize("t,k,h,fmt", [
     (1024, 8, 2048, O.ROW_FP8), (1025, 8, 2048, O.ROW_FP8),  # 8192 entries, more
     (1025, 8, 4096, O.ROW_BF16), (1291, 7, 640, O.ROW_FP8_POW2), (1100, 8, 3584, O.ROW_FP8_UE8M0),
     (1773, 8, 2176, O.ROW_FP8), (1774, 8, 2176, O.ROW_FP8),  # 24 M entries for a token a workgroup to go through
