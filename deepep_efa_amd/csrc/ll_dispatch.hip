@@ -1186,6 +1186,7 @@ static int tokens_per_send_block(int items, int max_waves, int num_topk, int num
 }
 
 constexpr int kFusedMaxWaves = 8, kFusedManyPieces = 2, kFusedEvenEntries = 1792;
+constexpr int kFusedFewFrom = 4608, kFusedFewTokens = 1536;  // entries, tokens
 
 // Whether a one-call dispatch runs as one launch: up to 8192 entries and rows always.  Past them it saves a launch or two
 // (4 to 8 us) and pays with its workgroups' sweeps through the entries, fewer of them where a workgroup has several
@@ -1325,7 +1326,15 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         EP_HOST_ASSERT(num_src == 1 && src_ranks == nullptr);
         const int num_send_blocks = blocks_per_token * token_blocks;
         int64_t fused_recv_blocks = (fused_recv_wave_items + waves - 1) / waves;
-        const int64_t most = tokens_per_block > 1 ? 512 : 1024;
+        // Every receive workgroup goes through the batch's entries for the own counts.  Small ones of four waves do better with
+        // half as many of them once there are entries enough, as long as the send workgroups in front leave them places in
+        // the first round.  Microseconds of a step, top-8 in fp8 unless said, 1024 of them / 512:
+        //   580 x 4096   36.7 / 35.1    700 x 4096  42.2 / 40.8    820 x 4096  49.7 / 47.5    936 x 4096, top-6  44.6 / 43.1
+        //   1000 x 4096  56.1 / 55.4    600 x 2048 bf16  30.3 / 29.7    900 x 2048 bf16  36.9 / 35.6    1500 x 4096, top-4  49.1 / 48.6
+        //   400 x 4096   28.4 / 28.3    500 x 2048 bf16  23.8 / 24.6    1100 x 2048 bf16  44.7 / 45.6    2000 x 4096, top-4  58.9 / 60.0
+        // Workgroups of eight waves: 340 x 7168 bf16 47.6 / 48.2, 1000 x 7168 93.3 / 94.0.
+        const bool few = waves <= 4 && n > kFusedFewFrom && n <= kFusedMaxEntries && num_tokens <= kFusedFewTokens;
+        const int64_t most = tokens_per_block > 1 || few ? 512 : 1024;
         fused_recv_blocks = fused_recv_blocks < 1 ? 1 : (fused_recv_blocks > most ? most : fused_recv_blocks);
         const int64_t total = int64_t(num_send_blocks) + 1 + fused_recv_blocks + 1;  // + counting, + metadata
         EP_HOST_ASSERT(total < (int64_t(1) << 31));

@@ -1244,6 +1244,26 @@ def test_rows_cut_evenly_between_workgroups(rt, t, k, h, fmt):
 
 
 @pytest.mark.parametrize("t,k,h,fmt", [
+    (576, 8, 4096, O.ROW_FP8), (577, 8, 4096, O.ROW_FP8), (1024, 8, 3072, O.ROW_FP8_UE8M0), (1536, 5, 2048, O.ROW_BF16),
+    (1537, 5, 2048, O.ROW_BF16)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_fewer_receive_workgroups(rt, t, k, h, fmt, skew):
+    """Either side of where the single-launch dispatch has half as many receive workgroups, which go round for the rows:
+    as many as were expected, and twice as many."""
+    r, rank, e, m = 4, 1, 16, t
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + k, drop=9)
+    if skew:  # every token's first two selections are this rank's
+        topk_all[:, :, 0], topk_all[:, :, 1] = 4, 6
+    st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, m, fmt, one_call=True)
+    want = O.ll_dispatch(list(x_all), list(topk_all), rank, e, m, fmt)
+    check_dispatch(st, want, fmt)
+    x, topk = world.own_inputs()
+    st.expected_rows = 1  # far too few
+    run_dispatch(st, world, x, topk, None, one_call=True)
+    check_dispatch(st, want, fmt)
+
+
+@pytest.mark.parametrize("t,k,h,fmt", [
     (1024, 8, 2048, O.ROW_FP8), (1025, 8, 2048, O.ROW_FP8),  # 8192 entries, more
     (1025, 8, 4096, O.ROW_BF16), (1291, 7, 640, O.ROW_FP8_POW2), (1100, 8, 3584, O.ROW_FP8_UE8M0),
     (1773, 8, 2176, O.ROW_FP8), (1774, 8, 2176, O.ROW_FP8),  # 24 M entries for a token a workgroup to go through
