@@ -861,10 +861,11 @@ __global__ __launch_bounds__(kSendMaxWaves* kWave, 8) void ll_send_ranked_kernel
 // experts are not in the staging area — the send side puts them straight into
 // the packed tensors, behind the rows of the lower ranks — so the copying waves
 // skip the own segments and move the segments of the higher ranks up by the
-// expert's own count.  With own_topk (single launch) that count is recounted
-// from the rank's own indices, because the launch that reads recv_count's own
-// entries is the one that writes them; without it (the send kernel has
-// finished) recv_count holds it.
+// expert's own count.  With own_entries >= 0 (single launch) that count is
+// recounted from the rank's own indices, because the launch that reads
+// recv_count's own entries is the one that writes them; with kOwnCounted (the
+// send kernel has finished) recv_count holds it.  It takes a value of its own to
+// say so: the list of a rank without tokens is empty, and its address may be null.
 // ---------------------------------------------------------------------
 struct RecvArgs {
     const uint8_t* recv_staging;
@@ -888,6 +889,7 @@ __device__ __forceinline__ int clamp_count(int c, int max_tokens) {
 // workgroup in two steps so that other loads can be issued in between: `begin` issues the first index
 // loads and clears the counters, `finish` counts and ends with a barrier.
 constexpr int kOwnAhead = 4;  // index loads in flight per thread, two entries each
+constexpr int kOwnCounted = -1;
 
 struct OwnCountLoads {
     EntryPair v[kOwnAhead];
@@ -896,7 +898,7 @@ struct OwnCountLoads {
 __device__ __forceinline__ void own_row_counts_begin(const RecvArgs& a, const int64_t* own_topk, int own_entries,
                                                      int32_t* own_cnt, OwnCountLoads& loads) {
     const int tid = threadIdx.x, threads = block_threads();
-    if (own_topk == nullptr) return;
+    if (own_entries == kOwnCounted) return;
     const auto list = entry_list(own_topk, own_entries);
 #pragma unroll
     for (int r = 0; r < kOwnAhead; ++r) loads.v[r].load(list, tid + r * threads);
@@ -907,7 +909,7 @@ __device__ __forceinline__ void own_row_counts_begin(const RecvArgs& a, const in
 __device__ __forceinline__ void own_row_counts_finish(const RecvArgs& a, const int64_t* own_topk, int own_entries,
                                                       int own_rank, int32_t* own_cnt, OwnCountLoads& loads) {
     const int tid = threadIdx.x, threads = block_threads();
-    if (own_topk == nullptr) {  // the send kernel has finished: recv_count holds the own counts
+    if (own_entries == kOwnCounted) {
         for (int le = tid; le < a.num_local_experts; le += threads)
             own_cnt[le] = a.recv_count[le * a.num_ranks + own_rank];
         lds_barrier();
@@ -1091,11 +1093,10 @@ __device__ __forceinline__ void recv_rows(const RecvArgs& a, int block, int num_
 }
 
 // own_rank >= 0: the send side has already put this rank's own rows at their packed position.
-__global__ __launch_bounds__(256) void ll_recv_kernel(RecvArgs a, const int64_t* own_topk, int own_entries,
-                                                      int own_rank) {
+__global__ __launch_bounds__(256) void ll_recv_kernel(RecvArgs a, int own_rank) {
     extern __shared__ int32_t flat[];  // [num_segments + 1 + E_l]
     __shared__ int32_t wave_totals[kMaxBlockWaves];
-    recv_rows<false>(a, blockIdx.x, int(gridDim.x) - 1, own_topk, own_entries, own_rank, flat, wave_totals);
+    recv_rows<false>(a, blockIdx.x, int(gridDim.x) - 1, nullptr, kOwnCounted, own_rank, flat, wave_totals);
 }
 
 // ---------------------------------------------------------------------
@@ -1662,7 +1663,7 @@ static int launch_recv_side(const void* recv_staging, const int32_t* recv_count,
     const int64_t cap = large ? 4096 : 1024;
     if (blocks > cap) blocks = cap;
     const size_t lds = size_t(num_experts + 1 + num_local_experts) * sizeof(int32_t);
-    launch(ll_recv_kernel, dim3(unsigned(blocks) + 1), 256, lds, hs, ra, nullptr, 0, own_rank);  // + the metadata workgroup
+    launch(ll_recv_kernel, dim3(unsigned(blocks) + 1), 256, lds, hs, ra, own_rank);  // + the metadata workgroup
     EP_LAUNCH_CHECK();
     return 0;
 }

@@ -790,6 +790,34 @@ def test_empty_batch(rt, one_call):
     assert (st.send_count == 0).all()
 
 
+@pytest.mark.parametrize("hint", [180, 9000, 18000], ids=["one_launch", "past_8192_rows", "past_72_MB"])
+@pytest.mark.parametrize("rank", [0, 1, 3])
+def test_empty_batch_after_one_with_own_rows(rt, rank, hint):
+    """A rank that ran out of tokens: the counts of its own rows that the call before left are gone from ranges, counts,
+    statistics and the places of the higher ranks' rows.  An empty tensor's address is null, which says nothing else."""
+    r, t, m, h, k, e = 4, 60, 1200, 4096, 3, 16
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=8 + rank, drop=3)
+    st = rt.ll.LowLatencyState(rt.ll.LLShape(r, rank, e, m, h, k, O.ROW_FP8))
+    st.expected_rows = hint
+    st.segment_workspace = torch.empty(rt.capi.load().deepep_ll_segment_workspace_bytes(e, m), dtype=torch.uint8, device="cuda")
+    world = rt.lb.LoopbackWorld(r, rank)
+    world.set_inputs(x_all.cuda(), topk_all.cuda())
+    xs, topks = list(x_all), list(topk_all)
+    for tokens in (t, 0, t, 0):
+        x, topk = x_all[rank, :tokens].cuda(), topk_all[rank, :tokens].cuda()
+        assert (x.data_ptr() == 0) == (tokens == 0)
+        stats = torch.zeros(e // r, dtype=torch.int32, device="cuda")
+        run_dispatch(st, world, x, topk, stats, one_call=True)
+        xs[rank], topks[rank] = x_all[rank, :tokens], topk_all[rank, :tokens]
+        want = O.ll_dispatch(xs, topks, rank, e, m, O.ROW_FP8)
+        check_dispatch(st, want, O.ROW_FP8)
+        assert torch.equal(stats.cpu(), want["packed_recv_count"])
+        send_count, _ = O.route(topks[rank], e, m)
+        assert torch.equal(st.send_count.cpu(), send_count)
+        own = st.recv_count.view(e // r, r)[:, rank].cpu()
+        assert torch.equal(own, send_count[rank * (e // r):(rank + 1) * (e // r)])
+
+
 def test_large_batch_without_the_segment_workspace(rt, oracle_c):
     """A large batch but no workspace for the row index: receive and row return fall back to the
     kernels of the small-batch path and must give the same answers."""
