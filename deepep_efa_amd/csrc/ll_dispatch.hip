@@ -1200,14 +1200,27 @@ constexpr int kFusedFewFrom = 4608, kFusedFewTokens = 1536;  // entries, tokens
 //   4096 x 2048  33.5   70  115.4 / 114.0    3000 x 2048 bf16, top-6                       1500 x 5120 bf16
 //   1700 x 4096  23     58  100.7 / 94.0                       54    74   84.8 / 90.3                   18   123  127.7 / 140.0
 // The rank of the hottest of 256 experts on 64 ranks: 100 tokens of 4096 86.2 / 77.4, 200 of 2048 86.7 / 80.2.
+// One workgroup counts all entries, one a thread and round, and the launch waits for it: 96 rounds at most, and 44 for rows of
+// one wave, whose launches are short.  Those also have more sweeps for their bytes, and so does a token of more than 32
+// selections.  Microseconds of the dispatch alone, three launches / one:
+//   rows of one wave    1375 x 512 13.2 / 11.5    1750 x 512 bf16 16.5 / 17.2    2200 x 512 16.4 / 18.5    3500 x 128 bf16 17.7 / 25.8
+//     top-2, 5000 x 512 14.3 / 13.7 (12.5 M), 5500 15.0 / 15.3 (15 M)    top-64, 129 x 512 14.5 / 15.9, 257 x 1024 21.9 / 22.5
+//   top-32, 750 x 2048 36.1 / 34.5 (94 rounds), 1000 43.5 / 49.3 (125)   top-16, 2000 x 2048 42.5 / 33.6 (62, in eight waves)
+//   top-64 in rows of 1152 to 2048 bytes, 131 tokens 16.6 / 17.8 and 20.3 / 19.1
+//   rows of 256 bytes, some 66000 29.4 / 23.4, 116000 39.5 / 42.4
 static bool dispatch_in_one_launch(int num_tokens, int num_topk, int num_experts, int max_tokens, int hidden,
                                    int row_format, int64_t expected_rows) {
     if (deepep_ll_dispatch_is_single_launch(num_tokens, num_topk, num_experts, max_tokens, expected_rows) != 0) return true;
     const int pieces = row_pieces(hidden, row_format);
     const int tokens = pieces <= kFusedManyPieces ? tokens_per_send_block(pieces, kFusedMaxWaves, num_topk, num_tokens) : 1;
+    const int64_t entries = int64_t(num_tokens) * num_topk;
     const int64_t send_blocks = (num_tokens + tokens - 1) / tokens * int64_t((pieces + kFusedMaxWaves - 1) / kFusedMaxWaves);
-    return send_blocks * num_tokens * num_topk <= (int64_t(24) << 20) &&
-           estimated_rows(expected_rows, num_experts, max_tokens) * row_payload_bytes(hidden, row_format) <= (int64_t(72) << 20);
+    const int counting_threads = (pieces * tokens <= 4 ? 4 : kFusedMaxWaves) * kWave;
+    if (num_topk > 32 && row_data_bytes(hidden, row_format) < 2048) return false;
+    const int64_t rows = estimated_rows(expected_rows, num_experts, max_tokens);
+    return entries <= int64_t(pieces == 1 ? 44 : 96) * counting_threads &&
+           send_blocks * entries <= (int64_t(pieces == 1 ? 14 : 24) << 20) && rows <= 96 * 1024 &&
+           rows * row_payload_bytes(hidden, row_format) <= (int64_t(72) << 20);
 }
 
 static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_t* src_ranks, int num_src,
@@ -1685,6 +1698,14 @@ int deepep_ll_dispatch_is_single_launch(int num_tokens, int num_topk, int num_ex
                                         int num_max_dispatch_tokens_per_rank, int64_t expected_rows) {
     return int64_t(num_tokens) * num_topk <= kFusedMaxEntries &&
                    estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank) <= kLargeBatchRows
+               ? 1
+               : 0;
+}
+
+int deepep_ll_dispatch_takes_one_launch(int num_tokens, int hidden, int num_topk, int num_experts,
+                                        int num_max_dispatch_tokens_per_rank, int row_format, int64_t expected_rows) {
+    return dispatch_in_one_launch(num_tokens, num_topk, num_experts, num_max_dispatch_tokens_per_rank, hidden, row_format,
+                                  expected_rows)
                ? 1
                : 0;
 }

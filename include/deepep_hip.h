@@ -557,14 +557,19 @@ int deepep_ll_combine_recv_flat(const void* recv_flat, int64_t recv_flat_rows, i
  * send_count, send_slots and pair_slot are written as by
  * deepep_ll_dispatch_send.  Small batches (num_tokens * num_topk <= 8192 and at
  * most 8192 rows expected, and larger ones of up to 72 MB of rows and some
- * thousand tokens) run as one kernel launch, others as the send
- * and receive launches back to back; the result is the same.
+ * thousand tokens: deepep_ll_dispatch_takes_one_launch) run as one kernel
+ * launch, others as the send and receive launches back to back; the result is
+ * the same.
  *   workspace          as for deepep_ll_dispatch_send
  *   segment_workspace  as the workspace of deepep_ll_dispatch_recv */
 /* 1 when deepep_ll_dispatch runs a batch of this shape as one kernel launch whatever the size of its rows, else 0: then
  * it depends on that, too (the result does not depend on it).  No counterpart in the reference. */
 int deepep_ll_dispatch_is_single_launch(int num_tokens, int num_topk, int num_experts,
                                         int num_max_dispatch_tokens_per_rank, int64_t expected_rows);
+/* 1 when deepep_ll_dispatch runs a batch of this shape, of rows of this size and format, as one kernel launch, else 0.
+ * No counterpart in the reference. */
+int deepep_ll_dispatch_takes_one_launch(int num_tokens, int hidden, int num_topk, int num_experts,
+                                        int num_max_dispatch_tokens_per_rank, int row_format, int64_t expected_rows);
 
 int deepep_ll_dispatch(const void* x, const int64_t* topk_idx,
                        int num_tokens, int hidden, int num_topk, int num_experts,

@@ -129,6 +129,31 @@ def test_rows_expected_of_a_batch_follow_the_last_one(tokens, seen_tokens, seen_
         assert lib.deepep_ll_dispatch_is_single_launch(tokens, 8, 256, 128, got) == 1
 
 
+@pytest.mark.parametrize("t,h,k,e,fmt,rows,want", [
+    (1024, 512, 8, 64, 1, 8192, 1),                                 # 8192 entries and rows, whatever these hold
+    (1408, 512, 8, 64, 0, 0, 1), (1409, 512, 8, 64, 0, 0, 0),       # rows of one wave: 44 rounds of the counting workgroup
+    (1408, 1024, 8, 64, 1, 0, 1), (1409, 1024, 8, 64, 1, 0, 0),
+    (5416, 512, 2, 64, 1, 0, 1), (5417, 512, 2, 64, 1, 0, 0),       # and 14 M entries for the send workgroups
+    (3500, 128, 8, 64, 0, 0, 0),
+    (3546, 1024, 8, 64, 0, 0, 1), (3547, 1024, 8, 64, 0, 0, 0),     # four tokens a workgroup: 24 M
+    (1773, 2176, 8, 64, 1, 0, 1), (1774, 2176, 8, 64, 1, 0, 0),     # one
+    (768, 1152, 32, 256, 1, 0, 1), (769, 1152, 32, 256, 1, 0, 0),   # 96 rounds of four waves
+    (1000, 1152, 16, 64, 1, 0, 1), (2000, 1152, 16, 64, 1, 0, 1),   # and of eight
+    (140, 1920, 64, 256, 1, 0, 0), (140, 2048, 64, 256, 1, 0, 1),   # more than 32 selections: rows of 2 KB
+    (140, 896, 64, 256, 0, 0, 0), (140, 1024, 64, 256, 0, 0, 1),
+    (600, 2048, 8, 64, 1, (72 << 20) // 2128, 1), (600, 2048, 8, 64, 1, (72 << 20) // 2128 + 1, 0),  # 72 MB of rows
+    (600, 128, 8, 256, 0, 96 << 10, 1), (600, 128, 8, 256, 0, (96 << 10) + 1, 0),
+    (0, 512, 8, 64, 1, 20000, 1), (0, 7168, 8, 64, 1, 20000, 0),    # a rank without tokens
+])
+def test_batches_that_a_one_call_dispatch_takes_in_one_launch(t, h, k, e, fmt, rows, want):
+    from deepep_efa_amd import _capi
+    lib, m = _capi.load(), max(t, 4096)
+    rows = rows or t * k
+    assert lib.deepep_ll_dispatch_takes_one_launch(t, h, k, e, m, fmt, rows) == want
+    if lib.deepep_ll_dispatch_is_single_launch(t, k, e, m, rows):
+        assert want == 1
+
+
 @pytest.mark.parametrize("tokens,a,b,want", [
     (1000, (0, 0), (0, 0), 8000),
     (1000, (1000, 160000), (0, 0), 160000),           # one report so far

@@ -105,6 +105,24 @@ def dispatch_on_gpu(rt, x_all, topk_all, rank, e, m, fmt, stats=None, one_call=F
     return st, world
 
 
+def takes_one_launch(rt, st, t):
+    """Whether a one-call dispatch of t tokens takes the single launch."""
+    s = st.shape
+    return rt.capi.load().deepep_ll_dispatch_takes_one_launch(t, s.hidden, s.num_topk, s.num_experts, s.max_tokens, s.fmt,
+                                                              st.expected_rows) == 1
+
+
+def kernels_launched(call, tmp_path):
+    """The low-latency kernels of a call, by the nodes of a captured graph."""
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    graph.enable_debug_mode()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        call()
+    graph.debug_dump(str(tmp_path / "graph.dot"))
+    return set(re.findall(r"ll_[a-z_]*?kernel", (tmp_path / "graph.dot").read_text()))
+
+
 def check_dispatch(st, want, fmt):
     count = st.packed_recv_count.cpu()
     assert torch.equal(count, want["packed_recv_count"])
@@ -1295,10 +1313,12 @@ def test_fewer_receive_workgroups(rt, t, k, h, fmt, skew):
     (1024, 8, 2048, O.ROW_FP8), (1025, 8, 2048, O.ROW_FP8),  # 8192 entries, more
     (1025, 8, 4096, O.ROW_BF16), (1291, 7, 640, O.ROW_FP8_POW2), (1100, 8, 3584, O.ROW_FP8_UE8M0),
     (1773, 8, 2176, O.ROW_FP8), (1774, 8, 2176, O.ROW_FP8),  # 24 M entries for a token a workgroup to go through
-    (3546, 8, 512, O.ROW_BF16), (3547, 8, 512, O.ROW_BF16)])  # and for four tokens a workgroup
-def test_one_call_dispatch_past_8192_entries(rt, t, k, h, fmt):
+    (3546, 8, 1024, O.ROW_BF16), (3547, 8, 1024, O.ROW_BF16),  # and for four tokens a workgroup
+    (3546, 8, 512, O.ROW_BF16), (1408, 8, 512, O.ROW_BF16), (1409, 8, 512, O.ROW_BF16)])  # rows of one wave: 11264 entries
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
+def test_one_call_dispatch_past_8192_entries(rt, t, k, h, fmt, tmp_path):
     """One launch or several, by entries, rows expected and what these hold in all: the oracle's rows either way, also
-    where far more or fewer of them arrive than were expected."""
+    where far more or fewer of them arrive than were expected; and the launches that a caller is told of."""
     r, rank, e, m = 4, 2, 20, t
     g = torch.Generator().manual_seed(t * k)
     x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + k, drop=0)
@@ -1313,11 +1333,16 @@ def test_one_call_dispatch_past_8192_entries(rt, t, k, h, fmt):
     if st.segment_workspace is None:
         st.segment_workspace = torch.empty(rt.capi.load().deepep_ll_segment_workspace_bytes(e, m), dtype=torch.uint8,
                                            device="cuda")
+    few = t * k <= 8192 or (t, h) in ((1025, 4096), (1025, 2048), (1291, 640), (1100, 3584), (1773, 2176), (3546, 1024), (1408, 512))
     for hint in (8192, 8193, most, most + 1):
         st.expected_rows = hint
         run_dispatch(st, world, x, topk, None, one_call=True)
         check_dispatch(st, want, fmt)
         assert torch.equal(st.pair_slot, slots)
+        one = takes_one_launch(rt, st, t)
+        assert one == (few and hint <= most)
+        launched = kernels_launched(lambda: st.dispatch(x, topk), tmp_path)
+        assert launched == {"ll_dispatch_fused_kernel"} if one else "ll_rank_chunk_kernel" in launched
 
 
 @pytest.mark.parametrize("receive", ["from_tails", "ordered"])
