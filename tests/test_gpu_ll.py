@@ -1324,7 +1324,7 @@ def test_one_call_dispatch_past_8192_entries(rt, t, k, h, fmt, tmp_path):
     x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + k, drop=0)
     topk_all[torch.rand(topk_all.shape, generator=g) < 0.1] = 11  # the rank's own, and more often than a token has slots for
     topk_all[torch.rand(topk_all.shape, generator=g) < 0.05] = -1
-    most = (72 << 20) // rt.capi.load().deepep_ll_row_payload_bytes(h, fmt)
+    most = min(96 << 10, (72 << 20) // rt.capi.load().deepep_ll_row_payload_bytes(h, fmt))
     st, world = dispatch_on_gpu(rt, x_all, topk_all, rank, e, m, fmt, one_call=True)
     x, topk = world.own_inputs()
     want = O.ll_dispatch(list(x_all), list(topk_all), rank, e, m, fmt)
