@@ -434,7 +434,8 @@ static CombineSendArgs make_combine_send_args(const void* x, const int64_t* layo
     sa.hidden = hidden, sa.num_local_experts = num_experts / num_ranks, sa.num_ranks = num_ranks, sa.rank = rank;
     sa.expert_of = make_rank_divider(num_ranks);
     sa.max_tokens = max_tokens;
-    sa.parts_log2 = choose_row_parts_log2(estimated_rows(expected_rows, num_experts, max_tokens), int64_t(hidden) * 2);
+    sa.parts_log2 = choose_row_parts_log2(estimated_rows(expected_rows, num_experts, max_tokens), int64_t(hidden) * 2,
+                                          num_experts);
     sa.combine_staging = reinterpret_cast<uint8_t*>(combine_staging);
     sa.combine_send_slots = reinterpret_cast<uint8_t*>(combine_send_slots);
     return sa;
@@ -694,9 +695,11 @@ int deepep_ll_combine_recv_flat(const void* recv_flat, int64_t recv_flat_rows, i
 //   16800 of  8 KB 121.8 / 116.6      9000 of 10 KB (top-6)     88.1 /  89.7
 //   28000 of  4 KB 101.8 / 101.8     10000 of 10 KB (top-4)     93.6 /  94.6
 //   skewed, 64 ranks: 10324 rows for 7200 selections 130.8 / 137.8, 13638 for 1600 130.0 / 119.8
-static bool combine_in_one_launch(int64_t rows, int num_tokens, int num_topk, int64_t row_bytes) {
+// Past 256 experts, whose rows are not moved in parts (choose_row_parts_log2), up to 220 MB.
+static bool combine_in_one_launch(int64_t rows, int num_tokens, int num_topk, int64_t row_bytes, int num_experts) {
     if (rows <= kLargeBatchRows) return true;
-    return rows <= 2 * int64_t(num_tokens) * num_topk && (rows + num_tokens) * row_bytes <= (int64_t(132) << 20) &&
+    const int64_t most = int64_t(num_experts <= 4 * kWave ? 132 : 220) << 20;
+    return rows <= 2 * int64_t(num_tokens) * num_topk && (rows + num_tokens) * row_bytes <= most &&
            (row_bytes >= 2048 || rows <= 12288);
 }
 
@@ -710,7 +713,7 @@ int deepep_ll_combine(const void* x, const int64_t* layout_range, const int64_t*
     const int64_t estimated = estimated_rows(expected_rows, num_experts, num_max_dispatch_tokens_per_rank);
     const bool large = estimated > kLargeBatchRows;
     if (large && (combine_send_slots == nullptr ||
-                  !combine_in_one_launch(estimated, num_tokens, num_topk, int64_t(hidden) * 2))) {
+                  !combine_in_one_launch(estimated, num_tokens, num_topk, int64_t(hidden) * 2, num_experts))) {
         // the two phases back to back, with the single launch's shortcut: the rows owed to this rank
         // itself are not moved, the reduce reads them from x.  Without send slots (zero copy: the transport
         // sends layout_range's ranges straight from x) there is nothing to return.

@@ -1610,7 +1610,7 @@ static RecvArgs make_recv_args(const void* recv_staging, const int32_t* recv_cou
     ra.hidden = hidden, ra.num_local_experts = num_experts / num_ranks, ra.num_ranks = num_ranks;
     ra.max_tokens = max_tokens, ra.fmt = row_format, ra.expert_of = make_rank_divider(num_ranks);
     const int64_t rows = estimated_rows(expected_rows, num_experts, max_tokens), row_bytes = row_data_bytes(hidden, row_format);
-    ra.parts_log2 = choose_row_parts_log2(rows, row_bytes);
+    ra.parts_log2 = choose_row_parts_log2(rows, row_bytes, num_experts);
     // A row of up to 4 KiB is what a wave loads at once (kRecvDepth): with enough rows to occupy the chip a wave
     // takes it whole, which halves the lookups and the trips of a wave.  The dispatch alone, halves against whole
     // rows: 1200 x 4096 bytes 7.4 -> 6.8 us, 2400 x 4096 12.0 -> 10.7, 4072 x 4096 17.0 -> 15.8, 2048 x 2048 8.7 ->

@@ -633,14 +633,16 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
 }
 
 // Past 52 MB, or 40 past 8192 rows, the flat copy gains more than the index's launch costs; and past 8192 rows of less than
-// 2 KB.  Microseconds of the five calls of an exchange, 8 ranks x 8 experts, one launch against two:
+// 2 KB, or from more than 256 experts, whose counts every workgroup goes through (the receive of 8240 rows of 2 KB alone: 512
+// experts 12.7 / 16.6 in two launches and one, 1024 18.6 / 24.2, 256 11.8 / 9.9).  Microseconds of the five calls of an exchange, 8 ranks x 8 experts, one launch against two:
 //   6400 rows of  7 KB (45 MB)  91.3 / 94.7      8800 rows of  2 KB (18 MB) 48.7 / 50.1     16376 rows of 2 KB (33 MB) 72.0 / 73.0
 //   7200 (52 MB)               101.4 / 98.1      8800 rows of  4 KB (36 MB) 74.6 / 77.0     16376 rows of 1 KB         50.2 / 47.5
 //   4000 rows of 14 KB (57 MB)  79.4 / 75.8     10000 rows of  4 KB (41 MB) 84.3 / 85.2     16376 rows of 512 B        38.1 / 36.5
 //   5600 (80 MB)               101.7 / 99.6     12000 rows of  4 KB (49 MB)101.3 / 97.6
-static bool ordered_in_one_launch(int64_t rows, int64_t row_bytes) {
+static bool ordered_in_one_launch(int64_t rows, int64_t row_bytes, int num_experts) {
     if (rows <= kLargeBatchRows) return rows * row_bytes <= (int64_t(52) << 20);
-    return rows <= 2 * kLargeBatchRows && row_bytes >= 2048 && rows * row_bytes <= (int64_t(40) << 20);
+    return rows <= 2 * kLargeBatchRows && num_experts <= 4 * kWave && row_bytes >= 2048 &&
+           rows * row_bytes <= (int64_t(40) << 20);
 }
 
 int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_t slot_rows,
@@ -678,14 +680,14 @@ int deepep_ll_dispatch_recv_by_source_ordered(const void* recv_by_source, int64_
     const int num_local_experts = num_experts / num_ranks;
     hipStream_t hs = reinterpret_cast<hipStream_t>(stream);
     const int64_t expected = expected_rows > 0 ? expected_rows : most_rows;
-    if (ordered_in_one_launch(expected, row_data_bytes(hidden, row_format))) {  // every workgroup indexes for itself
+    if (ordered_in_one_launch(expected, row_data_bytes(hidden, row_format), num_experts)) {  // every workgroup indexes for itself
         OrderedRecvArgs oa;
         oa.rows = reinterpret_cast<const uint8_t*>(recv_by_source);
         oa.all_num_routed = all_num_routed;
         oa.num_experts = num_experts, oa.num_local_experts = num_local_experts, oa.num_ranks = num_ranks;
         oa.rank = rank, oa.max_tokens = num_max_dispatch_tokens_per_rank;
         oa.hidden = hidden, oa.fmt = row_format;
-        oa.parts_log2 = choose_row_parts_log2(expected, row_data_bytes(hidden, row_format));
+        oa.parts_log2 = choose_row_parts_log2(expected, row_data_bytes(hidden, row_format), num_experts);
         oa.slot_rows = slot_rows, oa.row_capacity = row_capacity, oa.expert_of = make_rank_divider(num_ranks);
         oa.packed_x = reinterpret_cast<uint8_t*>(packed_recv_x);
         oa.packed_scales = row_format == kRowBF16 ? nullptr : reinterpret_cast<uint8_t*>(packed_recv_scales);

@@ -207,8 +207,11 @@ struct RowPart {
 // in larger ones a wave that takes a whole row is what the launch ends up waiting for.  Microseconds of a dispatch and a
 // combine in one launch, rows whole / in parts: 8800 rows of 14 KB 112.5 / 109.4, 10400 of 8 KB 82.2 / 80.8, 14400 of 4 KB
 // 61.6 / 60.8, 21600 of 4 KB 85.2 / 82.8, 28000 of 4 KB 103.1 / 100.8, but of 3 KB 84.0 / 85.0, 32768 of 2 KB 69.4 / 71.5.
-inline int choose_row_parts_log2(int64_t estimated_rows, int64_t row_bytes) {
-    if (estimated_rows > (row_bytes < 4096 ? 16384 : 32768)) return 0;
+// Past 8192 rows not those of less than 4 KB, nor past 256 segments, where finding a row's place costs four times as much.
+// The combine alone: 12000 rows of 256 bytes 6.5 / 9.6, of 1 KB 8.6 / 12.2, of 2 KB 12.4 / 15.0, of 3 KB 17.8 / 18.2, of 4 KB
+// 23.3 / 22.8; 8240 rows from 1024 experts of 256 bytes 13.0 / 21.9, of 4 KB 19.9 / 26.2, of 14 KB 61.5 / 68.1.
+inline int choose_row_parts_log2(int64_t estimated_rows, int64_t row_bytes, int num_segments) {
+    if (estimated_rows > 8192 && (row_bytes < 4096 || num_segments > 4 * kWave || estimated_rows > 32768)) return 0;
     return row_bytes > 8192 ? 2 : 1;
 }
 

@@ -423,7 +423,7 @@ int deepep_ll_dispatch_recv_by_source(const void* recv_by_source, int64_t slot_r
  * gathered route counts every row's place then follows by arithmetic -- row j of source s belongs to
  * the expert whose run of that source's column of the counts holds j -- so nothing is read from the
  * rows to index them and no record list is needed: one launch for up to 8192 expected rows and 52 MB (or
- * 16384 of at least 2 KB and 40 MB), one index launch and the row copy beyond, both sides of every
+ * 16384 of at least 2 KB and 40 MB from up to 256 experts), one index launch and the row copy beyond, both sides of every
  * (expert, source) pair contiguous.  Outputs as deepep_ll_dispatch_recv_by_source.
  *   all_num_routed     [R, E] int32, as for deepep_ll_exchange_metadata (counts above M read as M)
  *   record_packed_row  [row_capacity] int32 (out) or NULL, indexed like the records of
@@ -617,7 +617,7 @@ int64_t deepep_ll_expected_rows_of_two(int num_tokens, int num_topk, int num_exp
  * answers of this rank's own experts are read from x directly — the own
  * experts' part of combine_staging is neither written nor read.  When at most
  * 8192 rows are expected, or more that are not many more than the batch sends
- * (up to some 132 MB), both phases run as one kernel launch; other batches launch
+ * (up to some 132 MB, 220 past 256 experts), both phases run as one kernel launch; other batches launch
  * them back to back.  combine_send_slots may be NULL (the reference's
  * zero_copy, deep_ep/buffer.py:2831-2852: "the next combine kernel can skip the
  * copying"): no row is returned, the call is the reduce alone, and the caller's

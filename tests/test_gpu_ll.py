@@ -113,14 +113,14 @@ def takes_one_launch(rt, st, t):
 
 
 def kernels_launched(call, tmp_path):
-    """The low-latency kernels of a call, by the nodes of a captured graph."""
+    """The low-latency kernels of a call and their workgroups (along x), by the nodes of a captured graph."""
     graph = torch.cuda.CUDAGraph(keep_graph=True)
     graph.enable_debug_mode()
     torch.cuda.synchronize()
     with torch.cuda.graph(graph):
         call()
     graph.debug_dump(str(tmp_path / "graph.dot"))
-    return set(re.findall(r"ll_[a-z_]*?kernel", (tmp_path / "graph.dot").read_text()))
+    return {name: int(blocks) for name, blocks in re.findall(r"(ll_[a-z_]*?kernel)[^\n(]*\((\d+),", (tmp_path / "graph.dot").read_text())}
 
 
 def check_dispatch(st, want, fmt):
@@ -1342,7 +1342,7 @@ def test_one_call_dispatch_past_8192_entries(rt, t, k, h, fmt, tmp_path):
         one = takes_one_launch(rt, st, t)
         assert one == (few and hint <= most)
         launched = kernels_launched(lambda: st.dispatch(x, topk), tmp_path)
-        assert launched == {"ll_dispatch_fused_kernel"} if one else "ll_rank_chunk_kernel" in launched
+        assert set(launched) == {"ll_dispatch_fused_kernel"} if one else "ll_rank_chunk_kernel" in launched
 
 
 @pytest.mark.parametrize("receive", ["from_tails", "ordered"])
@@ -2223,12 +2223,15 @@ def test_ordered_receive_in_one_launch_and_in_two(rt, fmt, h, hints):
         assert torch.equal(st.record_packed_row[:rec.numel()].cpu().long(), rec)
 
 
-@pytest.mark.parametrize("fmt,h,hints", [
-    (O.ROW_BF16, 2048, (8192, 8193, 10240, 10241)),  # 40 MB past 8192 rows
-    (O.ROW_FP8, 2048, (16384, 16385)), (O.ROW_FP8, 1920, (8192, 8193))])  # the last rows, and too narrow ones
-def test_ordered_receive_past_8192_rows(rt, fmt, h, hints):
-    """One launch or two past 8192 expected rows: the oracle's rows and records either way."""
-    r, rank, t, k, e = 4, 3, 33, 5, 24
+@pytest.mark.parametrize("fmt,h,e,hints", [
+    (O.ROW_BF16, 2048, 24, (8192, 8193, 10240, 10241)),  # 40 MB past 8192 rows
+    (O.ROW_FP8, 2048, 24, (16384, 16385)), (O.ROW_FP8, 1920, 24, (8192, 8193)),  # the last rows, and too narrow ones
+    (O.ROW_FP8, 2048, 256, (8193, 16385)), (O.ROW_FP8, 2048, 260, (8192, 8193))])  # the last experts, and too many
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
+def test_ordered_receive_past_8192_rows(rt, fmt, h, e, hints, tmp_path):
+    """One launch or two past 8192 expected rows: the oracle's rows and records either way.  All hints but the last take
+    one launch."""
+    r, rank, t, k = 4, 3, 33, 5
     x_all, topk_all, _ = make_world(r, t, h, k, e, seed=h, drop=9)
     states = [rt.ll.AllToAllState(rt.ll.LLShape(r, s, e, t, h, k, fmt)) for s in range(r)]
     for s, st in enumerate(states):
@@ -2244,6 +2247,9 @@ def test_ordered_receive_past_8192_rows(rt, fmt, h, hints):
         torch.cuda.synchronize()
         check_dispatch(st, want, fmt)
         assert torch.equal(st.record_packed_row[:rec.numel()].cpu().long(), rec)
+        launched = kernels_launched(lambda: st.dispatch_recv_ordered(routed), tmp_path)
+        assert set(launched) == ({"ll_recv_ordered_kernel"} if hint != hints[-1] else
+                                 {"ll_by_source_ordered_index_kernel", "ll_rows_flat_kernel"}), hint
 
 
 @pytest.mark.parametrize("h,hints", [
@@ -2275,12 +2281,16 @@ def test_combine_in_one_launch_and_in_two(rt, h, hints):
     assert all(torch.equal(sums[0], o) for o in sums[1:])
 
 
-@pytest.mark.parametrize("r,e,h,hints", [
-    (8, 16, 1024, (8193, 16384, 16385)),  # rows of 2 KB: in two parts, the last hint that splits them, whole
-    (8, 16, 2048, (8193, 16384, 16385)),  # rows of 4 KB: in two parts throughout
-    (2, 16, 7168, (8192, 8193, 8629, 8630)),  # rows of 14 KB in four parts; 132 MB with the tokens' rows, two launches
+@pytest.mark.parametrize("r,e,h,hints,parts", [
+    (8, 16, 512, (8192, 8193), (2, 1)), (8, 16, 1024, (8192, 8193), (2, 1)),  # rows of less than 4 KB: past 8192 whole
+    (8, 16, 1920, (8192, 8193, 16384), (2, 1, 1)),
+    (8, 16, 2048, (8193, 16384), (2, 2)),  # rows of 4 KB: in two parts throughout
+    (8, 256, 2048, (8193,), (2,)), (8, 264, 2048, (8192, 8193), (2, 1)),  # past 256 experts whole
+    (2, 16, 7168, (8192, 8193, 8629, 8630), (4, 4, 4, 0)),  # rows of 14 KB in four parts; 132 MB with the tokens' rows, two launches
+    (2, 258, 7168, (8193, 15066, 15067), (1, 1, 0)),  # and 220
 ])
-def test_combine_past_8192_rows_in_parts(rt, r, e, h, hints):
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
+def test_combine_past_8192_rows_in_parts(rt, r, e, h, hints, parts, tmp_path):
     """How the rows of a single-launch combine are cut, and whether it is one, changes no row and no sum."""
     rank, t, k = 1, 1025, 8
     x_all, topk_all, w = make_world(r, t, h, k, e, seed=h + r, drop=30)
@@ -2298,6 +2308,12 @@ def test_combine_past_8192_rows_in_parts(rt, r, e, h, hints):
         else:
             st.expected_rows = hint
             st.combine(y, topk, weights, out)
+            launched = kernels_launched(lambda: st.combine(y, topk, weights, out), tmp_path)
+            fused = [n for name, n in launched.items() if "fused" in name]
+            reduce_waves = t * -(-h // 512)
+            rows = min(hint + hint // 8 + 16, e * t)
+            cut = parts[hints.index(hint)]
+            assert fused == ([-(-reduce_waves // 4) + min(16384, -(-rows * cut // 4))] if cut else []), hint
         torch.cuda.synchronize()
         got.append((st.combine_send_slots.view(torch.int16).clone(), out))
     assert not torch.equal(got[0][0], torch.full_like(got[0][0], 0x7FC0))
