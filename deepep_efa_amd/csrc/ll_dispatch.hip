@@ -118,8 +118,15 @@ constexpr int kSendMaxWaves = 16;
 //   step, 1000 x 2048     39.2 / 36.3     exchange, 1000 x 2048  47.2 / 44.8     step, 509 x 4096  23.5 / 23.8 and 24.4 / 23.9
 //   700 x 2048            28.6 / 27.4     700 x 2048             38.4 / 36.8     400 x 4096, in 200 workgroups  28.6 / 30.2
 //   900 x 2048, top-6     31.2 / 29.7     1000 x 5120            91.1 / 87.6     700 x 4096        42.0 / 41.7
-//   500 x 2048            22.2 / 21.4     512 x 7168             65.5 / 64.4     1000 x 4096       57.5 / 57.4
+//   500 x 2048            22.2 / 21.4                                            1000 x 4096       57.5 / 57.4
+// A send of its own fits two tokens in up to sixteen waves.  In more than eight of them it pays from 480 workgroups and 4096
+// entries on, in twelve, and in sixteen by destination, whose tokens go through all entries; fourteen leave four of a compute
+// unit's places empty.  Microseconds of the send alone, one token a workgroup / two, staged and by destination:
+//   960 x 3072     9.7 /  9.3  10.7 /  9.4     1000 x 4096  10.8 / 10.8  12.3 / 11.1     1000 x 7168        14.8 / 14.3  15.8 / 15.4
+//   1000 x 5120   11.8 / 11.6  14.4 / 13.0     600 x 4096    8.3 /  9.1   8.7 / 10.1     2000 x 7168, top-4 16.5 / 19.0  18.8 / 20.3
+//   600 x 3072     7.7 /  8.0   8.2 /  8.0     1500 x 5120, top-2  8.6 / 9.1  10.0 / 9.9    600 x 7168       10.0 / 11.6  11.2 / 11.7
 constexpr int kManyBlocks = 240;
+constexpr int kTwoTokensFrom = 4096;  // entries
 
 struct ByDestTables {
     int32_t* expert_prefix;  // [E + 1]
@@ -1308,6 +1315,9 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     int tokens_per_block = 1;
     if (!ranked && blocks_per_token == 1 && (fused_recv == nullptr || items <= kFusedManyPieces))
         tokens_per_block = tokens_per_send_block(items, max_waves, num_topk, num_tokens);
+    if (fused_recv == nullptr && 2 * items > 8 &&
+        (n < kTwoTokensFrom || num_tokens < 4 * kManyBlocks || (items > 6 && (items != 8 || by_dest == nullptr))))
+        tokens_per_block = 1;
     const int token_blocks = (num_tokens + tokens_per_block - 1) / tokens_per_block;
     if (tokens_per_block > 1) waves = std::max(waves, items * tokens_per_block);
     // floor(e / E_l) == umulhi(e, ceil(2^32 / E_l)) for every e below 2^16.

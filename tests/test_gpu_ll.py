@@ -113,14 +113,15 @@ def takes_one_launch(rt, st, t):
 
 
 def kernels_launched(call, tmp_path):
-    """The low-latency kernels of a call and their workgroups (along x), by the nodes of a captured graph."""
+    """The low-latency kernels of a call and their workgroups, by the nodes of a captured graph."""
     graph = torch.cuda.CUDAGraph(keep_graph=True)
     graph.enable_debug_mode()
     torch.cuda.synchronize()
     with torch.cuda.graph(graph):
         call()
     graph.debug_dump(str(tmp_path / "graph.dot"))
-    return {name: int(blocks) for name, blocks in re.findall(r"(ll_[a-z_]*?kernel)[^\n(]*\((\d+),", (tmp_path / "graph.dot").read_text())}
+    found = re.findall(r"(ll_[a-z_]*?kernel)[^\n(]*\((\d+),(\d+),(\d+)\)", (tmp_path / "graph.dot").read_text())
+    return {name: int(x) * int(y) * int(z) for name, x, y, z in found}
 
 
 def check_dispatch(st, want, fmt):
@@ -1267,6 +1268,28 @@ def test_several_tokens_a_workgroup(rt, t, k, h, fmt):
     got, _ = dispatch_on_gpu(rt, x_all, topk_all, rank, e, m, fmt, one_call=True)
     check_dispatch(got, O.ll_dispatch(list(x_all), list(topk), rank, e, m, fmt), fmt)
     assert torch.equal(got.pair_slot.cpu().view(-1)[:t * k], st.pair_slot.cpu().view(-1)[:t * k])
+
+
+@pytest.mark.parametrize("t,k,h,fmt,staged,by_dest", [
+    (479, 8, 2048, O.ROW_FP8, 1, 1), (480, 8, 2048, O.ROW_FP8, 2, 2), (960, 8, 2048, O.ROW_FP8, 4, 4),  # four waves a token
+    (959, 8, 3072, O.ROW_FP8, 1, 1), (960, 8, 3072, O.ROW_FP8, 2, 2),  # six: from 480 workgroups
+    (1365, 3, 2560, O.ROW_FP8, 1, 1), (1365, 4, 2560, O.ROW_FP8, 2, 2),  # and 4096 entries
+    (1000, 8, 7168, O.ROW_FP8, 1, 1), (600, 8, 7168, O.ROW_FP8, 1, 1),  # seven
+    (959, 8, 4096, O.ROW_FP8, 1, 1), (960, 8, 4096, O.ROW_FP8, 1, 2), (1000, 8, 4096, O.ROW_BF16, 1, 2),  # eight
+    (1000, 8, 4224, O.ROW_FP8, 2, 2), (1024, 8, 4096, O.ROW_FP8, 4, 4)])  # five, and four again
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
+def test_tokens_of_a_send_workgroup(rt, t, k, h, fmt, staged, by_dest, tmp_path):
+    """How many tokens a workgroup of a send takes, by the workgroups of its launch; the slots are the same."""
+    r, rank, e = 4, 2, 64
+    x_all, topk_all, _ = make_world(r, t, h, k, e, seed=t + k, drop=20)
+    x, topk = x_all[rank].cuda(), topk_all[rank].cuda()
+    send_count, pair_slot = O.route(topk_all[rank], e, t)
+    shape = rt.ll.LLShape(r, rank, e, t, h, k, fmt)
+    for st, tokens in ((rt.ll.LowLatencyState(shape), staged), (rt.ll.AllToAllState(shape), by_dest)):
+        launched = kernels_launched(lambda: st.dispatch_send(x, topk), tmp_path)
+        assert launched == {"ll_send_kernel": -(-t // tokens) + 1}
+        st.dispatch_send(x, topk)
+        assert torch.equal(st.send_count.cpu(), send_count) and torch.equal(st.pair_slot[:t].cpu(), pair_slot)
 
 
 @pytest.mark.parametrize("t,k,h,fmt", [
