@@ -5,6 +5,8 @@
 #include "common.hpp"
 #include "../../include/deepep_hip.h"
 
+#include <algorithm>
+
 namespace deepep {
 
 constexpr int kLayoutThreads = 256;
@@ -19,7 +21,13 @@ constexpr int kLayoutOneBlockThreads = 1024;
 //   1500         4.3 / 4.3    5.0 / 4.6    6.0 / 4.9    10.3 / 5.5
 //   2048         4.4 / 4.5    5.3 / 4.8    6.4 / 5.1    11.4 / 5.9
 //   3000         5.6 / 4.7    6.8 / 4.9    8.5 / 5.2    16.6 / 6.0
-inline int layout_one_block_tokens(int num_ranks) { return num_ranks <= 8 ? 2048 : num_ranks <= 32 ? 1024 : 768; }
+// Past 1024 tokens up to 16384 entries, which one workgroup takes one after another (8 ranks, 2048 tokens, top-8 4.9 / 5.0, top-12
+// 5.7 / 5.3, top-16 10.4 / 6.8, top-32 17.9 / 8.5), and past 512 with more than 32 ranks only of whole eights, whose bytes are stored a
+// word at a time (63 ranks, 768 tokens 9.2 / 7.1; 250 ranks, 700 tokens 27.1 / 16.1).
+inline int layout_one_block_tokens(int num_ranks, int num_topk) {
+    if (num_ranks <= 8) return std::min(2048, std::max(1024, 16384 / num_topk));
+    return num_ranks <= 32 ? 1024 : num_ranks % 8 == 0 ? 768 : 512;
+}
 
 // Spreads the 8 bits of b into 8 bytes (byte i = bit i, value 0 or 1).
 __device__ __forceinline__ uint64_t bits_to_bool_bytes(uint32_t b) {
@@ -40,6 +48,20 @@ __device__ __forceinline__ int byte_sums_to_lanes(uint64_t v, int first, int oth
     const uint32_t hi = __builtin_amdgcn_readlane(wave_inclusive_sum(int(uint32_t(v >> 32))), kWave - 1);
     const int i = lane_id() - first;
     return i >= 0 && i < 8 ? int((((i & 4) != 0 ? hi : lo) >> ((i & 3) * 8)) & 0xff) : otherwise;
+}
+
+// e / E_l by multiply-high (exact below 2^16 experts); magic 0 stands for E_l == 1.
+__device__ __forceinline__ int rank_of_expert(uint32_t e, uint32_t rank_magic) {
+    return rank_magic != 0 ? int(__umulhi(e, rank_magic)) : int(e);
+}
+
+// Counts the expert that entry 0 or 1 of two names and marks its rank, one of up to 64.
+__device__ __forceinline__ void count_entry(u32x4 two, int which, int num_experts, uint32_t rank_magic, int32_t* hist,
+                                            uint64_t& member) {
+    const uint32_t e = two[which * 2];
+    if (two[which * 2 + 1] != 0u || e >= uint32_t(num_experts)) return;
+    atomicAdd(&hist[e], 1);
+    member |= uint64_t(1) << (rank_of_expert(e, rank_magic) & 63);
 }
 
 // ---------------------------------------------------------------------
@@ -84,35 +106,54 @@ __global__ __launch_bounds__(kLayoutOneBlockThreads) void layout_count_kernel(
         const auto rows = row_buffer(reinterpret_cast<const uint8_t*>(topk_idx + int64_t(t0) * num_topk), tokens * num_topk * 8);
         for (int k0 = 0; k0 < num_topk; k0 += 8) {
             u32x4 two[4];  // all in flight before the first is used
+            const auto load = [&](int u) { two[u] = load_row_u32x4<false>(rows, (tid * num_topk + k0 + 2 * u) * 8); };
+            if constexpr (kRankWords == 1) {
+                if (k0 + 8 <= num_topk) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) two[u] = load_row_u32x4<false>(rows, (tid * num_topk + k0 + 2 * u) * 8);
+                    for (int u = 0; u < 4; ++u) load(u);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t e = two[u / 2][u % 2 * 2];
-                if (two[u / 2][u % 2 * 2 + 1] != 0u || e >= uint32_t(num_experts) || k0 + u >= num_topk || t >= num_tokens) continue;
-                atomicAdd(&hist[e], 1);
-                // e / E_l by multiply-high (exact below 2^16 experts); magic 0 stands for E_l == 1
-                const int r = rank_magic != 0 ? int(__umulhi(e, rank_magic)) : int(e);
+                    for (int u = 0; u < 8; ++u)
+                        if (t < num_tokens) count_entry(two[u / 2], u % 2, num_experts, rank_magic, hist, member[0]);
+                } else {  // no more loads and tests than there are entries: 8 ranks, 1024 tokens, top-2 3.2 -> 2.9 us
 #pragma unroll
-                for (int q = 0; q < kRankWords; ++q)
-                    if (kRankWords == 1 || (r >> 6) == q) member[q] |= uint64_t(1) << (r & 63);
+                    for (int u = 0; u < 4; ++u) {
+                        if (k0 + 2 * u >= num_topk) break;
+                        load(u);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        if (k0 + u >= num_topk) break;
+                        if (t < num_tokens) count_entry(two[u / 2], u % 2, num_experts, rank_magic, hist, member[0]);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) load(u);
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const uint32_t e = two[u / 2][u % 2 * 2];
+                    if (two[u / 2][u % 2 * 2 + 1] != 0u || e >= uint32_t(num_experts) || k0 + u >= num_topk || t >= num_tokens) continue;
+                    atomicAdd(&hist[e], 1);
+                    const int r = rank_of_expert(e, rank_magic);
+#pragma unroll
+                    for (int q = 0; q < kRankWords; ++q)
+                        if ((r >> 6) == q) member[q] |= uint64_t(1) << (r & 63);
+                }
             }
         }
         // lane r keeps rank (q * 64 + r)'s count of the wave, so that one atomic per lane adds them all
         uint8_t* out = is_token_in_rank + int64_t(t) * num_ranks;
+        const bool in_words = (num_ranks & 7) == 0;
 #pragma unroll
         for (int q = 0; q < kRankWords; ++q) {
             const int begin = q * kWave, end = num_ranks < begin + kWave ? num_ranks : begin + kWave;
             int count = 0;
+            if (!in_words && t < num_tokens)
+                for (int r = begin; r < end; ++r) out[r] = uint8_t((member[q] >> (r - begin)) & 1);
             for (int r8 = begin; r8 < end; r8 += 8) {
                 const uint64_t in = bits_to_bool_bytes(uint32_t(member[q] >> (r8 - begin)));
                 count = byte_sums_to_lanes(in, r8 - begin, count);
-                if (t >= num_tokens) continue;
-                if ((num_ranks & 7) == 0) {
-                    *reinterpret_cast<uint64_t*>(out + r8) = in;
-                } else {
-                    for (int i = 0; i < 8 && r8 + i < end; ++i) out[r8 + i] = uint8_t(in >> (8 * i));
-                }
+                if (in_words && t < num_tokens) *reinterpret_cast<uint64_t*>(out + r8) = in;
             }
             if (count != 0) atomicAdd(&hist[num_experts + begin + lane], count);
             if (q * 8 < num_nodes) {  // 8 ranks per node (reference: NUM_MAX_NVL_PEERS, csrc/kernels/configs.cuh:3)
@@ -760,7 +801,7 @@ int deepep_get_dispatch_layout(const int64_t* topk_idx, int num_tokens, int num_
     EP_HOST_ASSERT(size_t(width) * 4 <= 64 * 1024);
     const int partials = num_tokens == 0 ? 1 : (num_tokens + kLayoutThreads - 1) / kLayoutThreads;
     EP_HOST_ASSERT(workspace != nullptr && workspace_bytes >= size_t(partials) * width * 4);
-    const int blocks = num_tokens <= layout_one_block_tokens(num_ranks) ? 1 : partials;
+    const int blocks = num_tokens <= layout_one_block_tokens(num_ranks, num_topk) ? 1 : partials;
     const int threads = blocks == 1 && num_tokens > kLayoutThreads ? kLayoutOneBlockThreads : kLayoutThreads;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     int32_t* partial = reinterpret_cast<int32_t*>(workspace);

@@ -4,6 +4,7 @@ Every call goes through the C ABI (ctypes on libdeepep_hip.so); the expected
 values come from the CPU oracle.  Integer and byte outputs must be bit-exact.
 """
 import os
+import re
 
 import numpy as np
 import pytest
@@ -206,6 +207,35 @@ def test_layout_counts_ranks_and_nodes(capi, t, r, e, k, shift):
     want = O.get_dispatch_layout(torch.where((topk >= 0) & (topk < e), topk, -1), e, r)
     assert torch.equal(per_rank.cpu(), want[0]) and torch.equal(per_expert.cpu(), want[2])
     assert not nodes or torch.equal(per_node.cpu(), want[1])
+    assert torch.equal(is_in[:t].cpu(), want[3].to(torch.uint8)) and (is_in[t] == 7).all()
+
+
+@pytest.mark.parametrize("t,r,k,launches", [
+    (2048, 8, 8, 1), (2049, 8, 8, 2), (1365, 8, 12, 1), (1366, 8, 12, 2), (1024, 4, 32, 1), (1025, 4, 32, 2),  # up to 16384 entries
+    (1024, 20, 16, 1), (1025, 20, 16, 2), (768, 64, 5, 1), (769, 64, 5, 2), (512, 63, 9, 1), (513, 63, 9, 2),
+    (512, 100, 8, 1), (513, 100, 8, 2)])
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
+def test_layout_in_one_launch_and_in_two(capi, t, r, k, launches, tmp_path):
+    """Which batches one workgroup counts, by the nodes of a captured graph; the oracle's counts either way."""
+    lib, e = capi.load(), r * max(4, 40 // r)
+    topk = _topk(t, k, e, seed=t + r, drop=9)
+    dev = topk.cuda()
+    per_rank, per_expert = (torch.full((n,), -1, dtype=torch.int32, device="cuda") for n in (r, e))
+    is_in = torch.full((t + 1, r), 7, dtype=torch.uint8, device="cuda")
+    ws = torch.empty(lib.deepep_layout_workspace_bytes(t, r, e), dtype=torch.uint8, device="cuda")
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    graph.enable_debug_mode()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        capi.check(lib.deepep_get_dispatch_layout(capi.ptr(dev), t, k, r, e, capi.ptr(per_rank), None, capi.ptr(per_expert),
+                                                  capi.ptr(is_in), capi.ptr(ws), ws.numel(), stream()))
+    graph.debug_dump(str(tmp_path / "graph.dot"))
+    assert len(re.findall(r"layout_[a-z]+_kernel", (tmp_path / "graph.dot").read_text())) == launches
+    graph.instantiate()
+    graph.replay()
+    torch.cuda.synchronize()
+    want = O.get_dispatch_layout(topk, e, r)
+    assert torch.equal(per_rank.cpu(), want[0]) and torch.equal(per_expert.cpu(), want[2])
     assert torch.equal(is_in[:t].cpu(), want[3].to(torch.uint8)) and (is_in[t] == 7).all()
 
 
