@@ -189,8 +189,10 @@ extern "C" int deepep_ll_exchange_metadata(const int32_t* all_num_routed, int nu
     EP_HOST_ASSERT(combine_remote_recv_offset != nullptr && num_recv_tokens != nullptr && tokens_per_expert != nullptr);
     EP_HOST_ASSERT(row_capacity == 0 || (source_rank != nullptr && source_offset != nullptr &&
                                          padded_index != nullptr && combine_send_offset != nullptr));
-    int64_t records = (row_capacity + 8 * kExchangeThreads - 1) / (8 * kExchangeThreads);  // workgroups for them
-    records = records > 64 ? 64 : records;
+    // Workgroups for the records, one after another for a thread: 8 ranks x 256 experts, 3800 rows of 4096 4.4 -> 5.1 us with
+    // eight a thread, 8 x 64, 256000 of 300000 5.3 -> 7.8 with 64 workgroups.
+    int64_t records = (row_capacity + 4 * kExchangeThreads - 1) / (4 * kExchangeThreads);
+    records = records > 256 ? 256 : records;
     const int64_t blocks = 1 + (num_ranks + kExchangeWaves - 1) / kExchangeWaves + records;
     launch(ll_exchange_meta_kernel, unsigned(blocks), kExchangeThreads, 0, reinterpret_cast<hipStream_t>(stream),
         all_num_routed, num_experts, num_ranks, rank, num_max_dispatch_tokens_per_rank, row_capacity, send_counts,

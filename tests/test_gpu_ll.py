@@ -301,6 +301,34 @@ def test_exchange_metadata_of_every_count(rt, r, e, rank, capacity):
             assert out[key][:n].cpu().tolist() == want[key][:n].tolist(), key
 
 
+@pytest.mark.parametrize("capacity,record_blocks", [(0, 0), (1024, 1), (1025, 2), (262144, 256), (300000, 256)])
+@pytest.mark.filterwarnings("ignore:DEBUG")  # the graph is written out
+def test_exchange_metadata_workgroups(rt, capacity, record_blocks, tmp_path):
+    """A workgroup for every 1024 records there is room for, up to 256: full to the last record."""
+    r, e, rank, m = 6, 48, 4, 8192
+    routed = torch.randint(5000, 6300, (r, e), generator=torch.Generator().manual_seed(capacity), dtype=torch.int32)
+    dev, lib, capi = routed.cuda(), rt.capi.load(), rt.capi
+    out = {name: torch.full((max(1, n),), -7, dtype=torch.int64 if name == "combine_remote_recv_offset" else torch.int32, device="cuda")
+           for name, n in (("send_counts", r), ("recv_counts", r), ("totals", 3), ("combine_remote_recv_offset", r),
+                           ("source_rank", capacity), ("source_offset", capacity), ("padded_index", capacity),
+                           ("combine_send_offset", capacity), ("num_recv_tokens", 2), ("tokens_per_expert", e // r))}
+
+    def call():
+        capi.check(lib.deepep_ll_exchange_metadata(capi.ptr(dev), e, r, rank, m, capacity, *(capi.ptr(v) for v in out.values()),
+                                                   torch.cuda.current_stream().cuda_stream))
+
+    assert kernels_launched(call, tmp_path) == {"ll_exchange_meta_kernel": 1 + 2 + record_blocks}
+    call()
+    torch.cuda.synchronize()
+    want = O.ll_exchange_metadata(routed, rank, m)
+    n = min(want["total_recv"], capacity)
+    assert n == min(capacity, int(routed[:, rank * (e // r):(rank + 1) * (e // r)].sum()))
+    assert out["num_recv_tokens"].cpu().tolist() == [want["total_recv"], n]
+    for key in ("source_rank", "source_offset", "padded_index", "combine_send_offset"):
+        assert torch.equal(out[key][:n].cpu().long(), torch.as_tensor(want[key][:n]).long()), key
+        assert (out[key][n:] == -7).all()
+
+
 def test_exchange_metadata_hand_derived_world(rt):
     g, _, _ = load_tiny_world()
     routed = torch.tensor(g["all_num_routed"], dtype=torch.int32)
