@@ -842,7 +842,8 @@ size_t deepep_routing_sort_workspace_bytes(int num_tokens, int num_ranks) {
 // 7.2 against 16.5 before the wide form's own time was halved; 24 ranks, 12289 7.8 against 34.2), past that its work
 // grows with the square of the batch.
 static bool sort_is_wide(const uint8_t* is_token_in_rank, int num_tokens, int num_ranks) {
-    const int from = num_ranks == 8 ? 1024 : num_ranks == 16 ? 1280 : 2048;
+    // (up to 2048 tokens a thread of one workgroup per rank has two: 24 ranks 5.7 / 5.5, 40 ranks 7.8 / 7.4, 56 ranks 10.1 / 10.6)
+    const int from = num_ranks == 8 ? 1024 : num_ranks == 16 ? 1280 : num_ranks == 24 || num_ranks == 40 ? 2049 : 2048;
     return num_ranks % 8 == 0 && num_ranks <= 64 && (reinterpret_cast<uintptr_t>(is_token_in_rank) & 7) == 0 &&
            num_tokens >= from && int64_t(num_tokens) * num_ranks <= kWideSortMaxBytes;
 }

@@ -308,12 +308,14 @@ def test_routing_sort_reports_every_workgroup(capi, t, r):
     assert int(report[words - 1]) == int(is_in.sum()) == int(cumsum[r])
 
 
-@pytest.mark.parametrize("t,r", [(1, 8), (131, 16), (2000, 64), (4096, 48)])
-def test_routing_sort_takes_the_form_measured_fastest(capi, t, r):
-    """One workgroup per rank up to 2047 tokens (1023 at 8 ranks, 1279 at 16), where the form that adds up eight ranks at
-    a time is up to twice as slow; a matrix whose address does not allow 8-byte loads never takes that form."""
+@pytest.mark.parametrize("t,r,wide", [(1, 8, 0), (1023, 8, 0), (1024, 8, 1), (131, 16, 0), (1279, 16, 0), (1280, 16, 1), (2048, 24, 0),
+                                      (2049, 24, 1), (2047, 32, 0), (2048, 32, 1), (2048, 40, 0), (2049, 40, 1), (2047, 48, 0),
+                                      (4096, 48, 1), (2047, 56, 0), (2048, 56, 1), (2000, 64, 0), (2047, 64, 0), (2048, 64, 1)])
+def test_routing_sort_takes_the_form_measured_fastest(capi, t, r, wide):
+    """One workgroup per rank up to 2047 tokens (1023 at 8 ranks, 1279 at 16, 2048 at 24 and 40), where the form that adds up
+    eight ranks at a time is up to twice as slow; a matrix whose address does not allow 8-byte loads never takes that form."""
     lib = capi.load()
-    assert lib.deepep_routing_sort_report_words(None, t, r) == (r if t < 4096 else (t + 255) // 256)
+    assert lib.deepep_routing_sort_report_words(None, t, r) == ((t + 255) // 256 if wide else r)
     assert lib.deepep_routing_sort_report_words(4, t, r) == r
     is_in = torch.rand((t, r), generator=torch.Generator().manual_seed(t + r)) < 0.3
     shifted = torch.zeros(t * r + 4, dtype=torch.bool, device="cuda")[4:].view(t, r)
