@@ -613,6 +613,8 @@ def test_dispatch_and_combine_replay_in_a_hip_graph(deep_ep, num_ranks, rank, t,
     """Decode loops capture the dispatch + combine pair once and replay it.  The captured calls must
     allocate nothing and record no memset; every replay, with eager work and synchronisations in
     between, must give the eager result."""
+    from deepep_efa_amd import _capi
+    assert _capi.load().deepep_ll_dispatch_takes_one_launch(t, h, k, e, t, 1, t * k) == (t == 64)
     buffer = deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=num_ranks,
                             sim_rank=rank, sim_seed=21)
     x, topk_idx = buffer.loopback_synthesise(t, h, k, e)
@@ -689,7 +691,8 @@ def test_the_bound_methods_give_what_the_wrappers_give(deep_ep, use_fp8):
 def test_batches_that_change_from_call_to_call(deep_ep):
     """Uneven, skewed and balanced batches in turn through one buffer, each sized by the one before, give what a
     buffer of their own gives; they take the single launch and the index + copy form in both directions."""
-    num_ranks, rank, m, h, k, e = 16, 0, 640, 512, 8, 64
+    from deepep_efa_amd import _capi
+    num_ranks, rank, m, h, k, e = 16, 0, 640, 4096, 8, 64
 
     def make():
         return deep_ep.Buffer(None, low_latency_mode=True, explicitly_destroy=True, sim_num_ranks=num_ranks,
@@ -725,7 +728,7 @@ def test_batches_that_change_from_call_to_call(deep_ep):
         alone.destroy()
         received.append(int(want[0].sum()))
         assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want)), (key, own)
-    assert min(received) < 8192 < max(received)
+    assert min(received) < 8192 and not _capi.load().deepep_ll_dispatch_takes_one_launch(4, h, k, e, m, 1, max(received))
     shared.destroy()
 
 

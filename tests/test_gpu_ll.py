@@ -146,8 +146,8 @@ def check_dispatch(st, want, fmt):
     (4, 1, 40, 512, 9, 64),    # K > 8
     (2, 1, 600, 512, 8, 16),   # a mid-sized batch: the send side sweeps every earlier entry, in the single launch too
     (4, 3, 300, 512, 11, 32),  # both
-    (2, 0, 1100, 512, 8, 16),  # T*K > 8192: chunk histograms under the send kernel's sweep, small receive path
-    (8, 5, 4200, 512, 4, 64),  # more than 8192 expected rows: receive runs as index kernel + flat row copy
+    (2, 0, 1500, 512, 8, 16),  # more entries than one launch takes: chunk histograms ahead of the send, index kernel + flat row copy
+    (8, 5, 4200, 512, 4, 64),  # the same on 8 ranks
     (8, 2, 20, 512, 4, 512),   # more than 256 segments: 16 counts per lane in the register segment table
     (16, 9, 12, 512, 6, 1024),  # the most experts the path takes
     (1, 0, 16, 512, 2, 4),     # a world of one rank: every row is the rank's own
@@ -1020,7 +1020,7 @@ def test_exchange_metadata_through_the_host_module(rt):
 @pytest.mark.parametrize("hint", ["batch", "unknown", "huge"])
 def test_capacity_far_above_the_batch(rt, hint):
     """A caller may size M for its largest batch and dispatch a small one.  The kernels are picked from the
-    expected-rows hint, not from the capacity, and every hint gives the same result."""
+    expected-rows hint or, without one, a thirty-second of the capacity, and every hint gives the same result."""
     r, rank, t, m, h, k, e = 8, 2, 40, 5000, 512, 4, 64
     x_all, topk_all, w_all = make_world(r, t, h, k, e, seed=4242, drop=7)
     shape = rt.ll.LLShape(num_ranks=r, rank=rank, num_experts=e, max_tokens=m, hidden=h, num_topk=k, fmt=O.ROW_FP8)
@@ -1035,6 +1035,7 @@ def test_capacity_far_above_the_batch(rt, hint):
     run_dispatch(st, world, x, topk, None, one_call=True)
     single = rt.capi.load().deepep_ll_dispatch_is_single_launch(t, k, e, m, st.expected_rows) == 1
     assert single == (hint == "batch")
+    assert takes_one_launch(rt, st, t) == (hint != "huge")
     want = O.ll_dispatch(list(x_all), list(topk_all), rank, e, m, O.ROW_FP8)
     check_dispatch(st, want, O.ROW_FP8)
     # combine with identity experts
@@ -1513,7 +1514,8 @@ def test_one_call_dispatch_of_few_entries_and_many_rows(rt, rank):
     want = O.ll_dispatch(x_all, topk.contiguous(), rank, e, t, O.ROW_FP8)
     shape = rt.ll.LLShape(num_ranks=r, rank=rank, num_experts=e, max_tokens=t, hidden=h, num_topk=k, fmt=O.ROW_FP8)
     st = rt.ll.LowLatencyState(shape)
-    st.expected_rows = 8193
+    st.expected_rows = 96 * 1024 + 1
+    assert not takes_one_launch(rt, st, t)
     st.segment_workspace = torch.empty(rt.capi.load().deepep_ll_segment_workspace_bytes(e, t), dtype=torch.uint8,
                                        device="cuda")
     world = rt.lb.LoopbackWorld(r, rank, seed=0)
@@ -1524,7 +1526,7 @@ def test_one_call_dispatch_of_few_entries_and_many_rows(rt, rank):
     check_dispatch(st, want, O.ROW_FP8)
 
 
-@pytest.mark.parametrize("t,k,e,rows", [(300, 8, 64, 8193), (1100, 8, 64, 0), (1100, 8, 64, 9000), (1171, 7, 96, 9000),
+@pytest.mark.parametrize("t,k,e,rows", [(300, 8, 64, 99000), (1500, 8, 64, 0), (1500, 8, 64, 12000), (1611, 7, 96, 12000),
                                         (8300, 8, 64, 70000)])  # the last of more than 32 chunks
 def test_workspace_that_holds_the_chunk_histograms_alone(rt, t, k, e, rows):
     """ceil(T / floor(2048 / K)) * E * 4 bytes, rounded up to 256, for each source: every send works with them."""
@@ -1546,6 +1548,7 @@ def test_workspace_that_holds_the_chunk_histograms_alone(rt, t, k, e, rows):
     def dispatch(small):
         st = rt.ll.LowLatencyState(rt.ll.LLShape(num_ranks=r, rank=rank, num_experts=e, max_tokens=t, hidden=h, num_topk=k, fmt=fmt))
         st.expected_rows = rows
+        assert not takes_one_launch(rt, st, t)
         st.segment_workspace = (torch.empty(lib.deepep_ll_segment_workspace_bytes(e, t), dtype=torch.uint8, device="cuda")
                                 if rows > 0 else None)
         world = rt.lb.LoopbackWorld(r, rank, seed=0)

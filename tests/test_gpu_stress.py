@@ -48,7 +48,9 @@ def run_skew_stress(r, rank, t, h, k, e, seed, one_call):
     world = loopback.LoopbackWorld(r, rank, seed=seed)
     world.synthesise(t, h, k, e, popularity="zipf", outlier_period=100)
     x, topk = world.own_inputs()
-    if one_call:  # peers' rows first, then send + receive in one call
+    if one_call:  # peers' rows first, then send + receive in one call, sized by what arrives
+        st.expected_rows = int((world.topk_idx_all // epr == rank).sum())
+        assert not _capi.load().deepep_ll_dispatch_takes_one_launch(t, h, k, e, t, shape.fmt, st.expected_rows)
         world.dispatch_from_peers(st)
         st.dispatch(x, topk)
     else:
