@@ -90,20 +90,23 @@ __device__ __forceinline__ void emit_expert_count(int e, int total, int num_expe
 // (reference idea: csrc/kernels/coop_dispatch_send.cuh:572-607).
 //
 // Per-selection bookkeeping (slot, destination row address, row tail,
-// pair_slot) is done once per token by lanes 0..K-1 of wave 0 and handed to the
-// other waves through LDS; each wave reads all K destinations with one LDS
-// access and takes them back per selection with readlane.  Quantisation runs
+// pair_slot) is done once per workgroup by the first lanes of wave 0, one for
+// each selection of its one, two or four tokens (at most 64), and handed to the
+// other waves through LDS; each wave reads its token's K destinations with one
+// LDS access and takes them back per selection with readlane.  Quantisation runs
 // while wave 0 does that.  Barriers fence LDS only, so the row loads stay in
 // flight across them.
 //
 // The slot of a selection is the number of earlier (token,k) entries naming its
 // expert (reference: the serial scan of csrc/kernels/efa_kernels.cu:617-637 and
 // token_offset / expert_offsets of csrc/kernels/coop_dispatch_send.cuh:360-420).
-// Up to 8192 entries the workgroup counts them itself: while the row loads are in
-// flight every thread fetches up to four entries that precede the token (more in a
-// loop) and adds them to a histogram by expert in LDS; the per-expert totals come
-// from one extra workgroup per source.  Larger batches get their slots from
-// ll_rank_chunk_kernel, one launch ahead.  Deterministic: integer adds only.
+// Up to kSelfRankMaxEntries entries, and in the single-launch dispatch for as many
+// as dispatch_in_one_launch() lets it have, the workgroup counts them itself: while
+// the row loads are in flight every thread fetches up to four entries that precede
+// the token (more in a loop) and adds them to a histogram by expert in LDS; the
+// per-expert totals come from one extra workgroup per source.  Larger batches get
+// their slots from ll_rank_chunk_kernel, one launch ahead.  Deterministic: integer
+// adds only.
 // ---------------------------------------------------------------------
 constexpr int kMaxTopk = 64;
 constexpr int kFusedMaxEntries = 8192;     // send + receive in one launch up to here, whatever the rows
@@ -140,7 +143,7 @@ struct SendArgs {
     const int32_t* src_ranks;  // null: the rows are this rank's own
     int num_tokens, hidden, num_topk, num_experts, num_ranks, rank, max_tokens;
     int pieces_per_row, split_log2;
-    int tokens_per_block;  // 2 or 4: whole tokens, pieces_per_row << split_log2 waves each
+    int tokens_per_block;  // 1, 2 or 4: whole tokens, pieces_per_row << split_log2 waves each
     RankDivider token_of;  // a workgroup's entry to the token among its own: division by K
     uint32_t rank_of_expert_magic;
     uint8_t* recv_staging;
@@ -1304,8 +1307,9 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
     // for is worth its place (256 tokens, top-8 15.9 -> 15.1 us, 1024 tokens 40.9 -> 39.6; 128 tokens 8.0 -> 8.1).
     if (fused_recv != nullptr && n > 1536 && waves > 4) waves = 8;
     // A row of several workgroups is cut evenly in the single launch where that does without two waves or more of each: the
-    // waves that have no piece take others' places on the chip.  Past 1792 entries they pay for it with what they do for the
-    // sweeps.  Microseconds of a step in bf16, eight waves / five (six at hidden 6144), top-8 to 32 ranks:
+    // waves that have no piece take others' places on the chip.  Past 1792 entries a step has lost by it, in other worlds than
+    // those in which it gained below; the dispatch alone gains past them too (300 x 5120 to 8 13.9 / 12.9, 400 at top-6 13.8 /
+    // 12.1, 1000 41.3 / 39.9; 260 x 6144 12.7 / 13.4).  Microseconds of a step in bf16, eight waves / five (six at hidden 6144), top-8 to 32 ranks:
     //   100 x 5120 to 8    16.7 / 16.2    128 x 5120  21.8 / 20.6    180 to 16  28.0 / 26.3    220  30.6 / 29.5
     //   190 x 4608 to 64   28.8 / 27.3    150 x 6144  27.6 / 26.6    16 and 60  12.2 and 14.4 either way
     //   250 x 5120 to 64   28.1 / 28.7    400 to 8    39.0 / 39.9    1000 to 8  91.0 / 92.7; seven of eight, 128 x 7168 26.7 / 27.0
@@ -1356,7 +1360,8 @@ static int launch_send_side(const void* x, const int64_t* topk_idx, const int32_
         //   580 x 4096   36.7 / 35.1    700 x 4096  42.2 / 40.8    820 x 4096  49.7 / 47.5    936 x 4096, top-6  44.6 / 43.1
         //   1000 x 4096  56.1 / 55.4    600 x 2048 bf16  30.3 / 29.7    900 x 2048 bf16  36.9 / 35.6    1500 x 4096, top-4  49.1 / 48.6
         //   400 x 4096   28.4 / 28.3    500 x 2048 bf16  23.8 / 24.6    1100 x 2048 bf16  44.7 / 45.6    2000 x 4096, top-4  58.9 / 60.0
-        // Workgroups of eight waves: 340 x 7168 bf16 47.6 / 48.2, 1000 x 7168 93.3 / 94.0.
+        // Workgroups of eight waves: 340 x 7168 bf16 47.6 / 48.2, 1000 x 7168 93.3 / 94.0.  Where far more rows come in than the
+        // batch sends, three launches against one with 512: 1000 of 2048, 14900 rows 23.5 / 15.3; 600 of 4096, 14500 33.2 / 24.1.
         const bool few = waves <= 4 && n > kFusedFewFrom && n <= kFusedMaxEntries && num_tokens <= kFusedFewTokens;
         const int64_t most = tokens_per_block > 1 || few ? 512 : 1024;
         fused_recv_blocks = fused_recv_blocks < 1 ? 1 : (fused_recv_blocks > most ? most : fused_recv_blocks);
