@@ -102,13 +102,23 @@ __global__ __launch_bounds__(kExchangeThreads) void ll_exchange_meta_kernel(
     }
     const uint64_t bad = __ballot(most > max_per_expert);
     if (lane == 0) wave_found[w] = bad != 0 ? 1u : 0u;
+    // Lanes of one rank would wait for one another at its word: where a wave's are all of one, it hands in their sum (8 ranks x
+    // 1024 experts 4.3 -> 3.8 us, 8 x 4096 10.9 -> 9.7).
+    const bool waves_of_one_rank = experts_per_rank % kWave == 0;
+    const auto add = [&](int32_t* to, uint32_t i, int count) {
+        if (waves_of_one_rank) {
+            count = wave_inclusive_sum(count);
+            if (lane != kWave - 1) return;
+        }
+        atomicAdd(&to[i / experts_per_rank], count);
+    };
     if (uint32_t(tid) < experts) {
-        atomicAdd(&recv_of[tid / experts_per_rank], received);
-        if (writes_totals) atomicAdd(&send_to[tid / experts_per_rank], sent);
+        add(recv_of, tid, received);
+        if (writes_totals) add(send_to, tid, sent);
     }
     for (uint32_t i = tid + kExchangeThreads; i < experts; i += kExchangeThreads) {
-        atomicAdd(&recv_of[i / experts_per_rank], *to_me(i));
-        if (writes_totals) atomicAdd(&send_to[i / experts_per_rank], mine[i]);
+        add(recv_of, i, *to_me(i));
+        if (writes_totals) add(send_to, i, mine[i]);
     }
     lds_barrier();
     bool is_corrupt = false;

@@ -273,7 +273,8 @@ def test_exchange_metadata(rt, r, e, m, k, rank, capacity):
 
 @pytest.mark.parametrize("r,e,rank,capacity", [(1, 1, 0, 8), (1, 7, 0, 0), (3, 9, 2, 300), (2, 10, 1, 40), (5, 255, 4, 2100),
                                                (7, 259, 3, 2049), (32, 256, 31, 4096), (4, 2048, 3, 70000),
-                                               (64, 1024, 1, 300000), (300, 300, 299, 500), (1024, 1024, 700, 20000)])
+                                               (64, 1024, 1, 300000), (300, 300, 299, 500), (1024, 1024, 700, 20000),
+                                               (2, 128, 1, 900), (1, 320, 0, 2000), (3, 576, 1, 700), (5, 480, 2, 700)])
 def test_exchange_metadata_of_every_count(rt, r, e, rank, capacity):
     """Lists of counts that end within a vector, pass a workgroup's loads, or name more experts than it has threads:
     every count is added up, and one too large anywhere is seen."""
